@@ -218,6 +218,27 @@ int xattn_block_sparse_fwd(const void* q, const void* k, const void* v, void* ou
                            int causal, float softmax_scale, void* stream);
 
 /* ---------------------------------------------------------------------------
+ * The prefill operator in one call (Xattention_prefill, xattn/src/Xattention.py:
+ * 302-402): estimate, selection and block-sparse attention enqueued back to
+ * back, everything between them in `workspace` (at least
+ * xattn_prefill_workspace_bytes() bytes, 16-byte aligned, contents undefined on
+ * entry and on return; 0 bytes means the geometry is refused).  Arguments as in
+ * xattn_estimate_select and xattn_block_sparse_fwd, over all query chunks.
+ * Thresholds: `tau_device` (fp64 [H] on the device) or, when that is null,
+ * `tau_host` with one value for all heads or one per head (at most 64), copied
+ * at the call.  At most 8192 key blocks (padded).
+ */
+size_t xattn_prefill_workspace_bytes(int num_heads, int q_len, int k_len, int stride, int chunk_size);
+
+int xattn_prefill_fwd(const void* q, const void* k, const void* v, void* out, void* workspace,
+                      size_t workspace_bytes, int num_heads, int num_kv_heads, int q_len, int k_len, int head_dim,
+                      int64_t q_stride_h, int64_t q_stride_n, int64_t k_stride_h, int64_t k_stride_n,
+                      int64_t v_stride_h, int64_t v_stride_n, int64_t o_stride_h, int64_t o_stride_n, int stride,
+                      int chunk_size, int causal, int own_chunk_only, float estimate_scale, int zero_rows_from,
+                      const double* tau_host, int tau_host_count, const double* tau_device, int keep_sink,
+                      int keep_recent, float softmax_scale, void* stream);
+
+/* ---------------------------------------------------------------------------
  * Single-token decode attention over a KV cache.  Replaces the call to the
  * third-party flashinfer.single_decode_with_kv_cache(q, k, v, kv_layout="HND")
  * in the reference's Llama attention forward, xattn/src/load_llama.py:191-196:

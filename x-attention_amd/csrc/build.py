@@ -1,19 +1,24 @@
-"""Builds libxattn_hip.so (gfx950) next to its sources with hipcc.
+"""Builds libxattn_hip.so (gfx950 kernels behind the C ABI) and xattn_host.so
+(the Python package's native host path) next to their sources.
 
     python x-attention_amd/csrc/build.py
 
-The library is built in-tree so that it travels with the source tree; nothing
+The libraries are built in-tree so that they travel with the source tree; nothing
 is compiled at import time.
 """
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(os.path.dirname(HERE))
-SOURCES = ["capi.hip", "block_sparse_attn.hip", "estimate.hip", "select_blocks.hip", "decode_attn.hip", "profile_threshold.hip", "softmax_block_sum.hip"]
+SOURCES = ["capi.hip", "block_sparse_attn.hip", "estimate.hip", "select_blocks.hip", "decode_attn.hip", "profile_threshold.hip", "softmax_block_sum.hip",
+           "prefill.hip"]
 LIB = os.path.join(HERE, "libxattn_hip.so")
+HOST_SOURCE = os.path.join(HERE, "host_torch.cpp")
+HOST_LIB = os.path.join(HERE, "xattn_host.so")
 FLAGS = [
     "--offload-arch=gfx950",
     "-O3",
@@ -37,6 +42,23 @@ def _run(cmd):
     return out
 
 
+def build_host():
+    """The CPython module over torch's C++ tensors; finds libxattn_hip.so beside itself."""
+    import torch
+
+    tdir = os.path.dirname(torch.__file__)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    return _run([
+        os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        "-I" + os.path.join(ROOT, "include"), "-I" + HERE,
+        "-isystem", os.path.join(tdir, "include"), "-isystem", os.path.join(tdir, "include", "torch", "csrc", "api", "include"),
+        "-isystem", os.path.join(rocm, "include"), "-isystem", sysconfig.get_paths()["include"],
+        HOST_SOURCE, "-o", HOST_LIB, "-L" + HERE, "-lxattn_hip", "-L" + os.path.join(tdir, "lib"),
+        "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN",
+    ])
+
+
 def build(verbose=True):
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     extra = os.environ.get("XATTN_HIPCC_EXTRA", "").split()
@@ -49,12 +71,13 @@ def build(verbose=True):
 
     with ThreadPoolExecutor(max_workers=4) as ex:
         outs = list(ex.map(compile_one, zip(srcs, objs)))
-    outs.append(_run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs))
+    outs.append(_run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, "-Wl,-soname,libxattn_hip.so"] + objs))
+    outs.append(build_host())
     if verbose:
         for o in outs:
             if o.strip():
                 print(o)
-        print("built", LIB)
+        print("built", LIB, HOST_LIB)
     return LIB
 
 

@@ -1,0 +1,53 @@
+// Host side of the estimator as the library's own entry points call it (estimate.hip, prefill.hip).
+#pragma once
+#include <atomic>
+
+#include "xattn_common.h"
+
+namespace xattn {
+
+// Raises a kernel's dynamic LDS limit to the CU's 160 KiB, once per device: the call is host work that every launch
+// would otherwise repeat.
+class LdsLimit {
+ public:
+  hipError_t raise(const void* kernel) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    const uint64_t bit = 1ull << (dev & 63);
+    if (done_.load(std::memory_order_acquire) & bit) return hipSuccess;
+    e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    if (e == hipSuccess) done_.fetch_or(bit, std::memory_order_release);
+    return e;
+  }
+
+ private:
+  std::atomic<uint64_t> done_{0};
+};
+
+// what the fused normalise-and-select pass needs beside the estimator's own arguments
+struct SelectArgs {
+  const double* tau;        // per head, on the device; or null and
+  const double* tau_host;   // one value, or one per head (at most kMaxTauHost), copied into the kernel's arguments
+  int tau_host_count;
+  uint8_t* mask;
+  int32_t* col_idx;
+  int32_t* col_cnt;
+  int64_t idx_pitch;
+  int keep_sink, keep_recent;
+  int real_q_blocks_only;   // leave out the rows of q-blocks past the sequence end
+  int stages;               // bit 0: run the GEMM pass, bit 1: run the normalise-and-select pass
+};
+
+int estimate_impl(const void* q, const void* k, float* block_sums, void* workspace, size_t workspace_size,
+                  float* scores_out, int num_heads, int num_kv_heads, int q_len, int k_len, int head_dim,
+                  int64_t q_stride_h, int64_t q_stride_n, int64_t k_stride_h, int64_t k_stride_n, int stride,
+                  int block_size, int chunk_size, int chunk_begin, int chunk_end, int causal, int own_chunk_only,
+                  float scale, const int32_t* slab_pairs, int num_slab_pairs, int softmax, int kdb,
+                  int zero_rows_from, int window_row0, int window_rows, void* stream, const SelectArgs* sel);
+
+// estimator workspace of one launch over every query chunk when only the rows of real q-blocks are computed; 0 if the
+// geometry is not accepted
+size_t estimate_real_rows_bytes(int num_heads, int q_len, int k_len, int stride, int block_size, int chunk_size);
+
+}  // namespace xattn

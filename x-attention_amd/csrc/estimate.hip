@@ -23,6 +23,7 @@
 //    and adds the block_size/S rows of each query block.
 #include <mutex>
 
+#include "estimate.h"
 #include "select_row.h"
 #include "xattn_hip.h"
 
@@ -51,7 +52,9 @@ struct EstParams {
   int kdb;                  // query-row subsampling: query row m stands for reshaped row m * kdb
   int rcs_q, rbs_q;         // query rows per chunk / per query block (rcs / kdb, rbs / kdb)
   int row_begin, row_end;   // query rows handled by this call
-  int rows;                 // row_end - row_begin (pitch of P / Mt / Lt)
+  int live_end;             // rows at or past it give zero block sums (padding) or are not asked for: never computed
+  int rows;                 // live_end - row_begin (pitch of P / Mt / Lt)
+  int nT_real;              // 128-key tiles from here on hold padded keys only (nT when causal): not computed either
   int off;                  // position of reshaped row 0 on the key axis: n_rk - n_rq * kdb
   int real_rows;            // query rows >= real_rows give all-zero block sums
   int causal, own_chunk_only;
@@ -148,7 +151,7 @@ __device__ __forceinline__ bool decode_tile(const EstParams& p, int64_t id, Tile
   int nt_first = 0;
   for (;;) {
     const int mfirst = p.row_begin + c.mt_row * kTile;
-    const int mlast = (mfirst + kTile - 1 < p.row_end ? mfirst + kTile - 1 : p.row_end - 1);
+    const int mlast = (mfirst + kTile - 1 < p.live_end ? mfirst + kTile - 1 : p.live_end - 1);
     int hi = row_hi(p, mlast) / kTile;
     hi = hi < p.nNT - 1 ? hi : p.nNT - 1;
     nt_first = row_lo(p, mfirst) / kTile;
@@ -337,7 +340,7 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
 #pragma unroll
   for (int mt = 0; mt < 2; ++mt) {
     const int m = m0 + wm * kRowsW + mt * 32 + r;
-    const bool row_ok = m < p.row_end;
+    const bool row_ok = m < p.live_end;
     const int lo = row_lo(p, m), hi = row_hi(p, m);
     if (kDump && row_ok) {
       float* dst = p.scores + ((int64_t)head * p.n_rq + m) * p.n_rk;
@@ -470,6 +473,37 @@ __device__ __forceinline__ float group_sum4(const f32x4& pv, const f32x4& mt, co
 }
 #pragma clang fp contract(fast)
 
+// A 128-key tile that holds nothing but padded keys is not computed: its scores are zero, so its maximum is 0, every
+// visible key adds 2^0 and a key block's partial sum is its key count - what the MFMA pass would have written.
+// Only without causality (a causal row sees such a tile partly; nT_real is nT then).
+__device__ __forceinline__ void tile_stat(const EstParams& p, const float* Mst, const float* Lst, int T, int mrel, float& mt,
+                                          float& lt) {
+  if (T < p.nT_real) {
+    mt = Mst[(int64_t)T * p.rows + mrel];
+    lt = Lst[(int64_t)T * p.rows + mrel];
+  } else {
+    const int left = p.n_rk - T * kSub;
+    mt = 0.f;
+    lt = (float)(left < kSub ? left : kSub);
+  }
+}
+// tile maxima and partial sums of key block kb for four consecutive rows
+template <int RBS>
+__device__ __forceinline__ void load_partial(const EstParams& p, const float* Mst, const float* Pst, int kb, int mrel4, f32x4& mt,
+                                             f32x4& pv) {
+  const int T = (kb * RBS) / kSub;
+  if (T < p.nT_real) {
+    mt = *reinterpret_cast<const f32x4*>(Mst + (int64_t)T * p.rows + mrel4);
+    pv = *reinterpret_cast<const f32x4*>(Pst + (int64_t)kb * p.rows + mrel4);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      mt[i] = 0.f;
+      pv[i] = (float)RBS;
+    }
+  }
+}
+
 // One workgroup = 64 consecutive reshaped query rows of one head.
 // Pass 1 (lane <-> row, wavefronts split the 128-key tiles) combines the tile
 // maxima / sums into each row's softmax statistics.  Pass 2 rescales the partial
@@ -491,15 +525,19 @@ __global__ __launch_bounds__(256) void estimate_normalize_kernel(EstParams p) {
 
   {
     const int m = strip0 + lane;
-    const bool row_ok = m < p.row_end;
-    const int mc = row_ok ? m : p.row_end - 1;
+    const bool row_ok = m < p.live_end;
+    const int mc = row_ok ? m : p.row_begin;
     const int mrel = mc - p.row_begin;
     const int lo = row_lo(p, mc);
     int hi = row_hi(p, mc);
     hi = hi < p.n_rk - 1 ? hi : p.n_rk - 1;
     float M = -INFINITY, L = 0.f;
-    for (int T = lo / kSub + wave; T <= hi / kSub; T += 4)
-      stat_step(M, L, Mst[(int64_t)T * p.rows + mrel], Lst[(int64_t)T * p.rows + mrel]);
+    if (row_ok)
+      for (int T = lo / kSub + wave; T <= hi / kSub; T += 4) {
+        float mt, lt;
+        tile_stat(p, Mst, Lst, T, mrel, mt, lt);
+        stat_step(M, L, mt, lt);
+      }
     redM[wave][lane] = M;
     redL[wave][lane] = L;
     __syncthreads();
@@ -514,6 +552,7 @@ __global__ __launch_bounds__(256) void estimate_normalize_kernel(EstParams p) {
   const int l16 = lane & 15, kgrp = lane >> 4;
   const int m4 = strip0 + l16 * 4;                 // first of this lane's 4 rows
   const bool rows_ok = m4 < p.row_end;             // row ranges are multiples of 8: all 4 or none
+  const bool rows_live = m4 < p.live_end;
   const int mc4 = rows_ok ? m4 : p.row_begin;
   const int mrel4 = mc4 - p.row_begin;
   const f32x4 rM = *reinterpret_cast<const f32x4*>(rowM + l16 * 4);
@@ -536,12 +575,8 @@ __global__ __launch_bounds__(256) void estimate_normalize_kernel(EstParams p) {
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
       const int kb = kb0 + 16 * u + kgrp;
-      live[u] = rows_ok && kb < p.nkb && kb >= kb_lo && kb <= kb_hi;
-      if (live[u]) {
-        const int T = (kb * RBS) / kSub;
-        mt[u] = *reinterpret_cast<const f32x4*>(Mst + (int64_t)T * p.rows + mrel4);
-        pv[u] = *reinterpret_cast<const f32x4*>(Pst + (int64_t)kb * p.rows + mrel4);
-      }
+      live[u] = rows_live && kb < p.nkb && kb >= kb_lo && kb <= kb_hi;
+      if (live[u]) load_partial<RBS>(p, Mst, Pst, kb, mrel4, mt[u], pv[u]);
     }
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
@@ -575,7 +610,7 @@ __global__ __launch_bounds__(256) void estimate_select_kernel(EstParams p, SelPa
   const size_t wave_bytes = (size_t)sp.npow2 * 8 + nkb_pad;
   const size_t xs_off = (size_t)sp.npow2 * 8 - (size_t)nkb_pad * 4;
 
-  const int qrows = (p.row_end - p.row_begin) / RBS;     // q-block rows of this call
+  const int qrows = sp.row_end - sp.row_begin;           // q-block rows of this call
   const int groups = (qrows + qb_per_wg - 1) / qb_per_wg;
   const int head = blockIdx.x / groups;
   const int grp = blockIdx.x % groups;
@@ -588,26 +623,25 @@ __global__ __launch_bounds__(256) void estimate_select_kernel(EstParams p, SelPa
   for (int idx = tid; idx < rows_wg * 4; idx += blockDim.x) {
     const int lrow = idx % rows_wg, w = idx / rows_wg;
     const int m = strip0 + lrow;
-    const int mc = m < p.row_end ? m : p.row_end - 1;
+    const bool row_ok = m < p.live_end;
+    const int mc = row_ok ? m : p.row_begin;
     const int mrel = mc - p.row_begin;
     const int lo = row_lo(p, mc);
     int hi = row_hi(p, mc);
     hi = hi < p.n_rk - 1 ? hi : p.n_rk - 1;
+    const int last = row_ok ? hi / kSub : -1;
     float M = -INFINITY, L = 0.f;
     // eight tiles' statistics are requested before the first is folded in (the folding is a dependent chain)
-    for (int T0 = lo / kSub + w; T0 <= hi / kSub; T0 += 32) {
+    for (int T0 = lo / kSub + w; T0 <= last; T0 += 32) {
       float mt[8], lt[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         const int T = T0 + 4 * u;
-        if (T <= hi / kSub) {
-          mt[u] = Mst[(int64_t)T * p.rows + mrel];
-          lt[u] = Lst[(int64_t)T * p.rows + mrel];
-        }
+        if (T <= last) tile_stat(p, Mst, Lst, T, mrel, mt[u], lt[u]);
       }
 #pragma unroll
       for (int u = 0; u < 8; ++u)
-        if (T0 + 4 * u <= hi / kSub) stat_step(M, L, mt[u], lt[u]);
+        if (T0 + 4 * u <= last) stat_step(M, L, mt[u], lt[u]);
     }
     redM[w * rows_wg + lrow] = M;
     redL[w * rows_wg + lrow] = L;
@@ -615,7 +649,7 @@ __global__ __launch_bounds__(256) void estimate_select_kernel(EstParams p, SelPa
   __syncthreads();
   for (int lrow = tid; lrow < rows_wg; lrow += blockDim.x) {
     const int m = strip0 + lrow;
-    const bool row_ok = m < p.row_end;
+    const bool row_ok = m < p.live_end;
     const float Mw[4] = {redM[lrow], redM[rows_wg + lrow], redM[2 * rows_wg + lrow], redM[3 * rows_wg + lrow]};
     const float Lw[4] = {redL[lrow], redL[rows_wg + lrow], redL[2 * rows_wg + lrow], redL[3 * rows_wg + lrow]};
     stat_combine(Mw, Lw, row_ok && m < p.real_rows, p.no_softmax, &rowM[lrow], &rowInv[lrow]);
@@ -630,6 +664,7 @@ __global__ __launch_bounds__(256) void estimate_select_kernel(EstParams p, SelPa
     const int l = tid % lpk, kgrp = tid / lpk, kb_step = blockDim.x / lpk;
     const int m4 = strip0 + l * 4;
     const bool rows_ok = m4 < p.row_end;
+    const bool rows_live = m4 < p.live_end;
     const int mc4 = rows_ok ? m4 : p.row_begin;
     const int mrel4 = mc4 - p.row_begin;
     const f32x4 rM = *reinterpret_cast<const f32x4*>(rowM + l * 4);
@@ -647,12 +682,8 @@ __global__ __launch_bounds__(256) void estimate_select_kernel(EstParams p, SelPa
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
         const int kb = kb0 + kb_step * u;
-        live[u] = rows_ok && kb < p.nkb && kb >= kb_lo && kb <= kb_hi;
-        if (live[u]) {
-          const int T = (kb * RBS) / kSub;
-          mt[u] = *reinterpret_cast<const f32x4*>(Mst + (int64_t)T * p.rows + mrel4);
-          pv[u] = *reinterpret_cast<const f32x4*>(Pst + (int64_t)kb * p.rows + mrel4);
-        }
+        live[u] = rows_live && kb < p.nkb && kb >= kb_lo && kb <= kb_hi;
+        if (live[u]) load_partial<RBS>(p, Mst, Pst, kb, mrel4, mt[u], pv[u]);
       }
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
@@ -672,7 +703,7 @@ __global__ __launch_bounds__(256) void estimate_select_kernel(EstParams p, SelPa
   // selection: wavefront i takes q-block row i of the group
   if (wave < qb_per_wg) {
     const int row = strip0 / RBS + wave;                 // q-block row (row_begin is a multiple of RBS)
-    if (row < p.row_end / RBS) {
+    if (row < sp.row_end) {
       char* mine = per_wave + (size_t)wave * wave_bytes;
       select_row(sp, reinterpret_cast<const float*>(mine + xs_off), head, row, reinterpret_cast<uint64_t*>(mine),
                  reinterpret_cast<uint8_t*>(mine + (size_t)sp.npow2 * 8), lane);
@@ -696,16 +727,16 @@ __global__ __launch_bounds__(256) void estimate_normalize_rows_kernel(EstParams 
   const float* Pst = p.P + (int64_t)head * p.nkb * p.rows;
   const float* Mst = p.Mt + (int64_t)head * p.nT * p.rows;
   const float* Lst = p.Lt + (int64_t)head * p.nT * p.rows;
-  const bool row_ok = row < p.rbs_q && m0 + row < p.row_end;
-  const int m = row_ok ? m0 + row : m0;
+  const bool row_ok = row < p.rbs_q && m0 + row < p.live_end;
+  const int m = row_ok ? m0 + row : p.row_begin;
   const int mrel = m - p.row_begin;
   const int lo = row_lo(p, m);
   int hi = row_hi(p, m);
   hi = hi < p.n_rk - 1 ? hi : p.n_rk - 1;
   float M = -INFINITY, L = 0.f;
-  for (int T = lo / kSub + part; T <= hi / kSub; T += 8) {
-    const float mt = Mst[(int64_t)T * p.rows + mrel];
-    const float lt = Lst[(int64_t)T * p.rows + mrel];
+  for (int T = lo / kSub + part; row_ok && T <= hi / kSub; T += 8) {
+    float mt, lt;
+    tile_stat(p, Mst, Lst, T, mrel, mt, lt);
     const float Mn = fmaxf(M, mt);
     const float safe = (Mn == -INFINITY) ? 0.f : Mn;
     L = L * fast_exp2(M - safe) + lt * fast_exp2(mt - safe);
@@ -731,12 +762,15 @@ __global__ __launch_bounds__(256) void estimate_normalize_rows_kernel(EstParams 
     float acc = 0.f;
     for (int r = 0; r < p.rbs_q; ++r) {
       const int mr = m0 + r;
-      if (mr >= p.row_end || rowInv[r] == 0.f) continue;
+      if (mr >= p.live_end || rowInv[r] == 0.f) continue;
       int h2 = row_hi(p, mr);
       h2 = h2 < p.n_rk - 1 ? h2 : p.n_rk - 1;
       if (kb < row_lo(p, mr) / p.rbs || kb > h2 / p.rbs) continue;
       const int rel = mr - p.row_begin;
-      acc += Pst[(int64_t)kb * p.rows + rel] * fast_exp2(Mst[(int64_t)T * p.rows + rel] - rowM[r]) * rowInv[r];
+      const bool real = T < p.nT_real;
+      const float pv = real ? Pst[(int64_t)kb * p.rows + rel] : (float)p.rbs;
+      const float mt = real ? Mst[(int64_t)T * p.rows + rel] : 0.f;
+      acc += pv * fast_exp2(mt - rowM[r]) * rowInv[r];
     }
     out[kb] = acc;
   }
@@ -747,14 +781,27 @@ __global__ __launch_bounds__(256) void estimate_normalize_rows_kernel(EstParams 
 using namespace xattn;
 
 namespace {
-template <int RBS>
-hipError_t launch_gemm(const EstParams& p, dim3 grid, size_t lds, hipStream_t s) {
-  auto kernel = p.n_pairs ? (p.scores ? &estimate_gemm_kernel<RBS, true, true> : &estimate_gemm_kernel<RBS, false, true>)
-                          : (p.scores ? &estimate_gemm_kernel<RBS, true, false> : &estimate_gemm_kernel<RBS, false, false>);
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+template <int RBS, bool kDump, bool kTable>
+hipError_t launch_gemm_as(const EstParams& p, dim3 grid, size_t lds, hipStream_t s) {
+  auto kernel = &estimate_gemm_kernel<RBS, kDump, kTable>;
+  static LdsLimit limit;
+  hipError_t e = limit.raise(reinterpret_cast<const void*>(kernel));
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(kernel, grid, dim3(kWaves * 64), lds, s, p);
+  return hipSuccess;
+}
+template <int RBS>
+hipError_t launch_gemm(const EstParams& p, dim3 grid, size_t lds, hipStream_t s) {
+  if (p.n_pairs) return p.scores ? launch_gemm_as<RBS, true, true>(p, grid, lds, s) : launch_gemm_as<RBS, false, true>(p, grid, lds, s);
+  return p.scores ? launch_gemm_as<RBS, true, false>(p, grid, lds, s) : launch_gemm_as<RBS, false, false>(p, grid, lds, s);
+}
+template <int RBS>
+hipError_t launch_select(const EstParams& p, const SelParams& sp, int qb_per_wg, dim3 grid, size_t lds, hipStream_t s) {
+  auto kernel = &estimate_select_kernel<RBS>;
+  static LdsLimit limit;
+  hipError_t e = limit.raise(reinterpret_cast<const void*>(kernel));
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kernel, grid, dim3(64 * qb_per_wg), lds, s, p, sp, qb_per_wg);
   return hipSuccess;
 }
 
@@ -800,6 +847,13 @@ size_t workspace_bytes(int H, const Geometry& g, int rows) {
 }
 }  // namespace
 
+size_t xattn::estimate_real_rows_bytes(int num_heads, int q_len, int k_len, int stride, int block_size, int chunk_size) {
+  Geometry g;
+  if (num_heads <= 0 || block_size != 128 || (stride != 4 && stride != 8 && stride != 16)) return 0;
+  if (!geometry(q_len, k_len, stride, block_size, chunk_size, &g)) return 0;
+  return workspace_bytes(num_heads, g, (int)(((int64_t)q_len + block_size - 1) / block_size * (block_size / stride)));
+}
+
 extern "C" size_t xattn_estimate_workspace_bytes(int num_heads, int q_len, int k_len, int stride,
                                                  int block_size, int chunk_size, int chunks_per_call) {
   Geometry g;
@@ -809,18 +863,7 @@ extern "C" size_t xattn_estimate_workspace_bytes(int num_heads, int q_len, int k
   return workspace_bytes(num_heads, g, c * g.rcs);   // (an upper bound when query rows are subsampled)
 }
 
-namespace {
-// what the fused normalise-and-select pass needs beside the estimator's own arguments
-struct SelectArgs {
-  const double* tau;
-  uint8_t* mask;
-  int32_t* col_idx;
-  int32_t* col_cnt;
-  int64_t idx_pitch;
-  int keep_sink, keep_recent;
-  int stages;               // bit 0: run the GEMM pass, bit 1: run the normalise-and-select pass
-};
-
+namespace xattn {
 int estimate_impl(const void* q, const void* k, float* block_sums, void* workspace, size_t workspace_size,
                   float* scores_out, int num_heads, int num_kv_heads, int q_len, int k_len, int head_dim,
                   int64_t q_stride_h, int64_t q_stride_n, int64_t k_stride_h, int64_t k_stride_n, int stride,
@@ -830,7 +873,8 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
   if (!q || !k || !workspace) return XATTN_ERR_NULL;
   if (!block_sums && !sel) return XATTN_ERR_NULL;
   if (sel) {
-    if (!sel->tau) return XATTN_ERR_NULL;
+    if (!sel->tau && !sel->tau_host) return XATTN_ERR_NULL;
+    if (!sel->tau && sel->tau_host_count != 1 && (sel->tau_host_count != num_heads || num_heads > kMaxTauHost)) return XATTN_ERR_HEADS;
     if ((sel->col_idx == nullptr) != (sel->col_cnt == nullptr)) return XATTN_ERR_NULL;
     if (!sel->mask && !sel->col_idx) return XATTN_ERR_NULL;     // nothing to write
     if (sel->col_idx && sel->idx_pitch < 1) return XATTN_ERR_SHAPE;
@@ -865,7 +909,6 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
   p.kdb = kdb; p.rcs_q = g.rcs / kdb; p.rbs_q = p.rbs / kdb;
   p.row_begin = chunk_begin * p.rcs_q;
   p.row_end = chunk_end * p.rcs_q;
-  p.rows = p.row_end - p.row_begin;
   p.off = g.n_rk - g.n_rq;
   // default: the torch branch's rule for kdb = 1 (the padded tail, xattn/src/Xattention.py:237-238)
   p.real_rows = zero_rows_from >= 0 ? zero_rows_from : p.n_rq - g.q_pad / stride / kdb;
@@ -873,6 +916,22 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
   p.own_chunk_only = own_chunk_only ? 1 : 0;
   p.scale_log2 = scale * kLog2e;
   p.no_softmax = softmax ? 0 : 1;
+  // Rows past the real ones give zero block sums, and the operator has no use for the rows of q-blocks past the
+  // sequence end: neither is computed (a 1000-token prompt is padded to 2048 tokens, a 500-token turn on a 9k cache to
+  // 16384).  The scores dump of the seam keeps every row.
+  p.live_end = p.row_end;
+  const int nqb_real = (q_len + block_size - 1) / block_size;
+  if (!scores_out) {
+    int64_t live = ((int64_t)p.real_rows + p.rbs_q - 1) / p.rbs_q * p.rbs_q;
+    if (sel && sel->real_q_blocks_only && live > (int64_t)nqb_real * p.rbs_q) live = (int64_t)nqb_real * p.rbs_q;
+    if (live < p.live_end) p.live_end = live < p.row_begin ? p.row_begin : (int)live;
+  }
+  p.rows = p.live_end - p.row_begin;
+  p.nT_real = g.nT;
+  if (!causal && !scores_out) {
+    const int64_t keys = ((int64_t)k_len + stride - 1) / stride;
+    p.nT_real = (int)((keys + kSub - 1) / kSub);
+  }
   p.n_pairs = 0;
   if (num_slab_pairs < 0 || num_slab_pairs > 64 || (num_slab_pairs > 0 && !slab_pairs)) return XATTN_ERR_SHAPE;
   for (int j = 0; j < num_slab_pairs; ++j) {
@@ -887,8 +946,9 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
   {
     const int bpc = chunk_size / block_size;
     if (window_rows <= 0) { window_row0 = 0; window_rows = g.nqb; }
-    if (window_row0 < 0 || chunk_begin * bpc < window_row0 || chunk_end * bpc > window_row0 + window_rows)
-      return XATTN_ERR_SHAPE;
+    int qb_end = chunk_end * bpc;
+    if (sel && sel->real_q_blocks_only && qb_end > nqb_real) qb_end = nqb_real;
+    if (window_row0 < 0 || chunk_begin * bpc < window_row0 || qb_end > window_row0 + window_rows) return XATTN_ERR_SHAPE;
     p.win_row0 = window_row0;
     p.win_rows = window_rows;
   }
@@ -900,11 +960,11 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
 
   hipStream_t s = static_cast<hipStream_t>(stream);
   p.nMT = (p.rows + kTile - 1) / kTile;
-  p.nNT = (g.n_rk + kTile - 1) / kTile;
+  p.nNT = ((p.nT_real < g.nT ? p.nT_real * kSub : g.n_rk) + kTile - 1) / kTile;
   p.tiles_per_head = 0;
   for (int r = 0; r < p.nMT; ++r) {   // same visibility rule as the kernel's row_lo / row_hi
     const int mfirst = p.row_begin + r * kTile;
-    const int mlast = (mfirst + kTile - 1 < p.row_end ? mfirst + kTile - 1 : p.row_end - 1);
+    const int mlast = (mfirst + kTile - 1 < p.live_end ? mfirst + kTile - 1 : p.live_end - 1);
     int hi = row_hi(p, mlast) / kTile;
     hi = hi < p.nNT - 1 ? hi : p.nNT - 1;
     const int lo = row_lo(p, mfirst) / kTile;
@@ -917,7 +977,7 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
   const int resident = resident_workgroups();
   if (resident <= 0) return XATTN_ERR_LAUNCH;
   const dim3 grid1((unsigned)(ids < resident ? ids : resident));
-  const dim3 grid2((p.rows + 63) / 64, num_heads);
+  const dim3 grid2((p.row_end - p.row_begin + 63) / 64, num_heads);
   if (grid2.y > 65535) return XATTN_ERR_SHAPE;
   const size_t lds = 2 * (size_t)kStageBytes;
   // the fused normalise-and-select pass: QB q-block rows (one wavefront each) per workgroup, as many as keep a
@@ -929,9 +989,16 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
   if (sel) {
     if (g.nkb > 8192) return XATTN_ERR_SHAPE;      // (longer rows: block sums through memory, xattn_select_blocks)
     const int bpc = chunk_size / block_size;
-    sp.sums = nullptr; sp.tau = sel->tau; sp.mask = sel->mask; sp.col_idx = sel->col_idx; sp.col_cnt = sel->col_cnt;
+    sp.sums = nullptr;
+    sp.tau = sel->tau;
+    sp.tau_step = sel->tau_host_count == 1 ? 0 : 1;
+    if (!sel->tau)
+      for (int h = 0; h < sel->tau_host_count; ++h) sp.tau_val[h] = sel->tau_host[h];
+    sp.mask = sel->mask; sp.col_idx = sel->col_idx; sp.col_cnt = sel->col_cnt;
     sp.idx_pitch = sel->idx_pitch; sp.H = num_heads; sp.nqb = g.nqb; sp.nkb = g.nkb;
-    sp.row_begin = chunk_begin * bpc; sp.row_end = chunk_end * bpc; sp.diag_offset = g.nkb - g.nqb;
+    sp.row_begin = chunk_begin * bpc;
+    sp.row_end = sel->real_q_blocks_only && nqb_real < chunk_end * bpc ? nqb_real : chunk_end * bpc;
+    sp.diag_offset = g.nkb - g.nqb;
     sp.win_row0 = p.win_row0; sp.win_rows = p.win_rows;
     sp.causal = p.causal; sp.keep_sink = sel->keep_sink ? 1 : 0; sp.keep_recent = sel->keep_recent ? 1 : 0;
     sp.list_cols = (k_len + block_size - 1) / block_size; sp.q_len = q_len; sp.kv_off = k_len - q_len;
@@ -945,41 +1012,39 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
     while (qb_per_wg > 1 && (qb_per_wg * (wave_bytes + 10 * p.rbs * sizeof(float)) > 64 * 1024 || qb_per_wg * p.rbs > 128))
       qb_per_wg >>= 1;
     lds_sel = qb_per_wg * (wave_bytes + 10 * p.rbs * sizeof(float));
-    const int qrows = p.rows / p.rbs;
+    const int qrows = sp.row_end > sp.row_begin ? sp.row_end - sp.row_begin : 0;
     const int64_t wgs = (int64_t)num_heads * ((qrows + qb_per_wg - 1) / qb_per_wg);
     if (wgs > 0x7fffffff) return XATTN_ERR_SHAPE;
     grid_sel = dim3((unsigned)wgs);
   }
-  auto launch_rest = [&](auto normalize, auto fused) -> hipError_t {
+  auto launch_rest = [&](auto rbs) -> hipError_t {
+    constexpr int RBS = decltype(rbs)::value;
     if (!sel) {
-      if (kdb == 1) hipLaunchKernelGGL(normalize, grid2, dim3(256), 0, s, p);
+      if (kdb == 1) hipLaunchKernelGGL(estimate_normalize_kernel<RBS>, grid2, dim3(256), 0, s, p);
       return hipSuccess;
     }
-    hipError_t e2 = hipFuncSetAttribute(reinterpret_cast<const void*>(fused), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                        (int)lds_sel);
-    if (e2 != hipSuccess) return e2;
-    hipLaunchKernelGGL(fused, grid_sel, dim3(64 * qb_per_wg), lds_sel, s, p, sp, qb_per_wg);
-    return hipSuccess;
+    if (sp.row_end <= sp.row_begin) return hipSuccess;   // a chunk of padding alone
+    return launch_select<RBS>(p, sp, qb_per_wg, grid_sel, lds_sel, s);
   };
   const bool run_gemm = !sel || (sel->stages & 1), run_rest = !sel || (sel->stages & 2);
   hipError_t e = hipSuccess;
   switch (p.rbs) {
     case 8:
-      if (run_gemm) e = launch_gemm<8>(p, grid1, lds, s);
-      if (e == hipSuccess && run_rest) e = launch_rest(&estimate_normalize_kernel<8>, &estimate_select_kernel<8>);
+      if (run_gemm && p.total_tiles > 0) e = launch_gemm<8>(p, grid1, lds, s);
+      if (e == hipSuccess && run_rest) e = launch_rest(std::integral_constant<int, 8>());
       break;
     case 16:
-      if (run_gemm) e = launch_gemm<16>(p, grid1, lds, s);
-      if (e == hipSuccess && run_rest) e = launch_rest(&estimate_normalize_kernel<16>, &estimate_select_kernel<16>);
+      if (run_gemm && p.total_tiles > 0) e = launch_gemm<16>(p, grid1, lds, s);
+      if (e == hipSuccess && run_rest) e = launch_rest(std::integral_constant<int, 16>());
       break;
     default:
-      if (run_gemm) e = launch_gemm<32>(p, grid1, lds, s);
-      if (e == hipSuccess && run_rest) e = launch_rest(&estimate_normalize_kernel<32>, &estimate_select_kernel<32>);
+      if (run_gemm && p.total_tiles > 0) e = launch_gemm<32>(p, grid1, lds, s);
+      if (e == hipSuccess && run_rest) e = launch_rest(std::integral_constant<int, 32>());
       break;
   }
   if (e != hipSuccess) return XATTN_ERR_LAUNCH;
   if (kdb != 1) {
-    const dim3 grid3(p.rows / p.rbs_q, num_heads);
+    const dim3 grid3((p.row_end - p.row_begin) / p.rbs_q, num_heads);
     hipLaunchKernelGGL(estimate_normalize_rows_kernel, grid3, dim3(256), 0, s, p);
   }
   return hipGetLastError() == hipSuccess ? XATTN_OK : XATTN_ERR_LAUNCH;
@@ -1011,7 +1076,9 @@ extern "C" int xattn_estimate_select(const void* q, const void* k, float* block_
                                      int window_row0, int window_rows, const double* tau_per_head, uint8_t* mask,
                                      int32_t* col_idx, int32_t* col_cnt, int64_t idx_pitch, int keep_sink,
                                      int keep_recent, int stages, void* stream) {
-  const SelectArgs sel = {tau_per_head, mask, col_idx, col_cnt, idx_pitch, keep_sink, keep_recent, stages};
+  SelectArgs sel{};
+  sel.tau = tau_per_head; sel.mask = mask; sel.col_idx = col_idx; sel.col_cnt = col_cnt; sel.idx_pitch = idx_pitch;
+  sel.keep_sink = keep_sink; sel.keep_recent = keep_recent; sel.stages = stages;
   return estimate_impl(q, k, block_sums, workspace, workspace_size, nullptr, num_heads, num_kv_heads, q_len, k_len,
                        head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, stride, block_size, chunk_size,
                        chunk_begin, chunk_end, causal, own_chunk_only, scale, slab_pairs, num_slab_pairs, softmax, 1,

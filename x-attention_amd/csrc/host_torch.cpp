@@ -1,0 +1,147 @@
+// Native host path of the Python package: reads sizes, strides and pointers straight from the tensors, allocates the
+// output and one workspace from torch's caching allocator, and enqueues through the C ABI of libxattn_hip.so on the
+// current stream.
+//
+// The short calls - a prompt of a thousand tokens, a decode step - are bound by host time when every size is a Python
+// attribute lookup and every launch a ctypes call with forty conversions.  Each function here handles the ordinary
+// form of its call and returns None for anything else (tensors to be made contiguous, other devices, arguments to be
+// refused); the Python code then takes over, and raises where there is something to raise.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cmath>
+#include <optional>
+
+#include "xattn_hip.h"
+
+namespace {
+
+// A bf16 tensor on a ROCm device as the kernels read it: feature dimension contiguous, 16-byte aligned rows.
+inline bool kernel_ready(const at::Tensor& t, int64_t dim) {
+  const int64_t n = t.dim();
+  return t.is_cuda() && t.scalar_type() == at::kBFloat16 && n == dim && t.size(n - 1) == 128 && t.stride(n - 1) == 1 &&
+         t.stride(n - 2) % 8 == 0 && t.stride(n - 3) % 8 == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
+}
+
+inline const at::Tensor* tensor_of(PyObject* o) { return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
+
+// Makes a tensor's device current for the launches, and only if it is not.
+struct OnDevice {
+  explicit OnDevice(c10::Device d) {
+    if (c10::hip::current_device() != d.index()) guard.emplace(d);
+  }
+  std::optional<c10::DeviceGuard> guard;
+};
+
+inline void* stream_of(c10::Device d) { return static_cast<void*>(c10::hip::getCurrentHIPStream(d.index()).stream()); }
+
+PyObject* fail(const char* what, int code) {
+  // the package's own error type, looked up only when something went wrong
+  PyObject* mod = PyImport_ImportModule("xattn.src.hip_backend");
+  PyObject* type = mod ? PyObject_GetAttrString(mod, "XattnHipError") : nullptr;
+  if (type) PyErr_Format(type, "%s failed: %s (code %d)", what, xattn_error_string(code), code);
+  Py_XDECREF(type);
+  Py_XDECREF(mod);
+  return nullptr;
+}
+
+// Thresholds of a call: host values (one, or one per head), or a float64 [H] device tensor.
+struct Tau {
+  double host[64];
+  int count = 0;
+  at::Tensor device;
+};
+
+bool read_tau(PyObject* o, int64_t heads, c10::Device dev, Tau* tau) {
+  const at::Tensor* t = tensor_of(o);
+  if (!t) {
+    tau->host[0] = PyFloat_AsDouble(o);
+    if (PyErr_Occurred()) {
+      PyErr_Clear();
+      return false;
+    }
+    tau->count = 1;
+    return true;
+  }
+  const int64_t n = t->numel();
+  if (n != 1 && n != heads) return false;
+  if (t->is_cpu() && n <= 64) {
+    // a tensor keeps its own precision (xattn/src/utils.py:91-92): converted to double value by value, no copy to the
+    // device and no wait for it
+    const at::Tensor d = t->scalar_type() == at::kDouble && t->is_contiguous() ? *t : t->detach().to(at::kDouble).contiguous();
+    const double* src = d.const_data_ptr<double>();
+    for (int64_t i = 0; i < n; ++i) tau->host[i] = src[i];
+    tau->count = (int)n;
+    return true;
+  }
+  tau->device = t->detach().to(at::kDouble).reshape({-1}).expand({heads}).contiguous().to(dev);
+  return true;
+}
+
+// prefill(q, k, v, stride, norm, threshold, use_triton, causal, chunk_size, keep_sink, keep_recent, workspace_limit)
+PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 12) return PyErr_Format(PyExc_TypeError, "prefill takes 12 arguments");
+  HANDLE_TH_ERRORS
+  const at::Tensor *q = tensor_of(args[0]), *k = tensor_of(args[1]), *v = tensor_of(args[2]);
+  if (!q || !k || !v) Py_RETURN_NONE;
+  const long stride = PyLong_AsLong(args[3]);
+  const double norm = PyFloat_AsDouble(args[4]);
+  const long chunk = PyLong_AsLong(args[8]);
+  const long long limit = PyLong_AsLongLong(args[11]);
+  const int use_triton = PyObject_IsTrue(args[6]), causal = PyObject_IsTrue(args[7]);
+  const int keep_sink = PyObject_IsTrue(args[9]), keep_recent = PyObject_IsTrue(args[10]);
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  if (!kernel_ready(*q, 4) || !kernel_ready(*k, 4) || !kernel_ready(*v, 4)) Py_RETURN_NONE;
+  const c10::Device dev = q->device();
+  if (k->device() != dev || v->device() != dev) Py_RETURN_NONE;
+  const int64_t H = q->size(1), Lq = q->size(2), Hkv = k->size(1), Lk = k->size(2);
+  if (q->size(0) != 1 || k->size(0) != 1 || v->size(0) != 1 || v->size(1) != Hkv || v->size(2) != Lk) Py_RETURN_NONE;
+  if ((stride != 4 && stride != 8 && stride != 16) || !(norm > 0) || H < 1 || Hkv < 1 || H % Hkv || Lq < 1 || Lk < Lq ||
+      Lk > (int64_t(1) << 30) || chunk < 128 || chunk % 128 || chunk > (1 << 30))
+    Py_RETURN_NONE;
+  const size_t bytes = xattn_prefill_workspace_bytes((int)H, (int)Lq, (int)Lk, (int)stride, (int)chunk);
+  if (bytes == 0 || (long long)bytes > limit || (Lk + chunk - 1) / chunk * chunk / 128 > 8192) Py_RETURN_NONE;
+  // which rows and keys the reference's branches hide (see _Plan in xattn/src/Xattention.py of this package)
+  const int64_t q_pad = (chunk - Lq % chunk) % chunk, k_pad = (chunk - Lk % chunk) % chunk;
+  const int own_chunk = causal && !use_triton && k_pad / stride == 0;
+  const int64_t n_rq = (Lq + q_pad) / stride;
+  int64_t zero_from;
+  if (use_triton)
+    zero_from = std::max<int64_t>(0, n_rq - k_pad / stride);
+  else
+    zero_from = n_rq - q_pad / stride;
+  OnDevice on(dev);
+  Tau tau;
+  if (!read_tau(args[5], H, dev, &tau)) Py_RETURN_NONE;
+  const auto opts = at::TensorOptions().device(dev);
+  at::Tensor out = at::empty_strided({1, H, Lq, 128}, {Lq * H * 128, 128, H * 128, 1}, opts.dtype(at::kBFloat16));
+  at::Tensor ws = at::empty({(int64_t)bytes}, opts.dtype(at::kByte));
+  const int rc = xattn_prefill_fwd(
+      q->data_ptr(), k->data_ptr(), v->data_ptr(), out.data_ptr(), ws.data_ptr(), bytes, (int)H, (int)Hkv, (int)Lq, (int)Lk,
+      128, q->stride(1), q->stride(2), k->stride(1), k->stride(2), v->stride(1), v->stride(2), 128, H * 128, (int)stride,
+      (int)chunk, causal, own_chunk, (float)(1.0 / std::sqrt(128.0) / (double)stride / norm), (int)zero_from,
+      tau.count ? tau.host : nullptr, tau.count, tau.count ? nullptr : tau.device.const_data_ptr<double>(), keep_sink,
+      keep_recent, (float)(1.0 / std::sqrt(128.0)), stream_of(dev));
+  if (rc != XATTN_OK) return fail("xattn_prefill_fwd", rc);
+  return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef methods[] = {
+    {"prefill", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(prefill)), METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "xattn_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_xattn_host(void) { return PyModule_Create(&module_def); }

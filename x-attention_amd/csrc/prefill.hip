@@ -1,0 +1,77 @@
+// The prefill operator as one call: antidiagonal estimate, block selection and
+// block-sparse attention enqueued back to back on one stream (what
+// Xattention_prefill, xattn/src/Xattention.py:302-402, runs for a sequence
+// whose temporaries fit one launch per stage).
+//
+// A short prompt is bound by what happens around the kernels.  As three calls
+// from Python with a tensor each for the estimator's workspace, the
+// thresholds (a fill kernel of their own), the column lists, the counts and
+// the output, a 1000-token prompt took 75 us of host time for 40-60 us of GPU
+// work.  Here the temporaries share one caller-provided buffer, thresholds that
+// live on the host travel in the kernel arguments, and the rows the padding to
+// chunk_size adds are left out of all three stages.
+#include "estimate.h"
+#include "xattn_hip.h"
+
+using namespace xattn;
+
+namespace {
+struct PrefillLayout {
+  size_t est_bytes, cnt_off, idx_off, total;
+  int nqb, nkb;
+};
+
+size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
+
+// false if the estimator refuses the geometry
+bool prefill_layout(int num_heads, int q_len, int k_len, int stride, int chunk_size, PrefillLayout* l) {
+  l->est_bytes = estimate_real_rows_bytes(num_heads, q_len, k_len, stride, 128, chunk_size);
+  if (l->est_bytes == 0) return false;
+  l->nqb = (q_len + 127) / 128;
+  l->nkb = (k_len + 127) / 128;
+  l->cnt_off = up256(l->est_bytes);
+  l->idx_off = l->cnt_off + up256((size_t)num_heads * l->nqb * sizeof(int32_t));
+  l->total = l->idx_off + up256((size_t)num_heads * l->nqb * l->nkb * sizeof(int32_t));
+  return true;
+}
+}  // namespace
+
+extern "C" size_t xattn_prefill_workspace_bytes(int num_heads, int q_len, int k_len, int stride, int chunk_size) {
+  PrefillLayout l;
+  return prefill_layout(num_heads, q_len, k_len, stride, chunk_size, &l) ? l.total : 0;
+}
+
+extern "C" int xattn_prefill_fwd(const void* q, const void* k, const void* v, void* out, void* workspace,
+                                 size_t workspace_bytes, int num_heads, int num_kv_heads, int q_len, int k_len,
+                                 int head_dim, int64_t q_stride_h, int64_t q_stride_n, int64_t k_stride_h,
+                                 int64_t k_stride_n, int64_t v_stride_h, int64_t v_stride_n, int64_t o_stride_h,
+                                 int64_t o_stride_n, int stride, int chunk_size, int causal, int own_chunk_only,
+                                 float estimate_scale, int zero_rows_from, const double* tau_host, int tau_host_count,
+                                 const double* tau_device, int keep_sink, int keep_recent, float softmax_scale,
+                                 void* stream) {
+  if (!workspace || !v || !out) return XATTN_ERR_NULL;
+  PrefillLayout l;
+  if (!prefill_layout(num_heads, q_len, k_len, stride, chunk_size, &l)) return XATTN_ERR_SHAPE;
+  if (workspace_bytes < l.total) return XATTN_ERR_WORKSPACE;
+  if (reinterpret_cast<uintptr_t>(workspace) & 15) return XATTN_ERR_ALIGN;
+  char* ws = static_cast<char*>(workspace);
+  SelectArgs sel{};
+  sel.tau = tau_device;
+  sel.tau_host = tau_host;
+  sel.tau_host_count = tau_host_count;
+  sel.col_cnt = reinterpret_cast<int32_t*>(ws + l.cnt_off);
+  sel.col_idx = reinterpret_cast<int32_t*>(ws + l.idx_off);
+  sel.idx_pitch = l.nkb;
+  sel.keep_sink = keep_sink;
+  sel.keep_recent = keep_recent;
+  sel.real_q_blocks_only = 1;
+  sel.stages = 3;
+  const int q_chunks = (int)(((int64_t)q_len + chunk_size - 1) / chunk_size);
+  int rc = estimate_impl(q, k, nullptr, ws, l.est_bytes, nullptr, num_heads, num_kv_heads, q_len, k_len, head_dim,
+                         q_stride_h, q_stride_n, k_stride_h, k_stride_n, stride, 128, chunk_size, 0, q_chunks, causal,
+                         own_chunk_only, estimate_scale, nullptr, 0, 1, 1, zero_rows_from, 0, l.nqb, stream, &sel);
+  if (rc != XATTN_OK) return rc;
+  return xattn_block_sparse_fwd(q, k, v, out, sel.col_idx, sel.col_cnt, l.nkb, l.nqb, 0, num_heads, num_kv_heads, q_len,
+                                k_len, head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n,
+                                o_stride_h, o_stride_n, 0, l.nqb, causal, softmax_scale, stream);
+}

@@ -5,9 +5,13 @@
 
 namespace xattn {
 
+constexpr int kMaxTauHost = 64;   // per-head thresholds that fit the kernel arguments
+
 struct SelParams {
   const float* sums;
-  const double* tau;
+  const double* tau;               // per head on the device, or null: tau_val[head * tau_step]
+  double tau_val[kMaxTauHost];
+  int tau_step;
   uint8_t* mask;
   int32_t* col_idx;
   int32_t* col_cnt;
@@ -117,7 +121,7 @@ __device__ __forceinline__ void select_row(const SelParams& p, const float* x, i
   }
   for (int c = lane; c < p.nkb; c += 64) flags[c] = 0;
   total = wave_sum(total);
-  const double required = total * p.tau[head];
+  const double required = total * (p.tau ? p.tau[head] : p.tau_val[head * p.tau_step]);
   const int n_forced = one_forced ? 1 : 2;
   // forced keys ranked ahead of an ordinary block of sum v (all of them unless v is beyond 100000)
   auto forced_ahead = [&](double v) -> int {

@@ -478,6 +478,12 @@ def Xattention_prefill(
     if pipeline_chunks:
         return _prefill_pipelined(query_states, key_states, value_states, stride, norm, threshold, block_size,
                                   use_triton, causal, chunk_size, keep_sink, keep_recent, kdb)
+    if kdb == 1:
+        # the ordinary call: temporaries of one launch per stage fit, tensors are as the kernels read them
+        out = _hb.host().prefill(query_states, key_states, value_states, stride, norm, threshold, use_triton, causal,
+                                 chunk_size, keep_sink, keep_recent, min(WORKSPACE_LIMIT, GROUP_LIMIT))
+        if out is not None:
+            return out
     # One launch per stage when the block sums and column lists of the whole sequence fit GROUP_LIMIT
     # (128k tokens: 0.26 GB); longer sequences go through the three stages one group of query chunks at a
     # time on buffers of one group, so the extra memory stays bounded however long the sequence is.
