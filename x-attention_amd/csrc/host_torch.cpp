@@ -10,6 +10,7 @@
 
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
@@ -136,8 +137,48 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// decode(q, k, v, token_major, sm_scale): single_decode_with_kv_cache without caller-provided buffers
+PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 5) return PyErr_Format(PyExc_TypeError, "decode takes 5 arguments");
+  HANDLE_TH_ERRORS
+  const at::Tensor *q = tensor_of(args[0]), *k = tensor_of(args[1]), *v = tensor_of(args[2]);
+  if (!q || !k || !v) Py_RETURN_NONE;
+  const int nhd = PyObject_IsTrue(args[3]);
+  double scale = 1.0 / std::sqrt(128.0);
+  if (args[4] != Py_None) scale = PyFloat_AsDouble(args[4]);
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  if (!q->is_cuda() || q->scalar_type() != at::kBFloat16 || q->dim() != 2 || q->size(1) != 128 || q->stride(1) != 1 ||
+      q->stride(0) % 8 || (reinterpret_cast<uintptr_t>(q->data_ptr()) & 15))
+    Py_RETURN_NONE;
+  if (!kernel_ready(*k, 3) || !kernel_ready(*v, 3) || k->sizes() != v->sizes()) Py_RETURN_NONE;
+  const c10::Device dev = q->device();
+  if (k->device() != dev || v->device() != dev) Py_RETURN_NONE;
+  const int hd = nhd ? 1 : 0, td = 1 - hd;       // head and token dimension of k and v
+  const int64_t H = q->size(0), Hkv = k->size(hd), L = k->size(td);
+  if (H < 1 || Hkv < 1 || H % Hkv || H / Hkv > 32 || L < 1 || L > (int64_t(1) << 30)) Py_RETURN_NONE;
+  const size_t bytes = xattn_decode_workspace_bytes((int)H, (int)Hkv, (int)L);
+  if (bytes == 0) Py_RETURN_NONE;
+  OnDevice on(dev);
+  at::Tensor out = at::empty({H, 128}, at::TensorOptions().device(dev).dtype(at::kBFloat16));
+  const c10::DataPtr ws = c10::hip::HIPCachingAllocator::get()->allocate(bytes);
+  const int rc = xattn_decode_fwd(q->data_ptr(), k->data_ptr(), v->data_ptr(), out.data_ptr(), ws.get(), bytes, (int)H, (int)Hkv,
+                                  (int)L, 128, q->stride(0), k->stride(hd), k->stride(td), v->stride(hd), v->stride(td), 128,
+                                  (float)scale, stream_of(dev));
+  if (rc != XATTN_OK) return fail("xattn_decode_fwd", rc);
+  return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
+template <PyObject* (*F)(PyObject*, PyObject* const*, Py_ssize_t)>
+PyMethodDef method(const char* name) {
+  return {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(F)), METH_FASTCALL, nullptr};
+}
 PyMethodDef methods[] = {
-    {"prefill", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(prefill)), METH_FASTCALL, nullptr},
+    method<prefill>("prefill"),
+    method<decode>("decode"),
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "xattn_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -31,6 +31,11 @@ def single_decode_with_kv_cache(q, k, v, kv_layout="NHD", sm_scale=None, out=Non
     library, shared by every such call on the GPU - calls that may overlap on
     one GPU must then be ordered by the caller.
     """
+    if out is None and workspace is None and not static_scratch and kv_layout in ("HND", "NHD"):
+        # the ordinary call: tensors are as the kernels read them
+        res = _hb.host().decode(q, k, v, kv_layout == "NHD", sm_scale)
+        if res is not None:
+            return res
     lib = _hb.lib()
     if kv_layout not in ("NHD", "HND"):
         raise KeyError(f"Invalid kv_layout {kv_layout}")
