@@ -280,6 +280,32 @@ int xattn_decode_fwd_static(const void* q, const void* k, const void* v, void* o
                             int64_t o_stride_h, float softmax_scale, void* stream);
 
 /* ---------------------------------------------------------------------------
+ * Projections and rotary embedding of the Llama attention forward
+ * (xattn/src/load_llama.py:119-150, 207-218).  bf16 throughout, fp32 sums,
+ * rounded to bf16 where the reference's tensor expressions round.  These
+ * tensors are dense: no head or token strides beside the ones named.
+ *
+ * xattn_qkv_rope_gemv: ONE token.  x [width]; wq [num_heads*128][width], wk and
+ * wv [num_kv_heads*128][width] with row strides in elements (multiples of 8);
+ * biases null or one per row; cos, sin [128].  q [num_heads][128] and
+ * k [num_kv_heads][128] come out rotated, v [num_kv_heads][128] as projected.
+ * xattn_gemv: y[rows] = w x (+ bias) for one token, rows a multiple of 4.
+ * width: a multiple of 8, at most 2^24.
+ * xattn_rope: rotates q [tokens][num_heads][128] and k [tokens][num_kv_heads][128]
+ * in place; cos and sin [tokens][128] with a token stride.
+ */
+int xattn_qkv_rope_gemv(const void* x, int width, const void* wq, int64_t wq_stride, const void* bq, const void* wk,
+                        int64_t wk_stride, const void* bk, const void* wv, int64_t wv_stride, const void* bv,
+                        const void* cos, const void* sin, void* q, void* k, void* v, int num_heads,
+                        int num_kv_heads, int head_dim, void* stream);
+
+int xattn_gemv(const void* x, int width, const void* w, int64_t w_stride, const void* bias, void* y, int rows,
+               void* stream);
+
+int xattn_rope(void* q, void* k, const void* cos, const void* sin, int64_t cos_stride, int64_t sin_stride, int tokens,
+               int num_heads, int num_kv_heads, int head_dim, void* stream);
+
+/* ---------------------------------------------------------------------------
  * Stand-alone softmax + block sums over a score matrix in memory: the seam
  * softmax_fuse_block_sum, xattn/src/kernels.py:238-289 (kernels :5-156), for
  * callers that hold the strided scores themselves (the fused estimator above

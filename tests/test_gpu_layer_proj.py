@@ -1,0 +1,61 @@
+"""GPU: the projection and rotation kernels of the attention layer (through the native host path) against the torch
+expressions they stand for."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _reference(x, weights, biases, heads, cos, sin):
+    """q, k, v as the reference's layer computes them, the products in fp32 and rounded once."""
+    from xattn.src.load_llama import apply_rotary_pos_emb
+
+    out = []
+    for w, b, n in zip(weights, biases, heads):
+        y = x.float() @ w.float().t() + (b.float() if b is not None else 0.0)
+        out.append(y.bfloat16().view(1, x.shape[1], n, 128).transpose(1, 2))
+    out[0], out[1] = apply_rotary_pos_emb(out[0], out[1], cos, sin)
+    return out
+
+
+# widths around the loads of a row: less than one chunk of 512, chunk and batch (2048) edges, an odd number of batches
+@pytest.mark.parametrize("width", [8, 504, 512, 520, 2048, 2056, 6144])
+@pytest.mark.parametrize("tokens,heads,kv_heads,bias", [(1, 4, 1, True), (1, 6, 6, False), (2, 4, 2, True), (77, 3, 1, False)])
+def test_projection_and_rotation(width, tokens, heads, kv_heads, bias):
+    from xattn.src import hip_backend as hb
+
+    g = torch.Generator(device="cuda").manual_seed(width + tokens)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    n = (heads, kv_heads, kv_heads)
+    weights = [(rnd(h * 128, width) / width ** 0.5).bfloat16() for h in n]
+    biases = [rnd(h * 128).bfloat16() if bias else None for h in n]
+    x = rnd(1, tokens, width).bfloat16()
+    ang = rnd(1, tokens, 128) * 3
+    cos, sin = ang.cos().bfloat16(), ang.sin().bfloat16()
+    with torch.no_grad():
+        got = hb.host().project(x, weights[0], biases[0], weights[1], biases[1], weights[2], biases[2], cos, sin, heads, kv_heads)
+        want = _reference(x, weights, biases, n, cos, sin)
+        # fp32 sums in another order: a result next to a rounding boundary may land one bf16 step (2^-8 of its
+        # magnitude) away; the rotation adds two such values and rounds once more
+        for a, b in zip(got, want):
+            assert a.shape == b.shape
+            assert ((a.float() - b.float()).abs() <= 3 * 2.0 ** -8 * (b.float().abs() + 1)).all()
+            assert (a != b).float().mean() < 0.02
+        if tokens == 1:
+            y = hb.host().output(x, weights[0], biases[0])
+            ref = (x.float() @ weights[0].float().t() + (biases[0].float() if bias else 0.0)).bfloat16()
+            assert ((y.float() - ref.float()).abs() <= 2.0 ** -8 * (ref.float().abs() + 1)).all()
+
+
+def test_modules_that_are_more_than_a_linear_are_called():
+    """A hook or a replaced forward on a projection means that the module itself runs."""
+    from xattn.src.load_llama import _linear_params
+
+    lin = torch.nn.Linear(512, 512, bias=False)
+    assert _linear_params(lin) is not None
+    handle = lin.register_forward_hook(lambda *a: None)
+    assert _linear_params(lin) is None
+    handle.remove()
+    lin.forward = lambda x: x
+    assert _linear_params(lin) is None
+    assert _linear_params(torch.nn.Identity()) is None

@@ -9,6 +9,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPFunctions.h>
@@ -172,6 +173,103 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// A weight and bias (or None) as the projection kernels read them, on device dev.
+struct Linear {
+  const at::Tensor* w = nullptr;
+  std::optional<at::Tensor> b;
+  bool read(PyObject* weight, PyObject* bias, int64_t rows, int64_t width, c10::Device dev) {
+    w = tensor_of(weight);
+    if (!w || w->dim() != 2 || w->size(0) != rows || w->size(1) != width || w->stride(1) != 1 || w->stride(0) % 8 ||
+        w->stride(0) < width || w->scalar_type() != at::kBFloat16 || w->device() != dev ||
+        (reinterpret_cast<uintptr_t>(w->data_ptr()) & 15))
+      return false;
+    if (bias != Py_None) {
+      const at::Tensor* t = tensor_of(bias);
+      if (!t || t->dim() != 1 || t->size(0) != rows || t->stride(0) != 1 || t->scalar_type() != at::kBFloat16 || t->device() != dev)
+        return false;
+      b = *t;
+    }
+    return !at::GradMode::is_enabled() || (!w->requires_grad() && !(b && b->requires_grad()));
+  }
+  const void* bias_ptr() const { return b ? b->data_ptr() : nullptr; }
+};
+
+// Hidden states a layer's projections take natively: bf16 [1, tokens, width] without gaps, no autograd, no autocast.
+const at::Tensor* hidden_of(PyObject* o) {
+  const at::Tensor* x = tensor_of(o);
+  if (!x || !x->is_cuda() || x->scalar_type() != at::kBFloat16 || x->dim() != 3 || x->size(0) != 1 || x->size(1) < 1 ||
+      !x->is_contiguous() || x->size(2) % 8 || (reinterpret_cast<uintptr_t>(x->data_ptr()) & 15) ||
+      (at::GradMode::is_enabled() && x->requires_grad()) || at::autocast::is_autocast_enabled(at::kCUDA))
+    return nullptr;
+  return x;
+}
+
+// project(hidden, wq, bq, wk, bk, wv, bv, cos, sin, heads, kv_heads) -> (q, k, v): the projections of a layer with q and
+// k rotated, [1, heads, tokens, 128] views of token-major memory (what the projections write)
+PyObject* project(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 11) return PyErr_Format(PyExc_TypeError, "project takes 11 arguments");
+  HANDLE_TH_ERRORS
+  const at::Tensor *x = hidden_of(args[0]), *cos = tensor_of(args[7]), *sin = tensor_of(args[8]);
+  if (!x || !cos || !sin) Py_RETURN_NONE;
+  const long heads[3] = {PyLong_AsLong(args[9]), PyLong_AsLong(args[10]), PyLong_AsLong(args[10])};
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  const c10::Device dev = x->device();
+  const int64_t L = x->size(1), K = x->size(2);
+  if (heads[0] < 1 || heads[1] < 1 || heads[0] > 4096 || heads[1] > 4096 || L * (heads[0] + heads[1]) > 0x7fffffff) Py_RETURN_NONE;
+  for (const at::Tensor* t : {cos, sin})
+    if (t->dim() != 3 || t->size(0) != 1 || t->size(1) != L || t->size(2) != 128 || t->stride(2) != 1 || t->stride(1) % 8 ||
+        t->scalar_type() != at::kBFloat16 || t->device() != dev || (reinterpret_cast<uintptr_t>(t->data_ptr()) & 15))
+      Py_RETURN_NONE;
+  Linear lin[3];
+  for (int i = 0; i < 3; ++i)
+    if (!lin[i].read(args[1 + 2 * i], args[2 + 2 * i], heads[i] * 128, K, dev)) Py_RETURN_NONE;
+  OnDevice on(dev);
+  at::Tensor y[3];
+  int rc;
+  if (L == 1) {
+    const auto opts = at::TensorOptions().device(dev).dtype(at::kBFloat16);
+    for (int i = 0; i < 3; ++i) y[i] = at::empty_strided({1, heads[i], 1, 128}, {heads[i] * 128, 128, heads[i] * 128, 1}, opts);
+    rc = xattn_qkv_rope_gemv(x->data_ptr(), (int)K, lin[0].w->data_ptr(), lin[0].w->stride(0), lin[0].bias_ptr(),
+                             lin[1].w->data_ptr(), lin[1].w->stride(0), lin[1].bias_ptr(), lin[2].w->data_ptr(),
+                             lin[2].w->stride(0), lin[2].bias_ptr(), cos->data_ptr(), sin->data_ptr(), y[0].data_ptr(),
+                             y[1].data_ptr(), y[2].data_ptr(), (int)heads[0], (int)heads[1], 128, stream_of(dev));
+  } else {
+    for (int i = 0; i < 3; ++i) y[i] = at::linear(*x, *lin[i].w, lin[i].b);
+    rc = xattn_rope(y[0].data_ptr(), y[1].data_ptr(), cos->data_ptr(), sin->data_ptr(), cos->stride(1), sin->stride(1), (int)L,
+                    (int)heads[0], (int)heads[1], 128, stream_of(dev));
+    for (int i = 0; i < 3; ++i)
+      y[i] = y[i].as_strided({1, heads[i], L, 128}, {L * heads[i] * 128, 128, heads[i] * 128, 1});
+  }
+  if (rc != XATTN_OK) return fail(L == 1 ? "xattn_qkv_rope_gemv" : "xattn_rope", rc);
+  PyObject* result = PyTuple_New(3);
+  if (!result) return nullptr;
+  for (int i = 0; i < 3; ++i) PyTuple_SET_ITEM(result, i, THPVariable_Wrap(std::move(y[i])));
+  return result;
+  END_HANDLE_TH_ERRORS
+}
+
+// output(hidden, w, b): the output projection of one token
+PyObject* output(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 3) return PyErr_Format(PyExc_TypeError, "output takes 3 arguments");
+  HANDLE_TH_ERRORS
+  const at::Tensor *x = hidden_of(args[0]), *w = tensor_of(args[1]);
+  if (!x || x->size(1) != 1 || !w || w->dim() != 2 || w->size(0) % 4) Py_RETURN_NONE;
+  const c10::Device dev = x->device();
+  const int64_t N = w->size(0), K = x->size(2);
+  Linear lin;
+  if (N < 4 || N > 0x7fffffff || !lin.read(args[1], args[2], N, K, dev)) Py_RETURN_NONE;
+  OnDevice on(dev);
+  at::Tensor y = at::empty({1, 1, N}, at::TensorOptions().device(dev).dtype(at::kBFloat16));
+  const int rc = xattn_gemv(x->data_ptr(), (int)K, lin.w->data_ptr(), lin.w->stride(0), lin.bias_ptr(), y.data_ptr(), (int)N,
+                            stream_of(dev));
+  if (rc != XATTN_OK) return fail("xattn_gemv", rc);
+  return THPVariable_Wrap(std::move(y));
+  END_HANDLE_TH_ERRORS
+}
+
 template <PyObject* (*F)(PyObject*, PyObject* const*, Py_ssize_t)>
 PyMethodDef method(const char* name) {
   return {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(F)), METH_FASTCALL, nullptr};
@@ -179,6 +277,8 @@ PyMethodDef method(const char* name) {
 PyMethodDef methods[] = {
     method<prefill>("prefill"),
     method<decode>("decode"),
+    method<project>("project"),
+    method<output>("output"),
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "xattn_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

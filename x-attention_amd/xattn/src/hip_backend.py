@@ -56,6 +56,12 @@ _SIGNATURES = {
         c_i32,
         [c_vp] * 4 + [c_i32] * 4 + [c_i64] * 6 + [c_f32, c_vp],
     ),
+    "xattn_qkv_rope_gemv": (
+        c_i32,
+        [c_vp, c_i32] + [c_vp, c_i64, c_vp] * 3 + [c_vp] * 5 + [c_i32] * 3 + [c_vp],
+    ),
+    "xattn_gemv": (c_i32, [c_vp, c_i32, c_vp, c_i64, c_vp, c_vp, c_i32, c_vp]),
+    "xattn_rope": (c_i32, [c_vp] * 4 + [c_i64] * 2 + [c_i32] * 4 + [c_vp]),
     "xattn_block_sparse_fwd": (
         c_i32,
         [c_vp] * 6 + [c_i64] + [c_i32] * 7 + [c_i64] * 8 + [c_i32, c_i32, c_i32, c_f32, c_vp],

@@ -17,10 +17,12 @@ differences that the kernels make possible:
 reference carries for comparison; they are not provided here.
 """
 import inspect
+import sys
 import time
 
 import torch
 
+from . import hip_backend as _hb
 from .decode import single_decode_with_kv_cache
 from .Xattention import Xattention_prefill, block_sparse_attention
 
@@ -86,11 +88,40 @@ class FastPrefillConfig(dict):
 
 
 def _is_static_cache(cache):
+    if "transformers" not in sys.modules:      # then nobody holds one
+        return False
     try:
         from transformers import StaticCache
     except ImportError:
         return False
     return isinstance(cache, StaticCache)
+
+
+_module_hooks = torch.nn.modules.module
+
+
+def _linear_params(mod):
+    """(weight, bias) of a projection that is nothing but ``torch.nn.Linear`` - no hooks, no replaced forward, no
+    wrapped or quantized weight - so that its product may be computed without calling the module; else None."""
+    own = mod.__dict__
+    if (type(mod) is not torch.nn.Linear or "forward" in own or own["_forward_hooks"] or own["_forward_pre_hooks"]
+            or _module_hooks._global_forward_hooks or _module_hooks._global_forward_pre_hooks):
+        return None
+    weight, bias = own["_parameters"].get("weight"), own["_parameters"].get("bias")
+    if type(weight) is not torch.nn.Parameter or (bias is not None and type(bias) is not torch.nn.Parameter):
+        return None
+    return weight, bias
+
+
+def _project(self, hidden_states, cos, sin, heads, kv_heads):
+    """Rotated q and k and v of a layer from the native host path (one kernel for one token, the library GEMMs and one
+    rotation kernel for more), or None where the layer's own modules have to be called."""
+    if not hidden_states.is_cuda or self.head_dim != 128:
+        return None
+    q, k, v = _linear_params(self.q_proj), _linear_params(self.k_proj), _linear_params(self.v_proj)
+    if q is None or k is None or v is None:
+        return None
+    return _hb.host().project(hidden_states, *q, *k, *v, cos, sin, heads, kv_heads)
 
 
 def _stamp(cfg, label, start):
@@ -121,16 +152,21 @@ def forward_eval(self, hidden_states, position_embeddings=None, attention_mask=N
     kv_heads = self.config.num_key_value_heads
     head_dim = self.head_dim
 
-    query_states = self.q_proj(hidden_states).view(bsz, q_len, heads, head_dim).transpose(1, 2)
-    key_states = self.k_proj(hidden_states).view(bsz, q_len, kv_heads, head_dim).transpose(1, 2)
-    value_states = self.v_proj(hidden_states).view(bsz, q_len, kv_heads, head_dim).transpose(1, 2)
-    start = _stamp(cfg, "Reshape", start)
-
-    if position_embeddings is None:
-        cos, sin = self.rotary_emb(value_states, position_ids)
-    else:
+    qkv = None
+    if position_embeddings is not None:
         cos, sin = position_embeddings
-    query_states, key_states = apply_rotary_pos_emb(query_states, key_states, cos, sin)
+        qkv = _project(self, hidden_states, cos, sin, heads, kv_heads)
+    if qkv is not None:
+        query_states, key_states, value_states = qkv
+        start = _stamp(cfg, "Reshape", start)
+    else:
+        query_states = self.q_proj(hidden_states).view(bsz, q_len, heads, head_dim).transpose(1, 2)
+        key_states = self.k_proj(hidden_states).view(bsz, q_len, kv_heads, head_dim).transpose(1, 2)
+        value_states = self.v_proj(hidden_states).view(bsz, q_len, kv_heads, head_dim).transpose(1, 2)
+        start = _stamp(cfg, "Reshape", start)
+        if position_embeddings is None:
+            cos, sin = self.rotary_emb(value_states, position_ids)
+        query_states, key_states = apply_rotary_pos_emb(query_states, key_states, cos, sin)
 
     cache = past_key_values if past_key_values is not None else past_key_value
     if cache is not None:
@@ -165,7 +201,7 @@ def forward_eval(self, hidden_states, position_embeddings=None, attention_mask=N
     if decoding:
         attn_output = single_decode_with_kv_cache(
             query_states[0, :, 0], key_states[0], value_states[0], kv_layout="HND"
-        )[None, :, None, :]
+        ).reshape(1, heads, 1, head_dim)
     elif cfg.metric == "xattn":
         threshold = cfg.layer_threshold(self.layer_idx)
         attn_output = Xattention_prefill(
@@ -180,7 +216,9 @@ def forward_eval(self, hidden_states, position_embeddings=None, attention_mask=N
             f"`attn_output` should be of size {(bsz, heads, q_len, head_dim)}, but is {attn_output.size()}"
         )
     attn_output = attn_output.transpose(1, 2).reshape(bsz, q_len, heads * head_dim)
-    attn_output = self.o_proj(attn_output)
+    out_proj = _linear_params(self.o_proj) if q_len == 1 and attn_output.is_cuda else None
+    projected = _hb.host().output(attn_output, *out_proj) if out_proj is not None else None
+    attn_output = projected if projected is not None else self.o_proj(attn_output)
     _stamp(cfg, "Post-attention processing", start)
     if getattr(self, "_xattn_three_outputs", False):
         return attn_output, None, cache
