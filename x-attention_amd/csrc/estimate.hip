@@ -24,61 +24,18 @@
 #include <mutex>
 
 #include "estimate.h"
+#include "estimate_params.h"
+#include "estimate_small.h"
 #include "select_row.h"
 #include "xattn_hip.h"
 
 namespace xattn {
 
 constexpr int kTile = 256;       // workgroup tile edge (reshaped rows / keys)
-constexpr int kSub = 128;        // keys per wavefront tile (and per softmax tile)
 constexpr int kRowsW = 64;       // reshaped query rows per wavefront tile
 constexpr int kWaves = 8;        // wavefronts per workgroup: 2 key halves x 4 query quarters
 constexpr int kDepth = 64;       // bf16 per k-step (one 128-byte line per row)
 constexpr int kStageBytes = 2 * kTile * kDepth * 2;  // K' + Q' slabs of one stage
-
-struct EstParams {
-  const __bf16* q;
-  const __bf16* k;
-  int64_t q_sh, q_sn, k_sh, k_sn;
-  float* P;        // [H][nkb][rows]  partial block sums relative to the tile maximum
-  float* Mt;       // [H][nT][rows]   tile maximum (exp2 domain)
-  float* Lt;       // [H][nT][rows]   tile sum
-  float* scores;   // optional [H][n_rq][n_rk] raw scores
-  float* sums;     // output block sums: [H][win_rows][nkb], q-block row i stored at row i - win_row0
-  int win_row0, win_rows;
-  int H, Hkv, Lq, Lk, S, rbs;
-  int n_rq, n_rk, nkb, nqb, nT;
-  int rcs;                  // reshaped keys per chunk
-  int kdb;                  // query-row subsampling: query row m stands for reshaped row m * kdb
-  int rcs_q, rbs_q;         // query rows per chunk / per query block (rcs / kdb, rbs / kdb)
-  int row_begin, row_end;   // query rows handled by this call
-  int live_end;             // rows at or past it give zero block sums (padding) or are not asked for: never computed
-  int rows;                 // live_end - row_begin (pitch of P / Mt / Lt)
-  int nT_real;              // 128-key tiles from here on hold padded keys only (nT when causal): not computed either
-  int off;                  // position of reshaped row 0 on the key axis: n_rk - n_rq * kdb
-  int real_rows;            // query rows >= real_rows give all-zero block sums
-  int causal, own_chunk_only;
-  int no_softmax;           // block sums of exp(scaled score) instead of softmax probabilities
-  float scale_log2;
-  // Depth slabs of the reshaped GEMM.  Slab j multiplies query token
-  // m*S + (pairs[j] >> 4) with key token n*S + (pairs[j] & 15); n_pairs = 0 means
-  // the S pairs (S-1-i, i) of the antidiagonal reshape, in closed form.
-  int n_pairs;
-  uint8_t pairs[64];
-  int nMT, nNT;             // tile rows over [row_begin, row_end) / tile columns over n_rk
-  int tiles_per_head;       // tiles with a visible pair, per head
-  int64_t total_tiles;      // tiles_per_head * H
-};
-
-// first / last visible reshaped key of reshaped query row m
-// (with kdb > 1 the row's causal limit is that of the LAST reshaped row of its
-// group, xattn/src/Xattention.py:217-222, while its tokens are those of the first, :88-93)
-__host__ __device__ inline int row_lo(const EstParams& p, int m) {
-  return (p.causal && p.own_chunk_only) ? (m / p.rcs_q) * p.rcs + p.off : 0;
-}
-__host__ __device__ inline int row_hi(const EstParams& p, int m) {
-  return p.causal ? m * p.kdb + p.kdb - 1 + p.off : p.n_rk - 1;
-}
 
 // A k-step slab is 256 rows x 64 bf16 (one 128-byte line per row) per operand.
 // It travels global -> registers -> LDS: each wavefront instruction loads
@@ -781,6 +738,21 @@ __global__ __launch_bounds__(256) void estimate_normalize_rows_kernel(EstParams 
 using namespace xattn;
 
 namespace {
+// Which MFMA pass a launch takes: the smallest predicted time
+//   5 us + steps * max(lat, per_tile * tiles),   steps = 2 * stride
+// of estimate_small_kernel's variants - lat: one step when there are few tiles, per_tile: a tile's share of a step when
+// the chip is full - and for the 256x256 tiles, which 256 workgroups take in turns,
+//   5 us + steps * 1.75 us * ceil(tiles / 256).
+// The constants are fits to measured times of the passes over 200 .. 16384 tokens and chunks of 64 .. 8000 tokens on
+// 8700 .. 100000 cached ones, stride 8 and 16 (us, 256x256 / chosen): 1000 tokens, stride 16: 45.2 / 10.6 (MT 1);
+// 2000, stride 8: 31.1 / 9.8 (MT 2, 3 stages); 4096, stride 8: 35.0 / 19.2; 8192, stride 16: 60.9 / 31.6;
+// 16384, stride 16: 117.9 / 96; 15000, stride 8: 147.5 (stays).
+struct SmallVariant {
+  int mt, ns;
+  float lat, per_tile;
+};
+constexpr SmallVariant kSmall[] = {{1, 4, 0.20f, 0.00106f}, {2, 3, 0.27f, 0.00129f}, {2, 2, 0.35f, 0.00126f}, {4, 2, 0.50f, 0.00238f}};
+
 template <int RBS, bool kDump, bool kTable>
 hipError_t launch_gemm_as(const EstParams& p, dim3 grid, size_t lds, hipStream_t s) {
   auto kernel = &estimate_gemm_kernel<RBS, kDump, kTable>;
@@ -794,6 +766,24 @@ template <int RBS>
 hipError_t launch_gemm(const EstParams& p, dim3 grid, size_t lds, hipStream_t s) {
   if (p.n_pairs) return p.scores ? launch_gemm_as<RBS, true, true>(p, grid, lds, s) : launch_gemm_as<RBS, false, true>(p, grid, lds, s);
   return p.scores ? launch_gemm_as<RBS, true, false>(p, grid, lds, s) : launch_gemm_as<RBS, false, false>(p, grid, lds, s);
+}
+template <int RBS, int MT, int NS>
+hipError_t launch_small_as(const EstParams& p, hipStream_t s) {
+  auto kernel = &estimate_small_kernel<RBS, MT, NS>;
+  static LdsLimit limit;
+  hipError_t e = limit.raise(reinterpret_cast<const void*>(kernel));
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((p.total_tiles + 7) / 8 * 8)), dim3(256), NS * (kSub + 32 * MT) * 128, s, p);
+  return hipSuccess;
+}
+template <int RBS>
+hipError_t launch_small(const EstParams& p, int variant, hipStream_t s) {
+  switch (variant) {
+    case 0: return launch_small_as<RBS, kSmall[0].mt, kSmall[0].ns>(p, s);
+    case 1: return launch_small_as<RBS, kSmall[1].mt, kSmall[1].ns>(p, s);
+    case 2: return launch_small_as<RBS, kSmall[2].mt, kSmall[2].ns>(p, s);
+    default: return launch_small_as<RBS, kSmall[3].mt, kSmall[3].ns>(p, s);
+  }
 }
 template <int RBS>
 hipError_t launch_select(const EstParams& p, const SelParams& sp, int qb_per_wg, dim3 grid, size_t lds, hipStream_t s) {
@@ -959,18 +949,45 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
   p.Lt = p.Mt + (size_t)num_heads * g.nT * p.rows;
 
   hipStream_t s = static_cast<hipStream_t>(stream);
+  // tiles holding a visible pair, per head: same visibility rule as the kernels' row_lo / row_hi
+  auto tiles_of = [&](int tile_rows, int tile_keys, int key_tiles) {
+    int n = 0;
+    for (int mfirst = p.row_begin; mfirst < p.live_end; mfirst += tile_rows) {
+      const int mlast = (mfirst + tile_rows < p.live_end ? mfirst + tile_rows : p.live_end) - 1;
+      int hi = row_hi(p, mlast) / tile_keys;
+      hi = hi < key_tiles - 1 ? hi : key_tiles - 1;
+      n += hi - row_lo(p, mfirst) / tile_keys + 1;
+    }
+    return n;
+  };
   p.nMT = (p.rows + kTile - 1) / kTile;
   p.nNT = ((p.nT_real < g.nT ? p.nT_real * kSub : g.n_rk) + kTile - 1) / kTile;
-  p.tiles_per_head = 0;
-  for (int r = 0; r < p.nMT; ++r) {   // same visibility rule as the kernel's row_lo / row_hi
-    const int mfirst = p.row_begin + r * kTile;
-    const int mlast = (mfirst + kTile - 1 < p.live_end ? mfirst + kTile - 1 : p.live_end - 1);
-    int hi = row_hi(p, mlast) / kTile;
-    hi = hi < p.nNT - 1 ? hi : p.nNT - 1;
-    const int lo = row_lo(p, mfirst) / kTile;
-    p.tiles_per_head += hi - lo + 1;
-  }
+  p.tiles_per_head = tiles_of(kTile, kTile, p.nNT);
   p.total_tiles = (int64_t)p.tiles_per_head * num_heads;
+  int variant = -1;
+  if (kdb == 1 && num_slab_pairs == 0 && !scores_out && p.total_tiles > 0 && p.total_tiles <= 4096) {
+    const int group = num_heads / num_kv_heads;
+    EstParams best = p;
+    float best_t = 1.75f * (float)((p.total_tiles + 255) / 256);
+    for (int i = 0; i < 4; ++i) {
+      EstParams c = p;
+      const int rows = 32 * kSmall[i].mt;
+      // heads whose rows fit a tile together (one buffer resource spans them: < 2^31 bytes)
+      for (c.pack = 1; c.pack < group && p.rows * c.pack * 2 <= rows && c.pack * 2 * q_stride_h < 0x20000000;) c.pack *= 2;
+      c.tile_rows = rows / c.pack;
+      c.tile_shift = __builtin_ctz(c.tile_rows);
+      c.nNT = p.nT_real;
+      c.tiles_per_head = tiles_of(c.tile_rows, kSub, c.nNT);
+      c.total_tiles = (int64_t)c.tiles_per_head * num_kv_heads * ((group + c.pack - 1) / c.pack);
+      const float t = fmaxf(kSmall[i].lat, kSmall[i].per_tile * (float)c.total_tiles);
+      if (t < best_t) {
+        best_t = t;
+        best = c;
+        variant = i;
+      }
+    }
+    p = best;
+  }
   const int64_t ids = (p.total_tiles + 255) / 256 * 256;
   if (ids > 0x7fffffff) return XATTN_ERR_SHAPE;
   // one workgroup per CU (its LDS stages fill a CU), each working through tile ids b, b + grid, ...
@@ -1030,15 +1047,15 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
   hipError_t e = hipSuccess;
   switch (p.rbs) {
     case 8:
-      if (run_gemm && p.total_tiles > 0) e = launch_gemm<8>(p, grid1, lds, s);
+      if (run_gemm && p.total_tiles > 0) e = variant >= 0 ? launch_small<8>(p, variant, s) : launch_gemm<8>(p, grid1, lds, s);
       if (e == hipSuccess && run_rest) e = launch_rest(std::integral_constant<int, 8>());
       break;
     case 16:
-      if (run_gemm && p.total_tiles > 0) e = launch_gemm<16>(p, grid1, lds, s);
+      if (run_gemm && p.total_tiles > 0) e = variant >= 0 ? launch_small<16>(p, variant, s) : launch_gemm<16>(p, grid1, lds, s);
       if (e == hipSuccess && run_rest) e = launch_rest(std::integral_constant<int, 16>());
       break;
     default:
-      if (run_gemm && p.total_tiles > 0) e = launch_gemm<32>(p, grid1, lds, s);
+      if (run_gemm && p.total_tiles > 0) e = variant >= 0 ? launch_small<32>(p, variant, s) : launch_gemm<32>(p, grid1, lds, s);
       if (e == hipSuccess && run_rest) e = launch_rest(std::integral_constant<int, 32>());
       break;
   }

@@ -1,0 +1,55 @@
+// What the estimator's kernels share: the launch parameters and the visibility rule of a reshaped query row.
+#pragma once
+#include "xattn_common.h"
+
+namespace xattn {
+
+constexpr int kSub = 128;        // keys of a softmax tile: what one (maximum, sum) pair covers
+
+struct EstParams {
+  const __bf16* q;
+  const __bf16* k;
+  int64_t q_sh, q_sn, k_sh, k_sn;
+  float* P;        // [H][nkb][rows]  partial block sums relative to the tile maximum
+  float* Mt;       // [H][nT][rows]   tile maximum (exp2 domain)
+  float* Lt;       // [H][nT][rows]   tile sum
+  float* scores;   // optional [H][n_rq][n_rk] raw scores
+  float* sums;     // output block sums: [H][win_rows][nkb], q-block row i stored at row i - win_row0
+  int win_row0, win_rows;
+  int H, Hkv, Lq, Lk, S, rbs;
+  int n_rq, n_rk, nkb, nqb, nT;
+  int rcs;                  // reshaped keys per chunk
+  int kdb;                  // query-row subsampling: query row m stands for reshaped row m * kdb
+  int rcs_q, rbs_q;         // query rows per chunk / per query block (rcs / kdb, rbs / kdb)
+  int row_begin, row_end;   // query rows handled by this call
+  int live_end;             // rows at or past it give zero block sums (padding) or are not asked for: never computed
+  int rows;                 // live_end - row_begin (pitch of P / Mt / Lt)
+  int nT_real;              // 128-key tiles from here on hold padded keys only (nT when causal): not computed either
+  int off;                  // position of reshaped row 0 on the key axis: n_rk - n_rq * kdb
+  int real_rows;            // query rows >= real_rows give all-zero block sums
+  int causal, own_chunk_only;
+  int no_softmax;           // block sums of exp(scaled score) instead of softmax probabilities
+  float scale_log2;
+  // Depth slabs of the reshaped GEMM.  Slab j multiplies query token
+  // m*S + (pairs[j] >> 4) with key token n*S + (pairs[j] & 15); n_pairs = 0 means
+  // the S pairs (S-1-i, i) of the antidiagonal reshape, in closed form.
+  int n_pairs;
+  uint8_t pairs[64];
+  int nMT, nNT;             // tile rows over [row_begin, row_end) / tile columns over n_rk
+  int tiles_per_head;       // tiles with a visible pair, per head
+  int64_t total_tiles;      // tiles_per_head * H
+  // estimate_small_kernel: a tile's rows are tile_rows rows of each of pack heads of one KV group
+  int pack, tile_rows, tile_shift;   // powers of two, tile_rows = 1 << tile_shift
+};
+
+// first / last visible reshaped key of reshaped query row m
+// (with kdb > 1 the row's causal limit is that of the LAST reshaped row of its
+// group, xattn/src/Xattention.py:217-222, while its tokens are those of the first, :88-93)
+__host__ __device__ inline int row_lo(const EstParams& p, int m) {
+  return (p.causal && p.own_chunk_only) ? (m / p.rcs_q) * p.rcs + p.off : 0;
+}
+__host__ __device__ inline int row_hi(const EstParams& p, int m) {
+  return p.causal ? m * p.kdb + p.kdb - 1 + p.off : p.n_rk - 1;
+}
+
+}  // namespace xattn

@@ -1,0 +1,245 @@
+// The estimator's MFMA pass for launches that leave the 256x256 tiles of estimate_gemm_kernel mostly empty: short
+// prompts, and chunks of a few hundred tokens on top of a long cache.  Same scores, same partial results, to the bit.
+//
+// A workgroup of four wavefronts takes 128 keys (one softmax tile) x 32 * MT query rows; wavefront w computes the scores
+// of keys 32w .. 32w+31 against all rows.  Where a head has fewer rows than that, the rows of several heads of the KV
+// group share a tile (`pack`), so that every key is read once per group.  64-deep slabs of both operands go straight to
+// a ring of NS LDS stages (buffer loads that write LDS), NS - 1 steps ahead of their use, one barrier per step.
+//
+// Bound: with at most a tile per CU the time is the chain of 2 * stride steps - 0.17 to 0.25 us each, the barrier and the
+// dependent MFMAs of a step, against 1.1 us of a 256x256 step.  With more tiles per CU two or three workgroups share it
+// and the copies into LDS (about 50 bytes per clock and CU) and the fragment reads (1 + MT per MT MFMAs) are the limit:
+// 0.7 (MT 2) and 0.8 (MT 4) of the flop rate of the large tiles.  More stages help only while a CU has one workgroup;
+// beyond that a third workgroup is worth more than a third stage.
+#pragma once
+#include "estimate_params.h"
+
+namespace xattn {
+
+typedef __attribute__((address_space(3))) char* lds_char_ptr;
+
+// one KiB of a slab (8 rows of 128 bytes), global -> LDS; the caller counts it in vmcnt
+__device__ __forceinline__ void slab_copy_1k(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t dst) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(dst), "v"(voff), "s"(rsrc) : "memory", "m0");
+}
+
+template <int RBS, int MT, int NS>
+__global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p) {
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  constexpr int kKeys = kSub, kRows = 32 * MT;
+  constexpr int kStage = (kKeys + kRows) * 128;     // bytes of one 64-deep step
+  constexpr int kLoads = 4 + MT;                    // KiB a wavefront copies per step
+  constexpr int kPer = (kLoads + 2) / 3;            // ... and in each of the step's first three sub-steps
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 31, hh = lane >> 5;
+
+  // Tile of this workgroup.  Ids are dealt round-robin to the 8 XCDs; an XCD gets one contiguous run of tiles, ordered by
+  // KV group, query-tile row, key tile, head set, so that it works on few KV heads and the sets share a key tile.
+  const uint32_t G = (uint32_t)(p.H / p.Hkv), sets = (G + p.pack - 1) / (uint32_t)p.pack;
+  const uint32_t per_group = (uint32_t)p.tiles_per_head * sets, total = per_group * (uint32_t)p.Hkv;
+  const uint32_t per_xcd = (total + 7) / 8;
+  const uint32_t lin = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (lin >= total) return;
+  const uint32_t g = lin / per_group, rem = lin - g * per_group;
+  const uint32_t set = rem % sets;
+  int tt = (int)(rem / sets), m0 = p.row_begin, n0 = 0, hi_tile = 0;
+  for (;; m0 += p.tile_rows) {
+    const int mlast = m0 + p.tile_rows - 1 < p.live_end ? m0 + p.tile_rows - 1 : p.live_end - 1;
+    hi_tile = row_hi(p, mlast);
+    int last = hi_tile / kSub;
+    last = last < p.nNT - 1 ? last : p.nNT - 1;
+    const int first = row_lo(p, m0) / kSub;
+    const int cnt = last - first + 1;
+    if (tt < cnt || m0 + p.tile_rows >= p.live_end) {
+      n0 = (first + tt) * kSub;
+      break;
+    }
+    tt -= cnt;
+  }
+  const int h0 = (int)(g * G + set * (uint32_t)p.pack);
+  const int h_end = (int)((g + 1) * G);
+
+  // operands: K' slab rows 32w..32w+31 are copied by the wavefront that multiplies them, and not at all when none of
+  // its keys is visible; tokens past the real length read as zeros
+  const int64_t k_snb = p.k_sn * 2, q_snb = p.q_sn * 2;
+  const int n_w = n0 + wave * 32;                   // first key of this wavefront
+  const bool live_w = n_w <= hi_tile && n_w < p.n_rk;
+  const int64_t tok0 = (int64_t)n0 * p.S, left = p.Lk - tok0, span = (int64_t)kKeys * p.S;
+  const int64_t krows = left < 0 || !live_w ? 0 : (left < span ? left : span);
+  const __amdgpu_buffer_rsrc_t kres = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(p.k + (int64_t)g * p.k_sh + (krows > 0 ? tok0 * p.k_sn : 0)), 0, (int)(krows * k_snb), 0x00020000);
+  const __amdgpu_buffer_rsrc_t qres = __builtin_amdgcn_make_buffer_rsrc((void*)(p.q + (int64_t)h0 * p.q_sh + (int64_t)m0 * p.S * p.q_sn), 0, 0x7fffffff, 0x00020000);
+  // slab row of a lane: instruction i of K' covers rows 32w + 8i + lane / 8, of Q' rows 8 (w MT + i) + lane / 8; 16-byte
+  // chunk c of row r sits at c ^ ((r >> 1) & 7) (conflict-free fragment reads)
+  const int rl = lane >> 3, c = lane & 7;
+  uint32_t voffK[4], voffQ[MT];
+  int qtok[MT];                                     // token of the row at reshape offset 0; past the end: never valid
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = wave * 32 + i * 8 + rl;
+    voffK[i] = (uint32_t)((int64_t)row * p.S * k_snb) + (uint32_t)((c ^ ((row >> 1) & 7)) << 4);
+  }
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int row = (wave * MT + i) * 8 + rl;
+    const int hs = row >> p.tile_shift, m = m0 + (row & (p.tile_rows - 1));
+    const bool ok = m < p.live_end && h0 + hs < h_end;
+    qtok[i] = ok ? m * p.S : 0x40000000;
+    voffQ[i] = (uint32_t)((int64_t)hs * p.q_sh * 2 + (int64_t)(m - m0) * p.S * q_snb) + (uint32_t)((c ^ ((row >> 1) & 7)) << 4);
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_char_ptr)lds;
+  const int steps = p.S * 2;
+  // Piece j of step t: 0 .. 3 are K' (not copied by a wavefront whose keys nobody sees), then Q'.  Past the last step a
+  // copy moves nothing (its offset is outside the resource) but keeps the count of loads in flight.
+  auto copy_piece = [&](int t, int j) __attribute__((always_inline)) {
+    const int i = t >> 1;
+    const uint32_t st = lds0 + (uint32_t)(t % NS) * kStage;
+    if (j < 4) {
+      const uint32_t ko = (uint32_t)(i * (int)k_snb + (t & 1) * 128);
+      slab_copy_1k(kres, t < steps ? voffK[j] + ko : 0xffffffffu, st + (uint32_t)(wave * 4 + j) * 1024);
+    } else {
+      const int qi = p.S - 1 - i;
+      const uint32_t qo = (uint32_t)(qi * (int)q_snb + (t & 1) * 128);
+      slab_copy_1k(qres, t < steps && qtok[j - 4] + qi < p.Lq ? voffQ[j - 4] + qo : 0xffffffffu,
+                   st + 16384 + (uint32_t)(wave * MT + j - 4) * 1024);
+    }
+  };
+  f32x16 acc[MT];
+#pragma unroll
+  for (int a = 0; a < MT; ++a)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[a][v] = 0.f;
+  const int swz = (r >> 1) & 7;
+  // A step is four sub-steps of MT MFMAs; the fragments of the next sub-step and the copies of step t + NS - 1 are issued
+  // between them.  The barrier sits before the last sub-step's MFMAs: by then this wavefront has read every fragment of
+  // step t and its copies of step t + 1 have landed, so behind it step t + 1 may be read and step t's stage refilled.
+  if (live_w) {
+#pragma unroll
+    for (int t = 0; t < NS - 1; ++t)
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j) copy_piece(t, j);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 2) * kLoads) : "memory");
+    bf16x8 fa[2], fb[2][MT];
+    auto read = [&](int t, int s, int buf) __attribute__((always_inline)) {
+      const char* st = lds + (t % NS) * kStage;
+      const int ch = ((2 * s + hh) ^ swz) << 4;
+      fa[buf] = *reinterpret_cast<const bf16x8*>(st + (wave * 32 + r) * 128 + ch);
+#pragma unroll
+      for (int a = 0; a < MT; ++a) fb[buf][a] = *reinterpret_cast<const bf16x8*>(st + 16384 + (a * 32 + r) * 128 + ch);
+    };
+    read(0, 0, 0);
+    for (int t = 0; t < steps; ++t) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (s == 3) {
+          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * kLoads) : "memory");
+          read(t + 1, 0, 0);     // (a repeat of old data behind the last step)
+        } else {
+          read(t, s + 1, (s + 1) & 1);
+#pragma unroll
+          for (int j = s * kPer; j < kLoads && j < (s + 1) * kPer; ++j) copy_piece(t + NS - 1, j);
+        }
+#pragma unroll
+        for (int a = 0; a < MT; ++a) acc[a] = mfma32(fa[s & 1], fb[s & 1][a], acc[a]);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int t = 0; t < NS - 1; ++t)
+#pragma unroll
+      for (int j = 4; j < kLoads; ++j) copy_piece(t, j);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 2) * MT) : "memory");
+    for (int t = 0; t < steps; ++t) {
+#pragma unroll
+      for (int j = 4; j < kLoads; ++j) copy_piece(t + NS - 1, j);
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 2) * MT) : "memory");
+    }
+  }
+  // every copy has landed and every fragment has been read: the LDS is free for the exchange below
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+
+  // ---- epilogue, in the operations and the order of estimate_gemm_kernel: there one wavefront has all 128 keys of a
+  // row; here the four wavefronts' maxima and sums meet in LDS
+  float* maxes = reinterpret_cast<float*>(lds);                 // [4][kRows]
+  float* parts = maxes + 4 * kRows;                             // [4][2][MT][64]
+  float mx[MT];
+#pragma unroll
+  for (int a = 0; a < MT; ++a) {
+    const int m = m0 + ((a * 32 + r) & (p.tile_rows - 1));
+    const int lo = row_lo(p, m), hi = row_hi(p, m);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int n = n_w + (v >> 2) * 8 + hh * 4 + (v & 3);
+      acc[a][v] = n >= lo && n <= hi && n < p.n_rk ? acc[a][v] : -INFINITY;
+    }
+    float w = -INFINITY;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) w = fmaxf(w, acc[a][v]);
+    w = half_max(w * p.scale_log2);
+    if (hh == 0) maxes[wave * kRows + a * 32 + r] = w;
+  }
+  __syncthreads();
+  const int kb_first = n0 / RBS, kb_left = p.nkb - kb_first;
+#pragma unroll
+  for (int a = 0; a < MT; ++a) {
+    const int rr = a * 32 + r;
+    mx[a] = fmaxf(fmaxf(maxes[rr], maxes[kRows + rr]), fmaxf(maxes[2 * kRows + rr], maxes[3 * kRows + rr]));
+    const float safe = mx[a] == -INFINITY ? 0.f : mx[a];
+    const int head = h0 + (rr >> p.tile_shift), m = m0 + (rr & (p.tile_rows - 1));
+    const bool row_ok = m < p.live_end && head < h_end;
+    float* const prow = p.P + ((int64_t)(row_ok ? head : h0) * p.nkb + kb_first) * p.rows + (m - p.row_begin);
+    const int64_t rows64 = p.rows;
+    const bool st0 = row_ok && hh == 0, st1 = row_ok && hh == 1;
+    float s[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      s[q] = 0.f;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) s[q] += fast_exp2(__builtin_fmaf(acc[a][q * 4 + u], p.scale_log2, -safe));
+    }
+    float* const part = parts + (wave * 2 * MT + a) * 64 + lane;
+    constexpr int Gk = RBS / 8;
+    if (Gk == 1) {
+#pragma unroll
+      for (int q2 = 0; q2 < 2; ++q2) {
+        const float both = half_sum_pair(s[2 * q2], s[2 * q2 + 1]);
+        part[q2 * MT * 64] = both;
+        const int k = wave * 4 + 2 * q2;
+        if (k < kb_left && st0) prow[k * rows64] = both;
+        if (k + 1 < kb_left && st1) prow[(k + 1) * rows64] = both;
+      }
+    } else if (Gk == 2) {
+      const float both = half_sum_pair(s[0] + s[1], s[2] + s[3]);
+      part[0] = both;
+      const int k = wave * 2;
+      if (k < kb_left && st0) prow[k * rows64] = both;
+      if (k + 1 < kb_left && st1) prow[(k + 1) * rows64] = both;
+    } else {
+      const float all = half_sum(s[0] + s[1] + s[2] + s[3]);
+      part[0] = hh == 0 ? all : 0.f;
+      if (wave < kb_left && st0) prow[wave * rows64] = all;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int a = 0; a < MT; ++a) {
+    if (a % 4 != wave) continue;
+    const int rr = a * 32 + r;
+    const int head = h0 + (rr >> p.tile_shift), m = m0 + (rr & (p.tile_rows - 1));
+    float tot = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+#pragma unroll
+      for (int q2 = 0; q2 < (RBS == 8 ? 2 : 1); ++q2) tot += parts[((w * 2 + q2) * MT + a) * 64 + lane];
+    tot = half_sum(tot);
+    if (m < p.live_end && head < h_end && hh == 0) {
+      const int64_t at = ((int64_t)head * p.nT + n0 / kSub) * p.rows + (m - p.row_begin);
+      p.Mt[at] = mx[a];
+      p.Lt[at] = tot;
+    }
+  }
+}
+
+}  // namespace xattn
