@@ -217,11 +217,31 @@ int xattn_block_sparse_fwd(const void* q, const void* k, const void* v, void* ou
                            int64_t o_stride_h, int64_t o_stride_n, int q_block_begin, int q_block_end,
                            int causal, float softmax_scale, void* stream);
 
+/* The same launch with long lists cut among workgroups where there are too few
+ * (head, q-block) units for the longest not to matter (attn_plan.h).
+ * `workspace`: xattn_block_sparse_workspace_bytes() bytes for the q_blocks =
+ * q_block_end - q_block_begin q-blocks of the launch, 256-byte aligned,
+ * contents undefined on entry and on return; 0 bytes (null allowed) means that
+ * nothing is cut.  Without lists (col_idx null; idx_rows = ceil(q_len / 128))
+ * the visible blocks of a unit are its list.  Where lists are cut depends on their lengths, num_heads and
+ * q_len only, so results do not depend on how q-blocks are spread over launches;
+ * a cut list's row sums are added in another order than an uncut one's.
+ */
+size_t xattn_block_sparse_workspace_bytes(int num_heads, int q_len, int k_len, int idx_rows, int q_blocks);
+
+int xattn_block_sparse_fwd_ws(const void* q, const void* k, const void* v, void* out, void* workspace,
+                              size_t workspace_bytes, const int32_t* col_idx, const int32_t* col_cnt,
+                              int64_t idx_pitch, int idx_rows, int idx_row0, int num_heads, int num_kv_heads,
+                              int q_len, int k_len, int head_dim, int64_t q_stride_h, int64_t q_stride_n,
+                              int64_t k_stride_h, int64_t k_stride_n, int64_t v_stride_h, int64_t v_stride_n,
+                              int64_t o_stride_h, int64_t o_stride_n, int q_block_begin, int q_block_end,
+                              int causal, float softmax_scale, void* stream);
+
 /* ---------------------------------------------------------------------------
  * The prefill operator in one call (Xattention_prefill, xattn/src/Xattention.py:
  * 302-402): estimate, selection and block-sparse attention enqueued back to
  * back, everything between them in `workspace` (at least
- * xattn_prefill_workspace_bytes() bytes, 16-byte aligned, contents undefined on
+ * xattn_prefill_workspace_bytes() bytes, 256-byte aligned, contents undefined on
  * entry and on return; 0 bytes means the geometry is refused).  Arguments as in
  * xattn_estimate_select and xattn_block_sparse_fwd, over all query chunks.
  * Thresholds: `tau_device` (fp64 [H] on the device) or, when that is null,

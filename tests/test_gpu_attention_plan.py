@@ -1,0 +1,58 @@
+"""GPU: the operator's attention with long lists cut among workgroups against the same lists swept whole."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(q_len, k_len, heads, kv_heads, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    rnd = lambda h, n: torch.randn(1, h, n, 128, generator=g, device="cuda").bfloat16()
+    return rnd(heads, q_len), rnd(kv_heads, k_len), rnd(kv_heads, k_len)
+
+
+def _swept_whole(q, k, v, idx, cnt, causal):
+    """The entry point that never cuts a list."""
+    from xattn.src import hip_backend as hb
+
+    heads, q_len, k_len = q.shape[1], q.shape[2], k.shape[2]
+    out = torch.empty(1, q_len, heads, 128, dtype=torch.bfloat16, device="cuda")
+    hb.check(hb.lib().xattn_block_sparse_fwd(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), idx.data_ptr(), cnt.data_ptr(), idx.shape[2], idx.shape[1], 0,
+        heads, k.shape[1], q_len, k_len, 128, q.stride(1), q.stride(2), k.stride(1), k.stride(2), v.stride(1), v.stride(2),
+        out.stride(2), out.stride(1), 0, -1, int(causal), 128 ** -0.5, torch.cuda.current_stream().cuda_stream), "fwd")
+    return out.transpose(1, 2).float()
+
+
+# every list full (threshold 1): all of one length, one to many pieces, lengths next to multiples of a piece, one ragged
+# query row, no causality; and mixed lists
+@pytest.mark.parametrize("q_len,cache,heads,kv_heads,threshold,causal", [
+    (1, 128 * 17, 4, 2, 1.0, True),
+    (64, 20000, 32, 8, 1.0, True),
+    (129, 128 * 24 - 1, 6, 2, 1.0, True),
+    (300, 128 * 40, 3, 1, 1.0, True),
+    (2500, 0, 8, 8, 1.0, True),
+    (2500, 0, 4, 2, 1.0, False),
+    (700, 9000, 28, 4, 0.95, True),
+    (2048, 30000, 32, 8, 0.9, True),
+])
+def test_cut_lists_give_the_same_attention(q_len, cache, heads, kv_heads, threshold, causal):
+    from xattn.src.Xattention import Xattention_prefill, block_sparse_attention, estimate_and_select
+
+    q, k, v = _inputs(q_len, q_len + cache, heads, kv_heads, q_len + cache)
+    chunk = 128                                                   # no padding between the last query and the last key
+    r = estimate_and_select(q, k, 8, threshold, chunk, causal=causal, want_mask=False, want_sums=False)
+    nq = (q_len + 127) // 128
+    idx, cnt = r["col_idx"][:, :nq].contiguous(), r["col_cnt"][:, :nq].contiguous()
+    assert cnt.max().item() > 8                                   # some list is long enough to be cut
+    want = _swept_whole(q, k, v, idx, cnt, causal)
+    # lists in memory are noted and cut the same way
+    assert torch.equal(block_sparse_attention(q, k, v, idx, cnt, causal=causal),
+                       Xattention_prefill(q, k, v, 8, threshold=threshold, chunk_size=chunk, causal=causal))
+    outs = [Xattention_prefill(q, k, v, 8, threshold=threshold, chunk_size=chunk, causal=causal) for _ in range(3)]
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])     # whoever combines the pieces
+    # Probabilities are rounded to bf16 (2^-9 relative) against another reference maximum, and the result once more:
+    # |difference| <= 2^-8 sum p |v| + 2^-8 |out| <= 2^-8 (max |v| + |out|)
+    bound = 2.0 ** -8 * (v.float().abs().amax() + want.abs())
+    assert ((outs[0].float() - want).abs() <= bound).all()
+    assert (outs[0].float() - want).norm() <= 4e-3 * want.norm()

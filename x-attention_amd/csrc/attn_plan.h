@@ -1,0 +1,82 @@
+// How long lists of the block-sparse attention are shared among workgroups.
+//
+// A workgroup works through its list one 128-key block after the other, 1.7 to 3.5 us each, and the longest list bounds
+// the launch: a chunk on top of a cache has few (head, q-block) units (32 .. 2000) and lists of up to hundreds of blocks,
+// and some heads of a prompt keep a hundred times as many blocks as others.  So lists of more than kMinPiece blocks are
+// noted when they are made, cut into at most `items` pieces of equal length and a rest; the attention launch has workgroups
+// for the pieces ahead of the units', and the unit's own workgroup takes the rest.  Each leaves (output, maximum, sum)
+// unnormalised in fp32, and whichever of them comes last combines them in their order.
+//
+// Where a list is cut depends on its length and on the size of the whole problem alone, so results do
+// not depend on how a problem is spread over launches.
+#pragma once
+#include "xattn_common.h"
+
+namespace xattn {
+
+constexpr int kMinPiece = 8;
+constexpr int kPartFloats = 128 * 128 + 2 * 128;   // of one item: outputs (accumulator order), row maxima, row sums
+
+struct AttnPlan {
+  unsigned long long* head;   // low half: pieces noted, high half: lists; set to zero before lists are noted
+  int32_t* pieces;            // [units * (items - 1)][2] unit, index of the piece in its list
+  int32_t* number;            // [lists] where a noted list stands among those
+  int32_t* done;              // [units] items finished, by that number
+  float* part;                // [units * items][kPartFloats], a list's own from number * items on
+  int items;                  // most items of a list; 0: no plan
+};
+
+// Items a list may be cut into, for a problem of `units` lists (heads x q-blocks) over nkb key blocks; 1: never.  The
+// launch has units * (items - 1) workgroups for pieces, and where lists are short they cost 1.5 - 2 us per thousand: up to
+// 2048 for a prompt by itself (whole call at 4096 tokens, us: uneven lists 125 -> 109, even ones 67.5 -> 68), up to 8192 on
+// top of a cache at least as long as the chunk, where lists are long and few (2048 tokens on 63488: 1426 -> 881 with
+// 8192, 1005 with 2048; 64 on 100000: 1461 -> 334; 8000 on 100000: 3865 -> 2765).  16 key blocks or fewer make short lists.
+inline int plan_items(int64_t units, int nqb, int nkb) {
+  const int64_t most = nkb >= 2 * nqb ? 8192 : 2048;
+  if (nkb <= 16 || units > most) return 1;
+  const int64_t n = most / units + 1;
+  return n > 16 ? 16 : (int)n;
+}
+// Bytes of a plan for `units` of the `lists` lists in memory, and the plan laid out there (256-byte aligned).
+inline size_t plan_round(size_t x) { return (x + 255) & ~(size_t)255; }
+inline size_t plan_bytes(int64_t lists, int64_t units, int items) {
+  if (items <= 1) return 0;
+  return 256 + plan_round((size_t)units * (items - 1) * 8) + plan_round((size_t)lists * 4) + plan_round((size_t)units * 4) +
+         (size_t)units * items * kPartFloats * sizeof(float);
+}
+inline AttnPlan plan_at(char* at, int64_t lists, int64_t units, int items) {
+  AttnPlan p{};
+  if (items <= 1) return p;
+  p.items = items;
+  p.head = reinterpret_cast<unsigned long long*>(at);
+  p.pieces = reinterpret_cast<int32_t*>(at += 256);
+  p.number = reinterpret_cast<int32_t*>(at += plan_round((size_t)units * (items - 1) * 8));
+  p.done = reinterpret_cast<int32_t*>(at += plan_round((size_t)lists * 4));
+  p.part = reinterpret_cast<float*>(at + plan_round((size_t)units * 4));
+  return p;
+}
+
+__host__ __device__ inline int piece_length(int count, int items) {
+  const int n = (int)(((uint32_t)count + (uint32_t)items - 1) / (uint32_t)items);
+  return n > kMinPiece ? n : kMinPiece;
+}
+// pieces taken off a list of `count` blocks, at most items - 1
+__host__ __device__ inline int piece_count(int count, int items) {
+  return count > kMinPiece ? (int)((uint32_t)(count - 1) / (uint32_t)piece_length(count, items)) : 0;
+}
+
+// Notes list `unit` of `count` blocks (called by one lane).
+__device__ __forceinline__ void note_list(const AttnPlan& p, int unit, int count) {
+  const int n = piece_count(count, p.items);
+  if (n == 0) return;
+  const unsigned long long old = __hip_atomic_fetch_add(p.head, (1ull << 32) | (unsigned long long)n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const int at = (int)(uint32_t)old, number = (int)(old >> 32);
+  p.number[unit] = number;
+  p.done[number] = 0;
+  for (int i = 0; i < n; ++i) {
+    p.pieces[2 * (at + i)] = unit;
+    p.pieces[2 * (at + i) + 1] = i;
+  }
+}
+
+}  // namespace xattn

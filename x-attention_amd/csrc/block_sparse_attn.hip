@@ -28,7 +28,9 @@
 // sweep): row-per-lane accesses to global memory would be hundreds of partial
 // line requests per wavefront, and a workgroup keeps its registers and LDS
 // until the last of its stores is acknowledged.
+#include "attn_plan.h"
 #include "attn_tiles.h"
+#include "estimate.h"
 #include "xattn_hip.h"
 
 namespace xattn {
@@ -49,6 +51,8 @@ struct AttnParams {
   int causal, kv_off;       // kv_off = Lk - Lq
   float scale_log2;         // softmax_scale * log2(e)
   DispatchShape shape;      // dispatch_shape(H, Hkv), computed on the host
+  AttnPlan plan;            // kPlanned only
+  int piece_grid;           // workgroups ahead of the units', for the pieces of cut lists (a multiple of 8)
 };
 
 __device__ __forceinline__ int clamp_block(int kb, int nkb) { return kb < 0 ? 0 : (kb < nkb ? kb : nkb - 1); }
@@ -246,10 +250,68 @@ __device__ __forceinline__ void store_out(const AttnParams& p, int head, int qb,
   }
 }
 
+// What an item of a cut list leaves behind: accumulators as the lanes hold them (1 KiB per store), row maxima and sums.
+// Items of a list run on any XCD, each with an L2 of its own: stores and loads are at device scope (kDeviceScope: they go
+// through to, and come from, memory that all of them share).
+constexpr int kDeviceScope = 16;   // sc1
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t part_resource(float* part) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)part, 0, kPartFloats * 4, 0x00020000);
+}
+__device__ __forceinline__ void store_partial(float* part, int wave, int lane, int r, int hh, const f32x16 (&oacc)[4], float m_run,
+                                              float l_run) {
+  const __amdgpu_buffer_rsrc_t res = part_resource(part);
+  const float l_tot = half_sum(l_run);
+  const int dst = (wave * 16 * 64 + lane) * 16;
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      f32x4 w;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) w[u] = oacc[dt][g * 4 + u];
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, w), res, dst + (dt * 4 + g) * 1024, 0, kDeviceScope);
+    }
+  if (hh == 0) {
+    const int at = (128 * 128 + wave * 32 + r) * 4;
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, m_run), res, at, 0, kDeviceScope);
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, l_tot), res, at + 512, 0, kDeviceScope);
+  }
+}
+// The items' results combined into the registers of a finished sweep, in the order of the list.
+__device__ __forceinline__ void load_partials(float* part, int items, int wave, int lane, int r, int hh, f32x16 (&oacc)[4], float& l_run) {
+  const int at = (128 * 128 + wave * 32 + r) * 4;
+  auto ml = [&](int s, int which) __attribute__((always_inline)) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(part_resource(part + (int64_t)s * kPartFloats), at + which * 512, 0, kDeviceScope));
+  };
+  float m = -INFINITY, l = 0.f;
+#pragma unroll 4
+  for (int s = 0; s < items; ++s) m = fmaxf(m, ml(s, 0));
+  const float safe = m == -INFINITY ? 0.f : m;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) oacc[i][v] = 0.f;
+  for (int s = 0; s < items; ++s) {
+    const __amdgpu_buffer_rsrc_t res = part_resource(part + (int64_t)s * kPartFloats);
+    const float w = fast_exp2(ml(s, 0) - safe);      // 0 where the item saw no key of this row
+    l += w * ml(s, 1);
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 o = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(res, (wave * 16 * 64 + lane) * 16 + (dt * 4 + g) * 1024, 0, kDeviceScope));
+#pragma unroll
+        for (int u = 0; u < 4; ++u) oacc[dt][g * 4 + u] += w * o[u];
+      }
+  }
+  l_run = hh == 0 ? l : 0.f;
+}
+
 typedef const __attribute__((address_space(4))) int32_t* const_i32_ptr;
 
-// kHasList = false is the dense baseline (its own symbol, so profiles tell the two apart)
-template <bool kHasList>
+// kHasList = false visits every visible block, the dense baseline (its own symbol, so profiles tell the two apart);
+// kPlanned: long lists are cut (attn_plan.h)
+template <bool kHasList, bool kPlanned>
 __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) {
   __shared__ __attribute__((aligned(1024))) char Ks[kTileBytes];
   __shared__ __attribute__((aligned(1024))) char Vs[kTileBytes];
@@ -258,7 +320,23 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
   const int r = lane & 31, hh = lane >> 5;
 
   int head, qb, kvh;
-  if (!map_workgroup(blockIdx.x, p.shape, p.qb_begin, p.qb_end, &head, &qb, &kvh)) return;
+  bool is_piece = false;
+  int index = 0;                     // which piece of its list a workgroup ahead of the units' has
+  if (kPlanned && (int)blockIdx.x < p.piece_grid) {
+    // an XCD gets a run of adjacent pieces, which are of adjacent lists
+    const int pieces = ((const_i32_ptr)(uintptr_t)p.plan.head)[0], per_xcd = (pieces + 7) / 8;
+    const int at = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per_xcd || at >= pieces) return;
+    const_i32_ptr entry = (const_i32_ptr)(uintptr_t)p.plan.pieces + 2 * at;
+    const int unit = entry[0];
+    index = entry[1];
+    is_piece = true;
+    head = unit / p.idx_rows;
+    qb = unit - head * p.idx_rows + p.idx_row0;
+    kvh = head / p.shape.group;
+  } else if (!map_workgroup((int)blockIdx.x - (kPlanned ? p.piece_grid : 0), p.shape, p.qb_begin, p.qb_end, &head, &qb, &kvh)) {
+    return;
+  }
   const __bf16* qbase = p.q + (int64_t)head * p.q_sh;
   const __bf16* kbase = p.k + (int64_t)kvh * p.k_sh;
   const __bf16* vbase = p.v + (int64_t)kvh * p.v_sh;
@@ -269,18 +347,31 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
   // the column list is read through the scalar cache (uniform, read-only), so that
   // fetching the next block id never waits on the tile copies in flight
   const_i32_ptr list = nullptr;
+  int cuts = 0, number = 0;          // pieces taken off this list, its number in the plan
   {
     const int q_last = (qb * kBlk + kBlk - 1 < p.Lq ? qb * kBlk + kBlk - 1 : p.Lq - 1) + p.kv_off;
     int visible = p.causal ? (q_last < 0 ? 0 : q_last / kBlk + 1) : p.nkb;
     visible = visible < p.nkb ? visible : p.nkb;
+    const int64_t slot = (int64_t)head * p.idx_rows + (qb - p.idx_row0);
     if (kHasList) {
-      const int64_t slot = (int64_t)head * p.idx_rows + (qb - p.idx_row0);
       list = (const_i32_ptr)(uintptr_t)(p.col_idx + slot * p.idx_pitch);
       n_blocks = ((const_i32_ptr)(uintptr_t)p.col_cnt)[slot];
-      first = list[0];                     // idx_pitch >= 1: readable whatever the count
+      if (!kPlanned) first = list[0];                          // idx_pitch >= 1: readable whatever the count
       n_blocks = n_blocks < 0 ? 0 : (n_blocks > p.idx_pitch ? (int)p.idx_pitch : n_blocks);
     } else {
       n_blocks = visible;
+    }
+    if (kPlanned) {
+      cuts = piece_count(n_blocks, p.plan.items);
+      if (cuts > 0) {
+        const int piece = piece_length(n_blocks, p.plan.items);
+        number = ((const_i32_ptr)(uintptr_t)p.plan.number)[slot];
+        if (!is_piece) index = cuts;
+        if (kHasList) list += index * piece;
+        else first = index * piece;
+        n_blocks = is_piece ? piece : n_blocks - cuts * piece;
+      }
+      if (kHasList) first = list[0];
     }
   }
 
@@ -304,7 +395,7 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
     tile_offsets(p.q_sn, lane, wave, voffQ);
     copy_tile(qbase, p.q_sn, p.Lq, qb, voffQ, Vs, wave);
     if (n_blocks > 0) {
-      kb = kHasList ? clamp_block(first, p.nkb) : 0;
+      kb = kHasList ? clamp_block(first, p.nkb) : first;
       copy_tile(kbase, p.k_sn, p.Lk, kb, la.voffK, Ks, wave);
     }
     wait_vm0();
@@ -319,7 +410,7 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
   for (int j = 0; j < n_blocks; ++j) {
-    const int kb_next = (j + 1 < n_blocks) ? (kHasList ? clamp_block(list[j + 1], p.nkb) : j + 1) : -1;
+    const int kb_next = (j + 1 < n_blocks) ? (kHasList ? clamp_block(list[j + 1], p.nkb) : kb + 1) : -1;
     f32x16 sacc[4];
     qk_tile(Ks, la.kaddr, qreg, sacc);
     wait_vm0();
@@ -337,7 +428,42 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
     kb = kb_next;
   }
   // the last barrier of the sweep (or the one before it, for an empty list) left both tiles unused
+  if (kPlanned && cuts > 0) {
+    float* const part = p.plan.part + (int64_t)number * p.plan.items * kPartFloats;
+    store_partial(part + (int64_t)index * kPartFloats, wave, lane, r, hh, oacc, m_run, l_run);
+    wait_vm0();                              // written through to memory
+    __syncthreads();
+    int* const scratch = reinterpret_cast<int*>(Ks);
+    if (tid == 0) scratch[0] = __hip_atomic_fetch_add(p.plan.done + number, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (scratch[0] != cuts) return;          // the item that comes last combines them
+    __syncthreads();
+    load_partials(part, cuts + 1, wave, lane, r, hh, oacc, l_run);
+  }
   store_out(p, head, qb, wave, lane, r, hh, oacc, l_run, Ks + wave * 8192);
+}
+
+// Notes the long lists of q-blocks [qb_begin, qb_end) of every head, where the pass that made them has not (or, without
+// lists, the visible blocks of each).  One workgroup: it also clears the plan's head.
+__global__ __launch_bounds__(1024) void note_lists_kernel(AttnParams p) {
+  if (threadIdx.x == 0) *p.plan.head = 0;
+  __threadfence();
+  __syncthreads();
+  const int rows = p.qb_end - p.qb_begin;
+  for (int i = threadIdx.x; i < p.H * rows; i += 1024) {
+    const int qb = p.qb_begin + i % rows;
+    const int unit = i / rows * p.idx_rows + qb - p.idx_row0;
+    int n = p.nkb;
+    if (p.col_cnt) {
+      n = p.col_cnt[unit];
+      n = n > p.idx_pitch ? (int)p.idx_pitch : n;
+    } else if (p.causal) {
+      const int q_last = (qb * kBlk + kBlk - 1 < p.Lq ? qb * kBlk + kBlk - 1 : p.Lq - 1) + p.kv_off;
+      const int visible = q_last < 0 ? 0 : q_last / kBlk + 1;
+      n = visible < n ? visible : n;
+    }
+    note_list(p.plan, unit, n);
+  }
 }
 
 }  // namespace xattn
@@ -346,14 +472,15 @@ using namespace xattn;
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-extern "C" int xattn_block_sparse_fwd(const void* q, const void* k, const void* v, void* out,
+int xattn::block_sparse_impl(const void* q, const void* k, const void* v, void* out,
                                       const int32_t* col_idx, const int32_t* col_cnt, int64_t idx_pitch,
                                       int idx_rows, int idx_row0, int num_heads, int num_kv_heads, int q_len, int k_len,
                                       int head_dim,
                                       int64_t q_stride_h, int64_t q_stride_n, int64_t k_stride_h,
                                       int64_t k_stride_n, int64_t v_stride_h, int64_t v_stride_n,
                                       int64_t o_stride_h, int64_t o_stride_n, int q_block_begin, int q_block_end,
-                                      int causal, float softmax_scale, void* stream) {
+                                      int causal, float softmax_scale, void* stream,
+                                      const AttnPlan* plan, bool note) {
   if (!q || !k || !v || !out) return XATTN_ERR_NULL;
   if (head_dim != kHeadDim) return XATTN_ERR_HEAD_DIM;
   if (num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads) return XATTN_ERR_HEADS;
@@ -394,11 +521,72 @@ extern "C" int xattn_block_sparse_fwd(const void* q, const void* k, const void* 
   p.shape = dispatch_shape(p.H, p.Hkv);
   const int64_t grid = grid_for(p.H, p.Hkv, q_block_end - q_block_begin);
   if (grid > 0x7fffffff) return XATTN_ERR_SHAPE;
-  if (col_idx)
-    hipLaunchKernelGGL(block_sparse_fwd_kernel<true>, dim3((unsigned)grid), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), p);
-  else
-    hipLaunchKernelGGL(block_sparse_fwd_kernel<false>, dim3((unsigned)grid), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), p);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  p.plan = AttnPlan{};
+  p.piece_grid = 0;
+  if (plan) {
+    p.plan = *plan;
+    p.piece_grid = (int)(((int64_t)p.H * (q_block_end - q_block_begin) * (plan->items - 1) + 7) / 8 * 8);
+    if (grid + p.piece_grid > 0x7fffffff) return XATTN_ERR_SHAPE;
+    const dim3 wgs((unsigned)(grid + p.piece_grid));
+    if (note) hipLaunchKernelGGL(note_lists_kernel, dim3(1), dim3(1024), 0, s, p);
+    if (col_idx)
+      hipLaunchKernelGGL((block_sparse_fwd_kernel<true, true>), wgs, dim3(256), 0, s, p);
+    else
+      hipLaunchKernelGGL((block_sparse_fwd_kernel<false, true>), wgs, dim3(256), 0, s, p);
+  } else if (col_idx) {
+    hipLaunchKernelGGL((block_sparse_fwd_kernel<true, false>), dim3((unsigned)grid), dim3(256), 0, s, p);
+  } else {
+    hipLaunchKernelGGL((block_sparse_fwd_kernel<false, false>), dim3((unsigned)grid), dim3(256), 0, s, p);
+  }
   return hipGetLastError() == hipSuccess ? XATTN_OK : XATTN_ERR_LAUNCH;
+}
+
+extern "C" int xattn_block_sparse_fwd(const void* q, const void* k, const void* v, void* out,
+                                      const int32_t* col_idx, const int32_t* col_cnt, int64_t idx_pitch,
+                                      int idx_rows, int idx_row0, int num_heads, int num_kv_heads, int q_len, int k_len,
+                                      int head_dim,
+                                      int64_t q_stride_h, int64_t q_stride_n, int64_t k_stride_h,
+                                      int64_t k_stride_n, int64_t v_stride_h, int64_t v_stride_n,
+                                      int64_t o_stride_h, int64_t o_stride_n, int q_block_begin, int q_block_end,
+                                      int causal, float softmax_scale, void* stream) {
+  return block_sparse_impl(q, k, v, out, col_idx, col_cnt, idx_pitch, idx_rows, idx_row0, num_heads, num_kv_heads, q_len, k_len,
+                           head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n, o_stride_h,
+                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, nullptr, false);
+}
+
+namespace {
+int items_of(int num_heads, int q_len, int k_len) {
+  const int nqb = (q_len + kBlk - 1) / kBlk;
+  return plan_items((int64_t)num_heads * nqb, nqb, (k_len + kBlk - 1) / kBlk);
+}
+}  // namespace
+
+extern "C" size_t xattn_block_sparse_workspace_bytes(int num_heads, int q_len, int k_len, int idx_rows, int q_blocks) {
+  if (num_heads <= 0 || q_len <= 0 || k_len <= 0 || idx_rows <= 0 || q_blocks <= 0) return 0;
+  return plan_bytes((int64_t)num_heads * idx_rows, (int64_t)num_heads * q_blocks, items_of(num_heads, q_len, k_len));
+}
+
+extern "C" int xattn_block_sparse_fwd_ws(const void* q, const void* k, const void* v, void* out, void* workspace,
+                                         size_t workspace_bytes, const int32_t* col_idx, const int32_t* col_cnt,
+                                         int64_t idx_pitch, int idx_rows, int idx_row0, int num_heads, int num_kv_heads,
+                                         int q_len, int k_len, int head_dim, int64_t q_stride_h, int64_t q_stride_n,
+                                         int64_t k_stride_h, int64_t k_stride_n, int64_t v_stride_h, int64_t v_stride_n,
+                                         int64_t o_stride_h, int64_t o_stride_n, int q_block_begin, int q_block_end,
+                                         int causal, float softmax_scale, void* stream) {
+  if (q_len <= 0 || k_len <= 0) return XATTN_ERR_SHAPE;
+  if (q_block_end < 0) q_block_end = (q_len + kBlk - 1) / kBlk;
+  if (!col_idx) idx_rows = (q_len + kBlk - 1) / kBlk, idx_row0 = 0;
+  const int q_blocks = q_block_end - q_block_begin;
+  const size_t need = xattn_block_sparse_workspace_bytes(num_heads, q_len, k_len, idx_rows, q_blocks);
+  AttnPlan plan{};
+  if (need) {
+    if (!workspace) return XATTN_ERR_NULL;
+    if (workspace_bytes < need) return XATTN_ERR_WORKSPACE;
+    if (reinterpret_cast<uintptr_t>(workspace) & 255) return XATTN_ERR_ALIGN;
+    plan = plan_at(static_cast<char*>(workspace), (int64_t)num_heads * idx_rows, (int64_t)num_heads * q_blocks, items_of(num_heads, q_len, k_len));
+  }
+  return block_sparse_impl(q, k, v, out, col_idx, col_cnt, idx_pitch, idx_rows, idx_row0, num_heads, num_kv_heads, q_len, k_len,
+                           head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n, o_stride_h,
+                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, need ? &plan : nullptr, true);
 }

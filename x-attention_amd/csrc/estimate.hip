@@ -132,6 +132,7 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 31, hh = lane >> 5;
   const int wm = wave & 3, wn = wave >> 2;   // query quarter, key half
+  if (blockIdx.x == 0 && tid == 0 && p.noted) *p.noted = 0;
   // A workgroup works through tiles id, id + grid, ...: one workgroup fits a CU, so nothing else could hide
   // the wait for a tile's first slabs.  The slab pipeline therefore runs on across the tile boundary: the load
   // slots of a tile's last two k-steps fetch the first slabs of the NEXT tile, and the last sub-step reads its
@@ -932,6 +933,7 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
   p.n_pairs = num_slab_pairs;
   p.scores = scores_out;
   p.sums = block_sums;
+  p.noted = sel && sel->plan ? sel->plan->head : nullptr;
   // block_sums may hold a window of q-block rows only; the chunks of this call must lie inside it
   {
     const int bpc = chunk_size / block_size;
@@ -1011,6 +1013,7 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
     sp.tau_step = sel->tau_host_count == 1 ? 0 : 1;
     if (!sel->tau)
       for (int h = 0; h < sel->tau_host_count; ++h) sp.tau_val[h] = sel->tau_host[h];
+    sp.plan = sel->plan ? *sel->plan : AttnPlan{};
     sp.mask = sel->mask; sp.col_idx = sel->col_idx; sp.col_cnt = sel->col_cnt;
     sp.idx_pitch = sel->idx_pitch; sp.H = num_heads; sp.nqb = g.nqb; sp.nkb = g.nkb;
     sp.row_begin = chunk_begin * bpc;

@@ -39,6 +39,7 @@ struct EstParams {
   int tiles_per_head;       // tiles with a visible pair, per head
   int64_t total_tiles;      // tiles_per_head * H
   // estimate_small_kernel: a tile's rows are tile_rows rows of each of pack heads of one KV group
+  unsigned long long* noted;   // set to zero for the selection pass that follows (AttnPlan::head), or null
   int pack, tile_rows, tile_shift;   // powers of two, tile_rows = 1 << tile_shift
 };
 

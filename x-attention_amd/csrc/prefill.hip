@@ -17,8 +17,9 @@ using namespace xattn;
 
 namespace {
 struct PrefillLayout {
-  size_t est_bytes, cnt_off, idx_off, total;
+  size_t est_bytes, cnt_off, idx_off, plan_off, total;
   int nqb, nkb;
+  int items;   // most items of a list (attn_plan.h)
 };
 
 size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -31,7 +32,10 @@ bool prefill_layout(int num_heads, int q_len, int k_len, int stride, int chunk_s
   l->nkb = (k_len + 127) / 128;
   l->cnt_off = up256(l->est_bytes);
   l->idx_off = l->cnt_off + up256((size_t)num_heads * l->nqb * sizeof(int32_t));
-  l->total = l->idx_off + up256((size_t)num_heads * l->nqb * l->nkb * sizeof(int32_t));
+  l->plan_off = l->idx_off + up256((size_t)num_heads * l->nqb * l->nkb * sizeof(int32_t));
+  const int64_t units = (int64_t)num_heads * l->nqb;
+  l->items = plan_items(units, l->nqb, l->nkb);
+  l->total = l->plan_off + plan_bytes(units, units, l->items);
   return true;
 }
 }  // namespace
@@ -53,7 +57,7 @@ extern "C" int xattn_prefill_fwd(const void* q, const void* k, const void* v, vo
   PrefillLayout l;
   if (!prefill_layout(num_heads, q_len, k_len, stride, chunk_size, &l)) return XATTN_ERR_SHAPE;
   if (workspace_bytes < l.total) return XATTN_ERR_WORKSPACE;
-  if (reinterpret_cast<uintptr_t>(workspace) & 15) return XATTN_ERR_ALIGN;
+  if (reinterpret_cast<uintptr_t>(workspace) & 255) return XATTN_ERR_ALIGN;
   char* ws = static_cast<char*>(workspace);
   SelectArgs sel{};
   sel.tau = tau_device;
@@ -66,12 +70,16 @@ extern "C" int xattn_prefill_fwd(const void* q, const void* k, const void* v, vo
   sel.keep_recent = keep_recent;
   sel.real_q_blocks_only = 1;
   sel.stages = 3;
+  const int64_t units = (int64_t)num_heads * l.nqb;
+  const AttnPlan plan = plan_at(ws + l.plan_off, units, units, l.items);
+  // (with zero_rows_from 0 no row is estimated, and no MFMA pass would clear the plan's head: noted afterwards)
+  if (plan.items && zero_rows_from != 0) sel.plan = &plan;
   const int q_chunks = (int)(((int64_t)q_len + chunk_size - 1) / chunk_size);
   int rc = estimate_impl(q, k, nullptr, ws, l.est_bytes, nullptr, num_heads, num_kv_heads, q_len, k_len, head_dim,
                          q_stride_h, q_stride_n, k_stride_h, k_stride_n, stride, 128, chunk_size, 0, q_chunks, causal,
                          own_chunk_only, estimate_scale, nullptr, 0, 1, 1, zero_rows_from, 0, l.nqb, stream, &sel);
   if (rc != XATTN_OK) return rc;
-  return xattn_block_sparse_fwd(q, k, v, out, sel.col_idx, sel.col_cnt, l.nkb, l.nqb, 0, num_heads, num_kv_heads, q_len,
-                                k_len, head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n,
-                                o_stride_h, o_stride_n, 0, l.nqb, causal, softmax_scale, stream);
+  return block_sparse_impl(q, k, v, out, sel.col_idx, sel.col_cnt, l.nkb, l.nqb, 0, num_heads, num_kv_heads, q_len,
+                           k_len, head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n,
+                           o_stride_h, o_stride_n, 0, l.nqb, causal, softmax_scale, stream, plan.items ? &plan : nullptr, !sel.plan);
 }

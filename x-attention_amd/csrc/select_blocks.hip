@@ -59,7 +59,7 @@ extern "C" int xattn_select_blocks(const float* block_sums, const double* tau_pe
   if (row_begin < 0 || row_end > nq_blocks || row_begin >= row_end) return XATTN_ERR_SHAPE;
   if (col_idx && idx_pitch < 1) return XATTN_ERR_SHAPE;
   if (diag_offset < 0 || blocks_per_chunk < 1) return XATTN_ERR_SHAPE;
-  SelParams p;
+  SelParams p{};
   p.sums = block_sums; p.tau = tau_per_head; p.mask = mask; p.col_idx = col_idx; p.col_cnt = col_cnt;
   p.idx_pitch = idx_pitch; p.H = num_heads; p.nqb = nq_blocks; p.nkb = nk_blocks;
   p.row_begin = row_begin; p.row_end = row_end; p.diag_offset = diag_offset;

@@ -1,6 +1,7 @@
 // Threshold block selection of one q-block row by one wavefront: shared by the stand-alone selection kernel
 // (block sums from memory) and the estimator's fused normalise-and-select kernel (block sums from LDS).
 #pragma once
+#include "attn_plan.h"
 #include "xattn_common.h"
 
 namespace xattn {
@@ -21,6 +22,7 @@ struct SelParams {
   int causal, keep_sink, keep_recent, list_cols, q_len, kv_off;
   int blocks_per_chunk;
   int npow2;   // LDS key capacity (power of two >= nkb)
+  AttnPlan plan;   // head null: nothing is noted
 };
 
 constexpr int kSlots = 16;        // candidates per lane held in registers (rows up to 1024 candidates)
@@ -274,7 +276,11 @@ __device__ __forceinline__ void select_row(const SelParams& p, const float* x, i
       if (keep && pos < p.idx_pitch) list[pos] = c;
       count += __popcll(ballot);
     }
-    if (lane == 0) p.col_cnt[slot] = count < p.idx_pitch ? count : (int)p.idx_pitch;
+    if (lane == 0) {
+      count = count < p.idx_pitch ? count : (int)p.idx_pitch;
+      p.col_cnt[slot] = count;
+      if (p.plan.head) note_list(p.plan, (int)slot, count);
+    }
   }
 }
 

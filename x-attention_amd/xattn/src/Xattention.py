@@ -434,9 +434,17 @@ def block_sparse_attention(query_states, key_states, value_states, col_idx=None,
         pitch, idx_rows = 0, 0
     with torch.cuda.device(dev):
         stream_ptr = stream.cuda_stream if stream is not None else _stream_ptr(dev)
+        # long lists are cut among workgroups where the problem has few q-blocks
+        nb = (q_len + 127) // 128
+        ws_bytes = lib.xattn_block_sparse_workspace_bytes(
+            heads, q_len, k_len, idx_rows if col_idx is not None else nb, (qb1 if qb1 >= 0 else nb) - qb0)
+        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+        if workspace is not None and stream is not None:
+            workspace.record_stream(stream)
         _hb.check(
-            lib.xattn_block_sparse_fwd(
+            lib.xattn_block_sparse_fwd_ws(
                 q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+                workspace.data_ptr() if workspace is not None else None, ws_bytes,
                 col_idx.data_ptr() if col_idx is not None else None,
                 col_cnt.data_ptr() if col_cnt is not None else None,
                 pitch, idx_rows, idx_row0, heads, kv_heads, q_len, k_len, 128,
@@ -444,7 +452,7 @@ def block_sparse_attention(query_states, key_states, value_states, col_idx=None,
                 out.stride(2), out.stride(1), qb0, qb1, int(bool(causal)), scale,
                 stream_ptr,
             ),
-            "xattn_block_sparse_fwd",
+            "xattn_block_sparse_fwd_ws",
         )
     return out.transpose(1, 2)
 

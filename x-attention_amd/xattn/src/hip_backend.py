@@ -62,6 +62,11 @@ _SIGNATURES = {
     ),
     "xattn_gemv": (c_i32, [c_vp, c_i32, c_vp, c_i64, c_vp, c_vp, c_i32, c_vp]),
     "xattn_rope": (c_i32, [c_vp] * 4 + [c_i64] * 2 + [c_i32] * 4 + [c_vp]),
+    "xattn_block_sparse_workspace_bytes": (c_sz, [c_i32] * 5),
+    "xattn_block_sparse_fwd_ws": (
+        c_i32,
+        [c_vp] * 5 + [c_sz] + [c_vp] * 2 + [c_i64] + [c_i32] * 7 + [c_i64] * 8 + [c_i32, c_i32, c_i32, c_f32, c_vp],
+    ),
     "xattn_block_sparse_fwd": (
         c_i32,
         [c_vp] * 6 + [c_i64] + [c_i32] * 7 + [c_i64] * 8 + [c_i32, c_i32, c_i32, c_f32, c_vp],
