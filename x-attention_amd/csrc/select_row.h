@@ -27,6 +27,9 @@ struct SelParams {
 
 constexpr int kSlots = 16;        // candidates per lane held in registers (rows up to 1024 candidates)
 constexpr int kMaxExtract = 32;   // blocks pulled out one by one before falling back to the sort
+constexpr int kRankAll = 16;      // up to so many candidates are ranked at once
+constexpr int kBeforeRank = 4;    // ... and what is left of up to 64 after so many were pulled out one by one
+constexpr int kBeforeSearch = 6;  // blocks pulled out of more than 64 before the search for where a long list ends
 
 // value encoded in a sort key (0 for forced blocks and padding)
 __device__ __forceinline__ double key_value(uint64_t key) {
@@ -34,10 +37,44 @@ __device__ __forceinline__ double key_value(uint64_t key) {
   return hi ? (double)__uint_as_float(hi - 1u) : 0.0;
 }
 
+// Reductions over the wavefront through the data-parallel lane moves: within rows of 16 lanes by shifts of 1, 2, 4 and 8,
+// then over the rows; lane 63 ends up with the result, which comes back as a uniform value.  (A butterfly of lane permutes
+// takes a trip through the LDS crossbar per step, about 700 clk for a search step of the selection.)
+template <int kCtrl, int kRows>
+__device__ __forceinline__ uint32_t lane_move(uint32_t old, uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)x, kCtrl, kRows, 0xf, false);
+}
+template <typename F>
+__device__ __forceinline__ uint32_t wave_fold(uint32_t x, F f) {   // f idempotent: max or min
+  x = f(x, lane_move<0x111, 0xf>(x, x));
+  x = f(x, lane_move<0x112, 0xf>(x, x));
+  x = f(x, lane_move<0x114, 0xf>(x, x));
+  x = f(x, lane_move<0x118, 0xf>(x, x));
+  x = f(x, lane_move<0x142, 0xa>(x, x));
+  x = f(x, lane_move<0x143, 0xc>(x, x));
+  return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+__device__ __forceinline__ uint32_t wave_max(uint32_t x) {
+  return wave_fold(x, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
+}
+__device__ __forceinline__ uint32_t wave_min(uint32_t x) {
+  return wave_fold(x, [](uint32_t a, uint32_t b) { return a < b ? a : b; });
+}
+template <int kCtrl, int kRows>
+__device__ __forceinline__ double lane_move(double x) {            // 0 where no lane is moved from
+  const uint64_t b = __builtin_bit_cast(uint64_t, x);
+  return __builtin_bit_cast(double, ((uint64_t)lane_move<kCtrl, kRows>(0u, (uint32_t)(b >> 32)) << 32) | lane_move<kCtrl, kRows>(0u, (uint32_t)b));
+}
 __device__ __forceinline__ double wave_sum(double x) {
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) x += __shfl_xor(x, d, 64);
-  return x;
+  x += lane_move<0x111, 0xf>(x);
+  x += lane_move<0x112, 0xf>(x);
+  x += lane_move<0x114, 0xf>(x);
+  x += lane_move<0x118, 0xf>(x);
+  x += lane_move<0x142, 0xa>(x);
+  x += lane_move<0x143, 0xc>(x);
+  const uint64_t b = __builtin_bit_cast(uint64_t, x);
+  return __builtin_bit_cast(double, ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(b >> 32), 63) << 32) |
+                                        (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, 63));
 }
 
 // M(i + ahead) from the masses before the i-th ordinary block (b0), before its predecessor (b1) and before
@@ -116,7 +153,7 @@ __device__ __forceinline__ void select_row(const SelParams& p, const float* x, i
     for (int u = 0; u < kSlots; ++u)
       if (u * 64 < np2) {
         vals[u] = load_one(u * 64 + lane, true);
-        n_others += vals[u] != 0;
+        n_others += __popcll(__ballot(vals[u] != 0));
       }
   } else {
     for (int c = lane; c < np2; c += 64) keys[c] = sort_key(c, load_one(c, true));
@@ -137,18 +174,124 @@ __device__ __forceinline__ void select_row(const SelParams& p, const float* x, i
   // no block sum can exceed a forced key unless the row's total does: otherwise the forced blocks rank first
   // and a decision does not need the block's own value
   const bool may_outrank = p.causal && total > key_lo;
-  if (small) {
+  // At most 64 candidates, one per lane: each lane adds up what ranks ahead of its own, on top of the mass `before` that
+  // is already taken.  A candidate costs about 80 clk with nothing to wait for.
+  auto rank_all = [&](double before, double prev_before, int taken) {
+    const uint32_t mine = vals[0];
+    double mass = before;
+    uint32_t last = 0xffffffffu;       // the smallest value ahead: the predecessor in rank
+    bool first = true;
+    for (int c = 0; c < ncand; ++c) {
+      const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)mine, c);
+      if (o == 0) continue;
+      const bool ahead = o > mine || (o == mine && c < lane);
+      mass += ahead ? (double)__uint_as_float(o - 1u) : 0.0;
+      last = ahead && o < last ? o : last;
+      first = first && !ahead;
+    }
+    if (mine != 0) {
+      if (one_forced) mass = first ? (taken > 0 ? prev_before : 0.0) : mass - (double)__uint_as_float(last - 1u);
+      if (mass < required) flags[lane] = 1;
+      else dropped = 1;
+    }
+    finished = true;
+  };
+  if (ncand <= kRankAll && !may_outrank) {
+    rank_all(forced_sum, 0.0, 0);
+  } else if (small) {
+    // slots that hold candidates, four at a time (the others are skipped)
+    auto in_use = [&](int u) { return (u & ~3) * 64 < np2; };
     // ---- extraction: keep pulling out the largest remaining block while the rule says "keep"
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) n_others += __shfl_xor(n_others, d, 64);
     double before = forced_sum, prev_before = 0.0, prev2_before = 0.0;
+    int taken = 0;               // blocks kept so far
     for (int it = 0; it < kMaxExtract; ++it) {
+      if (it == kBeforeRank && np2 == 64 && !may_outrank) {
+        rank_all(before, prev_before, taken);
+        break;
+      }
+      if (it == kBeforeSearch && n_others > 0 && !may_outrank) {
+        // ---- a long list: bisection on the value for hi > lo with  before + (sum of values >= hi) < required  and
+        // before + (sum of values >= lo) >= required.  Everything from hi on is kept, and what is left to decide one by
+        // one lies between.  Rows of more than kMaxExtract blocks used to be sorted, 20 us for 512 candidates.
+        uint32_t hi = 0;
+#pragma unroll
+        for (int u = 0; u < kSlots; ++u) hi = vals[u] > hi ? vals[u] : hi;
+        hi = wave_max(hi) + 1;
+        uint32_t lo = 0, step = 1u << 22;        // (lo 0: not known yet; first the search goes down by growing steps)
+        int above = 0, from_lo = n_others;       // candidates >= hi, >= lo
+        double mass_hi = 0.0;
+        while (hi - lo > 1 && from_lo - above > 4) {
+          const uint32_t mid = lo ? lo + (hi - lo) / 2 : (hi > step + 1 ? hi - step : 1);
+          int n = 0;
+          double sum = 0.0;
+#pragma unroll
+          for (int u = 0; u < kSlots; ++u) {
+            uint32_t w = vals[u];
+            asm volatile("" : "+v"(w));          // (else every value is kept as a double across the loop)
+            const bool in = w >= mid;
+            n += __popcll(__ballot(in));
+            sum += in ? (double)__uint_as_float(w - 1u) : 0.0;
+          }
+          sum = wave_sum(sum);
+          if (before + sum < required) {
+            hi = mid;
+            mass_hi = sum;
+            above = n;
+            step <<= 1;
+          } else {
+            lo = mid;
+            from_lo = n;
+          }
+        }
+        if (above > 0) {
+          uint32_t least = 0xffffffffu;          // the last of the blocks taken
+#pragma unroll
+          for (int u = 0; u < kSlots; ++u) {
+            const bool in = vals[u] >= hi;
+            least = in && vals[u] < least ? vals[u] : least;
+            if (in) flags[u * 64 + lane] = 1;
+            vals[u] = in ? 0u : vals[u];
+          }
+          least = wave_min(least);
+          before += mass_hi;
+          prev_before = before - (double)__uint_as_float(least - 1u);
+          n_others -= above;
+          taken += above;
+        }
+        if (lo && hi - lo == 1 && from_lo - above > 4) {
+          // a run of equal sums: they come out by ascending column, each adding the same mass
+          const double t = (double)__uint_as_float(lo - 1u);
+          const int shift = one_forced && taken > 0 ? 1 : 0;     // judged against the mass before its predecessor
+          int seen = 0, kept = 0;
+#pragma unroll
+          for (int u = 0; u < kSlots; ++u) {
+            const bool in = vals[u] == lo;
+            const uint64_t tied = __ballot(in);
+            const int i = seen + __popcll(tied & ((1ull << lane) - 1ull));
+            const double mass = shift && i == 0 ? prev_before : before + (double)(i - shift) * t;
+            const bool keep = in && mass < required;
+            if (keep) flags[u * 64 + lane] = 1;
+            vals[u] = keep ? 0u : vals[u];
+            kept += __popcll(__ballot(keep));
+            seen += __popcll(tied);
+          }
+          if (kept < seen) {
+            finished = true;
+            dropped = 1;
+            break;
+          }
+          before += (double)kept * t;
+          prev_before = before - t;
+          n_others -= kept;
+          taken += kept;
+        }
+      }
       if (n_others == 0) {
         finished = true;
         break;
       }
       if (!may_outrank) {
-        const double mass = p.causal ? rank_mass(it, n_forced, before, prev_before, prev2_before) : before;
+        const double mass = p.causal ? rank_mass(taken, n_forced, before, prev_before, prev2_before) : before;
         if (!(mass < required)) {
           finished = true;
           dropped = 1;
@@ -157,15 +300,12 @@ __device__ __forceinline__ void select_row(const SelParams& p, const float* x, i
       }
       uint32_t best = 0;
 #pragma unroll
-      for (int u = 0; u < kSlots; ++u) best = vals[u] > best ? vals[u] : best;
-#pragma unroll
-      for (int d = 32; d > 0; d >>= 1) {
-        const uint32_t o = __shfl_xor(best, d, 64);
-        best = o > best ? o : best;
-      }
+      for (int u = 0; u < kSlots; ++u)
+        if (in_use(u)) best = vals[u] > best ? vals[u] : best;
+      best = wave_max(best);
       const double best_val = (double)__uint_as_float(best - 1u);
       if (may_outrank) {
-        const double mass = rank_mass(it, forced_ahead(best_val), before, prev_before, prev2_before);
+        const double mass = rank_mass(taken, forced_ahead(best_val), before, prev_before, prev2_before);
         if (!(mass < required)) {
           finished = true;
           dropped = 1;
@@ -174,19 +314,18 @@ __device__ __forceinline__ void select_row(const SelParams& p, const float* x, i
       }
       uint32_t col = 0xffffffffu;     // lowest column holding the maximum
 #pragma unroll
-      for (int u = kSlots - 1; u >= 0; --u) col = vals[u] == best ? (uint32_t)(u * 64 + lane) : col;
+      for (int u = kSlots - 1; u >= 0; --u)
+        if (in_use(u)) col = vals[u] == best ? (uint32_t)(u * 64 + lane) : col;
+      col = wave_min(col);
 #pragma unroll
-      for (int d = 32; d > 0; d >>= 1) {
-        const uint32_t o = __shfl_xor(col, d, 64);
-        col = o < col ? o : col;
-      }
-#pragma unroll
-      for (int u = 0; u < kSlots; ++u) vals[u] = (uint32_t)(u * 64 + lane) == col ? 0u : vals[u];
+      for (int u = 0; u < kSlots; ++u)
+        if (in_use(u)) vals[u] = (uint32_t)(u * 64 + lane) == col ? 0u : vals[u];
       if (lane == 0) flags[col] = 1;
       prev2_before = prev_before;
       prev_before = before;
       before += best_val;
       --n_others;
+      ++taken;
     }
   }
 
