@@ -258,6 +258,19 @@ int xattn_prefill_fwd(const void* q, const void* k, const void* v, void* out, vo
                       const double* tau_host, int tau_host_count, const double* tau_device, int keep_sink,
                       int keep_recent, float softmax_scale, void* stream);
 
+/* Block sums and mask in one call (what xattn_estimate returns, xattn/src/
+ * Xattention.py:13-299): block_sums bf16 and mask bytes, both
+ * [num_heads][q_len_padded/128][k_len_padded/128], every entry written;
+ * workspace as for xattn_estimate_block_sums over all query chunks, thresholds
+ * and limits as in xattn_prefill_fwd.
+ */
+int xattn_estimate_fwd(const void* q, const void* k, void* block_sums, uint8_t* mask, void* workspace,
+                       size_t workspace_bytes, int num_heads, int num_kv_heads, int q_len, int k_len, int head_dim,
+                       int64_t q_stride_h, int64_t q_stride_n, int64_t k_stride_h, int64_t k_stride_n, int stride,
+                       int chunk_size, int causal, int own_chunk_only, float estimate_scale, int zero_rows_from,
+                       const double* tau_host, int tau_host_count, const double* tau_device, int keep_sink,
+                       int keep_recent, void* stream);
+
 /* ---------------------------------------------------------------------------
  * Single-token decode attention over a KV cache.  Replaces the call to the
  * third-party flashinfer.single_decode_with_kv_cache(q, k, v, kv_layout="HND")

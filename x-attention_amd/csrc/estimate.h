@@ -12,6 +12,7 @@ struct SelectArgs {
   const double* tau_host;   // one value, or one per head (at most kMaxTauHost), copied into the kernel's arguments
   int tau_host_count;
   uint8_t* mask;
+  void* sums_out;           // bf16 [H][rows][nkb] block sums, or null
   int32_t* col_idx;
   int32_t* col_cnt;
   int64_t idx_pitch;

@@ -26,7 +26,6 @@
 #include "estimate.h"
 #include "estimate_params.h"
 #include "estimate_small.h"
-#include "select_row.h"
 #include "xattn_hip.h"
 
 namespace xattn {
@@ -398,39 +397,6 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
   }   // tiles of this workgroup
 }
 
-// The arithmetic of the normalisation, shared by the stand-alone pass and the fused normalise-and-select kernel
-// so that both give the same bits (fixed operation order, no contraction into fused multiply-adds).
-#pragma clang fp contract(off)
-// folds tile T's maximum / sum into a running (M, L)
-__device__ __forceinline__ void stat_step(float& M, float& L, float mt, float lt) {
-  const float Mn = fmaxf(M, mt);
-  const float safe = (Mn == -INFINITY) ? 0.f : Mn;
-  L = L * fast_exp2(M - safe) + lt * fast_exp2(mt - safe);
-  M = Mn;
-}
-// combines the four partial (M, L) of a row (tiles T = first + w, + 4, ... for w = 0..3) into the row's
-// maximum (0 when the row sees nothing, or without softmax) and 1 / sum (0 for rows that give zeros)
-__device__ __forceinline__ void stat_combine(const float (&Mw)[4], const float (&Lw)[4], bool real_row, int no_softmax,
-                                             float* rowM, float* rowInv) {
-  const float Mr = fmaxf(fmaxf(Mw[0], Mw[1]), fmaxf(Mw[2], Mw[3]));
-  const float safe = (Mr == -INFINITY) ? 0.f : Mr;
-  float Lr = 0.f;
-#pragma unroll
-  for (int w = 0; w < 4; ++w) Lr += Lw[w] * fast_exp2(Mw[w] - safe);
-  const bool real = real_row && Lr > 0.f;
-  // without softmax the partial sums are referred to 2^0 and left unnormalised
-  *rowM = no_softmax ? 0.f : safe;
-  *rowInv = real ? (no_softmax ? 1.f : 1.f / Lr) : 0.f;
-}
-// normalised partial sums of four consecutive rows, added up
-__device__ __forceinline__ float group_sum4(const f32x4& pv, const f32x4& mt, const f32x4& rM, const f32x4& rI) {
-  float acc = 0.f;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) acc += (rI[i] != 0.f) ? pv[i] * (fast_exp2(mt[i] - rM[i]) * rI[i]) : 0.f;
-  return acc;
-}
-#pragma clang fp contract(fast)
-
 // A 128-key tile that holds nothing but padded keys is not computed: its scores are zero, so its maximum is 0, every
 // visible key adds 2^0 and a key block's partial sum is its key count - what the MFMA pass would have written.
 // Only without causality (a causal row sees such a tile partly; nT_real is nT then).
@@ -663,6 +629,7 @@ __global__ __launch_bounds__(256) void estimate_select_kernel(EstParams p, SelPa
     const int row = strip0 / RBS + wave;                 // q-block row (row_begin is a multiple of RBS)
     if (row < sp.row_end) {
       char* mine = per_wave + (size_t)wave * wave_bytes;
+      if (sp.sums_out) store_sums(sp, reinterpret_cast<const float*>(mine + xs_off), head, row, lane);
       select_row(sp, reinterpret_cast<const float*>(mine + xs_off), head, row, reinterpret_cast<uint64_t*>(mine),
                  reinterpret_cast<uint8_t*>(mine + (size_t)sp.npow2 * 8), lane);
     }
@@ -770,11 +737,21 @@ hipError_t launch_gemm(const EstParams& p, dim3 grid, size_t lds, hipStream_t s)
 }
 template <int RBS, int MT, int NS>
 hipError_t launch_small_as(const EstParams& p, hipStream_t s) {
-  auto kernel = &estimate_small_kernel<RBS, MT, NS>;
+  auto kernel = &estimate_small_kernel<RBS, MT, NS, false>;
   static LdsLimit limit;
   hipError_t e = limit.raise(reinterpret_cast<const void*>(kernel));
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)((p.total_tiles + 7) / 8 * 8)), dim3(256), NS * (kSub + 32 * MT) * 128, s, p);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((p.total_tiles + 7) / 8 * 8)), dim3(256), NS * (kSub + 32 * MT) * 128, s, p, SelParams{});
+  return hipSuccess;
+}
+// estimate_small_kernel<RBS, 1, 4> with the selection behind it, for rows that see one key tile
+template <int RBS>
+hipError_t launch_small_select(const EstParams& p, const SelParams& sp, hipStream_t s) {
+  auto kernel = &estimate_small_kernel<RBS, kSmall[0].mt, kSmall[0].ns, true>;
+  static LdsLimit limit;
+  hipError_t e = limit.raise(reinterpret_cast<const void*>(kernel));
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((p.total_tiles + 7) / 8 * 8)), dim3(256), kSmall[0].ns * (kSub + 32 * kSmall[0].mt) * 128, s, p, sp);
   return hipSuccess;
 }
 template <int RBS>
@@ -1003,7 +980,7 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
   // workgroup's LDS (statistics + per wavefront: the row's sums, sort keys, flags) within 64 KiB
   SelParams sp;
   int qb_per_wg = 0;
-  size_t lds_sel = 0;
+  size_t lds_sel = 0, sel_wave_bytes = 0;
   dim3 grid_sel(1);
   if (sel) {
     if (g.nkb > 8192) return XATTN_ERR_SHAPE;      // (longer rows: block sums through memory, xattn_select_blocks)
@@ -1014,6 +991,7 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
     if (!sel->tau)
       for (int h = 0; h < sel->tau_host_count; ++h) sp.tau_val[h] = sel->tau_host[h];
     sp.plan = sel->plan ? *sel->plan : AttnPlan{};
+    sp.sums_out = static_cast<__bf16*>(sel->sums_out);
     sp.mask = sel->mask; sp.col_idx = sel->col_idx; sp.col_cnt = sel->col_cnt;
     sp.idx_pitch = sel->idx_pitch; sp.H = num_heads; sp.nqb = g.nqb; sp.nkb = g.nkb;
     sp.row_begin = chunk_begin * bpc;
@@ -1027,7 +1005,7 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
     while (np2 < g.nkb) np2 <<= 1;
     sp.npow2 = np2;
     const size_t nkb_pad = ((size_t)g.nkb + 15) & ~(size_t)15;
-    const size_t wave_bytes = (size_t)np2 * 8 + nkb_pad;
+    const size_t wave_bytes = sel_wave_bytes = (size_t)np2 * 8 + nkb_pad;
     qb_per_wg = 4;
     while (qb_per_wg > 1 && (qb_per_wg * (wave_bytes + 10 * p.rbs * sizeof(float)) > 64 * 1024 || qb_per_wg * p.rbs > 128))
       qb_per_wg >>= 1;
@@ -1046,8 +1024,17 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
     if (sp.row_end <= sp.row_begin) return hipSuccess;   // a chunk of padding alone
     return launch_select<RBS>(p, sp, qb_per_wg, grid_sel, lds_sel, s);
   };
+  // one pass instead of two where every row asked for is estimated, in 32-row tiles, and sees a single key tile
+  bool one_pass = variant == 0 && sel && sel->stages == 3 && !p.no_softmax && !p.sums && !sel->plan && p.nT_real == g.nT &&
+                  p.live_end == sp.row_end * p.rbs && row_lo(p, p.live_end - 1) == 0 &&
+                  (row_hi(p, p.live_end - 1) < kSub || g.n_rk <= kSub) && 4 * sel_wave_bytes <= 64 * 1024;
   const bool run_gemm = !sel || (sel->stages & 1), run_rest = !sel || (sel->stages & 2);
   hipError_t e = hipSuccess;
+  if (one_pass) {
+    e = p.rbs == 8 ? launch_small_select<8>(p, sp, s) : p.rbs == 16 ? launch_small_select<16>(p, sp, s) : launch_small_select<32>(p, sp, s);
+    if (e != hipSuccess) return XATTN_ERR_LAUNCH;
+    return hipGetLastError() == hipSuccess ? XATTN_OK : XATTN_ERR_LAUNCH;
+  }
   switch (p.rbs) {
     case 8:
       if (run_gemm && p.total_tiles > 0) e = variant >= 0 ? launch_small<8>(p, variant, s) : launch_gemm<8>(p, grid1, lds, s);

@@ -53,4 +53,36 @@ __host__ __device__ inline int row_hi(const EstParams& p, int m) {
   return p.causal ? m * p.kdb + p.kdb - 1 + p.off : p.n_rk - 1;
 }
 
+// The arithmetic of the normalisation, shared by the stand-alone pass and the fused forms so that all give the same bits (fixed operation order, no contraction into fused multiply-adds).
+#pragma clang fp contract(off)
+// folds tile T's maximum / sum into a running (M, L)
+__device__ __forceinline__ void stat_step(float& M, float& L, float mt, float lt) {
+  const float Mn = fmaxf(M, mt);
+  const float safe = (Mn == -INFINITY) ? 0.f : Mn;
+  L = L * fast_exp2(M - safe) + lt * fast_exp2(mt - safe);
+  M = Mn;
+}
+// combines the four partial (M, L) of a row (tiles T = first + w, + 4, ... for w = 0..3) into the row's
+// maximum (0 when the row sees nothing, or without softmax) and 1 / sum (0 for rows that give zeros)
+__device__ __forceinline__ void stat_combine(const float (&Mw)[4], const float (&Lw)[4], bool real_row, int no_softmax,
+                                             float* rowM, float* rowInv) {
+  const float Mr = fmaxf(fmaxf(Mw[0], Mw[1]), fmaxf(Mw[2], Mw[3]));
+  const float safe = (Mr == -INFINITY) ? 0.f : Mr;
+  float Lr = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) Lr += Lw[w] * fast_exp2(Mw[w] - safe);
+  const bool real = real_row && Lr > 0.f;
+  // without softmax the partial sums are referred to 2^0 and left unnormalised
+  *rowM = no_softmax ? 0.f : safe;
+  *rowInv = real ? (no_softmax ? 1.f : 1.f / Lr) : 0.f;
+}
+// normalised partial sums of four consecutive rows, added up
+__device__ __forceinline__ float group_sum4(const f32x4& pv, const f32x4& mt, const f32x4& rM, const f32x4& rI) {
+  float acc = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc += (rI[i] != 0.f) ? pv[i] * (fast_exp2(mt[i] - rM[i]) * rI[i]) : 0.f;
+  return acc;
+}
+#pragma clang fp contract(fast)
+
 }  // namespace xattn

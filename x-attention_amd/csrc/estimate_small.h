@@ -13,6 +13,7 @@
 // beyond that a third workgroup is worth more than a third stage.
 #pragma once
 #include "estimate_params.h"
+#include "select_row.h"
 
 namespace xattn {
 
@@ -23,8 +24,11 @@ __device__ __forceinline__ void slab_copy_1k(__amdgpu_buffer_rsrc_t rsrc, uint32
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(dst), "v"(voff), "s"(rsrc) : "memory", "m0");
 }
 
-template <int RBS, int MT, int NS>
-__global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p) {
+// kSelect (MT 1, rows that see no key past the first softmax tile): normalisation and selection follow in the same
+// workgroup, which has whole rows.  A 1000-token prompt then takes one launch of 13.6 us instead of two of 10.6 and 7.0.
+template <int RBS, int MT, int NS, bool kSelect>
+__global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p, SelParams sp) {
+  static_assert(!kSelect || MT == 1, "the selection takes a wavefront per query block of 32 rows");
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   constexpr int kKeys = kSub, kRows = 32 * MT;
   constexpr int kStage = (kKeys + kRows) * 128;     // bytes of one 64-deep step
@@ -165,6 +169,9 @@ __global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p) {
   // row; here the four wavefronts' maxima and sums meet in LDS
   float* maxes = reinterpret_cast<float*>(lds);                 // [4][kRows]
   float* parts = maxes + 4 * kRows;                             // [4][2][MT][64]
+  float* psum = parts + 8 * MT * 64;                            // kSelect: [128 / RBS][32] partial block sums,
+  float* row_m = psum + (kSub / RBS) * 32;                      // row maxima
+  float* row_inv = row_m + 32;                                  // and 1 / row sums
   float mx[MT];
 #pragma unroll
   for (int a = 0; a < MT; ++a) {
@@ -193,6 +200,13 @@ __global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p) {
     float* const prow = p.P + ((int64_t)(row_ok ? head : h0) * p.nkb + kb_first) * p.rows + (m - p.row_begin);
     const int64_t rows64 = p.rows;
     const bool st0 = row_ok && hh == 0, st1 = row_ok && hh == 1;
+    auto put = [&](int k, bool on, float x) __attribute__((always_inline)) {
+      if (kSelect) {
+        if (on) psum[k * 32 + r] = x;
+      } else if (k < kb_left && on) {
+        prow[k * rows64] = x;
+      }
+    };
     float s[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -208,19 +222,19 @@ __global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p) {
         const float both = half_sum_pair(s[2 * q2], s[2 * q2 + 1]);
         part[q2 * MT * 64] = both;
         const int k = wave * 4 + 2 * q2;
-        if (k < kb_left && st0) prow[k * rows64] = both;
-        if (k + 1 < kb_left && st1) prow[(k + 1) * rows64] = both;
+        put(k, st0, both);
+        put(k + 1, st1, both);
       }
     } else if (Gk == 2) {
       const float both = half_sum_pair(s[0] + s[1], s[2] + s[3]);
       part[0] = both;
       const int k = wave * 2;
-      if (k < kb_left && st0) prow[k * rows64] = both;
-      if (k + 1 < kb_left && st1) prow[(k + 1) * rows64] = both;
+      put(k, st0, both);
+      put(k + 1, st1, both);
     } else {
       const float all = half_sum(s[0] + s[1] + s[2] + s[3]);
       part[0] = hh == 0 ? all : 0.f;
-      if (wave < kb_left && st0) prow[wave * rows64] = all;
+      put(wave, st0, all);
     }
   }
   __syncthreads();
@@ -235,11 +249,42 @@ __global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p) {
 #pragma unroll
       for (int q2 = 0; q2 < (RBS == 8 ? 2 : 1); ++q2) tot += parts[((w * 2 + q2) * MT + a) * 64 + lane];
     tot = half_sum(tot);
-    if (m < p.live_end && head < h_end && hh == 0) {
+    if (kSelect) {
+      const float Mw[4] = {mx[a], -INFINITY, -INFINITY, -INFINITY}, Lw[4] = {tot, 0.f, 0.f, 0.f};
+      if (hh == 0) stat_combine(Mw, Lw, m < p.live_end && head < h_end && m < p.real_rows, 0, &row_m[r], &row_inv[r]);
+    } else if (m < p.live_end && head < h_end && hh == 0) {
       const int64_t at = ((int64_t)head * p.nT + n0 / kSub) * p.rows + (m - p.row_begin);
       p.Mt[at] = mx[a];
       p.Lt[at] = tot;
     }
+  }
+  if (kSelect) {
+    __syncthreads();
+    // wavefront b: query block b of the tile
+    const int head = h0 + ((wave * RBS) >> p.tile_shift), m = m0 + ((wave * RBS) & (p.tile_rows - 1));
+    if (wave * RBS >= 32 || head >= h_end || m >= p.live_end) return;
+    const size_t wave_bytes = (size_t)sp.npow2 * 8 + ((sp.nkb + 15) & ~15);
+    char* mine = reinterpret_cast<char*>(row_inv + 32) + wave * wave_bytes;
+    float* xs = reinterpret_cast<float*>(mine + (size_t)sp.npow2 * 8 - (size_t)((sp.nkb + 15) & ~15) * 4);
+    // lane (kb, l): rows 4l .. 4l+3 of the block, summed as estimate_select_kernel does
+    constexpr int kLanes = RBS / 4;
+    const int l = lane % kLanes, kb = lane / kLanes;
+    const int m4 = m + l * 4, row4 = wave * RBS + l * 4;
+    int hi = row_hi(p, m4);
+    hi = hi < p.n_rk - 1 ? hi : p.n_rk - 1;
+    float sum = 0.f;
+    if (kb < kSub / RBS && kb <= hi / RBS) {
+      const f32x4 rM = *reinterpret_cast<const f32x4*>(row_m + row4);
+      sum = group_sum4(*reinterpret_cast<const f32x4*>(psum + kb * 32 + row4), rM, rM, *reinterpret_cast<const f32x4*>(row_inv + row4));
+    }
+#pragma unroll
+    for (int d = 1; d < kLanes; d <<= 1) sum += __shfl_xor(sum, d, 64);
+    if (l == 0 && kb < kSub / RBS && kb < sp.nkb) xs[kb] = sum;
+    for (int c = kSub / RBS + lane; c < sp.nkb; c += 64) xs[c] = 0.f;
+    __builtin_amdgcn_wave_barrier();
+    const int row = m / RBS;
+    if (sp.sums_out) store_sums(sp, xs, head, row, lane);
+    select_row(sp, xs, head, row, reinterpret_cast<uint64_t*>(mine), reinterpret_cast<uint8_t*>(mine + (size_t)sp.npow2 * 8), lane);
   }
 }
 

@@ -86,6 +86,32 @@ bool read_tau(PyObject* o, int64_t heads, c10::Device dev, Tau* tau) {
   return true;
 }
 
+// What prefill and estimate share: geometry of a call and which rows and keys the reference's branches hide (see _Plan in
+// xattn/src/Xattention.py of this package).
+struct Call {
+  int64_t H, Hkv, Lq, Lk, chunk;
+  int stride, causal, own_chunk, zero_from;
+  float scale;
+  // false: not an ordinary call
+  bool read(const at::Tensor& q, const at::Tensor& k, long stride_, double norm, int use_triton, int causal_, long chunk_) {
+    if (!kernel_ready(q, 4) || !kernel_ready(k, 4) || k.device() != q.device()) return false;
+    H = q.size(1), Lq = q.size(2), Hkv = k.size(1), Lk = k.size(2), chunk = chunk_;
+    if (q.size(0) != 1 || k.size(0) != 1) return false;
+    if ((stride_ != 4 && stride_ != 8 && stride_ != 16) || !(norm > 0) || H < 1 || Hkv < 1 || H % Hkv || Lq < 1 || Lk < Lq ||
+        Lk > (int64_t(1) << 30) || chunk < 128 || chunk % 128 || chunk > (1 << 30))
+      return false;
+    if (padded(Lk) / 128 > 8192) return false;
+    stride = (int)stride_;
+    causal = causal_;
+    const int64_t q_pad = padded(Lq) - Lq, k_pad = padded(Lk) - Lk, n_rq = padded(Lq) / stride;
+    own_chunk = causal && !use_triton && k_pad / stride == 0;
+    zero_from = (int)(use_triton ? std::max<int64_t>(0, n_rq - k_pad / stride) : n_rq - q_pad / stride);
+    scale = (float)(1.0 / std::sqrt(128.0) / (double)stride / norm);
+    return true;
+  }
+  int64_t padded(int64_t n) const { return (n + chunk - 1) / chunk * chunk; }
+};
+
 // prefill(q, k, v, stride, norm, threshold, use_triton, causal, chunk_size, keep_sink, keep_recent, workspace_limit)
 PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (nargs != 12) return PyErr_Format(PyExc_TypeError, "prefill takes 12 arguments");
@@ -102,39 +128,70 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     PyErr_Clear();
     Py_RETURN_NONE;
   }
-  if (!kernel_ready(*q, 4) || !kernel_ready(*k, 4) || !kernel_ready(*v, 4)) Py_RETURN_NONE;
+  Call c;
+  if (!c.read(*q, *k, stride, norm, use_triton, causal, chunk) || !kernel_ready(*v, 4)) Py_RETURN_NONE;
   const c10::Device dev = q->device();
-  if (k->device() != dev || v->device() != dev) Py_RETURN_NONE;
-  const int64_t H = q->size(1), Lq = q->size(2), Hkv = k->size(1), Lk = k->size(2);
-  if (q->size(0) != 1 || k->size(0) != 1 || v->size(0) != 1 || v->size(1) != Hkv || v->size(2) != Lk) Py_RETURN_NONE;
-  if ((stride != 4 && stride != 8 && stride != 16) || !(norm > 0) || H < 1 || Hkv < 1 || H % Hkv || Lq < 1 || Lk < Lq ||
-      Lk > (int64_t(1) << 30) || chunk < 128 || chunk % 128 || chunk > (1 << 30))
-    Py_RETURN_NONE;
-  const size_t bytes = xattn_prefill_workspace_bytes((int)H, (int)Lq, (int)Lk, (int)stride, (int)chunk);
-  if (bytes == 0 || (long long)bytes > limit || (Lk + chunk - 1) / chunk * chunk / 128 > 8192) Py_RETURN_NONE;
-  // which rows and keys the reference's branches hide (see _Plan in xattn/src/Xattention.py of this package)
-  const int64_t q_pad = (chunk - Lq % chunk) % chunk, k_pad = (chunk - Lk % chunk) % chunk;
-  const int own_chunk = causal && !use_triton && k_pad / stride == 0;
-  const int64_t n_rq = (Lq + q_pad) / stride;
-  int64_t zero_from;
-  if (use_triton)
-    zero_from = std::max<int64_t>(0, n_rq - k_pad / stride);
-  else
-    zero_from = n_rq - q_pad / stride;
+  if (v->device() != dev || v->size(0) != 1 || v->size(1) != c.Hkv || v->size(2) != c.Lk) Py_RETURN_NONE;
+  const int H = (int)c.H, Lq = (int)c.Lq;
+  const size_t bytes = xattn_prefill_workspace_bytes(H, Lq, (int)c.Lk, c.stride, (int)chunk);
+  if (bytes == 0 || (long long)bytes > limit) Py_RETURN_NONE;
   OnDevice on(dev);
   Tau tau;
   if (!read_tau(args[5], H, dev, &tau)) Py_RETURN_NONE;
-  const auto opts = at::TensorOptions().device(dev);
-  at::Tensor out = at::empty_strided({1, H, Lq, 128}, {Lq * H * 128, 128, H * 128, 1}, opts.dtype(at::kBFloat16));
-  at::Tensor ws = at::empty({(int64_t)bytes}, opts.dtype(at::kByte));
+  at::Tensor out = at::empty_strided({1, H, Lq, 128}, {(int64_t)Lq * H * 128, 128, (int64_t)H * 128, 1},
+                                     at::TensorOptions().device(dev).dtype(at::kBFloat16));
+  const c10::DataPtr ws = c10::hip::HIPCachingAllocator::get()->allocate(bytes);
   const int rc = xattn_prefill_fwd(
-      q->data_ptr(), k->data_ptr(), v->data_ptr(), out.data_ptr(), ws.data_ptr(), bytes, (int)H, (int)Hkv, (int)Lq, (int)Lk,
-      128, q->stride(1), q->stride(2), k->stride(1), k->stride(2), v->stride(1), v->stride(2), 128, H * 128, (int)stride,
-      (int)chunk, causal, own_chunk, (float)(1.0 / std::sqrt(128.0) / (double)stride / norm), (int)zero_from,
-      tau.count ? tau.host : nullptr, tau.count, tau.count ? nullptr : tau.device.const_data_ptr<double>(), keep_sink,
-      keep_recent, (float)(1.0 / std::sqrt(128.0)), stream_of(dev));
+      q->data_ptr(), k->data_ptr(), v->data_ptr(), out.data_ptr(), ws.get(), bytes, H, (int)c.Hkv, Lq, (int)c.Lk, 128, q->stride(1),
+      q->stride(2), k->stride(1), k->stride(2), v->stride(1), v->stride(2), 128, (int64_t)H * 128, c.stride, (int)chunk, causal,
+      c.own_chunk, c.scale, c.zero_from, tau.count ? tau.host : nullptr, tau.count,
+      tau.count ? nullptr : tau.device.const_data_ptr<double>(), keep_sink, keep_recent, (float)(1.0 / std::sqrt(128.0)), stream_of(dev));
   if (rc != XATTN_OK) return fail("xattn_prefill_fwd", rc);
   return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
+// estimate(q, k, stride, norm, threshold, use_triton, causal, chunk_size, keep_sink, keep_recent, workspace_limit)
+//   -> (block sums, mask) of xattn_estimate
+PyObject* estimate(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 11) return PyErr_Format(PyExc_TypeError, "estimate takes 11 arguments");
+  HANDLE_TH_ERRORS
+  const at::Tensor *q = tensor_of(args[0]), *k = tensor_of(args[1]);
+  if (!q || !k) Py_RETURN_NONE;
+  const long stride = PyLong_AsLong(args[2]);
+  const double norm = PyFloat_AsDouble(args[3]);
+  const long chunk = PyLong_AsLong(args[7]);
+  const long long limit = PyLong_AsLongLong(args[10]);
+  const int use_triton = PyObject_IsTrue(args[5]), causal = PyObject_IsTrue(args[6]);
+  const int keep_sink = PyObject_IsTrue(args[8]), keep_recent = PyObject_IsTrue(args[9]);
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  Call c;
+  if (!c.read(*q, *k, stride, norm, use_triton, causal, chunk)) Py_RETURN_NONE;
+  const c10::Device dev = q->device();
+  const int H = (int)c.H, Lq = (int)c.Lq;
+  const size_t bytes = xattn_estimate_workspace_bytes(H, Lq, (int)c.Lk, c.stride, 128, (int)chunk, 0);
+  if (bytes == 0 || (long long)bytes > limit) Py_RETURN_NONE;
+  OnDevice on(dev);
+  Tau tau;
+  if (!read_tau(args[4], H, dev, &tau)) Py_RETURN_NONE;
+  const auto opts = at::TensorOptions().device(dev);
+  at::Tensor sums = at::empty({1, H, c.padded(Lq) / 128, c.padded(c.Lk) / 128}, opts.dtype(at::kBFloat16));
+  at::Tensor mask = at::empty(sums.sizes(), opts.dtype(at::kBool));
+  const c10::DataPtr ws = c10::hip::HIPCachingAllocator::get()->allocate(bytes);
+  const int rc = xattn_estimate_fwd(q->data_ptr(), k->data_ptr(), sums.data_ptr(), static_cast<uint8_t*>(mask.data_ptr()), ws.get(),
+                                    bytes, H, (int)c.Hkv, Lq, (int)c.Lk, 128, q->stride(1), q->stride(2), k->stride(1), k->stride(2),
+                                    c.stride, (int)chunk, causal, c.own_chunk, c.scale, c.zero_from, tau.count ? tau.host : nullptr,
+                                    tau.count, tau.count ? nullptr : tau.device.const_data_ptr<double>(), keep_sink, keep_recent,
+                                    stream_of(dev));
+  if (rc != XATTN_OK) return fail("xattn_estimate_fwd", rc);
+  PyObject* result = PyTuple_New(2);
+  if (!result) return nullptr;
+  PyTuple_SET_ITEM(result, 0, THPVariable_Wrap(std::move(sums)));
+  PyTuple_SET_ITEM(result, 1, THPVariable_Wrap(std::move(mask)));
+  return result;
   END_HANDLE_TH_ERRORS
 }
 
@@ -276,6 +333,7 @@ PyMethodDef method(const char* name) {
 }
 PyMethodDef methods[] = {
     method<prefill>("prefill"),
+    method<estimate>("estimate"),
     method<decode>("decode"),
     method<project>("project"),
     method<output>("output"),

@@ -73,13 +73,41 @@ extern "C" int xattn_prefill_fwd(const void* q, const void* k, const void* v, vo
   const int64_t units = (int64_t)num_heads * l.nqb;
   const AttnPlan plan = plan_at(ws + l.plan_off, units, units, l.items);
   // (with zero_rows_from 0 no row is estimated, and no MFMA pass would clear the plan's head: noted afterwards)
-  if (plan.items && zero_rows_from != 0) sel.plan = &plan;
-  const int q_chunks = (int)(((int64_t)q_len + chunk_size - 1) / chunk_size);
+  // Where no list can be long enough to be cut, nothing is noted (nor planned below): then the selection may follow the
+  // estimate in the same kernel.
+  const int q_chunks = (int)(((int64_t)q_len + chunk_size - 1) / chunk_size), k_chunks = (int)(((int64_t)k_len + chunk_size - 1) / chunk_size);
+  const int64_t last_token = (int64_t)l.nqb * 128 - 1 + (int64_t)(k_chunks - q_chunks) * chunk_size;   // on the key axis, both padded
+  const bool may_cut = plan.items && (!causal || keep_sink || last_token / 128 + 1 > kMinPiece);
+  if (may_cut && zero_rows_from != 0) sel.plan = &plan;
   int rc = estimate_impl(q, k, nullptr, ws, l.est_bytes, nullptr, num_heads, num_kv_heads, q_len, k_len, head_dim,
                          q_stride_h, q_stride_n, k_stride_h, k_stride_n, stride, 128, chunk_size, 0, q_chunks, causal,
                          own_chunk_only, estimate_scale, nullptr, 0, 1, 1, zero_rows_from, 0, l.nqb, stream, &sel);
   if (rc != XATTN_OK) return rc;
   return block_sparse_impl(q, k, v, out, sel.col_idx, sel.col_cnt, l.nkb, l.nqb, 0, num_heads, num_kv_heads, q_len,
                            k_len, head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n,
-                           o_stride_h, o_stride_n, 0, l.nqb, causal, softmax_scale, stream, plan.items ? &plan : nullptr, !sel.plan);
+                           o_stride_h, o_stride_n, 0, l.nqb, causal, softmax_scale, stream, may_cut ? &plan : nullptr, !sel.plan);
+}
+
+extern "C" int xattn_estimate_fwd(const void* q, const void* k, void* block_sums, uint8_t* mask, void* workspace,
+                                  size_t workspace_bytes, int num_heads, int num_kv_heads, int q_len, int k_len,
+                                  int head_dim, int64_t q_stride_h, int64_t q_stride_n, int64_t k_stride_h,
+                                  int64_t k_stride_n, int stride, int chunk_size, int causal, int own_chunk_only,
+                                  float estimate_scale, int zero_rows_from, const double* tau_host, int tau_host_count,
+                                  const double* tau_device, int keep_sink, int keep_recent, void* stream) {
+  if (!workspace || !block_sums || !mask) return XATTN_ERR_NULL;
+  if (reinterpret_cast<uintptr_t>(block_sums) & 1) return XATTN_ERR_ALIGN;
+  if (q_len <= 0 || chunk_size <= 0) return XATTN_ERR_SHAPE;
+  SelectArgs sel{};
+  sel.tau = tau_device;
+  sel.tau_host = tau_host;
+  sel.tau_host_count = tau_host_count;
+  sel.mask = mask;
+  sel.sums_out = block_sums;
+  sel.keep_sink = keep_sink;
+  sel.keep_recent = keep_recent;
+  sel.stages = 3;
+  const int q_chunks = (int)(((int64_t)q_len + chunk_size - 1) / chunk_size);
+  return estimate_impl(q, k, nullptr, workspace, workspace_bytes, nullptr, num_heads, num_kv_heads, q_len, k_len, head_dim,
+                       q_stride_h, q_stride_n, k_stride_h, k_stride_n, stride, 128, chunk_size, 0, q_chunks, causal,
+                       own_chunk_only, estimate_scale, nullptr, 0, 1, 1, zero_rows_from, 0, 0, stream, &sel);
 }

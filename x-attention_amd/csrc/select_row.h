@@ -14,6 +14,7 @@ struct SelParams {
   double tau_val[kMaxTauHost];
   int tau_step;
   uint8_t* mask;
+  __bf16* sums_out;                // block sums for the caller, or null
   int32_t* col_idx;
   int32_t* col_cnt;
   int64_t idx_pitch;
@@ -83,6 +84,12 @@ __device__ __forceinline__ double rank_mass(int i, int ahead, double b0, double 
   const int back = 2 - ahead;          // 0, 1 or 2 ordinary blocks fewer than all those ahead of it
   if (i < back) return 0.0;
   return back == 0 ? b0 : (back == 1 ? b1 : b2);
+}
+
+// a row's block sums for the caller
+__device__ __forceinline__ void store_sums(const SelParams& p, const float* x, int head, int row, int lane) {
+  __bf16* out = p.sums_out + ((int64_t)head * p.win_rows + (row - p.win_row0)) * p.nkb;
+  for (int c = lane; c < p.nkb; c += 64) out[c] = (__bf16)x[c];
 }
 
 // Selection for q-block row `row` of `head` by ONE wavefront (lane = its lane number).  x: the row's nkb block

@@ -376,6 +376,12 @@ def xattn_estimate(
     """
     if kdb != 1 and use_triton:
         raise ValueError("use_triton and kdb cannot be used together")
+    if kdb == 1 and softmax and block_size == BLOCK and select_mode in ("inverse", ""):
+        # the ordinary call: block sums for the caller and the mask from one normalise-and-select pass
+        res = _hb.host().estimate(query_states, key_states, stride, norm, threshold, use_triton, causal, chunk_size, keep_sink,
+                                  keep_recent, WORKSPACE_LIMIT)
+        if res is not None:
+            return res
     r = estimate_and_select(
         query_states, key_states, stride, threshold, chunk_size, causal=causal, norm=norm,
         use_triton=use_triton, keep_sink=keep_sink, keep_recent=keep_recent, block_size=block_size,

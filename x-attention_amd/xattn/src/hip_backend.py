@@ -47,6 +47,11 @@ _SIGNATURES = {
         [c_vp] * 5 + [c_sz] + [c_i32] * 5 + [c_i64] * 8 + [c_i32] * 4 + [c_f32, c_i32]
         + [ctypes.POINTER(ctypes.c_double), c_i32, c_vp, c_i32, c_i32, c_f32, c_vp],
     ),
+    "xattn_estimate_fwd": (
+        c_i32,
+        [c_vp] * 5 + [c_sz] + [c_i32] * 5 + [c_i64] * 4 + [c_i32] * 4 + [c_f32, c_i32]
+        + [ctypes.POINTER(ctypes.c_double), c_i32, c_vp, c_i32, c_i32, c_vp],
+    ),
     "xattn_decode_workspace_bytes": (c_sz, [c_i32] * 3),
     "xattn_decode_fwd": (
         c_i32,
