@@ -326,6 +326,12 @@ int xattn_decode_fwd_static(const void* q, const void* k, const void* v, void* o
  * width: a multiple of 8, at most 2^24.
  * xattn_rope: rotates q [tokens][num_heads][128] and k [tokens][num_kv_heads][128]
  * in place; cos and sin [tokens][128] with a token stride.
+ * xattn_qkv_rope_gemm, xattn_gemm: the products of the first two for x [tokens][width]
+ * of up to about a thousand tokens, results [tokens][features]; width a multiple of
+ * 64, at most 65536, features a multiple of 128, pointers 16-byte aligned.
+ * xattn_proj_gemm_fits says whether they take a product of that size (features: the
+ * three products' together for q, k and v); larger ones are refused with
+ * XATTN_ERR_SHAPE and belong to a library.
  */
 int xattn_qkv_rope_gemv(const void* x, int width, const void* wq, int64_t wq_stride, const void* bq, const void* wk,
                         int64_t wk_stride, const void* bk, const void* wv, int64_t wv_stride, const void* bv,
@@ -334,6 +340,16 @@ int xattn_qkv_rope_gemv(const void* x, int width, const void* wq, int64_t wq_str
 
 int xattn_gemv(const void* x, int width, const void* w, int64_t w_stride, const void* bias, void* y, int rows,
                void* stream);
+
+int xattn_proj_gemm_fits(int tokens, int width, int features, int qkv);
+
+int xattn_qkv_rope_gemm(const void* x, int tokens, int width, const void* wq, int64_t wq_stride, const void* bq,
+                        const void* wk, int64_t wk_stride, const void* bk, const void* wv, int64_t wv_stride,
+                        const void* bv, const void* cos, const void* sin, int64_t cos_stride, int64_t sin_stride,
+                        void* q, void* k, void* v, int num_heads, int num_kv_heads, int head_dim, void* stream);
+
+int xattn_gemm(const void* x, int tokens, int width, const void* w, int64_t w_stride, const void* bias, void* y,
+               int features, void* stream);
 
 int xattn_rope(void* q, void* k, const void* cos, const void* sin, int64_t cos_stride, int64_t sin_stride, int tokens,
                int num_heads, int num_kv_heads, int head_dim, void* stream);

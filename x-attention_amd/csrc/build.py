@@ -15,7 +15,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(os.path.dirname(HERE))
 SOURCES = ["capi.hip", "block_sparse_attn.hip", "estimate.hip", "select_blocks.hip", "decode_attn.hip", "profile_threshold.hip", "softmax_block_sum.hip",
-           "prefill.hip", "layer_proj.hip"]
+           "prefill.hip", "layer_proj.hip", "proj_gemm.hip"]
 LIB = os.path.join(HERE, "libxattn_hip.so")
 HOST_SOURCE = os.path.join(HERE, "host_torch.cpp")
 HOST_LIB = os.path.join(HERE, "xattn_host.so")

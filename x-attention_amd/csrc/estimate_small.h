@@ -17,13 +17,6 @@
 
 namespace xattn {
 
-typedef __attribute__((address_space(3))) char* lds_char_ptr;
-
-// one KiB of a slab (8 rows of 128 bytes), global -> LDS; the caller counts it in vmcnt
-__device__ __forceinline__ void slab_copy_1k(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t dst) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(dst), "v"(voff), "s"(rsrc) : "memory", "m0");
-}
-
 // kSelect (MT 1, rows that see no key past the first softmax tile): normalisation and selection follow in the same
 // workgroup, which has whole rows.  A 1000-token prompt then takes one launch of 13.6 us instead of two of 10.6 and 7.0.
 template <int RBS, int MT, int NS, bool kSelect>

@@ -286,13 +286,24 @@ PyObject* project(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   OnDevice on(dev);
   at::Tensor y[3];
   int rc;
-  if (L == 1) {
+  const int64_t features = (heads[0] + 2 * heads[1]) * 128;
+  bool gemm = L > 1 && L <= 0x7fffffff && K <= 65536 && xattn_proj_gemm_fits((int)L, (int)K, (int)features, 1);
+  for (int i = 0; i < 3; ++i) gemm = gemm && lin[i].w->stride(0) <= (1 << 22);
+  if (L == 1 || gemm) {
     const auto opts = at::TensorOptions().device(dev).dtype(at::kBFloat16);
-    for (int i = 0; i < 3; ++i) y[i] = at::empty_strided({1, heads[i], 1, 128}, {heads[i] * 128, 128, heads[i] * 128, 1}, opts);
+    for (int i = 0; i < 3; ++i) y[i] = at::empty_strided({1, heads[i], L, 128}, {L * heads[i] * 128, 128, heads[i] * 128, 1}, opts);
+  }
+  if (L == 1) {
     rc = xattn_qkv_rope_gemv(x->data_ptr(), (int)K, lin[0].w->data_ptr(), lin[0].w->stride(0), lin[0].bias_ptr(),
                              lin[1].w->data_ptr(), lin[1].w->stride(0), lin[1].bias_ptr(), lin[2].w->data_ptr(),
                              lin[2].w->stride(0), lin[2].bias_ptr(), cos->data_ptr(), sin->data_ptr(), y[0].data_ptr(),
                              y[1].data_ptr(), y[2].data_ptr(), (int)heads[0], (int)heads[1], 128, stream_of(dev));
+  } else if (gemm) {
+    rc = xattn_qkv_rope_gemm(x->data_ptr(), (int)L, (int)K, lin[0].w->data_ptr(), lin[0].w->stride(0), lin[0].bias_ptr(),
+                             lin[1].w->data_ptr(), lin[1].w->stride(0), lin[1].bias_ptr(), lin[2].w->data_ptr(),
+                             lin[2].w->stride(0), lin[2].bias_ptr(), cos->data_ptr(), sin->data_ptr(), cos->stride(1),
+                             sin->stride(1), y[0].data_ptr(), y[1].data_ptr(), y[2].data_ptr(), (int)heads[0], (int)heads[1], 128,
+                             stream_of(dev));
   } else {
     for (int i = 0; i < 3; ++i) y[i] = at::linear(*x, *lin[i].w, lin[i].b);
     rc = xattn_rope(y[0].data_ptr(), y[1].data_ptr(), cos->data_ptr(), sin->data_ptr(), cos->stride(1), sin->stride(1), (int)L,
@@ -300,7 +311,7 @@ PyObject* project(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     for (int i = 0; i < 3; ++i)
       y[i] = y[i].as_strided({1, heads[i], L, 128}, {L * heads[i] * 128, 128, heads[i] * 128, 1});
   }
-  if (rc != XATTN_OK) return fail(L == 1 ? "xattn_qkv_rope_gemv" : "xattn_rope", rc);
+  if (rc != XATTN_OK) return fail(L == 1 ? "xattn_qkv_rope_gemv" : gemm ? "xattn_qkv_rope_gemm" : "xattn_rope", rc);
   PyObject* result = PyTuple_New(3);
   if (!result) return nullptr;
   for (int i = 0; i < 3; ++i) PyTuple_SET_ITEM(result, i, THPVariable_Wrap(std::move(y[i])));
@@ -308,21 +319,24 @@ PyObject* project(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
-// output(hidden, w, b): the output projection of one token
+// output(hidden, w, b): the output projection of one token, or of as many as proj_gemm.hip takes
 PyObject* output(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (nargs != 3) return PyErr_Format(PyExc_TypeError, "output takes 3 arguments");
   HANDLE_TH_ERRORS
   const at::Tensor *x = hidden_of(args[0]), *w = tensor_of(args[1]);
-  if (!x || x->size(1) != 1 || !w || w->dim() != 2 || w->size(0) % 4) Py_RETURN_NONE;
+  if (!x || !w || w->dim() != 2) Py_RETURN_NONE;
   const c10::Device dev = x->device();
-  const int64_t N = w->size(0), K = x->size(2);
+  const int64_t N = w->size(0), L = x->size(1), K = x->size(2);
   Linear lin;
-  if (N < 4 || N > 0x7fffffff || !lin.read(args[1], args[2], N, K, dev)) Py_RETURN_NONE;
+  if (N < 4 || N % 4 || N > 0x7fffffff || L > 0x7fffffff || !lin.read(args[1], args[2], N, K, dev)) Py_RETURN_NONE;
+  if (L > 1 && (K > 65536 || lin.w->stride(0) > (1 << 22) || !xattn_proj_gemm_fits((int)L, (int)K, (int)N, 0))) Py_RETURN_NONE;
   OnDevice on(dev);
-  at::Tensor y = at::empty({1, 1, N}, at::TensorOptions().device(dev).dtype(at::kBFloat16));
-  const int rc = xattn_gemv(x->data_ptr(), (int)K, lin.w->data_ptr(), lin.w->stride(0), lin.bias_ptr(), y.data_ptr(), (int)N,
-                            stream_of(dev));
-  if (rc != XATTN_OK) return fail("xattn_gemv", rc);
+  at::Tensor y = at::empty({1, L, N}, at::TensorOptions().device(dev).dtype(at::kBFloat16));
+  const int rc = L == 1 ? xattn_gemv(x->data_ptr(), (int)K, lin.w->data_ptr(), lin.w->stride(0), lin.bias_ptr(), y.data_ptr(), (int)N,
+                                     stream_of(dev))
+                        : xattn_gemm(x->data_ptr(), (int)L, (int)K, lin.w->data_ptr(), lin.w->stride(0), lin.bias_ptr(), y.data_ptr(),
+                                     (int)N, stream_of(dev));
+  if (rc != XATTN_OK) return fail(L == 1 ? "xattn_gemv" : "xattn_gemm", rc);
   return THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS
 }

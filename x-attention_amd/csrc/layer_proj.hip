@@ -6,30 +6,19 @@
 //    rotary pairs d, d + 64 and their neighbours, so that the rotation happens in registers), every load is a full
 //    1 KiB of one row, and 20 of them are in flight per wavefront before the first is used.  The library GEMM with
 //    one row left most of the chip idle: 47 us for the four products of that layer (1.8 TB/s), and the rotation
-//    another 13 launches.
+//    another 13 launches.  proj_gemm.hip has the products of more tokens.
 //  rope_kernel: the rotation of q and k of many tokens in place, one read and one write of both.  The reference's
 //    expression is ten elementwise kernels over them.
 //
 // Both round where the reference's bf16 tensor expression q * cos + rotate_half(q) * sin rounds: after the projection,
 // after each product and after the sum.
-#include "xattn_common.h"
+#include "rotate.h"
 #include "xattn_hip.h"
 
 namespace xattn {
 
-__device__ __forceinline__ float bf16_round(float x) { return (float)(__bf16)x; }
 __device__ __forceinline__ float bf16_lo(uint32_t w) { return __builtin_bit_cast(float, w << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
-
-// contraction would skip the roundings in between
-#pragma clang fp contract(off)
-__device__ __forceinline__ void rotate_pair(float& x0, float& x1, float c0, float c1, float s0, float s1) {
-  const float a0 = bf16_round(x0 * c0) + bf16_round(-x1 * s0);
-  const float a1 = bf16_round(x1 * c1) + bf16_round(x0 * s1);
-  x0 = bf16_round(a0);
-  x1 = bf16_round(a1);
-}
-#pragma clang fp contract(fast)
 
 struct GemvParams {
   const __bf16* x;
@@ -141,17 +130,8 @@ __global__ __launch_bounds__(256) void rope_kernel(RopeParams p) {
   base += c * 8;
   const __bf16* cs = p.cos + (int64_t)tok * p.cos_sn + c * 8;
   const __bf16* sn = p.sin + (int64_t)tok * p.sin_sn + c * 8;
-  const bf16x8 x0 = *reinterpret_cast<const bf16x8*>(base), x1 = *reinterpret_cast<const bf16x8*>(base + 64);
-  const bf16x8 c0 = *reinterpret_cast<const bf16x8*>(cs), c1 = *reinterpret_cast<const bf16x8*>(cs + 64);
-  const bf16x8 s0 = *reinterpret_cast<const bf16x8*>(sn), s1 = *reinterpret_cast<const bf16x8*>(sn + 64);
-  bf16x8 y0, y1;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    float a = (float)x0[e], b = (float)x1[e];
-    rotate_pair(a, b, (float)c0[e], (float)c1[e], (float)s0[e], (float)s1[e]);
-    y0[e] = (__bf16)a;
-    y1[e] = (__bf16)b;
-  }
+  bf16x8 y0 = *reinterpret_cast<const bf16x8*>(base), y1 = *reinterpret_cast<const bf16x8*>(base + 64);
+  rotate_chunks(y0, y1, cs, sn);
   *reinterpret_cast<bf16x8*>(base) = y0;
   *reinterpret_cast<bf16x8*>(base + 64) = y1;
 }

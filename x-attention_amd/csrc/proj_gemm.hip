@@ -1,0 +1,297 @@
+// The projections of an attention layer for turns of up to about a thousand tokens: y = x W^T with rows as long as the
+// hidden state; q, k and v in one launch with the rotation of q and k in its epilogue, or the output projection.
+//
+// Bound: with at most a tile per CU, by how fast one CU fills its LDS - 75 to 80 GB/s whatever the number of stages or
+// CUs at work, half of it W's - so the tile is the largest that still gives most CUs one: 64 x 64 up to 256 tiles, then
+// 64 tokens x 128 features, then 128 x 128, and two workgroups per CU for q, k and v beyond that.  Splitting a
+// step's depth over two groups of wavefronts helps the smallest tile only (17.6 -> 13.3 us at 64 tokens), where the
+// chain of 64 steps is the time.  4096 wide, 32 + 2 * 8 heads, library products against this kernel, us: q, k, v (three
+// launches; the rotation's own 4 to 5 come on top) 57 -> 13.3 at 64 tokens, 57 -> 21 at 200, 57 -> 30 at 500, 65 -> 51 at
+// 700, 71 -> 54 at 1000, 90 -> 94 at 1500; output 19 -> 13 at 64, 19 -> 14 at 200, 24.5 -> 22 at 500, 35.5 -> 33.6 at 1000,
+// 47 -> 54 at 1500.  Weights of that layer are 50 and 34 MB: 10 and 6.5 us at the rate of a large copy.
+#include "lds_limit.h"
+#include "rotate.h"
+#include "xattn_hip.h"
+
+namespace xattn {
+
+struct ProjParams {
+  const __bf16* x;           // [tokens][K]
+  const __bf16* w[3];        // weights, rows of K contiguous elements
+  const __bf16* bias[3];     // or null
+  __bf16* y[3];              // [tokens][features of the product]
+  int64_t w_sn[3];           // row stride, elements
+  int n[3];                  // features, multiples of 128 (0: no such product)
+  int M, K;                  // tokens, depth (a multiple of 64)
+  const __bf16* cos;         // [tokens][128]; products 0 and 1 are rotated (kRope)
+  const __bf16* sin;
+  int64_t cos_sn, sin_sn;
+};
+
+// Four wavefronts (2 x 2) take 64 * NB features x 64 * MB tokens; 64-deep slabs of both operands go straight to a ring of NS
+// LDS stages, NS - 1 steps ahead of their use, one barrier per step.  KS = 2: four more multiply the second half of each
+// slab, and the two sums of every element are added at the end.
+template <int NB, int MB, int NS, int KS, bool kRope>
+__global__ __launch_bounds__(256 * KS, 2) void proj_gemm_kernel(ProjParams p) {
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  constexpr int kN = 64 * NB, kM = 64 * MB;
+  constexpr int kStage = (kN + kM) * 128;           // bytes of one 64-deep step
+  constexpr int kSubs = 4 / KS;                     // 16-deep sub-steps of a wavefront
+  constexpr int kLoads = 2 * (NB + MB) / KS;        // KiB a wavefront copies per step: first W's, then x's
+  constexpr int kLoadsW = 2 * NB / KS, kLoadsX = 2 * MB / KS;
+  constexpr int kPer = (kLoads + kSubs - 2) / (kSubs - 1);   // ... and in each of its sub-steps but the last
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wk = wave >> 2, wn = (wave >> 1) & 1, wm = wave & 1;
+  const int r = lane & 31, hh = lane >> 5;
+
+  // Ids are dealt round-robin to the 8 XCDs; an XCD gets one contiguous run of tiles, token tiles fastest, so that the
+  // weights - most of the bytes - enter one XCD's L2 only
+  const uint32_t mt = (uint32_t)(p.M + kM - 1) / kM;
+  const uint32_t total = mt * (uint32_t)((p.n[0] + p.n[1] + p.n[2]) / kN), per_xcd = (total + 7) / 8;
+  const uint32_t lin = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if ((blockIdx.x >> 3) >= per_xcd || lin >= total) return;
+  int f0 = (int)(lin / mt) * kN, t3 = 0;
+  const int m0 = (int)(lin % mt) * kM;
+  if (kRope) {
+    if (f0 >= p.n[0]) { f0 -= p.n[0]; t3 = 1; }
+    if (t3 == 1 && f0 >= p.n[1]) { f0 -= p.n[1]; t3 = 2; }
+  }
+  // With 64 features a tile holds features 32j .. 32j + 31 of a head and their rotation partners 64 further on: 16-byte
+  // chunk c of a tile's row is chunk feature_chunk(c) of the product's
+  const int head_c = f0 / 128 * 16, j4 = f0 % 128 / 64 * 4;
+  auto feature_chunk = [&](int c) __attribute__((always_inline)) { return head_c + (NB == 2 ? c : (c & 3) + j4 + (c >> 2) * 8); };
+
+  const int64_t w_snb = p.w_sn[t3] * 2;
+  const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc((void*)(p.w[t3] + (int64_t)head_c * 8 * p.w_sn[t3]), 0, (int)(128 * w_snb), 0x00020000);
+  const int rows_left = p.M - m0;
+  const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(p.x + (int64_t)m0 * p.K), 0, (rows_left < kM ? rows_left : kM) * p.K * 2, 0x00020000);
+  // a lane's part of a copied KiB: row lane / 8 of 8, chunk lane % 8 of the slab, stored at c ^ ((row >> 1) & 7)
+  const int rl = lane >> 3, c = lane & 7;
+  uint32_t voff[kLoads];
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const bool is_w = i < kLoadsW;
+    const int row = is_w ? (wave * kLoadsW + i) * 8 + rl : (wave * kLoadsX + i - kLoadsW) * 8 + rl;
+    const int src = is_w ? (feature_chunk(row >> 3) - head_c) * 8 + (row & 7) : row;
+    voff[i] = (uint32_t)src * (uint32_t)(is_w ? w_snb : (int64_t)p.K * 2) + (uint32_t)((c ^ ((row >> 1) & 7)) << 4);
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_char_ptr)lds;
+  const int steps = p.K / 64;
+  // past the last step a copy moves nothing (its offset is outside the resource) but keeps the count of loads in flight
+  auto copy_piece = [&](int t, int st, int i) __attribute__((always_inline)) {
+    const bool is_w = i < kLoadsW;
+    const uint32_t dst = lds0 + (uint32_t)st * kStage + (is_w ? (uint32_t)(wave * kLoadsW + i) : (uint32_t)(kN / 8 + wave * kLoadsX + i - kLoadsW)) * 1024;
+    slab_copy_1k(is_w ? wres : xres, t < steps ? voff[i] + (uint32_t)t * 128 : 0xffffffffu, dst);
+  };
+  f32x16 acc[NB][MB];
+#pragma unroll
+  for (int a = 0; a < NB; ++a)
+#pragma unroll
+    for (int b = 0; b < MB; ++b)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.f;
+  const int sw = (r >> 1) & 7;
+  bf16x8 fa[2][NB], fb[2][MB];
+  auto read = [&](int st, int s, int buf) __attribute__((always_inline)) {
+    const char* at = lds + st * kStage + r * 128 + (((2 * (s + wk * kSubs) + hh) ^ sw) << 4);
+#pragma unroll
+    for (int a = 0; a < NB; ++a) fa[buf][a] = *reinterpret_cast<const bf16x8*>(at + (wn * NB + a) * 4096);
+#pragma unroll
+    for (int b = 0; b < MB; ++b) fb[buf][b] = *reinterpret_cast<const bf16x8*>(at + kN * 128 + (wm * MB + b) * 4096);
+  };
+#pragma unroll
+  for (int t = 0; t < NS - 1; ++t)
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) copy_piece(t, t, i);
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 2) * kLoads) : "memory");
+  read(0, 0, 0);
+  // A step is four sub-steps of NB * MB MFMAs; the fragments of the next sub-step and the copies of step t + NS - 1 are
+  // issued between them.  The barrier sits before the last sub-step's MFMAs: by then this wavefront has read every
+  // fragment of step t and its copies of step t + 1 have landed, so behind it step t + 1 may be read and step t's stage
+  // refilled.
+  int st = 0;
+  for (int t = 0; t < steps; ++t) {
+    const int next = st + 1 == NS ? 0 : st + 1, fill = st == 0 ? NS - 1 : st - 1;
+#pragma unroll
+    for (int s = 0; s < kSubs; ++s) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (s == kSubs - 1) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * kLoads) : "memory");
+        read(next, 0, 0);     // (a repeat of old data behind the last step)
+      } else {
+        read(st, s + 1, (s + 1) & 1);
+#pragma unroll
+        for (int i = s * kPer; i < kLoads && i < (s + 1) * kPer; ++i) copy_piece(t + NS - 1, fill, i);
+      }
+#pragma unroll
+      for (int a = 0; a < NB; ++a)
+#pragma unroll
+        for (int b = 0; b < MB; ++b) acc[a][b] = mfma32(fa[s & 1][a], fb[s & 1][b], acc[a][b]);
+    }
+    st = next;
+  }
+  // every copy has landed and every fragment has been read: the LDS takes the tile, token-major, chunk c of token m at
+  // c ^ (m & (chunks - 1))
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  constexpr int kChunks = 8 * NB;
+  char* const tile = lds + (KS - 1) * 4 * NB * MB * 4096;
+  if (KS == 2) {
+    f32x4* const half = reinterpret_cast<f32x4*>(lds + (wave & 3) * NB * MB * 4096) + lane;
+#pragma unroll
+    for (int i = 0; i < NB * MB * 4; ++i) {
+      f32x16& x = acc[i / 4 / MB][i / 4 % MB];
+      if (wk == 1) half[i * 64] = f32x4{x[i % 4 * 4], x[i % 4 * 4 + 1], x[i % 4 * 4 + 2], x[i % 4 * 4 + 3]};
+    }
+    __syncthreads();
+    if (wk == 0) {
+#pragma unroll
+      for (int i = 0; i < NB * MB * 4; ++i) {
+        f32x16& x = acc[i / 4 / MB][i / 4 % MB];
+        const f32x4 o = half[i * 64];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[i % 4 * 4 + u] += o[u];
+      }
+    }
+  }
+#pragma unroll
+  for (int a = 0; a < NB; ++a)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      if (wk) continue;
+      const int ch = (wn * NB + a) * 4 + g;          // features 8 ch + 4 hh .. + 3 of the tile
+      float bs[4] = {0.f, 0.f, 0.f, 0.f};
+      if (p.bias[t3]) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) bs[u] = (float)p.bias[t3][feature_chunk(ch) * 8 + hh * 4 + u];
+      }
+#pragma unroll
+      for (int b = 0; b < MB; ++b) {
+        const int m = (wm * MB + b) * 32 + r;
+        u32x2 o;
+        o[0] = pack_bf16(acc[a][b][g * 4 + 0] + bs[0], acc[a][b][g * 4 + 1] + bs[1]);
+        o[1] = pack_bf16(acc[a][b][g * 4 + 2] + bs[2], acc[a][b][g * 4 + 3] + bs[3]);
+        *reinterpret_cast<u32x2*>(tile + m * (kN * 2) + ((ch ^ (m & (kChunks - 1))) << 4) + hh * 8) = o;
+      }
+    }
+  __syncthreads();
+  // chunk pairs (rotation partners): kChunks / 2 lanes write a token's
+  constexpr int kPairs = kChunks / 2;
+  __bf16* const y = p.y[t3];
+  const int64_t y_sn = p.n[t3];
+#pragma unroll
+  for (int i = 0; i < (kM * kPairs + 256 * KS - 1) / (256 * KS); ++i) {
+    const int m = (i * 256 * KS + tid) / kPairs, ch = tid % kPairs;
+    if (m >= kM || m >= rows_left) break;
+    const char* row = tile + m * (kN * 2);
+    bf16x8 y0 = *reinterpret_cast<const bf16x8*>(row + ((ch ^ (m & (kChunks - 1))) << 4));
+    bf16x8 y1 = *reinterpret_cast<const bf16x8*>(row + (((ch + kPairs) ^ (m & (kChunks - 1))) << 4));
+    const int f = feature_chunk(ch) * 8;             // its partner's is 64 further on
+    if (kRope && t3 < 2) rotate_chunks(y0, y1, p.cos + (int64_t)(m0 + m) * p.cos_sn + f % 128, p.sin + (int64_t)(m0 + m) * p.sin_sn + f % 128);
+    __bf16* const at = y + (int64_t)(m0 + m) * y_sn + f;
+    *reinterpret_cast<bf16x8*>(at) = y0;
+    *reinterpret_cast<bf16x8*>(at + 64) = y1;
+  }
+}
+
+}  // namespace xattn
+
+using namespace xattn;
+
+namespace {
+bool a16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+// The tile for `features` features of `tokens` tokens (see the head of the file), or none: the products are large enough
+// for the library.  Past 256 tiles of 128 x 128 only the three products of q, k and v gain from being one launch.
+enum Tile { kNone, k64x64, k128x64, k128x128, k128x128Twice };
+Tile tile_for(int64_t tokens, int64_t features, bool qkv) {
+  const int64_t m64 = (tokens + 63) / 64, m128 = (tokens + 127) / 128;
+  if (features / 64 * m64 <= 256) return k64x64;
+  if (features / 128 * m64 <= 256) return k128x64;
+  if (features / 128 * m128 <= 256) return k128x128;
+  return qkv && features / 128 * m128 <= 512 ? k128x128Twice : kNone;
+}
+
+template <int NB, int MB, int NS, int KS, bool kRope>
+int launch(const ProjParams& p, hipStream_t s) {
+  constexpr int kLds = (NB + MB) * 64 * 128 * NS;
+  static LdsLimit limit;
+  if (limit.raise((const void*)proj_gemm_kernel<NB, MB, NS, KS, kRope>) != hipSuccess) return XATTN_ERR_LAUNCH;
+  const unsigned tiles = (unsigned)((p.M + 64 * MB - 1) / (64 * MB)) * (unsigned)((p.n[0] + p.n[1] + p.n[2]) / (64 * NB));
+  hipLaunchKernelGGL((proj_gemm_kernel<NB, MB, NS, KS, kRope>), dim3((tiles + 7) / 8 * 8), dim3(256 * KS), kLds, s, p);
+  return hipGetLastError() == hipSuccess ? XATTN_OK : XATTN_ERR_LAUNCH;
+}
+
+// offsets inside a tile are held in 32 bits
+bool shape_ok(int tokens, int width) { return tokens > 0 && width >= 64 && width % 64 == 0 && width <= 65536; }
+bool stride_ok(int64_t sn, int width) { return sn >= width && sn <= ((int64_t)1 << 22); }
+
+template <bool kRope>
+int run(const ProjParams& p, void* stream) {
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  switch (tile_for(p.M, (int64_t)p.n[0] + p.n[1] + p.n[2], kRope)) {
+    case k64x64: return launch<1, 1, 6, 2, kRope>(p, s);
+    case k128x64: return launch<2, 1, 4, 1, kRope>(p, s);
+    case k128x128: return launch<2, 2, 4, 1, kRope>(p, s);
+    case k128x128Twice: return launch<2, 2, 2, 1, kRope>(p, s);
+    default: return XATTN_ERR_SHAPE;
+  }
+}
+}  // namespace
+
+extern "C" int xattn_proj_gemm_fits(int tokens, int width, int features, int qkv) {
+  return shape_ok(tokens, width) && features >= 128 && features % 128 == 0 && tile_for(tokens, features, qkv != 0) != kNone;
+}
+
+extern "C" int xattn_qkv_rope_gemm(const void* x, int tokens, int width, const void* wq, int64_t wq_stride, const void* bq,
+                                   const void* wk, int64_t wk_stride, const void* bk, const void* wv, int64_t wv_stride,
+                                   const void* bv, const void* cos, const void* sin, int64_t cos_stride, int64_t sin_stride,
+                                   void* q, void* k, void* v, int num_heads, int num_kv_heads, int head_dim, void* stream) {
+  if (!x || !wq || !wk || !wv || !cos || !sin || !q || !k || !v) return XATTN_ERR_NULL;
+  if (head_dim != kHeadDim) return XATTN_ERR_HEAD_DIM;
+  if (num_heads <= 0 || num_kv_heads <= 0 || num_heads > 4096 || num_kv_heads > 4096) return XATTN_ERR_HEADS;
+  if (!shape_ok(tokens, width) || !stride_ok(wq_stride, width) || !stride_ok(wk_stride, width) || !stride_ok(wv_stride, width) ||
+      cos_stride < 0 || sin_stride < 0)
+    return XATTN_ERR_SHAPE;
+  if (wq_stride % 8 || wk_stride % 8 || wv_stride % 8 || cos_stride % 8 || sin_stride % 8) return XATTN_ERR_ALIGN;
+  for (const void* a : {x, wq, wk, wv, cos, sin, (const void*)q, (const void*)k, (const void*)v})
+    if (!a16(a)) return XATTN_ERR_ALIGN;
+  ProjParams p{};
+  p.x = static_cast<const __bf16*>(x);
+  const void *w[3] = {wq, wk, wv}, *b[3] = {bq, bk, bv};
+  void* y[3] = {q, k, v};
+  const int64_t sn[3] = {wq_stride, wk_stride, wv_stride};
+  const int n[3] = {num_heads, num_kv_heads, num_kv_heads};
+  for (int i = 0; i < 3; ++i) {
+    p.w[i] = static_cast<const __bf16*>(w[i]);
+    p.bias[i] = static_cast<const __bf16*>(b[i]);
+    p.y[i] = static_cast<__bf16*>(y[i]);
+    p.w_sn[i] = sn[i];
+    p.n[i] = n[i] * kHeadDim;
+  }
+  p.M = tokens;
+  p.K = width;
+  p.cos = static_cast<const __bf16*>(cos);
+  p.sin = static_cast<const __bf16*>(sin);
+  p.cos_sn = cos_stride;
+  p.sin_sn = sin_stride;
+  return run<true>(p, stream);
+}
+
+extern "C" int xattn_gemm(const void* x, int tokens, int width, const void* w, int64_t w_stride, const void* bias, void* y,
+                          int features, void* stream) {
+  if (!x || !w || !y) return XATTN_ERR_NULL;
+  if (!shape_ok(tokens, width) || !stride_ok(w_stride, width) || features < 128 || features % 128) return XATTN_ERR_SHAPE;
+  if (w_stride % 8 || !a16(x) || !a16(w) || !a16(y)) return XATTN_ERR_ALIGN;
+  ProjParams p{};
+  p.x = static_cast<const __bf16*>(x);
+  p.w[0] = static_cast<const __bf16*>(w);
+  p.bias[0] = static_cast<const __bf16*>(bias);
+  p.y[0] = static_cast<__bf16*>(y);
+  p.w_sn[0] = w_stride;
+  p.n[0] = features;
+  p.M = tokens;
+  p.K = width;
+  return run<false>(p, stream);
+}

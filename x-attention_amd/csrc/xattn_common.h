@@ -70,4 +70,11 @@ __device__ __forceinline__ float half_max(float x) {
   return fmaxf(lo, hi);
 }
 
+typedef __attribute__((address_space(3))) char* lds_char_ptr;
+
+// one KiB of a slab of rows of 128 bytes (8 of them), global -> LDS; the caller counts it in vmcnt
+__device__ __forceinline__ void slab_copy_1k(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t dst) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(dst), "v"(voff), "s"(rsrc) : "memory", "m0");
+}
+
 }  // namespace xattn

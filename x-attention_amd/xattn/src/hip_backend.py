@@ -66,6 +66,12 @@ _SIGNATURES = {
         [c_vp, c_i32] + [c_vp, c_i64, c_vp] * 3 + [c_vp] * 5 + [c_i32] * 3 + [c_vp],
     ),
     "xattn_gemv": (c_i32, [c_vp, c_i32, c_vp, c_i64, c_vp, c_vp, c_i32, c_vp]),
+    "xattn_proj_gemm_fits": (c_i32, [c_i32] * 4),
+    "xattn_qkv_rope_gemm": (
+        c_i32,
+        [c_vp, c_i32, c_i32] + [c_vp, c_i64, c_vp] * 3 + [c_vp] * 2 + [c_i64] * 2 + [c_vp] * 3 + [c_i32] * 3 + [c_vp],
+    ),
+    "xattn_gemm": (c_i32, [c_vp, c_i32, c_i32, c_vp, c_i64, c_vp, c_vp, c_i32, c_vp]),
     "xattn_rope": (c_i32, [c_vp] * 4 + [c_i64] * 2 + [c_i32] * 4 + [c_vp]),
     "xattn_block_sparse_workspace_bytes": (c_sz, [c_i32] * 5),
     "xattn_block_sparse_fwd_ws": (

@@ -114,8 +114,8 @@ def _linear_params(mod):
 
 
 def _project(self, hidden_states, cos, sin, heads, kv_heads):
-    """Rotated q and k and v of a layer from the native host path (one kernel for one token, the library GEMMs and one
-    rotation kernel for more), or None where the layer's own modules have to be called."""
+    """Rotated q and k and v of a layer from the native host path (one kernel up to about a thousand tokens, the library
+    GEMMs and one rotation kernel for more), or None where the layer's own modules have to be called."""
     if not hidden_states.is_cuda or self.head_dim != 128:
         return None
     q, k, v = _linear_params(self.q_proj), _linear_params(self.k_proj), _linear_params(self.v_proj)
@@ -216,7 +216,7 @@ def forward_eval(self, hidden_states, position_embeddings=None, attention_mask=N
             f"`attn_output` should be of size {(bsz, heads, q_len, head_dim)}, but is {attn_output.size()}"
         )
     attn_output = attn_output.transpose(1, 2).reshape(bsz, q_len, heads * head_dim)
-    out_proj = _linear_params(self.o_proj) if q_len == 1 and attn_output.is_cuda else None
+    out_proj = _linear_params(self.o_proj) if attn_output.is_cuda else None
     projected = _hb.host().output(attn_output, *out_proj) if out_proj is not None else None
     attn_output = projected if projected is not None else self.o_proj(attn_output)
     _stamp(cfg, "Post-attention processing", start)
