@@ -24,6 +24,12 @@ pytestmark = pytest.mark.gpu
     (2048, 30000, 32, 8, 16, 2048, True),
     (700, 0, 8, 8, 8, 1024, False),
     (100, 3000, 32, 8, 8, 128, False),
+    # rows of several heads packed into large tiles: whole quarters, 64-row pieces of 7 heads with two left empty, a ragged
+    # last piece, no causality
+    (2048, 60000, 32, 8, 16, 2048, True),
+    (1500, 18000, 28, 4, 8, 2048, True),
+    (5000, 30000, 32, 8, 16, 2048, True),
+    (1900, 60001, 32, 8, 16, 4096, False),
 ])
 @pytest.mark.parametrize("use_triton", [True, False])
 def test_same_bits_as_the_large_tiles(q_len, cache, heads, kv_heads, stride, chunk, causal, use_triton):

@@ -41,6 +41,8 @@ struct EstParams {
   // estimate_small_kernel: a tile's rows are tile_rows rows of each of pack heads of one KV group
   unsigned long long* noted;   // set to zero for the selection pass that follows (AttnPlan::head), or null
   int pack, tile_rows, tile_shift;   // powers of two, tile_rows = 1 << tile_shift
+  // estimate_gemm_kernel with packed rows: quarters of 64 rows per head, 256-row tiles per KV group, first key tile, key tiles
+  int quarters, group_tiles, first_key_tile, key_tiles;
 };
 
 // first / last visible reshaped key of reshaped query row m
