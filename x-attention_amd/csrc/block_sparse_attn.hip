@@ -52,7 +52,6 @@ struct AttnParams {
   float scale_log2;         // softmax_scale * log2(e)
   DispatchShape shape;      // dispatch_shape(H, Hkv), computed on the host
   AttnPlan plan;            // kPlanned only
-  int piece_grid;           // workgroups ahead of the units', for the pieces of cut lists (a multiple of 8)
 };
 
 __device__ __forceinline__ int clamp_block(int kb, int nkb) { return kb < 0 ? 0 : (kb < nkb ? kb : nkb - 1); }
@@ -250,8 +249,8 @@ __device__ __forceinline__ void store_out(const AttnParams& p, int head, int qb,
   }
 }
 
-// What an item of a cut list leaves behind: accumulators as the lanes hold them (1 KiB per store), row maxima and sums.
-// Items of a list run on any XCD, each with an L2 of its own: stores and loads are at device scope (kDeviceScope: they go
+// What a piece of a cut list leaves behind: accumulators as the lanes hold them (1 KiB per store), row maxima and sums.
+// Pieces of a list run on any XCD, each with an L2 of its own: stores and loads are at device scope (kDeviceScope: they go
 // through to, and come from, memory that all of them share).
 constexpr int kDeviceScope = 16;   // sc1
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t part_resource(float* part) {
@@ -277,7 +276,7 @@ __device__ __forceinline__ void store_partial(float* part, int wave, int lane, i
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, l_tot), res, at + 512, 0, kDeviceScope);
   }
 }
-// The items' results combined into the registers of a finished sweep, in the order of the list.
+// The pieces' results combined into the registers of a finished sweep, in the order of the list.
 __device__ __forceinline__ void load_partials(float* part, int items, int wave, int lane, int r, int hh, f32x16 (&oacc)[4], float& l_run) {
   const int at = (128 * 128 + wave * 32 + r) * 4;
   auto ml = [&](int s, int which) __attribute__((always_inline)) {
@@ -320,23 +319,24 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
   const int r = lane & 31, hh = lane >> 5;
 
   int head, qb, kvh;
-  bool is_piece = false;
-  int index = 0;                     // which piece of its list a workgroup ahead of the units' has
-  if (kPlanned && (int)blockIdx.x < p.piece_grid) {
+  int piece = -1;                    // which piece of its list a workgroup has, if any
+  int skip = 0;                      // workgroups ahead of the units'
+  if (kPlanned) {
     // an XCD gets a run of adjacent pieces, which are of adjacent lists
     const int pieces = ((const_i32_ptr)(uintptr_t)p.plan.head)[0], per_xcd = (pieces + 7) / 8;
-    const int at = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= per_xcd || at >= pieces) return;
-    const_i32_ptr entry = (const_i32_ptr)(uintptr_t)p.plan.pieces + 2 * at;
-    const int unit = entry[0];
-    index = entry[1];
-    is_piece = true;
-    head = unit / p.idx_rows;
-    qb = unit - head * p.idx_rows + p.idx_row0;
-    kvh = head / p.shape.group;
-  } else if (!map_workgroup((int)blockIdx.x - (kPlanned ? p.piece_grid : 0), p.shape, p.qb_begin, p.qb_end, &head, &qb, &kvh)) {
-    return;
+    skip = per_xcd * 8;
+    if ((int)blockIdx.x < skip) {
+      const int at = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+      if (at >= pieces) return;
+      const_i32_ptr entry = (const_i32_ptr)(uintptr_t)p.plan.pieces + 2 * at;
+      const int unit = entry[0];
+      piece = entry[1];
+      head = unit / p.idx_rows;
+      qb = unit - head * p.idx_rows + p.idx_row0;
+      kvh = head / p.shape.group;
+    }
   }
+  if (piece < 0 && !map_workgroup((int)blockIdx.x - skip, p.shape, p.qb_begin, p.qb_end, &head, &qb, &kvh)) return;
   const __bf16* qbase = p.q + (int64_t)head * p.q_sh;
   const __bf16* kbase = p.k + (int64_t)kvh * p.k_sh;
   const __bf16* vbase = p.v + (int64_t)kvh * p.v_sh;
@@ -347,7 +347,7 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
   // the column list is read through the scalar cache (uniform, read-only), so that
   // fetching the next block id never waits on the tile copies in flight
   const_i32_ptr list = nullptr;
-  int cuts = 0, number = 0;          // pieces taken off this list, its number in the plan
+  int cuts = 0, number = 0;          // pieces of this list, its number in the plan
   {
     const int q_last = (qb * kBlk + kBlk - 1 < p.Lq ? qb * kBlk + kBlk - 1 : p.Lq - 1) + p.kv_off;
     int visible = p.causal ? (q_last < 0 ? 0 : q_last / kBlk + 1) : p.nkb;
@@ -362,14 +362,14 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
       n_blocks = visible;
     }
     if (kPlanned) {
-      cuts = piece_count(n_blocks, p.plan.items);
+      cuts = piece_count(n_blocks, p.plan);
       if (cuts > 0) {
-        const int piece = piece_length(n_blocks, p.plan.items);
+        if (piece < 0) return;           // others have it
+        const int length = piece_length(n_blocks, p.plan);
         number = ((const_i32_ptr)(uintptr_t)p.plan.number)[slot];
-        if (!is_piece) index = cuts;
-        if (kHasList) list += index * piece;
-        else first = index * piece;
-        n_blocks = is_piece ? piece : n_blocks - cuts * piece;
+        if (kHasList) list += piece * length;
+        else first = piece * length;
+        n_blocks = piece + 1 < cuts ? length : n_blocks - piece * length;
       }
       if (kHasList) first = list[0];
     }
@@ -430,15 +430,15 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
   // the last barrier of the sweep (or the one before it, for an empty list) left both tiles unused
   if (kPlanned && cuts > 0) {
     float* const part = p.plan.part + (int64_t)number * p.plan.items * kPartFloats;
-    store_partial(part + (int64_t)index * kPartFloats, wave, lane, r, hh, oacc, m_run, l_run);
+    store_partial(part + (int64_t)piece * kPartFloats, wave, lane, r, hh, oacc, m_run, l_run);
     wait_vm0();                              // written through to memory
     __syncthreads();
     int* const scratch = reinterpret_cast<int*>(Ks);
     if (tid == 0) scratch[0] = __hip_atomic_fetch_add(p.plan.done + number, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
-    if (scratch[0] != cuts) return;          // the item that comes last combines them
+    if (scratch[0] != cuts - 1) return;      // the piece that comes last combines them
     __syncthreads();
-    load_partials(part, cuts + 1, wave, lane, r, hh, oacc, l_run);
+    load_partials(part, cuts, wave, lane, r, hh, oacc, l_run);
   }
   store_out(p, head, qb, wave, lane, r, hh, oacc, l_run, Ks + wave * 8192);
 }
@@ -523,12 +523,11 @@ int xattn::block_sparse_impl(const void* q, const void* k, const void* v, void* 
   if (grid > 0x7fffffff) return XATTN_ERR_SHAPE;
   hipStream_t s = static_cast<hipStream_t>(stream);
   p.plan = AttnPlan{};
-  p.piece_grid = 0;
   if (plan) {
     p.plan = *plan;
-    p.piece_grid = (int)(((int64_t)p.H * (q_block_end - q_block_begin) * (plan->items - 1) + 7) / 8 * 8);
-    if (grid + p.piece_grid > 0x7fffffff) return XATTN_ERR_SHAPE;
-    const dim3 wgs((unsigned)(grid + p.piece_grid));
+    const int64_t most = ((int64_t)p.H * (q_block_end - q_block_begin) * plan->items + 7) / 8 * 8;
+    if (grid + most > 0x7fffffff) return XATTN_ERR_SHAPE;
+    const dim3 wgs((unsigned)(grid + most));
     if (note) hipLaunchKernelGGL(note_lists_kernel, dim3(1), dim3(1024), 0, s, p);
     if (col_idx)
       hipLaunchKernelGGL((block_sparse_fwd_kernel<true, true>), wgs, dim3(256), 0, s, p);
@@ -584,7 +583,7 @@ extern "C" int xattn_block_sparse_fwd_ws(const void* q, const void* k, const voi
     if (!workspace) return XATTN_ERR_NULL;
     if (workspace_bytes < need) return XATTN_ERR_WORKSPACE;
     if (reinterpret_cast<uintptr_t>(workspace) & 255) return XATTN_ERR_ALIGN;
-    plan = plan_at(static_cast<char*>(workspace), (int64_t)num_heads * idx_rows, (int64_t)num_heads * q_blocks, items_of(num_heads, q_len, k_len));
+    plan = plan_at(static_cast<char*>(workspace), (int64_t)num_heads * idx_rows, (int64_t)num_heads * q_blocks, items_of(num_heads, q_len, k_len), (k_len + kBlk - 1) / kBlk);
   }
   return block_sparse_impl(q, k, v, out, col_idx, col_cnt, idx_pitch, idx_rows, idx_row0, num_heads, num_kv_heads, q_len, k_len,
                            head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n, o_stride_h,

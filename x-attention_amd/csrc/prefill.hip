@@ -71,13 +71,13 @@ extern "C" int xattn_prefill_fwd(const void* q, const void* k, const void* v, vo
   sel.real_q_blocks_only = 1;
   sel.stages = 3;
   const int64_t units = (int64_t)num_heads * l.nqb;
-  const AttnPlan plan = plan_at(ws + l.plan_off, units, units, l.items);
+  const AttnPlan plan = plan_at(ws + l.plan_off, units, units, l.items, l.nkb);
   // (with zero_rows_from 0 no row is estimated, and no MFMA pass would clear the plan's head: noted afterwards)
   // Where no list can be long enough to be cut, nothing is noted (nor planned below): then the selection may follow the
   // estimate in the same kernel.
   const int q_chunks = (int)(((int64_t)q_len + chunk_size - 1) / chunk_size), k_chunks = (int)(((int64_t)k_len + chunk_size - 1) / chunk_size);
   const int64_t last_token = (int64_t)l.nqb * 128 - 1 + (int64_t)(k_chunks - q_chunks) * chunk_size;   // on the key axis, both padded
-  const bool may_cut = plan.items && (!causal || keep_sink || last_token / 128 + 1 > kMinPiece);
+  const bool may_cut = plan.items && (!causal || keep_sink || last_token / 128 + 1 > plan.min_piece);
   if (may_cut && zero_rows_from != 0) sel.plan = &plan;
   int rc = estimate_impl(q, k, nullptr, ws, l.est_bytes, nullptr, num_heads, num_kv_heads, q_len, k_len, head_dim,
                          q_stride_h, q_stride_n, k_stride_h, k_stride_n, stride, 128, chunk_size, 0, q_chunks, causal,
