@@ -27,16 +27,18 @@ struct AttnPlan {
   int min_piece;              // blocks of the shortest
 };
 
-// Items a list may be cut into, for a problem of `units` lists (heads x q-blocks) over nkb key blocks; 1: never.  The
-// launch has units * (items - 1) workgroups for pieces, and where lists are short they cost 1.5 - 2 us per thousand: up to
-// 2048 for a prompt by itself (whole call at 4096 tokens, us: uneven lists 125 -> 109, even ones 67.5 -> 68), up to 8192 on
-// top of a cache at least as long as the chunk, where lists are long and few (2048 tokens on 63488: 1426 -> 881 with
-// 8192, 1005 with 2048; 64 on 100000: 1461 -> 334; 8000 on 100000: 3865 -> 2765).  16 key blocks or fewer make short lists.
+// Pieces a list may be cut into, for a problem of `units` lists (heads x q-blocks) over nkb key blocks; 1: never.  The
+// launch has units * pieces workgroups for them, and where lists are short the spare ones cost 1 - 2 us per thousand: for a
+// prompt by itself about 2048 beside the units, and two pieces up to 4096 units (whole calls, us, uneven lists: 4096 tokens
+// 125 uncut, 92 cut; 16000 tokens 679 and 497 uncut, 652 and 478 in two; 32768 tokens 2158 uncut, 2781 in two - partial
+// results and the spread of a KV head over the chip cost more than the end of a long launch).  On top of a cache at least
+// as long as the chunk, where lists are long and few, 8192 (2048 tokens on 63488: 1426 uncut, 881 with 8192, 1005 with 2048;
+// 64 on 100000: 1461 and 334; 8000 on 100000: 3865 and 2765).  16 key blocks or fewer make short lists.
 inline int plan_items(int64_t units, int nqb, int nkb) {
-  const int64_t most = nkb >= 2 * nqb ? 8192 : 2048;
-  if (nkb <= 16 || units > most) return 1;
-  const int64_t n = most / units + 1;
-  return n > 16 ? 16 : (int)n;
+  const bool cached = nkb >= 2 * nqb;
+  if (nkb <= 16 || units > (cached ? 8192 : 4096)) return 1;
+  const int64_t n = (cached ? 8192 : 2048) / units + 1;
+  return n > 16 ? 16 : n < 2 ? 2 : (int)n;
 }
 // A piece costs about 7 us beside its blocks (first tiles, partial result, its part of the combination), so it is not made
 // short where lists are long; where keys are few the longest list still bounds the launch.  Whole calls with pieces of at
