@@ -30,6 +30,11 @@ pytestmark = pytest.mark.gpu
     (1500, 18000, 28, 4, 8, 2048, True),
     (5000, 30000, 32, 8, 16, 2048, True),
     (1900, 60001, 32, 8, 16, 4096, False),
+    # half tiles behind whole rounds: what does not fill a round, a last row tile of one half, both, no causality
+    (32768, 0, 30, 10, 16, 2048, True),
+    (15000, 0, 32, 8, 8, 2048, True),
+    (10500, 0, 28, 4, 8, 1024, True),
+    (18000, 0, 28, 4, 16, 1024, False),
 ])
 @pytest.mark.parametrize("use_triton", [True, False])
 def test_same_bits_as_the_large_tiles(q_len, cache, heads, kv_heads, stride, chunk, causal, use_triton):

@@ -89,10 +89,8 @@ struct TileCursor {
   int row_base = 0;    // (row, key tile) pairs of the group before that row
 };
 
-__device__ __forceinline__ bool decode_tile(const EstParams& p, int64_t id, TileCursor& c, int* head, int* m0, int* n0) {
-  const int64_t lin64 = ((id >> 8) * 8 + (id & 7)) * 32 + ((id >> 3) & 31);
-  if (lin64 >= p.total_tiles) return false;
-  const uint32_t lin = (uint32_t)lin64;                  // the host refuses launches of 2^31 tiles or more
+__device__ __forceinline__ int64_t place_of(int64_t id) { return ((id >> 8) * 8 + (id & 7)) * 32 + ((id >> 3) & 31); }
+__device__ __forceinline__ void decode_place(const EstParams& p, uint32_t lin, TileCursor& c, int* head, int* m0, int* n0) {
   const uint32_t G = (uint32_t)(p.H / p.Hkv);
   const uint32_t per_group = (uint32_t)p.tiles_per_head * G;
   const uint32_t g = lin / per_group;
@@ -118,6 +116,11 @@ __device__ __forceinline__ bool decode_tile(const EstParams& p, int64_t id, Tile
   }
   *m0 = p.row_begin + c.mt_row * kTile;
   *n0 = (nt_first + (tt - c.row_base)) * kTile;
+}
+__device__ __forceinline__ bool decode_tile(const EstParams& p, int64_t id, TileCursor& c, int* head, int* m0, int* n0) {
+  const int64_t lin = place_of(id);
+  if (lin >= p.total_tiles) return false;
+  decode_place(p, (uint32_t)lin, c, head, m0, n0);       // the host refuses launches of 2^31 tiles or more
   return true;
 }
 
@@ -137,7 +140,7 @@ __device__ __forceinline__ Quarter tile_quarter(const EstParams& p, int group, i
 }
 // head and m0 come out as KV group and row tile; row tiles of a key tile follow each other (they share its K' slabs)
 __device__ __forceinline__ bool decode_packed(const EstParams& p, int64_t id, int* group, int* row_tile, int* n0) {
-  const int64_t lin64 = ((id >> 8) * 8 + (id & 7)) * 32 + ((id >> 3) & 31);
+  const int64_t lin64 = place_of(id);
   if (lin64 >= p.total_tiles) return false;
   const uint32_t lin = (uint32_t)lin64, per_group = (uint32_t)(p.group_tiles * p.key_tiles);
   const uint32_t g = lin / per_group, rem = lin - g * per_group;
@@ -147,9 +150,30 @@ __device__ __forceinline__ bool decode_packed(const EstParams& p, int64_t id, in
   return true;
 }
 
+// Half tiles: a launch of few rounds loses much of its last one when that is not full, and a last row tile may have 128 rows
+// or fewer.  Behind a launch of a whole number of rounds of whole tiles a second one takes the rest as halves of 128 rows,
+// 0.65 of a whole tile's time each (a wavefront then has 32 rows: five fragments for four MFMAs instead of six for eight).
+// (Both in one launch: the accumulators meet behind two k-loops, and 85 registers were spilled.)  15000 tokens, stride 8: 146 -> 138 us; 10500 with 28 heads 92 -> 85.
+__device__ __forceinline__ bool decode_half(const EstParams& p, int64_t id, TileCursor& c, int* head, int* m0, int* n0) {
+  const int64_t lin64 = place_of(id);
+  if (lin64 >= p.total_tiles) return false;
+  const uint32_t lin = (uint32_t)lin64, split = (uint32_t)p.split_tiles;
+  if (lin < 2 * split) {
+    decode_place(p, (uint32_t)p.whole_tiles + lin / 2, c, head, m0, n0);
+    *m0 += (int)(lin & 1) * (kTile / 2);
+    return true;
+  }
+  const uint32_t G = (uint32_t)(p.H / p.Hkv), per_group = (uint32_t)p.last_row_tiles * G;
+  const uint32_t at = lin - 2 * split, g = at / per_group, rem = at - g * per_group;
+  *head = (int)(g * G + rem % G);
+  *m0 = p.row_begin + p.nMT * kTile;
+  *n0 = (p.first_key_tile + (int)(rem / G)) * kTile;
+  return true;
+}
+
 // kDump: also write the raw scores (test / seam builds only; kept out of the production instantiation)
 // kTable: the depth slabs come from p.pairs (the non-default select modes); the default keeps its closed form
-template <int RBS, bool kDump, bool kTable, bool kPacked>
+template <int RBS, bool kDump, bool kTable, bool kPacked, bool kHalf>
 __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
 
@@ -157,6 +181,7 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 31, hh = lane >> 5;
   const int wm = wave & 3, wn = wave >> 2;   // query quarter, key half
+  constexpr int kMT = kHalf ? 1 : 2;         // 32-row query tiles of a wavefront
   if (blockIdx.x == 0 && tid == 0 && p.noted) *p.noted = 0;
   // A workgroup works through tiles id, id + grid, ...: one workgroup fits a CU, so nothing else could hide
   // the wait for a tile's first slabs.  The slab pipeline therefore runs on across the tile boundary: the load
@@ -167,7 +192,7 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
   TileCursor cursor;
   // kPacked: head and m0 are the tile's KV group and its row tile of the group
   auto decode = [&](int64_t i, int* h, int* m, int* n) {
-    return kPacked ? decode_packed(p, i, h, m, n) : decode_tile(p, i, cursor, h, m, n);
+    return kPacked ? decode_packed(p, i, h, m, n) : kHalf ? decode_half(p, i, cursor, h, m, n) : decode_tile(p, i, cursor, h, m, n);
   };
   if (!decode(id, &head, &m0, &n0)) return;
 
@@ -177,8 +202,8 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
   // sequence end (or the tile's end), so lane offsets stay small whatever the
   // token stride, and tokens past the real length read as zeros.
   auto q_resource = [&](int h, int m) {
-    const int64_t tok0 = (int64_t)m * p.S * p.kdb, left = p.Lq - tok0;
-    const int64_t rows = left < 0 ? 0 : (left < span * p.kdb ? left : span * p.kdb);
+    const int64_t tok0 = (int64_t)m * p.S * p.kdb, left = p.Lq - tok0, most = span * p.kdb / (kHalf ? 2 : 1);
+    const int64_t rows = left < 0 ? 0 : (left < most ? left : most);
     return __builtin_amdgcn_make_buffer_rsrc((void*)(p.q + (int64_t)h * p.q_sh + (rows > 0 ? tok0 * p.q_sn : 0)), 0,
                                              (int)(rows * q_snb), 0x00020000);
   };
@@ -267,11 +292,11 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
 #pragma unroll
   for (int j = 0; j < 8; ++j) load_j(j, 1);
   lds_barrier();
-  bf16x8 fa[2][4], fb[2][2];
+  bf16x8 fa[2][4], fb[2][kMT];
 #pragma unroll
   for (int x = 0; x < 4; ++x) fa[0][x] = read_frag(lds, wn * kSub + x * 32 + r, hh);
 #pragma unroll
-  for (int x = 0; x < 2; ++x) fb[0][x] = read_frag(lds + kTile * 128, wm * kRowsW + x * 32 + r, hh);
+  for (int x = 0; x < kMT; ++x) fb[0][x] = read_frag(lds + kTile * 128, wm * 32 * kMT + x * 32 + r, hh);
 
   for (;;) {
   const int64_t id_next = id + gridDim.x;
@@ -281,11 +306,11 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
     q_resources(qres_next, head_next, m0_next);
     kres_next = k_resource(head_next, n0_next);
   }
-  f32x16 acc[4][2];   // [key tile nt][query tile mt]
+  f32x16 acc[4][kMT];   // [key tile nt][query tile mt]
 #pragma unroll
   for (int a = 0; a < 4; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < kMT; ++b)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.f;
 
@@ -309,7 +334,8 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
         {
           // pieces 0..2 | 3..5 | 6..7 of step t+1 go to the other stage; their registers then take step t+2
           const int j = ss * 3 + c;
-          if (ss < 3 && c < 3 && j < 8) {
+          // (half tiles have no rows for the odd pieces from 5 on)
+          if (ss < 3 && c < 3 && j < 8 && !(kHalf && (j & 1) && j >= 5)) {
             write_j(j, nxt);
             load_j(j, t + 2);
           }
@@ -318,11 +344,11 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
           fa[(ss + 1) & 1][2 * c] = read_frag(fragK, wn * kSub + (2 * c) * 32 + r, nss * 2 + hh);
           fa[(ss + 1) & 1][2 * c + 1] = read_frag(fragK, wn * kSub + (2 * c + 1) * 32 + r, nss * 2 + hh);
         } else if (c == 2) {
-          fb[(ss + 1) & 1][0] = read_frag(fragQ, wm * kRowsW + r, nss * 2 + hh);
-          fb[(ss + 1) & 1][1] = read_frag(fragQ, wm * kRowsW + 32 + r, nss * 2 + hh);
+#pragma unroll
+          for (int x = 0; x < kMT; ++x) fb[(ss + 1) & 1][x] = read_frag(fragQ, wm * 32 * kMT + x * 32 + r, nss * 2 + hh);
         }
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt) acc[c][mt] = mfma32(fa[ss & 1][c], fb[ss & 1][mt], acc[c][mt]);
+        for (int mt = 0; mt < kMT; ++mt) acc[c][mt] = mfma32(fa[ss & 1][c], fb[ss & 1][mt], acc[c][mt]);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -333,7 +359,7 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
   // ---- epilogue: this wavefront's 128 keys x 64 query rows
   const int nbase = n0 + wn * kSub;       // first key of the wavefront tile
   const int T = nbase / kSub;
-  const Quarter own = kPacked ? tile_quarter(p, head, m0, wm) : Quarter{head, m0 + wm * kRowsW};
+  const Quarter own = kPacked ? tile_quarter(p, head, m0, wm) : Quarter{head, m0 + wm * 32 * kMT};
   if (nbase < p.n_rk && (!kPacked || own.head >= 0)) {
   float* Pst = p.P + (int64_t)own.head * p.nkb * p.rows;
   float* Mst = p.Mt + ((int64_t)own.head * p.nT + T) * p.rows;
@@ -344,7 +370,7 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
   const bool all_visible = nbase + kSub <= p.n_rk && nbase + kSub - 1 <= row_hi(p, mw0) &&
                            nbase >= row_lo(p, mw0 + kRowsW - 1);
 #pragma unroll
-  for (int mt = 0; mt < 2; ++mt) {
+  for (int mt = 0; mt < kMT; ++mt) {
     const int m = mw0 + mt * 32 + r;
     const bool row_ok = m < p.live_end;
     const int lo = row_lo(p, m), hi = row_hi(p, m);
@@ -761,7 +787,8 @@ namespace {
 // of estimate_small_kernel's variants - lat: one step when there are few tiles, per_tile: a tile's share of a step when
 // the chip is full - and for the 256x256 tiles, which 256 workgroups take in turns,
 //   5 us + steps * 1.75 us * ceil(tiles / 256),
-// with a head's rows in tiles of their own or packed with those of the other heads of its KV group.
+// with a head's rows in tiles of their own or packed with those of the other heads of its KV group, or, with 0.65 of a
+// tile's time for a half and 6 us for the second launch, the last of them as half tiles.
 // The constants are fits to measured times of the passes over 200 .. 16384 tokens and chunks of 64 .. 8000 tokens on
 // 8700 .. 100000 cached ones, stride 8 and 16 (us, 256x256 / chosen): 1000 tokens, stride 16: 45.2 / 10.6 (MT 1);
 // 2000, stride 8: 31.1 / 9.8 (MT 2, 3 stages); 4096, stride 8: 35.0 / 19.2; 8192, stride 16: 60.9 / 31.6;
@@ -772,9 +799,9 @@ struct SmallVariant {
 };
 constexpr SmallVariant kSmall[] = {{1, 4, 0.20f, 0.00106f}, {2, 3, 0.27f, 0.00129f}, {2, 2, 0.35f, 0.00126f}, {4, 2, 0.50f, 0.00238f}};
 
-template <int RBS, bool kDump, bool kTable, bool kPacked = false>
+template <int RBS, bool kDump, bool kTable, bool kPacked = false, bool kHalf = false>
 hipError_t launch_gemm_as(const EstParams& p, dim3 grid, size_t lds, hipStream_t s) {
-  auto kernel = &estimate_gemm_kernel<RBS, kDump, kTable, kPacked>;
+  auto kernel = &estimate_gemm_kernel<RBS, kDump, kTable, kPacked, kHalf>;
   static LdsLimit limit;
   hipError_t e = limit.raise(reinterpret_cast<const void*>(kernel));
   if (e != hipSuccess) return e;
@@ -783,6 +810,13 @@ hipError_t launch_gemm_as(const EstParams& p, dim3 grid, size_t lds, hipStream_t
 }
 template <int RBS>
 hipError_t launch_gemm(const EstParams& p, dim3 grid, size_t lds, hipStream_t s) {
+  if (p.split_tiles || p.last_row_tiles) {
+    EstParams c = p;
+    c.total_tiles = p.whole_tiles;
+    hipError_t e = c.total_tiles ? launch_gemm_as<RBS, false, false>(c, grid, lds, s) : hipSuccess;
+    c.total_tiles = p.total_tiles - p.whole_tiles;
+    return e != hipSuccess ? e : launch_gemm_as<RBS, false, false, false, true>(c, grid, lds, s);
+  }
   if (p.group_tiles) return launch_gemm_as<RBS, false, false, true>(p, grid, lds, s);
   if (p.n_pairs) return p.scores ? launch_gemm_as<RBS, true, true>(p, grid, lds, s) : launch_gemm_as<RBS, false, true>(p, grid, lds, s);
   return p.scores ? launch_gemm_as<RBS, true, false>(p, grid, lds, s) : launch_gemm_as<RBS, false, false>(p, grid, lds, s);
@@ -995,7 +1029,7 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
   p.nNT = ((p.nT_real < g.nT ? p.nT_real * kSub : g.n_rk) + kTile - 1) / kTile;
   p.tiles_per_head = tiles_of(kTile, kTile, p.nNT);
   p.total_tiles = (int64_t)p.tiles_per_head * num_heads;
-  p.group_tiles = 0;
+  p.group_tiles = p.split_tiles = p.last_row_tiles = 0;
   int variant = -1;
   if (kdb == 1 && num_slab_pairs == 0 && !scores_out && p.total_tiles > 0 && p.total_tiles <= 4096) {
     const int group = num_heads / num_kv_heads;
@@ -1029,8 +1063,35 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
       c.key_tiles = last - c.first_key_tile + 1;
       c.total_tiles = (int64_t)c.group_tiles * c.key_tiles * num_kv_heads;
       if (c.key_tiles > 0 && c.total_tiles < p.total_tiles && 1.75f * (float)((c.total_tiles + 255) / 256) < best_t) {
+        best_t = 1.75f * (float)((c.total_tiles + 255) / 256);
         best = c;
         variant = -1;
+      }
+    }
+    // a last row tile of 128 rows or fewer, and what does not fill a round, as half tiles
+    {
+      EstParams c = p;
+      const int last_rows = p.rows - (p.nMT - 1) * kTile, last_m0 = p.row_begin + (p.nMT - 1) * kTile;
+      if (last_rows <= kTile / 2) {
+        c.nMT -= 1;
+        c.first_key_tile = row_lo(p, last_m0) / kTile;
+        int last = row_hi(p, p.live_end - 1) / kTile;
+        last = last < p.nNT - 1 ? last : p.nNT - 1;
+        c.last_row_tiles = last - c.first_key_tile + 1;
+        c.tiles_per_head -= c.last_row_tiles;
+      }
+      const int tiles = c.tiles_per_head * num_heads, halves = c.last_row_tiles * num_heads;
+      for (int rounds = tiles / 256; rounds >= 0 && rounds >= tiles / 256 - 1; --rounds) {
+        c.whole_tiles = rounds * 256;
+        c.split_tiles = tiles - c.whole_tiles;
+        const int units = 2 * c.split_tiles + halves;
+        const float t = 1.75f * ((float)rounds + 0.65f * (float)((units + 255) / 256)) + (rounds ? 6.f / (float)(2 * stride) : 0.f);
+        if (units > 0 && t < best_t) {
+          best_t = t;
+          best = c;
+          best.total_tiles = (int64_t)c.whole_tiles + units;
+          variant = -1;
+        }
       }
     }
     p = best;

@@ -43,6 +43,9 @@ struct EstParams {
   int pack, tile_rows, tile_shift;   // powers of two, tile_rows = 1 << tile_shift
   // estimate_gemm_kernel with packed rows: quarters of 64 rows per head, 256-row tiles per KV group, first key tile, key tiles
   int quarters, group_tiles, first_key_tile, key_tiles;
+  // estimate_gemm_kernel with half tiles: tiles taken whole, tiles behind them taken as two halves of 128 rows, and per head
+  // the tiles (of keys from first_key_tile on) of a last row tile that has one half
+  int whole_tiles, split_tiles, last_row_tiles;
 };
 
 // first / last visible reshaped key of reshaped query row m
