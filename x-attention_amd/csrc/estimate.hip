@@ -590,7 +590,7 @@ __global__ __launch_bounds__(256) void estimate_normalize_kernel(EstParams p) {
 }
 
 // Normalisation and selection in one pass, for callers that want the column lists (or the mask) and not the
-// block sums: a workgroup of QB wavefronts takes QB consecutive q-block rows of one head (QB * RBS reshaped
+// block sums: a workgroup takes QB consecutive q-block rows of one head (QB * RBS reshaped
 // query rows), computes their softmax statistics and normalised block sums exactly as the kernel above does -
 // same loads, same operation order - but leaves the sums in LDS, where wavefront i then runs the selection of
 // row i (select_row.h).  The block sums never travel to memory and back.
@@ -850,12 +850,12 @@ hipError_t launch_small(const EstParams& p, int variant, hipStream_t s) {
   }
 }
 template <int RBS>
-hipError_t launch_select(const EstParams& p, const SelParams& sp, int qb_per_wg, dim3 grid, size_t lds, hipStream_t s) {
+hipError_t launch_select(const EstParams& p, const SelParams& sp, int qb_per_wg, int threads, dim3 grid, size_t lds, hipStream_t s) {
   auto kernel = &estimate_select_kernel<RBS>;
   static LdsLimit limit;
   hipError_t e = limit.raise(reinterpret_cast<const void*>(kernel));
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kernel, grid, dim3(64 * qb_per_wg), lds, s, p, sp, qb_per_wg);
+  hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, s, p, sp, qb_per_wg);
   return hipSuccess;
 }
 
@@ -1108,7 +1108,7 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
   // the fused normalise-and-select pass: QB q-block rows (one wavefront each) per workgroup, as many as keep a
   // workgroup's LDS (statistics + per wavefront: the row's sums, sort keys, flags) within 64 KiB
   SelParams sp;
-  int qb_per_wg = 0;
+  int qb_per_wg = 0, sel_threads = 0;
   size_t lds_sel = 0, sel_wave_bytes = 0;
   dim3 grid_sel(1);
   if (sel) {
@@ -1138,6 +1138,15 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
     qb_per_wg = 4;
     while (qb_per_wg > 1 && (qb_per_wg * (wave_bytes + 10 * p.rbs * sizeof(float)) > 64 * 1024 || qb_per_wg * p.rbs > 128))
       qb_per_wg >>= 1;
+    sel_threads = 64 * qb_per_wg;
+    // Few rows leave CUs idle: then a workgroup takes fewer of them, still with four wavefronts for the sums (us, by rows of a
+    // workgroup, 4 / 2 / 1: 512 rows of 512 blocks 38 / 34.5 / 35, 32 of 800 45 / 40 / 37, 1024 of 32 9.5 / 8.5 / 8.3, 2016 of 63
+    // 15.2 / 14.5 / 17.3; 4000 of 125 20.7 / 24 / 30)
+    const int64_t rows = (int64_t)num_heads * (sp.row_end > sp.row_begin ? sp.row_end - sp.row_begin : 0);
+    while (qb_per_wg > 1 && rows / qb_per_wg <= 512) {
+      sel_threads = 256;
+      qb_per_wg >>= 1;
+    }
     lds_sel = qb_per_wg * (wave_bytes + 10 * p.rbs * sizeof(float));
     const int qrows = sp.row_end > sp.row_begin ? sp.row_end - sp.row_begin : 0;
     const int64_t wgs = (int64_t)num_heads * ((qrows + qb_per_wg - 1) / qb_per_wg);
@@ -1151,7 +1160,7 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
       return hipSuccess;
     }
     if (sp.row_end <= sp.row_begin) return hipSuccess;   // a chunk of padding alone
-    return launch_select<RBS>(p, sp, qb_per_wg, grid_sel, lds_sel, s);
+    return launch_select<RBS>(p, sp, qb_per_wg, sel_threads, grid_sel, lds_sel, s);
   };
   // one pass instead of two where every row asked for is estimated, in 32-row tiles, and sees a single key tile
   bool one_pass = variant == 0 && sel && sel->stages == 3 && !p.no_softmax && !p.sums && !sel->plan && p.nT_real == g.nT &&
