@@ -344,8 +344,8 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
           fa[(ss + 1) & 1][2 * c] = read_frag(fragK, wn * kSub + (2 * c) * 32 + r, nss * 2 + hh);
           fa[(ss + 1) & 1][2 * c + 1] = read_frag(fragK, wn * kSub + (2 * c + 1) * 32 + r, nss * 2 + hh);
         } else if (c == 2) {
-#pragma unroll
-          for (int x = 0; x < kMT; ++x) fb[(ss + 1) & 1][x] = read_frag(fragQ, wm * 32 * kMT + x * 32 + r, nss * 2 + hh);
+          fb[(ss + 1) & 1][0] = read_frag(fragQ, wm * 32 * kMT + r, nss * 2 + hh);
+          if (kMT == 2) fb[(ss + 1) & 1][kMT - 1] = read_frag(fragQ, wm * 32 * kMT + 32 + r, nss * 2 + hh);
         }
 #pragma unroll
         for (int mt = 0; mt < kMT; ++mt) acc[c][mt] = mfma32(fa[ss & 1][c], fb[ss & 1][mt], acc[c][mt]);
