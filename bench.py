@@ -39,8 +39,8 @@ PEAK_HBM_GBS = 8000.0
 # this process): the summary of those runs for the headline workload is kept as a table under profiles/ and read here.
 TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "bench_headline_hbm_traffic.md")
 HEADLINE = "cfg2_llama8b_L131072_gqa32x8_S16"
-KERNEL_SOURCES = ("attn_tiles.h", "block_sparse_attn.hip", "estimate.hip", "select_row.h", "select_blocks.hip",
-                  "xattn_common.h")
+KERNEL_SOURCES = ("attn_plan.h", "attn_tiles.h", "block_sparse_attn.hip", "estimate.hip", "estimate_params.h", "select_row.h",
+                  "select_blocks.hip", "xattn_common.h")
 
 
 def kernel_source_hash():
@@ -320,7 +320,7 @@ def summarize(w, L, tau, chunk, m, headline_traffic=False):
         "kernel": "block_sparse_fwd_kernel<true>", "bound": "mfma", "achieved": round(att_tf, 1),
         "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s", "frac": round(att_tf / PEAK_BF16_TFLOPS, 4), "ms": round(t_att, 3),
         "flop": fb["f_sparse"],
-        "traffic": measured_traffic_bytes("xattn::block_sparse_fwd_kernel<true>") if headline_traffic else None,
+        "traffic": measured_traffic_bytes("xattn::block_sparse_fwd_kernel<true") if headline_traffic else None,
     }
     sel_gbs = fb["pass_bytes"] / (t_sel * 1e-3) / 1e9
     rl_sel = {
