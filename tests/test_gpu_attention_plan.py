@@ -56,3 +56,32 @@ def test_cut_lists_give_the_same_attention(q_len, cache, heads, kv_heads, thresh
     bound = 2.0 ** -8 * (v.float().abs().amax() + want.abs())
     assert ((outs[0].float() - want).abs() <= bound).all()
     assert (outs[0].float() - want).norm() <= 4e-3 * want.norm()
+
+
+def test_a_side_stream_leaves_memory_of_queued_work_alone():
+    """`stream` does not wait for the current stream: memory that Python has released there, but queued work still reads,
+    must not become the workspace."""
+    from xattn.src import hip_backend as hb
+    from xattn.src.Xattention import block_sparse_attention, estimate_and_select
+
+    q, k, v = _inputs(1024, 9216, 8, 2, 5)
+    r = estimate_and_select(q, k, 8, 1.0, 128, want_mask=False, want_sums=False)
+    idx, cnt = r["col_idx"], r["col_cnt"]
+    want = block_sparse_attention(q, k, v, idx, cnt)
+    bytes_ = hb.lib().xattn_block_sparse_workspace_bytes(8, 1024, 9216, idx.shape[1], 8)
+    assert bytes_ > 0
+    out = torch.empty(1, 1024, 8, 128, dtype=torch.bfloat16, device="cuda")
+    side = torch.cuda.Stream()
+    a = torch.randn(8192, 8192, device="cuda", dtype=torch.bfloat16)
+    b = torch.empty_like(a)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    t = torch.full((bytes_,), 7, dtype=torch.uint8, device="cuda")
+    for _ in range(20):                                            # some 15 ms
+        torch.mm(a, a, out=b)
+    touched = (t != 7).any()
+    del t                                                          # the next allocation of this size on this stream is t's block
+    got = block_sparse_attention(q, k, v, idx, cnt, out=out, stream=side)
+    torch.cuda.synchronize()
+    assert not touched.item()
+    assert torch.equal(got, want)

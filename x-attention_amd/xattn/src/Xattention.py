@@ -444,9 +444,12 @@ def block_sparse_attention(query_states, key_states, value_states, col_idx=None,
         nb = (q_len + 127) // 128
         ws_bytes = lib.xattn_block_sparse_workspace_bytes(
             heads, q_len, k_len, idx_rows if col_idx is not None else nb, (qb1 if qb1 >= 0 else nb) - qb0)
-        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-        if workspace is not None and stream is not None:
-            workspace.record_stream(stream)
+        workspace = None
+        if ws_bytes:
+            # from the pool of the stream that writes it: what the current stream's pool hands out may still be in use by
+            # work queued there, for which `stream` does not wait
+            with torch.cuda.stream(stream):
+                workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         _hb.check(
             lib.xattn_block_sparse_fwd_ws(
                 q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
