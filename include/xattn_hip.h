@@ -222,10 +222,12 @@ int xattn_block_sparse_fwd(const void* q, const void* k, const void* v, void* ou
  * `workspace`: xattn_block_sparse_workspace_bytes() bytes for the q_blocks =
  * q_block_end - q_block_begin q-blocks of the launch, 256-byte aligned,
  * contents undefined on entry and on return; 0 bytes (null allowed) means that
- * nothing is cut.  Without lists (col_idx null; idx_rows = ceil(q_len / 128))
- * the visible blocks of a unit are its list.  Where lists are cut depends on their lengths, num_heads and
- * q_len only, so results do not depend on how q-blocks are spread over launches;
- * a cut list's row sums are added in another order than an uncut one's.
+ * nothing is cut.  Without lists (col_idx null; idx_rows = 0 for the size) the
+ * visible blocks of a unit are its list.  Where a list is cut depends on the
+ * lengths of its q-block's lists over all heads, num_heads, q_len and k_len
+ * only, so results do not depend on how q-blocks are spread over launches; a
+ * cut list's row sums are added in another order than an uncut one's, and its
+ * probabilities are rounded against another reference maximum.
  */
 size_t xattn_block_sparse_workspace_bytes(int num_heads, int q_len, int k_len, int idx_rows, int q_blocks);
 

@@ -58,6 +58,59 @@ def test_cut_lists_give_the_same_attention(q_len, cache, heads, kv_heads, thresh
     assert (outs[0].float() - want).norm() <= 4e-3 * want.norm()
 
 
+def _taus(heads, long_heads):
+    """Thresholds that let a few heads keep every block and the others almost none."""
+    t = torch.full((heads,), 0.02, dtype=torch.float32)
+    t[torch.tensor(long_heads)] = 1.0
+    return t
+
+
+# Heads whose lists differ: more than 64 heads (a lane of the noting wavefront has two), the long ones at its edges, lists
+# next to multiples of a piece, ragged, no causality, half of the lists long (their longest is 1.3 to 2 times the mean)
+@pytest.mark.parametrize("q_len,cache,heads,kv_heads,long_heads,causal", [
+    (3000, 0, 32, 8, [0, 31], True),
+    (1500, 128 * 20 + 5, 72, 8, [0, 63, 64, 71], True),
+    (2048, 9000, 32, 8, list(range(0, 32, 2)), True),
+    (1100, 128 * 47, 40, 8, [7], False),
+    (2500, 0, 66, 2, [65], False),
+    (2048, 30000, 32, 8, [3, 4, 30], True),
+])
+def test_lists_of_unlike_heads_are_cut_the_same_way_by_every_path(q_len, cache, heads, kv_heads, long_heads, causal):
+    from xattn.src.Xattention import Xattention_prefill, block_sparse_attention, estimate_and_select
+
+    q, k, v = _inputs(q_len, q_len + cache, heads, kv_heads, heads)
+    taus, chunk, nq = _taus(heads, long_heads), 128, (q_len + 127) // 128
+    r = estimate_and_select(q, k, 8, taus, chunk, causal=causal, want_mask=False, want_sums=False)
+    idx, cnt = r["col_idx"][:, :nq].contiguous(), r["col_cnt"][:, :nq].contiguous()
+    got = Xattention_prefill(q, k, v, 8, threshold=taus, chunk_size=chunk, causal=causal)
+    assert torch.equal(block_sparse_attention(q, k, v, idx, cnt, causal=causal), got)
+    # q-blocks spread over launches
+    parts = torch.empty(1, q_len, heads, 128, dtype=torch.bfloat16, device="cuda")
+    for a, b in ((0, 1), (1, nq // 2), (nq // 2, nq)):
+        block_sparse_attention(q, k, v, idx, cnt, causal=causal, out=parts, q_blocks=(a, b))
+    assert torch.equal(parts.transpose(1, 2), got)
+    want = _swept_whole(q, k, v, idx, cnt, causal)
+    # the bound of the test above
+    bound = 2.0 ** -8 * (v.float().abs().amax() + want.abs())
+    assert ((got.float() - want).abs() <= bound).all()
+    assert (got.float() - want).norm() <= 4e-3 * want.norm()
+
+
+# (512 units on a cache, 544 by themselves, 720; every list of a q-block equally long)
+@pytest.mark.parametrize("q_len,cache,heads,kv_heads,causal", [(2048, 8192, 32, 8, True), (2100, 0, 32, 8, True), (3800, 0, 24, 24, False)])
+def test_even_lists_are_swept_whole(q_len, cache, heads, kv_heads, causal):
+    from xattn.src.Xattention import Xattention_prefill, block_sparse_attention, estimate_and_select
+
+    q, k, v = _inputs(q_len, q_len + cache, heads, kv_heads, 3)
+    nq = (q_len + 127) // 128
+    r = estimate_and_select(q, k, 8, 1.0, 128, causal=causal, want_mask=False, want_sums=False)
+    idx, cnt = r["col_idx"][:, :nq].contiguous(), r["col_cnt"][:, :nq].contiguous()
+    want = _swept_whole(q, k, v, idx, cnt, causal)
+    assert torch.equal(Xattention_prefill(q, k, v, 8, threshold=1.0, chunk_size=128, causal=causal).float(), want)
+    assert torch.equal(block_sparse_attention(q, k, v, idx, cnt, causal=causal).float(), want)
+    assert torch.equal(block_sparse_attention(q, k, v, causal=causal).float(), want)
+
+
 def test_a_side_stream_leaves_memory_of_queued_work_alone():
     """`stream` does not wait for the current stream: memory that Python has released there, but queued work still reads,
     must not become the workspace."""

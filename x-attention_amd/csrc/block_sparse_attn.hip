@@ -322,11 +322,10 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
   int piece = -1;                    // which piece of its list a workgroup has, if any
   int skip = 0;                      // workgroups ahead of the units'
   if (kPlanned) {
-    // an XCD gets a run of adjacent pieces, which are of adjacent lists
-    const int pieces = ((const_i32_ptr)(uintptr_t)p.plan.head)[0], per_xcd = (pieces + 7) / 8;
+    const int pieces = ((const_i32_ptr)(uintptr_t)p.plan.noted)[0], per_xcd = (pieces + 7) / 8;   // (the low half)
     skip = per_xcd * 8;
     if ((int)blockIdx.x < skip) {
-      const int at = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+      const int at = p.plan.in_turn ? (int)blockIdx.x : (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
       if (at >= pieces) return;
       const_i32_ptr entry = (const_i32_ptr)(uintptr_t)p.plan.pieces + 2 * at;
       const int unit = entry[0];
@@ -347,7 +346,7 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
   // the column list is read through the scalar cache (uniform, read-only), so that
   // fetching the next block id never waits on the tile copies in flight
   const_i32_ptr list = nullptr;
-  int cuts = 0, number = 0;          // pieces of this list, its number in the plan
+  int cuts = 0, part0 = 0;           // pieces of this list, the first one's place in the plan
   {
     const int q_last = (qb * kBlk + kBlk - 1 < p.Lq ? qb * kBlk + kBlk - 1 : p.Lq - 1) + p.kv_off;
     int visible = p.causal ? (q_last < 0 ? 0 : q_last / kBlk + 1) : p.nkb;
@@ -362,11 +361,12 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
       n_blocks = visible;
     }
     if (kPlanned) {
-      cuts = piece_count(n_blocks, p.plan);
-      if (cuts > 0) {
+      const uint32_t cut = n_blocks > p.plan.min_piece ? (uint32_t)((const_i32_ptr)(uintptr_t)p.plan.cut)[slot] : 0;
+      if (cut != 0) {
         if (piece < 0) return;           // others have it
-        const int length = piece_length(n_blocks, p.plan);
-        number = ((const_i32_ptr)(uintptr_t)p.plan.number)[slot];
+        cuts = cut_pieces(cut);
+        part0 = cut_at(cut);
+        const int length = cut_length(cut);
         if (kHasList) list += piece * length;
         else first = piece * length;
         n_blocks = piece + 1 < cuts ? length : n_blocks - piece * length;
@@ -429,12 +429,12 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
   }
   // the last barrier of the sweep (or the one before it, for an empty list) left both tiles unused
   if (kPlanned && cuts > 0) {
-    float* const part = p.plan.part + (int64_t)number * p.plan.items * kPartFloats;
+    float* const part = p.plan.part + (int64_t)part0 * kPartFloats;
     store_partial(part + (int64_t)piece * kPartFloats, wave, lane, r, hh, oacc, m_run, l_run);
     wait_vm0();                              // written through to memory
     __syncthreads();
     int* const scratch = reinterpret_cast<int*>(Ks);
-    if (tid == 0) scratch[0] = __hip_atomic_fetch_add(p.plan.done + number, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) scratch[0] = __hip_atomic_fetch_add(p.plan.done + (int64_t)head * p.idx_rows + (qb - p.idx_row0), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     if (scratch[0] != cuts - 1) return;      // the piece that comes last combines them
     __syncthreads();
@@ -443,26 +443,26 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
   store_out(p, head, qb, wave, lane, r, hh, oacc, l_run, Ks + wave * 8192);
 }
 
-// Notes the long lists of q-blocks [qb_begin, qb_end) of every head, where the pass that made them has not (or, without
-// lists, the visible blocks of each).  One workgroup: it also clears the plan's head.
+// Notes the lists of q-blocks [qb_begin, qb_end) of every head, where the pass that made them has not (or, without
+// lists, the visible blocks of each).  One workgroup: it also clears the count of pieces.
 __global__ __launch_bounds__(1024) void note_lists_kernel(AttnParams p) {
-  if (threadIdx.x == 0) *p.plan.head = 0;
+  if (threadIdx.x == 0) *p.plan.noted = 0;
   __threadfence();
   __syncthreads();
-  const int rows = p.qb_end - p.qb_begin;
-  for (int i = threadIdx.x; i < p.H * rows; i += 1024) {
-    const int qb = p.qb_begin + i % rows;
-    const int unit = i / rows * p.idx_rows + qb - p.idx_row0;
-    int n = p.nkb;
-    if (p.col_cnt) {
-      n = p.col_cnt[unit];
-      n = n > p.idx_pitch ? (int)p.idx_pitch : n;
-    } else if (p.causal) {
-      const int q_last = (qb * kBlk + kBlk - 1 < p.Lq ? qb * kBlk + kBlk - 1 : p.Lq - 1) + p.kv_off;
-      const int visible = q_last < 0 ? 0 : q_last / kBlk + 1;
-      n = visible < n ? visible : n;
-    }
-    note_list(p.plan, unit, n);
+  const int lane = threadIdx.x & 63;
+  for (int qb = p.qb_begin + (int)(threadIdx.x >> 6); qb < p.qb_end; qb += 16) {
+    const int row = qb - p.idx_row0;
+    const int q_last = (qb * kBlk + kBlk - 1 < p.Lq ? qb * kBlk + kBlk - 1 : p.Lq - 1) + p.kv_off;
+    int visible = p.causal ? (q_last < 0 ? 0 : q_last / kBlk + 1) : p.nkb;
+    visible = visible < p.nkb ? visible : p.nkb;
+    auto count = [&](int h) {
+      if (!p.col_cnt) return visible;
+      const int n = p.col_cnt[(int64_t)h * p.idx_rows + row];
+      return n < 0 ? 0 : n > p.idx_pitch ? (int)p.idx_pitch : n;
+    };
+    int total = 0;
+    for (int h = lane; h < p.H; h += 64) total += count(h) < 65536 ? count(h) : 65536;   // (a sum of at most 8192)
+    note_q_block(p.plan, p.H, __builtin_amdgcn_readlane(wave_scan(total), 63), row, p.idx_rows, lane, count);
   }
 }
 
@@ -562,8 +562,13 @@ int items_of(int num_heads, int q_len, int k_len) {
 }  // namespace
 
 extern "C" size_t xattn_block_sparse_workspace_bytes(int num_heads, int q_len, int k_len, int idx_rows, int q_blocks) {
-  if (num_heads <= 0 || q_len <= 0 || k_len <= 0 || idx_rows <= 0 || q_blocks <= 0) return 0;
-  return plan_bytes((int64_t)num_heads * idx_rows, (int64_t)num_heads * q_blocks, items_of(num_heads, q_len, k_len));
+  if (num_heads <= 0 || q_len <= 0 || k_len <= 0 || idx_rows < 0 || q_blocks <= 0) return 0;
+  const int nqb = (q_len + kBlk - 1) / kBlk;
+  if (idx_rows == 0) {                 // all lists of a q-block alike
+    if ((int64_t)num_heads * nqb > kEvenUnits) return 0;
+    idx_rows = nqb;
+  }
+  return plan_bytes((int64_t)num_heads * idx_rows, (int64_t)num_heads * q_blocks, nqb, items_of(num_heads, q_len, k_len));
 }
 
 extern "C" int xattn_block_sparse_fwd_ws(const void* q, const void* k, const void* v, void* out, void* workspace,
@@ -575,15 +580,16 @@ extern "C" int xattn_block_sparse_fwd_ws(const void* q, const void* k, const voi
                                          int causal, float softmax_scale, void* stream) {
   if (q_len <= 0 || k_len <= 0) return XATTN_ERR_SHAPE;
   if (q_block_end < 0) q_block_end = (q_len + kBlk - 1) / kBlk;
-  if (!col_idx) idx_rows = (q_len + kBlk - 1) / kBlk, idx_row0 = 0;
-  const int q_blocks = q_block_end - q_block_begin;
-  const size_t need = xattn_block_sparse_workspace_bytes(num_heads, q_len, k_len, idx_rows, q_blocks);
+  const int nqb = (q_len + kBlk - 1) / kBlk, q_blocks = q_block_end - q_block_begin;
+  const size_t need = xattn_block_sparse_workspace_bytes(num_heads, q_len, k_len, col_idx ? idx_rows : 0, q_blocks);
+  if (!col_idx) idx_rows = nqb, idx_row0 = 0;
   AttnPlan plan{};
   if (need) {
     if (!workspace) return XATTN_ERR_NULL;
     if (workspace_bytes < need) return XATTN_ERR_WORKSPACE;
     if (reinterpret_cast<uintptr_t>(workspace) & 255) return XATTN_ERR_ALIGN;
-    plan = plan_at(static_cast<char*>(workspace), (int64_t)num_heads * idx_rows, (int64_t)num_heads * q_blocks, items_of(num_heads, q_len, k_len), (k_len + kBlk - 1) / kBlk);
+    plan = plan_at(static_cast<char*>(workspace), (int64_t)num_heads * idx_rows, (int64_t)num_heads * q_blocks, (int64_t)num_heads * nqb,
+                   nqb, (k_len + kBlk - 1) / kBlk, items_of(num_heads, q_len, k_len));
   }
   return block_sparse_impl(q, k, v, out, col_idx, col_cnt, idx_pitch, idx_rows, idx_row0, num_heads, num_kv_heads, q_len, k_len,
                            head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n, o_stride_h,

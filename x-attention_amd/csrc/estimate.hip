@@ -182,7 +182,7 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
   const int r = lane & 31, hh = lane >> 5;
   const int wm = wave & 3, wn = wave >> 2;   // query quarter, key half
   constexpr int kMT = kHalf ? 1 : 2;         // 32-row query tiles of a wavefront
-  if (blockIdx.x == 0 && tid == 0 && p.noted) *p.noted = 0;
+  for (int i = (int)blockIdx.x * kWaves * 64 + tid; i < p.noted_words; i += (int)gridDim.x * kWaves * 64) p.noted[i] = 0;
   // A workgroup works through tiles id, id + grid, ...: one workgroup fits a CU, so nothing else could hide
   // the wait for a tile's first slabs.  The slab pipeline therefore runs on across the tile boundary: the load
   // slots of a tile's last two k-steps fetch the first slabs of the NEXT tile, and the last sub-step reads its
@@ -996,7 +996,8 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
   p.n_pairs = num_slab_pairs;
   p.scores = scores_out;
   p.sums = block_sums;
-  p.noted = sel && sel->plan ? sel->plan->head : nullptr;
+  p.noted = sel && sel->plan ? sel->plan->noted : nullptr;
+  p.noted_words = p.noted ? (int)((plan_noted_bytes(nqb_real) + plan_round((size_t)num_heads * nqb_real * 4)) / 8) : 0;
   // block_sums may hold a window of q-block rows only; the chunks of this call must lie inside it
   {
     const int bpc = chunk_size / block_size;

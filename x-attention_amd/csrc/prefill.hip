@@ -35,7 +35,7 @@ bool prefill_layout(int num_heads, int q_len, int k_len, int stride, int chunk_s
   l->plan_off = l->idx_off + up256((size_t)num_heads * l->nqb * l->nkb * sizeof(int32_t));
   const int64_t units = (int64_t)num_heads * l->nqb;
   l->items = plan_items(units, l->nqb, l->nkb);
-  l->total = l->plan_off + plan_bytes(units, units, l->items);
+  l->total = l->plan_off + plan_bytes(units, units, l->nqb, l->items);
   return true;
 }
 }  // namespace
@@ -71,8 +71,8 @@ extern "C" int xattn_prefill_fwd(const void* q, const void* k, const void* v, vo
   sel.real_q_blocks_only = 1;
   sel.stages = 3;
   const int64_t units = (int64_t)num_heads * l.nqb;
-  const AttnPlan plan = plan_at(ws + l.plan_off, units, units, l.items, l.nkb);
-  // (with zero_rows_from 0 no row is estimated, and no MFMA pass would clear the plan's head: noted afterwards)
+  const AttnPlan plan = plan_at(ws + l.plan_off, units, units, units, l.nqb, l.nkb, l.items);
+  // (with zero_rows_from 0 no row is estimated, and no MFMA pass would clear what is noted: noted afterwards)
   // Where no list can be long enough to be cut, nothing is noted (nor planned below): then the selection may follow the
   // estimate in the same kernel.
   const int q_chunks = (int)(((int64_t)q_len + chunk_size - 1) / chunk_size), k_chunks = (int)(((int64_t)k_len + chunk_size - 1) / chunk_size);

@@ -23,7 +23,7 @@ struct SelParams {
   int causal, keep_sink, keep_recent, list_cols, q_len, kv_off;
   int blocks_per_chunk;
   int npow2;   // LDS key capacity (power of two >= nkb)
-  AttnPlan plan;   // head null: nothing is noted
+  AttnPlan plan;   // items 0: nothing is noted
 };
 
 constexpr int kSlots = 16;        // candidates per lane held in registers (rows up to 1024 candidates)
@@ -38,29 +38,6 @@ __device__ __forceinline__ double key_value(uint64_t key) {
   return hi ? (double)__uint_as_float(hi - 1u) : 0.0;
 }
 
-// Reductions over the wavefront through the data-parallel lane moves: within rows of 16 lanes by shifts of 1, 2, 4 and 8,
-// then over the rows; lane 63 ends up with the result, which comes back as a uniform value.  (A butterfly of lane permutes
-// takes a trip through the LDS crossbar per step, about 700 clk for a search step of the selection.)
-template <int kCtrl, int kRows>
-__device__ __forceinline__ uint32_t lane_move(uint32_t old, uint32_t x) {
-  return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)x, kCtrl, kRows, 0xf, false);
-}
-template <typename F>
-__device__ __forceinline__ uint32_t wave_fold(uint32_t x, F f) {   // f idempotent: max or min
-  x = f(x, lane_move<0x111, 0xf>(x, x));
-  x = f(x, lane_move<0x112, 0xf>(x, x));
-  x = f(x, lane_move<0x114, 0xf>(x, x));
-  x = f(x, lane_move<0x118, 0xf>(x, x));
-  x = f(x, lane_move<0x142, 0xa>(x, x));
-  x = f(x, lane_move<0x143, 0xc>(x, x));
-  return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
-}
-__device__ __forceinline__ uint32_t wave_max(uint32_t x) {
-  return wave_fold(x, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
-}
-__device__ __forceinline__ uint32_t wave_min(uint32_t x) {
-  return wave_fold(x, [](uint32_t a, uint32_t b) { return a < b ? a : b; });
-}
 template <int kCtrl, int kRows>
 __device__ __forceinline__ double lane_move(double x) {            // 0 where no lane is moved from
   const uint64_t b = __builtin_bit_cast(uint64_t, x);
@@ -422,11 +399,10 @@ __device__ __forceinline__ void select_row(const SelParams& p, const float* x, i
       if (keep && pos < p.idx_pitch) list[pos] = c;
       count += __popcll(ballot);
     }
-    if (lane == 0) {
-      count = count < p.idx_pitch ? count : (int)p.idx_pitch;
-      p.col_cnt[slot] = count;
-      if (p.plan.head) note_list(p.plan, (int)slot, count);
-    }
+    count = count < p.idx_pitch ? count : (int)p.idx_pitch;
+    if (lane == 0) p.col_cnt[slot] = count;
+    if (p.plan.items && (p.causal ? q_last / 128 + 1 : p.list_cols) > p.plan.min_piece)   // else too few blocks to be cut
+      list_made(p.plan, p.H, p.win_rows, row - p.win_row0, head, count, lane);
   }
 }
 

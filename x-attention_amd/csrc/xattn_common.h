@@ -70,6 +70,40 @@ __device__ __forceinline__ float half_max(float x) {
   return fmaxf(lo, hi);
 }
 
+// Reductions over the wavefront through the data-parallel lane moves: within rows of 16 lanes by shifts of 1, 2, 4 and 8,
+// then over the rows; lane 63 ends up with the result, which comes back as a uniform value.  (A butterfly of lane permutes
+// takes a trip through the LDS crossbar per step, about 700 clk for a search step of the selection.)
+template <int kCtrl, int kRows>
+__device__ __forceinline__ uint32_t lane_move(uint32_t old, uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)x, kCtrl, kRows, 0xf, false);
+}
+template <typename F>
+__device__ __forceinline__ uint32_t wave_fold(uint32_t x, F f) {   // f idempotent: max or min
+  x = f(x, lane_move<0x111, 0xf>(x, x));
+  x = f(x, lane_move<0x112, 0xf>(x, x));
+  x = f(x, lane_move<0x114, 0xf>(x, x));
+  x = f(x, lane_move<0x118, 0xf>(x, x));
+  x = f(x, lane_move<0x142, 0xa>(x, x));
+  x = f(x, lane_move<0x143, 0xc>(x, x));
+  return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+__device__ __forceinline__ uint32_t wave_max(uint32_t x) {
+  return wave_fold(x, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
+}
+__device__ __forceinline__ uint32_t wave_min(uint32_t x) {
+  return wave_fold(x, [](uint32_t a, uint32_t b) { return a < b ? a : b; });
+}
+// sum of the lanes up to and including the lane's own
+__device__ __forceinline__ int wave_scan(int x) {
+  auto add = [](int a, uint32_t b) { return a + (int)b; };
+  x = add(x, lane_move<0x111, 0xf>(0u, (uint32_t)x));
+  x = add(x, lane_move<0x112, 0xf>(0u, (uint32_t)x));
+  x = add(x, lane_move<0x114, 0xf>(0u, (uint32_t)x));
+  x = add(x, lane_move<0x118, 0xf>(0u, (uint32_t)x));
+  x = add(x, lane_move<0x142, 0xa>(0u, (uint32_t)x));
+  return add(x, lane_move<0x143, 0xc>(0u, (uint32_t)x));
+}
+
 typedef __attribute__((address_space(3))) char* lds_char_ptr;
 
 // one KiB of a slab of rows of 128 bytes (8 of them), global -> LDS; the caller counts it in vmcnt

@@ -442,8 +442,7 @@ def block_sparse_attention(query_states, key_states, value_states, col_idx=None,
         stream_ptr = stream.cuda_stream if stream is not None else _stream_ptr(dev)
         # long lists are cut among workgroups where the problem has few q-blocks
         nb = (q_len + 127) // 128
-        ws_bytes = lib.xattn_block_sparse_workspace_bytes(
-            heads, q_len, k_len, idx_rows if col_idx is not None else nb, (qb1 if qb1 >= 0 else nb) - qb0)
+        ws_bytes = lib.xattn_block_sparse_workspace_bytes(heads, q_len, k_len, idx_rows, (qb1 if qb1 >= 0 else nb) - qb0)
         workspace = None
         if ws_bytes:
             # from the pool of the stream that writes it: what the current stream's pool hands out may still be in use by
