@@ -277,20 +277,20 @@ __device__ __forceinline__ void store_partial(float* part, int wave, int lane, i
   }
 }
 // The pieces' results combined into the registers of a finished sweep, in the order of the list.
-__device__ __forceinline__ void load_partials(float* part, int items, int wave, int lane, int r, int hh, f32x16 (&oacc)[4], float& l_run) {
+__device__ __forceinline__ void load_partials(float* part, int pieces, int wave, int lane, int r, int hh, f32x16 (&oacc)[4], float& l_run) {
   const int at = (128 * 128 + wave * 32 + r) * 4;
   auto ml = [&](int s, int which) __attribute__((always_inline)) {
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(part_resource(part + (int64_t)s * kPartFloats), at + which * 512, 0, kDeviceScope));
   };
   float m = -INFINITY, l = 0.f;
 #pragma unroll 4
-  for (int s = 0; s < items; ++s) m = fmaxf(m, ml(s, 0));
+  for (int s = 0; s < pieces; ++s) m = fmaxf(m, ml(s, 0));
   const float safe = m == -INFINITY ? 0.f : m;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int v = 0; v < 16; ++v) oacc[i][v] = 0.f;
-  for (int s = 0; s < items; ++s) {
+  for (int s = 0; s < pieces; ++s) {
     const __amdgpu_buffer_rsrc_t res = part_resource(part + (int64_t)s * kPartFloats);
     const float w = fast_exp2(ml(s, 0) - safe);      // 0 where the item saw no key of this row
     l += w * ml(s, 1);
@@ -325,7 +325,7 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
     const int pieces = ((const_i32_ptr)(uintptr_t)p.plan.noted)[0], per_xcd = (pieces + 7) / 8;   // (the low half)
     skip = per_xcd * 8;
     if ((int)blockIdx.x < skip) {
-      const int at = p.plan.in_turn ? (int)blockIdx.x : (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+      const int at = p.plan.shape.in_turn ? (int)blockIdx.x : (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
       if (at >= pieces) return;
       const_i32_ptr entry = (const_i32_ptr)(uintptr_t)p.plan.pieces + 2 * at;
       const int unit = entry[0];
@@ -361,7 +361,7 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
       n_blocks = visible;
     }
     if (kPlanned) {
-      const uint32_t cut = n_blocks > p.plan.min_piece ? (uint32_t)((const_i32_ptr)(uintptr_t)p.plan.cut)[slot] : 0;
+      const uint32_t cut = n_blocks > p.plan.shape.min_piece ? (uint32_t)((const_i32_ptr)(uintptr_t)p.plan.cut)[slot] : 0;
       if (cut != 0) {
         if (piece < 0) return;           // others have it
         cuts = cut_pieces(cut);
@@ -525,7 +525,7 @@ int xattn::block_sparse_impl(const void* q, const void* k, const void* v, void* 
   p.plan = AttnPlan{};
   if (plan) {
     p.plan = *plan;
-    const int64_t most = ((int64_t)p.H * (q_block_end - q_block_begin) * plan->items + 7) / 8 * 8;
+    const int64_t most = ((int64_t)(q_block_end - q_block_begin) * plan->shape.per_qb + 7) / 8 * 8;
     if (grid + most > 0x7fffffff) return XATTN_ERR_SHAPE;
     const dim3 wgs((unsigned)(grid + most));
     if (note) hipLaunchKernelGGL(note_lists_kernel, dim3(1), dim3(1024), 0, s, p);
@@ -555,10 +555,7 @@ extern "C" int xattn_block_sparse_fwd(const void* q, const void* k, const void* 
 }
 
 namespace {
-int items_of(int num_heads, int q_len, int k_len) {
-  const int nqb = (q_len + kBlk - 1) / kBlk;
-  return plan_items((int64_t)num_heads * nqb, nqb, (k_len + kBlk - 1) / kBlk);
-}
+PlanShape shape_of(int num_heads, int q_len, int k_len) { return plan_shape(num_heads, (q_len + kBlk - 1) / kBlk, (k_len + kBlk - 1) / kBlk); }
 }  // namespace
 
 extern "C" size_t xattn_block_sparse_workspace_bytes(int num_heads, int q_len, int k_len, int idx_rows, int q_blocks) {
@@ -568,7 +565,7 @@ extern "C" size_t xattn_block_sparse_workspace_bytes(int num_heads, int q_len, i
     if ((int64_t)num_heads * nqb > kEvenUnits) return 0;
     idx_rows = nqb;
   }
-  return plan_bytes((int64_t)num_heads * idx_rows, (int64_t)num_heads * q_blocks, nqb, items_of(num_heads, q_len, k_len));
+  return plan_bytes(shape_of(num_heads, q_len, k_len), (int64_t)num_heads * idx_rows, q_blocks);
 }
 
 extern "C" int xattn_block_sparse_fwd_ws(const void* q, const void* k, const void* v, void* out, void* workspace,
@@ -588,8 +585,7 @@ extern "C" int xattn_block_sparse_fwd_ws(const void* q, const void* k, const voi
     if (!workspace) return XATTN_ERR_NULL;
     if (workspace_bytes < need) return XATTN_ERR_WORKSPACE;
     if (reinterpret_cast<uintptr_t>(workspace) & 255) return XATTN_ERR_ALIGN;
-    plan = plan_at(static_cast<char*>(workspace), (int64_t)num_heads * idx_rows, (int64_t)num_heads * q_blocks, (int64_t)num_heads * nqb,
-                   nqb, (k_len + kBlk - 1) / kBlk, items_of(num_heads, q_len, k_len));
+    plan = plan_at(shape_of(num_heads, q_len, k_len), static_cast<char*>(workspace), (int64_t)num_heads * idx_rows, q_blocks);
   }
   return block_sparse_impl(q, k, v, out, col_idx, col_cnt, idx_pitch, idx_rows, idx_row0, num_heads, num_kv_heads, q_len, k_len,
                            head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n, o_stride_h,

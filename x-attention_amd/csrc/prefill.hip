@@ -19,7 +19,7 @@ namespace {
 struct PrefillLayout {
   size_t est_bytes, cnt_off, idx_off, plan_off, total;
   int nqb, nkb;
-  int items;   // most items of a list (attn_plan.h)
+  PlanShape plan;
 };
 
 size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -34,8 +34,8 @@ bool prefill_layout(int num_heads, int q_len, int k_len, int stride, int chunk_s
   l->idx_off = l->cnt_off + up256((size_t)num_heads * l->nqb * sizeof(int32_t));
   l->plan_off = l->idx_off + up256((size_t)num_heads * l->nqb * l->nkb * sizeof(int32_t));
   const int64_t units = (int64_t)num_heads * l->nqb;
-  l->items = plan_items(units, l->nqb, l->nkb);
-  l->total = l->plan_off + plan_bytes(units, units, l->nqb, l->items);
+  l->plan = plan_shape(num_heads, l->nqb, l->nkb);
+  l->total = l->plan_off + plan_bytes(l->plan, units, l->nqb);
   return true;
 }
 }  // namespace
@@ -71,13 +71,13 @@ extern "C" int xattn_prefill_fwd(const void* q, const void* k, const void* v, vo
   sel.real_q_blocks_only = 1;
   sel.stages = 3;
   const int64_t units = (int64_t)num_heads * l.nqb;
-  const AttnPlan plan = plan_at(ws + l.plan_off, units, units, units, l.nqb, l.nkb, l.items);
+  const AttnPlan plan = plan_at(l.plan, ws + l.plan_off, units, l.nqb);
   // (with zero_rows_from 0 no row is estimated, and no MFMA pass would clear what is noted: noted afterwards)
   // Where no list can be long enough to be cut, nothing is noted (nor planned below): then the selection may follow the
   // estimate in the same kernel.
   const int q_chunks = (int)(((int64_t)q_len + chunk_size - 1) / chunk_size), k_chunks = (int)(((int64_t)k_len + chunk_size - 1) / chunk_size);
   const int64_t last_token = (int64_t)l.nqb * 128 - 1 + (int64_t)(k_chunks - q_chunks) * chunk_size;   // on the key axis, both padded
-  const bool may_cut = plan.items && (!causal || keep_sink || last_token / 128 + 1 > plan.min_piece);
+  const bool may_cut = l.plan.per_qb && (!causal || keep_sink || last_token / 128 + 1 > l.plan.min_piece);
   if (may_cut && zero_rows_from != 0) sel.plan = &plan;
   int rc = estimate_impl(q, k, nullptr, ws, l.est_bytes, nullptr, num_heads, num_kv_heads, q_len, k_len, head_dim,
                          q_stride_h, q_stride_n, k_stride_h, k_stride_n, stride, 128, chunk_size, 0, q_chunks, causal,

@@ -23,7 +23,7 @@ struct SelParams {
   int causal, keep_sink, keep_recent, list_cols, q_len, kv_off;
   int blocks_per_chunk;
   int npow2;   // LDS key capacity (power of two >= nkb)
-  AttnPlan plan;   // items 0: nothing is noted
+  AttnPlan plan;   // per_qb 0: nothing is noted
 };
 
 constexpr int kSlots = 16;        // candidates per lane held in registers (rows up to 1024 candidates)
@@ -401,7 +401,7 @@ __device__ __forceinline__ void select_row(const SelParams& p, const float* x, i
     }
     count = count < p.idx_pitch ? count : (int)p.idx_pitch;
     if (lane == 0) p.col_cnt[slot] = count;
-    if (p.plan.items && (p.causal ? q_last / 128 + 1 : p.list_cols) > p.plan.min_piece)   // else too few blocks to be cut
+    if (p.plan.shape.per_qb && (p.causal ? q_last / 128 + 1 : p.list_cols) > p.plan.shape.min_piece)   // else too few blocks to be cut
       list_made(p.plan, p.H, p.win_rows, row - p.win_row0, head, count, lane);
   }
 }
