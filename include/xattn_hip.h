@@ -221,8 +221,8 @@ int xattn_block_sparse_fwd(const void* q, const void* k, const void* v, void* ou
  * (head, q-block) units for the longest not to matter (attn_plan.h).
  * `workspace`: xattn_block_sparse_workspace_bytes() bytes for the q_blocks =
  * q_block_end - q_block_begin q-blocks of the launch, 256-byte aligned,
- * contents undefined on entry and on return; 0 bytes (null allowed) means that
- * nothing is cut.  Without lists (col_idx null; idx_rows = 0 for the size) the
+ * contents undefined on entry and on return, at most 170 MB; 0 bytes (null
+ * allowed) means that nothing is cut.  Without lists (col_idx null; idx_rows = 0 for the size) the
  * visible blocks of a unit are its list.  Where a list is cut depends on the
  * lengths of its q-block's lists over all heads, num_heads, q_len and k_len
  * only, so results do not depend on how q-blocks are spread over launches; a
@@ -243,14 +243,18 @@ int xattn_block_sparse_fwd_ws(const void* q, const void* k, const void* v, void*
  * The prefill operator in one call (Xattention_prefill, xattn/src/Xattention.py:
  * 302-402): estimate, selection and block-sparse attention enqueued back to
  * back, everything between them in `workspace` (at least
- * xattn_prefill_workspace_bytes() bytes, 256-byte aligned, contents undefined on
- * entry and on return; 0 bytes means the geometry is refused).  Arguments as in
+ * xattn_prefill_least_workspace_bytes() bytes, 256-byte aligned, contents
+ * undefined on entry and on return; 0 bytes means the geometry is refused).  With
+ * xattn_prefill_workspace_bytes() bytes, up to 170 MB more, long lists may be cut
+ * among workgroups as in xattn_block_sparse_fwd_ws; with less they stay whole.
+ * Arguments as in
  * xattn_estimate_select and xattn_block_sparse_fwd, over all query chunks.
  * Thresholds: `tau_device` (fp64 [H] on the device) or, when that is null,
  * `tau_host` with one value for all heads or one per head (at most 64), copied
  * at the call.  At most 8192 key blocks (padded).
  */
 size_t xattn_prefill_workspace_bytes(int num_heads, int q_len, int k_len, int stride, int chunk_size);
+size_t xattn_prefill_least_workspace_bytes(int num_heads, int q_len, int k_len, int stride, int chunk_size);
 
 int xattn_prefill_fwd(const void* q, const void* k, const void* v, void* out, void* workspace,
                       size_t workspace_bytes, int num_heads, int num_kv_heads, int q_len, int k_len, int head_dim,

@@ -138,3 +138,34 @@ def test_a_side_stream_leaves_memory_of_queued_work_alone():
     torch.cuda.synchronize()
     assert not touched.item()
     assert torch.equal(got, want)
+
+
+def test_lists_stay_whole_on_a_full_gpu():
+    """No memory for partial results: the calls run, as they do without them."""
+    from xattn.src import hip_backend as hb
+    from xattn.src.Xattention import Xattention_prefill, block_sparse_attention, estimate_and_select
+
+    heads, kv_heads, q_len, k_len = 32, 8, 2048, 14336
+    q, k, v = _inputs(q_len, k_len, heads, kv_heads, 9)
+    taus = _taus(heads, [2, 17])
+    r = estimate_and_select(q, k, 8, taus, 128, want_mask=False, want_sums=False)
+    idx, cnt = r["col_idx"], r["col_cnt"]
+    r = None
+    whole = _swept_whole(q, k, v, idx, cnt, True)
+    cut = Xattention_prefill(q, k, v, 8, threshold=taus, chunk_size=128)
+    assert not torch.equal(cut.float(), whole)                   # (there is something to cut)
+    lib = hb.lib()
+    least = lib.xattn_prefill_least_workspace_bytes(heads, q_len, k_len, 8, 128)
+    assert lib.xattn_prefill_workspace_bytes(heads, q_len, k_len, 8, 128) - least > 150 << 20
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    room = torch.cuda.memory_reserved() + least + 2 * q.numel() * 2 + (64 << 20)
+    torch.cuda.set_per_process_memory_fraction(room / torch.cuda.get_device_properties(0).total_memory)
+    try:
+        full = Xattention_prefill(q, k, v, 8, threshold=taus, chunk_size=128)
+        listed = block_sparse_attention(q, k, v, idx, cnt)
+        torch.cuda.synchronize()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(full.float(), whole) and torch.equal(listed.float(), whole)
+    assert torch.equal(Xattention_prefill(q, k, v, 8, threshold=taus, chunk_size=128), cut)

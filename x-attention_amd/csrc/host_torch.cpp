@@ -133,14 +133,22 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const c10::Device dev = q->device();
   if (v->device() != dev || v->size(0) != 1 || v->size(1) != c.Hkv || v->size(2) != c.Lk) Py_RETURN_NONE;
   const int H = (int)c.H, Lq = (int)c.Lq;
-  const size_t bytes = xattn_prefill_workspace_bytes(H, Lq, (int)c.Lk, c.stride, (int)chunk);
+  size_t bytes = xattn_prefill_workspace_bytes(H, Lq, (int)c.Lk, c.stride, (int)chunk);
   if (bytes == 0 || (long long)bytes > limit) Py_RETURN_NONE;
   OnDevice on(dev);
   Tau tau;
   if (!read_tau(args[5], H, dev, &tau)) Py_RETURN_NONE;
   at::Tensor out = at::empty_strided({1, H, Lq, 128}, {(int64_t)Lq * H * 128, 128, (int64_t)H * 128, 1},
                                      at::TensorOptions().device(dev).dtype(at::kBFloat16));
-  const c10::DataPtr ws = c10::hip::HIPCachingAllocator::get()->allocate(bytes);
+  c10::DataPtr ws;
+  try {
+    ws = c10::hip::HIPCachingAllocator::get()->allocate(bytes);
+  } catch (const c10::OutOfMemoryError&) {
+    // most of it (up to 170 MB) is for lists cut into pieces: on a GPU that is full they stay whole
+    const size_t least = xattn_prefill_least_workspace_bytes(H, Lq, (int)c.Lk, c.stride, (int)chunk);
+    if (least >= bytes) throw;
+    ws = c10::hip::HIPCachingAllocator::get()->allocate(bytes = least);
+  }
   const int rc = xattn_prefill_fwd(
       q->data_ptr(), k->data_ptr(), v->data_ptr(), out.data_ptr(), ws.get(), bytes, H, (int)c.Hkv, Lq, (int)c.Lk, 128, q->stride(1),
       q->stride(2), k->stride(1), k->stride(2), v->stride(1), v->stride(2), 128, (int64_t)H * 128, c.stride, (int)chunk, causal,

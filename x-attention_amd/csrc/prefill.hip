@@ -45,6 +45,11 @@ extern "C" size_t xattn_prefill_workspace_bytes(int num_heads, int q_len, int k_
   return prefill_layout(num_heads, q_len, k_len, stride, chunk_size, &l) ? l.total : 0;
 }
 
+extern "C" size_t xattn_prefill_least_workspace_bytes(int num_heads, int q_len, int k_len, int stride, int chunk_size) {
+  PrefillLayout l;
+  return prefill_layout(num_heads, q_len, k_len, stride, chunk_size, &l) ? l.plan_off : 0;
+}
+
 extern "C" int xattn_prefill_fwd(const void* q, const void* k, const void* v, void* out, void* workspace,
                                  size_t workspace_bytes, int num_heads, int num_kv_heads, int q_len, int k_len,
                                  int head_dim, int64_t q_stride_h, int64_t q_stride_n, int64_t k_stride_h,
@@ -56,7 +61,7 @@ extern "C" int xattn_prefill_fwd(const void* q, const void* k, const void* v, vo
   if (!workspace || !v || !out) return XATTN_ERR_NULL;
   PrefillLayout l;
   if (!prefill_layout(num_heads, q_len, k_len, stride, chunk_size, &l)) return XATTN_ERR_SHAPE;
-  if (workspace_bytes < l.total) return XATTN_ERR_WORKSPACE;
+  if (workspace_bytes < l.plan_off) return XATTN_ERR_WORKSPACE;
   if (reinterpret_cast<uintptr_t>(workspace) & 255) return XATTN_ERR_ALIGN;
   char* ws = static_cast<char*>(workspace);
   SelectArgs sel{};
@@ -71,6 +76,7 @@ extern "C" int xattn_prefill_fwd(const void* q, const void* k, const void* v, vo
   sel.real_q_blocks_only = 1;
   sel.stages = 3;
   const int64_t units = (int64_t)num_heads * l.nqb;
+  if (workspace_bytes < l.total) l.plan = PlanShape{};      // lists stay whole
   const AttnPlan plan = plan_at(l.plan, ws + l.plan_off, units, l.nqb);
   // (with zero_rows_from 0 no row is estimated, and no MFMA pass would clear what is noted: noted afterwards)
   // Where no list can be long enough to be cut, nothing is noted (nor planned below): then the selection may follow the

@@ -448,20 +448,22 @@ def block_sparse_attention(query_states, key_states, value_states, col_idx=None,
             # from the pool of the stream that writes it: what the current stream's pool hands out may still be in use by
             # work queued there, for which `stream` does not wait
             with torch.cuda.stream(stream):
-                workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-        _hb.check(
-            lib.xattn_block_sparse_fwd_ws(
-                q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-                workspace.data_ptr() if workspace is not None else None, ws_bytes,
-                col_idx.data_ptr() if col_idx is not None else None,
-                col_cnt.data_ptr() if col_cnt is not None else None,
-                pitch, idx_rows, idx_row0, heads, kv_heads, q_len, k_len, 128,
-                q.stride(1), q.stride(2), k.stride(1), k.stride(2), v.stride(1), v.stride(2),
-                out.stride(2), out.stride(1), qb0, qb1, int(bool(causal)), scale,
-                stream_ptr,
-            ),
-            "xattn_block_sparse_fwd_ws",
+                try:
+                    workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+                except torch.OutOfMemoryError:
+                    pass                        # up to 170 MB: on a GPU that is full, lists stay whole
+        args = (
+            col_idx.data_ptr() if col_idx is not None else None,
+            col_cnt.data_ptr() if col_cnt is not None else None,
+            pitch, idx_rows, idx_row0, heads, kv_heads, q_len, k_len, 128,
+            q.stride(1), q.stride(2), k.stride(1), k.stride(2), v.stride(1), v.stride(2),
+            out.stride(2), out.stride(1), qb0, qb1, int(bool(causal)), scale, stream_ptr,
         )
+        tensors = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr())
+        if workspace is not None:
+            _hb.check(lib.xattn_block_sparse_fwd_ws(*tensors, workspace.data_ptr(), ws_bytes, *args), "xattn_block_sparse_fwd_ws")
+        else:
+            _hb.check(lib.xattn_block_sparse_fwd(*tensors, *args), "xattn_block_sparse_fwd")
     return out.transpose(1, 2)
 
 

@@ -42,6 +42,7 @@ _SIGNATURES = {
     "xattn_block_mass": (c_i32, [c_vp] * 3 + [c_i32] * 5 + [c_i64] * 4 + [c_i32, c_f32, c_vp]),
     "xattn_threshold_rows": (c_i32, [c_vp] * 3 + [c_i32] * 3 + [c_i64] * 2 + [c_f32, c_vp]),
     "xattn_prefill_workspace_bytes": (c_sz, [c_i32] * 5),
+    "xattn_prefill_least_workspace_bytes": (c_sz, [c_i32] * 5),
     "xattn_prefill_fwd": (
         c_i32,
         [c_vp] * 5 + [c_sz] + [c_i32] * 5 + [c_i64] * 8 + [c_i32] * 4 + [c_f32, c_i32]
