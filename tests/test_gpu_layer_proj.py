@@ -59,3 +59,49 @@ def test_modules_that_are_more_than_a_linear_are_called():
     lin.forward = lambda x: x
     assert _linear_params(lin) is None
     assert _linear_params(torch.nn.Identity()) is None
+
+
+def test_a_linear_replaced_on_the_class_is_called(monkeypatch):
+    """A wrapper around torch.nn.Linear.forward, or a mode, sees the layer's four products."""
+    import types
+
+    from xattn.src.load_llama import FastPrefillConfig, forward_eval
+
+    heads, kv_heads, width, tokens = 4, 2, 256, 70
+    g = torch.Generator(device="cuda").manual_seed(0)
+    mod = types.SimpleNamespace(config=types.SimpleNamespace(num_attention_heads=heads, num_key_value_heads=kv_heads), head_dim=128,
+                                layer_idx=0, fastprefillconfig=FastPrefillConfig(threshold=0.9))
+    for name, n, k in (("q_proj", heads * 128, width), ("k_proj", kv_heads * 128, width), ("v_proj", kv_heads * 128, width),
+                       ("o_proj", width, heads * 128)):
+        lin = torch.nn.Linear(k, n, bias=False, device="cuda", dtype=torch.bfloat16).requires_grad_(False)
+        lin.weight.copy_(torch.randn(n, k, generator=g, device="cuda") / k ** 0.5)
+        setattr(mod, name, lin)
+    x = torch.randn(1, tokens, width, generator=g, device="cuda").bfloat16()
+    ang = torch.rand(1, tokens, 128, generator=g, device="cuda") * 3
+    pos = (ang.cos().bfloat16(), ang.sin().bfloat16())
+    plain = torch.nn.Linear.forward
+    calls = []
+
+    def forward(self, a):
+        calls.append(tuple(self.weight.shape))
+        return plain(self, a)
+
+    with torch.no_grad():
+        want = forward_eval(mod, x, position_embeddings=pos)[0]
+        assert not calls
+        monkeypatch.setattr(torch.nn.Linear, "forward", forward)
+        got = forward_eval(mod, x, position_embeddings=pos)[0]
+        assert len(calls) == 4
+        monkeypatch.undo()
+        seen = []
+
+        class Mode(torch.overrides.TorchFunctionMode):
+            def __torch_function__(self, func, types, args=(), kwargs=None):
+                seen.append(func)
+                return func(*args, **(kwargs or {}))
+
+        with Mode():
+            forward_eval(mod, x, position_embeddings=pos)
+        assert seen.count(torch.nn.functional.linear) == 4
+    # products rounded to bf16 by both, their sums in another order, through a softmax and one more product
+    assert (got.float() - want.float()).norm() <= 2e-2 * want.float().norm()

@@ -143,3 +143,57 @@ def test_static_cache_branch_on_the_host(monkeypatch, mode):
         cos, sin = ours.model.rotary_emb(h, pos)
         out = layer(h, position_embeddings=(cos, sin), past_key_values=cache2, position_ids=pos)[0]
         assert out.shape == (1, 10, 256) and torch.isfinite(out).all()
+
+
+class _Function(torch.overrides.TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+class _Dispatch(torch.utils._python_dispatch.TorchDispatchMode):
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+def _wrapped(fn):
+    import functools
+
+    @functools.wraps(fn)
+    def call(*args, **kwargs):
+        return fn(*args, **kwargs)
+
+    return call
+
+
+@pytest.mark.parametrize("owner,name", [(torch.nn.Linear, "forward"), (torch.nn.functional, "linear"), (torch.nn.Module, "__call__"),
+                                        (torch.nn.Module, "_call_impl")])
+def test_a_replaced_linear_is_called(monkeypatch, owner, name):
+    from xattn.src import load_llama
+
+    assert not load_llama._observed()
+    monkeypatch.setattr(owner, name, _wrapped(getattr(owner, name)))
+    assert load_llama._observed()
+    # ... also by a wrapper that was there before the import
+    assert not load_llama._torch_own(getattr(owner, name), torch.nn.modules.linear)
+    assert not load_llama._torch_own(getattr(owner, name), torch.nn.modules.module)
+
+
+def test_modes_and_transforms_see_the_projections():
+    from xattn.src import load_llama
+
+    for mode in (_Function, _Dispatch, torch.autograd.forward_ad.dual_level):
+        with mode():
+            assert load_llama._observed()
+    seen = []
+    torch.func.vmap(lambda x: (seen.append(load_llama._observed()), x)[1])(torch.zeros(2, 3))
+    torch.jit.trace(lambda x: (seen.append(load_llama._observed()), x + 1)[1], torch.zeros(3), check_trace=False)
+    assert seen == [True, True]
+    with torch.device("cpu"):                       # a default device concerns new tensors only
+        assert not load_llama._observed()
+        with _Function():
+            assert load_llama._observed()
+    assert not load_llama._observed()
+    lin = torch.nn.Linear(128, 128)
+    assert load_llama._linear_params(lin) is not None
+    lin._compiled_call_impl = lin._call_impl
+    assert load_llama._linear_params(lin) is None

@@ -21,6 +21,8 @@ import sys
 import time
 
 import torch
+import torch.autograd.forward_ad
+import torch.utils._device
 
 from . import hip_backend as _hb
 from .decode import single_decode_with_kv_cache
@@ -100,11 +102,47 @@ def _is_static_cache(cache):
 _module_hooks = torch.nn.modules.module
 
 
+def _torch_own(fn, module):
+    """Whether a function comes from the file of a torch module, as it does unless something has replaced it."""
+    code = getattr(fn, "__code__", None)
+    return code is not None and code.co_filename == module.__file__
+
+
+_Linear, _functional = torch.nn.Linear, torch.nn.functional
+
+
+def _linear_call():
+    """What a call of a ``torch.nn.Linear`` goes through."""
+    return _Linear.__call__, _Linear._call_impl, _Linear.forward, _functional.linear
+
+
+_own_linear_call = _linear_call()
+if not (all(_torch_own(fn, _module_hooks) for fn in _own_linear_call[:2])
+        and _torch_own(_own_linear_call[2], torch.nn.modules.linear) and _own_linear_call[3] is torch._C._nn.linear):
+    _own_linear_call = None      # replaced before this module was imported
+_function_modes, _dispatch_modes = torch._C._len_torch_function_stack, torch._C._len_torch_dispatch_stack
+_forward_ad, _transform, _tracer = torch.autograd.forward_ad, torch._C._functorch.peek_interpreter_stack, torch._C._get_tracing_state
+
+
+def _observed():
+    """Whether something wants to see the calls that torch functions and modules make: a function or dispatch mode
+    (other than a default device, which only concerns new tensors), forward-mode differentiation, a functorch transform, a
+    tracer, or a replaced part of ``torch.nn.Linear``'s call."""
+    if _linear_call() != _own_linear_call:
+        return True
+    if _function_modes() and any(type(m) is not torch.utils._device.DeviceContext
+                                 for m in torch.overrides._get_current_function_mode_stack()):
+        return True
+    return bool(_dispatch_modes()) or _forward_ad._current_level >= 0 or _transform() is not None or _tracer() is not None
+
+
 def _linear_params(mod):
-    """(weight, bias) of a projection that is nothing but ``torch.nn.Linear`` - no hooks, no replaced forward, no
-    wrapped or quantized weight - so that its product may be computed without calling the module; else None."""
+    """(weight, bias) of a projection that is nothing but ``torch.nn.Linear`` - no hooks, no replaced forward, not
+    compiled, no wrapped or quantized weight - so that its product may be computed without calling the module where
+    nothing observes the call; else None."""
     own = mod.__dict__
     if (type(mod) is not torch.nn.Linear or "forward" in own or own["_forward_hooks"] or own["_forward_pre_hooks"]
+            or own.get("_compiled_call_impl") is not None
             or _module_hooks._global_forward_hooks or _module_hooks._global_forward_pre_hooks):
         return None
     weight, bias = own["_parameters"].get("weight"), own["_parameters"].get("bias")
@@ -116,7 +154,7 @@ def _linear_params(mod):
 def _project(self, hidden_states, cos, sin, heads, kv_heads):
     """Rotated q and k and v of a layer from the native host path (one kernel up to about a thousand tokens, the library
     GEMMs and one rotation kernel for more), or None where the layer's own modules have to be called."""
-    if not hidden_states.is_cuda or self.head_dim != 128:
+    if self.head_dim != 128:
         return None
     q, k, v = _linear_params(self.q_proj), _linear_params(self.k_proj), _linear_params(self.v_proj)
     if q is None or k is None or v is None:
@@ -152,9 +190,11 @@ def forward_eval(self, hidden_states, position_embeddings=None, attention_mask=N
     kv_heads = self.config.num_key_value_heads
     head_dim = self.head_dim
 
+    native = hidden_states.is_cuda and type(hidden_states) is torch.Tensor and not _observed()
     qkv = None
     if position_embeddings is not None:
         cos, sin = position_embeddings
+    if position_embeddings is not None and native:
         qkv = _project(self, hidden_states, cos, sin, heads, kv_heads)
     if qkv is not None:
         query_states, key_states, value_states = qkv
@@ -216,7 +256,7 @@ def forward_eval(self, hidden_states, position_embeddings=None, attention_mask=N
             f"`attn_output` should be of size {(bsz, heads, q_len, head_dim)}, but is {attn_output.size()}"
         )
     attn_output = attn_output.transpose(1, 2).reshape(bsz, q_len, heads * head_dim)
-    out_proj = _linear_params(self.o_proj) if attn_output.is_cuda else None
+    out_proj = _linear_params(self.o_proj) if native else None
     projected = _hb.host().output(attn_output, *out_proj) if out_proj is not None else None
     attn_output = projected if projected is not None else self.o_proj(attn_output)
     _stamp(cfg, "Post-attention processing", start)
