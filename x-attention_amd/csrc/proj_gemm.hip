@@ -5,10 +5,24 @@
 // CUs at work, half of it W's - so the tile is the largest that still gives most CUs one: 64 x 64 up to 256 tiles, then
 // 64 tokens x 128 features, then 128 x 128, and two workgroups per CU for q, k and v beyond that.  Splitting a
 // step's depth over two groups of wavefronts helps the smallest tile only (17.6 -> 13.3 us at 64 tokens), where the
-// chain of 64 steps is the time.  4096 wide, 32 + 2 * 8 heads, library products against this kernel, us: q, k, v (three
-// launches; the rotation's own 4 to 5 come on top) 57 -> 13.3 at 64 tokens, 57 -> 21 at 200, 57 -> 30 at 500, 65 -> 51 at
-// 700, 71 -> 54 at 1000, 90 -> 94 at 1500; output 19 -> 13 at 64, 19 -> 14 at 200, 24.5 -> 22 at 500, 35.5 -> 33.6 at 1000,
-// 47 -> 54 at 1500.  Weights of that layer are 50 and 34 MB: 10 and 6.5 us at the rate of a large copy.
+// chain of 64 steps is the time.
+//
+// Library products against this kernel, weights from memory, in a captured graph, us.  q, k, v (three launches, and 4 to 5 for
+// the rotation) by tokens:
+//   width, heads      64         200        500        700        1000       1280       1500
+//   1024   8 + 2*8    27 / 7     27 / 7     28 / 9.5   30 / 12.5  30 / 13    33 / 14    34 / 19
+//   2048   32 + 2*8   36 / 14    38 / 16.5  43 / 24    50 / 36    53 / 41    59 / 43    library
+//   3584   28 + 2*4   40 / 19    42 / 23.5  50 / 35    67 / 33    71 / 55    81 / 61    82 / 66
+//   4096   32 + 2*8   46 / 22    48 / 28    63 / 39    75 / 64    87 / 72    100 / 78   library
+//   5120   40 + 2*8   60 / 31    61 / 36    89 / 54    105 / 83   118 / 98   library
+//   8192   64 + 2*8   62 / 45    95 / 65    134 / 134  165 / 144  library
+// Output (features x depth): 1024 x 1024 8.8 / 6.2, 8.4 / 6.1, 8.6 / 6.3, 9.1 / 6.5, 9.0 / 6.6, 9.6 / 7.8, 9.6 / 7.9;
+// 4096 x 4096 14.4 / 19.3, 20.8 / 16.5, 28 / 27, 31 / 33, 39 / 37, library; 3072 x 3072 16 / 18, 17.5 / 14, 21 / 24, 26 / 28,
+// 29.5 / 31.6, 32 / 34; 8192 x 8192 33 / 43, 53 / 52, 81 / 77.  The library's stand within 16 % of this kernel's from 65 tokens on,
+// one way or the other.  Up to 64 there is a single row of tiles, each a chain over the whole depth, which the library splits;
+// so it does where the features are fewer than the depth (2048 x 4096 at 64 / 128 / 200 / 257 tokens 14 / 21, 13 / 20, 14.5 / 16,
+// 21 / 16).  Such a turn is bound by the host's calls, though, and the library's is the dearer one: the whole layer, 4096 wide, on
+// 6000 tokens with the library's output product / this kernel's, 2 tokens 70 / 62, 16 68 / 64, 64 68 / 74.5, 100 68 / 68.
 #include "lds_limit.h"
 #include "rotate.h"
 #include "xattn_hip.h"
