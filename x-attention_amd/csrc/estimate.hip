@@ -182,7 +182,6 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
   const int r = lane & 31, hh = lane >> 5;
   const int wm = wave & 3, wn = wave >> 2;   // query quarter, key half
   constexpr int kMT = kHalf ? 1 : 2;         // 32-row query tiles of a wavefront
-  for (int i = (int)blockIdx.x * kWaves * 64 + tid; i < p.noted_words; i += (int)gridDim.x * kWaves * 64) p.noted[i] = 0;
   // A workgroup works through tiles id, id + grid, ...: one workgroup fits a CU, so nothing else could hide
   // the wait for a tile's first slabs.  The slab pipeline therefore runs on across the tile boundary: the load
   // slots of a tile's last two k-steps fetch the first slabs of the NEXT tile, and the last sub-step reads its
@@ -195,6 +194,8 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
     return kPacked ? decode_packed(p, i, h, m, n) : kHalf ? decode_half(p, i, cursor, h, m, n) : decode_tile(p, i, cursor, h, m, n);
   };
   if (!decode(id, &head, &m0, &n0)) return;
+  if (blockIdx.x == 0)                       // (it always has a tile)
+    for (int i = tid; i < p.noted_words; i += kWaves * 64) p.noted[i] = 0;
 
   const int64_t q_snb = p.q_sn * 2, k_snb = p.k_sn * 2;
   const int64_t span = (int64_t)kTile * p.S;
