@@ -148,9 +148,9 @@ __host__ __device__ inline int cut_pieces(uint32_t w) { return (int)(w >> 14 & 1
 __host__ __device__ inline int cut_length(uint32_t w) { return (int)(w & 16383); }
 
 // Notes the lists of one q-block, `total` blocks in all, by a whole wavefront: count(h) is the length of head h's where it
-// is longer than min_piece, unit0 + h * unit_step its place.
-template <typename F>
-__device__ __forceinline__ void note_q_block(const AttnPlan& p, int heads, int total, int unit0, int unit_step, int lane, F count) {
+// is longer than min_piece, unit0 + h * unit_step its place; reserve(n), called by one lane, gives the place of its n pieces.
+template <typename F, typename R>
+__device__ __forceinline__ void note_q_block(const AttnPlan& p, int heads, int total, int unit0, int unit_step, int lane, F count, R reserve) {
   const int first = lane < heads ? count(lane) : 0;
   auto length = [&](int h) { return h < 64 ? first : count(h); };
   int longest = 0;
@@ -166,7 +166,7 @@ __device__ __forceinline__ void note_q_block(const AttnPlan& p, int heads, int t
   });
   const int sum = blocks ? __builtin_amdgcn_readlane(upto, 63) : 0;
   int at = 0;
-  if (lane == 63 && sum > 0) at = (int)__hip_atomic_fetch_add(p.noted, (unsigned long long)sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (lane == 63 && sum > 0) at = reserve(sum);
   at = __builtin_amdgcn_readlane(at, 63) + upto - mine;
   for (int h = lane; h < heads; h += 64) {
     const int len = length(h), n = list_pieces(len, blocks), unit = unit0 + h * unit_step;
@@ -200,9 +200,10 @@ __device__ __forceinline__ void list_made(const AttnPlan& p, int heads, int rows
   const uint32_t lists = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)before);
   const int total = __builtin_amdgcn_readfirstlane((int)(uint32_t)(before >> 32)) + count;
   if ((lists & 0xffff) != (uint32_t)heads - 1 || (lists >> 16 == 0 && !is_long)) return;
-  note_q_block(p, heads, total, row, rows, lane, [&](int h) {
-    return (int)__hip_atomic_load(p.cut + (int64_t)h * rows + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  });
+  note_q_block(
+      p, heads, total, row, rows, lane,
+      [&](int h) { return (int)__hip_atomic_load(p.cut + (int64_t)h * rows + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); },
+      [&](int n) { return (int)__hip_atomic_fetch_add(p.noted, (unsigned long long)n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); });
 }
 
 }  // namespace xattn

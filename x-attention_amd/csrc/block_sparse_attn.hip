@@ -444,10 +444,10 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
 }
 
 // Notes the lists of q-blocks [qb_begin, qb_end) of every head, where the pass that made them has not (or, without
-// lists, the visible blocks of each).  One workgroup: it also clears the count of pieces.
+// lists, the visible blocks of each).  One workgroup, which counts the pieces in LDS.
 __global__ __launch_bounds__(1024) void note_lists_kernel(AttnParams p) {
-  if (threadIdx.x == 0) *p.plan.noted = 0;
-  __threadfence();
+  __shared__ int pieces;
+  if (threadIdx.x == 0) pieces = 0;
   __syncthreads();
   const int lane = threadIdx.x & 63;
   for (int qb = p.qb_begin + (int)(threadIdx.x >> 6); qb < p.qb_end; qb += 16) {
@@ -462,8 +462,11 @@ __global__ __launch_bounds__(1024) void note_lists_kernel(AttnParams p) {
     };
     int total = 0;
     for (int h = lane; h < p.H; h += 64) total += count(h) < 65536 ? count(h) : 65536;   // (a sum of at most 8192)
-    note_q_block(p.plan, p.H, __builtin_amdgcn_readlane(wave_scan(total), 63), row, p.idx_rows, lane, count);
+    note_q_block(p.plan, p.H, __builtin_amdgcn_readlane(wave_scan(total), 63), row, p.idx_rows, lane, count,
+                 [&](int n) { return __hip_atomic_fetch_add(&pieces, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); });
   }
+  __syncthreads();
+  if (threadIdx.x == 0) *p.plan.noted = (unsigned long long)pieces;
 }
 
 }  // namespace xattn
