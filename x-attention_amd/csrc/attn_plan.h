@@ -29,6 +29,7 @@ struct PlanShape {
   int units;                  // lists of the whole problem, heads x q-blocks
   int nqb;
   int in_turn;                // pieces go to the XCDs in turn
+  int last, last_pieces;      // the problem's last q-block, if rows are missing from it (else -1), and its share
 };
 
 struct AttnPlan {
@@ -38,15 +39,16 @@ struct AttnPlan {
   uint32_t* cut;              // [lists] of a list longer than min_piece: its length, until its q-block is noted, then its pieces
                               // (cut_word), or 0 if it stays whole
   int32_t* done;              // [lists] pieces of a cut list that are finished
-  int32_t* pieces;            // [q-blocks of the launch * per_qb][2] unit, index of the piece in its list
+  int32_t* pieces;            // [plan_pieces()][2] unit, index of the piece in its list
   float* part;                // [the same][kPartFloats]
   PlanShape shape;
 };
 
 // The 512 workgroup slots get about four pieces each (the problem taken to be like the q-block), fewer of which even out
 // less: 2048 tokens on 63488 806 us with up to 8192 pieces, 884 with 2048, 977 with 1024.  Of a prompt by itself, whose
-// units are many, two each up to 2048 units.  A quarter on top is for the pieces that rounding adds.  A plan so takes 85 or
-// 170 MB, and its launch has 1280 or 2560 workgroups beside the units, 1 to 2 us per thousand where they are spare.
+// units are many, two each up to 2048 units.  A quarter on top is for the pieces that rounding adds.  A last q-block that
+// lacks rows (see piece_blocks) may have 512.  A plan so takes up to 120 or 200 MB, and its launch has up to 1792 or 3072
+// workgroups beside the units, 1 to 2 us per thousand where they are spare.
 // Not cut: 16 key blocks or fewer, which make short lists; more than 4096 units of a prompt or 8192 on top of a cache at
 // least as long as the chunk (a prompt of 32768 tokens 2158 us uncut, 2781 in two: partial results and the spread of a KV
 // head over the chip cost more than the end of a long launch).
@@ -57,8 +59,9 @@ struct AttnPlan {
 // Pieces are noted q-block after q-block.  An XCD gets a run of them, adjacent q-blocks over the same keys - but of a long
 // prompt's, whose last q-blocks have pieces several times as long as the first, each XCD gets every eighth (runs / in turn, us:
 // prompts of 8000 tokens 211 / 218, 12000 430 / 392, 16000 664 / 609; 2048 on 63488 411 / 463, 1000 on 30000 219 / 248).
-inline PlanShape plan_shape(int heads, int nqb, int nkb) {
+inline PlanShape plan_shape(int heads, int q_len, int k_len) {
   PlanShape s{};
+  const int nqb = (int)(((int64_t)q_len + 127) / 128), nkb = (int)(((int64_t)k_len + 127) / 128);
   const int64_t units = (int64_t)heads * nqb;
   const bool cached = nkb >= 2 * nqb;
   if (nkb <= 16 || units > (cached ? 8192 : 4096)) return s;
@@ -71,6 +74,9 @@ inline PlanShape plan_shape(int heads, int nqb, int nkb) {
   const int64_t share = s.spread * 5 / 4 / nqb;
   s.per_qb = (int)(share < most ? share : most);
   if (s.per_qb < 2) s.per_qb = 0;
+  s.last = q_len % 128 ? nqb - 1 : -1;
+  s.last_pieces = (int)(most < 512 ? most : 512);
+  if (s.last_pieces < s.per_qb) s.last_pieces = s.per_qb;
   return s;
 }
 
@@ -78,9 +84,10 @@ inline PlanShape plan_shape(int heads, int nqb, int nkb) {
 // aligned).
 inline size_t plan_round(size_t x) { return (x + 255) & ~(size_t)255; }
 inline size_t plan_noted_bytes(int nqb) { return plan_round((size_t)(nqb + 1) * kNotedStep * 8); }
+inline size_t plan_pieces(const PlanShape& s, int q_blocks) { return (size_t)q_blocks * s.per_qb + (s.last >= 0 ? s.last_pieces - s.per_qb : 0); }
 inline size_t plan_bytes(const PlanShape& s, int64_t lists, int q_blocks) {
   if (s.per_qb == 0) return 0;
-  const size_t pieces = (size_t)q_blocks * s.per_qb;
+  const size_t pieces = plan_pieces(s, q_blocks);
   return plan_noted_bytes(s.nqb) + 2 * plan_round((size_t)lists * 4) + plan_round(pieces * 8) + pieces * kPartFloats * sizeof(float);
 }
 inline AttnPlan plan_at(const PlanShape& s, char* at, int64_t lists, int q_blocks) {
@@ -91,7 +98,7 @@ inline AttnPlan plan_at(const PlanShape& s, char* at, int64_t lists, int q_block
   p.cut = reinterpret_cast<uint32_t*>(at += plan_noted_bytes(s.nqb));
   p.done = reinterpret_cast<int32_t*>(at += plan_round((size_t)lists * 4));
   p.pieces = reinterpret_cast<int32_t*>(at += plan_round((size_t)lists * 4));
-  p.part = reinterpret_cast<float*>(at + plan_round((size_t)q_blocks * s.per_qb * 8));
+  p.part = reinterpret_cast<float*>(at + plan_round(plan_pieces(s, q_blocks) * 8));
   return p;
 }
 
@@ -99,15 +106,17 @@ inline AttnPlan plan_at(const PlanShape& s, char* at, int64_t lists, int q_block
 // workgroup slots.
 constexpr int kEvenUnits = 341;
 
-// Blocks of a piece of the lists of a q-block - `heads` of them with `total` blocks, the longest with `longest` - or 0: they
-// stay whole.  Of text whose heads keep unlike lists the longest is 2 to 5 times the mean, of video, fields, diffuse text
+// Blocks of a piece of the lists of q-block qb - `heads` of them with `total` blocks, the longest with `longest` - or 0: they
+// stay whole.  Where the last q-block lacks rows, its estimate is flat and the lists of all its heads are long, whatever the
+// others' are: 228 blocks against 6 for 1554 tokens on 37213.  These always are cut.  Otherwise, of text whose heads keep unlike lists the longest is 2 to 5 times the mean, of video, fields, diffuse text
 // and dense attention 1.0 to 1.25 times; these are cut where units leave slots idle (into three: long ones only).
 // Whole calls, us, not cut / cut whatever the lists: uneven text, 2048 tokens on 63488 1346 / 806, 4096 on 100000
 // 2283 / 1397, a prompt of 8000 248 / 211; video of 4096 tokens 135 / 152, of 18000 1432 / 1906; a field of 4096 230 / 297;
 // diffuse text of 16000 1654 / 2251; dense 2100 49 / 63, 16384 2008 / 2475; dense 500 on 8700 (128 units) 153 / 115; in
 // three with 512 units, dense 2048 on 16000 525 / 587, diffuse text 2048 on 63488 1700 / 1885.
-__host__ __device__ inline int piece_blocks(const PlanShape& s, int heads, int total, int longest) {
+__host__ __device__ inline int piece_blocks(const PlanShape& s, int qb, int heads, int total, int longest) {
   if (longest <= s.min_piece) return 0;
+  if (qb == s.last) return s.min_piece;
   int64_t n;
   if (2 * (int64_t)longest * heads >= 3 * (int64_t)total)
     n = ((int64_t)total * s.nqb + s.spread - 1) / s.spread;
@@ -117,7 +126,7 @@ __host__ __device__ inline int piece_blocks(const PlanShape& s, int heads, int t
     n = (longest + 2) / 3;
   else
     return 0;
-  return n > s.min_piece ? (int)(n < 0x3fffffff ? n : 0x3fffffff) : s.min_piece;
+  return n > s.min_piece ? (int)(n < 1 << 28 ? n : 1 << 28) : s.min_piece;
 }
 // Pieces of a list of `count` blocks, and their length, where a q-block's have `blocks`; 0: it is not cut (or too long for
 // cut_word: over 30 million keys)
@@ -129,15 +138,14 @@ __host__ __device__ inline int list_pieces(int count, int blocks) {
   if (blocks == 0 || count <= blocks || list_piece(count, blocks) >= 1 << 14) return 0;
   return (int)((uint32_t)(count - 1) / (uint32_t)list_piece(count, blocks)) + 1;
 }
-// The blocks of a q-block's pieces, given what its lists' pieces of a length add up to: twice as many if they are more than it
-// may have.  A list of n > b blocks has less than n / b + 1 < 2 n / b pieces of b, so with twice the b that piece_blocks gave
-// they are less than total / b, which is within a q-block's share.  (A caller's lists that repeat blocks may still have
-// more: then they stay whole.)
+// The blocks of a q-block's pieces, given what its lists' pieces of a length add up to: twice as many, and again, if they are
+// more than its share.  (A list of n > b blocks has less than n / b + 1 < 2 n / b pieces of b, so of twice the b that piece_blocks
+// gave an ordinary q-block they are less than total / b, which is within its share.)
 template <typename F>
-__host__ __device__ inline int fitting_blocks(const PlanShape& s, int heads, int total, int longest, F pieces_of) {
-  const int blocks = piece_blocks(s, heads, total, longest);
-  if (pieces_of(blocks) <= s.per_qb) return blocks;
-  return pieces_of(2 * blocks) <= s.per_qb ? 2 * blocks : 0;
+__host__ __device__ inline int fitting_blocks(const PlanShape& s, int qb, int heads, int total, int longest, F pieces_of) {
+  int blocks = piece_blocks(s, qb, heads, total, longest);
+  while (pieces_of(blocks) > (qb == s.last ? s.last_pieces : s.per_qb)) blocks *= 2;      // (none once no list is longer)
+  return blocks;
 }
 
 // Where the first piece of a list stands among all pieces (less than 2^14), how many there are (2 .. 16) and the length of all
@@ -147,10 +155,10 @@ __host__ __device__ inline int cut_at(uint32_t w) { return (int)(w >> 18); }
 __host__ __device__ inline int cut_pieces(uint32_t w) { return (int)(w >> 14 & 15) + 1; }
 __host__ __device__ inline int cut_length(uint32_t w) { return (int)(w & 16383); }
 
-// Notes the lists of one q-block, `total` blocks in all, by a whole wavefront: count(h) is the length of head h's where it
+// Notes the lists of q-block qb, `total` blocks in all, by a whole wavefront: count(h) is the length of head h's where it
 // is longer than min_piece, unit0 + h * unit_step its place; reserve(n), called by one lane, gives the place of its n pieces.
 template <typename F, typename R>
-__device__ __forceinline__ void note_q_block(const AttnPlan& p, int heads, int total, int unit0, int unit_step, int lane, F count, R reserve) {
+__device__ __forceinline__ void note_q_block(const AttnPlan& p, int qb, int heads, int total, int unit0, int unit_step, int lane, F count, R reserve) {
   const int first = lane < heads ? count(lane) : 0;
   auto length = [&](int h) { return h < 64 ? first : count(h); };
   int longest = 0;
@@ -158,7 +166,7 @@ __device__ __forceinline__ void note_q_block(const AttnPlan& p, int heads, int t
   longest = (int)wave_max((uint32_t)longest);
   if (longest <= p.shape.min_piece) return;
   int mine = 0, upto = 0;
-  const int blocks = fitting_blocks(p.shape, heads, total, longest, [&](int b) {
+  const int blocks = fitting_blocks(p.shape, qb, heads, total, longest, [&](int b) {
     mine = 0;
     for (int h = lane; h < heads; h += 64) mine += list_pieces(length(h), b);
     upto = wave_scan(mine);
@@ -181,8 +189,8 @@ __device__ __forceinline__ void note_q_block(const AttnPlan& p, int heads, int t
   }
 }
 
-// A wavefront has made the list of `count` blocks (the same in every lane) of `head` and the q-block in row `row` of the
-// `rows` rows that the lists hold per head.  Whoever brings the last of the q-block's lists notes them all: a long list's
+// A wavefront has made the list of `count` blocks (the same in every lane) of `head` and q-block `row`, one of the `rows` that
+// the lists hold per head (all of the problem's).  Whoever brings the last of the q-block's lists notes them all: a long list's
 // length has reached memory that every XCD sees before it is counted, short ones are counted only.  That is a wait for one
 // atomic (0.5 us of a prompt's 63 where no list is long), and for the last of unlike lists a store, a load and a second atomic
 // (the selection of 4096 tokens 14.3 -> 16.4 us, of 2048 on 63488 32 -> 34.5).
@@ -202,7 +210,7 @@ __device__ __forceinline__ void list_made(const AttnPlan& p, int heads, int rows
   const int total = __builtin_amdgcn_readfirstlane((int)(uint32_t)(before >> 32)) + count;
   if ((lists & 0xffff) != (uint32_t)heads - 1 || (lists >> 16 == 0 && !is_long)) return;
   note_q_block(
-      p, heads, total, row, rows, lane,
+      p, row, heads, total, row, rows, lane,
       [&](int h) { return (int)__hip_atomic_load(p.cut + (int64_t)h * rows + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); },
       [&](int n) { return (int)__hip_atomic_fetch_add(p.noted, (unsigned long long)n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); });
 }

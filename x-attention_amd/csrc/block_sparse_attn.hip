@@ -462,7 +462,7 @@ __global__ __launch_bounds__(1024) void note_lists_kernel(AttnParams p) {
     };
     int total = 0;
     for (int h = lane; h < p.H; h += 64) total += count(h) < 65536 ? count(h) : 65536;   // (a sum of at most 8192)
-    note_q_block(p.plan, p.H, __builtin_amdgcn_readlane(wave_scan(total), 63), row, p.idx_rows, lane, count,
+    note_q_block(p.plan, qb, p.H, __builtin_amdgcn_readlane(wave_scan(total), 63), row, p.idx_rows, lane, count,
                  [&](int n) { return __hip_atomic_fetch_add(&pieces, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); });
   }
   __syncthreads();
@@ -528,7 +528,7 @@ int xattn::block_sparse_impl(const void* q, const void* k, const void* v, void* 
   p.plan = AttnPlan{};
   if (plan) {
     p.plan = *plan;
-    const int64_t most = ((int64_t)(q_block_end - q_block_begin) * plan->shape.per_qb + 7) / 8 * 8;
+    const int64_t most = ((int64_t)plan_pieces(plan->shape, q_block_end - q_block_begin) + 7) / 8 * 8;
     if (grid + most > 0x7fffffff) return XATTN_ERR_SHAPE;
     const dim3 wgs((unsigned)(grid + most));
     if (note) hipLaunchKernelGGL(note_lists_kernel, dim3(1), dim3(1024), 0, s, p);
@@ -558,17 +558,19 @@ extern "C" int xattn_block_sparse_fwd(const void* q, const void* k, const void* 
 }
 
 namespace {
-PlanShape shape_of(int num_heads, int q_len, int k_len) { return plan_shape(num_heads, (q_len + kBlk - 1) / kBlk, (k_len + kBlk - 1) / kBlk); }
+PlanShape shape_of(int num_heads, int q_len, int k_len, bool listed) {
+  PlanShape s = plan_shape(num_heads, q_len, k_len);
+  if (listed) return s;
+  s.last = -1;                          // all lists of a q-block alike, and the last q-block's like the others'
+  if (s.units > kEvenUnits) s.per_qb = 0;
+  return s;
+}
 }  // namespace
 
 extern "C" size_t xattn_block_sparse_workspace_bytes(int num_heads, int q_len, int k_len, int idx_rows, int q_blocks) {
   if (num_heads <= 0 || q_len <= 0 || k_len <= 0 || idx_rows < 0 || q_blocks <= 0) return 0;
-  const int nqb = (q_len + kBlk - 1) / kBlk;
-  if (idx_rows == 0) {                 // all lists of a q-block alike
-    if ((int64_t)num_heads * nqb > kEvenUnits) return 0;
-    idx_rows = nqb;
-  }
-  return plan_bytes(shape_of(num_heads, q_len, k_len), (int64_t)num_heads * idx_rows, q_blocks);
+  const int64_t rows = idx_rows ? idx_rows : ((int64_t)q_len + kBlk - 1) / kBlk;
+  return plan_bytes(shape_of(num_heads, q_len, k_len, idx_rows != 0), num_heads * rows, q_blocks);
 }
 
 extern "C" int xattn_block_sparse_fwd_ws(const void* q, const void* k, const void* v, void* out, void* workspace,
@@ -588,7 +590,7 @@ extern "C" int xattn_block_sparse_fwd_ws(const void* q, const void* k, const voi
     if (!workspace) return XATTN_ERR_NULL;
     if (workspace_bytes < need) return XATTN_ERR_WORKSPACE;
     if (reinterpret_cast<uintptr_t>(workspace) & 255) return XATTN_ERR_ALIGN;
-    plan = plan_at(shape_of(num_heads, q_len, k_len), static_cast<char*>(workspace), (int64_t)num_heads * idx_rows, q_blocks);
+    plan = plan_at(shape_of(num_heads, q_len, k_len, col_idx != nullptr), static_cast<char*>(workspace), (int64_t)num_heads * idx_rows, q_blocks);
   }
   return block_sparse_impl(q, k, v, out, col_idx, col_cnt, idx_pitch, idx_rows, idx_row0, num_heads, num_kv_heads, q_len, k_len,
                            head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n, o_stride_h,

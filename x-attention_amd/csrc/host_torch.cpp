@@ -144,7 +144,7 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   try {
     ws = c10::hip::HIPCachingAllocator::get()->allocate(bytes);
   } catch (const c10::OutOfMemoryError&) {
-    // most of it (up to 170 MB) is for lists cut into pieces: on a GPU that is full they stay whole
+    // most of it (up to 200 MB) is for lists cut into pieces: on a GPU that is full they stay whole
     const size_t least = xattn_prefill_least_workspace_bytes(H, Lq, (int)c.Lk, c.stride, (int)chunk);
     if (least >= bytes) throw;
     ws = c10::hip::HIPCachingAllocator::get()->allocate(bytes = least);

@@ -34,7 +34,7 @@ bool prefill_layout(int num_heads, int q_len, int k_len, int stride, int chunk_s
   l->idx_off = l->cnt_off + up256((size_t)num_heads * l->nqb * sizeof(int32_t));
   l->plan_off = l->idx_off + up256((size_t)num_heads * l->nqb * l->nkb * sizeof(int32_t));
   const int64_t units = (int64_t)num_heads * l->nqb;
-  l->plan = plan_shape(num_heads, l->nqb, l->nkb);
+  l->plan = plan_shape(num_heads, q_len, k_len);
   l->total = l->plan_off + plan_bytes(l->plan, units, l->nqb);
   return true;
 }

@@ -451,7 +451,7 @@ def block_sparse_attention(query_states, key_states, value_states, col_idx=None,
                 try:
                     workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
                 except torch.OutOfMemoryError:
-                    pass                        # up to 170 MB: on a GPU that is full, lists stay whole
+                    pass                        # up to 200 MB: on a GPU that is full, lists stay whole
         args = (
             col_idx.data_ptr() if col_idx is not None else None,
             col_cnt.data_ptr() if col_cnt is not None else None,
