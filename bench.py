@@ -317,10 +317,10 @@ def summarize(w, L, tau, chunk, m, headline_traffic=False):
         "traffic": measured_traffic_bytes("xattn::estimate_gemm_kernel") if headline_traffic else None,
     }
     rl_att = {
-        "kernel": "block_sparse_fwd_kernel<true>", "bound": "mfma", "achieved": round(att_tf, 1),
+        "kernel": "block_sparse_fwd64_kernel<true>, block_sparse_fwd_kernel<true>", "bound": "mfma", "achieved": round(att_tf, 1),
         "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s", "frac": round(att_tf / PEAK_BF16_TFLOPS, 4), "ms": round(t_att, 3),
         "flop": fb["f_sparse"],
-        "traffic": measured_traffic_bytes("xattn::block_sparse_fwd_kernel<true") if headline_traffic else None,
+        "traffic": measured_traffic_bytes("xattn::block_sparse_fwd64_kernel<true") if headline_traffic else None,
     }
     sel_gbs = fb["pass_bytes"] / (t_sel * 1e-3) / 1e9
     rl_sel = {
@@ -511,7 +511,7 @@ def main():
         "timing": {"warmup_steps": args.warmup, "timed_steps": args.steps, "value_is": "mean of the timed steps",
                    "dense_warmup": args.dense_warmup, "dense_timed": args.dense_steps, "dense_fa_ms_is": "median",
                    "stages": "estimate_ms = the estimator's MFMA pass (estimate_gemm_kernel), select_ms = its normalisation "
-                             "fused with the block selection (estimate_select_kernel), sparse_attn_ms = block_sparse_fwd_kernel"},
+                             "fused with the block selection (estimate_select_kernel), sparse_attn_ms = block_sparse_fwd64_kernel"},
         "kernel_sources_sha256_16": kernel_source_hash(),
     }
     result.update({key: val for key, val in head.items() if not key.startswith("roofline_")})

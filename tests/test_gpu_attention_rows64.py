@@ -1,0 +1,97 @@
+"""GPU: the attention kernel of 64 query rows per wavefront (no causality and more than 512 units, 16384 cached tokens, or the
+later q-blocks of 49152 tokens and more) against plain fp32 attention."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+HEADS, KV_HEADS = 72, 8        # 9 q-blocks make 648 units
+
+
+def _inputs(q_len, k_len, seed, heads=HEADS, kv_heads=KV_HEADS):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    rnd = lambda h, n: torch.randn(1, h, n, 128, generator=g, device="cuda").bfloat16()
+    return rnd(heads, q_len), rnd(kv_heads, k_len), rnd(kv_heads, k_len)
+
+
+def _reference(q, k, v, blocks, causal):
+    """blocks: bool [heads, q-blocks, k-blocks]; rows that see nothing give zeros."""
+    q_len, k_len = q.shape[2], k.shape[2]
+    group = q.shape[1] // k.shape[1]
+    pos = torch.arange(q_len, device="cuda")[:, None] + (k_len - q_len)
+    out = torch.empty(q.shape[1], q_len, 128, device="cuda")
+    for h in range(q.shape[1]):
+        s = q[0, h].float() @ k[0, h // group].float().t() * 128 ** -0.5
+        see = blocks[h].repeat_interleave(128, 0)[:q_len].repeat_interleave(128, 1)[:, :k_len]
+        if causal:
+            see = see & (torch.arange(k_len, device="cuda")[None] <= pos)
+        s = s.masked_fill(~see, float("-inf"))
+        m = s.amax(-1, keepdim=True).clamp_min(-3e38)
+        p = torch.exp(s - m)
+        out[h] = p @ v[0, h // group].float() / p.sum(-1, keepdim=True).clamp_min(1e-30)
+    return out[None]
+
+
+def _check(out, want, v):
+    # probabilities are rounded to bf16 (2^-9 relative), and the result once more: see test_gpu_attention_plan.py
+    assert torch.isfinite(out.float()).all()
+    bound = 2.0 ** -8 * (v.float().abs().amax() + want.abs())
+    assert ((out.float() - want).abs() <= bound).all()
+    assert (out.float() - want).norm() <= 4e-3 * want.norm()
+
+
+@pytest.mark.parametrize("heads,kv_heads,q_len,k_len,causal", [(72, 8, 1100, 333, False), (72, 8, 1090, 33, False), (8, 2, 1, 16385, True), (8, 8, 300, 32896, True), (6, 2, 257, 33000, True),
+    (1, 1, 49100, 49100, True)])
+def test_dense(heads, kv_heads, q_len, k_len, causal):
+    from xattn.src.Xattention import block_sparse_attention
+
+    q, k, v = _inputs(q_len, k_len, 1, heads, kv_heads)
+    blocks = torch.ones(heads, (q_len + 127) // 128, (k_len + 127) // 128, dtype=torch.bool, device="cuda")
+    _check(block_sparse_attention(q, k, v, causal=causal), _reference(q, k, v, blocks, causal), v)
+
+
+# lists of no, one, two, three and many blocks; more than the 64 entries that are fetched at a time; token strides of a
+# projection's output; a cache, where lists are cut
+@pytest.mark.parametrize("heads,kv_heads,q_len,k_len,causal,keep", [
+    (72, 8, 1100, 1100, False, 0.4),
+    (72, 8, 1030, 9300, False, 0.5),
+    (8, 2, 515, 32900, True, 0.3),
+    (32, 8, 600, 32769, True, 0.02),
+])
+def test_lists(heads, kv_heads, q_len, k_len, causal, keep):
+    from helpers import lists_from_mask
+    from test_gpu_attention_plan import _swept_whole
+    from xattn.src.Xattention import block_sparse_attention
+
+    q, k, v = _inputs(q_len, k_len, 2, heads, kv_heads)
+    v = v.transpose(1, 2).contiguous().transpose(1, 2)
+    nq, nk = (q_len + 127) // 128, (k_len + 127) // 128
+    g = torch.Generator(device="cuda").manual_seed(3)
+    blocks = torch.rand(heads, nq, nk, generator=g, device="cuda") < keep
+    blocks[1, :, 3:] = False
+    blocks[:3, 2] = False
+    blocks[1, 2, 0] = blocks[2, 2, 0] = blocks[2, 2, 1] = True
+    if causal:
+        last = (torch.arange(nq, device="cuda") * 128 + 127).clamp_max(q_len - 1) + k_len - q_len
+        blocks &= torch.arange(nk, device="cuda")[None] * 128 <= last[:, None]
+    idx, cnt = lists_from_mask(blocks)
+    want = _reference(q, k, v, blocks, causal)
+    whole = _swept_whole(q, k, v, idx, cnt, causal)
+    _check(whole, want, v)
+    assert (whole[0, 0, 256:384] == 0).all()
+    _check(block_sparse_attention(q, k, v, idx, cnt, causal=causal), want, v)
+
+
+@pytest.mark.parametrize("heads,kv_heads,q_len,k_len,causal", [(72, 8, 1100, 1100, False), (8, 2, 260, 32900, True)])
+def test_scores_that_outgrow_the_reference_maximum(heads, kv_heads, q_len, k_len, causal):
+    """The sweep starts at the end of a list: scores grow by up to 2^260 on the way, by 32-key steps of any order."""
+    from xattn.src.Xattention import block_sparse_attention
+
+    q, k, v = _inputs(q_len, k_len, 4, heads, kv_heads)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    steps = (k_len + 31) // 32
+    level = torch.linspace(8, -8, steps, device="cuda") + 4 * torch.randn(steps, generator=g, device="cuda").clamp(-2, 2)
+    k = (0.2 * k + level.repeat_interleave(32)[:k_len, None]).bfloat16()
+    q = (0.2 * q + torch.sign(torch.randn(heads, q_len, 1, generator=g, device="cuda"))[None]).bfloat16()
+    blocks = torch.ones(heads, (q_len + 127) // 128, (k_len + 127) // 128, dtype=torch.bool, device="cuda")
+    _check(block_sparse_attention(q, k, v, causal=causal), _reference(q, k, v, blocks, causal), v)
