@@ -24,32 +24,54 @@ struct AttnParams {
   float scale_log2;         // softmax_scale * log2(e)
   DispatchShape shape;      // dispatch_shape(H, Hkv), computed on the host
   AttnPlan plan;            // kPlanned only
+  int32_t* queue;           // this launch's work queue (kQueueWords, zero), or null: one workgroup per id
+  int unit_ids;             // ids of units, grid_for()
 };
+
+// The kernel's parameters, read anew: between two units nothing that is computed from them is kept, which would take more
+// scalar registers than there are.
+__device__ __forceinline__ const AttnParams& reread_params() {
+  auto at = __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(at));
+  return *(const AttnParams*)at;
+}
 
 __device__ __forceinline__ int clamp_block(int kb, int nkb) { return kb < 0 ? 0 : (kb < nkb ? kb : nkb - 1); }
 
 typedef const __attribute__((address_space(4))) int32_t* const_i32_ptr;
 
-// What a workgroup works on.
+// What an id stands for.
 struct Unit {
   int head, qb, kvh;
   int piece;                 // which piece of its list, or -1: all of it
-  int skip;                  // workgroups ahead of the units'
+  int skip;                  // ids ahead of the units'
   int n_blocks, first;       // blocks of the list or piece; first: where it starts among the visible blocks (no list)
   const_i32_ptr list;        // the column list is read through the scalar cache (uniform, read-only)
   int cuts, part0;           // pieces of this list, the first one's place in the plan
+  int kb, kb_next;           // the sweep's first two blocks
 };
 
-// The (head, q-block) of this workgroup; false: nothing is left for it.
+// The same in scalar registers: from one turn of a loop to the next the compiler does not see that all lanes have the same.
+__device__ __forceinline__ Unit uniform(const Unit& u) {
+  auto one = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+  Unit v;
+  v.head = one(u.head), v.qb = one(u.qb), v.kvh = one(u.kvh), v.piece = one(u.piece), v.skip = one(u.skip);
+  v.n_blocks = one(u.n_blocks), v.first = one(u.first), v.cuts = one(u.cuts), v.part0 = one(u.part0), v.kb = one(u.kb), v.kb_next = one(u.kb_next);
+  const uintptr_t list = (uintptr_t)u.list;
+  v.list = (const_i32_ptr)((uintptr_t)(uint32_t)one((int)list) | (uintptr_t)(uint32_t)one((int)(list >> 32)) << 32);
+  return v;
+}
+
+// The (head, q-block) with this id; false: there is none.
 template <bool kPlanned>
-__device__ __forceinline__ bool find_unit(const AttnParams& p, Unit& u) {
+__device__ __forceinline__ bool find_unit(const AttnParams& p, int id, Unit& u) {
   u.piece = -1;
   u.skip = 0;
   if (kPlanned) {
     const int pieces = ((const_i32_ptr)(uintptr_t)p.plan.noted)[0], per_xcd = (pieces + 7) / 8;   // (the low half)
     u.skip = per_xcd * 8;
-    if ((int)blockIdx.x < u.skip) {
-      const int at = p.plan.shape.in_turn ? (int)blockIdx.x : (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+    if (id < u.skip) {
+      const int at = p.plan.shape.in_turn ? id : (id & 7) * per_xcd + (id >> 3);
       if (at >= pieces) return false;
       const_i32_ptr entry = (const_i32_ptr)(uintptr_t)p.plan.pieces + 2 * at;
       const int unit = entry[0];
@@ -60,9 +82,44 @@ __device__ __forceinline__ bool find_unit(const AttnParams& p, Unit& u) {
       return u.qb >= p.qb_begin && u.qb < p.qb_end;      // (q-blocks may be shared among two launches)
     }
   }
-  return map_workgroup((int)blockIdx.x - u.skip, p.shape, p.qb_begin, p.qb_end, &u.head, &u.qb, &u.kvh);
+  return map_workgroup(id - u.skip, p.shape, p.qb_begin, p.qb_end, &u.head, &u.qb, &u.kvh);
 }
 __device__ __forceinline__ int64_t unit_slot(const AttnParams& p, const Unit& u) { return (int64_t)u.head * p.idx_rows + (u.qb - p.idx_row0); }
+
+// The work queue.  Workgroups of a launch are dealt to the XCDs in turn, one XCD's are never another's, and a workgroup keeps
+// its place until its stores are acknowledged.  So XCDs with like numbers of workgroups ended far apart (2048 tokens on 63488
+// 506 to 615 us, where heads differ; video of 65536 14.5 to 16.0 ms, where only clocks do), and a tenth of the places stood
+// empty.  With a queue as many workgroups are launched as fit.
+// Workgroup b starts with id b and goes on with those of its queue, b % 32: ids that leave the same rest, which its XCD has
+// anyway.  (An answer takes 1 to 2 us, and a counter gives four in a us: with one per XCD the wait was 4 us of a short list's 15.)
+// queue[32 c]: what queue c has handed out beyond the ids that its workgroups start with.
+constexpr int kQueues = 32, kQueueWords = kQueues * 32;
+// Takes the next id of this workgroup's queue; one lane (resolved by next_id).
+__device__ __forceinline__ int ask_next(const AttnParams& p) {
+  return __hip_atomic_fetch_add(p.queue + (blockIdx.x % kQueues) * 32, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The id that lane 0 was given, or that another queue has left, or -1.  By a whole wavefront.  Short lists (`few` blocks the
+// last time) are left to their own workgroups where a queue has a single one left; so are others after four vain tries.
+template <bool kPlanned>
+__device__ __forceinline__ int next_id(const AttnParams& p, int ticket, int lane, bool few) {
+  const int pieces = kPlanned ? ((const_i32_ptr)(uintptr_t)p.plan.noted)[0] : 0;
+  const int ids = (pieces + 7) / 8 * 8 + p.unit_ids, first = (int)(gridDim.x / kQueues);
+  const int id = (first + __builtin_amdgcn_readfirstlane(ticket)) * kQueues + (int)(blockIdx.x % kQueues);
+  if (id < ids) return id;
+  for (int i = 0; i < 4; ++i) {
+    int left = 0;
+    if (lane < kQueues)
+      left = (ids - lane + kQueues - 1) / kQueues - first - __hip_atomic_load(p.queue + lane * 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t most = wave_max(left > (few ? 1 : 0) ? (uint32_t)left * kQueues + (uint32_t)lane : 0u);
+    if (most == 0) return -1;
+    const int c = (int)(most % kQueues);
+    int taken = 0;
+    if (lane == 0) taken = __hip_atomic_fetch_add(p.queue + c * 32, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int other = (first + __builtin_amdgcn_readfirstlane(taken)) * kQueues + c;
+    if (other < ids) return other;
+  }
+  return -1;
+}
 
 // Its list; false: others have it.
 template <bool kHasList, bool kPlanned>
@@ -92,6 +149,25 @@ __device__ __forceinline__ bool find_list(const AttnParams& p, Unit& u) {
     }
   }
   return true;
+}
+
+// The next id that has work, from the ticket of thread 0, the same for all wavefronts; -1: there is none.
+template <bool kHasList, bool kPlanned>
+__device__ __forceinline__ int hand_out(const AttnParams& p, int ticket, int wave, int lane, bool few, char* scratch) {
+  if (wave == 0) {
+    int next;
+    for (;;) {
+      next = next_id<kPlanned>(p, ticket, lane, few);
+      Unit u;
+      if (next < 0 || (find_unit<kPlanned>(p, next, u) && find_list<kHasList, kPlanned>(p, u))) break;
+      if (lane == 0) ticket = ask_next(p);
+    }
+    if (lane == 0) *reinterpret_cast<int*>(scratch) = next;
+  }
+  __syncthreads();
+  const int id = __builtin_amdgcn_readfirstlane(*reinterpret_cast<const int*>(scratch));
+  __syncthreads();
+  return id;
 }
 
 // A lane's place in the fragments of a tile in LDS.
@@ -134,8 +210,9 @@ __device__ __forceinline__ void mask_step(f32x16& s, int key0, int hh, int q_pos
 // Normalises 32 output rows (group `wave` of the q-block's four) and stores them through LDS.  Lane (r, hh) holds half of row r in
 // 8-byte pieces; written straight to memory those are 512 sixteen-byte requests per wavefront, and a
 // workgroup's registers and LDS stay allocated until its last store is acknowledged - on lists of a few blocks
-// that wait was a quarter of a workgroup's life.  Staged through 8 KiB of LDS
-// (free once the sweep is over), 16 lanes write one 256-byte row: 64 full-line requests.
+// that wait was a quarter of a workgroup's life.  Staged through 8 KiB of LDS,
+// 16 lanes write one 256-byte row: 64 full-line requests.
+constexpr int kOutStage = 8192;      // bytes per wavefront
 __device__ __forceinline__ void store_out(const AttnParams& p, int head, int qb, int wave, int lane, int r, int hh,
                                           const f32x16 (&oacc)[4], float l_run, char* stage) {
   const float l_tot = half_sum(l_run);
@@ -195,32 +272,52 @@ __device__ __forceinline__ void store_partial(float* part, int wave, int lane, i
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, l_tot), res, at + 512, 0, kDeviceScope);
   }
 }
-// The pieces' results combined into the registers of a finished sweep, in the order of the list.
+// The pieces' results combined into the registers of a finished sweep, in the order of the list.  One workgroup reads up to
+// 16 x 66 KiB here while the others may be done: a piece's 16 KiB per wavefront are requested while the one before it is added
+// up (each load behind the last one's sum: 160 us for 16 pieces).  Loads past the last piece arrive as zeros.
 __device__ __forceinline__ void load_partials(float* part, int pieces, int wave, int lane, int r, int hh, f32x16 (&oacc)[4], float& l_run) {
-  const int at = (128 * 128 + wave * 32 + r) * 4;
+  const __amdgpu_buffer_rsrc_t res = __builtin_amdgcn_make_buffer_rsrc((void*)part, 0, pieces * kPartFloats * 4, 0x00020000);
+  const int at = (128 * 128 + wave * 32 + r) * 4, from = (wave * 16 * 64 + lane) * 16;
   auto ml = [&](int s, int which) __attribute__((always_inline)) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(part_resource(part + (int64_t)s * kPartFloats), at + which * 512, 0, kDeviceScope));
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(res, at + which * 512, s * kPartFloats * 4, kDeviceScope));
   };
-  float m = -INFINITY, l = 0.f;
-#pragma unroll 4
-  for (int s = 0; s < pieces; ++s) m = fmaxf(m, ml(s, 0));
+  struct Piece {
+    float m, l;
+    f32x4 o[16];
+  } a, b;
+  auto request = [&](Piece& x, int s) __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    x.m = ml(s, 0);
+    x.l = ml(s, 1);
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      x.o[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(res, from + i * 1024, s * kPartFloats * 4, kDeviceScope));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  float tops[kMostPieces], m = -INFINITY, l = 0.f;
+#pragma unroll
+  for (int s = 0; s < kMostPieces; ++s) tops[s] = ml(s, 0);
+#pragma unroll
+  for (int s = 0; s < kMostPieces; ++s) m = fmaxf(m, s < pieces ? tops[s] : -INFINITY);
   const float safe = m == -INFINITY ? 0.f : m;
+  request(a, 0);
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int v = 0; v < 16; ++v) oacc[i][v] = 0.f;
-  for (int s = 0; s < pieces; ++s) {
-    const __amdgpu_buffer_rsrc_t res = part_resource(part + (int64_t)s * kPartFloats);
-    const float w = fast_exp2(ml(s, 0) - safe);      // 0 where the item saw no key of this row
-    l += w * ml(s, 1);
+  auto add = [&](const Piece& x, bool there) __attribute__((always_inline)) {
+    const float w = there ? fast_exp2(x.m - safe) : 0.f;      // 0 where the piece saw no key of this row
+    l += w * x.l;
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+    for (int i = 0; i < 16; ++i)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x4 o = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(res, (wave * 16 * 64 + lane) * 16 + (dt * 4 + g) * 1024, 0, kDeviceScope));
-#pragma unroll
-        for (int u = 0; u < 4; ++u) oacc[dt][g * 4 + u] += w * o[u];
-      }
+      for (int u = 0; u < 4; ++u) oacc[i >> 2][(i & 3) * 4 + u] += w * x.o[i][u];
+  };
+  for (int s = 0; s < pieces; s += 2) {
+    request(b, s + 1);
+    add(a, true);
+    request(a, s + 2);
+    add(b, s + 1 < pieces);
   }
   l_run = hh == 0 ? l : 0.f;
 }

@@ -56,27 +56,44 @@ using namespace xattn;
 // The first q-blocks of a long prompt see few blocks and keep short lists.  They are a launch of their own behind the others',
 // so they are few: with the line at 128 blocks instead of 16 the units next to it, of 300 us, ended the first launch alone
 // (131072 tokens with long lists 13.56 ms for 13.28).
-static int first_rows64(const AttnParams& p) {
-  if (!p.causal) return (int64_t)p.H * p.nqb > 512 || p.nkb >= 192 ? 0 : p.nqb;
-  if (p.nkb < 384 && p.kv_off < 128 * kBlk) return p.nqb;
-  const int64_t query = 15 * kBlk - (int64_t)p.kv_off;           // the first that sees 16 blocks
+static int first_rows64(int H, int nqb, int nkb, int kv_off, int causal) {
+  if (!causal) return (int64_t)H * nqb > 512 || nkb >= 192 ? 0 : nqb;
+  if (nkb < 384 && kv_off < 128 * kBlk) return nqb;
+  const int64_t query = 15 * kBlk - (int64_t)kv_off;             // the first that sees 16 blocks
   const int64_t qb = query <= 0 ? 0 : query / kBlk;
-  return qb < p.nqb ? (int)qb : p.nqb;
+  return qb < nqb ? (int)qb : nqb;
+}
+
+// Whether the 64-row kernel has a work queue: where units, or the pieces of a chunk's, go several times through the places
+// (us without / with: 2048 on 63488 716 / 648, 1000 on 30000 221 / 214; but 500 on 60000, 128 units, 181 / 195; a field of
+// 4000, 768 like units, 229 / 235: dealt by the launch, the second round's find CUs of their own).
+bool xattn::attention_queued(int num_heads, int q_len, int k_len, int causal) {
+  const int nqb = (int)(((int64_t)q_len + kBlk - 1) / kBlk), nkb = (int)(((int64_t)k_len + kBlk - 1) / kBlk);
+  const int64_t units = (int64_t)num_heads * nqb;
+  return first_rows64(num_heads, nqb, nkb, k_len - q_len, causal) < nqb && (units > 1024 || (units >= 256 && nkb >= 2 * nqb));
 }
 
 template <bool kHasList, bool kPlanned>
 static int launch_fwd(AttnParams p, int64_t extra, hipStream_t s) {
-  const int begin = p.qb_begin, end = p.qb_end, split = first_rows64(p);
-  auto grid = [&]() { return dim3((unsigned)(grid_for(p.H, p.Hkv, p.qb_end - p.qb_begin) + extra)); };
+  const int begin = p.qb_begin, end = p.qb_end, split = first_rows64(p.H, p.nqb, p.nkb, p.kv_off, p.causal);
+  const int cus = resident_workgroups();
+  if (cus <= 0) return XATTN_ERR_LAUNCH;
+  const int places = 2 * cus / kQueues * kQueues;
+  auto grid = [&](bool queued) {
+    p.unit_ids = (int)grid_for(p.H, p.Hkv, p.qb_end - p.qb_begin);
+    const int64_t ids = p.unit_ids + extra;
+    if (!queued || places == 0 || ids <= places) p.queue = nullptr;
+    return dim3((unsigned)(p.queue ? places : ids));
+  };
   p.qb_begin = begin > split ? begin : split;
   if (p.qb_begin < end) {
-    hipLaunchKernelGGL((block_sparse_fwd64_kernel<kHasList, kPlanned>), grid(), dim3(128), 0, s, p);
+    hipLaunchKernelGGL((block_sparse_fwd64_kernel<kHasList, kPlanned>), grid(true), dim3(128), 0, s, p);
     if (hipGetLastError() != hipSuccess) return XATTN_ERR_LAUNCH;
   }
   p.qb_begin = begin;
   p.qb_end = end < split ? end : split;
   if (begin < p.qb_end) {
-    hipLaunchKernelGGL((block_sparse_fwd_kernel<kHasList, kPlanned>), grid(), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((block_sparse_fwd_kernel<kHasList, kPlanned>), grid(false), dim3(256), 0, s, p);
     if (hipGetLastError() != hipSuccess) return XATTN_ERR_LAUNCH;
   }
   return XATTN_OK;
@@ -92,7 +109,7 @@ int xattn::block_sparse_impl(const void* q, const void* k, const void* v, void* 
                                       int64_t k_stride_n, int64_t v_stride_h, int64_t v_stride_n,
                                       int64_t o_stride_h, int64_t o_stride_n, int q_block_begin, int q_block_end,
                                       int causal, float softmax_scale, void* stream,
-                                      const AttnPlan* plan, bool note) {
+                                      const AttnPlan* plan, bool note, int32_t* queue) {
   if (!q || !k || !v || !out) return XATTN_ERR_NULL;
   if (head_dim != kHeadDim) return XATTN_ERR_HEAD_DIM;
   if (num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads) return XATTN_ERR_HEADS;
@@ -135,6 +152,7 @@ int xattn::block_sparse_impl(const void* q, const void* k, const void* v, void* 
   if (grid > 0x7fffffff) return XATTN_ERR_SHAPE;
   hipStream_t s = static_cast<hipStream_t>(stream);
   p.plan = AttnPlan{};
+  p.queue = queue;
   if (plan) {
     p.plan = *plan;
     const int64_t most = ((int64_t)plan_pieces(plan->shape, q_block_end - q_block_begin) + 7) / 8 * 8;
@@ -155,7 +173,7 @@ extern "C" int xattn_block_sparse_fwd(const void* q, const void* k, const void* 
                                       int causal, float softmax_scale, void* stream) {
   return block_sparse_impl(q, k, v, out, col_idx, col_cnt, idx_pitch, idx_rows, idx_row0, num_heads, num_kv_heads, q_len, k_len,
                            head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n, o_stride_h,
-                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, nullptr, false);
+                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, nullptr, false, nullptr);
 }
 
 namespace {
@@ -195,5 +213,5 @@ extern "C" int xattn_block_sparse_fwd_ws(const void* q, const void* k, const voi
   }
   return block_sparse_impl(q, k, v, out, col_idx, col_cnt, idx_pitch, idx_rows, idx_row0, num_heads, num_kv_heads, q_len, k_len,
                            head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n, o_stride_h,
-                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, need ? &plan : nullptr, true);
+                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, need ? &plan : nullptr, true, nullptr);
 }

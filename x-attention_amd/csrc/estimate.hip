@@ -195,7 +195,7 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
   };
   if (!decode(id, &head, &m0, &n0)) return;
   if (blockIdx.x == 0)                       // (it always has a tile)
-    for (int i = tid; i < p.noted_words; i += kWaves * 64) p.noted[i] = 0;
+    for (int i = tid; i < p.clear_words; i += kWaves * 64) p.clear[i] = 0;
 
   const int64_t q_snb = p.q_sn * 2, k_snb = p.k_sn * 2;
   const int64_t span = (int64_t)kTile * p.S;
@@ -860,21 +860,6 @@ hipError_t launch_select(const EstParams& p, const SelParams& sp, int qb_per_wg,
   return hipSuccess;
 }
 
-// CUs of the current device, rounded down to a multiple of 8 (tile ids are dealt to the 8 XCDs in turn)
-int resident_workgroups() {
-  static std::mutex mu;
-  static int per_device[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  std::lock_guard<std::mutex> lock(mu);
-  if (per_device[dev] == 0) {
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-    per_device[dev] = cus >= 8 ? cus / 8 * 8 : 8;
-  }
-  return per_device[dev];
-}
-
 struct Geometry {
   int q_pad, k_pad, n_rq, n_rk, nqb, nkb, nT, rcs, q_chunks;   // n_rq: reshaped query rows before subsampling
 };
@@ -919,6 +904,21 @@ extern "C" size_t xattn_estimate_workspace_bytes(int num_heads, int q_len, int k
 }
 
 namespace xattn {
+// CUs of the current device, rounded down to a multiple of 8 (tile ids are dealt to the 8 XCDs in turn)
+int resident_workgroups() {
+  static std::mutex mu;
+  static int per_device[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  std::lock_guard<std::mutex> lock(mu);
+  if (per_device[dev] == 0) {
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    per_device[dev] = cus >= 8 ? cus / 8 * 8 : 8;
+  }
+  return per_device[dev];
+}
+
 int estimate_impl(const void* q, const void* k, float* block_sums, void* workspace, size_t workspace_size,
                   float* scores_out, int num_heads, int num_kv_heads, int q_len, int k_len, int head_dim,
                   int64_t q_stride_h, int64_t q_stride_n, int64_t k_stride_h, int64_t k_stride_n, int stride,
@@ -997,8 +997,8 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
   p.n_pairs = num_slab_pairs;
   p.scores = scores_out;
   p.sums = block_sums;
-  p.noted = sel && sel->plan ? sel->plan->noted : nullptr;
-  p.noted_words = p.noted ? (int)((plan_noted_bytes(nqb_real) + plan_round((size_t)num_heads * nqb_real * 4)) / 8) : 0;
+  p.clear = sel ? sel->clear : nullptr;
+  p.clear_words = p.clear ? sel->clear_words : 0;
   // block_sums may hold a window of q-block rows only; the chunks of this call must lie inside it
   {
     const int bpc = chunk_size / block_size;
@@ -1165,7 +1165,7 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
     return launch_select<RBS>(p, sp, qb_per_wg, sel_threads, grid_sel, lds_sel, s);
   };
   // one pass instead of two where every row asked for is estimated, in 32-row tiles, and sees a single key tile
-  bool one_pass = variant == 0 && sel && sel->stages == 3 && !p.no_softmax && !p.sums && !sel->plan && p.nT_real == g.nT &&
+  bool one_pass = variant == 0 && sel && sel->stages == 3 && !p.no_softmax && !p.sums && !sel->plan && !p.clear && p.nT_real == g.nT &&
                   p.live_end == sp.row_end * p.rbs && row_lo(p, p.live_end - 1) == 0 &&
                   (row_hi(p, p.live_end - 1) < kSub || g.n_rk <= kSub) && 4 * sel_wave_bytes <= 64 * 1024;
   const bool run_gemm = !sel || (sel->stages & 1), run_rest = !sel || (sel->stages & 2);

@@ -39,14 +39,14 @@ struct EstParams {
   int tiles_per_head;       // tiles with a visible pair, per head
   int64_t total_tiles;      // tiles_per_head * H
   // estimate_small_kernel: a tile's rows are tile_rows rows of each of pack heads of one KV group
-  unsigned long long* noted;   // noted_words words set to zero for the selection pass that follows (AttnPlan::noted and ::cut)
+  unsigned long long* clear;   // clear_words words set to zero for the passes that follow
   int pack, tile_rows, tile_shift;   // powers of two, tile_rows = 1 << tile_shift
   // estimate_gemm_kernel with packed rows: quarters of 64 rows per head, 256-row tiles per KV group, first key tile, key tiles
   int quarters, group_tiles, first_key_tile, key_tiles;
   // estimate_gemm_kernel with half tiles: tiles taken whole, tiles behind them taken as two halves of 128 rows, and per head
   // the tiles (of keys from first_key_tile on) of a last row tile that has one half
   int whole_tiles, split_tiles, last_row_tiles;
-  int noted_words;
+  int clear_words;
 };
 
 // first / last visible reshaped key of reshaped query row m

@@ -37,7 +37,7 @@ __global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p, Sel
   const uint32_t per_group = (uint32_t)p.tiles_per_head * sets, total = per_group * (uint32_t)p.Hkv;
   const uint32_t per_xcd = (total + 7) / 8;
   const uint32_t lin = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  for (int i = (int)blockIdx.x * 256 + tid; i < p.noted_words; i += (int)gridDim.x * 256) p.noted[i] = 0;
+  for (int i = (int)blockIdx.x * 256 + tid; i < p.clear_words; i += (int)gridDim.x * 256) p.clear[i] = 0;
   if (lin >= total) return;
   const uint32_t g = lin / per_group, rem = lin - g * per_group;
   const uint32_t set = rem % sets;
