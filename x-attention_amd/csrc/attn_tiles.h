@@ -80,13 +80,20 @@ __device__ __forceinline__ void tile_offsets(int64_t sn, int lane, int wave, int
 // dispatch group of its own).  Units are dealt to XCDs in turn; the dispatch
 // group of a unit rotates with the q-block run, so every XCD sees every head
 // equally often (heads differ by orders of magnitude in list length).  Runs go
-// out last (longest, when causal) first.
+// out last (longest, when causal) first, so of eight runs an XCD that sees a
+// head in the first has more of it than one that sees it in the eighth: of the
+// next eight it sees it that much later, the rotation runs backwards.  (Where
+// two of 8 groups keep long lists of 256 q-blocks, an XCD had 20 % more than
+// its share: text of 32768 tokens 1986 us, 1738 with the turn.)  Groups fewer
+// than XCDs rotate every second or fourth run, or half the XCDs would never see
+// a group.
 struct DispatchShape {
   int group;       // query heads per KV head
   int sets;        // head sets per KV head (1 unless group > kUnit)
   int set_heads;   // query heads per set (<= kUnit)
   int n_groups;    // dispatch groups: Hkv * sets
   int unit_rows;   // q-blocks per unit
+  int turn_shift;  // groups rotate once per 1 << turn_shift runs
 };
 __host__ __device__ inline DispatchShape dispatch_shape(int H, int Hkv) {
   DispatchShape d;
@@ -95,6 +102,7 @@ __host__ __device__ inline DispatchShape dispatch_shape(int H, int Hkv) {
   d.set_heads = (d.group + d.sets - 1) / d.sets;
   d.n_groups = Hkv * d.sets;
   d.unit_rows = kUnit / d.set_heads;
+  d.turn_shift = d.n_groups == 4 ? 1 : d.n_groups == 2 ? 2 : 0;
   return d;
 }
 
@@ -108,7 +116,8 @@ __host__ __device__ inline bool map_workgroup(int id, const DispatchShape& d, in
   const uint32_t unit = (s / kUnit) * 8u + x, w = s % kUnit;
   const uint32_t ng = (uint32_t)d.n_groups, sh = (uint32_t)d.set_heads;
   const uint32_t run = unit / ng;
-  const uint32_t dg = (unit + run) % ng;      // the unit's group, rotated by its run
+  const uint32_t turn = (run & 8u ? ~run : run) & 7u;
+  const uint32_t dg = (unit - run * ng + (turn >> d.turn_shift)) % ng;      // the unit's group, rotated by its run
   const uint32_t w_row = w / sh, w_head = w - w_row * sh;
   const uint32_t from_end = run * (uint32_t)d.unit_rows + w_row;
   uint32_t set = 0, kvh = dg;
