@@ -362,7 +362,6 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
   const int T = nbase / kSub;
   const Quarter own = kPacked ? tile_quarter(p, head, m0, wm) : Quarter{head, m0 + wm * 32 * kMT};
   if (nbase < p.n_rk && (!kPacked || own.head >= 0)) {
-  float* Pst = p.P + (int64_t)own.head * p.nkb * p.rows;
   float* Mst = p.Mt + ((int64_t)own.head * p.nT + T) * p.rows;
   float* Lst = p.Lt + ((int64_t)own.head * p.nT + T) * p.rows;
   // every key of this wavefront tile visible to every one of its query rows?
@@ -411,12 +410,11 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
     const int mrel = m - p.row_begin;
     constexpr int G = RBS / 8;   // 8-key groups (one per accumulator quad pair) per key block
     // what the stores below share: the first key block of this wavefront tile and how many of its key blocks
-    // exist (uniform), the row of P they start from (uniform) and each half-wave's predicate
+    // exist (uniform), each lane's place in P and the key blocks that it may store
     const int kb_first = (int)((uint32_t)nbase / (uint32_t)RBS);
     const int kb_left = p.nkb - kb_first;
-    float* const prow = Pst + (int64_t)kb_first * p.rows + mrel;
-    const int64_t rows64 = p.rows;
-    const bool st0 = row_ok && hh == 0, st1 = row_ok && hh == 1;
+    float* const prow = p.P + partial_at(p, own.head, row_ok ? mrel : 0) + (int64_t)(kb_first + (G < 4 ? hh : 0)) * kStrip;
+    const int st = !row_ok ? 0 : G < 4 ? kb_left - hh : hh == 0 ? kb_left : 0;
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
       float s[4];       // this lane's share of the sums over keys nbase + nt*32 + 8g .. +7 (the other half-wave has the rest)
@@ -438,19 +436,17 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
           const float both = half_sum_pair(s[2 * q2], s[2 * q2 + 1]);
           tot += both;
           const int k = nt * 4 + 2 * q2;
-          if (k < kb_left && st0) prow[k * rows64] = both;
-          if (k + 1 < kb_left && st1) prow[(k + 1) * rows64] = both;
+          if (k < st) prow[k * kStrip] = both;
         }
       } else if (G == 2) {
         const float both = half_sum_pair(s[0] + s[1], s[2] + s[3]);
         tot += both;
         const int k = nt * 2;
-        if (k < kb_left && st0) prow[k * rows64] = both;
-        if (k + 1 < kb_left && st1) prow[(k + 1) * rows64] = both;
+        if (k < st) prow[k * kStrip] = both;
       } else {
         const float all = half_sum(s[0] + s[1] + s[2] + s[3]);
         tot += hh == 0 ? all : 0.f;
-        if (nt < kb_left && st0) prow[nt * rows64] = all;
+        if (nt < st) prow[nt * kStrip] = all;
       }
     }
     tot = half_sum(tot);
@@ -490,12 +486,12 @@ __device__ __forceinline__ void tile_stat(const EstParams& p, const float* Mst, 
 }
 // tile maxima and partial sums of key block kb for four consecutive rows
 template <int RBS>
-__device__ __forceinline__ void load_partial(const EstParams& p, const float* Mst, const float* Pst, int kb, int mrel4, f32x4& mt,
+__device__ __forceinline__ void load_partial(const EstParams& p, const float* Mst, const float* prow, int kb, int mrel4, f32x4& mt,
                                              f32x4& pv) {
   const int T = (kb * RBS) / kSub;
   if (T < p.nT_real) {
     mt = *reinterpret_cast<const f32x4*>(Mst + (int64_t)T * p.rows + mrel4);
-    pv = *reinterpret_cast<const f32x4*>(Pst + (int64_t)kb * p.rows + mrel4);
+    pv = *reinterpret_cast<const f32x4*>(prow + (int64_t)kb * kStrip);
   } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -520,7 +516,6 @@ __global__ __launch_bounds__(256) void estimate_normalize_kernel(EstParams p) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int head = blockIdx.y;
   const int strip0 = p.row_begin + blockIdx.x * 64;
-  const float* Pst = p.P + (int64_t)head * p.nkb * p.rows;
   const float* Mst = p.Mt + (int64_t)head * p.nT * p.rows;
   const float* Lst = p.Lt + (int64_t)head * p.nT * p.rows;
 
@@ -556,6 +551,7 @@ __global__ __launch_bounds__(256) void estimate_normalize_kernel(EstParams p) {
   const bool rows_live = m4 < p.live_end;
   const int mc4 = rows_ok ? m4 : p.row_begin;
   const int mrel4 = mc4 - p.row_begin;
+  const float* const prow = p.P + partial_at(p, head, mrel4);
   const f32x4 rM = *reinterpret_cast<const f32x4*>(rowM + l16 * 4);
   const f32x4 rI = *reinterpret_cast<const f32x4*>(rowInv + l16 * 4);
   // the RBS rows of a query block share their first / last visible key block
@@ -577,7 +573,7 @@ __global__ __launch_bounds__(256) void estimate_normalize_kernel(EstParams p) {
     for (int u = 0; u < kUnroll; ++u) {
       const int kb = kb0 + 16 * u + kgrp;
       live[u] = rows_live && kb < p.nkb && kb >= kb_lo && kb <= kb_hi;
-      if (live[u]) load_partial<RBS>(p, Mst, Pst, kb, mrel4, mt[u], pv[u]);
+      if (live[u]) load_partial<RBS>(p, Mst, prow, kb, mrel4, mt[u], pv[u]);
     }
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
@@ -616,7 +612,6 @@ __global__ __launch_bounds__(256) void estimate_select_kernel(EstParams p, SelPa
   const int head = blockIdx.x / groups;
   const int grp = blockIdx.x % groups;
   const int strip0 = p.row_begin + grp * rows_wg;        // first reshaped row of the workgroup
-  const float* Pst = p.P + (int64_t)head * p.nkb * p.rows;
   const float* Mst = p.Mt + (int64_t)head * p.nT * p.rows;
   const float* Lst = p.Lt + (int64_t)head * p.nT * p.rows;
 
@@ -668,6 +663,7 @@ __global__ __launch_bounds__(256) void estimate_select_kernel(EstParams p, SelPa
     const bool rows_live = m4 < p.live_end;
     const int mc4 = rows_ok ? m4 : p.row_begin;
     const int mrel4 = mc4 - p.row_begin;
+    const float* const prow = p.P + partial_at(p, head, mrel4);
     const f32x4 rM = *reinterpret_cast<const f32x4*>(rowM + l * 4);
     const f32x4 rI = *reinterpret_cast<const f32x4*>(rowInv + l * 4);
     const int kb_lo = row_lo(p, mc4) / RBS;
@@ -684,7 +680,7 @@ __global__ __launch_bounds__(256) void estimate_select_kernel(EstParams p, SelPa
       for (int u = 0; u < kUnroll; ++u) {
         const int kb = kb0 + kb_step * u;
         live[u] = rows_live && kb < p.nkb && kb >= kb_lo && kb <= kb_hi;
-        if (live[u]) load_partial<RBS>(p, Mst, Pst, kb, mrel4, mt[u], pv[u]);
+        if (live[u]) load_partial<RBS>(p, Mst, prow, kb, mrel4, mt[u], pv[u]);
       }
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
@@ -726,7 +722,6 @@ __global__ __launch_bounds__(256) void estimate_normalize_rows_kernel(EstParams 
   const int tid = threadIdx.x, row = tid & 31, part = tid >> 5;
   const int head = blockIdx.y;
   const int m0 = p.row_begin + blockIdx.x * p.rbs_q;     // first query row of the block
-  const float* Pst = p.P + (int64_t)head * p.nkb * p.rows;
   const float* Mst = p.Mt + (int64_t)head * p.nT * p.rows;
   const float* Lst = p.Lt + (int64_t)head * p.nT * p.rows;
   const bool row_ok = row < p.rbs_q && m0 + row < p.live_end;
@@ -770,7 +765,7 @@ __global__ __launch_bounds__(256) void estimate_normalize_rows_kernel(EstParams 
       if (kb < row_lo(p, mr) / p.rbs || kb > h2 / p.rbs) continue;
       const int rel = mr - p.row_begin;
       const bool real = T < p.nT_real;
-      const float pv = real ? Pst[(int64_t)kb * p.rows + rel] : (float)p.rbs;
+      const float pv = real ? p.P[partial_at(p, head, rel) + (int64_t)kb * kStrip] : (float)p.rbs;
       const float mt = real ? Mst[(int64_t)T * p.rows + rel] : 0.f;
       acc += pv * fast_exp2(mt - rowM[r]) * rowInv[r];
     }
@@ -883,7 +878,7 @@ bool geometry(int q_len, int k_len, int stride, int block_size, int chunk_size, 
 }
 
 size_t workspace_bytes(int H, const Geometry& g, int rows) {
-  return (size_t)H * rows * ((size_t)g.nkb + 2 * (size_t)g.nT) * sizeof(float);
+  return (size_t)H * ((size_t)strips_of(rows) * kStrip * g.nkb + 2 * (size_t)rows * g.nT) * sizeof(float);
 }
 }  // namespace
 
@@ -1012,7 +1007,7 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
   if (workspace_size < workspace_bytes(num_heads, g, p.rows)) return XATTN_ERR_WORKSPACE;
   float* ws = static_cast<float*>(workspace);
   p.P = ws;
-  p.Mt = ws + (size_t)num_heads * g.nkb * p.rows;
+  p.Mt = ws + (size_t)num_heads * g.nkb * strips_of(p.rows) * kStrip;
   p.Lt = p.Mt + (size_t)num_heads * g.nT * p.rows;
 
   hipStream_t s = static_cast<hipStream_t>(stream);

@@ -49,6 +49,16 @@ struct EstParams {
   int clear_words;
 };
 
+// Place of row `rel` (counted from row_begin) in P, for key block 0; the next key block's is kStrip on.  Strips of 32 rows, key
+// block after key block: what one workgroup of the selection reads lies together, and a wavefront of the estimate writes the
+// key blocks of a tile in a row with constant offsets (key block after key block of all rows, 128 bytes every 4 * rows:
+// @@).
+constexpr int kStrip = 32;
+__host__ __device__ inline int strips_of(int rows) { return (rows + kStrip - 1) / kStrip; }
+__device__ __forceinline__ int64_t partial_at(const EstParams& p, int head, int rel) {
+  return (int64_t)(head * strips_of(p.rows) + rel / kStrip) * p.nkb * kStrip + rel % kStrip;
+}
+
 // first / last visible reshaped key of reshaped query row m
 // (with kdb > 1 the row's causal limit is that of the LAST reshaped row of its
 // group, xattn/src/Xattention.py:217-222, while its tokens are those of the first, :88-93)

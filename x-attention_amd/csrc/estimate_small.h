@@ -190,14 +190,13 @@ __global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p, Sel
     const float safe = mx[a] == -INFINITY ? 0.f : mx[a];
     const int head = h0 + (rr >> p.tile_shift), m = m0 + (rr & (p.tile_rows - 1));
     const bool row_ok = m < p.live_end && head < h_end;
-    float* const prow = p.P + ((int64_t)(row_ok ? head : h0) * p.nkb + kb_first) * p.rows + (m - p.row_begin);
-    const int64_t rows64 = p.rows;
+    float* const prow = p.P + partial_at(p, row_ok ? head : h0, row_ok ? m - p.row_begin : 0) + (int64_t)kb_first * kStrip;
     const bool st0 = row_ok && hh == 0, st1 = row_ok && hh == 1;
     auto put = [&](int k, bool on, float x) __attribute__((always_inline)) {
       if (kSelect) {
         if (on) psum[k * 32 + r] = x;
       } else if (k < kb_left && on) {
-        prow[k * rows64] = x;
+        prow[k * kStrip] = x;
       }
     };
     float s[4];
