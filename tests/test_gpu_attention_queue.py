@@ -29,3 +29,41 @@ def test_queue_gives_the_same_as_a_workgroup_per_unit(q_len, cache, heads, kv_he
     want = block_sparse_attention(q, k, v, idx, cnt, causal=causal)
     for _ in range(3):                                            # whoever takes what
         assert torch.equal(Xattention_prefill(q, k, v, 8, threshold=taus, chunk_size=chunk, causal=causal), want)
+
+
+# prompts of 3584 units and more that see fewer than 384 blocks: of some q-blocks all lists are long (64 rows per wavefront), of
+# others a few heads' or none (32 rows); more heads than lanes
+@pytest.mark.parametrize("q_len,heads,kv_heads,long_heads", [
+    (14300, 32, 8, list(range(0, 32))),
+    (14300, 32, 8, list(range(0, 32, 3))),
+    (6700, 70, 7, list(range(0, 66))),
+    (14336, 32, 32, []),
+])
+def test_lists_choose_the_kernel_the_same_way_by_every_path(q_len, heads, kv_heads, long_heads):
+    from xattn.src.Xattention import Xattention_prefill, block_sparse_attention, estimate_and_select
+
+    g = torch.Generator(device="cuda").manual_seed(heads)
+    rnd = lambda h, n: torch.randn(1, h, n, 128, generator=g, device="cuda").bfloat16()
+    q, k, v = rnd(heads, q_len), rnd(kv_heads, q_len), rnd(kv_heads, q_len)
+    taus, nq = torch.full((heads,), 0.02), (q_len + 127) // 128
+    taus[torch.tensor(long_heads, dtype=torch.long)] = 0.9
+    r = estimate_and_select(q, k, 16, taus, 128, want_mask=False, want_sums=False)
+    idx, cnt = r["col_idx"][:, :nq].contiguous(), r["col_cnt"][:, :nq].contiguous()
+    got = Xattention_prefill(q, k, v, 16, threshold=taus, chunk_size=128)
+    assert torch.equal(block_sparse_attention(q, k, v, idx, cnt), got)
+    parts = torch.empty(1, q_len, heads, 128, dtype=torch.bfloat16, device="cuda")
+    for a, b in ((0, nq // 3), (nq // 3, nq)):
+        block_sparse_attention(q, k, v, idx, cnt, out=parts, q_blocks=(a, b))
+    assert torch.equal(parts.transpose(1, 2), got)
+    # fp32 attention over the same lists, a q-block at a time; the bound of test_gpu_attention_plan.py
+    for h in (0, heads - 1):
+        for b in (0, 9, nq // 2, nq - 1):
+            cols = idx[h, b, :cnt[h, b]].long()
+            keys = (cols[:, None] * 128 + torch.arange(128, device="cuda")).flatten()
+            rows = torch.arange(b * 128, min(q_len, b * 128 + 128), device="cuda")
+            keys = keys[keys < q_len]
+            s = q[0, h, rows].float() @ k[0, h * kv_heads // heads, keys].float().t() * 128 ** -0.5
+            p = s.masked_fill(keys[None] > rows[:, None], float("-inf")).softmax(-1)
+            vals = v[0, h * kv_heads // heads, keys].float()
+            want = p @ vals
+            assert ((got[0, h, rows].float() - want).abs() <= 2.0 ** -8 * (vals.abs().amax() + want.abs())).all()

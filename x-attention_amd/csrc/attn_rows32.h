@@ -149,7 +149,7 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
   const int r = lane & 31, hh = lane >> 5;
 
   Unit u;
-  if (!find_unit<kPlanned>(p, (int)blockIdx.x, u) || !find_list<kHasList, kPlanned>(p, u)) return;
+  if (!find_unit<kHasList, kPlanned, false>(p, (int)blockIdx.x, u) || !find_list<kHasList, kPlanned>(p, u)) return;
   const int n_blocks = u.n_blocks;
   const int first = !kHasList ? u.first : n_blocks > 0 ? u.list[0] : 0;
   const __bf16* qbase = p.q + (int64_t)u.head * p.q_sh;

@@ -303,7 +303,7 @@ __global__ __launch_bounds__(128, 1) void block_sparse_fwd64_kernel(AttnParams) 
   // The sweep goes from the end of the list to its start: where attention is local, the blocks nearest the queries set the
   // reference maxima, and little outgrows them.
   auto find = [&](const AttnParams& p, int id, Unit& u) __attribute__((always_inline)) {
-    if (!find_unit<kPlanned>(p, id, u) || !find_list<kHasList, kPlanned>(p, u)) return false;
+    if (!find_unit<kHasList, kPlanned, true>(p, id, u) || !find_list<kHasList, kPlanned>(p, u)) return false;
     u.kb = u.kb_next = 0;
     if (u.n_blocks > 0) {
       u.kb = kHasList ? clamp_block(u.list[u.n_blocks - 1], p.nkb) : u.first + u.n_blocks - 1;
@@ -334,6 +334,11 @@ __global__ __launch_bounds__(128, 1) void block_sparse_fwd64_kernel(AttnParams) 
   Unit u;
   {
     const AttnParams& p = reread_params();
+    if (p.lists_decide && p.totals) {          // mostly no q-block is this kernel's, or many are
+      bool any = false;
+      for (int qb = p.qb_begin + (int)(threadIdx.x & 63); qb < p.qb_end; qb += 64) any = any || long_and_alike(p.H, (int)p.totals[32 * (qb - p.idx_row0)], (int)p.totals[32 * (qb - p.idx_row0) + 1]);
+      if (!__any(any)) return;
+    }
     if (!find(p, (int)blockIdx.x, u)) {
       if (!p.queue) return;
       const int id = hand_out<kHasList, kPlanned>(p, threadIdx.x == 0 ? ask_next(p) : 0, wave, (int)threadIdx.x & 63, true, stage);

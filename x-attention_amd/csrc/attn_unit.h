@@ -26,6 +26,8 @@ struct AttnParams {
   AttnPlan plan;            // kPlanned only
   int32_t* queue;           // this launch's work queue (kQueueWords, zero), or null: one workgroup per id
   int unit_ids;             // ids of units, grid_for()
+  int lists_decide;         // q-blocks with long lists, all much alike, are the 64-row kernel's, others the 32-row's (has_rows64)
+  const uint32_t* totals;   // blocks of a q-block's lists and of the longest at 32 * (q-block - idx_row0), or null: to be found
 };
 
 // The kernel's parameters, read anew: between two units nothing that is computed from them is kept, which would take more
@@ -39,6 +41,32 @@ __device__ __forceinline__ const AttnParams& reread_params() {
 __device__ __forceinline__ int clamp_block(int kb, int nkb) { return kb < 0 ? 0 : (kb < nkb ? kb : nkb - 1); }
 
 typedef const __attribute__((address_space(4))) int32_t* const_i32_ptr;
+
+// Blocks that a q-block sees without lists.
+__device__ __forceinline__ int visible_blocks(const AttnParams& p, int qb) {
+  const int q_last = (qb * kBlk + kBlk - 1 < p.Lq ? qb * kBlk + kBlk - 1 : p.Lq - 1) + p.kv_off;
+  const int visible = p.causal ? (q_last < 0 ? 0 : q_last / kBlk + 1) : p.nkb;
+  return visible < p.nkb ? visible : p.nkb;
+}
+
+// Whether q-block qb is the 64-row kernel's, where its lists decide.  By whole wavefronts, the same for all.
+__device__ __forceinline__ bool long_and_alike(int heads, int total, int longest) { return total >= 8 * heads && longest * heads < 2 * total; }
+template <bool kHasList>
+__device__ __forceinline__ bool has_rows64(const AttnParams& p, int qb) {
+  if (!kHasList) return long_and_alike(p.H, p.H * visible_blocks(p, qb), visible_blocks(p, qb));
+  if (p.totals) {
+    const const_i32_ptr of = (const_i32_ptr)(uintptr_t)(p.totals + 32 * (qb - p.idx_row0));
+    return long_and_alike(p.H, of[0], of[1]);
+  }
+  int total = 0, longest = 0;
+  for (int h = (int)(threadIdx.x & 63); h < p.H; h += 64) {
+    int n = p.col_cnt[(int64_t)h * p.idx_rows + (qb - p.idx_row0)];
+    n = n < 0 ? 0 : n > p.idx_pitch ? (int)p.idx_pitch : n;
+    total += n;
+    longest = longest > n ? longest : n;
+  }
+  return long_and_alike(p.H, __builtin_amdgcn_readlane(wave_scan(total), 63), (int)wave_max((uint32_t)longest));
+}
 
 // What an id stands for.
 struct Unit {
@@ -64,7 +92,7 @@ __device__ __forceinline__ Unit uniform(const Unit& u) {
 
 // The (head, q-block) with this id; false: there is none.
 template <bool kPlanned>
-__device__ __forceinline__ bool find_unit(const AttnParams& p, int id, Unit& u) {
+__device__ __forceinline__ bool find_place(const AttnParams& p, int id, Unit& u) {
   u.piece = -1;
   u.skip = 0;
   if (kPlanned) {
@@ -83,6 +111,11 @@ __device__ __forceinline__ bool find_unit(const AttnParams& p, int id, Unit& u) 
     }
   }
   return map_workgroup(id - u.skip, p.shape, p.qb_begin, p.qb_end, &u.head, &u.qb, &u.kvh);
+}
+// ... or it is the other kernel's.
+template <bool kHasList, bool kPlanned, bool kRows64>
+__device__ __forceinline__ bool find_unit(const AttnParams& p, int id, Unit& u) {
+  return find_place<kPlanned>(p, id, u) && (!p.lists_decide || has_rows64<kHasList>(p, u.qb) == kRows64);
 }
 __device__ __forceinline__ int64_t unit_slot(const AttnParams& p, const Unit& u) { return (int64_t)u.head * p.idx_rows + (u.qb - p.idx_row0); }
 
@@ -132,9 +165,7 @@ __device__ __forceinline__ bool find_list(const AttnParams& p, Unit& u) {
     const int n = ((const_i32_ptr)(uintptr_t)p.col_cnt)[slot];
     u.n_blocks = n < 0 ? 0 : (n > p.idx_pitch ? (int)p.idx_pitch : n);
   } else {
-    const int q_last = (u.qb * kBlk + kBlk - 1 < p.Lq ? u.qb * kBlk + kBlk - 1 : p.Lq - 1) + p.kv_off;
-    const int visible = p.causal ? (q_last < 0 ? 0 : q_last / kBlk + 1) : p.nkb;
-    u.n_blocks = visible < p.nkb ? visible : p.nkb;
+    u.n_blocks = visible_blocks(p, u.qb);
   }
   if (kPlanned) {
     const uint32_t cut = u.n_blocks > p.plan.shape.min_piece ? (uint32_t)((const_i32_ptr)(uintptr_t)p.plan.cut)[slot] : 0;
@@ -159,7 +190,7 @@ __device__ __forceinline__ int hand_out(const AttnParams& p, int ticket, int wav
     for (;;) {
       next = next_id<kPlanned>(p, ticket, lane, few);
       Unit u;
-      if (next < 0 || (find_unit<kPlanned>(p, next, u) && find_list<kHasList, kPlanned>(p, u))) break;
+      if (next < 0 || (find_unit<kHasList, kPlanned, true>(p, next, u) && find_list<kHasList, kPlanned>(p, u))) break;
       if (lane == 0) ticket = ask_next(p);
     }
     if (lane == 0) *reinterpret_cast<int*>(scratch) = next;

@@ -64,18 +64,30 @@ static int first_rows64(int H, int nqb, int nkb, int kv_off, int causal) {
   return qb < nqb ? (int)qb : nqb;
 }
 
+// In between - prompts whose q-blocks see up to 384 blocks, with units enough that a second launch costs little (3 us where it
+// has nothing to do) - the lists decide, q-block for q-block (long_and_alike): 64 rows where they have 8 blocks on average and
+// the longest is less than twice that, as of video.  Whole calls, us, 32 rows / by the lists: video of 18000 tokens 1425 / 1274,
+// of 32000 4180 / 3700; text of 32768, which stays with 32 rows, 535 / 533.  Unlike lists would give two launches with an
+// end of their own each, and one long list takes twice as long (32768 tokens, few long heads, with a line on the total alone: 1340 / 1640).
+static bool lists_decide(int H, int nqb, int nkb, int kv_off, int causal) {
+  return causal && nkb < 384 && kv_off < 128 * kBlk && (int64_t)H * nqb >= 3584;
+}
+
 // Whether the 64-row kernel has a work queue: where units, or the pieces of a chunk's, go several times through the places
 // (us without / with: 2048 on 63488 716 / 648, 1000 on 30000 221 / 214; but 500 on 60000, 128 units, 181 / 195; a field of
 // 4000, 768 like units, 229 / 235: dealt by the launch, the second round's find CUs of their own).
 bool xattn::attention_queued(int num_heads, int q_len, int k_len, int causal) {
   const int nqb = (int)(((int64_t)q_len + kBlk - 1) / kBlk), nkb = (int)(((int64_t)k_len + kBlk - 1) / kBlk);
   const int64_t units = (int64_t)num_heads * nqb;
-  return first_rows64(num_heads, nqb, nkb, k_len - q_len, causal) < nqb && (units > 1024 || (units >= 256 && nkb >= 2 * nqb));
+  return (first_rows64(num_heads, nqb, nkb, k_len - q_len, causal) < nqb || lists_decide(num_heads, nqb, nkb, k_len - q_len, causal)) &&
+         (units > 1024 || (units >= 256 && nkb >= 2 * nqb));
 }
 
 template <bool kHasList, bool kPlanned>
 static int launch_fwd(AttnParams p, int64_t extra, hipStream_t s) {
-  const int begin = p.qb_begin, end = p.qb_end, split = first_rows64(p.H, p.nqb, p.nkb, p.kv_off, p.causal);
+  p.lists_decide = lists_decide(p.H, p.nqb, p.nkb, p.kv_off, p.causal);
+  const int begin = p.qb_begin, end = p.qb_end, first64 = first_rows64(p.H, p.nqb, p.nkb, p.kv_off, p.causal);
+  const int split = p.lists_decide ? begin : first64, end32 = p.lists_decide || end < split ? end : split;
   const int cus = resident_workgroups();
   if (cus <= 0) return XATTN_ERR_LAUNCH;
   const int places = 2 * cus / kQueues * kQueues;
@@ -91,7 +103,7 @@ static int launch_fwd(AttnParams p, int64_t extra, hipStream_t s) {
     if (hipGetLastError() != hipSuccess) return XATTN_ERR_LAUNCH;
   }
   p.qb_begin = begin;
-  p.qb_end = end < split ? end : split;
+  p.qb_end = end32;
   if (begin < p.qb_end) {
     hipLaunchKernelGGL((block_sparse_fwd_kernel<kHasList, kPlanned>), grid(false), dim3(256), 0, s, p);
     if (hipGetLastError() != hipSuccess) return XATTN_ERR_LAUNCH;
@@ -109,7 +121,8 @@ int xattn::block_sparse_impl(const void* q, const void* k, const void* v, void* 
                                       int64_t k_stride_n, int64_t v_stride_h, int64_t v_stride_n,
                                       int64_t o_stride_h, int64_t o_stride_n, int q_block_begin, int q_block_end,
                                       int causal, float softmax_scale, void* stream,
-                                      const AttnPlan* plan, bool note, int32_t* queue) {
+                                      const AttnPlan* plan, bool note, int32_t* queue,
+                                      const uint32_t* totals) {
   if (!q || !k || !v || !out) return XATTN_ERR_NULL;
   if (head_dim != kHeadDim) return XATTN_ERR_HEAD_DIM;
   if (num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads) return XATTN_ERR_HEADS;
@@ -153,6 +166,7 @@ int xattn::block_sparse_impl(const void* q, const void* k, const void* v, void* 
   hipStream_t s = static_cast<hipStream_t>(stream);
   p.plan = AttnPlan{};
   p.queue = queue;
+  p.totals = totals;
   if (plan) {
     p.plan = *plan;
     const int64_t most = ((int64_t)plan_pieces(plan->shape, q_block_end - q_block_begin) + 7) / 8 * 8;
@@ -173,7 +187,7 @@ extern "C" int xattn_block_sparse_fwd(const void* q, const void* k, const void* 
                                       int causal, float softmax_scale, void* stream) {
   return block_sparse_impl(q, k, v, out, col_idx, col_cnt, idx_pitch, idx_rows, idx_row0, num_heads, num_kv_heads, q_len, k_len,
                            head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n, o_stride_h,
-                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, nullptr, false, nullptr);
+                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, nullptr, false, nullptr, nullptr);
 }
 
 namespace {
@@ -213,5 +227,9 @@ extern "C" int xattn_block_sparse_fwd_ws(const void* q, const void* k, const voi
   }
   return block_sparse_impl(q, k, v, out, col_idx, col_cnt, idx_pitch, idx_rows, idx_row0, num_heads, num_kv_heads, q_len, k_len,
                            head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n, o_stride_h,
-                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, need ? &plan : nullptr, true, nullptr);
+                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, need ? &plan : nullptr, true, nullptr, nullptr);
+}
+
+bool xattn::attention_asks_totals(int num_heads, int q_len, int k_len, int causal) {
+  return lists_decide(num_heads, (int)(((int64_t)q_len + kBlk - 1) / kBlk), (int)(((int64_t)k_len + kBlk - 1) / kBlk), k_len - q_len, causal);
 }

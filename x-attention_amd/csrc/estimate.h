@@ -19,6 +19,7 @@ struct SelectArgs {
   int keep_sink, keep_recent;
   int real_q_blocks_only;   // leave out the rows of q-blocks past the sequence end
   const AttnPlan* plan;     // null, or where to note long lists for the attention (lists of all q-blocks of a head)
+  uint32_t* totals;         // null, or where to find blocks of each q-block's lists, and of its longest, at 32 * (row)
   unsigned long long* clear;   // words set to zero for what follows, or null
   int clear_words;
   int stages;               // bit 0: run the GEMM pass, bit 1: run the normalise-and-select pass
@@ -42,11 +43,13 @@ size_t estimate_real_rows_bytes(int num_heads, int q_len, int k_len, int stride,
 // kQueueBytes zeros (null: a workgroup for each list and piece)
 constexpr size_t kQueueBytes = 4096;
 bool attention_queued(int num_heads, int q_len, int k_len, int causal);
+// whether the attention asks for the blocks of each q-block's lists and of its longest, 128 bytes apart (null: it finds them)
+bool attention_asks_totals(int num_heads, int q_len, int k_len, int causal);
 int block_sparse_impl(const void* q, const void* k, const void* v, void* out, const int32_t* col_idx, const int32_t* col_cnt,
                       int64_t idx_pitch, int idx_rows, int idx_row0, int num_heads, int num_kv_heads, int q_len, int k_len,
                       int head_dim, int64_t q_stride_h, int64_t q_stride_n, int64_t k_stride_h, int64_t k_stride_n,
                       int64_t v_stride_h, int64_t v_stride_n, int64_t o_stride_h, int64_t o_stride_n, int q_block_begin,
                       int q_block_end, int causal, float softmax_scale, void* stream, const AttnPlan* plan, bool note,
-                      int32_t* queue);
+                      int32_t* queue, const uint32_t* totals);
 
 }  // namespace xattn

@@ -1117,6 +1117,7 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
     if (!sel->tau)
       for (int h = 0; h < sel->tau_host_count; ++h) sp.tau_val[h] = sel->tau_host[h];
     sp.plan = sel->plan ? *sel->plan : AttnPlan{};
+    sp.totals = sel->totals;
     sp.sums_out = static_cast<__bf16*>(sel->sums_out);
     sp.mask = sel->mask; sp.col_idx = sel->col_idx; sp.col_cnt = sel->col_cnt;
     sp.idx_pitch = sel->idx_pitch; sp.H = num_heads; sp.nqb = g.nqb; sp.nkb = g.nkb;

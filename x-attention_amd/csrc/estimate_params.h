@@ -52,8 +52,8 @@ struct EstParams {
 // Place of row `rel` (counted from row_begin) in P, for key block 0; the next key block's is kStrip on.  Strips of 32 rows, key
 // block after key block: what a workgroup of the selection reads lies together, and a wavefront of the estimate writes two key
 // blocks of its rows with one store at a constant offset.  Key block after key block with all rows of each, the selection read
-// 128 bytes every 4 * rows and half a wavefront wrote at a time: estimate of 131072 tokens 505 us per chunk of 16384, 494 now,
-// selection of 32768 tokens 52 / 48, of a video of 65536 160 / 147.
+// 128 bytes every 4 * rows and half a wavefront wrote at a time (us, that way / this way: estimate and selection of 131072
+// tokens 3831 / 3790, of 15000 153.5 / 149; selection alone of 32768 52 / 48, of a video of 65536 160 / 147).
 constexpr int kStrip = 32;
 __host__ __device__ inline int strips_of(int rows) { return (rows + kStrip - 1) / kStrip; }
 __device__ __forceinline__ int64_t partial_at(const EstParams& p, int head, int rel) {

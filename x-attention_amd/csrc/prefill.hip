@@ -17,7 +17,7 @@ using namespace xattn;
 
 namespace {
 struct PrefillLayout {
-  size_t est_bytes, cnt_off, idx_off, queue_off, plan_off, total;
+  size_t est_bytes, cnt_off, idx_off, queue_off, totals_bytes, plan_off, total;
   int nqb, nkb;
   PlanShape plan;
 };
@@ -33,7 +33,8 @@ bool prefill_layout(int num_heads, int q_len, int k_len, int stride, int chunk_s
   l->cnt_off = up256(l->est_bytes);
   l->idx_off = l->cnt_off + up256((size_t)num_heads * l->nqb * sizeof(int32_t));
   l->queue_off = l->idx_off + up256((size_t)num_heads * l->nqb * l->nkb * sizeof(int32_t));
-  l->plan_off = l->queue_off + kQueueBytes;                  // (cleared together)
+  l->totals_bytes = up256((size_t)l->nqb * 128);
+  l->plan_off = l->queue_off + kQueueBytes + l->totals_bytes;                  // (cleared together)
   const int64_t units = (int64_t)num_heads * l->nqb;
   l->plan = plan_shape(num_heads, q_len, k_len);
   l->total = l->plan_off + plan_bytes(l->plan, units, l->nqb);
@@ -86,14 +87,15 @@ extern "C" int xattn_prefill_fwd(const void* q, const void* k, const void* v, vo
   const int64_t last_token = (int64_t)l.nqb * 128 - 1 + (int64_t)(k_chunks - q_chunks) * chunk_size;   // on the key axis, both padded
   const bool may_cut = l.plan.per_qb && (!causal || keep_sink || last_token / 128 + 1 > l.plan.min_piece);
   if (may_cut && zero_rows_from != 0) sel.plan = &plan;
-  int32_t* const queue = zero_rows_from != 0 && attention_queued(num_heads, q_len, k_len, causal) ? reinterpret_cast<int32_t*>(ws + l.queue_off) : nullptr;
-  if (sel.plan) {
-    sel.clear = plan.noted;
-    sel.clear_words = (int)((plan_noted_bytes(l.nqb) + plan_round((size_t)units * 4)) / 8);
-  }
-  if (queue) {
-    sel.clear = reinterpret_cast<unsigned long long*>(queue);        // (what is noted lies behind it)
-    sel.clear_words += (int)(kQueueBytes / 8);
+  // Ahead of what is noted lie the attention's queue and the q-blocks' totals; the estimate clears them together.
+  const bool cleared = zero_rows_from != 0, queued = cleared && attention_queued(num_heads, q_len, k_len, causal);
+  int32_t* const queue = queued ? reinterpret_cast<int32_t*>(ws + l.queue_off) : nullptr;
+  if (cleared && attention_asks_totals(num_heads, q_len, k_len, causal)) sel.totals = reinterpret_cast<uint32_t*>(ws + l.queue_off + kQueueBytes);
+  if (queue || sel.totals || sel.plan) {
+    const size_t from = queue ? l.queue_off : sel.totals ? l.queue_off + kQueueBytes : l.plan_off;
+    const size_t noted = sel.plan ? plan_noted_bytes(l.nqb) + plan_round((size_t)units * 4) : 0;
+    sel.clear = reinterpret_cast<unsigned long long*>(ws + from);
+    sel.clear_words = (int)((l.plan_off - from + noted) / 8);
   }
   int rc = estimate_impl(q, k, nullptr, ws, l.est_bytes, nullptr, num_heads, num_kv_heads, q_len, k_len, head_dim,
                          q_stride_h, q_stride_n, k_stride_h, k_stride_n, stride, 128, chunk_size, 0, q_chunks, causal,
@@ -101,7 +103,7 @@ extern "C" int xattn_prefill_fwd(const void* q, const void* k, const void* v, vo
   if (rc != XATTN_OK) return rc;
   return block_sparse_impl(q, k, v, out, sel.col_idx, sel.col_cnt, l.nkb, l.nqb, 0, num_heads, num_kv_heads, q_len,
                            k_len, head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n,
-                           o_stride_h, o_stride_n, 0, l.nqb, causal, softmax_scale, stream, may_cut ? &plan : nullptr, !sel.plan, queue);
+                           o_stride_h, o_stride_n, 0, l.nqb, causal, softmax_scale, stream, may_cut ? &plan : nullptr, !sel.plan, queue, sel.totals);
 }
 
 extern "C" int xattn_estimate_fwd(const void* q, const void* k, void* block_sums, uint8_t* mask, void* workspace,

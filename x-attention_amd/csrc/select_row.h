@@ -24,6 +24,7 @@ struct SelParams {
   int blocks_per_chunk;
   int npow2;   // LDS key capacity (power of two >= nkb)
   AttnPlan plan;   // per_qb 0: nothing is noted
+  uint32_t* totals;   // null, or where blocks of each q-block's lists, and of its longest, are found: 32 * (row - win_row0)
 };
 
 constexpr int kSlots = 16;        // candidates per lane held in registers (rows up to 1024 candidates)
@@ -401,6 +402,11 @@ __device__ __forceinline__ void select_row(const SelParams& p, const float* x, i
     }
     count = count < p.idx_pitch ? count : (int)p.idx_pitch;
     if (lane == 0) p.col_cnt[slot] = count;
+    if (lane == 0 && p.totals) {
+      uint32_t* const of = p.totals + 32 * (row - p.win_row0);
+      __hip_atomic_fetch_add(of, (uint32_t)count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_fetch_max(of + 1, (uint32_t)count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     if (p.plan.shape.per_qb && (p.causal ? q_last / 128 + 1 : p.list_cols) > p.plan.shape.min_piece)   // else too few blocks to be cut
       list_made(p.plan, p.H, p.win_rows, row - p.win_row0, head, count, lane);
   }
