@@ -6,6 +6,19 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
+def _workgroup_per_unit(q, k, v, idx, cnt, causal):
+    """The entry point without a workspace: no queue, no list cut."""
+    from xattn.src import hip_backend as hb
+
+    heads, q_len, k_len = q.shape[1], q.shape[2], k.shape[2]
+    out = torch.empty(1, q_len, heads, 128, dtype=torch.bfloat16, device="cuda")
+    hb.check(hb.lib().xattn_block_sparse_fwd(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), idx.data_ptr(), cnt.data_ptr(), idx.shape[2], idx.shape[1], 0,
+        heads, k.shape[1], q_len, k_len, 128, q.stride(1), q.stride(2), k.stride(1), k.stride(2), v.stride(1), v.stride(2),
+        out.stride(2), out.stride(1), 0, -1, int(causal), 128 ** -0.5, torch.cuda.current_stream().cuda_stream), "fwd")
+    return out.transpose(1, 2)
+
+
 # units just past the rules' lines; pieces beside units that are whole; groups of heads that fill a run of ids (64) and that
 # do not (7, 3), so that some ids stand for nothing; few long heads; two launches (the first q-blocks have 32 rows)
 @pytest.mark.parametrize("q_len,cache,heads,kv_heads,long_heads,causal", [
@@ -15,6 +28,7 @@ pytestmark = pytest.mark.gpu
     (2048, 20000, 28, 4, list(range(0, 28, 2)), True),
     (2048, 30000, 16, 16, list(range(16)), True),
     (66000, 0, 16, 4, [6], True),
+    (10000, 0, 56, 8, [6], False),
 ])
 def test_queue_gives_the_same_as_a_workgroup_per_unit(q_len, cache, heads, kv_heads, long_heads, causal):
     from xattn.src.Xattention import Xattention_prefill, block_sparse_attention, estimate_and_select
@@ -26,9 +40,15 @@ def test_queue_gives_the_same_as_a_workgroup_per_unit(q_len, cache, heads, kv_he
     taus[torch.tensor(long_heads)] = 1.0
     r = estimate_and_select(q, k, 8, taus, chunk, causal=causal, want_mask=False, want_sums=False)
     idx, cnt = r["col_idx"][:, :nq].contiguous(), r["col_cnt"][:, :nq].contiguous()
-    want = block_sparse_attention(q, k, v, idx, cnt, causal=causal)
-    for _ in range(3):                                            # whoever takes what
-        assert torch.equal(Xattention_prefill(q, k, v, 8, threshold=taus, chunk_size=chunk, causal=causal), want)
+    got = Xattention_prefill(q, k, v, 8, threshold=taus, chunk_size=chunk, causal=causal)
+    for _ in range(2):                                            # whoever takes what
+        assert torch.equal(Xattention_prefill(q, k, v, 8, threshold=taus, chunk_size=chunk, causal=causal), got)
+        assert torch.equal(block_sparse_attention(q, k, v, idx, cnt, causal=causal), got)
+    want = _workgroup_per_unit(q, k, v, idx, cnt, causal)
+    if heads * nq > 4096:                                         # no list is cut
+        assert torch.equal(got, want)
+    bound = 2.0 ** -8 * (v.float().abs().amax() + want.float().abs())          # as in test_gpu_attention_plan.py
+    assert ((got.float() - want.float()).abs() <= bound).all()
 
 
 # prompts of 3584 units and more that see fewer than 384 blocks: of some q-blocks all lists are long (64 rows per wavefront), of
@@ -38,6 +58,7 @@ def test_queue_gives_the_same_as_a_workgroup_per_unit(q_len, cache, heads, kv_he
     (14300, 32, 8, list(range(0, 32, 3))),
     (6700, 70, 7, list(range(0, 66))),
     (14336, 32, 32, []),
+    (17000, 32, 8, list(range(0, 32))),
 ])
 def test_lists_choose_the_kernel_the_same_way_by_every_path(q_len, heads, kv_heads, long_heads):
     from xattn.src.Xattention import Xattention_prefill, block_sparse_attention, estimate_and_select
@@ -51,6 +72,8 @@ def test_lists_choose_the_kernel_the_same_way_by_every_path(q_len, heads, kv_hea
     idx, cnt = r["col_idx"][:, :nq].contiguous(), r["col_cnt"][:, :nq].contiguous()
     got = Xattention_prefill(q, k, v, 16, threshold=taus, chunk_size=128)
     assert torch.equal(block_sparse_attention(q, k, v, idx, cnt), got)
+    if heads * nq > 4096:
+        assert torch.equal(_workgroup_per_unit(q, k, v, idx, cnt, True), got)
     parts = torch.empty(1, q_len, heads, 128, dtype=torch.bfloat16, device="cuda")
     for a, b in ((0, nq // 3), (nq // 3, nq)):
         block_sparse_attention(q, k, v, idx, cnt, out=parts, q_blocks=(a, b))

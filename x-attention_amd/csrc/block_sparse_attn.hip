@@ -40,6 +40,10 @@ __global__ __launch_bounds__(1024) void note_lists_kernel(AttnParams p) {
   if (threadIdx.x == 0) *p.plan.noted = (unsigned long long)pieces;
 }
 
+static_assert(kQueueBytes == kQueueWords * 4, "estimate.h");
+// Makes a work queue ready, where no pass before the launch has.
+__global__ void clear_queue_kernel(int32_t* queue) { queue[blockIdx.x * 256 + threadIdx.x] = 0; }
+
 }  // namespace xattn
 
 using namespace xattn;
@@ -203,7 +207,9 @@ PlanShape shape_of(int num_heads, int q_len, int k_len, bool listed) {
 extern "C" size_t xattn_block_sparse_workspace_bytes(int num_heads, int q_len, int k_len, int idx_rows, int q_blocks) {
   if (num_heads <= 0 || q_len <= 0 || k_len <= 0 || idx_rows < 0 || q_blocks <= 0) return 0;
   const int64_t rows = idx_rows ? idx_rows : ((int64_t)q_len + kBlk - 1) / kBlk;
-  return plan_bytes(shape_of(num_heads, q_len, k_len, idx_rows != 0), num_heads * rows, q_blocks);
+  const size_t plan = plan_bytes(shape_of(num_heads, q_len, k_len, idx_rows != 0), num_heads * rows, q_blocks);
+  const bool queued = attention_queued(num_heads, q_len, k_len, 0) || attention_queued(num_heads, q_len, k_len, 1);
+  return plan_round(plan) + (queued ? kQueueBytes : 0);
 }
 
 extern "C" int xattn_block_sparse_fwd_ws(const void* q, const void* k, const void* v, void* out, void* workspace,
@@ -217,17 +223,24 @@ extern "C" int xattn_block_sparse_fwd_ws(const void* q, const void* k, const voi
   if (q_block_end < 0) q_block_end = (q_len + kBlk - 1) / kBlk;
   const int nqb = (q_len + kBlk - 1) / kBlk, q_blocks = q_block_end - q_block_begin;
   const size_t need = xattn_block_sparse_workspace_bytes(num_heads, q_len, k_len, col_idx ? idx_rows : 0, q_blocks);
+  const PlanShape shape = num_heads > 0 ? shape_of(num_heads, q_len, k_len, col_idx != nullptr) : PlanShape{};
   if (!col_idx) idx_rows = nqb, idx_row0 = 0;
   AttnPlan plan{};
-  if (need) {
+  int32_t* queue = nullptr;
+  if (shape.per_qb && need) {
     if (!workspace) return XATTN_ERR_NULL;
     if (workspace_bytes < need) return XATTN_ERR_WORKSPACE;
     if (reinterpret_cast<uintptr_t>(workspace) & 255) return XATTN_ERR_ALIGN;
-    plan = plan_at(shape_of(num_heads, q_len, k_len, col_idx != nullptr), static_cast<char*>(workspace), (int64_t)num_heads * idx_rows, q_blocks);
+    plan = plan_at(shape, static_cast<char*>(workspace), (int64_t)num_heads * idx_rows, q_blocks);
+  }
+  if (workspace && workspace_bytes >= need && need >= kQueueBytes && !(reinterpret_cast<uintptr_t>(workspace) & 255) &&
+      attention_queued(num_heads, q_len, k_len, causal)) {
+    queue = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + need - kQueueBytes);
+    hipLaunchKernelGGL(clear_queue_kernel, dim3(kQueueWords / 256), dim3(256), 0, static_cast<hipStream_t>(stream), queue);
   }
   return block_sparse_impl(q, k, v, out, col_idx, col_cnt, idx_pitch, idx_rows, idx_row0, num_heads, num_kv_heads, q_len, k_len,
                            head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n, o_stride_h,
-                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, need ? &plan : nullptr, true, nullptr, nullptr);
+                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, plan.noted ? &plan : nullptr, true, queue, nullptr);
 }
 
 bool xattn::attention_asks_totals(int num_heads, int q_len, int k_len, int causal) {
