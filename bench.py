@@ -39,8 +39,8 @@ PEAK_HBM_GBS = 8000.0
 # this process): the summary of those runs for the headline workload is kept as a table under profiles/ and read here.
 TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "bench_headline_hbm_traffic.md")
 HEADLINE = "cfg2_llama8b_L131072_gqa32x8_S16"
-KERNEL_SOURCES = ("attn_plan.h", "attn_tiles.h", "block_sparse_attn.hip", "estimate.hip", "estimate_params.h", "select_row.h",
-                  "select_blocks.hip", "xattn_common.h")
+KERNEL_SOURCES = ("attn_plan.h", "attn_rows32.h", "attn_rows64.h", "attn_tiles.h", "attn_unit.h", "block_sparse_attn.hip",
+                  "estimate.hip", "estimate_params.h", "select_row.h", "select_blocks.hip", "xattn_common.h")
 
 
 def kernel_source_hash():
