@@ -336,7 +336,7 @@ __global__ __launch_bounds__(128, 1) void block_sparse_fwd64_kernel(AttnParams) 
     const AttnParams& p = reread_params();
     if (p.lists_decide && p.totals) {          // mostly no q-block is this kernel's, or many are
       bool any = false;
-      for (int qb = p.qb_begin + (int)(threadIdx.x & 63); qb < p.qb_end; qb += 64) any = any || long_and_alike(p.H, (int)p.totals[32 * (qb - p.idx_row0)], (int)p.totals[32 * (qb - p.idx_row0) + 1]);
+      for (int qb = p.qb_begin + (int)(threadIdx.x & 63); qb < p.qb_end; qb += 64) any = any || long_lists(p, (int)p.totals[32 * (qb - p.idx_row0)], (int)p.totals[32 * (qb - p.idx_row0) + 1]);
       if (!__any(any)) return;
     }
     if (!find(p, (int)blockIdx.x, u)) {

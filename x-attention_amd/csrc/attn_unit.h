@@ -7,6 +7,9 @@
 
 namespace xattn {
 
+// Which q-blocks are the 64-row kernel's: those of its launch; those whose lists have so many blocks on average (and are much alike).
+enum ListsDecide { kNot, kFrom8, kFrom8Alike, kFrom24 };
+
 struct AttnParams {
   const __bf16* q;
   const __bf16* k;
@@ -26,7 +29,7 @@ struct AttnParams {
   AttnPlan plan;            // kPlanned only
   int32_t* queue;           // this launch's work queue (kQueueWords, zero), or null: one workgroup per id
   int unit_ids;             // ids of units, grid_for()
-  int lists_decide;         // q-blocks with long lists, all much alike, are the 64-row kernel's, others the 32-row's (has_rows64)
+  int lists_decide;         // ListsDecide: q-blocks with long lists are the 64-row kernel's, others the 32-row's
   const uint32_t* totals;   // blocks of a q-block's lists and of the longest at 32 * (q-block - idx_row0), or null: to be found
 };
 
@@ -50,13 +53,15 @@ __device__ __forceinline__ int visible_blocks(const AttnParams& p, int qb) {
 }
 
 // Whether q-block qb is the 64-row kernel's, where its lists decide.  By whole wavefronts, the same for all.
-__device__ __forceinline__ bool long_and_alike(int heads, int total, int longest) { return total >= 8 * heads && longest * heads < 2 * total; }
+__device__ __forceinline__ bool long_lists(const AttnParams& p, int total, int longest) {
+  return total >= (p.lists_decide == kFrom24 ? 24 : 8) * p.H && (p.lists_decide != kFrom8Alike || longest * p.H < 2 * total);
+}
 template <bool kHasList>
 __device__ __forceinline__ bool has_rows64(const AttnParams& p, int qb) {
-  if (!kHasList) return long_and_alike(p.H, p.H * visible_blocks(p, qb), visible_blocks(p, qb));
+  if (!kHasList) return long_lists(p, p.H * visible_blocks(p, qb), visible_blocks(p, qb));
   if (p.totals) {
     const const_i32_ptr of = (const_i32_ptr)(uintptr_t)(p.totals + 32 * (qb - p.idx_row0));
-    return long_and_alike(p.H, of[0], of[1]);
+    return long_lists(p, of[0], of[1]);
   }
   int total = 0, longest = 0;
   for (int h = (int)(threadIdx.x & 63); h < p.H; h += 64) {
@@ -65,7 +70,7 @@ __device__ __forceinline__ bool has_rows64(const AttnParams& p, int qb) {
     total += n;
     longest = longest > n ? longest : n;
   }
-  return long_and_alike(p.H, __builtin_amdgcn_readlane(wave_scan(total), 63), (int)wave_max((uint32_t)longest));
+  return long_lists(p, __builtin_amdgcn_readlane(wave_scan(total), 63), (int)wave_max((uint32_t)longest));
 }
 
 // What an id stands for.

@@ -41,8 +41,28 @@ __global__ __launch_bounds__(1024) void note_lists_kernel(AttnParams p) {
 }
 
 static_assert(kQueueBytes == kQueueWords * 4, "estimate.h");
-// Makes a work queue ready, where no pass before the launch has.
-__global__ void clear_queue_kernel(int32_t* queue) { queue[blockIdx.x * 256 + threadIdx.x] = 0; }
+// What no pass before the launch has made ready: a work queue (or null), and of each q-block the blocks of its lists and of the
+// longest (or null).  A wavefront per q-block.
+__global__ __launch_bounds__(64) void ready_kernel(AttnParams p, int32_t* queue, uint32_t* totals) {
+  const int lane = threadIdx.x;
+  if (queue)
+    for (int i = (int)blockIdx.x * 64 + lane; i < kQueueWords; i += (int)gridDim.x * 64) queue[i] = 0;
+  if (!totals) return;
+  const int row = p.qb_begin + (int)blockIdx.x - p.idx_row0;
+  int total = 0, longest = 0;
+  for (int h = lane; h < p.H; h += 64) {
+    int n = p.col_cnt[(int64_t)h * p.idx_rows + row];
+    n = n < 0 ? 0 : n > p.idx_pitch ? (int)p.idx_pitch : n;
+    total += n;
+    longest = longest > n ? longest : n;
+  }
+  total = wave_scan(total);
+  longest = (int)wave_max((uint32_t)longest);
+  if (lane == 63) {
+    totals[32 * row] = (uint32_t)total;
+    totals[32 * row + 1] = (uint32_t)longest;
+  }
+}
 
 }  // namespace xattn
 
@@ -68,13 +88,20 @@ static int first_rows64(int H, int nqb, int nkb, int kv_off, int causal) {
   return qb < nqb ? (int)qb : nqb;
 }
 
-// In between - prompts whose q-blocks see up to 384 blocks, with units enough that a second launch costs little (3 us where it
-// has nothing to do) - the lists decide, q-block for q-block (long_and_alike): 64 rows where they have 8 blocks on average and
-// the longest is less than twice that, as of video.  Whole calls, us, 32 rows / by the lists: video of 18000 tokens 1425 / 1274,
-// of 32000 4180 / 3700; text of 32768, which stays with 32 rows, 535 / 533.  Unlike lists would give two launches with an
-// end of their own each, and one long list takes twice as long (32768 tokens, few long heads, with a line on the total alone: 1340 / 1640).
-static bool lists_decide(int H, int nqb, int nkb, int kv_off, int causal) {
-  return causal && nkb < 384 && kv_off < 128 * kBlk && (int64_t)H * nqb >= 3584;
+// Of prompts by themselves, with units enough that a second launch costs little (3 us without a q-block of its own, 50 for
+// 32768 units that are the other's), the lists decide, q-block for q-block (long_lists).  Where q-blocks see fewer than 384
+// blocks: 64 rows where lists have 8 blocks on average and the longest is less than twice that, as of video - unlike lists would
+// give two launches with an end of their own each, and one long list takes twice as long (32768 tokens, few long heads, with a
+// line on the total alone: 1340 us with 32 rows / 1640).  Whole calls, us, 32 rows / by the lists: video of 18000 tokens
+// 1425 / 1274, of 32000 4180 / 3700; text of 32768, which stays with 32 rows, 535 / 533.  Longer ones outlast such ends: from 24 blocks
+// on average, of 24576 units and more from 8.  Text of six seeds, 32 rows / 64 from the 15th q-block on / from 24 / from 8: 131072
+// tokens 7386, 4741, 4787, 24708, 4735, 13665 / 6879, 4740, 4820, 21438, 4723, 11915 / 7279, 4657, 4731, 22069, 4644, 12431 / 7051, 4690,
+// 4790, 21534, 4634, 12029; 80000 3368, 2103, 2151, 9773, 2079, 5904 / 3173, 2154, 2194, 8326, 2124, 5136 / 3313, 2091, 2149, 8818,
+// 2064, 5667 / 3358, 2086, 2143, 8379, 2061, 5281; 50000, the first seed, 1671 / 1578 / 1645 / 1731.
+static int lists_decide(int H, int nqb, int nkb, int kv_off, int causal) {
+  const int64_t units = (int64_t)H * nqb;
+  if (!causal || kv_off >= 128 * kBlk || units < 3584) return kNot;
+  return nkb < 384 ? kFrom8Alike : units < 24576 ? kFrom24 : kFrom8;
 }
 
 // Whether the 64-row kernel has a work queue: where units, or the pieces of a chunk's, go several times through the places
@@ -126,7 +153,7 @@ int xattn::block_sparse_impl(const void* q, const void* k, const void* v, void* 
                                       int64_t o_stride_h, int64_t o_stride_n, int q_block_begin, int q_block_end,
                                       int causal, float softmax_scale, void* stream,
                                       const AttnPlan* plan, bool note, int32_t* queue,
-                                      const uint32_t* totals) {
+                                      uint32_t* totals, bool ready) {
   if (!q || !k || !v || !out) return XATTN_ERR_NULL;
   if (head_dim != kHeadDim) return XATTN_ERR_HEAD_DIM;
   if (num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads) return XATTN_ERR_HEADS;
@@ -171,6 +198,8 @@ int xattn::block_sparse_impl(const void* q, const void* k, const void* v, void* 
   p.plan = AttnPlan{};
   p.queue = queue;
   p.totals = totals;
+  if (!ready && (queue || totals))
+    hipLaunchKernelGGL(ready_kernel, dim3((unsigned)(q_block_end - q_block_begin)), dim3(64), 0, s, p, queue, totals);
   if (plan) {
     p.plan = *plan;
     const int64_t most = ((int64_t)plan_pieces(plan->shape, q_block_end - q_block_begin) + 7) / 8 * 8;
@@ -191,7 +220,7 @@ extern "C" int xattn_block_sparse_fwd(const void* q, const void* k, const void* 
                                       int causal, float softmax_scale, void* stream) {
   return block_sparse_impl(q, k, v, out, col_idx, col_cnt, idx_pitch, idx_rows, idx_row0, num_heads, num_kv_heads, q_len, k_len,
                            head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n, o_stride_h,
-                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, nullptr, false, nullptr, nullptr);
+                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, nullptr, false, nullptr, nullptr, true);
 }
 
 namespace {
@@ -204,12 +233,14 @@ PlanShape shape_of(int num_heads, int q_len, int k_len, bool listed) {
 }
 }  // namespace
 
+static size_t totals_bytes(int64_t rows, bool asked) { return asked ? plan_round((size_t)rows * 128) : 0; }
+
 extern "C" size_t xattn_block_sparse_workspace_bytes(int num_heads, int q_len, int k_len, int idx_rows, int q_blocks) {
   if (num_heads <= 0 || q_len <= 0 || k_len <= 0 || idx_rows < 0 || q_blocks <= 0) return 0;
   const int64_t rows = idx_rows ? idx_rows : ((int64_t)q_len + kBlk - 1) / kBlk;
   const size_t plan = plan_bytes(shape_of(num_heads, q_len, k_len, idx_rows != 0), num_heads * rows, q_blocks);
   const bool queued = attention_queued(num_heads, q_len, k_len, 0) || attention_queued(num_heads, q_len, k_len, 1);
-  return plan_round(plan) + (queued ? kQueueBytes : 0);
+  return plan_round(plan) + (queued ? kQueueBytes + totals_bytes(rows, idx_rows != 0 && attention_asks_totals(num_heads, q_len, k_len, 1)) : 0);
 }
 
 extern "C" int xattn_block_sparse_fwd_ws(const void* q, const void* k, const void* v, void* out, void* workspace,
@@ -233,16 +264,19 @@ extern "C" int xattn_block_sparse_fwd_ws(const void* q, const void* k, const voi
     if (reinterpret_cast<uintptr_t>(workspace) & 255) return XATTN_ERR_ALIGN;
     plan = plan_at(shape, static_cast<char*>(workspace), (int64_t)num_heads * idx_rows, q_blocks);
   }
+  uint32_t* totals = nullptr;
   if (workspace && workspace_bytes >= need && need >= kQueueBytes && !(reinterpret_cast<uintptr_t>(workspace) & 255) &&
       attention_queued(num_heads, q_len, k_len, causal)) {
-    queue = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + need - kQueueBytes);
-    hipLaunchKernelGGL(clear_queue_kernel, dim3(kQueueWords / 256), dim3(256), 0, static_cast<hipStream_t>(stream), queue);
+    const bool asked = col_idx && attention_asks_totals(num_heads, q_len, k_len, 1);
+    char* at = static_cast<char*>(workspace) + need - kQueueBytes - totals_bytes(idx_rows, asked);
+    queue = reinterpret_cast<int32_t*>(at);
+    if (asked && causal) totals = reinterpret_cast<uint32_t*>(at + kQueueBytes);
   }
   return block_sparse_impl(q, k, v, out, col_idx, col_cnt, idx_pitch, idx_rows, idx_row0, num_heads, num_kv_heads, q_len, k_len,
                            head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n, o_stride_h,
-                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, plan.noted ? &plan : nullptr, true, queue, nullptr);
+                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, plan.noted ? &plan : nullptr, true, queue, totals, false);
 }
 
 bool xattn::attention_asks_totals(int num_heads, int q_len, int k_len, int causal) {
-  return lists_decide(num_heads, (int)(((int64_t)q_len + kBlk - 1) / kBlk), (int)(((int64_t)k_len + kBlk - 1) / kBlk), k_len - q_len, causal);
+  return lists_decide(num_heads, (int)(((int64_t)q_len + kBlk - 1) / kBlk), (int)(((int64_t)k_len + kBlk - 1) / kBlk), k_len - q_len, causal) != 0;
 }

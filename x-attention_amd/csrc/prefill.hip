@@ -103,7 +103,7 @@ extern "C" int xattn_prefill_fwd(const void* q, const void* k, const void* v, vo
   if (rc != XATTN_OK) return rc;
   return block_sparse_impl(q, k, v, out, sel.col_idx, sel.col_cnt, l.nkb, l.nqb, 0, num_heads, num_kv_heads, q_len,
                            k_len, head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n,
-                           o_stride_h, o_stride_n, 0, l.nqb, causal, softmax_scale, stream, may_cut ? &plan : nullptr, !sel.plan, queue, sel.totals);
+                           o_stride_h, o_stride_n, 0, l.nqb, causal, softmax_scale, stream, may_cut ? &plan : nullptr, !sel.plan, queue, sel.totals, true);
 }
 
 extern "C" int xattn_estimate_fwd(const void* q, const void* k, void* block_sums, uint8_t* mask, void* workspace,
