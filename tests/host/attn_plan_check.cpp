@@ -71,5 +71,15 @@ int main() {
                 cut_lists, whole, faults);
     bad += faults != 0;
   }
+  // every piece of a list is added once, in order, and no other is read
+  for (int pieces = 1; pieces <= kMostPieces; ++pieces) {
+    int a = -1, b = -1, added = 0, faults = 0;
+    read_ahead(
+        pieces, a, b, [&](int& x, int s) { faults += s < 0 || s >= pieces, x = s; },
+        [&](int& x) { faults += x != added++, x = -1; });
+    faults += added != pieces;
+    std::printf("%d pieces combined, faults %d\n", pieces, faults);
+    bad += faults != 0;
+  }
   return bad ? 1 : 0;
 }

@@ -172,3 +172,39 @@ def test_lists_stay_whole_on_a_full_gpu():
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert torch.equal(full.float(), whole) and torch.equal(listed.float(), whole)
     assert torch.equal(Xattention_prefill(q, k, v, 8, threshold=taus, chunk_size=128), cut)
+
+
+# Lists of so many pieces of 16 blocks (below 48 key blocks, of 8), all of them and the one noted last alone; 64 rows per
+# wavefront from 192 key blocks on
+@pytest.mark.parametrize("cut,q_len,k_len,heads,kv_heads", [
+    (4, 128, 128 * 32, 2, 1), (3, 200, 128 * 23, 4, 2), (3, 1, 128 * 48, 2, 1), (4, 64, 128 * 64, 4, 1), (5, 128, 128 * 79, 4, 1),
+    (5, 300, 128 * 37 - 5, 4, 1), (7, 100, 128 * 111, 2, 2), (13, 257, 128 * 207, 2, 1), (15, 130, 128 * 239, 2, 1),
+    (16, 130, 128 * 256, 2, 1),
+])
+@pytest.mark.parametrize("only_last", [False, True])
+def test_nothing_but_the_pieces_of_a_list_is_combined(cut, q_len, k_len, heads, kv_heads, only_last):
+    """Whatever the workspace, and the memory behind it, held."""
+    from xattn.src import hip_backend as hb
+
+    q, k, v = _inputs(q_len, k_len, heads, kv_heads, cut)
+    nq, nk = (q_len + 127) // 128, (k_len + 127) // 128
+    assert cut == -(-nk // (16 if nk >= 48 else 8))
+    cnt = torch.full((heads, nq), 1 if only_last else nk, dtype=torch.int32, device="cuda")
+    cnt[-1, -1] = nk
+    idx = torch.arange(nk, dtype=torch.int32, device="cuda").expand(heads, nq, nk).contiguous()
+    need = hb.lib().xattn_block_sparse_workspace_bytes(heads, q_len, k_len, nq, nq)
+    assert need > cut * 66560                                     # some list is cut
+    outs = []
+    for fill in (0, 0xFF):                                        # zeros; NaN in every float
+        ws = torch.full((need + (16 << 16),), fill, dtype=torch.uint8, device="cuda")
+        out = torch.empty(1, q_len, heads, 128, dtype=torch.bfloat16, device="cuda")
+        hb.check(hb.lib().xattn_block_sparse_fwd_ws(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), ws.data_ptr(), need, idx.data_ptr(), cnt.data_ptr(), nk, nq, 0,
+            heads, kv_heads, q_len, k_len, 128, q.stride(1), q.stride(2), k.stride(1), k.stride(2), v.stride(1), v.stride(2),
+            out.stride(2), out.stride(1), 0, -1, 0, 128 ** -0.5, torch.cuda.current_stream().cuda_stream), "fwd_ws")
+        outs.append(out.transpose(1, 2).float())
+    assert torch.isfinite(outs[1]).all()
+    assert torch.equal(outs[0], outs[1])
+    want = _swept_whole(q, k, v, idx, cnt, False)
+    bound = 2.0 ** -8 * (v.float().abs().amax() + want.abs())      # as above
+    assert ((outs[1] - want).abs() <= bound).all()

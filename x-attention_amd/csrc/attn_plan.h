@@ -155,6 +155,27 @@ __host__ __device__ inline int cut_at(uint32_t w) { return (int)(w >> 18); }
 __host__ __device__ inline int cut_pieces(uint32_t w) { return (int)(w >> 14 & 15) + 1; }
 __host__ __device__ inline int cut_length(uint32_t w) { return (int)(w & 16383); }
 
+// Pieces 0 .. pieces - 1 of a list, each read while the one before it is added: request(x, s) has piece s on its way to x, one
+// of a and b.  None beyond the last is requested.
+template <typename X, typename R, typename A>
+__host__ __device__ __forceinline__ void read_ahead(int pieces, X& a, X& b, R request, A add) {
+  request(a, 0);
+  int s = 0;
+  for (; s + 2 < pieces; s += 2) {
+    request(b, s + 1);
+    add(a);
+    request(a, s + 2);
+    add(b);
+  }
+  if (s + 1 < pieces) {
+    request(b, s + 1);
+    add(a);
+    add(b);
+  } else {
+    add(a);
+  }
+}
+
 // Notes the lists of q-block qb, `total` blocks in all, by a whole wavefront: count(h) is the length of head h's where it
 // is longer than min_piece, unit0 + h * unit_step its place; reserve(n), called by one lane, gives the place of its n pieces.
 template <typename F, typename R>

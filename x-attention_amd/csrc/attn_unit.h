@@ -310,7 +310,8 @@ __device__ __forceinline__ void store_partial(float* part, int wave, int lane, i
 }
 // The pieces' results combined into the registers of a finished sweep, in the order of the list.  One workgroup reads up to
 // 16 x 66 KiB here while the others may be done: a piece's 16 KiB per wavefront are requested while the one before it is added
-// up (each load behind the last one's sum: 160 us for 16 pieces).  Loads past the last piece arrive as zeros.
+// up (each load behind the last one's sum: 160 us for 16 pieces).  A piece's place is the loads' scalar offset, which the
+// buffer's bounds check does not see: only pieces of the list are named, and nothing else is added, not even times 0.
 __device__ __forceinline__ void load_partials(float* part, int pieces, int wave, int lane, int r, int hh, f32x16 (&oacc)[4], float& l_run) {
   const __amdgpu_buffer_rsrc_t res = __builtin_amdgcn_make_buffer_rsrc((void*)part, 0, pieces * kPartFloats * 4, 0x00020000);
   const int at = (128 * 128 + wave * 32 + r) * 4, from = (wave * 16 * 64 + lane) * 16;
@@ -332,29 +333,23 @@ __device__ __forceinline__ void load_partials(float* part, int pieces, int wave,
   };
   float tops[kMostPieces], m = -INFINITY, l = 0.f;
 #pragma unroll
-  for (int s = 0; s < kMostPieces; ++s) tops[s] = ml(s, 0);
+  for (int s = 0; s < kMostPieces; ++s) tops[s] = ml(s < pieces ? s : pieces - 1, 0);
 #pragma unroll
-  for (int s = 0; s < kMostPieces; ++s) m = fmaxf(m, s < pieces ? tops[s] : -INFINITY);
+  for (int s = 0; s < kMostPieces; ++s) m = fmaxf(m, tops[s]);
   const float safe = m == -INFINITY ? 0.f : m;
-  request(a, 0);
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int v = 0; v < 16; ++v) oacc[i][v] = 0.f;
-  auto add = [&](const Piece& x, bool there) __attribute__((always_inline)) {
-    const float w = there ? fast_exp2(x.m - safe) : 0.f;      // 0 where the piece saw no key of this row
+  auto add = [&](const Piece& x) __attribute__((always_inline)) {
+    const float w = fast_exp2(x.m - safe);      // 0 where the piece saw no key of this row
     l += w * x.l;
 #pragma unroll
     for (int i = 0; i < 16; ++i)
 #pragma unroll
       for (int u = 0; u < 4; ++u) oacc[i >> 2][(i & 3) * 4 + u] += w * x.o[i][u];
   };
-  for (int s = 0; s < pieces; s += 2) {
-    request(b, s + 1);
-    add(a, true);
-    request(a, s + 2);
-    add(b, s + 1 < pieces);
-  }
+  read_ahead(pieces, a, b, request, add);
   l_run = hh == 0 ? l : 0.f;
 }
 
