@@ -95,3 +95,47 @@ def test_scores_that_outgrow_the_reference_maximum(heads, kv_heads, q_len, k_len
     q = (0.2 * q + torch.sign(torch.randn(heads, q_len, 1, generator=g, device="cuda"))[None]).bfloat16()
     blocks = torch.ones(heads, (q_len + 127) // 128, (k_len + 127) // 128, dtype=torch.bool, device="cuda")
     _check(block_sparse_attention(q, k, v, causal=causal), _reference(q, k, v, blocks, causal), v)
+
+
+def _error(got, q, k, v):
+    """Relative error (2-norm) against attention without lists or causality in 64 bits."""
+    off = norm = 0.0
+    group = q.shape[1] // k.shape[1]
+    for h in range(q.shape[1]):
+        s = q[0, h].double() @ k[0, h // group].double().t() * 128 ** -0.5
+        want = s.softmax(-1) @ v[0, h // group].double()
+        off += (got[0, h].double() - want).square().sum().item()
+        norm += want.square().sum().item()
+    return (off / norm) ** 0.5
+
+
+def test_error_is_no_larger_than_with_32_rows():
+    """Correlated tokens without causality: 1536 units have 64 rows, the 512 of the first heads alone 32."""
+    from xattn.src.Xattention import block_sparse_attention
+    from xattn.synthetic import WORKLOADS, make_inputs
+
+    q, k, v = make_inputs(WORKLOADS[4], device="cuda", seed=6, L=8192)
+    heads = slice(0, 8)
+    rows64 = block_sparse_attention(q, k, v, causal=False)[:, heads]
+    q, k, v = (x[:, heads].contiguous() for x in (q, k, v))
+    rows32 = block_sparse_attention(q, k, v, causal=False)
+    assert not torch.equal(rows64, rows32)
+    # what rounding the result to bf16 costs is the same for both; 1 % is left for chance
+    assert _error(rows64, q, k, v) <= 1.01 * _error(rows32, q, k, v)
+
+
+def test_values_of_the_whole_range():
+    """Probabilities are at most 2^8 and the first key block's largest is 1: values may be as large and as small as with 32 rows."""
+    from xattn.src.Xattention import block_sparse_attention
+
+    q, k, v = _inputs(1100, 3000, 7)
+    g = torch.Generator(device="cuda").manual_seed(8)
+    level = torch.linspace(8, -8, 94, device="cuda") + 4 * torch.randn(94, generator=g, device="cuda").clamp(-2, 2)
+    k = (0.2 * k + level.repeat_interleave(32)[:3000, None]).bfloat16()       # scores grow by up to 2^260 on the way
+    q = (0.2 * q + torch.sign(torch.randn(HEADS, 1100, 1, generator=g, device="cuda"))[None]).bfloat16()
+    want = block_sparse_attention(q, k, v, causal=False).double()
+    # 16 keys' values of up to 2^(114 + 3) times 2^8 stay finite in a sum of 3000; a product below 2^-126 may vanish, 2^-14 of
+    # a value of 2^-112 for each probability that small
+    for exponent, bound in ((114, 1e-6), (-112, 1e-5)):
+        got = block_sparse_attention(q, k, (v.double() * 2.0 ** exponent).bfloat16(), causal=False).double() * 2.0 ** -exponent
+        assert (got - want).norm() <= bound * want.norm()

@@ -57,9 +57,13 @@ __device__ __forceinline__ u32x4 block_resource(const __bf16* base, uint32_t blo
 }
 
 constexpr int kAhead = 5;
-// A row's reference maximum stands kHeadroom (exp2 domain) above the largest score it was taken from, and is moved once a
-// lane's sum of 32 probabilities is beyond kOutgrown: scores may grow by 2^48 before.
-constexpr float kHeadroom = 24.f, kOutgrown = 0x1p24f;
+// A row's reference maximum is moved once a lane's sum of the 32 probabilities of a step, 16 of each of two rows, is beyond
+// kOutgrown.  So a probability is at most 2^8, as in the 32-row kernel, and where scores grow the largest of a row is brought
+// back to 1, which bf16 holds exactly.  (With the maximum 2^24 above the scores and moved beyond 2^24, most of what redoing
+// steps costs is saved, us 15450 / 15760 for video of 65536, 138500 / 141200 for a field of 119056 - but there the error of the
+// output against 64 bits was 2.10e-3 for 2.05e-3 with 32 rows, 2.02e-3 this way, and values beyond 2^103 overflowed, below
+// 2^-100 lost bits.)
+constexpr float kOutgrown = 0x1p8f;
 constexpr float kNoKey = -3.402823466e+38f;   // reference maximum of a row that has seen no key
 
 // What a sweep keeps in registers: 64 query rows of a wavefront as two groups of 32.
@@ -111,7 +115,7 @@ __device__ __forceinline__ void softmax_slow(SweepState& w, int set, int g, floa
 #pragma unroll
   for (int v = 0; v < 16; ++v) mx = fmaxf(mx, w.s[set][g][v]);
   mx = half_max(mx) * scale_log2;
-  const float m_new = fmaxf(w.m[g], mine ? mx + kHeadroom : -INFINITY);
+  const float m_new = fmaxf(w.m[g], mine ? mx : -INFINITY);
   const float alpha = fast_exp2(w.m[g] - m_new);
   w.m[g] = m_new;
   w.l[g] *= alpha;
@@ -263,9 +267,9 @@ __device__ __forceinline__ void sweep_step(SweepState& w, const bf16x8 (&q)[2][8
   pv(7, 1);
   read_v(7 + kAhead, 1, kVn);
   read_k(7 + kAhead, kKn);
-  // A lane's sum beyond 2^8 (or none at all: -inf against the initial maximum) says that the row has outgrown its reference
-  // maximum.  The scores are still there: the step's softmax is done again.  16 probabilities of at most 2^8 each, as with a
-  // maximum taken first, cost one compare this way instead of 16 maxima and an exchange per row group.
+  // A lane's sum beyond kOutgrown (infinite for the first keys that a row sees, against the initial maximum) says that one of
+  // its two rows may have outgrown its reference maximum; which, each row's 16 tell.  The scores are still there: the step's
+  // softmax is done again.  That costs one compare instead of 16 maxima and an exchange per row group.
   __builtin_amdgcn_sched_barrier(0);
   uint64_t outgrown = __ballot(!(psum[0] + psum[1] <= kOutgrown));
   asm volatile("" : "+s"(outgrown));
@@ -468,7 +472,7 @@ __global__ __launch_bounds__(128, 1) void block_sparse_fwd64_kernel(AttnParams) 
 #pragma unroll
         for (int v = 0; v < 16; ++v) mx = fmaxf(mx, w.s[0][g][v]);
         mx = half_max(mx);
-        w.m[g] = mx > kNoKey ? mx * p.scale_log2 + kHeadroom : kNoKey;
+        w.m[g] = mx > kNoKey ? mx * p.scale_log2 : kNoKey;
       }
       aim_k(kb_next);
       sweep_step<0, kU, 0, kH, 0, true, false, true, true, -1, -1>(w, q, lds, la, p.scale_log2, cp);
