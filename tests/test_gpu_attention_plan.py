@@ -174,12 +174,12 @@ def test_lists_stay_whole_on_a_full_gpu():
     assert torch.equal(Xattention_prefill(q, k, v, 8, threshold=taus, chunk_size=128), cut)
 
 
-# Lists of so many pieces of 16 blocks (below 48 key blocks, of 8), all of them and the one noted last alone; 64 rows per
-# wavefront from 192 key blocks on
+# Lists of so many pieces of 16 blocks (below 48 key blocks, of 8), all of them (or, of more than 341 units, the last q-block's) and
+# the one noted last alone; 64 rows per wavefront where there are as many queries as keys
 @pytest.mark.parametrize("cut,q_len,k_len,heads,kv_heads", [
     (4, 128, 128 * 32, 2, 1), (3, 200, 128 * 23, 4, 2), (3, 1, 128 * 48, 2, 1), (4, 64, 128 * 64, 4, 1), (5, 128, 128 * 79, 4, 1),
     (5, 300, 128 * 37 - 5, 4, 1), (7, 100, 128 * 111, 2, 2), (13, 257, 128 * 207, 2, 1), (15, 130, 128 * 239, 2, 1),
-    (16, 130, 128 * 256, 2, 1),
+    (16, 130, 128 * 256, 2, 1), (3, 2939, 2939, 24, 8), (5, 8300, 8300, 8, 2), (13, 26400, 26400, 3, 1),
 ])
 @pytest.mark.parametrize("only_last", [False, True])
 def test_nothing_but_the_pieces_of_a_list_is_combined(cut, q_len, k_len, heads, kv_heads, only_last):

@@ -1,4 +1,4 @@
-"""GPU: the operator's attention from a work queue (64 rows per wavefront, more than 1024 units or 256 on a cache) against a
+"""GPU: the operator's attention from a work queue (64 rows per wavefront, more than 1024 units) against a
 workgroup for each unit and piece, over the same lists."""
 import pytest
 import torch

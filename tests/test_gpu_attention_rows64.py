@@ -1,5 +1,5 @@
-"""GPU: the attention kernel of 64 query rows per wavefront (no causality and more than 512 units, 16384 cached tokens, or the
-later q-blocks of 49152 tokens and more) against plain fp32 attention."""
+"""GPU: the attention kernel of 64 query rows per wavefront (no causality and more than 512 units or 192 key blocks, or q-blocks
+of long lists of prompts of 3584 units and more) against plain fp32 attention; on a long cache calls have the 32-row kernel."""
 import pytest
 import torch
 
@@ -41,7 +41,7 @@ def _check(out, want, v):
 
 
 @pytest.mark.parametrize("heads,kv_heads,q_len,k_len,causal", [(72, 8, 1100, 333, False), (72, 8, 1090, 33, False), (8, 2, 1, 16385, True), (8, 8, 300, 32896, True), (6, 2, 257, 33000, True),
-    (1, 1, 49100, 49100, True)])
+    (1, 1, 49100, 49100, True), (56, 8, 8300, 8300, True), (56, 8, 8250, 8953, True), (2, 1, 24460, 24460, False)])
 def test_dense(heads, kv_heads, q_len, k_len, causal):
     from xattn.src.Xattention import block_sparse_attention
 
@@ -50,11 +50,13 @@ def test_dense(heads, kv_heads, q_len, k_len, causal):
     _check(block_sparse_attention(q, k, v, causal=causal), _reference(q, k, v, blocks, causal), v)
 
 
-# lists of no, one, two, three and many blocks; more than the 64 entries that are fetched at a time; token strides of a
-# projection's output; a cache, where lists are cut
+# lists of no, one, two, three and many blocks; more than the 64 entries that are fetched at a time, cut (8 heads; of many, but
+# for the last q-block's, not); token strides of a projection's output; a cache
 @pytest.mark.parametrize("heads,kv_heads,q_len,k_len,causal,keep", [
     (72, 8, 1100, 1100, False, 0.4),
     (72, 8, 1030, 9300, False, 0.5),
+    (8, 2, 9300, 9300, False, 0.95),
+    (56, 8, 8300, 8300, True, 0.95),
     (8, 2, 515, 32900, True, 0.3),
     (32, 8, 600, 32769, True, 0.02),
 ])
@@ -82,7 +84,7 @@ def test_lists(heads, kv_heads, q_len, k_len, causal, keep):
     _check(block_sparse_attention(q, k, v, idx, cnt, causal=causal), want, v)
 
 
-@pytest.mark.parametrize("heads,kv_heads,q_len,k_len,causal", [(72, 8, 1100, 1100, False), (8, 2, 260, 32900, True)])
+@pytest.mark.parametrize("heads,kv_heads,q_len,k_len,causal", [(72, 8, 1100, 1100, False), (8, 2, 260, 32900, True), (56, 8, 8300, 8300, True)])
 def test_scores_that_outgrow_the_reference_maximum(heads, kv_heads, q_len, k_len, causal):
     """The sweep starts at the end of a list: scores grow by up to 2^260 on the way, by 32-key steps of any order."""
     from xattn.src.Xattention import block_sparse_attention
@@ -128,14 +130,31 @@ def test_values_of_the_whole_range():
     """Probabilities are at most 2^8 and the first key block's largest is 1: values may be as large and as small as with 32 rows."""
     from xattn.src.Xattention import block_sparse_attention
 
-    q, k, v = _inputs(1100, 3000, 7)
+    q, k, v = _inputs(1100, 2100, 7)
     g = torch.Generator(device="cuda").manual_seed(8)
-    level = torch.linspace(8, -8, 94, device="cuda") + 4 * torch.randn(94, generator=g, device="cuda").clamp(-2, 2)
-    k = (0.2 * k + level.repeat_interleave(32)[:3000, None]).bfloat16()       # scores grow by up to 2^260 on the way
-    q = (0.2 * q + torch.sign(torch.randn(HEADS, 1100, 1, generator=g, device="cuda"))[None]).bfloat16()
+    level = torch.linspace(8, -8, 66, device="cuda") + 4 * torch.randn(66, generator=g, device="cuda").clamp(-2, 2)
+    k = (0.2 * k + level.repeat_interleave(32)[:2100, None]).bfloat16()       # scores grow, row by row more or less, on the way
+    q = (0.2 * q + torch.randn(HEADS, 1100, 1, generator=g, device="cuda")[None]).bfloat16()
     want = block_sparse_attention(q, k, v, causal=False).double()
-    # 16 keys' values of up to 2^(114 + 3) times 2^8 stay finite in a sum of 3000; a product below 2^-126 may vanish, 2^-14 of
+    # 16 keys' values of up to 2^(114 + 3) times 2^8 stay finite in a sum of 2100; a product below 2^-126 may vanish, 2^-14 of
     # a value of 2^-112 for each probability that small
     for exponent, bound in ((114, 1e-6), (-112, 1e-5)):
         got = block_sparse_attention(q, k, (v.double() * 2.0 ** exponent).bfloat16(), causal=False).double() * 2.0 ** -exponent
         assert (got - want).norm() <= bound * want.norm()
+
+
+def test_chunks_on_a_long_cache_have_the_32_row_kernel():
+    """Whole lists: of a cache of which they name the last 12000 tokens the others make no difference, not in the last bit."""
+    from helpers import lists_from_mask
+    from test_gpu_attention_plan import _swept_whole
+
+    heads, kv_heads, q_len, k_len, skip = 8, 2, 515, 32900, 160
+    for causal in (True, False):
+        q, k, v = _inputs(q_len, k_len, 9, heads, kv_heads)
+        nq, nk = (q_len + 127) // 128, (k_len + 127) // 128
+        blocks = torch.rand(heads, nq, nk, generator=torch.Generator(device="cuda").manual_seed(10), device="cuda") < 0.3
+        blocks[:, :, :skip] = False
+        idx, cnt = lists_from_mask(blocks)
+        whole = _swept_whole(q, k, v, idx, cnt, causal)
+        tail = slice(skip * 128, None)
+        assert torch.equal(whole, _swept_whole(q, k[:, :, tail], v[:, :, tail], (idx - skip).clamp_min(0), cnt, causal))

@@ -15,8 +15,7 @@
 // while this one waits for its first tiles: lists of 1, 2, 3, 8, 32 blocks 6.0, 7.0, 8.4, 16.3, 53 us per unit and CU,
 // against 4.8, 6.4, 8.0, 17.0, 58 - a workgroup per unit.  With a queue (attn_unit.h) workgroups stay and go from unit to unit,
 // whose queries and first keys are requested before the results of the last one leave; 0.8 us lie between two units.  Whole
-// calls, ms, without / with: 131072 tokens 13.45 / 12.85, video of 65536 16.84 / 15.88, a field of 119056 141.7 / 137.8, 2048 on
-// 63488 0.456 / 0.434.
+// calls, ms, without / with: 131072 tokens 13.45 / 12.85, video of 65536 16.84 / 15.88, a field of 119056 141.7 / 137.8.
 #pragma once
 #include <type_traits>
 

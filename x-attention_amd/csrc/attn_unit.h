@@ -125,9 +125,8 @@ __device__ __forceinline__ bool find_unit(const AttnParams& p, int id, Unit& u) 
 __device__ __forceinline__ int64_t unit_slot(const AttnParams& p, const Unit& u) { return (int64_t)u.head * p.idx_rows + (u.qb - p.idx_row0); }
 
 // The work queue.  Workgroups of a launch are dealt to the XCDs in turn, one XCD's are never another's, and a workgroup keeps
-// its place until its stores are acknowledged.  So XCDs with like numbers of workgroups ended far apart (2048 tokens on 63488
-// 506 to 615 us, where heads differ; video of 65536 14.5 to 16.0 ms, where only clocks do), and a tenth of the places stood
-// empty.  With a queue as many workgroups are launched as fit.
+// its place until its stores are acknowledged.  So XCDs with like numbers of workgroups ended far apart (video of 65536 14.5 to
+// 16.0 ms, where only clocks differ), and a tenth of the places stood empty.  With a queue as many workgroups are launched as fit.
 // Workgroup b starts with id b and goes on with those of its queue, b % 32: ids that leave the same rest, which its XCD has
 // anyway.  (An answer takes 1 to 2 us, and a counter gives four in a us: with one per XCD the wait was 4 us of a short list's 15.)
 // queue[32 c]: what queue c has handed out beyond the ids that its workgroups start with.

@@ -71,18 +71,19 @@ using namespace xattn;
 // First q-block that the kernel of 64 rows per wavefront takes; those before it are the 32-row kernel's.  It depends on the
 // whole problem and the q-block alone, so results do not depend on how a problem is spread over launches.
 // 64 rows are for long lists: mostly without causality, and where q-blocks see many blocks.  Whole calls, us, all q-blocks
-// with 32 / 64 rows: field 4000 243 / 228, 21000 5580 / 5036; video 65536 18100 / 15700; 2048 on 63488 269, 421, 739 /
-// 257, 402, 704; 500 on 60000 126, 173, 239 / 118, 181, 231, on 20000 85, 106, 109 / 87, 98, 103; text of three seeds (short
-// lists, short, long) of 32768 tokens 559, 568, 2028 / 584, 594, 1906, 16384 259, 268, 641 / 281, 283, 620 - nothing tells
-// them apart ahead of the call, and the short ones lose what the long ones gain.
-// Few units leave CUs to a single workgroup, where four wavefronts finish a list sooner than two: 1000 tokens 29.9 / 33.1,
-// 500 on 8700 25.2 / 27.6.
+// with 32 / 64 rows: field 4000 243 / 228, 21000 5580 / 5036, 30000 with 2 heads 1042 / 927; video 65536 18100 / 15700; text of
+// three seeds (short lists, short, long) of 32768 tokens 559, 568, 2028 / 584, 594, 1906, 16384 259, 268, 641 / 281, 283, 620 -
+// nothing tells them apart ahead of the call, and the short ones lose what the long ones gain.
+// Few units leave CUs to a single workgroup, where four wavefronts finish a list sooner than two: 1000 tokens 29.9 / 33.1.
+// On a cache lists are cut, and each piece starts with 32 keys that say little about the others: rows outgrow their reference
+// maxima often.  2048 on 63488, three seeds, 477, 264, 422 / 475, 297, 456, and the error against 64 bits is up to 1.5 % larger.
 // The first q-blocks of a long prompt see few blocks and keep short lists.  They are a launch of their own behind the others',
 // so they are few: with the line at 128 blocks instead of 16 the units next to it, of 300 us, ended the first launch alone
 // (131072 tokens with long lists 13.56 ms for 13.28).
 static int first_rows64(int H, int nqb, int nkb, int kv_off, int causal) {
+  if (nkb >= 2 * nqb || kv_off >= 128 * kBlk) return nqb;
   if (!causal) return (int64_t)H * nqb > 512 || nkb >= 192 ? 0 : nqb;
-  if (nkb < 384 && kv_off < 128 * kBlk) return nqb;
+  if (nkb < 384) return nqb;
   const int64_t query = 15 * kBlk - (int64_t)kv_off;             // the first that sees 16 blocks
   const int64_t qb = query <= 0 ? 0 : query / kBlk;
   return qb < nqb ? (int)qb : nqb;
@@ -104,14 +105,14 @@ static int lists_decide(int H, int nqb, int nkb, int kv_off, int causal) {
   return nkb < 384 ? kFrom8Alike : units < 24576 ? kFrom24 : kFrom8;
 }
 
-// Whether the 64-row kernel has a work queue: where units, or the pieces of a chunk's, go several times through the places
-// (us without / with: 2048 on 63488 716 / 648, 1000 on 30000 221 / 214; but 500 on 60000, 128 units, 181 / 195; a field of
-// 4000, 768 like units, 229 / 235: dealt by the launch, the second round's find CUs of their own).
+// Whether the 64-row kernel has a work queue: where units go several times through the places (us without / with: video of
+// 65536 16840 / 15880; but a field of 4000, 768 like units, 229 / 235: dealt by the launch, the second round's find CUs of
+// their own).
 bool xattn::attention_queued(int num_heads, int q_len, int k_len, int causal) {
   const int nqb = (int)(((int64_t)q_len + kBlk - 1) / kBlk), nkb = (int)(((int64_t)k_len + kBlk - 1) / kBlk);
   const int64_t units = (int64_t)num_heads * nqb;
-  return (first_rows64(num_heads, nqb, nkb, k_len - q_len, causal) < nqb || lists_decide(num_heads, nqb, nkb, k_len - q_len, causal)) &&
-         (units > 1024 || (units >= 256 && nkb >= 2 * nqb));
+  return units > 1024 &&
+         (first_rows64(num_heads, nqb, nkb, k_len - q_len, causal) < nqb || lists_decide(num_heads, nqb, nkb, k_len - q_len, causal));
 }
 
 template <bool kHasList, bool kPlanned>
