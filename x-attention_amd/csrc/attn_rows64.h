@@ -1,7 +1,7 @@
 // Block-sparse attention with 64 query rows per wavefront, for long lists (first_rows64 has the rule).
 //
-// One workgroup of two wavefronts per (head, q-block), two workgroups per CU: each wavefront has a SIMD to itself, 424 of its
-// 512 registers, and nothing but its own instruction order to keep the matrix pipe busy while it exponentiates.  So a sweep
+// One workgroup of two wavefronts per (head, q-block), two workgroups per CU: each wavefront has a SIMD to itself, 424 to 465
+// of its 512 registers, and nothing but its own instruction order to keep the matrix pipe busy while it exponentiates.  So a sweep
 // is a software pipeline of steps of 32 keys: beside the scores of the next step and the output of the last one - 16 MFMAs
 // each, alternating - the 32 exponentials of this step's scores are dealt out between the MFMAs, with the fragment reads of
 // five pairs of MFMAs ahead and the copies of the tiles (global -> LDS) of the next 64 keys.
@@ -56,12 +56,12 @@ __device__ __forceinline__ u32x4 block_resource(const __bf16* base, uint32_t blo
 }
 
 constexpr int kAhead = 5;
-// A row's reference maximum is moved once a lane's sum of the 32 probabilities of a step, 16 of each of two rows, is beyond
+// Rows' reference maxima are moved once a lane's sum of the 32 probabilities of a step, 16 of each of two rows, is beyond
 // kOutgrown.  So a probability is at most 2^8, as in the 32-row kernel, and where scores grow the largest of a row is brought
-// back to 1, which bf16 holds exactly.  (With the maximum 2^24 above the scores and moved beyond 2^24, most of what redoing
-// steps costs is saved, us 15450 / 15760 for video of 65536, 138500 / 141200 for a field of 119056 - but there the error of the
-// output against 64 bits was 2.10e-3 for 2.05e-3 with 32 rows, 2.02e-3 this way, and values beyond 2^103 overflowed, below
-// 2^-100 lost bits.)
+// back to 1, which bf16 holds exactly.  (Maxima 2^24 above the scores, moved beyond 2^24, are hardly ever moved and save up to
+// 2 % - field of 8000 tokens 757 / 745 us, 60000 35210 / 35370, video of 65536 15530 / 15480 - but the error of the field's output
+// against 64 bits is then 2.10e-3, with 32 rows 2.05e-3, this way 2.03e-3; values from 2^104 on overflow, below 2^-100 they lose
+// bits.)
 constexpr float kOutgrown = 0x1p8f;
 constexpr float kNoKey = -3.402823466e+38f;   // reference maximum of a row that has seen no key
 
@@ -105,16 +105,15 @@ __device__ __forceinline__ bf16x8 join(const i16x4& a, const i16x4& b) {
   return __builtin_bit_cast(bf16x8, x);
 }
 
-// Online softmax in the exp2 domain of the scores of a step, row group g, with the reference maximum brought up to date
-// where a lane's row asks for it.
-__device__ __forceinline__ void softmax_slow(SweepState& w, int set, int g, float scale_log2, bool outgrown, float& psum) {
-  const uint64_t b = __ballot(outgrown), rows = b | b >> 32;
-  const bool mine = (rows >> (threadIdx.x & 31)) & 1;
+// Online softmax in the exp2 domain of the scores of a step, row group g, with the reference maxima of all its rows brought up
+// to date (of none but those that have outgrown theirs, the others are soon the cause of another such step: us that way /
+// this way, field 4000 271 / 257, 8000 775 / 757, video 18000 1320 / 1294, 65536 15720 / 15530).
+__device__ __forceinline__ void softmax_slow(SweepState& w, int set, int g, float scale_log2, float& psum) {
   float mx = -INFINITY;
 #pragma unroll
   for (int v = 0; v < 16; ++v) mx = fmaxf(mx, w.s[set][g][v]);
   mx = half_max(mx) * scale_log2;
-  const float m_new = fmaxf(w.m[g], mine ? mx : -INFINITY);
+  const float m_new = fmaxf(w.m[g], mx);
   const float alpha = fast_exp2(w.m[g] - m_new);
   w.m[g] = m_new;
   w.l[g] *= alpha;
@@ -282,7 +281,7 @@ __device__ __forceinline__ void sweep_step(SweepState& w, const bf16x8 (&q)[2][8
     for (int g = 0; g < 2; ++g) {
       if (!__any(!(psum[g] <= kOutgrown))) continue;
       asm volatile("" : "+v"(w.s[kSet][g]));     // (or its maxima are taken ahead of the branch)
-      softmax_slow(w, kSet, g, scale_log2, !(psum[g] <= kOutgrown), psum[g]);
+      softmax_slow(w, kSet, g, scale_log2, psum[g]);
     }
     settle();
   }
