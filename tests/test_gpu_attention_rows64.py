@@ -158,3 +158,19 @@ def test_chunks_on_a_long_cache_have_the_32_row_kernel():
         whole = _swept_whole(q, k, v, idx, cnt, causal)
         tail = slice(skip * 128, None)
         assert torch.equal(whole, _swept_whole(q, k[:, :, tail], v[:, :, tail], (idx - skip).clamp_min(0), cnt, causal))
+
+
+def test_long_prompts_of_few_heads_have_the_32_row_kernel():
+    """Whole lists: the first 19968 tokens of 49300 have the output that they have by themselves, to the last bit."""
+    from helpers import lists_from_mask
+    from test_gpu_attention_plan import _swept_whole
+
+    heads, kv_heads, q_len, nq, cut = 4, 1, 49300, 386, 156
+    q, k, v = _inputs(q_len, q_len, 11, heads, kv_heads)
+    blocks = torch.rand(heads, nq, nq, generator=torch.Generator(device="cuda").manual_seed(12), device="cuda") < 0.05
+    blocks &= torch.ones(nq, nq, dtype=torch.bool, device="cuda").tril()
+    blocks[:, :, 0] = True
+    idx, cnt = lists_from_mask(blocks)
+    whole = _swept_whole(q, k, v, idx, cnt, True)
+    q, k, v = (x[:, :, :cut * 128].contiguous() for x in (q, k, v))
+    assert torch.equal(whole[:, :, :cut * 128], _swept_whole(q, k, v, idx[:, :cut, :cut].contiguous(), cnt[:, :cut].contiguous(), True))

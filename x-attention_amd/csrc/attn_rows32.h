@@ -1,4 +1,5 @@
-// Block-sparse attention with 32 query rows per wavefront, where lists may be short or units few (first_rows64 has the rule).
+// Block-sparse attention with 32 query rows per wavefront, where lists may be short or units few (all_rows64 and lists_decide
+// have the rule).
 //
 // Work decomposition: one workgroup (4 wavefronts) per (head, q-block); each
 // wavefront owns 32 query rows.  Scores are produced transposed,

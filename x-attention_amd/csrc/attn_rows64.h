@@ -1,4 +1,4 @@
-// Block-sparse attention with 64 query rows per wavefront, for long lists (first_rows64 has the rule).
+// Block-sparse attention with 64 query rows per wavefront, for long lists (all_rows64 and lists_decide have the rule).
 //
 // One workgroup of two wavefronts per (head, q-block), two workgroups per CU: each wavefront has a SIMD to itself, 424 to 465
 // of its 512 registers, and nothing but its own instruction order to keep the matrix pipe busy while it exponentiates.  So a sweep

@@ -68,25 +68,16 @@ __global__ __launch_bounds__(64) void ready_kernel(AttnParams p, int32_t* queue,
 
 using namespace xattn;
 
-// First q-block that the kernel of 64 rows per wavefront takes; those before it are the 32-row kernel's.  It depends on the
-// whole problem and the q-block alone, so results do not depend on how a problem is spread over launches.
-// 64 rows are for long lists: mostly without causality, and where q-blocks see many blocks.  Whole calls, us, all q-blocks
-// with 32 / 64 rows: field 4000 243 / 228, 21000 5580 / 5036, 30000 with 2 heads 1042 / 927; video 65536 18100 / 15700; text of
-// three seeds (short lists, short, long) of 32768 tokens 559, 568, 2028 / 584, 594, 1906, 16384 259, 268, 641 / 281, 283, 620 -
-// nothing tells them apart ahead of the call, and the short ones lose what the long ones gain.
-// Few units leave CUs to a single workgroup, where four wavefronts finish a list sooner than two: 1000 tokens 29.9 / 33.1.
+// Whether the kernel of 64 rows per wavefront takes all q-blocks (else lists_decide).  It depends on the whole problem alone, so
+// results do not depend on how a problem is spread over launches.
+// 64 rows are for long lists: mostly without causality.  Whole calls, us, 32 / 64 rows: field 4000 276 / 257, 8000 832 / 757, 20000
+// 4855 / 4344, 30000 with 2 heads 1037 / 921.
+// Few units leave CUs to a single workgroup, where four wavefronts finish a list sooner than two: 1000 tokens 29.9 / 33.1, long
+// text with few heads (64 rows from the 15th q-block on) 65536 with 4 241 / 273, 50000 with 8 257 / 299, 131072 with 2 339 / 367.
 // On a cache lists are cut, and each piece starts with 32 keys that say little about the others: rows outgrow their reference
 // maxima often.  2048 on 63488, three seeds, 477, 264, 422 / 475, 297, 456, and the error against 64 bits is up to 1.5 % larger.
-// The first q-blocks of a long prompt see few blocks and keep short lists.  They are a launch of their own behind the others',
-// so they are few: with the line at 128 blocks instead of 16 the units next to it, of 300 us, ended the first launch alone
-// (131072 tokens with long lists 13.56 ms for 13.28).
-static int first_rows64(int H, int nqb, int nkb, int kv_off, int causal) {
-  if (nkb >= 2 * nqb || kv_off >= 128 * kBlk) return nqb;
-  if (!causal) return (int64_t)H * nqb > 512 || nkb >= 192 ? 0 : nqb;
-  if (nkb < 384) return nqb;
-  const int64_t query = 15 * kBlk - (int64_t)kv_off;             // the first that sees 16 blocks
-  const int64_t qb = query <= 0 ? 0 : query / kBlk;
-  return qb < nqb ? (int)qb : nqb;
+static bool all_rows64(int H, int nqb, int nkb, int causal) {
+  return !causal && nkb < 2 * nqb && ((int64_t)H * nqb > 512 || nkb >= 192);
 }
 
 // Of prompts by themselves, with units enough that a second launch costs little (3 us without a q-block of its own, 50 for
@@ -111,15 +102,13 @@ static int lists_decide(int H, int nqb, int nkb, int kv_off, int causal) {
 bool xattn::attention_queued(int num_heads, int q_len, int k_len, int causal) {
   const int nqb = (int)(((int64_t)q_len + kBlk - 1) / kBlk), nkb = (int)(((int64_t)k_len + kBlk - 1) / kBlk);
   const int64_t units = (int64_t)num_heads * nqb;
-  return units > 1024 &&
-         (first_rows64(num_heads, nqb, nkb, k_len - q_len, causal) < nqb || lists_decide(num_heads, nqb, nkb, k_len - q_len, causal));
+  return units > 1024 && (all_rows64(num_heads, nqb, nkb, causal) || lists_decide(num_heads, nqb, nkb, k_len - q_len, causal));
 }
 
 template <bool kHasList, bool kPlanned>
 static int launch_fwd(AttnParams p, int64_t extra, hipStream_t s) {
   p.lists_decide = lists_decide(p.H, p.nqb, p.nkb, p.kv_off, p.causal);
-  const int begin = p.qb_begin, end = p.qb_end, first64 = first_rows64(p.H, p.nqb, p.nkb, p.kv_off, p.causal);
-  const int split = p.lists_decide ? begin : first64, end32 = p.lists_decide || end < split ? end : split;
+  const bool all64 = all_rows64(p.H, p.nqb, p.nkb, p.causal);
   const int cus = resident_workgroups();
   if (cus <= 0) return XATTN_ERR_LAUNCH;
   const int places = 2 * cus / kQueues * kQueues;
@@ -129,14 +118,11 @@ static int launch_fwd(AttnParams p, int64_t extra, hipStream_t s) {
     if (!queued || places == 0 || ids <= places) p.queue = nullptr;
     return dim3((unsigned)(p.queue ? places : ids));
   };
-  p.qb_begin = begin > split ? begin : split;
-  if (p.qb_begin < end) {
+  if (all64 || p.lists_decide) {
     hipLaunchKernelGGL((block_sparse_fwd64_kernel<kHasList, kPlanned>), grid(true), dim3(128), 0, s, p);
     if (hipGetLastError() != hipSuccess) return XATTN_ERR_LAUNCH;
   }
-  p.qb_begin = begin;
-  p.qb_end = end32;
-  if (begin < p.qb_end) {
+  if (!all64) {
     hipLaunchKernelGGL((block_sparse_fwd_kernel<kHasList, kPlanned>), grid(false), dim3(256), 0, s, p);
     if (hipGetLastError() != hipSuccess) return XATTN_ERR_LAUNCH;
   }
