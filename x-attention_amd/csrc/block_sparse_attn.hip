@@ -85,15 +85,18 @@ static bool all_rows64(int H, int nqb, int nkb, int causal) {
 // blocks: 64 rows where lists have 8 blocks on average and the longest is less than twice that, as of video - unlike lists would
 // give two launches with an end of their own each, and one long list takes twice as long (32768 tokens, few long heads, with a
 // line on the total alone: 1340 us with 32 rows / 1640).  Whole calls, us, 32 rows / by the lists: video of 18000 tokens
-// 1425 / 1274, of 32000 4180 / 3700; text of 32768, which stays with 32 rows, 535 / 533.  Longer ones outlast such ends: from 24 blocks
-// on average, of 24576 units and more from 8.  Text of six seeds, 32 rows / 64 from the 15th q-block on / from 24 / from 8: 131072
-// tokens 7386, 4741, 4787, 24708, 4735, 13665 / 6879, 4740, 4820, 21438, 4723, 11915 / 7279, 4657, 4731, 22069, 4644, 12431 / 7051, 4690,
-// 4790, 21534, 4634, 12029; 80000 3368, 2103, 2151, 9773, 2079, 5904 / 3173, 2154, 2194, 8326, 2124, 5136 / 3313, 2091, 2149, 8818,
-// 2064, 5667 / 3358, 2086, 2143, 8379, 2061, 5281; 50000, the first seed, 1671 / 1578 / 1645 / 1731.
+// 1425 / 1274, of 32000 4180 / 3700; text of 32768, which stays with 32 rows, 535 / 533.  Longer ones outlast such ends: from 8
+// blocks on average - but below 18432 units, where a prompt in which some heads keep a few long lists would lose, from 24.  Text of
+// six seeds with 32 heads, 32 rows / from 24 / from 8: 131072 tokens 7443, 4753, 4846, 25027, 4709, 13684 / 7358, 4731, 4833, 22174,
+// 4685, 12697 / 7149, 4728, 4831, 21813, 4684, 12264; 100000 4838, 3063, 3132, 15030, 3027, 8746 / 4768, 3045, 3115, 13150, 3012,
+// 7945 / 4629, 3040, 3116, 12974, 3006, 7729; 80000 (20000 units) 3315, 2107, 2167, 9887, 2089, 5921 / 3316, 2107, 2158, 8947, 2075,
+// 5748 / 3330, 2098, 2155, 8404, 2069, 5316; 64000 (16000) 2320, 1452, 1504, 6522, 1433, 3981 / 2312, 1456, 1493, 5846, 1424, 3973 /
+// 2369, 1445, 1490, 5509, 1426, 3621; 50000 1666, 1033, 1059, 4172, 1017, 2653 / 1630, 1028, 1053, 3852, 1021, 2524 / 1726, 1038, 1068,
+// 3517, 1014, 2442.
 static int lists_decide(int H, int nqb, int nkb, int kv_off, int causal) {
   const int64_t units = (int64_t)H * nqb;
   if (!causal || kv_off >= 128 * kBlk || units < 3584) return kNot;
-  return nkb < 384 ? kFrom8Alike : units < 24576 ? kFrom24 : kFrom8;
+  return nkb < 384 ? kFrom8Alike : units < 18432 ? kFrom24 : kFrom8;
 }
 
 // Whether the 64-row kernel has a work queue: where units go several times through the places (us without / with: video of
