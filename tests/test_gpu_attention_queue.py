@@ -90,3 +90,24 @@ def test_lists_choose_the_kernel_the_same_way_by_every_path(q_len, heads, kv_hea
             vals = v[0, h * kv_heads // heads, keys].float()
             want = p @ vals
             assert ((got[0, h, rows].float() - want).abs() <= 2.0 ** -8 * (vals.abs().amax() + want.abs())).all()
+
+
+def test_a_window_that_fits_at_once_has_no_queue():
+    """512 units or fewer: nothing is made ready ahead of the launch, which needs no workspace; the output is the whole launch's."""
+    from xattn.src import hip_backend as hb
+    from xattn.src.Xattention import block_sparse_attention
+
+    q_len, heads, kv_heads = 17000, 32, 8
+    g = torch.Generator(device="cuda").manual_seed(13)
+    rnd = lambda h: torch.randn(1, h, q_len, 128, generator=g, device="cuda").bfloat16()
+    q, k, v = rnd(heads), rnd(kv_heads), rnd(kv_heads)
+    nq = (q_len + 127) // 128
+    size = lambda n: hb.lib().xattn_block_sparse_workspace_bytes(heads, q_len, q_len, nq, n)
+    assert size(1) == size(16) == 0 and size(17) == size(nq) == 4096 + (128 * nq + 255) // 256 * 256
+    idx = torch.arange(nq, dtype=torch.int32, device="cuda").expand(heads, nq, nq).contiguous()
+    cnt = (torch.arange(nq, dtype=torch.int32, device="cuda") + 1).expand(heads, nq).contiguous()      # from 8 on: 64 rows
+    whole = block_sparse_attention(q, k, v, idx, cnt)
+    parts = torch.empty(1, q_len, heads, 128, dtype=torch.bfloat16, device="cuda")
+    for a in range(0, nq, 16):
+        block_sparse_attention(q, k, v, idx, cnt, out=parts, q_blocks=(a, min(nq, a + 16)))
+    assert torch.equal(parts.transpose(1, 2), whole)

@@ -108,25 +108,16 @@ bool xattn::attention_queued(int num_heads, int q_len, int k_len, int causal) {
   return units > 1024 && (all_rows64(num_heads, nqb, nkb, causal) || lists_decide(num_heads, nqb, nkb, k_len - q_len, causal));
 }
 
+// `ids` units and pieces; with a queue, `places` workgroups of the 64-row kernel.
 template <bool kHasList, bool kPlanned>
-static int launch_fwd(AttnParams p, int64_t extra, hipStream_t s) {
-  p.lists_decide = lists_decide(p.H, p.nqb, p.nkb, p.kv_off, p.causal);
+static int launch_fwd(const AttnParams& p, int64_t ids, int places, hipStream_t s) {
   const bool all64 = all_rows64(p.H, p.nqb, p.nkb, p.causal);
-  const int cus = resident_workgroups();
-  if (cus <= 0) return XATTN_ERR_LAUNCH;
-  const int places = 2 * cus / kQueues * kQueues;
-  auto grid = [&](bool queued) {
-    p.unit_ids = (int)grid_for(p.H, p.Hkv, p.qb_end - p.qb_begin);
-    const int64_t ids = p.unit_ids + extra;
-    if (!queued || places == 0 || ids <= places) p.queue = nullptr;
-    return dim3((unsigned)(p.queue ? places : ids));
-  };
   if (all64 || p.lists_decide) {
-    hipLaunchKernelGGL((block_sparse_fwd64_kernel<kHasList, kPlanned>), grid(true), dim3(128), 0, s, p);
+    hipLaunchKernelGGL((block_sparse_fwd64_kernel<kHasList, kPlanned>), dim3((unsigned)(p.queue ? places : ids)), dim3(128), 0, s, p);
     if (hipGetLastError() != hipSuccess) return XATTN_ERR_LAUNCH;
   }
   if (!all64) {
-    hipLaunchKernelGGL((block_sparse_fwd_kernel<kHasList, kPlanned>), grid(false), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((block_sparse_fwd_kernel<kHasList, kPlanned>), dim3((unsigned)ids), dim3(256), 0, s, p);
     if (hipGetLastError() != hipSuccess) return XATTN_ERR_LAUNCH;
   }
   return XATTN_OK;
@@ -182,22 +173,26 @@ int xattn::block_sparse_impl(const void* q, const void* k, const void* v, void* 
   p.qb_begin = q_block_begin;
   p.qb_end = q_block_end;
   p.shape = dispatch_shape(p.H, p.Hkv);
+  p.plan = plan ? *plan : AttnPlan{};
+  p.lists_decide = lists_decide(p.H, p.nqb, p.nkb, p.kv_off, p.causal);
   const int64_t grid = grid_for(p.H, p.Hkv, q_block_end - q_block_begin);
-  if (grid > 0x7fffffff) return XATTN_ERR_SHAPE;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  p.plan = AttnPlan{};
+  const int64_t ids = grid + (plan ? ((int64_t)plan_pieces(plan->shape, q_block_end - q_block_begin) + 7) / 8 * 8 : 0);
+  if (ids > 0x7fffffff) return XATTN_ERR_SHAPE;
+  p.unit_ids = (int)grid;
+  const int cus = resident_workgroups();
+  if (cus <= 0) return XATTN_ERR_LAUNCH;
+  const int places = 2 * cus / kQueues * kQueues;
+  if (places == 0) queue = nullptr;
   p.queue = queue;
   p.totals = totals;
+  hipStream_t s = static_cast<hipStream_t>(stream);
   if (!ready && (queue || totals))
     hipLaunchKernelGGL(ready_kernel, dim3((unsigned)(q_block_end - q_block_begin)), dim3(64), 0, s, p, queue, totals);
   if (plan) {
-    p.plan = *plan;
-    const int64_t most = ((int64_t)plan_pieces(plan->shape, q_block_end - q_block_begin) + 7) / 8 * 8;
-    if (grid + most > 0x7fffffff) return XATTN_ERR_SHAPE;
     if (note) hipLaunchKernelGGL(note_lists_kernel, dim3(1), dim3(1024), 0, s, p);
-    return col_idx ? launch_fwd<true, true>(p, most, s) : launch_fwd<false, true>(p, most, s);
+    return col_idx ? launch_fwd<true, true>(p, ids, places, s) : launch_fwd<false, true>(p, ids, places, s);
   }
-  return col_idx ? launch_fwd<true, false>(p, 0, s) : launch_fwd<false, false>(p, 0, s);
+  return col_idx ? launch_fwd<true, false>(p, ids, places, s) : launch_fwd<false, false>(p, ids, places, s);
 }
 
 extern "C" int xattn_block_sparse_fwd(const void* q, const void* k, const void* v, void* out,
@@ -223,13 +218,20 @@ PlanShape shape_of(int num_heads, int q_len, int k_len, bool listed) {
 }
 }  // namespace
 
+// Whether a launch over some of the q-blocks has the problem's queue, and totals: not where its units fit the places at once, for
+// which another launch ahead, and memory, cost more than they give (us per window of text, with / without: 4 q-blocks of 32 heads
+// 25.7 / 18.8, 16 29.4 / 27.4; video, 16 of 28 heads 165.5 / 162).
+static bool launch_queued(int num_heads, int q_len, int k_len, int q_blocks, int causal) {
+  return (int64_t)num_heads * q_blocks > 512 && attention_queued(num_heads, q_len, k_len, causal);
+}
+
 static size_t totals_bytes(int64_t rows, bool asked) { return asked ? plan_round((size_t)rows * 128) : 0; }
 
 extern "C" size_t xattn_block_sparse_workspace_bytes(int num_heads, int q_len, int k_len, int idx_rows, int q_blocks) {
   if (num_heads <= 0 || q_len <= 0 || k_len <= 0 || idx_rows < 0 || q_blocks <= 0) return 0;
   const int64_t rows = idx_rows ? idx_rows : ((int64_t)q_len + kBlk - 1) / kBlk;
   const size_t plan = plan_bytes(shape_of(num_heads, q_len, k_len, idx_rows != 0), num_heads * rows, q_blocks);
-  const bool queued = attention_queued(num_heads, q_len, k_len, 0) || attention_queued(num_heads, q_len, k_len, 1);
+  const bool queued = launch_queued(num_heads, q_len, k_len, q_blocks, 0) || launch_queued(num_heads, q_len, k_len, q_blocks, 1);
   return plan_round(plan) + (queued ? kQueueBytes + totals_bytes(rows, idx_rows != 0 && attention_asks_totals(num_heads, q_len, k_len, 1)) : 0);
 }
 
@@ -256,7 +258,7 @@ extern "C" int xattn_block_sparse_fwd_ws(const void* q, const void* k, const voi
   }
   uint32_t* totals = nullptr;
   if (workspace && workspace_bytes >= need && need >= kQueueBytes && !(reinterpret_cast<uintptr_t>(workspace) & 255) &&
-      attention_queued(num_heads, q_len, k_len, causal)) {
+      launch_queued(num_heads, q_len, k_len, q_blocks, causal)) {
     const bool asked = col_idx && attention_asks_totals(num_heads, q_len, k_len, 1);
     char* at = static_cast<char*>(workspace) + need - kQueueBytes - totals_bytes(idx_rows, asked);
     queue = reinterpret_cast<int32_t*>(at);
