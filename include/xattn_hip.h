@@ -222,9 +222,10 @@ int xattn_block_sparse_fwd(const void* q, const void* k, const void* v, void* ou
  * `workspace`: xattn_block_sparse_workspace_bytes() bytes for the q_blocks =
  * q_block_end - q_block_begin q-blocks of the launch, 256-byte aligned,
  * contents undefined on entry and on return, at most 200 MB; 0 bytes (null
- * allowed) means that nothing is cut and each unit has a workgroup of its own.  Some
- * of the larger problems that are not cut have a work queue there, 4 KiB, and 128
- * bytes per q-block row of the lists.  Without lists (col_idx null; idx_rows = 0 for the size) the
+ * allowed) means that nothing is cut and each unit has a workgroup of its own.  Launches
+ * of more than 512 units have, in some of the larger problems, a work queue there, 4 KiB,
+ * and 128 bytes per q-block row of the lists (where nothing is cut, the call does without
+ * both if the workspace is null or smaller).  Without lists (col_idx null; idx_rows = 0 for the size) the
  * visible blocks of a unit are its list.  Where a list is cut depends on the
  * lengths of its q-block's lists over all heads, num_heads, q_len and k_len
  * only, so results do not depend on how q-blocks are spread over launches; a

@@ -7,7 +7,8 @@
 
 namespace xattn {
 
-// Which q-blocks are the 64-row kernel's: those of its launch; those whose lists have so many blocks on average (and are much alike).
+// Which q-blocks are the 64-row kernel's: all of a problem's or none; those whose lists have so many blocks on average (and are much
+// alike).
 enum ListsDecide { kNot, kFrom8, kFrom8Alike, kFrom24 };
 
 struct AttnParams {
@@ -112,7 +113,7 @@ __device__ __forceinline__ bool find_place(const AttnParams& p, int id, Unit& u)
       u.head = unit / p.idx_rows;
       u.qb = unit - u.head * p.idx_rows + p.idx_row0;
       u.kvh = u.head / p.shape.group;
-      return u.qb >= p.qb_begin && u.qb < p.qb_end;      // (q-blocks may be shared among two launches)
+      return true;
     }
   }
   return map_workgroup(id - u.skip, p.shape, p.qb_begin, p.qb_end, &u.head, &u.qb, &u.kvh);
