@@ -82,3 +82,33 @@ def test_whole_operator_replays_from_a_graph():
         want = Xattention_prefill(q, k, v, 8, **kw)
         torch.cuda.synchronize()
         assert torch.equal(got, want), i
+
+
+@pytest.mark.parametrize("listed", [False, True])
+def test_attention_from_a_work_queue_replays_from_a_graph(listed):
+    """3612 units: the queue and the q-blocks' totals, which a call leaves used up, are made ready within the graph."""
+    from xattn.src.Xattention import Xattention_prefill, block_sparse_attention, estimate_and_select
+    from xattn.synthetic import WORKLOADS, make_inputs
+
+    w, L, nq = WORKLOADS[3], 16500, 129
+    kw = dict(threshold=0.9, chunk_size=128)
+    q, k, v = make_inputs(w, device="cuda", seed=3, L=L)
+    r = estimate_and_select(q, k, 16, 0.9, 128, want_mask=False, want_sums=False)
+    idx, cnt = r["col_idx"][:, :nq].contiguous(), r["col_cnt"][:, :nq].contiguous()
+    call = lambda: block_sparse_attention(q, k, v, idx, cnt) if listed else Xattention_prefill(q, k, v, 16, **kw)
+    call()                                                                    # warm-up outside the capture
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    for i in range(4):
+        for x, new in zip((q, k, v), make_inputs(w, device="cuda", seed=10 + i, L=L)):
+            x.copy_(new)                                                      # eager work between replays
+        if listed and i:
+            cnt.copy_((cnt * (0.5 + 0.2 * i)).int().clamp(1, nq))             # other lists, of which other kernels take care
+        graph.replay()
+        torch.cuda.synchronize()
+        got = out.clone()
+        want = call()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want), i
