@@ -39,8 +39,8 @@ PEAK_HBM_GBS = 8000.0
 # this process): the summary of those runs for the headline workload is kept as a table under profiles/ and read here.
 TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "bench_headline_hbm_traffic.md")
 HEADLINE = "cfg2_llama8b_L131072_gqa32x8_S16"
-KERNEL_SOURCES = ("attn_plan.h", "attn_rows32.h", "attn_rows64.h", "attn_tiles.h", "attn_unit.h", "block_sparse_attn.hip",
-                  "estimate.hip", "estimate_params.h", "select_row.h", "select_blocks.hip", "xattn_common.h")
+KERNEL_SOURCES = ("attn_plan.h", "attn_rows32.h", "attn_rows64.h", "attn_tiles.h", "attn_unit.h", "block_sparse_attn.hip", "estimate.h",
+                  "estimate.hip", "estimate_params.h", "estimate_small.h", "select_row.h", "select_blocks.hip", "xattn_common.h")
 
 
 def kernel_source_hash():
@@ -53,10 +53,10 @@ def kernel_source_hash():
     return h.hexdigest()[:16]
 
 
-def measured_traffic_bytes(kernel_prefix):
-    """Scaled total bytes of the first table row of the traffic summary whose kernel name starts with
-    ``kernel_prefix`` (last column, in GB); None when the summary or the row is missing, or when the summary
-    was taken at other kernel sources than the ones in the tree."""
+def measured_traffic_bytes(*kernel_prefixes):
+    """Scaled total bytes of the traffic summary's rows for these kernels, added up: of each the first row whose
+    kernel name starts with the prefix (last column, in GB).  None when the summary or a row is missing, or when
+    the summary was taken at other kernel sources than the ones in the tree."""
     try:
         with open(TRAFFIC_SUMMARY) as f:
             text = f.read()
@@ -64,14 +64,15 @@ def measured_traffic_bytes(kernel_prefix):
         return None
     if ("kernel sources sha256/16: " + kernel_source_hash()) not in text:
         return None
-    for line in text.splitlines():
-        cells = [c.strip().strip("`") for c in line.strip().strip("|").split("|")]
-        if len(cells) >= 6 and cells[0].startswith(kernel_prefix):
-            try:
-                return float(cells[-1]) * 1e9
-            except ValueError:
-                return None
-    return None
+    rows = [[c.strip().strip("`") for c in line.strip().strip("|").split("|")] for line in text.splitlines()]
+    total = 0.0
+    for prefix in kernel_prefixes:
+        row = next((cells for cells in rows if len(cells) >= 6 and cells[0].startswith(prefix)), None)
+        try:
+            total += float(row[-1]) * 1e9
+        except (TypeError, ValueError):
+            return None
+    return total
 
 
 def _ms(a, b):
@@ -320,7 +321,7 @@ def summarize(w, L, tau, chunk, m, headline_traffic=False):
         "kernel": "block_sparse_fwd64_kernel<true>, block_sparse_fwd_kernel<true>", "bound": "mfma", "achieved": round(att_tf, 1),
         "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s", "frac": round(att_tf / PEAK_BF16_TFLOPS, 4), "ms": round(t_att, 3),
         "flop": fb["f_sparse"],
-        "traffic": measured_traffic_bytes("xattn::block_sparse_fwd64_kernel<true") if headline_traffic else None,
+        "traffic": measured_traffic_bytes("xattn::block_sparse_fwd64_kernel<true", "xattn::block_sparse_fwd_kernel<true") if headline_traffic else None,
     }
     sel_gbs = fb["pass_bytes"] / (t_sel * 1e-3) / 1e9
     rl_sel = {
@@ -511,7 +512,7 @@ def main():
         "timing": {"warmup_steps": args.warmup, "timed_steps": args.steps, "value_is": "mean of the timed steps",
                    "dense_warmup": args.dense_warmup, "dense_timed": args.dense_steps, "dense_fa_ms_is": "median",
                    "stages": "estimate_ms = the estimator's MFMA pass (estimate_gemm_kernel), select_ms = its normalisation "
-                             "fused with the block selection (estimate_select_kernel), sparse_attn_ms = block_sparse_fwd64_kernel"},
+                             "fused with the block selection (estimate_select_kernel), sparse_attn_ms = block_sparse_fwd64_kernel and block_sparse_fwd_kernel"},
         "kernel_sources_sha256_16": kernel_source_hash(),
     }
     result.update({key: val for key, val in head.items() if not key.startswith("roofline_")})
