@@ -75,7 +75,8 @@ using namespace xattn;
 // Few units leave CUs to a single workgroup, where four wavefronts finish a list sooner than two: 1000 tokens 29.9 / 33.1, long
 // text with few heads (64 rows from the 15th q-block on) 65536 with 4 241 / 273, 50000 with 8 257 / 299, 131072 with 2 339 / 367.
 // On a cache lists are cut, and each piece starts with 32 keys that say little about the others: rows outgrow their reference
-// maxima often.  2048 on 63488, three seeds, 477, 264, 422 / 475, 297, 456, and the error against 64 bits is up to 1.5 % larger.
+// maxima often, and nothing is gained over all.  Text of three seeds, 2048 on 63488 479, 271, 429 / 455, 274, 420 (with a queue),
+// 500 on 60000 189, 132, 180 / 191, 129, 187, 8000 on 100000 665, 490, 495 / 659, 511, 517.
 static bool all_rows64(int H, int nqb, int nkb, int causal) {
   return !causal && nkb < 2 * nqb && ((int64_t)H * nqb > 512 || nkb >= 192);
 }
