@@ -8,7 +8,7 @@
 //
 // Bound: MFMA, under the power limit.  Why 64 rows: a K or V fragment read from LDS serves twice the MFMAs that it serves in
 // the 32-row kernel, whose LDS and vector pipes are shared by two wavefronts per SIMD.  Dense causal attention of 32768
-// tokens, 32/8 heads, both on one box: 7.7 ms -> 6.9 ms (1.14 -> 1.27 PFLOP/s; MFMA busy 63 -> 76 % of SIMD cycles at 1.72 ->
+// tokens, 32/8 heads, both on one box: 7.5 ms -> 6.65 ms (1.17 -> 1.32 PFLOP/s; MFMA busy 63 -> 75 % of SIMD cycles at 1.72 ->
 // 1.6 GHz).  A wave tile of 64 x 128 takes 5150 clk for 4096 of MFMA; without fragment reads and copies 4590, without what
 // keeps the order of instructions (pin, settle, MFMAs as assembly) 6200 - the compiler bunches the exponentials.
 // A unit costs 3.9 us per CU beside its tiles, against 3.1 with 32 rows, where the other workgroup's wavefronts use the SIMD
