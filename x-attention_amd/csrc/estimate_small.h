@@ -4,10 +4,10 @@
 // A workgroup of four wavefronts takes 128 keys (one softmax tile) x 32 * MT query rows; wavefront w computes the scores
 // of keys 32w .. 32w+31 against all rows.  Where a head has fewer rows than that, the rows of several heads of the KV
 // group share a tile (`pack`), so that every key is read once per group.  64-deep slabs of both operands go straight to
-// a ring of NS LDS stages (buffer loads that write LDS), NS - 1 steps ahead of their use, one barrier per step.
+// a ring of NS LDS stages (buffer loads that write LDS), NS - 1 steps ahead of their use (NS with MT 1), one barrier per step.
 //
-// Bound: with at most a tile per CU the time is the chain of 2 * stride steps - 0.17 to 0.25 us each, the barrier and the
-// dependent MFMAs of a step, against 1.1 us of a 256x256 step.  With more tiles per CU two or three workgroups share it
+// Bound: with at most a tile per CU the time is the chain of 2 * stride steps - 0.16 us each with MT 1, the barrier, the
+// dependent MFMAs and the fragment reads of a step, against 1.1 us of a 256x256 step.  With more tiles per CU two or three workgroups share it
 // and the copies into LDS (about 50 bytes per clock and CU) and the fragment reads (1 + MT per MT MFMAs) are the limit:
 // 0.7 (MT 2) and 0.8 (MT 4) of the flop rate of the large tiles.  More stages help only while a CU has one workgroup;
 // beyond that a third workgroup is worth more than a third stage.
@@ -18,7 +18,7 @@
 namespace xattn {
 
 // kSelect (MT 1, rows that see no key past the first softmax tile): normalisation and selection follow in the same
-// workgroup, which has whole rows.  A 1000-token prompt then takes one launch of 13.6 us instead of two of 10.6 and 7.0.
+// workgroup, which has whole rows.  A 1000-token prompt then takes one launch of 11.8 us instead of two of 9.2 and 7.0.
 template <int RBS, int MT, int NS, bool kSelect>
 __global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p, SelParams sp) {
   static_assert(!kSelect || MT == 1, "the selection takes a wavefront per query block of 32 rows");
@@ -27,6 +27,8 @@ __global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p, Sel
   constexpr int kStage = (kKeys + kRows) * 128;     // bytes of one 64-deep step
   constexpr int kLoads = 4 + MT;                    // KiB a wavefront copies per step
   constexpr int kPer = (kLoads + 2) / 3;            // ... and in each of the step's first three sub-steps
+  constexpr bool kAhead = MT == 1;
+  constexpr int kPer4 = (kLoads + 3) / 4;           // ... or (kAhead) in each of four
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 31, hh = lane >> 5;
@@ -109,6 +111,58 @@ __global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p, Sel
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[a][v] = 0.f;
   const int swz = (r >> 1) & 7;
+  if (kAhead) {
+    // A step's fragments are read together, a step ahead of its MFMAs: a sub-step is one MFMA of 32 clk, an answer of the LDS
+    // takes four times that, and with fragments read a sub-step ahead every sub-step waited for it (1000 tokens, stride 16, estimate
+    // and selection 13.2 -> 11.8 us; with MT 2, two MFMAs and more workgroups to a CU, no difference).  The barrier of step t: this
+    // wavefront has step t's fragments in registers and its copies of step t + 1 have landed, so behind it step t + 1 may be read and
+    // step t's stage refilled.
+    const int from = live_w ? 0 : 4;
+#pragma unroll
+    for (int t = 0; t < NS; ++t)
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j)
+        if (j >= from) copy_piece(t, j);
+    if (live_w) {
+      bf16x8 fa[2][4], fb[2][4][MT];
+      auto read = [&](int t, int buf) __attribute__((always_inline)) {
+        const char* st = lds + (t % NS) * kStage;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const int ch = ((2 * s + hh) ^ swz) << 4;
+          fa[buf][s] = *reinterpret_cast<const bf16x8*>(st + (wave * 32 + r) * 128 + ch);
+#pragma unroll
+          for (int a = 0; a < MT; ++a) fb[buf][s][a] = *reinterpret_cast<const bf16x8*>(st + 16384 + (a * 32 + r) * 128 + ch);
+        }
+      };
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 1) * kLoads) : "memory");
+      read(0, 0);
+      auto step = [&](int t, int buf) __attribute__((always_inline)) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * kLoads) : "memory");
+        read(t + 1, buf ^ 1);        // (a repeat of old data behind the last step)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+#pragma unroll
+          for (int a = 0; a < MT; ++a) acc[a] = mfma32(fa[buf][s], fb[buf][s][a], acc[a]);
+#pragma unroll
+          for (int j = s * kPer4; j < kLoads && j < (s + 1) * kPer4; ++j) copy_piece(t + NS, j);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+      for (int t = 0; t < steps; t += 2) {      // (steps = 2 S)
+        step(t, 0);
+        step(t + 1, 1);
+      }
+    } else {
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 1) * MT) : "memory");
+      for (int t = 0; t < steps; ++t) {
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 2) * MT) : "memory");
+#pragma unroll
+        for (int j = 4; j < kLoads; ++j) copy_piece(t + NS, j);
+      }
+    }
+  } else
   // A step is four sub-steps of MT MFMAs; the fragments of the next sub-step and the copies of step t + NS - 1 are issued
   // between them.  The barrier sits before the last sub-step's MFMAs: by then this wavefront has read every fragment of
   // step t and its copies of step t + 1 have landed, so behind it step t + 1 may be read and step t's stage refilled.
