@@ -18,6 +18,10 @@
 // four wavefronts combine (max, sum, unnormalised output) of their key ranges in
 // LDS and write one partial result per workgroup; a second small kernel merges
 // the workgroups of a head.
+//
+// Keys and values are loaded "not temporal": 32 query heads on 8 KV heads, caches from memory, 100003 keys 74.9 -> 67.2 us
+// (6.1 TB/s), 20000 21.1 -> 20.0, 9200 14.5 -> 14.1; 32 KV heads, 40000 keys 115 -> 103.  A cache that stays in the memory-side
+// cache from call to call loses nothing (9200 keys 12.4, 20000 18.9 -> 18.0).
 #include <mutex>
 
 #include "lds_limit.h"
@@ -77,7 +81,7 @@ __device__ __forceinline__ void dec_copy(const __bf16* base, int64_t sn, int len
       (void*)(base + (int64_t)t * kDecKeys * sn), 0, (int)((int64_t)rows * sn * 2), 0x00020000);
 #pragma unroll
   for (int i = 0; i < 8; ++i)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(slot + i * 1024), 16, voff[i], 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(slot + i * 1024), 16, voff[i], 0, 0, kLoadNt);
 }
 
 __global__ __launch_bounds__(256, 1) void decode_partial_kernel(DecodeParams p) {
