@@ -51,3 +51,45 @@ def test_projections_of_a_turn(tokens, heads, kv_heads, width, bias):
         if y is not None:
             ref = (x.float() @ weights[0].float().t() + (biases[0].float() if bias else 0.0)).bfloat16()
             assert close(y, ref, 2.0 ** -7 * ref.float().abs())
+
+
+# CUs without a tile pull weights ahead from the fourth to the seventh step on: few tiles and many such CUs, none but one XCD's
+# at work, runs of tiles that end inside a head; then tiles of 192 and 256 tokens, whole and with a remainder, steps odd and even
+@pytest.mark.parametrize("tokens,heads,kv_heads,width", [
+    (40, 1, 1, 4096), (2, 3, 1, 1088), (150, 5, 3, 2048), (500, 28, 4, 1024), (250, 32, 8, 704), (600, 32, 8, 4160),
+    (769, 32, 8, 576), (960, 32, 8, 512), (1025, 32, 8, 640), (1280, 32, 8, 832),
+])
+def test_weights_pulled_ahead_and_large_tiles(tokens, heads, kv_heads, width):
+    test_projections_of_a_turn(tokens, heads, kv_heads, width, True)
+
+
+def test_two_workgroups_per_cu():
+    """2600 tokens of 24 heads: 504 tiles of 128 x 128, but more than 256 of 256 tokens."""
+    from xattn.src import hip_backend as hb
+
+    g = torch.Generator(device="cuda").manual_seed(2600)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    assert hb.lib().xattn_proj_gemm_fits(2600, 448, 24 * 128, 1)
+    weights = [(rnd(h * 128, 448) / 448 ** 0.5).bfloat16() for h in (16, 4, 4)]
+    x, cos, sin = rnd(1, 2600, 448).bfloat16(), torch.ones(1, 2600, 128, device="cuda").bfloat16(), torch.zeros(1, 2600, 128, device="cuda").bfloat16()
+    with torch.no_grad():
+        got = hb.host().project(x, weights[0], None, weights[1], None, weights[2], None, cos, sin, 16, 4)
+        for a, b in zip(got, _reference(x, weights, (None,) * 3, (16, 4, 4), cos, sin)):
+            # one bf16 step where the fp32 sums, in another order, round to the other side (nothing is rotated)
+            assert ((a.float() - b.float()).abs() <= 2.0 ** -7 * b.float().abs() + 1e-5).all() and (a != b).float().mean() < 0.02
+
+
+@pytest.mark.parametrize("tokens,heads,taken", [(1100, 32, True), (1536, 32, True), (1537, 32, False), (640, 64, True)])
+def test_output_of_many_tokens(tokens, heads, taken):
+    from xattn.src import hip_backend as hb
+
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    x = torch.randn(1, tokens, 704, generator=g, device="cuda").bfloat16()
+    w = (torch.randn(heads * 128, 704, generator=g, device="cuda") / 704 ** 0.5).bfloat16()
+    with torch.no_grad():
+        y = hb.host().output(x, w, None)
+    assert (y is not None) == taken
+    if taken:
+        ref = (x.float() @ w.float().t()).bfloat16()
+        # one bf16 step where the fp32 sums, in another order, round to the other side
+        assert ((y.float() - ref.float()).abs() <= 2.0 ** -7 * ref.float().abs() + 1e-5).all() and (y != ref).float().mean() < 0.02

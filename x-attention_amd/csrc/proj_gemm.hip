@@ -1,28 +1,30 @@
 // The projections of an attention layer for turns of up to about a thousand tokens: y = x W^T with rows as long as the
 // hidden state; q, k and v in one launch with the rotation of q and k in its epilogue, or the output projection.
 //
-// Bound: with at most a tile per CU, by how fast one CU fills its LDS - 75 to 80 GB/s whatever the number of stages or
-// CUs at work, half of it W's - so the tile is the largest that still gives most CUs one: 64 x 64 up to 256 tiles, then
-// 64 tokens x 128 features, then 128 x 128, and two workgroups per CU for q, k and v beyond that.  Splitting a
-// step's depth over two groups of wavefronts helps the smallest tile only (17.6 -> 13.3 us at 64 tokens), where the
-// chain of 64 steps is the time.
+// Bound: with at most a tile per CU, by how fast one CU fills its LDS (a CU has 32 KiB of loads in flight, whatever is asked of
+// it: 76 GB/s from memory, 130 from the L2), so the tile is the largest that still gives most CUs one: 64 x 64 up to 256 tiles,
+// then 64 tokens x 128 features, 128 x 128, 192 x 128 and, for q, k and v, 256 x 128.  CUs left over pull the weights into the
+// L2 (pull_weights; q, k, v of 500 tokens, 4096 wide, 192 tiles: 39.6 -> 34 us; 3584 wide, 144 tiles: 36.5 -> 29).  The larger
+// tiles took the place of two 128 x 128 ones per CU (4096 wide, 700 tokens 65 -> 46 us, 1000 72 -> 57, 1280 75 -> 64).
+// Splitting a step's depth over two groups of wavefronts helps the smallest tile only (17.6 -> 13.3 us at 64 tokens), where the
+// chain of 64 steps is the time; on the larger ones, where it would save a third of the LDS reads, it is 1 to 8 % slower.
 //
-// Library products against this kernel, weights from memory, in a captured graph, us.  q, k, v (three launches, and 4 to 5 for
-// the rotation) by tokens:
+// Library products against this kernel, weights from memory, us (the library's in a captured graph).  q, k, v (three launches,
+// and 4 to 5 for the rotation) by tokens:
 //   width, heads      64         200        500        700        1000       1280       1500
-//   1024   8 + 2*8    27 / 7     27 / 7     28 / 9.5   30 / 12.5  30 / 13    33 / 14    34 / 19
-//   2048   32 + 2*8   36 / 14    38 / 16.5  43 / 24    50 / 36    53 / 41    59 / 43    library
-//   3584   28 + 2*4   40 / 19    42 / 23.5  50 / 35    67 / 33    71 / 55    81 / 61    82 / 66
-//   4096   32 + 2*8   46 / 22    48 / 28    63 / 39    75 / 64    87 / 72    100 / 78   library
-//   5120   40 + 2*8   60 / 31    61 / 36    89 / 54    105 / 83   118 / 98   library
-//   8192   64 + 2*8   62 / 45    95 / 65    134 / 134  165 / 144  library
-// Output (features x depth): 1024 x 1024 8.8 / 6.2, 8.4 / 6.1, 8.6 / 6.3, 9.1 / 6.5, 9.0 / 6.6, 9.6 / 7.8, 9.6 / 7.9;
-// 4096 x 4096 14.4 / 19.3, 20.8 / 16.5, 28 / 27, 31 / 33, 39 / 37, library; 3072 x 3072 16 / 18, 17.5 / 14, 21 / 24, 26 / 28,
-// 29.5 / 31.6, 32 / 34; 8192 x 8192 33 / 43, 53 / 52, 81 / 77.  The library's stand within 16 % of this kernel's from 65 tokens on,
-// one way or the other.  Up to 64 there is a single row of tiles, each a chain over the whole depth, which the library splits;
-// so it does where the features are fewer than the depth (2048 x 4096 at 64 / 128 / 200 / 257 tokens 14 / 21, 13 / 20, 14.5 / 16,
-// 21 / 16).  Such a turn is bound by the host's calls, though, and the library's is the dearer one: the whole layer, 4096 wide, on
-// 6000 tokens with the library's output product / this kernel's, 2 tokens 70 / 62, 16 68 / 64, 64 68 / 74.5, 100 68 / 68.
+//   1024   8 + 2*8    27 / 7     27 / 7     28 / 9     30 / 12    30 / 14    33 / 15    34 / 19
+//   2048   32 + 2*8   36 / 11.5  38 / 15    43 / 21    50 / 28    53 / 34    59 / 37    library
+//   3584   28 + 2*4   40 / 16    42 / 20.5  50 / 29    67 / 32    71 / 43    81 / 47    82 / 54
+//   4096   32 + 2*8   46 / 18.5  48 / 24.5  63 / 34    75 / 46    87 / 57    100 / 64   library
+//   5120   40 + 2*8   60 / 25    61 / 34    89 / 49    105 / 60   118 / 74   library
+//   8192   64 + 2*8   62 / 45    95 / 61    134 / 94   165 / 119  library
+// Output (features x depth): 1024 x 1024 8.8 / 6.6, 8.4 / 6.5, 8.6 / 6.7, 9.1 / 6.7, 9.0 / 7.5, 9.6 / 7.9, 9.6 / 8.0;
+// 4096 x 4096 14.4 / 16.3, 20.8 / 17.5, 28 / 28.3, 31 / 32, 39 / 39, 49 / 46, 52 / 51; 3072 x 3072 16 / 13, 17.5 / 12.7,
+// 21 / 18.4, 26 / 23, 29.5 / 26, 32 / 30, 41 / 35; 8192 x 8192 33 / 42, 53 / 51, 81 / 75, 98 / 96.  Up to 64 tokens there is a single
+// row of tiles, each a chain over the whole depth, which the library splits; so it does where the features are fewer than the
+// depth.  Such a turn is bound by the host's calls, though, and the library's is the dearer one: the whole layer, 4096 wide, on
+// 6000 tokens with the library's output product / this kernel's before weights were pulled ahead, 2 tokens 70 / 62, 16 68 / 64,
+// 64 68 / 74.5, 100 68 / 68.
 #include "lds_limit.h"
 #include "rotate.h"
 #include "xattn_hip.h"
@@ -41,6 +43,33 @@ struct ProjParams {
   const __bf16* sin;
   int64_t cos_sn, sin_sn;
 };
+
+// What CUs without a tile do: they pull the weights of their XCD's tiles into its L2, ahead of the tiles.  A CU has at most 32 KiB
+// of loads in flight and gets them back in order, so a tile's fill runs at 32 KiB per latency of the slowest load among them:
+// 76 GB/s where each step's weights come from memory, 130 where they are in the L2.  (Loads by the tile's own CU don't help: they
+// queue with the others.  Nor does the scalar cache, some 27 ns per line.)  Lane g takes line g % lines of every `reps`-th step.
+template <int kN, int kThreads, int kAhead>
+__device__ __forceinline__ void pull_weights(const ProjParams& p, uint32_t mt, uint32_t total, uint32_t per_xcd) {
+  const uint32_t first = (blockIdx.x & 7) * per_xcd;
+  if (first >= total) return;
+  const uint32_t last = (first + per_xcd < total ? first + per_xcd : total) - 1;
+  const uint32_t head0 = first / mt * kN / 128, heads = last / mt * kN / 128 + 1 - head0;
+  const uint32_t lines = heads * 128, lanes = ((gridDim.x >> 3) - per_xcd) * kThreads;
+  const uint32_t g = ((blockIdx.x >> 3) - per_xcd) * kThreads + threadIdx.x, reps = lanes / lines;
+  if (g >= reps * lines) return;
+  int f = (int)(head0 * 128 + g % lines), t3 = 0;
+  if (f >= p.n[0]) { f -= p.n[0]; t3 = 1; }
+  if (t3 == 1 && f >= p.n[1]) { f -= p.n[1]; t3 = 2; }
+  const char* const row = reinterpret_cast<const char*>(p.w[t3] + (int64_t)f * p.w_sn[t3]);
+  const uint32_t steps = (uint32_t)p.K / 64;
+  for (uint32_t t = kAhead + g / lines; t < steps; t += 8 * reps) {
+    uint32_t v[8];
+#pragma unroll
+    for (uint32_t u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const uint32_t*>(row + (int64_t)(t + u * reps < steps ? t + u * reps : t) * 128);
+#pragma unroll
+    for (uint32_t u = 0; u < 8; ++u) asm volatile("" ::"v"(v[u]));
+  }
+}
 
 // Four wavefronts (2 x 2) take 64 * NB features x 64 * MB tokens; 64-deep slabs of both operands go straight to a ring of NS
 // LDS stages, NS - 1 steps ahead of their use, one barrier per step.  KS = 2: four more multiply the second half of each
@@ -64,7 +93,11 @@ __global__ __launch_bounds__(256 * KS, 2) void proj_gemm_kernel(ProjParams p) {
   const uint32_t mt = (uint32_t)(p.M + kM - 1) / kM;
   const uint32_t total = mt * (uint32_t)((p.n[0] + p.n[1] + p.n[2]) / kN), per_xcd = (total + 7) / 8;
   const uint32_t lin = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if ((blockIdx.x >> 3) >= per_xcd || lin >= total) return;
+  if ((blockIdx.x >> 3) >= per_xcd) {
+    pull_weights<kN, 256 * KS, NS - 1>(p, mt, total, per_xcd);
+    return;
+  }
+  if (lin >= total) return;
   int f0 = (int)(lin / mt) * kN, t3 = 0;
   const int m0 = (int)(lin % mt) * kM;
   if (kRope) {
@@ -217,14 +250,20 @@ namespace {
 bool a16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // The tile for `features` features of `tokens` tokens (see the head of the file), or none: the products are large enough
-// for the library.  Past 256 tiles of 128 x 128 only the three products of q, k and v gain from being one launch.
-enum Tile { kNone, k64x64, k128x64, k128x128, k128x128Twice };
+// for the library.  An output product of 256-token tiles would only tie with it (1500 to 2000 tokens, 4096 wide: 54 to 63 us,
+// library 51 to 60), q, k and v are three of its launches.  Token counts that miss 256 tiles by the rounding (2600 tokens of
+// 3072 features: 504 tiles of 128 x 128, 264 of 128 x 256) have two workgroups per CU.
+enum Tile { kNone, k64x64, k128x64, k128x128, k128x192, k128x256, k128x128Twice };
+constexpr unsigned kCUs = 256;
 Tile tile_for(int64_t tokens, int64_t features, bool qkv) {
-  const int64_t m64 = (tokens + 63) / 64, m128 = (tokens + 127) / 128;
-  if (features / 64 * m64 <= 256) return k64x64;
-  if (features / 128 * m64 <= 256) return k128x64;
-  if (features / 128 * m128 <= 256) return k128x128;
-  return qkv && features / 128 * m128 <= 512 ? k128x128Twice : kNone;
+  auto tiles = [&](int n, int m) { return features / n * ((tokens + m - 1) / m); };
+  if (tiles(64, 64) <= kCUs) return k64x64;
+  if (tiles(128, 64) <= kCUs) return k128x64;
+  if (tiles(128, 128) <= kCUs) return k128x128;
+  if (tiles(128, 192) <= kCUs) return k128x192;
+  if (!qkv) return kNone;
+  if (tiles(128, 256) <= kCUs) return k128x256;
+  return tiles(128, 128) <= 2 * kCUs ? k128x128Twice : kNone;
 }
 
 template <int NB, int MB, int NS, int KS, bool kRope>
@@ -233,7 +272,10 @@ int launch(const ProjParams& p, hipStream_t s) {
   static LdsLimit limit;
   if (limit.raise((const void*)proj_gemm_kernel<NB, MB, NS, KS, kRope>) != hipSuccess) return XATTN_ERR_LAUNCH;
   const unsigned tiles = (unsigned)((p.M + 64 * MB - 1) / (64 * MB)) * (unsigned)((p.n[0] + p.n[1] + p.n[2]) / (64 * NB));
-  hipLaunchKernelGGL((proj_gemm_kernel<NB, MB, NS, KS, kRope>), dim3((tiles + 7) / 8 * 8), dim3(256 * KS), kLds, s, p);
+  static_assert(kLds <= 160 * 1024, "LDS of a CU");
+  // one workgroup per CU: the CUs left over pull weights
+  const unsigned grid = kLds > 80 * 1024 && tiles < kCUs ? kCUs : (tiles + 7) / 8 * 8;
+  hipLaunchKernelGGL((proj_gemm_kernel<NB, MB, NS, KS, kRope>), dim3(grid), dim3(256 * KS), kLds, s, p);
   return hipGetLastError() == hipSuccess ? XATTN_OK : XATTN_ERR_LAUNCH;
 }
 
@@ -248,6 +290,8 @@ int run(const ProjParams& p, void* stream) {
     case k64x64: return launch<1, 1, 6, 2, kRope>(p, s);
     case k128x64: return launch<2, 1, 4, 1, kRope>(p, s);
     case k128x128: return launch<2, 2, 4, 1, kRope>(p, s);
+    case k128x192: return launch<2, 3, 4, 1, kRope>(p, s);
+    case k128x256: return launch<2, 4, 3, 1, kRope>(p, s);
     case k128x128Twice: return launch<2, 2, 2, 1, kRope>(p, s);
     default: return XATTN_ERR_SHAPE;
   }
