@@ -26,7 +26,7 @@ struct AttnParams {
   int qb_begin, qb_end;     // q-blocks handled by this launch
   int causal, kv_off;       // kv_off = Lk - Lq
   float scale_log2;         // softmax_scale * log2(e)
-  DispatchShape shape;      // dispatch_shape(H, Hkv), computed on the host
+  DispatchShape shape;      // dispatch_shape of the launch, computed on the host
   AttnPlan plan;            // kPlanned only
   int32_t* queue;           // this launch's work queue (kQueueWords, zero), or null: one workgroup per id
   int unit_ids;             // ids of units, grid_for()

@@ -173,7 +173,7 @@ int xattn::block_sparse_impl(const void* q, const void* k, const void* v, void* 
   p.idx_row0 = idx_row0;
   p.qb_begin = q_block_begin;
   p.qb_end = q_block_end;
-  p.shape = dispatch_shape(p.H, p.Hkv);
+  p.shape = dispatch_shape(p.H, p.Hkv, q_block_end - q_block_begin);
   p.plan = plan ? *plan : AttnPlan{};
   p.lists_decide = lists_decide(p.H, p.nqb, p.nkb, p.kv_off, p.causal);
   const int64_t grid = grid_for(p.H, p.Hkv, q_block_end - q_block_begin);
