@@ -98,3 +98,14 @@ def test_decode_rejects_bad_arguments():
     code = lib.xattn_decode_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), ws.data_ptr(), 16,
                                 32, 8, 64, 128, 128, 64 * 128, 128, 64 * 128, 128, 128, 0.1, None)
     assert code == -7   # XATTN_ERR_WORKSPACE
+
+
+# the last cache loaded with the default policy and the first of those loaded "not temporal" (more than 96 MiB), whose last tile
+# has one key
+@pytest.mark.parametrize("shape", [(32, 8, 24576), (32, 8, 24577), (28, 4, 49153)])
+def test_decode_at_the_line_between_cache_policies(shape):
+    from xattn.src.decode import single_decode_with_kv_cache
+
+    H, Hkv, L = shape
+    q, k, v = _mk(H, Hkv, L, L, spread=3.0)
+    _check(single_decode_with_kv_cache(q.cuda(), k.cuda(), v.cuda(), kv_layout="HND"), O.single_decode_with_kv_cache(q, k, v, kv_layout="HND"))

@@ -19,9 +19,7 @@
 // LDS and write one partial result per workgroup; a second small kernel merges
 // the workgroups of a head.
 //
-// Keys and values are loaded "not temporal": 32 query heads on 8 KV heads, caches from memory, 100003 keys 74.9 -> 67.2 us
-// (6.1 TB/s), 20000 21.1 -> 20.0, 9200 14.5 -> 14.1; 32 KV heads, 40000 keys 115 -> 103.  A cache that stays in the memory-side
-// cache from call to call loses nothing (9200 keys 12.4, 20000 18.9 -> 18.0).
+// Keys and values of large caches are loaded "not temporal" (kNtBytes).
 #include <mutex>
 
 #include "lds_limit.h"
@@ -71,6 +69,7 @@ __device__ __forceinline__ void wait_lgkm0() {
 // One 32-key tile, global -> this wavefront's LDS slot.  Tiles outside
 // [0, n_tiles) are issued with an empty buffer resource: they move no data but
 // keep the count of outstanding loads the same on every iteration.
+template <bool kNt>
 __device__ __forceinline__ void dec_copy(const __bf16* base, int64_t sn, int len, int tile, int n_tiles,
                                          const int (&voff)[8], char* slot) {
   const bool live = tile < n_tiles;
@@ -81,9 +80,10 @@ __device__ __forceinline__ void dec_copy(const __bf16* base, int64_t sn, int len
       (void*)(base + (int64_t)t * kDecKeys * sn), 0, (int)((int64_t)rows * sn * 2), 0x00020000);
 #pragma unroll
   for (int i = 0; i < 8; ++i)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(slot + i * 1024), 16, voff[i], 0, 0, kLoadNt);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(slot + i * 1024), 16, voff[i], 0, 0, kNt ? kLoadNt : 0);
 }
 
+template <bool kNt>
 __global__ __launch_bounds__(256, 1) void decode_partial_kernel(DecodeParams p) {
   extern __shared__ __attribute__((aligned(1024))) char ring_all[];
 
@@ -153,10 +153,10 @@ __global__ __launch_bounds__(256, 1) void decode_partial_kernel(DecodeParams p) 
 
   // load number j of the sequence K_0 V_0 K_1 V_1 ... goes to slot j % 5
   const int t_end = t0 + n;
-  dec_copy(kbase, p.k_sn, p.Lk, t0, t_end, voffK, ring + 0 * kDecTileBytes);
-  dec_copy(vbase, p.v_sn, p.Lk, t0, t_end, voffV, ring + 1 * kDecTileBytes);
-  dec_copy(kbase, p.k_sn, p.Lk, t0 + 1, t_end, voffK, ring + 2 * kDecTileBytes);
-  dec_copy(vbase, p.v_sn, p.Lk, t0 + 1, t_end, voffV, ring + 3 * kDecTileBytes);
+  dec_copy<kNt>(kbase, p.k_sn, p.Lk, t0, t_end, voffK, ring + 0 * kDecTileBytes);
+  dec_copy<kNt>(vbase, p.v_sn, p.Lk, t0, t_end, voffV, ring + 1 * kDecTileBytes);
+  dec_copy<kNt>(kbase, p.k_sn, p.Lk, t0 + 1, t_end, voffK, ring + 2 * kDecTileBytes);
+  dec_copy<kNt>(vbase, p.v_sn, p.Lk, t0 + 1, t_end, voffV, ring + 3 * kDecTileBytes);
 
   int slot = 0;   // slot of K_i
   for (int i = 0; i < n; ++i) {
@@ -166,7 +166,7 @@ __global__ __launch_bounds__(256, 1) void decode_partial_kernel(DecodeParams p) 
     const int s4 = slot + 4 >= kDecSlots ? slot + 4 - kDecSlots : slot + 4;   // freed by V_{i-1}
 
     wait_lgkm0();   // this wavefront's reads of the slot about to be refilled have returned
-    dec_copy(kbase, p.k_sn, p.Lk, tile + 2, t_end, voffK, ring + s4 * kDecTileBytes);
+    dec_copy<kNt>(kbase, p.k_sn, p.Lk, tile + 2, t_end, voffK, ring + s4 * kDecTileBytes);
     wait_vm32();    // K_i landed
 
     f32x16 sacc;
@@ -188,7 +188,7 @@ __global__ __launch_bounds__(256, 1) void decode_partial_kernel(DecodeParams p) 
     }
     // K_i is in registers (the MFMAs above consumed every fragment): its slot takes V_{i+2}
     wait_lgkm0();
-    dec_copy(vbase, p.v_sn, p.Lk, tile + 2, t_end, voffV, Kt);
+    dec_copy<kNt>(vbase, p.v_sn, p.Lk, tile + 2, t_end, voffV, Kt);
 
     float mx = -INFINITY;
 #pragma unroll
@@ -384,6 +384,12 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p) {
   }
 }
 
+// Bytes of keys and values from which they are loaded "not temporal": such a cache does not stay in the memory-side cache (256 MB)
+// beside what else a step reads, and a stream from memory is faster by a sixth (100003 keys of 8 KV heads 75.9 -> 68.0 us, 6.1 TB/s;
+// 40000 34.5 -> 31.7; 70000 of 4 32.7 -> 29.8).  A smaller one may be there still from the call before (two or three in turn,
+// without / with: 82 MB 19.0 / 19.4 us, 38 MB 12.8 / 13.1).
+constexpr int64_t kNtBytes = 96 << 20;
+
 struct DecodeGeometry {
   int n_tiles, tiles_per_wave, ranges_per_head;
 };
@@ -447,10 +453,12 @@ int decode_launch(const void* q, const void* k, const void* v, void* out, void* 
   p.scale_log2 = softmax_scale * kLog2e;
 
   hipStream_t s = static_cast<hipStream_t>(stream);
-  static LdsLimit limit;
-  if (limit.raise(reinterpret_cast<const void*>(decode_partial_kernel)) != hipSuccess) return XATTN_ERR_LAUNCH;
+  static LdsLimit limit[2];
+  const bool nt = (int64_t)num_kv_heads * k_len * kHeadDim * 4 > kNtBytes;
+  const auto kernel = nt ? decode_partial_kernel<true> : decode_partial_kernel<false>;
+  if (limit[nt].raise(reinterpret_cast<const void*>(kernel)) != hipSuccess) return XATTN_ERR_LAUNCH;
   const unsigned grid = (unsigned)(num_kv_heads * (g.ranges_per_head / kDecWaves));
-  hipLaunchKernelGGL(decode_partial_kernel, dim3(grid), dim3(256), kDecLds, s, p);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), kDecLds, s, p);
   hipLaunchKernelGGL(decode_merge_kernel, dim3((unsigned)num_heads), dim3(256), 0, s, p);
   return hipGetLastError() == hipSuccess ? XATTN_OK : XATTN_ERR_LAUNCH;
 }

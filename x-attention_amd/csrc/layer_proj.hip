@@ -6,8 +6,8 @@
 //    rotary pairs d, d + 64 and their neighbours, so that the rotation happens in registers), every load is a full
 //    1 KiB of one row, and 20 of them are in flight per wavefront before the first is used.  The library GEMM with
 //    one row left most of the chip idle: 47 us for the four products of that layer (1.8 TB/s), and the rotation
-//    another 13 launches.  Weights are loaded "not temporal": from memory 4096 x 4096 8.5 -> 7.8 us, 6144 x 4096 11.3 -> 10.8,
-//    10240 x 8192 38.6 -> 36.4.  proj_gemm.hip has the products of more tokens.
+//    another 13 launches.  (Loaded "not temporal" the weights come 4 to 8 % faster from memory, but a layer whose weights are in the
+//    memory-side cache still is 1 to 3 % slower.)  proj_gemm.hip has the products of more tokens.
 //  rope_kernel: the rotation of q and k of many tokens in place, one read and one write of both.  The reference's
 //    expression is ten elementwise kernels over them.
 //
@@ -65,7 +65,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemvParams p) {
       xv[buf][c] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xres, off, 0, 0));
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        wv[buf][c][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wres[i], off, 0, kLoadNt));
+        wv[buf][c][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wres[i], off, 0, 0));
     }
   };
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
