@@ -1,0 +1,42 @@
+"""GPU: attention of few units, where a unit is two workgroups' of 64 rows and half of a tile's keys is a wavefront's."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# up to 128 units of at most 16 key blocks (the last shapes of each kind are the first beyond): rows and keys that end in the
+# first half, at its edge and in the second, keys ahead of the queries, no causality, rows that see no key of a tile's second half
+@pytest.mark.parametrize("q_len,k_len,heads,kv_heads,causal", [
+    (1, 1, 1, 1, True), (63, 63, 4, 2, True), (64, 64, 4, 4, True), (65, 65, 3, 1, True), (128, 128, 32, 8, True), (129, 129, 28, 4, False),
+    (500, 500, 32, 8, True), (512, 512, 32, 32, True), (513, 513, 32, 8, True), (300, 1500, 28, 4, True), (70, 2048, 8, 2, False),
+    (70, 2049, 8, 2, True), (2048, 2048, 8, 1, True), (200, 137, 4, 2, True),
+])
+def test_few_units(q_len, k_len, heads, kv_heads, causal):
+    from xattn.src.Xattention import block_sparse_attention
+
+    g = torch.Generator(device="cuda").manual_seed(q_len + k_len)
+    rnd = lambda h, n: torch.randn(1, h, n, 128, generator=g, device="cuda")
+    q, k, v = (2 * rnd(heads, q_len)).bfloat16(), rnd(kv_heads, k_len).bfloat16(), rnd(kv_heads, k_len).bfloat16()
+    nq, nk = -(-q_len // 128), -(-k_len // 128)
+    keep = torch.rand(heads, nq, nk, generator=g, device="cuda") < 0.6
+    last = torch.arange(nq, device="cuda").add(1).mul(128).clamp(max=q_len) - 1 + k_len - q_len if causal else torch.full((nq,), k_len - 1, device="cuda")
+    keep &= torch.arange(nk, device="cuda")[None, :] * 128 <= last[:, None]
+    keep[:, :, 0] |= last >= 0
+    keep[0, 0] = False                                                # an empty list gives zeros
+    cnt = keep.sum(-1).int()
+    idx = torch.where(keep, torch.arange(nk, device="cuda").expand_as(keep), nk).sort(-1).values.clamp(max=nk - 1).int()
+    got = block_sparse_attention(q, k, v, idx.contiguous(), cnt.contiguous(), causal=causal).float()
+    pos = torch.arange(q_len, device="cuda") + k_len - q_len
+    seen = keep.repeat_interleave(128, 1)[:, :q_len].repeat_interleave(128, 2)[:, :, :k_len]
+    if causal:
+        seen = seen & (torch.arange(k_len, device="cuda")[None, :] <= pos[:, None])
+    kf, vf = (x[0].float().repeat_interleave(heads // kv_heads, 0) for x in (k, v))
+    s = (q[0].float() @ kf.transpose(1, 2).contiguous() * 128 ** -0.5).masked_fill(~seen, float("-inf"))
+    p = torch.nan_to_num(torch.softmax(s, -1), nan=0.0)
+    want = p @ vf
+    # probabilities are rounded to bf16 (2^-9 relative), and the result once more
+    bound = 2.0 ** -8 * (p @ vf.abs() + want.abs()) + 1e-6
+    assert ((got[0] - want).abs() <= bound).all()
+    again = block_sparse_attention(q, k, v, idx.contiguous(), cnt.contiguous(), causal=causal).float()
+    assert torch.equal(got, again)

@@ -26,33 +26,34 @@
 
 namespace xattn {
 
-// S^T = K_j Q^T : lane owns query row r, key rows 8g + 4hh + t of each 32-row tile
-__device__ __forceinline__ void qk_tile(const char* Ks, const int (&kaddr)[8], const bf16x8 (&qreg)[8], f32x16 (&sacc)[4]) {
+// S^T = K_j Q^T on NT x 32 keys: lane owns query row r, key rows 8g + 4hh + t of each 32-row tile
+template <int NT>
+__device__ __forceinline__ void qk_tile(const char* Ks, const int (&kaddr)[8], const bf16x8 (&qreg)[8], f32x16 (&sacc)[NT]) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < NT; ++i)
 #pragma unroll
     for (int v = 0; v < 16; ++v) sacc[i][v] = 0.f;
-  bf16x8 kf[2][4];
+  bf16x8 kf[2][NT];
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) kf[0][nt] = *reinterpret_cast<const bf16x8*>(Ks + kaddr[0] + nt * 8192);
-  __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+  for (int nt = 0; nt < NT; ++nt) kf[0][nt] = *reinterpret_cast<const bf16x8*>(Ks + kaddr[0] + nt * 8192);
+  __builtin_amdgcn_sched_group_barrier(0x100, NT, 0);
 #pragma unroll
   for (int s = 0; s < 8; ++s) {
     if (s < 7) {
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt)
+      for (int nt = 0; nt < NT; ++nt)
         kf[(s + 1) & 1][nt] = *reinterpret_cast<const bf16x8*>(Ks + kaddr[s + 1] + nt * 8192);
     }
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt) sacc[nt] = mfma32(kf[s & 1][nt], qreg[s], sacc[nt]);
+    for (int nt = 0; nt < NT; ++nt) sacc[nt] = mfma32(kf[s & 1][nt], qreg[s], sacc[nt]);
     if (s < 7) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < NT; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       }
     } else {
-      __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, NT, 0);
     }
   }
 }
@@ -64,11 +65,12 @@ __device__ __forceinline__ void qk_tile(const char* Ks, const int (&kaddr)[8], c
 // stay <= 8, which fp32 sums and bf16 probabilities hold without loss, and
 // the rescaling of l and of the 64 output accumulators is skipped for the
 // wavefront whenever no row needs it.  O / l does not depend on the choice.
-__device__ __forceinline__ void softmax_tile(f32x16 (&sacc)[4], f32x16 (&oacc)[4], float& m_run, float& l_run,
-                                             float scale_log2, bf16x8 (&pfrag)[8]) {
+template <int NT>
+__device__ __forceinline__ void softmax_tile(f32x16 (&sacc)[NT], f32x16 (&oacc)[4], float& m_run, float& l_run,
+                                             float scale_log2, bf16x8 (&pfrag)[NT * 2]) {
   float mx = -INFINITY;
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt)
+  for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int v = 0; v < 16; ++v) mx = fmaxf(mx, sacc[nt][v]);
   mx = half_max(mx) * scale_log2;
@@ -86,7 +88,7 @@ __device__ __forceinline__ void softmax_tile(f32x16 (&sacc)[4], f32x16 (&oacc)[4
   const float m_safe = (m_run == -INFINITY) ? 0.f : m_run;
   float psum = 0.f;
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt)
+  for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
       const float e = fast_exp2(__builtin_fmaf(sacc[nt][v], scale_log2, -m_safe));
@@ -96,8 +98,9 @@ __device__ __forceinline__ void softmax_tile(f32x16 (&sacc)[4], f32x16 (&oacc)[4
   l_run += psum;
 }
 
-// O^T += V_j^T P^T
-__device__ __forceinline__ void pv_tile(const char* Vs, const int (&vaddr)[4][2], const bf16x8 (&pfrag)[8], f32x16 (&oacc)[4]) {
+// O^T += V_j^T P^T on KS x 16 keys
+template <int KS>
+__device__ __forceinline__ void pv_tile(const char* Vs, const int (&vaddr)[4][2], const bf16x8 (&pfrag)[KS], f32x16 (&oacc)[4]) {
   i16x4 vf[2][4][2];
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt)
@@ -107,8 +110,8 @@ __device__ __forceinline__ void pv_tile(const char* Vs, const int (&vaddr)[4][2]
           (__attribute__((address_space(3))) i16x4*)(Vs + vaddr[dt][a]));
   __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
 #pragma unroll
-  for (int ks = 0; ks < 8; ++ks) {
-    if (ks < 7) {
+  for (int ks = 0; ks < KS; ++ks) {
+    if (ks < KS - 1) {
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
@@ -127,7 +130,7 @@ __device__ __forceinline__ void pv_tile(const char* Vs, const int (&vaddr)[4][2]
       }
       oacc[dt] = mfma32(__builtin_bit_cast(bf16x8, av), pfrag[ks], oacc[dt]);
     }
-    if (ks < 7) {
+    if (ks < KS - 1) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
@@ -139,24 +142,23 @@ __device__ __forceinline__ void pv_tile(const char* Vs, const int (&vaddr)[4][2]
   }
 }
 
-// kHasList = false visits every visible block, the dense baseline (its own symbol, so profiles tell the two apart);
-// kPlanned: long lists are cut (attn_plan.h)
-template <bool kHasList, bool kPlanned>
-__global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) {
-  __shared__ __attribute__((aligned(1024))) char Ks[kTileBytes];
-  __shared__ __attribute__((aligned(1024))) char Vs[kTileBytes];
-
+// A unit's sweep.  kHalves: the workgroup has 64 rows of the q-block; wavefront (rg, kh) takes row group rg of them and the keys of
+// half kh of every tile, and the two halves' results meet in LDS at the end.  A tile is then half as long a chain of matrix and
+// vector work, which is what bounds a workgroup alone on its CU: a prompt of 500 tokens, lists of up to 4 blocks, 23.3 -> 21.5 us in
+// all, 2000 with 4 heads 25.2 -> 23.1 (figures of the rule: in_halves).
+template <bool kHasList, bool kPlanned, bool kHalves>
+__device__ __forceinline__ void sweep_unit(const AttnParams& p, const Unit& u, int half, char* Ks, char* Vs) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 31, hh = lane >> 5;
-
-  Unit u;
-  if (!find_unit<kHasList, kPlanned, false>(p, (int)blockIdx.x, u) || !find_list<kHasList, kPlanned>(p, u)) return;
+  const int kh = kHalves ? wave & 1 : 0;
+  const int rows = kHalves ? half * 2 + (wave >> 1) : wave;        // this wavefront's 32 rows of the q-block
+  constexpr int NT = kHalves ? 2 : 4;                              // ... and 32-key steps of a tile, from kh * NT on
   const int n_blocks = u.n_blocks;
   const int first = !kHasList ? u.first : n_blocks > 0 ? u.list[0] : 0;
   const __bf16* qbase = p.q + (int64_t)u.head * p.q_sh;
   const __bf16* kbase = p.k + (int64_t)u.kvh * p.k_sh;
   const __bf16* vbase = p.v + (int64_t)u.kvh * p.v_sh;
-  const int q_pos = u.qb * kBlk + wave * 32 + r + p.kv_off;   // position of this lane's query token on the key axis
+  const int q_pos = u.qb * kBlk + rows * 32 + r + p.kv_off;   // position of this lane's query token on the key axis
 
   bf16x8 qreg[8];   // Q^T fragments stay in registers for the whole sweep
   FragAddr la;
@@ -178,7 +180,7 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
     // The q-block is a tile like any other: copied row-wise (full lines) into the V tile, where each wavefront's
     // eighth-of-a-tile copies are its own 32 query rows, and read back as fragments before V_0 is requested.
     int voffQ[8];
-    tile_offsets(p.q_sn, lane, wave, voffQ);
+    tile_offsets(p.q_sn, lane, rows, voffQ);
     copy_tile(qbase, p.q_sn, p.Lq, u.qb, voffQ, Vs, wave);
     if (n_blocks > 0) {
       kb = kHasList ? clamp_block(first, p.nkb) : first;
@@ -197,8 +199,8 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
 
   for (int j = 0; j < n_blocks; ++j) {
     const int kb_next = (j + 1 < n_blocks) ? (kHasList ? clamp_block(u.list[j + 1], p.nkb) : kb + 1) : -1;
-    f32x16 sacc[4];
-    qk_tile(Ks, la.kaddr, qreg, sacc);
+    f32x16 sacc[NT];
+    qk_tile<NT>(Ks + kh * NT * 8192, la.kaddr, qreg, sacc);
     wait_vm0();
     __syncthreads();                       // everyone is done with K_j; V_j landed and visible
     if (kb_next >= 0) copy_tile_async(kbase, p.k_sn, p.Lk, kb_next, voffK, Ks, wave);
@@ -206,11 +208,11 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
     const bool need_mask = (kb * kBlk + kBlk > p.Lk) || (p.causal && kb * kBlk + kBlk - 1 > u.qb * kBlk + p.kv_off);
     if (need_mask) {
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt) mask_step(sacc[nt], kb * kBlk + nt * 32, hh, q_pos, p.Lk, p.causal);
+      for (int nt = 0; nt < NT; ++nt) mask_step(sacc[nt], kb * kBlk + (kh * NT + nt) * 32, hh, q_pos, p.Lk, p.causal);
     }
-    bf16x8 pfrag[8];
-    softmax_tile(sacc, oacc, m_run, l_run, p.scale_log2, pfrag);
-    pv_tile(Vs, la.vaddr, pfrag, oacc);
+    bf16x8 pfrag[NT * 2];
+    softmax_tile<NT>(sacc, oacc, m_run, l_run, p.scale_log2, pfrag);
+    pv_tile<NT * 2>(Vs + kh * NT * 8192, la.vaddr, pfrag, oacc);
     wait_vm0();
     __syncthreads();                       // everyone is done with V_j; K_{j+1} landed and visible
     if (kb_next >= 0) copy_tile_async(vbase, p.v_sn, p.Lk, kb_next, voffV, Vs, wave);
@@ -229,7 +231,51 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
     __syncthreads();
     load_partials(part, u.cuts, wave, lane, r, hh, oacc, l_run);
   }
+  if (kHalves) {
+    char* const o1 = Ks + (wave >> 1) * 16384 + lane * 16;
+    float* const ml = reinterpret_cast<float*>(Vs) + (wave >> 1) * 128 + lane;
+    if (kh == 1) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        f32x4 w;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) w[t] = oacc[i >> 2][(i & 3) * 4 + t];
+        *reinterpret_cast<f32x4*>(o1 + i * 1024) = w;
+      }
+      ml[0] = m_run;
+      ml[64] = l_run;
+    }
+    __syncthreads();
+    if (kh == 1) return;
+    const float m1 = ml[0], m = fmaxf(m_run, m1), safe = m == -INFINITY ? 0.f : m;
+    const float w0 = fast_exp2(m_run - safe), w1 = fast_exp2(m1 - safe);      // 0 where a half saw no key of this row
+    l_run = w0 * l_run + w1 * ml[64];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const f32x4 o = *reinterpret_cast<const f32x4*>(o1 + i * 1024);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) oacc[i >> 2][(i & 3) * 4 + t] = w0 * oacc[i >> 2][(i & 3) * 4 + t] + w1 * o[t];
+    }
+    store_out(p, u.head, u.qb, rows, lane, r, hh, oacc, l_run, Ks + (wave >> 1) * 16384);
+    return;
+  }
   store_out(p, u.head, u.qb, wave, lane, r, hh, oacc, l_run, Ks + wave * 8192);
+}
+
+// kHasList = false visits every visible block, the dense baseline (its own symbol, so profiles tell the two apart);
+// kPlanned: long lists are cut (attn_plan.h); kHalves: a unit is two workgroups', of 64 rows each
+template <bool kHasList, bool kPlanned, bool kHalves>
+__global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) {
+  __shared__ __attribute__((aligned(1024))) char Ks[kTileBytes];
+  __shared__ __attribute__((aligned(1024))) char Vs[kTileBytes];
+
+  // (both halves on the same XCD, one after the other)
+  const int id = kHalves ? (int)(blockIdx.x >> 4 << 3 | (blockIdx.x & 7)) : (int)blockIdx.x;
+  const int half = kHalves ? (int)(blockIdx.x >> 3 & 1) : 0;
+  Unit u;
+  if (!find_unit<kHasList, kPlanned, false>(p, id, u) || !find_list<kHasList, kPlanned>(p, u)) return;
+  if (kHalves && u.qb * kBlk + half * 64 >= p.Lq) return;
+  sweep_unit<kHasList, kPlanned, kHalves>(p, u, half, Ks, Vs);
 }
 
 }  // namespace xattn
