@@ -112,7 +112,8 @@ bool xattn::attention_queued(int num_heads, int q_len, int k_len, int causal) {
 // Whether a unit is two workgroups', of 64 rows each, with a wavefront for half of every tile's keys: where units leave half of the
 // CUs idle.  Only where lists are never cut; it depends on the whole problem alone.  A prompt of 500 tokens 23.3 -> 21.5 us,
 // 1000 with 8 heads 25.9 -> 23.1, 900 with 16 29.2 -> 25.6.  Two such workgroups on a CU gain where lists are long and lose where
-// they are short (192 units 32 heads 26.5 -> 24.5 us, 168 units of 28 heads 22.5 -> 23.6, 252 28.4 -> 31.3).
+// they are short (192 units 32 heads 26.5 -> 24.5 us, 168 units of 28 heads 22.5 -> 23.6, 252 28.4 -> 31.3).  Dense attention without
+// lists has whole units always: the sums' order differs, and its q-blocks are those of a longer prompt to the bit.
 static bool in_halves(int H, int nqb, int nkb) { return nkb <= 16 && (int64_t)H * nqb <= 128; }
 
 // `ids` units and pieces; with a queue, `places` workgroups of the 64-row kernel.
@@ -123,8 +124,8 @@ static int launch_fwd(const AttnParams& p, int64_t ids, int places, hipStream_t 
     hipLaunchKernelGGL((block_sparse_fwd64_kernel<kHasList, kPlanned>), dim3((unsigned)(p.queue ? places : ids)), dim3(128), 0, s, p);
     if (hipGetLastError() != hipSuccess) return XATTN_ERR_LAUNCH;
   }
-  if (!kPlanned && in_halves(p.H, p.nqb, p.nkb)) {
-    hipLaunchKernelGGL((block_sparse_fwd_kernel<kHasList, false, true>), dim3((unsigned)(2 * ids)), dim3(256), 0, s, p);
+  if (kHasList && !kPlanned && in_halves(p.H, p.nqb, p.nkb)) {
+    hipLaunchKernelGGL((block_sparse_fwd_kernel<true, false, true>), dim3((unsigned)(2 * ids)), dim3(256), 0, s, p);
     if (hipGetLastError() != hipSuccess) return XATTN_ERR_LAUNCH;
   } else if (!all64) {
     hipLaunchKernelGGL((block_sparse_fwd_kernel<kHasList, kPlanned, false>), dim3((unsigned)ids), dim3(256), 0, s, p);
