@@ -7,7 +7,7 @@
 
 int main() {
   const int cases[][3] = {{28, 4, 8}, {28, 4, 9}, {28, 4, 17}, {8, 2, 16}, {8, 2, 4}, {4, 4, 64}, {4, 4, 2}, {32, 1, 8}, {32, 1, 16},
-                          {40, 8, 3}, {12, 12, 40}, {6, 6, 12}, {96, 3, 25}, {28, 4, 63}, {28, 4, 72}};
+                          {40, 8, 3}, {12, 12, 40}, {6, 6, 12}, {96, 3, 25}, {24, 24, 313}, {32, 8, 100}, {28, 4, 63}, {28, 4, 72}};
   int bad = 0;
   for (const auto& c : cases) {
     const int H = c[0], Hkv = c[1], n = c[2];
@@ -25,5 +25,8 @@ int main() {
     std::printf("H=%d Hkv=%d q-blocks %d: wrong %d idle %d most %d of %d\n", H, Hkv, n, wrong, idle, most, H * n);
     bad += !ok;
   }
+  // runs that are even already keep whole units
+  const xattn::DispatchShape whole = xattn::dispatch_shape(24, 24, 313), one = xattn::dispatch_shape(24, 24, 40);
+  bad += whole.unit_rows != 64 || whole.unit_shift != 6 || one.unit_rows != 40;
   return bad ? 1 : 0;
 }
