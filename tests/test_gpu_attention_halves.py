@@ -1,18 +1,12 @@
-"""GPU: attention of few units, where a unit is two workgroups' of 64 rows and half of a tile's keys is a wavefront's."""
+"""GPU: attention of few units, where a unit is two workgroups' of 64 rows and half of a tile's keys is a wavefront's, and of outputs
+around the size from which rows are stored not temporal."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
 
-# up to 128 units of at most 16 key blocks (the last shapes of each kind are the first beyond): rows and keys that end in the
-# first half, at its edge and in the second, keys ahead of the queries, no causality, rows that see no key of a tile's second half
-@pytest.mark.parametrize("q_len,k_len,heads,kv_heads,causal", [
-    (1, 1, 1, 1, True), (63, 63, 4, 2, True), (64, 64, 4, 4, True), (65, 65, 3, 1, True), (128, 128, 32, 8, True), (129, 129, 28, 4, False),
-    (500, 500, 32, 8, True), (512, 512, 32, 32, True), (513, 513, 32, 8, True), (300, 1500, 28, 4, True), (70, 2048, 8, 2, False),
-    (70, 2049, 8, 2, True), (2048, 2048, 8, 1, True), (200, 137, 4, 2, True),
-])
-def test_few_units(q_len, k_len, heads, kv_heads, causal):
+def check(q_len, k_len, heads, kv_heads, causal):
     from xattn.src.Xattention import block_sparse_attention
 
     g = torch.Generator(device="cuda").manual_seed(q_len + k_len)
@@ -40,3 +34,22 @@ def test_few_units(q_len, k_len, heads, kv_heads, causal):
     assert ((got[0] - want).abs() <= bound).all()
     again = block_sparse_attention(q, k, v, idx.contiguous(), cnt.contiguous(), causal=causal).float()
     assert torch.equal(got, again)
+
+
+# up to 128 units of at most 16 key blocks (the last shapes of each kind are the first beyond): rows and keys that end in the
+# first half, at its edge and in the second, keys ahead of the queries, no causality, rows that see no key of a tile's second half
+@pytest.mark.parametrize("q_len,k_len,heads,kv_heads,causal", [
+    (1, 1, 1, 1, True), (63, 63, 4, 2, True), (64, 64, 4, 4, True), (65, 65, 3, 1, True), (128, 128, 32, 8, True), (129, 129, 28, 4, False),
+    (500, 500, 32, 8, True), (512, 512, 32, 32, True), (513, 513, 32, 8, True), (300, 1500, 28, 4, True), (70, 2048, 8, 2, False),
+    (70, 2049, 8, 2, True), (2048, 2048, 8, 1, True), (200, 137, 4, 2, True),
+])
+def test_few_units(q_len, k_len, heads, kv_heads, causal):
+    check(q_len, k_len, heads, kv_heads, causal)
+
+
+# 24 MiB of output and the first token count beyond, of both kernels (without causality: 64 rows), and a ragged end
+@pytest.mark.parametrize("q_len,k_len,heads,kv_heads,causal", [
+    (3072, 3072, 32, 8, True), (3073, 3073, 32, 32, True), (3073, 3400, 32, 8, False), (3519, 3519, 28, 4, True),
+])
+def test_large_outputs(q_len, k_len, heads, kv_heads, causal):
+    check(q_len, k_len, heads, kv_heads, causal)

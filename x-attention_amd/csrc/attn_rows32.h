@@ -146,7 +146,7 @@ __device__ __forceinline__ void pv_tile(const char* Vs, const int (&vaddr)[4][2]
 // half kh of every tile, and the two halves' results meet in LDS at the end.  A tile is then half as long a chain of matrix and
 // vector work, which is what bounds a workgroup alone on its CU: a prompt of 500 tokens, lists of up to 4 blocks, 23.3 -> 21.5 us in
 // all, 2000 with 4 heads 25.2 -> 23.1 (figures of the rule: in_halves).
-template <bool kHasList, bool kPlanned, bool kHalves>
+template <bool kHasList, bool kPlanned, bool kHalves, bool kOutNt>
 __device__ __forceinline__ void sweep_unit(const AttnParams& p, const Unit& u, int half, char* Ks, char* Vs) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 31, hh = lane >> 5;
@@ -178,10 +178,11 @@ __device__ __forceinline__ void sweep_unit(const AttnParams& p, const Unit& u, i
   int kb = 0;
   {
     // The q-block is a tile like any other: copied row-wise (full lines) into the V tile, where each wavefront's
-    // eighth-of-a-tile copies are its own 32 query rows, and read back as fragments before V_0 is requested.
+    // eighth-of-a-tile copies are its own 32 query rows, and read back as fragments before V_0 is requested.  Nobody reads it again:
+    // not temporal (4096 tokens of 32 / 32 heads 82.4 -> 80.2 us, 6000 130.3 -> 129.0, 32768 of 32 / 8 884 -> 880; smaller calls equal).
     int voffQ[8];
     tile_offsets(p.q_sn, lane, rows, voffQ);
-    copy_tile(qbase, p.q_sn, p.Lq, u.qb, voffQ, Vs, wave);
+    copy_tile<kLoadNt>(qbase, p.q_sn, p.Lq, u.qb, voffQ, Vs, wave);
     if (n_blocks > 0) {
       kb = kHasList ? clamp_block(first, p.nkb) : first;
       copy_tile(kbase, p.k_sn, p.Lk, kb, voffK, Ks, wave);
@@ -256,15 +257,16 @@ __device__ __forceinline__ void sweep_unit(const AttnParams& p, const Unit& u, i
 #pragma unroll
       for (int t = 0; t < 4; ++t) oacc[i >> 2][(i & 3) * 4 + t] = w0 * oacc[i >> 2][(i & 3) * 4 + t] + w1 * o[t];
     }
-    store_out(p, u.head, u.qb, rows, lane, r, hh, oacc, l_run, Ks + (wave >> 1) * 16384);
+    store_out(p, u.head, u.qb, rows, lane, r, hh, oacc, l_run, Ks + (wave >> 1) * 16384, false);
     return;
   }
-  store_out(p, u.head, u.qb, wave, lane, r, hh, oacc, l_run, Ks + wave * 8192);
+  store_out(p, u.head, u.qb, wave, lane, r, hh, oacc, l_run, Ks + wave * 8192, kOutNt);
 }
 
 // kHasList = false visits every visible block, the dense baseline (its own symbol, so profiles tell the two apart);
-// kPlanned: long lists are cut (attn_plan.h); kHalves: a unit is two workgroups', of 64 rows each
-template <bool kHasList, bool kPlanned, bool kHalves>
+// kPlanned: long lists are cut (attn_plan.h); kHalves: a unit is two workgroups', of 64 rows each; kOutNt: output rows
+// are stored not temporal (a parameter since the choice made in the kernel costs a call of 700 tokens 0.15 of 26.8 us)
+template <bool kHasList, bool kPlanned, bool kHalves, bool kOutNt>
 __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) {
   __shared__ __attribute__((aligned(1024))) char Ks[kTileBytes];
   __shared__ __attribute__((aligned(1024))) char Vs[kTileBytes];
@@ -275,7 +277,7 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
   Unit u;
   if (!find_unit<kHasList, kPlanned, false>(p, id, u) || !find_list<kHasList, kPlanned>(p, u)) return;
   if (kHalves && u.qb * kBlk + half * 64 >= p.Lq) return;
-  sweep_unit<kHasList, kPlanned, kHalves>(p, u, half, Ks, Vs);
+  sweep_unit<kHasList, kPlanned, kHalves, kOutNt>(p, u, half, Ks, Vs);
 }
 
 }  // namespace xattn
