@@ -11,7 +11,7 @@ SIZES = [
     (2, 1, 1, 64), (63, 4, 2, 128), (64, 4, 1, 320), (65, 4, 4, 384), (77, 3, 1, 448), (128, 32, 8, 64),
     # 64 tokens x 128 features
     (129, 32, 8, 128), (320, 32, 8, 192), (193, 28, 4, 320),
-    # 128 x 128, four stages and two
+    # 128 x 128, and tiles of 192 and 256 tokens
     (321, 32, 8, 256), (640, 32, 8, 64), (641, 32, 8, 128), (1280, 32, 8, 192), (900, 32, 8, 64),
     # the library's
     (1281, 32, 8, 64), (77, 4, 2, 72),
@@ -53,10 +53,11 @@ def test_projections_of_a_turn(tokens, heads, kv_heads, width, bias):
             assert close(y, ref, 2.0 ** -7 * ref.float().abs())
 
 
-# CUs without a tile pull weights ahead from the fourth to the seventh step on: few tiles and many such CUs, none but one XCD's
-# at work, runs of tiles that end inside a head; then tiles of 192 and 256 tokens, whole and with a remainder, steps odd and even
+# CUs without a tile pull weights ahead, from the sixth step on (64 x 64) or the fourth: few tiles, none but one XCD's at work, runs of
+# tiles that end inside a head, last token tiles with enough rows for it and with too few; then tiles of 192 and 256 tokens, whole
+# and with a remainder, steps odd and even
 @pytest.mark.parametrize("tokens,heads,kv_heads,width", [
-    (40, 1, 1, 4096), (2, 3, 1, 1088), (150, 5, 3, 2048), (500, 28, 4, 1024), (250, 32, 8, 704), (600, 32, 8, 4160),
+    (40, 1, 1, 4096), (2, 3, 1, 1088), (150, 5, 3, 2048), (115, 5, 3, 2048), (191, 32, 8, 448), (500, 28, 4, 1024), (250, 32, 8, 704), (600, 32, 8, 4160),
     (769, 32, 8, 576), (960, 32, 8, 512), (1025, 32, 8, 640), (1280, 32, 8, 832),
 ])
 def test_weights_pulled_ahead_and_large_tiles(tokens, heads, kv_heads, width):

@@ -3,8 +3,9 @@
 //
 // Bound: with at most a tile per CU, by how fast one CU fills its LDS (a CU has 32 KiB of loads in flight, whatever is asked of
 // it: 76 GB/s from memory, 130 from the L2), so the tile is the largest that still gives most CUs one: 64 x 64 up to 256 tiles,
-// then 64 tokens x 128 features, 128 x 128, 192 x 128 and, for q, k and v, 256 x 128.  CUs left over pull the weights into the
-// L2 (pull_weights; q, k, v of 500 tokens, 4096 wide, 192 tiles: 39.6 -> 34 us; 3584 wide, 144 tiles: 36.5 -> 29).  The larger
+// then 64 tokens x 128 features, 128 x 128, 192 x 128 and, for q, k and v, 256 x 128.  CUs left over may pull the
+// weights into the L2 (proj_pull.h; weights from memory: q, k, v of 64 tokens, 4096 wide, 22.3 -> 20.8 us, of 192 30.5 -> 27.7, of
+// 512 40.7 -> 39.9; the output of 320, 5120 wide, 38.3 -> 34.0).  The larger
 // tiles took the place of two 128 x 128 ones per CU (4096 wide, 700 tokens 65 -> 46 us, 1000 72 -> 57, 1280 75 -> 64).
 // Splitting a step's depth over two groups of wavefronts helps the smallest tile only (17.6 -> 13.3 us at 64 tokens), where the
 // chain of 64 steps is the time; on the larger ones, where it would save a third of the LDS reads, it is 1 to 8 % slower.
@@ -26,6 +27,7 @@
 // 6000 tokens with the library's output product / this kernel's before weights were pulled ahead, 2 tokens 70 / 62, 16 68 / 64,
 // 64 68 / 74.5, 100 68 / 68.
 #include "lds_limit.h"
+#include "proj_pull.h"
 #include "rotate.h"
 #include "xattn_hip.h"
 
@@ -44,28 +46,17 @@ struct ProjParams {
   int64_t cos_sn, sin_sn;
 };
 
-// What CUs without a tile do: they pull the weights of their XCD's tiles into its L2, ahead of the tiles.  A CU has at most 32 KiB
-// of loads in flight and gets them back in order, so a tile's fill runs at 32 KiB per latency of the slowest load among them:
-// 76 GB/s where each step's weights come from memory, 130 where they are in the L2.  (Loads by the tile's own CU don't help: they
-// queue with the others.  Nor does the scalar cache, some 27 ns per line.)  Lane g takes line g % lines of every `reps`-th step.
 template <int kN, int kThreads, int kAhead>
 __device__ __forceinline__ void pull_weights(const ProjParams& p, uint32_t mt, uint32_t total, uint32_t per_xcd) {
-  const uint32_t first = (blockIdx.x & 7) * per_xcd;
-  if (first >= total) return;
-  const uint32_t last = (first + per_xcd < total ? first + per_xcd : total) - 1;
-  const uint32_t head0 = first / mt * kN / 128, heads = last / mt * kN / 128 + 1 - head0;
-  const uint32_t lines = heads * 128, lanes = ((gridDim.x >> 3) - per_xcd) * kThreads;
-  const uint32_t g = ((blockIdx.x >> 3) - per_xcd) * kThreads + threadIdx.x, reps = lanes / lines;
-  if (g >= reps * lines) return;
-  int f = (int)(head0 * 128 + g % lines), t3 = 0;
-  if (f >= p.n[0]) { f -= p.n[0]; t3 = 1; }
-  if (t3 == 1 && f >= p.n[1]) { f -= p.n[1]; t3 = 2; }
-  const char* const row = reinterpret_cast<const char*>(p.w[t3] + (int64_t)f * p.w_sn[t3]);
+  PullLane l;
+  const uint32_t lane = ((blockIdx.x >> 3) - per_xcd) * kThreads + threadIdx.x, lanes = ((gridDim.x >> 3) - per_xcd) * kThreads;
+  if (!pull_lane(blockIdx.x & 7, lane, lanes, per_xcd, total, mt, kN, p.n[0], p.n[1], kAhead, &l)) return;
+  const char* const row = reinterpret_cast<const char*>(p.w[l.product] + (int64_t)l.row * p.w_sn[l.product]);
   const uint32_t steps = (uint32_t)p.K / 64;
-  for (uint32_t t = kAhead + g / lines; t < steps; t += 8 * reps) {
+  for (uint32_t t = l.step; t < steps; t += 8 * l.every) {
     uint32_t v[8];
 #pragma unroll
-    for (uint32_t u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const uint32_t*>(row + (int64_t)(t + u * reps < steps ? t + u * reps : t) * 128);
+    for (uint32_t u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const uint32_t*>(row + (int64_t)(t + u * l.every < steps ? t + u * l.every : t) * 128);
 #pragma unroll
     for (uint32_t u = 0; u < 8; ++u) asm volatile("" ::"v"(v[u]));
   }
@@ -73,8 +64,9 @@ __device__ __forceinline__ void pull_weights(const ProjParams& p, uint32_t mt, u
 
 // Four wavefronts (2 x 2) take 64 * NB features x 64 * MB tokens; 64-deep slabs of both operands go straight to a ring of NS
 // LDS stages, NS - 1 steps ahead of their use, one barrier per step.  KS = 2: four more multiply the second half of each
-// slab, and the two sums of every element are added at the end.
-template <int NB, int MB, int NS, int KS, bool kRope>
+// slab, and the two sums of every element are added at the end.  kPull: workgroups beyond the tiles pull weights (a kernel of its
+// own, since the code ahead of the tiles' loop moves it: 1 to 3 % of a narrow product's time).
+template <int NB, int MB, int NS, int KS, bool kRope, bool kPull>
 __global__ __launch_bounds__(256 * KS, 2) void proj_gemm_kernel(ProjParams p) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   constexpr int kN = 64 * NB, kM = 64 * MB;
@@ -94,7 +86,7 @@ __global__ __launch_bounds__(256 * KS, 2) void proj_gemm_kernel(ProjParams p) {
   const uint32_t total = mt * (uint32_t)((p.n[0] + p.n[1] + p.n[2]) / kN), per_xcd = (total + 7) / 8;
   const uint32_t lin = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if ((blockIdx.x >> 3) >= per_xcd) {
-    pull_weights<kN, 256 * KS, NS - 1>(p, mt, total, per_xcd);
+    if (kPull) pull_weights<kN, 256 * KS, NS - 1>(p, mt, total, per_xcd);
     return;
   }
   if (lin >= total) return;
@@ -266,17 +258,23 @@ Tile tile_for(int64_t tokens, int64_t features, bool qkv) {
   return tiles(128, 128) <= 2 * kCUs ? k128x128Twice : kNone;
 }
 
-template <int NB, int MB, int NS, int KS, bool kRope>
-int launch(const ProjParams& p, hipStream_t s) {
+template <int NB, int MB, int NS, int KS, bool kRope, bool kPull>
+int launch_tiles(const ProjParams& p, unsigned grid, hipStream_t s) {
   constexpr int kLds = (NB + MB) * 64 * 128 * NS;
-  static LdsLimit limit;
-  if (limit.raise((const void*)proj_gemm_kernel<NB, MB, NS, KS, kRope>) != hipSuccess) return XATTN_ERR_LAUNCH;
-  const unsigned tiles = (unsigned)((p.M + 64 * MB - 1) / (64 * MB)) * (unsigned)((p.n[0] + p.n[1] + p.n[2]) / (64 * NB));
   static_assert(kLds <= 160 * 1024, "LDS of a CU");
-  // one workgroup per CU: the CUs left over pull weights
-  const unsigned grid = kLds > 80 * 1024 && tiles < kCUs ? kCUs : (tiles + 7) / 8 * 8;
-  hipLaunchKernelGGL((proj_gemm_kernel<NB, MB, NS, KS, kRope>), dim3(grid), dim3(256 * KS), kLds, s, p);
+  static LdsLimit limit;
+  if (limit.raise((const void*)proj_gemm_kernel<NB, MB, NS, KS, kRope, kPull>) != hipSuccess) return XATTN_ERR_LAUNCH;
+  hipLaunchKernelGGL((proj_gemm_kernel<NB, MB, NS, KS, kRope, kPull>), dim3(grid), dim3(256 * KS), kLds, s, p);
   return hipGetLastError() == hipSuccess ? XATTN_OK : XATTN_ERR_LAUNCH;
+}
+
+// kMayPull: one workgroup per CU, and the rule of proj_pull.h gains
+template <int NB, int MB, int NS, int KS, bool kRope, bool kMayPull>
+int launch(const ProjParams& p, hipStream_t s) {
+  const unsigned tiles = (unsigned)((p.M + 64 * MB - 1) / (64 * MB)) * (unsigned)((p.n[0] + p.n[1] + p.n[2]) / (64 * NB));
+  const unsigned grid = (tiles + 7) / 8 * 8, places = pull_places((uint32_t)p.M, 64 * MB, tiles);
+  if (kMayPull && places) return launch_tiles<NB, MB, NS, KS, kRope, kMayPull>(p, grid + 8 * places, s);
+  return launch_tiles<NB, MB, NS, KS, kRope, false>(p, grid, s);
 }
 
 // offsets inside a tile are held in 32 bits
@@ -287,12 +285,12 @@ template <bool kRope>
 int run(const ProjParams& p, void* stream) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (tile_for(p.M, (int64_t)p.n[0] + p.n[1] + p.n[2], kRope)) {
-    case k64x64: return launch<1, 1, 6, 2, kRope>(p, s);
-    case k128x64: return launch<2, 1, 4, 1, kRope>(p, s);
-    case k128x128: return launch<2, 2, 4, 1, kRope>(p, s);
-    case k128x192: return launch<2, 3, 4, 1, kRope>(p, s);
-    case k128x256: return launch<2, 4, 3, 1, kRope>(p, s);
-    case k128x128Twice: return launch<2, 2, 2, 1, kRope>(p, s);
+    case k64x64: return launch<1, 1, 6, 2, kRope, true>(p, s);
+    case k128x64: return launch<2, 1, 4, 1, kRope, true>(p, s);
+    case k128x128: return launch<2, 2, 4, 1, kRope, true>(p, s);
+    case k128x192: return launch<2, 3, 4, 1, kRope, false>(p, s);
+    case k128x256: return launch<2, 4, 3, 1, kRope, false>(p, s);
+    case k128x128Twice: return launch<2, 2, 2, 1, kRope, false>(p, s);
     default: return XATTN_ERR_SHAPE;
   }
 }
