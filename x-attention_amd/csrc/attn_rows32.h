@@ -178,11 +178,12 @@ __device__ __forceinline__ void sweep_unit(const AttnParams& p, const Unit& u, i
   int kb = 0;
   {
     // The q-block is a tile like any other: copied row-wise (full lines) into the V tile, where each wavefront's
-    // eighth-of-a-tile copies are its own 32 query rows, and read back as fragments before V_0 is requested.  Nobody reads it again:
-    // not temporal (4096 tokens of 32 / 32 heads 82.4 -> 80.2 us, 6000 130.3 -> 129.0, 32768 of 32 / 8 884 -> 880; smaller calls equal).
+    // eighth-of-a-tile copies are its own 32 query rows, and read back as fragments before V_0 is requested.  (Loaded not temporal:
+    // prompts of 2000 tokens with 28 / 4 heads 41.2 -> 45.0 us, 32 / 32 47.3 -> 50.7, 3000 with 32 / 8 74.5 -> 78.0, video of 2500
+    // 76.8 -> 80.7, of 6000 with 28 / 4 204.9 -> 211.2; only 4096 and 6500 with 32 / 32 gain, 87.1 -> 85.8 and 132.3 -> 131.5.)
     int voffQ[8];
     tile_offsets(p.q_sn, lane, rows, voffQ);
-    copy_tile<kLoadNt>(qbase, p.q_sn, p.Lq, u.qb, voffQ, Vs, wave);
+    copy_tile(qbase, p.q_sn, p.Lq, u.qb, voffQ, Vs, wave);
     if (n_blocks > 0) {
       kb = kHasList ? clamp_block(first, p.nkb) : first;
       copy_tile(kbase, p.k_sn, p.Lk, kb, voffK, Ks, wave);
