@@ -258,10 +258,10 @@ __device__ __forceinline__ void sweep_unit(const AttnParams& p, const Unit& u, i
 #pragma unroll
       for (int t = 0; t < 4; ++t) oacc[i >> 2][(i & 3) * 4 + t] = w0 * oacc[i >> 2][(i & 3) * 4 + t] + w1 * o[t];
     }
-    store_out(p, u.head, u.qb, rows, lane, r, hh, oacc, l_run, Ks + (wave >> 1) * 16384, false);
+    store_out(p, u.head, u.qb, rows, lane, r, hh, oacc, l_run, Ks + (wave >> 1) * 16384);
     return;
   }
-  store_out(p, u.head, u.qb, wave, lane, r, hh, oacc, l_run, Ks + wave * 8192, kOutNt);
+  store_out<kOutNt>(p, u.head, u.qb, wave, lane, r, hh, oacc, l_run, Ks + wave * 8192);
 }
 
 // kHasList = false visits every visible block, the dense baseline (its own symbol, so profiles tell the two apart);

@@ -545,7 +545,7 @@ __global__ __launch_bounds__(128, 1) void block_sparse_fwd64_kernel(AttnParams) 
     }
     if (whole) {
 #pragma unroll
-      for (int g = 0; g < 2; ++g) store_out(p, u.head, u.qb, wave * 2 + g, lane, r, hh, w.o[g], w.l[g], stage + wave * kOutStage, p.out_nt);
+      for (int g = 0; g < 2; ++g) store_out(p, u.head, u.qb, wave * 2 + g, lane, r, hh, w.o[g], w.l[g], stage + wave * kOutStage);
     }
     if (id < 0) return;
     u = n;

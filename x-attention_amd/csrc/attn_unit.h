@@ -26,7 +26,6 @@ struct AttnParams {
   int qb_begin, qb_end;     // q-blocks handled by this launch
   int causal, kv_off;       // kv_off = Lk - Lq
   float scale_log2;         // softmax_scale * log2(e)
-  int out_nt;               // output rows are stored not temporal
   DispatchShape shape;      // dispatch_shape of the launch, computed on the host
   AttnPlan plan;            // kPlanned only
   int32_t* queue;           // this launch's work queue (kQueueWords, zero), or null: one workgroup per id
@@ -250,8 +249,9 @@ __device__ __forceinline__ void mask_step(f32x16& s, int key0, int hh, int q_pos
 // that wait was a quarter of a workgroup's life.  Staged through 8 KiB of LDS,
 // 16 lanes write one 256-byte row: 64 full-line requests.
 constexpr int kOutStage = 8192;      // bytes per wavefront
+template <bool kNt = false>
 __device__ __forceinline__ void store_out(const AttnParams& p, int head, int qb, int wave, int lane, int r, int hh,
-                                          const f32x16 (&oacc)[4], float l_run, char* stage, bool out_nt) {
+                                          const f32x16 (&oacc)[4], float l_run, char* stage) {
   const float l_tot = half_sum(l_run);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
 #pragma unroll
@@ -278,10 +278,7 @@ __device__ __forceinline__ void store_out(const AttnParams& p, int head, int qb,
   for (int i = 0; i < 8; ++i) {
     const int row = i * 4 + (lane >> 4);
     const u32x4 w = *reinterpret_cast<const u32x4*>(stage + row * 256 + ((c ^ (row & 15)) << 4));
-    if (out_nt)
-      __builtin_amdgcn_raw_buffer_store_b128(w, ores, (int)(voff0 + (uint32_t)(i * 4) * row_bytes), 0, kLoadNt);
-    else
-      __builtin_amdgcn_raw_buffer_store_b128(w, ores, (int)(voff0 + (uint32_t)(i * 4) * row_bytes), 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(w, ores, (int)(voff0 + (uint32_t)(i * 4) * row_bytes), 0, kNt ? kLoadNt : 0);
   }
 }
 

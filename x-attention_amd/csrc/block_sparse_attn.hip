@@ -116,10 +116,13 @@ bool xattn::attention_queued(int num_heads, int q_len, int k_len, int causal) {
 // lists has whole units always: the sums' order differs, and its q-blocks are those of a longer prompt to the bit.
 static bool in_halves(int H, int nqb, int nkb) { return nkb <= 16 && (int64_t)H * nqb <= 128; }
 
-// Bytes of output from which its rows are stored not temporal: they then leave the memory-side cache to q, k and v, which the estimate
-// has just read.  4096 tokens of 32 / 32 heads 88.0 -> 84.5 us, 6000 132.1 -> 130.5, 131072 of 32 / 8 8064 -> 8032.  The product that
+// Bytes of output from which the 32-row kernel stores its rows not temporal: they then leave the memory-side cache to q, k and v, which
+// the estimate has just read.  Prompts, us: 4096 tokens of 32 / 32 heads 88.5 -> 87.1, 6500 134.8 -> 132.3, 5000 of 32 / 8 124.3 -> 117.1, 6500 of
+// 28 / 4 124.1 -> 118.6, video of 7000 274.8 -> 270.3, 10000 of 32 / 8 258 -> 256; from 16000 tokens on they are equal.  The product that
 // reads the output next finds a small one in that cache (a layer's 900 tokens on 3000 135.6 -> 137.3 us if stored so, 2100 on
-// 6000 312.5 -> 313.9); with larger ones it is bound by its arithmetic (layers of 8000 and 16000 tokens are equal).
+// 6000 312.5 -> 313.9); with larger ones it is bound by its arithmetic (layers of 3500 to 12000 tokens are equal or gain).
+// Not in the 64-row kernel, whose lists are long: video of 65536 tokens 15306 -> 15366 us, text of 131072 14373 -> 14405, of 50000 2650 ->
+// 2675, fields equal.
 constexpr int64_t kOutNtBytes = 24 << 20;
 
 // `ids` units and pieces; with a queue, `places` workgroups of the 64-row kernel.
@@ -134,7 +137,8 @@ static int launch_fwd(const AttnParams& p, int64_t ids, int places, hipStream_t 
     hipLaunchKernelGGL((block_sparse_fwd_kernel<true, false, true, false>), dim3((unsigned)(2 * ids)), dim3(256), 0, s, p);
     if (hipGetLastError() != hipSuccess) return XATTN_ERR_LAUNCH;
   } else if (!all64) {
-    const auto kernel = p.out_nt ? block_sparse_fwd_kernel<kHasList, kPlanned, false, true> : block_sparse_fwd_kernel<kHasList, kPlanned, false, false>;
+    const bool out_nt = (int64_t)p.H * p.Lq * kHeadDim * 2 > kOutNtBytes;
+    const auto kernel = out_nt ? block_sparse_fwd_kernel<kHasList, kPlanned, false, true> : block_sparse_fwd_kernel<kHasList, kPlanned, false, false>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)ids), dim3(256), 0, s, p);
     if (hipGetLastError() != hipSuccess) return XATTN_ERR_LAUNCH;
   }
@@ -191,7 +195,6 @@ int xattn::block_sparse_impl(const void* q, const void* k, const void* v, void* 
   p.qb_begin = q_block_begin;
   p.qb_end = q_block_end;
   p.shape = dispatch_shape(p.H, p.Hkv, q_block_end - q_block_begin);
-  p.out_nt = (int64_t)num_heads * q_len * kHeadDim * 2 > kOutNtBytes;
   p.plan = plan ? *plan : AttnPlan{};
   p.lists_decide = lists_decide(p.H, p.nqb, p.nkb, p.kv_off, p.causal);
   const int64_t grid = grid_for(p.H, p.Hkv, q_block_end - q_block_begin);
