@@ -96,12 +96,27 @@ struct DispatchShape {
   int turn_shift;  // groups rotate once per 1 << turn_shift runs
   int unit_shift;  // a unit has 1 << unit_shift ids (kUnit, fewer where runs are few)
 };
-// Where a launch has fewer than eight runs, their number is made one that gives every XCD as many units, and a unit has no more
-// ids than it needs.  (9 q-blocks of 28 heads on 4 KV heads were one run, which left half of the XCDs idle; 8 q-blocks of 32 heads
-// on 32 KV heads had 1792 ids without work.  Prompts, us: 700 tokens with 28 / 4 heads 27.0 -> 24.3, 1100 31.3 -> 28.5, 2000 with 8 / 2
-// heads 31.2 -> 23.8, 500 with 32 / 32 24.4 -> 23.7.)  Runs that are even already stay as they are: 64 q-blocks of a head are what an
-// XCD has at once, and units of 63 straddle that (40003 tokens of 24 heads without causality 15.57 -> 15.68 ms, 40961 18.18 -> 18.36).
-__host__ __device__ inline DispatchShape dispatch_shape(int H, int Hkv, int n_qblocks) {
+// (head, q-block)s of the XCD that has most of them, units being dealt to the XCDs in turn.
+inline int64_t fullest_xcd(const DispatchShape& d, int n_qblocks) {
+  int64_t on[8] = {}, most = 0;
+  unsigned unit = 0;
+  for (int left = n_qblocks; left > 0; left -= d.unit_rows)
+    for (int g = 0; g < d.n_groups; ++g) on[unit++ & 7] += left < d.unit_rows ? left : d.unit_rows;
+  for (int64_t n : on) most = n > most ? n : most;
+  return most * d.set_heads;
+}
+
+// Where a launch has fewer than eight runs, some XCDs may have a unit more than others, or the only ones.  There the number of runs
+// is rounded up to one of which every XCD has as many, if the fullest XCD then has an eighth less to do (q-blocks per unit are rounded up,
+// too, which may leave fewer runs than that, or a short last one); and a unit has no more ids than it needs.
+// Prompts, us, whole units / rounded up: 650 tokens with 28 / 4 heads 29.1 / 26.9, 1150 33.7 / 32.0, 3000 (105 workgroups on the fullest XCD, 84)
+// 62.3 / 60.6, video 84.9 / 79.6; lists of about 4 blocks: 8000 tokens of one head 31.3 / 23.3, 4000 of 4 / 1 30.6 / 23.1, 5000 of 12 / 12
+// 38.5 / 33.8.  But 2800 tokens with 28 / 4 (91 and 84) 58.7 / 60.1, such lists 34.6 / 39.7, 5000 (154 and 147) 92.8 / 94.1, 52.8 / 56.4;
+// and where the fullest has more than before, 4224 tokens with 16 / 2 (72 and 80), lists of 8 blocks 42.4 / 53.8.  Units of more than 32
+// ids that a launch goes round in several times straddle an XCD's 64 places, which costs long lists 2 to 8 % of what evenness gives short ones
+// (3000 of 28 / 4: lists of about 2 blocks 29.5 / 28.0, 4 39.5 / 42.9).  40003 tokens of 24 heads without causality, runs even
+// already, in units of 63 instead of 64 15.57 -> 15.68 ms.
+inline DispatchShape dispatch_shape(int H, int Hkv, int n_qblocks) {
   DispatchShape d;
   d.group = H / Hkv;
   d.sets = (d.group + kUnit - 1) / kUnit;
@@ -111,10 +126,13 @@ __host__ __device__ inline DispatchShape dispatch_shape(int H, int Hkv, int n_qb
   d.turn_shift = d.n_groups == 4 ? 1 : d.n_groups == 2 ? 2 : 0;
   const int runs = (n_qblocks + d.unit_rows - 1) / d.unit_rows;
   const int even = d.n_groups % 8 == 0 ? 1 : d.n_groups % 4 == 0 ? 2 : d.n_groups % 2 == 0 ? 4 : 8;
-  if (runs < 8) {
-    const int wanted = (runs + even - 1) / even * even;
-    if (wanted != runs || runs == 1) d.unit_rows = n_qblocks > wanted ? (n_qblocks + wanted - 1) / wanted : 1;
+  const int wanted = (runs + even - 1) / even * even;
+  if (runs < 8 && wanted != runs) {
+    DispatchShape e = d;
+    e.unit_rows = (n_qblocks + wanted - 1) / wanted;
+    if (8 * fullest_xcd(e, n_qblocks) <= 7 * fullest_xcd(d, n_qblocks)) d = e;
   }
+  if (d.unit_rows > n_qblocks) d.unit_rows = n_qblocks;
   d.unit_shift = 0;
   while (1 << d.unit_shift < d.set_heads * d.unit_rows) ++d.unit_shift;
   return d;
@@ -147,17 +165,17 @@ __host__ __device__ inline bool map_workgroup(int id, const DispatchShape& d, in
   *kv_head = (int)kvh;
   return true;
 }
-__host__ __device__ inline bool map_workgroup(int id, int H, int Hkv, int qb_begin, int qb_end, int* head, int* qb) {
+inline bool map_workgroup(int id, int H, int Hkv, int qb_begin, int qb_end, int* head, int* qb) {
   int kv_head;
   return map_workgroup(id, dispatch_shape(H, Hkv, qb_end - qb_begin), qb_begin, qb_end, head, qb, &kv_head);
 }
 
 // grid size of a launch over n_qblocks q-blocks
-inline int64_t grid_for(int H, int Hkv, int n_qblocks) {
-  const DispatchShape d = dispatch_shape(H, Hkv, n_qblocks);
+inline int64_t grid_for(const DispatchShape& d, int n_qblocks) {
   const int64_t runs = (n_qblocks + d.unit_rows - 1) / d.unit_rows;
   return ((runs * d.n_groups + 7) / 8 * 8) << d.unit_shift;
 }
+inline int64_t grid_for(int H, int Hkv, int n_qblocks) { return grid_for(dispatch_shape(H, Hkv, n_qblocks), n_qblocks); }
 
 // Token strides of K and V the tile copies can address (byte offsets inside a
 // 128-row tile are held in 32 bits), and a usable softmax scale.

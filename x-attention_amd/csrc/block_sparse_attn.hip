@@ -197,7 +197,7 @@ int xattn::block_sparse_impl(const void* q, const void* k, const void* v, void* 
   p.shape = dispatch_shape(p.H, p.Hkv, q_block_end - q_block_begin);
   p.plan = plan ? *plan : AttnPlan{};
   p.lists_decide = lists_decide(p.H, p.nqb, p.nkb, p.kv_off, p.causal);
-  const int64_t grid = grid_for(p.H, p.Hkv, q_block_end - q_block_begin);
+  const int64_t grid = grid_for(p.shape, q_block_end - q_block_begin);
   const int64_t ids = grid + (plan ? ((int64_t)plan_pieces(plan->shape, q_block_end - q_block_begin) + 7) / 8 * 8 : 0);
   if (ids > 0x7fffffff) return XATTN_ERR_SHAPE;
   p.unit_ids = (int)grid;

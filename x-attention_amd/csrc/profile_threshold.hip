@@ -27,6 +27,7 @@ struct MassParams {
   int H, Hkv, Lq, Lk, nqb, nkb;
   int causal, kv_off;
   float scale_log2;
+  DispatchShape shape;      // computed on the host
 };
 
 __global__ __launch_bounds__(256, 2) void block_mass_kernel(MassParams p) {
@@ -36,9 +37,8 @@ __global__ __launch_bounds__(256, 2) void block_mass_kernel(MassParams p) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 31, hh = lane >> 5;
 
-  int head, qb;
-  if (!map_workgroup(blockIdx.x, p.H, p.Hkv, 0, p.nqb, &head, &qb)) return;
-  const int kvh = head / (p.H / p.Hkv);
+  int head, qb, kvh;
+  if (!map_workgroup(blockIdx.x, p.shape, 0, p.nqb, &head, &qb, &kvh)) return;
   const __bf16* qbase = p.q + (int64_t)head * p.q_sh;
   const __bf16* kbase = p.k + (int64_t)kvh * p.k_sh;
   float* out = p.mass + ((int64_t)head * p.nqb + qb) * p.nkb;
@@ -262,7 +262,8 @@ extern "C" int xattn_block_mass(const void* q, const void* k, float* mass, int n
   p.causal = causal ? 1 : 0;
   p.kv_off = k_len - q_len;
   p.scale_log2 = softmax_scale * kLog2e;
-  const int64_t grid = grid_for(p.H, p.Hkv, p.nqb);
+  p.shape = dispatch_shape(p.H, p.Hkv, p.nqb);
+  const int64_t grid = grid_for(p.shape, p.nqb);
   if (grid > 0x7fffffff) return XATTN_ERR_SHAPE;
   hipLaunchKernelGGL(block_mass_kernel, dim3((unsigned)grid), dim3(256), 0, static_cast<hipStream_t>(stream), p);
   return hipGetLastError() == hipSuccess ? XATTN_OK : XATTN_ERR_LAUNCH;
