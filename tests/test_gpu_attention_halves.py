@@ -47,9 +47,11 @@ def test_few_units(q_len, k_len, heads, kv_heads, causal):
     check(q_len, k_len, heads, kv_heads, causal)
 
 
-# 24 MiB of output and the first token count beyond, of both kernels (without causality: 64 rows), and a ragged end
+# 24 MiB of output and the first token count beyond, of both kernels (without causality: 64 rows), and a ragged end; with a KV head per
+# query head 30 MiB and the first beyond, from which queries are loaded not temporal, too
 @pytest.mark.parametrize("q_len,k_len,heads,kv_heads,causal", [
     (3072, 3072, 32, 8, True), (3073, 3073, 32, 32, True), (3073, 3400, 32, 8, False), (3519, 3519, 28, 4, True),
+    (3840, 3840, 32, 32, True), (3841, 3841, 32, 32, True), (1921, 6000, 64, 64, True),
 ])
 def test_large_outputs(q_len, k_len, heads, kv_heads, causal):
     check(q_len, k_len, heads, kv_heads, causal)

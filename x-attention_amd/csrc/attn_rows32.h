@@ -142,11 +142,14 @@ __device__ __forceinline__ void pv_tile(const char* Vs, const int (&vaddr)[4][2]
   }
 }
 
+// What is loaded and stored not temporal (the rule: not_temporal in block_sparse_attn.hip)
+enum { kNtNone, kNtOutput, kNtQueriesToo };
+
 // A unit's sweep.  kHalves: the workgroup has 64 rows of the q-block; wavefront (rg, kh) takes row group rg of them and the keys of
 // half kh of every tile, and the two halves' results meet in LDS at the end.  A tile is then half as long a chain of matrix and
 // vector work, which is what bounds a workgroup alone on its CU: a prompt of 500 tokens, lists of up to 4 blocks, 23.3 -> 21.5 us in
 // all, 2000 with 4 heads 25.2 -> 23.1 (figures of the rule: in_halves).
-template <bool kHasList, bool kPlanned, bool kHalves, bool kOutNt>
+template <bool kHasList, bool kPlanned, bool kHalves, int kNt>
 __device__ __forceinline__ void sweep_unit(const AttnParams& p, const Unit& u, int half, char* Ks, char* Vs) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 31, hh = lane >> 5;
@@ -178,12 +181,10 @@ __device__ __forceinline__ void sweep_unit(const AttnParams& p, const Unit& u, i
   int kb = 0;
   {
     // The q-block is a tile like any other: copied row-wise (full lines) into the V tile, where each wavefront's
-    // eighth-of-a-tile copies are its own 32 query rows, and read back as fragments before V_0 is requested.  (Loaded not temporal:
-    // prompts of 2000 tokens with 28 / 4 heads 41.2 -> 45.0 us, 32 / 32 47.3 -> 50.7, 3000 with 32 / 8 74.5 -> 78.0, video of 2500
-    // 76.8 -> 80.7, of 6000 with 28 / 4 204.9 -> 211.2; only 4096 and 6500 with 32 / 32 gain, 87.1 -> 85.8 and 132.3 -> 131.5.)
+    // eighth-of-a-tile copies are its own 32 query rows, and read back as fragments before V_0 is requested.
     int voffQ[8];
     tile_offsets(p.q_sn, lane, rows, voffQ);
-    copy_tile(qbase, p.q_sn, p.Lq, u.qb, voffQ, Vs, wave);
+    copy_tile<kNt == kNtQueriesToo ? kLoadNt : 0>(qbase, p.q_sn, p.Lq, u.qb, voffQ, Vs, wave);
     if (n_blocks > 0) {
       kb = kHasList ? clamp_block(first, p.nkb) : first;
       copy_tile(kbase, p.k_sn, p.Lk, kb, voffK, Ks, wave);
@@ -261,13 +262,13 @@ __device__ __forceinline__ void sweep_unit(const AttnParams& p, const Unit& u, i
     store_out(p, u.head, u.qb, rows, lane, r, hh, oacc, l_run, Ks + (wave >> 1) * 16384);
     return;
   }
-  store_out<kOutNt>(p, u.head, u.qb, wave, lane, r, hh, oacc, l_run, Ks + wave * 8192);
+  store_out<kNt != kNtNone>(p, u.head, u.qb, wave, lane, r, hh, oacc, l_run, Ks + wave * 8192);
 }
 
 // kHasList = false visits every visible block, the dense baseline (its own symbol, so profiles tell the two apart);
-// kPlanned: long lists are cut (attn_plan.h); kHalves: a unit is two workgroups', of 64 rows each; kOutNt: output rows
-// are stored not temporal (a parameter since the choice made in the kernel costs a call of 700 tokens 0.15 of 26.8 us)
-template <bool kHasList, bool kPlanned, bool kHalves, bool kOutNt>
+// kPlanned: long lists are cut (attn_plan.h); kHalves: a unit is two workgroups', of 64 rows each; kNt: what is
+// not temporal (a parameter since the choice made in the kernel costs a call of 700 tokens 0.15 of 26.8 us)
+template <bool kHasList, bool kPlanned, bool kHalves, int kNt>
 __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) {
   __shared__ __attribute__((aligned(1024))) char Ks[kTileBytes];
   __shared__ __attribute__((aligned(1024))) char Vs[kTileBytes];
@@ -278,7 +279,7 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
   Unit u;
   if (!find_unit<kHasList, kPlanned, false>(p, id, u) || !find_list<kHasList, kPlanned>(p, u)) return;
   if (kHalves && u.qb * kBlk + half * 64 >= p.Lq) return;
-  sweep_unit<kHasList, kPlanned, kHalves, kOutNt>(p, u, half, Ks, Vs);
+  sweep_unit<kHasList, kPlanned, kHalves, kNt>(p, u, half, Ks, Vs);
 }
 
 }  // namespace xattn

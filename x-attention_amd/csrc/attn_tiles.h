@@ -21,7 +21,8 @@ __device__ __forceinline__ int swz(int n) { return ((n & 3) << 2) | ((n >> 2) & 
 
 // Copies key block kb of one head (row stride sn elements) into an LDS tile.
 // Wavefront w issues 8 instructions of 1 KiB (4 rows) each; voff[i] is the
-// lane's byte offset inside the block for instruction i.
+// lane's byte offset inside the block for instruction i.  kPolicy: the loads' cache policy.
+template <int kPolicy = 0>
 __device__ __forceinline__ void copy_tile(const __bf16* base, int64_t sn, int len, int kb, const int (&voff)[8],
                                           char* tile, int wave) {
   const int rows_left = len - kb * kBlk;
@@ -30,7 +31,7 @@ __device__ __forceinline__ void copy_tile(const __bf16* base, int64_t sn, int le
       (void*)(base + (int64_t)kb * kBlk * sn), 0, (int)((int64_t)rows * sn * 2), 0x00020000);
 #pragma unroll
   for (int i = 0; i < 8; ++i)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(tile + (wave * 8 + i) * 1024), 16, voff[i], 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(tile + (wave * 8 + i) * 1024), 16, voff[i], 0, 0, kPolicy);
 }
 
 // The same copy issued from one assembly block, M0 (the LDS destination) included.  The compiler makes the

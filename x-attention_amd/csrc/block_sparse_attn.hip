@@ -124,6 +124,16 @@ static bool in_halves(int H, int nqb, int nkb) { return nkb <= 16 && (int64_t)H 
 // Not in the 64-row kernel, whose lists are long: video of 65536 tokens 15306 -> 15366 us, text of 131072 14373 -> 14405, of 50000 2650 ->
 // 2675, fields equal.
 constexpr int64_t kOutNtBytes = 24 << 20;
+// ... and from which the queries of calls with a KV head per query head are loaded so too, of 32 heads, text at two strides: 3100 tokens
+// 67.1 -> 70.8, 68.7 -> 71.4, 3500 75.5 -> 76.2, 76.4 -> 77.9, 3900 86.4 -> 86.3, 83.1 -> 82.0, 4300 101.5 -> 97.5, 98.8 -> 97.5, 5500 123.7 -> 121.2,
+// 116.5 -> 115.4, 8000 183.9 -> 183.0, 161.7 -> 160.4, 13000 327.6 -> 327.0, 294.1 -> 292.2; of 24 5000 equal, 6500 117.5 -> 116.7.  With fewer KV
+// heads most calls are slower: 28 / 4 2000 41.2 -> 45.0, video of 6000 204.9 -> 211.2, of 8000 332 -> 338, 32 / 8 5000 117.1 -> 124.8.
+constexpr int64_t kQueriesNtBytes = 30 << 20;
+
+static int not_temporal(const AttnParams& p, bool lists) {
+  const int64_t bytes = (int64_t)p.H * p.Lq * kHeadDim * 2;
+  return bytes <= kOutNtBytes ? kNtNone : lists && p.H == p.Hkv && bytes > kQueriesNtBytes ? kNtQueriesToo : kNtOutput;
+}
 
 // `ids` units and pieces; with a queue, `places` workgroups of the 64-row kernel.
 template <bool kHasList, bool kPlanned>
@@ -133,16 +143,17 @@ static int launch_fwd(const AttnParams& p, int64_t ids, int places, hipStream_t 
     hipLaunchKernelGGL((block_sparse_fwd64_kernel<kHasList, kPlanned>), dim3((unsigned)(p.queue ? places : ids)), dim3(128), 0, s, p);
     if (hipGetLastError() != hipSuccess) return XATTN_ERR_LAUNCH;
   }
+  if (all64) return XATTN_OK;
   if (kHasList && !kPlanned && in_halves(p.H, p.nqb, p.nkb)) {
-    hipLaunchKernelGGL((block_sparse_fwd_kernel<true, false, true, false>), dim3((unsigned)(2 * ids)), dim3(256), 0, s, p);
-    if (hipGetLastError() != hipSuccess) return XATTN_ERR_LAUNCH;
-  } else if (!all64) {
-    const bool out_nt = (int64_t)p.H * p.Lq * kHeadDim * 2 > kOutNtBytes;
-    const auto kernel = out_nt ? block_sparse_fwd_kernel<kHasList, kPlanned, false, true> : block_sparse_fwd_kernel<kHasList, kPlanned, false, false>;
+    hipLaunchKernelGGL((block_sparse_fwd_kernel<true, false, true, kNtNone>), dim3((unsigned)(2 * ids)), dim3(256), 0, s, p);
+  } else {
+    auto kernel = block_sparse_fwd_kernel<kHasList, kPlanned, false, kNtNone>;
+    const int nt = not_temporal(p, kHasList);
+    if (nt == kNtOutput) kernel = block_sparse_fwd_kernel<kHasList, kPlanned, false, kNtOutput>;
+    if (kHasList && nt == kNtQueriesToo) kernel = block_sparse_fwd_kernel<true, kPlanned, false, kNtQueriesToo>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)ids), dim3(256), 0, s, p);
-    if (hipGetLastError() != hipSuccess) return XATTN_ERR_LAUNCH;
   }
-  return XATTN_OK;
+  return hipGetLastError() == hipSuccess ? XATTN_OK : XATTN_ERR_LAUNCH;
 }
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
