@@ -9,7 +9,7 @@
 int main() {
   int bad = 0;
   const int heads[][3] = {{8, 8, 8}, {32, 8, 8}, {28, 4, 4}, {40, 8, 8}, {5, 3, 3}, {3, 1, 1}, {1, 1, 1}, {32, 0, 0}, {40, 0, 0}, {7, 0, 0}, {96, 8, 8}, {64, 8, 8}};
-  const int tile[][3] = {{64, 64, 512}, {128, 64, 256}, {128, 128, 256}};   // features, tokens, threads
+  const int tile[][3] = {{64, 64, 512}, {128, 64, 256}, {128, 128, 256}, {128, 192, 256}, {128, 256, 256}};   // features, tokens, threads
   long launches = 0, pulled = 0;
   for (const auto& h : heads)
     for (const auto& t : tile)
@@ -18,7 +18,7 @@ int main() {
         const uint32_t mt = (tokens + t[1] - 1) / t[1], total = mt * (uint32_t)((n0 + n1 + n2) / t[0]), per_xcd = (total + 7) / 8;
         if (total > 256) continue;
         ++launches;
-        const uint32_t places = xattn::pull_places(tokens, t[1], total);
+        const uint32_t places = xattn::pull_places(tokens, t[1], t[0], total);
         if (!places) continue;
         ++pulled;
         // one workgroup per CU, tiles included; a CU for every tile's features, half of one where several tiles share them
@@ -44,9 +44,10 @@ int main() {
   std::printf("%ld launches, %ld with pullers\n", launches, pulled);
   // too few CUs left over, which would still pull when the tiles are done: 2 tokens of 224 and 160 tiles, 128 of 224, 192 of 240
   const int late[][3] = {{2, 64, 224}, {2, 64, 160}, {128, 64, 224}, {192, 64, 240}, {2, 64, 256}};
-  for (const auto& c : late) bad += xattn::pull_places(c[0], c[1], c[2]) != 0;
-  // a last token tile with little to load goes ahead of the others by itself
-  const int tails[][4] = {{72, 64, 128, 0}, {111, 64, 128, 0}, {112, 64, 128, 1}, {400, 128, 192, 0}, {500, 128, 192, 1}, {2, 64, 16, 1}};
-  for (const auto& c : tails) bad += (xattn::pull_places(c[0], c[1], c[2]) != 0) != (c[3] != 0);
+  for (const auto& c : late) bad += xattn::pull_places(c[0], c[1], 64, c[2]) != 0;
+  // enough of them, with a last token tile that lacks rows or not: tokens, tile (tokens, features), tiles
+  const int gain[][4] = {{2, 64, 64, 16}, {64, 64, 64, 96}, {72, 64, 64, 128}, {128, 64, 64, 128}, {200, 64, 128, 160}, {330, 64, 128, 144},
+                         {400, 128, 128, 192}, {500, 128, 128, 192}, {1000, 128, 128, 192}, {1400, 192, 128, 192}, {1000, 256, 128, 192}};
+  for (const auto& c : gain) bad += xattn::pull_places(c[0], c[1], c[2], c[3]) == 0;
   return bad || pulled == 0 ? 1 : 0;
 }

@@ -272,7 +272,7 @@ int launch_tiles(const ProjParams& p, unsigned grid, hipStream_t s) {
 template <int NB, int MB, int NS, int KS, bool kRope, bool kMayPull>
 int launch(const ProjParams& p, hipStream_t s) {
   const unsigned tiles = (unsigned)((p.M + 64 * MB - 1) / (64 * MB)) * (unsigned)((p.n[0] + p.n[1] + p.n[2]) / (64 * NB));
-  const unsigned grid = (tiles + 7) / 8 * 8, places = pull_places((uint32_t)p.M, 64 * MB, tiles);
+  const unsigned grid = (tiles + 7) / 8 * 8, places = pull_places((uint32_t)p.M, 64 * MB, 64 * NB, tiles);
   if (kMayPull && places) return launch_tiles<NB, MB, NS, KS, kRope, kMayPull>(p, grid + 8 * places, s);
   return launch_tiles<NB, MB, NS, KS, kRope, false>(p, grid, s);
 }
@@ -288,8 +288,8 @@ int run(const ProjParams& p, void* stream) {
     case k64x64: return launch<1, 1, 6, 2, kRope, true>(p, s);
     case k128x64: return launch<2, 1, 4, 1, kRope, true>(p, s);
     case k128x128: return launch<2, 2, 4, 1, kRope, true>(p, s);
-    case k128x192: return launch<2, 3, 4, 1, kRope, false>(p, s);
-    case k128x256: return launch<2, 4, 3, 1, kRope, false>(p, s);
+    case k128x192: return launch<2, 3, 4, 1, kRope, true>(p, s);
+    case k128x256: return launch<2, 4, 3, 1, kRope, true>(p, s);
     case k128x128Twice: return launch<2, 2, 2, 1, kRope, false>(p, s);
     default: return XATTN_ERR_SHAPE;
   }
