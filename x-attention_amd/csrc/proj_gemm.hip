@@ -284,15 +284,16 @@ bool stride_ok(int64_t sn, int width) { return sn >= width && sn <= ((int64_t)1 
 template <bool kRope>
 int run(const ProjParams& p, void* stream) {
   hipStream_t s = static_cast<hipStream_t>(stream);
-  switch (tile_for(p.M, (int64_t)p.n[0] + p.n[1] + p.n[2], kRope)) {
-    case k64x64: return launch<1, 1, 6, 2, kRope, true>(p, s);
-    case k128x64: return launch<2, 1, 4, 1, kRope, true>(p, s);
-    case k128x128: return launch<2, 2, 4, 1, kRope, true>(p, s);
-    case k128x192: return launch<2, 3, 4, 1, kRope, true>(p, s);
-    case k128x256: return launch<2, 4, 3, 1, kRope, true>(p, s);
-    case k128x128Twice: return launch<2, 2, 2, 1, kRope, false>(p, s);
-    default: return XATTN_ERR_SHAPE;
+  const Tile tile = tile_for(p.M, (int64_t)p.n[0] + p.n[1] + p.n[2], kRope);
+  if (tile == k64x64) return launch<1, 1, 6, 2, kRope, true>(p, s);
+  if (tile == k128x64) return launch<2, 1, 4, 1, kRope, true>(p, s);
+  if (tile == k128x128) return launch<2, 2, 4, 1, kRope, true>(p, s);
+  if (tile == k128x192) return launch<2, 3, 4, 1, kRope, true>(p, s);
+  if constexpr (kRope) {        // (tile_for: q, k and v alone)
+    if (tile == k128x256) return launch<2, 4, 3, 1, kRope, true>(p, s);
+    if (tile == k128x128Twice) return launch<2, 2, 2, 1, kRope, false>(p, s);
   }
+  return XATTN_ERR_SHAPE;
 }
 }  // namespace
 
