@@ -47,6 +47,32 @@ def test_few_units(q_len, k_len, heads, kv_heads, causal):
     check(q_len, k_len, heads, kv_heads, causal)
 
 
+# queries as [tokens][heads] views, keys and values inside a larger cache, the output inside a larger buffer; and q-blocks spread over
+# launches, which have the whole call's bits (halves are the whole problem's choice, not a launch's)
+@pytest.mark.parametrize("q_len,k_len,heads,kv_heads,causal", [(500, 500, 32, 8, True), (513, 1300, 16, 2, True), (1000, 1000, 8, 8, False), (129, 2048, 28, 4, True)])
+def test_few_units_of_strided_views_and_in_windows(q_len, k_len, heads, kv_heads, causal):
+    from xattn.src.Xattention import block_sparse_attention
+
+    g = torch.Generator(device="cuda").manual_seed(q_len * 3 + k_len)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    q = rnd(1, q_len, heads, 128).transpose(1, 2)
+    cache = rnd(2, 1, kv_heads, k_len + 77, 128)
+    k, v = cache[0, :, :, :k_len], cache[1, :, :, :k_len]
+    nq, nk = -(-q_len // 128), -(-k_len // 128)
+    idx = torch.arange(nk, dtype=torch.int32, device="cuda").expand(heads, nq, nk).contiguous()
+    last = (torch.arange(nq, device="cuda").add(1).mul(128).clamp(max=q_len) - 1 + k_len - q_len) // 128 + 1 if causal else torch.full((nq,), nk, device="cuda")
+    cnt = last.int().expand(heads, nq).contiguous()
+    cnt[0, 0] = 0
+    want = block_sparse_attention(q.contiguous(), k.contiguous(), v.contiguous(), idx, cnt, causal=causal)
+    wide = torch.full((1, q_len, heads + 3, 128), 7.0, dtype=torch.bfloat16, device="cuda")
+    got = block_sparse_attention(q, k, v, idx, cnt, causal=causal, out=wide[:, :, 1:heads + 1])
+    assert torch.equal(got, want) and (wide[:, :, 0] == 7).all() and (wide[:, :, heads + 1:] == 7).all()
+    parts = torch.empty(1, q_len, heads, 128, dtype=torch.bfloat16, device="cuda")
+    for a in range(nq):
+        block_sparse_attention(q, k, v, idx, cnt, causal=causal, out=parts, q_blocks=(a, a + 1))
+    assert torch.equal(parts.transpose(1, 2), want)
+
+
 # 24 MiB of output and the first token count beyond, of both kernels (without causality: 64 rows), and a ragged end; with a KV head per
 # query head 30 MiB and the first beyond, from which queries are loaded not temporal, too
 @pytest.mark.parametrize("q_len,k_len,heads,kv_heads,causal", [
