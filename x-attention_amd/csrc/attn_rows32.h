@@ -184,7 +184,7 @@ __device__ __forceinline__ void sweep_unit(const AttnParams& p, const Unit& u, i
     // eighth-of-a-tile copies are its own 32 query rows, and read back as fragments before V_0 is requested.
     int voffQ[8];
     tile_offsets(p.q_sn, lane, rows, voffQ);
-    copy_tile<kNt == kNtQueriesToo ? kLoadNt : 0>(qbase, p.q_sn, p.Lq, u.qb, voffQ, Vs, wave);
+    copy_tile<kNt == kNtQueriesToo ? kNotTemporal : 0>(qbase, p.q_sn, p.Lq, u.qb, voffQ, Vs, wave);
     if (n_blocks > 0) {
       kb = kHasList ? clamp_block(first, p.nkb) : first;
       copy_tile(kbase, p.k_sn, p.Lk, kb, voffK, Ks, wave);

@@ -278,7 +278,7 @@ __device__ __forceinline__ void store_out(const AttnParams& p, int head, int qb,
   for (int i = 0; i < 8; ++i) {
     const int row = i * 4 + (lane >> 4);
     const u32x4 w = *reinterpret_cast<const u32x4*>(stage + row * 256 + ((c ^ (row & 15)) << 4));
-    __builtin_amdgcn_raw_buffer_store_b128(w, ores, (int)(voff0 + (uint32_t)(i * 4) * row_bytes), 0, kNt ? kLoadNt : 0);
+    __builtin_amdgcn_raw_buffer_store_b128(w, ores, (int)(voff0 + (uint32_t)(i * 4) * row_bytes), 0, kNt ? kNotTemporal : 0);
   }
 }
 

@@ -110,10 +110,11 @@ bool xattn::attention_queued(int num_heads, int q_len, int k_len, int causal) {
 }
 
 // Whether a unit is two workgroups', of 64 rows each, with a wavefront for half of every tile's keys: where units leave half of the
-// CUs idle.  Only where lists are never cut; it depends on the whole problem alone.  A prompt of 500 tokens 23.3 -> 21.5 us,
-// 1000 with 8 heads 25.9 -> 23.1, 900 with 16 29.2 -> 25.6.  Two such workgroups on a CU gain where lists are long and lose where
-// they are short (192 units 32 heads 26.5 -> 24.5 us, 168 units of 28 heads 22.5 -> 23.6, 252 28.4 -> 31.3).  Dense attention without
-// lists has whole units always: the sums' order differs, and its q-blocks are those of a longer prompt to the bit.
+// CUs idle.  Only up to 16 key blocks, where no list is ever cut (plan_shape); it depends on the whole problem alone.  A prompt of 500
+// tokens 23.3 -> 21.5 us, 1000 with 8 heads 25.9 -> 23.1, 900 with 16 29.2 -> 25.6.  Two such workgroups on a CU gain where lists are
+// long and lose where they are short (192 units 32 heads 26.5 -> 24.5 us, 168 units of 28 heads 22.5 -> 23.6, 252 28.4 -> 31.3).
+// Dense attention without lists has whole units always: the sums' order differs, and its q-blocks are those of a longer prompt to the
+// bit.  (With lists they are not, across this line: the same q-blocks in a call of more heads or tokens may differ in the last bits.)
 static bool in_halves(int H, int nqb, int nkb) { return nkb <= 16 && (int64_t)H * nqb <= 128; }
 
 // Bytes of output from which the 32-row kernel stores its rows not temporal: they then leave the memory-side cache to q, k and v, which

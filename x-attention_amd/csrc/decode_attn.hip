@@ -80,7 +80,7 @@ __device__ __forceinline__ void dec_copy(const __bf16* base, int64_t sn, int len
       (void*)(base + (int64_t)t * kDecKeys * sn), 0, (int)((int64_t)rows * sn * 2), 0x00020000);
 #pragma unroll
   for (int i = 0; i < 8; ++i)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(slot + i * 1024), 16, voff[i], 0, 0, kNt ? kLoadNt : 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(slot + i * 1024), 16, voff[i], 0, 0, kNt ? kNotTemporal : 0);
 }
 
 template <bool kNt>

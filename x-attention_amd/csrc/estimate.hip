@@ -785,10 +785,11 @@ namespace {
 //   5 us + steps * 1.75 us * ceil(tiles / 256),
 // with a head's rows in tiles of their own or packed with those of the other heads of its KV group, or, with 0.65 of a
 // tile's time for a half and 6 us for the second launch, the last of them as half tiles.
-// The constants are fits to measured times of the passes over 200 .. 16384 tokens and chunks of 64 .. 8000 tokens on
-// 8700 .. 100000 cached ones, stride 8 and 16 (us, 256x256 / chosen): 1000 tokens, stride 16: 45.2 / 10.6 (MT 1);
-// 2000, stride 8: 31.1 / 9.8 (MT 2, 3 stages); 4096, stride 8: 35.0 / 19.2; 8192, stride 16: 60.9 / 31.6;
-// 16384, stride 16: 117.9 / 96; 15000, stride 8: 147.5 (stays).
+// The constants are fits to measured times (MT 1's before its fragments were read a step ahead, 0.16 us a step since)
+// of the passes over 200 .. 16384 tokens and chunks of 64 .. 8000 tokens on 8700 .. 100000 cached ones, stride 8 and 16
+// (us, 256x256 / chosen): 1000 tokens, stride 16: 45.2 / 10.6 (MT 1; 9.2 since); 2000, stride 8: 31.1 / 9.8 (MT 2, 3
+// stages); 4096, stride 8: 35.0 / 19.2; 8192, stride 16: 60.9 / 31.6; 16384, stride 16: 117.9 / 96; 15000, stride 8:
+// 147.5 (stays).
 struct SmallVariant {
   int mt, ns;
   float lat, per_tile;

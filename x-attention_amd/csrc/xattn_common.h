@@ -15,9 +15,10 @@ typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t u32x2;
 constexpr int kWave = 64;
 constexpr int kHeadDim = 128;
 constexpr float kLog2e = 1.4426950408889634f;
-// Cache policy of a buffer load, "not temporal" (the instruction's nt bit): for what one CU reads once.  256 CUs stream 256 MiB at
-// 6.2 to 6.4 TB/s with it, at 5.1 to 5.5 without, whatever is in flight beyond 16 KiB per CU.
-constexpr int kLoadNt = 2;
+// Cache policy of a buffer load or store, "not temporal" (the instruction's nt bit): for what is read once, or not read
+// again soon.  256 CUs stream 256 MiB at 6.2 to 6.4 TB/s with it, at 5.1 to 5.5 without, whatever is in flight beyond
+// 16 KiB per CU.
+constexpr int kNotTemporal = 2;
 
 // D[32x32] += A[32x16] * B[16x32], bf16 in, fp32 accumulate.
 // Lane l (r = l % 32, h = l / 32) supplies A[r][8h..8h+7] and B[8h..8h+7][r];
