@@ -1,6 +1,7 @@
 // Host-only check of the workgroup map.  At chosen sizes launches of few q-blocks give all eight XCDs work, none more than twice the
 // mean rounded up.  At all sizes of up to 130 q-blocks and 26 head layouts every (head, q-block) comes once, the ids of a unit share
-// their KV head, and no XCD has more than the fullest of units of 64.  Exit status 0 when all hold.  No GPU call is made.
+// their KV head, and no XCD has more than the fullest of units of 64, and small
+// units have no ids without work.  Exit status 0 when all hold.  No GPU call is made.
 #include <cstdio>
 #include <vector>
 
@@ -34,7 +35,8 @@ int main() {
       const xattn::DispatchShape d = xattn::dispatch_shape(H, Hkv, n);
       xattn::DispatchShape whole = d;
       whole.unit_rows = 64 / d.set_heads;
-      whole.unit_shift = 6;
+      whole.unit_size = 64;
+      whole.unit_inv = 1u << 25;
       std::vector<int> seen((size_t)H * n, 0);
       auto fullest = [&](const xattn::DispatchShape& s, bool check) {
         std::vector<int> on(8, 0);
@@ -46,13 +48,23 @@ int main() {
           if (!check) continue;
           ++seen[(size_t)head * n + qb - begin];
           int other_head, other_qb, other_kv;                   // the unit's first id has work if any of its has
-          const long first = ((id >> 3) >> s.unit_shift << s.unit_shift << 3) + (id & 7);
+          const long first = ((id >> 3) / s.unit_size * s.unit_size << 3) + (id & 7);
           wrong += !xattn::map_workgroup((int)first, s, begin, begin + n, &other_head, &other_qb, &other_kv) || other_kv != kv || kv != head / (H / Hkv);
         }
         for (int v : on) most = v > most ? v : most;
         return wrong ? 1 << 30 : most;
       };
       const int now = fullest(d, true), then = fullest(whole, false);
+      // where runs are few, units of up to 32 have no ids without work between those with (they would cost their CUs a turn), but for
+      // a run that lacks rows
+      int gaps = 0;
+      if ((n + whole.unit_rows - 1) / whole.unit_rows < 8 && n % d.unit_rows == 0 && d.set_heads * d.unit_rows <= 32)
+        for (long id = 0; id < 8L * (d.n_groups * (n / d.unit_rows) / 8) * d.unit_size; ++id) {
+          int head, qb, kv;
+          gaps += d.sets == 1 && !xattn::map_workgroup((int)id, d, begin, begin + n, &head, &qb, &kv);
+        }
+      if (gaps) std::printf("H=%d Hkv=%d q-blocks %d: %d ids without work\n", H, Hkv, n, gaps);
+      bad += gaps != 0;
       int wrong = 0;
       for (int v : seen) wrong += v != 1;
       if (wrong || now > then) std::printf("H=%d Hkv=%d q-blocks %d: wrong %d, fullest XCD %d, of whole units %d\n", H, Hkv, n, wrong, now, then);
@@ -60,6 +72,6 @@ int main() {
     }
   // runs that are even already keep whole units
   const xattn::DispatchShape whole = xattn::dispatch_shape(24, 24, 313), one = xattn::dispatch_shape(24, 24, 40);
-  bad += whole.unit_rows != 64 || whole.unit_shift != 6 || one.unit_rows != 40;
+  bad += whole.unit_rows != 64 || whole.unit_size != 64 || one.unit_rows != 40;
   return bad ? 1 : 0;
 }

@@ -71,23 +71,22 @@ __device__ __forceinline__ void tile_offsets(int64_t sn, int lane, int wave, int
   }
 }
 
-
 // Workgroup ids are dealt round-robin to the 8 XCDs, and an XCD (32 CUs, two
-// workgroups each, one L2) starts its workgroups in id order.  The 64 ids that
-// land on one XCD one after the other form a unit: the query heads of ONE KV
-// head times a run of adjacent q-blocks, so everything resident on the XCD
-// streams the same K/V through its L2 at about the same place.  A KV head with
-// more than 64 query heads is dealt as several head sets of equal size (each a
-// dispatch group of its own).  Units are dealt to XCDs in turn; the dispatch
-// group of a unit rotates with the q-block run, so every XCD sees every head
-// equally often (heads differ by orders of magnitude in list length).  Runs go
-// out last (longest, when causal) first, so of eight runs an XCD that sees a
-// head in the first has more of it than one that sees it in the eighth: of the
-// next eight it sees it that much later, the rotation runs backwards.  (Where
-// two of 8 groups keep long lists of 256 q-blocks, an XCD had 20 % more than
-// its share: text of 32768 tokens 1986 us, 1738 with the turn.)  Groups fewer
-// than XCDs rotate every second or fourth run, or half the XCDs would never see
-// a group.
+// workgroups each, one L2) starts its workgroups in id order.  The ids, up to
+// 64, that land on one XCD one after the other form a unit: the query heads of
+// ONE KV head times a run of adjacent q-blocks, so what is resident on the XCD
+// together streams the same K/V through its L2 at about the same place.  A KV
+// head with more than 64 query heads is dealt as several head sets of equal
+// size (each a dispatch group of its own).  Units are dealt to XCDs in turn;
+// the dispatch group of a unit rotates with the q-block run, so every XCD sees
+// every head equally often (heads differ by orders of magnitude in list
+// length).  Runs go out last (longest, when causal) first, so of eight runs an
+// XCD that sees a head in the first has more of it than one that sees it in the
+// eighth: of the next eight it sees it that much later, the rotation runs
+// backwards.  (Where two of 8 groups keep long lists of 256 q-blocks, an XCD
+// had 20 % more than its share: text of 32768 tokens 1986 us, 1738 with the
+// turn.)  Groups fewer than XCDs rotate every second or fourth run, or half the
+// XCDs would never see a group.
 struct DispatchShape {
   int group;       // query heads per KV head
   int sets;        // head sets per KV head (1 unless group > kUnit)
@@ -95,7 +94,8 @@ struct DispatchShape {
   int n_groups;    // dispatch groups: Hkv * sets
   int unit_rows;   // q-blocks per unit
   int turn_shift;  // groups rotate once per 1 << turn_shift runs
-  int unit_shift;  // a unit has 1 << unit_shift ids (kUnit, fewer where runs are few)
+  uint32_t unit_size;   // ids of a unit: kUnit, or as many as it needs where runs are few and that is at most half
+  uint32_t unit_inv;    // 2^31 / unit_size, rounded up: ids are divided by a product
 };
 // (head, q-block)s of the XCD that has most of them, units being dealt to the XCDs in turn.
 inline int64_t fullest_xcd(const DispatchShape& d, int n_qblocks) {
@@ -109,7 +109,7 @@ inline int64_t fullest_xcd(const DispatchShape& d, int n_qblocks) {
 
 // Where a launch has fewer than eight runs, some XCDs may have a unit more than others, or the only ones.  There the number of runs
 // is rounded up to one of which every XCD has as many, if the fullest XCD then has an eighth less to do (q-blocks per unit are rounded up,
-// too, which may leave fewer runs than that, or a short last one); and a unit has no more ids than it needs.
+// too, which may leave fewer runs than that, or a short last one).
 // Prompts, us, whole units / rounded up: 650 tokens with 28 / 4 heads 29.1 / 26.9, 1150 33.7 / 32.0, 3000 (105 workgroups on the fullest XCD, 84)
 // 62.3 / 60.6, video 84.9 / 79.6; lists of about 4 blocks: 8000 tokens of one head 31.3 / 23.3, 4000 of 4 / 1 30.6 / 23.1, 5000 of 12 / 12
 // 38.5 / 33.8.  But 2800 tokens with 28 / 4 (91 and 84) 58.7 / 60.1, such lists 34.6 / 39.7, 5000 (154 and 147) 92.8 / 94.1, 52.8 / 56.4;
@@ -117,6 +117,11 @@ inline int64_t fullest_xcd(const DispatchShape& d, int n_qblocks) {
 // ids that a launch goes round in several times straddle an XCD's 64 places, which costs long lists 2 to 8 % of what evenness gives short ones
 // (3000 of 28 / 4: lists of about 2 blocks 29.5 / 28.0, 4 39.5 / 42.9).  40003 tokens of 24 heads without causality, runs even
 // already, in units of 63 instead of 64 15.57 -> 15.68 ms.
+// And a unit of at most 32 workgroups then has no more ids than it needs.  An XCD deals its workgroups to its 32 CUs in turn, also those without work, so
+// units rounded up to 16 or 32 ids put their work on the same CUs and left others idle (us, 64 ids / a power of two / now, text: 600
+// tokens of 64 / 16 heads 29.0 / 32.6 / 28.9, 1240 of 32 / 16 36.3 / 39.5 / 36.3, 1112 of 32 / 32 38.9 / 39.7 / 36.2, 1240 of 24 / 24 40.0 / 41.0 /
+// 37.0, 984 of 32 / 32 35.0 / 33.4 / 33.4); from 600 units on, of more
+// than 32 ids, and with 8 / 8, 32 / 8, 28 / 4 and 40 / 8 heads, the three are within 1 or 2 %.
 inline DispatchShape dispatch_shape(int H, int Hkv, int n_qblocks) {
   DispatchShape d;
   d.group = H / Hkv;
@@ -134,8 +139,9 @@ inline DispatchShape dispatch_shape(int H, int Hkv, int n_qblocks) {
     if (8 * fullest_xcd(e, n_qblocks) <= 7 * fullest_xcd(d, n_qblocks)) d = e;
   }
   if (d.unit_rows > n_qblocks) d.unit_rows = n_qblocks;
-  d.unit_shift = 0;
-  while (1 << d.unit_shift < d.set_heads * d.unit_rows) ++d.unit_shift;
+  const int work = d.set_heads * d.unit_rows;
+  d.unit_size = (uint32_t)(runs < 8 && work <= kUnit / 2 ? work : kUnit);
+  d.unit_inv = ((1u << 31) + d.unit_size - 1) / d.unit_size;
   return d;
 }
 
@@ -146,7 +152,8 @@ __host__ __device__ inline bool map_workgroup(int id, const DispatchShape& d, in
                                               int* qb, int* kv_head) {
   if (id < 0) return false;
   const uint32_t x = (uint32_t)id & 7u, s = (uint32_t)id >> 3;
-  const uint32_t unit = (s >> d.unit_shift) * 8u + x, w = s & ((1u << d.unit_shift) - 1);
+  const uint32_t at = (uint32_t)((uint64_t)s * d.unit_inv >> 31);      // s / unit_size (exact: s < 2^26 where it is not kUnit)
+  const uint32_t unit = at * 8u + x, w = s - at * d.unit_size;
   const uint32_t ng = (uint32_t)d.n_groups, sh = (uint32_t)d.set_heads;
   const uint32_t run = unit / ng;
   const uint32_t turn = (run & 8u ? ~run : run) & 7u;
@@ -174,7 +181,7 @@ inline bool map_workgroup(int id, int H, int Hkv, int qb_begin, int qb_end, int*
 // grid size of a launch over n_qblocks q-blocks
 inline int64_t grid_for(const DispatchShape& d, int n_qblocks) {
   const int64_t runs = (n_qblocks + d.unit_rows - 1) / d.unit_rows;
-  return ((runs * d.n_groups + 7) / 8 * 8) << d.unit_shift;
+  return (runs * d.n_groups + 7) / 8 * 8 * d.unit_size;
 }
 inline int64_t grid_for(int H, int Hkv, int n_qblocks) { return grid_for(dispatch_shape(H, Hkv, n_qblocks), n_qblocks); }
 
