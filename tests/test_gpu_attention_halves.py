@@ -74,10 +74,12 @@ def test_few_units_of_strided_views_and_in_windows(q_len, k_len, heads, kv_heads
 
 
 # 24 MiB of output and the first token count beyond, of both kernels (without causality: 64 rows), and a ragged end; with a KV head per
-# query head 30 MiB and the first beyond, from which queries are loaded not temporal, too
+# query head 30 MiB and the first beyond, from which queries are loaded not temporal, too, and with fewer
+# KV heads calls of more than 160 MiB
 @pytest.mark.parametrize("q_len,k_len,heads,kv_heads,causal", [
     (3072, 3072, 32, 8, True), (3073, 3073, 32, 32, True), (3073, 3400, 32, 8, False), (3519, 3519, 28, 4, True),
     (3840, 3840, 32, 32, True), (3841, 3841, 32, 32, True), (1921, 6000, 64, 64, True),
+    (3100, 14280, 32, 16, True), (3100, 14300, 32, 16, True), (5500, 5500, 40, 20, True),
 ])
 def test_large_outputs(q_len, k_len, heads, kv_heads, causal):
     check(q_len, k_len, heads, kv_heads, causal)

@@ -125,15 +125,22 @@ static bool in_halves(int H, int nqb, int nkb) { return nkb <= 16 && (int64_t)H 
 // Not in the 64-row kernel, whose lists are long: video of 65536 tokens 15306 -> 15366 us, text of 131072 14373 -> 14405, of 50000 2650 ->
 // 2675, fields equal.
 constexpr int64_t kOutNtBytes = 24 << 20;
-// ... and from which the queries of calls with a KV head per query head are loaded so too, of 32 heads, text at two strides: 3100 tokens
-// 67.1 -> 70.8, 68.7 -> 71.4, 3500 75.5 -> 76.2, 76.4 -> 77.9, 3900 86.4 -> 86.3, 83.1 -> 82.0, 4300 101.5 -> 97.5, 98.8 -> 97.5, 5500 123.7 -> 121.2,
-// 116.5 -> 115.4, 8000 183.9 -> 183.0, 161.7 -> 160.4, 13000 327.6 -> 327.0, 294.1 -> 292.2; of 24 5000 equal, 6500 117.5 -> 116.7.  With fewer KV
-// heads most calls are slower: 28 / 4 2000 41.2 -> 45.0, video of 6000 204.9 -> 211.2, of 8000 332 -> 338, 32 / 8 5000 117.1 -> 124.8.
+// Calls that load their queries so, too, where the estimate has read them and the attention reads them for the last time.  With a KV
+// head per query head from so many bytes of output on, of 32 heads, text at two strides: 3100 tokens 67.1 -> 70.8, 68.7 -> 71.4, 3500 75.5 ->
+// 76.2, 76.4 -> 77.9, 3900 86.4 -> 86.3, 83.1 -> 82.0, 4300 101.5 -> 97.5, 98.8 -> 97.5, 5500 123.7 -> 121.2, 116.5 -> 115.4, 8000 183.9 -> 183.0,
+// 161.7 -> 160.4, 13000 327.6 -> 327.0, 294.1 -> 292.2; of 24 5000 equal, 6500 117.5 -> 116.7.
 constexpr int64_t kQueriesNtBytes = 30 << 20;
+// With fewer KV heads from so many bytes of q, k, v and output on: below, all of a call stays in the memory-side cache beside what
+// came before it, and queries loaded so leave it (28 / 4 2000 tokens 41.2 -> 45.0, video of 6000 204.9 -> 211.2, of 8000 332 -> 338, 32 / 8 5000
+// 117.1 -> 124.8, 3500 on 5000 112.6 -> 116.7; 97 to 140 MiB).  Above, three or six inputs in turn: 9000 of 32 / 8 206.9 -> 201.2, 11000
+// 240 -> 236, 14000 of 28 / 4 219 -> 211, 5836 on 13528 136.9 -> 131.5, 4000 on 30000 145.4 -> 141.9, 7000 on 20000 215.0 -> 210.6; 8000 on 20000,
+// 4000 on 60000 and video of 10000 to 16000 equal.  (One input again and again, up to 256 MiB of which stay, would be 3 to 10 % slower.)
+constexpr int64_t kCallNtBytes = 160 << 20;
 
 static int not_temporal(const AttnParams& p, bool lists) {
-  const int64_t bytes = (int64_t)p.H * p.Lq * kHeadDim * 2;
-  return bytes <= kOutNtBytes ? kNtNone : lists && p.H == p.Hkv && bytes > kQueriesNtBytes ? kNtQueriesToo : kNtOutput;
+  const int64_t bytes = (int64_t)p.H * p.Lq * kHeadDim * 2, call = 2 * bytes + (int64_t)p.Hkv * p.Lk * kHeadDim * 4;
+  if (bytes <= kOutNtBytes) return kNtNone;
+  return lists && (p.H == p.Hkv ? bytes > kQueriesNtBytes : call > kCallNtBytes) ? kNtQueriesToo : kNtOutput;
 }
 
 // `ids` units and pieces; with a queue, `places` workgroups of the 64-row kernel.
