@@ -2,30 +2,32 @@
 // hidden state; q, k and v in one launch with the rotation of q and k in its epilogue, or the output projection.
 //
 // Bound: with at most a tile per CU, by how fast one CU fills its LDS (a CU has 32 KiB of loads in flight, whatever is asked of
-// it: 76 GB/s from memory, 130 from the L2), so the tile is the largest that still gives most CUs one: 64 x 64 up to 256 tiles,
-// then 64 tokens x 128 features, 128 x 128, 192 x 128 and, for q, k and v, 256 x 128.  CUs left over may pull the
-// weights into the L2 (proj_pull.h; weights from memory: q, k, v of 64 tokens, 4096 wide, 22.3 -> 20.8 us, of 192 30.5 -> 27.7, of
-// 512 40.7 -> 39.9; the output of 320, 5120 wide, 38.3 -> 34.0).  The larger
-// tiles took the place of two 128 x 128 ones per CU (4096 wide, 700 tokens 65 -> 46 us, 1000 72 -> 57, 1280 75 -> 64).
-// Splitting a step's depth over two groups of wavefronts helps the smallest tile only (17.6 -> 13.3 us at 64 tokens), where the
-// chain of 64 steps is the time; on the larger ones, where it would save a third of the LDS reads, it is 1 to 8 % slower.
+// it: at most 76 GB/s from memory, 130 from the L2), so the tile is the largest that still gives most CUs one: 64 x 64 up to 256
+// tiles, then 64 tokens x 128 features, 128 x 128, 192 x 128 and, for q, k and v, 256 x 128.  CUs left over may pull the weights
+// into the L2 (proj_pull.h; weights from memory: q, k, v of 64 tokens, 4096 wide, 22.9 -> 19.9 us, of 192 30.8 -> 23.1, of 512
+// 40.8 -> 33.6; the output of 320, 5120 wide, 38.8 -> 30.9).  Whole products stay below those rates: the tiles of those 512 tokens
+// copy 2.1 MB each, 51 GB/s without pullers and 62 with them; where the rest goes (start, first slab, barriers, epilogue) has not
+// been measured.  The larger tiles took the place of two 128 x 128 ones per CU (4096 wide, 700 tokens 66 -> 45 us, 1000 72 -> 57,
+// 1280 73 -> 63).  Splitting a step's depth over two groups of wavefronts helps the smallest tile only (17.6 -> 13.3 us at 64
+// tokens), where the chain of 64 steps is the time; on the larger ones, where it would save a third of the LDS reads, it is 1 to 8 %
+// slower.
 //
-// Library products against this kernel, weights from memory, us (the library's in a captured graph).  q, k, v (three launches,
+// Library products against this kernel, weights from memory, one box, in turn, in captured graphs, us.  q, k, v (three launches,
 // and 4 to 5 for the rotation) by tokens:
-//   width, heads      64         200        500        700        1000       1280       1500
-//   1024   8 + 2*8    27 / 7     27 / 7     28 / 9     30 / 12    30 / 14    33 / 15    34 / 19
-//   2048   32 + 2*8   36 / 11.5  38 / 15    43 / 21    50 / 28    53 / 34    59 / 37    library
-//   3584   28 + 2*4   40 / 16    42 / 20.5  50 / 29    67 / 32    71 / 43    81 / 47    82 / 54
-//   4096   32 + 2*8   46 / 18.5  48 / 24.5  63 / 34    75 / 46    87 / 57    100 / 64   library
-//   5120   40 + 2*8   60 / 25    61 / 34    89 / 49    105 / 60   118 / 74   library
-//   8192   64 + 2*8   62 / 45    95 / 61    134 / 94   165 / 119  library
-// Output (features x depth): 1024 x 1024 8.8 / 6.6, 8.4 / 6.5, 8.6 / 6.7, 9.1 / 6.7, 9.0 / 7.5, 9.6 / 7.9, 9.6 / 8.0;
-// 4096 x 4096 14.4 / 16.3, 20.8 / 17.5, 28 / 28.3, 31 / 32, 39 / 39, 49 / 46, 52 / 51; 3072 x 3072 16 / 13, 17.5 / 12.7,
-// 21 / 18.4, 26 / 23, 29.5 / 26, 32 / 30, 41 / 35; 8192 x 8192 33 / 42, 53 / 51, 81 / 75, 98 / 96.  Up to 64 tokens there is a single
-// row of tiles, each a chain over the whole depth, which the library splits; so it does where the features are fewer than the
-// depth.  Such a turn is bound by the host's calls, though, and the library's is the dearer one: the whole layer, 4096 wide, on
-// 6000 tokens with the library's output product / this kernel's before weights were pulled ahead, 2 tokens 70 / 62, 16 68 / 64,
-// 64 68 / 74.5, 100 68 / 68.
+//   width, heads      64          200         500         700         1000        1280        1500
+//   1024   8 + 2*8    37 / 7.8    34 / 7.6    35 / 9.6    37 / 12.5   38 / 13.4   40 / 14.3   41 / 18
+//   2048   32 + 2*8   36 / 12.3   38 / 14.9   44 / 20     51 / 26.2   53 / 32     58 / 36     library
+//   3584   28 + 2*4   42 / 17.5   43 / 20.4   50 / 28     70 / 30     73 / 41     83 / 45     85 / 52
+//   4096   32 + 2*8   47 / 20.4   49 / 24.6   64 / 33     76 / 43     86 / 55     98 / 62     library
+//   5120   40 + 2*8   60 / 26.7   61 / 35     90 / 48     107 / 57    118 / 71    library
+//   8192   64 + 2*8   64 / 51     98 / 64     133 / 90    165 / 114   library
+// Output (features x depth), by the same tokens: 1024 x 1024 11.3 / 6.7, 10.4 / 6.5, 10.6 / 6.7, 11.1 / 6.8, 11.2 / 7.5, 11.7 / 8,
+// 11.8 / 8.2; 3072 x 3072 15.7 / 14.4, 17.2 / 12.7, 20.4 / 17.8, 25.2 / 22.5, 29.2 / 23.9, 31 / 29.1, 38 / 32; 4096 x 4096 15 /
+// 18.2, 21.9 / 16.9, 28.7 / 28.4, 32 / 29.5, 41 / 38, 46 / 44, 50 / 49; 5120 x 5120 21.6 / 24.1, 28.8 / 26.7, 49 / 36, 51 / 44, 63
+// / 55; 8192 x 8192 35 / 47, 54 / 52, 81 / 75, 98 / 94.  Up to 64 tokens there is a single row of tiles, each a chain over the
+// whole depth, which the library splits; so it does where the features are fewer than the depth.  Such a turn is bound by the
+// host's calls, though, and the library's is the dearer one: the whole layer, 4096 wide, on 6000 tokens with the library's output
+// product / this kernel's before weights were pulled ahead, 2 tokens 70 / 62, 16 68 / 64, 64 68 / 74.5, 100 68 / 68.
 #include "lds_limit.h"
 #include "proj_pull.h"
 #include "rotate.h"
