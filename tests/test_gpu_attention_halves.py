@@ -73,6 +73,16 @@ def test_few_units_of_strided_views_and_in_windows(q_len, k_len, heads, kv_heads
     assert torch.equal(parts.transpose(1, 2), want)
 
 
+# few runs of small units, which have as many ids as workgroups, of 1, 11, 12, 18, 20 and 32, and of 34, which have 64 ids: several
+# to an XCD, KV groups, lists that may be cut, the 64-row kernel with its work queue, a run that lacks rows
+@pytest.mark.parametrize("q_len,k_len,heads,kv_heads,causal", [
+    (100, 3000, 200, 200, True), (1300, 1300, 24, 24, True), (1112, 1112, 32, 16, True), (600, 600, 64, 16, True), (4096, 4096, 8, 8, True),
+    (2100, 2100, 32, 16, True), (2500, 2500, 64, 64, False), (1500, 4000, 12, 12, True), (2000, 2000, 14, 2, True),
+])
+def test_few_runs_of_small_units(q_len, k_len, heads, kv_heads, causal):
+    check(q_len, k_len, heads, kv_heads, causal)
+
+
 # 24 MiB of output and the first token count beyond, of both kernels (without causality: 64 rows), and a ragged end; with a KV head per
 # query head 30 MiB and the first beyond, from which queries are loaded not temporal, too, and with fewer
 # KV heads calls of more than 160 MiB
