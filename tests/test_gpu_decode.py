@@ -109,3 +109,26 @@ def test_decode_at_the_line_between_cache_policies(shape):
     H, Hkv, L = shape
     q, k, v = _mk(H, Hkv, L, L, spread=3.0)
     _check(single_decode_with_kv_cache(q.cuda(), k.cuda(), v.cuda(), kv_layout="HND"), O.single_decode_with_kv_cache(q, k, v, kv_layout="HND"))
+
+
+# caches of one launch (up to 48 tiles of 32 keys, a wavefront every twelfth of them) and the first beyond: tiles that lack keys, fewer
+# tiles than parts and wavefronts, the edges of a wavefront's turns, groups of query heads that fill no copy of four rows, 32 and one;
+# views whose heads and tokens lie apart
+@pytest.mark.parametrize("H,Hkv,L", [
+    (32, 8, 2), (32, 1, 5), (62, 2, 70), (3, 3, 32), (5, 1, 65), (32, 8, 96), (28, 4, 100), (32, 32, 129), (32, 1, 383), (64, 2, 384), (32, 8, 385), (14, 2, 416),
+    (27, 9, 769), (32, 8, 1100), (40, 40, 1505), (32, 8, 1536), (32, 8, 1537), (28, 4, 1569), (130, 130, 1600), (257, 257, 40), (300, 300, 1700),
+])
+def test_decode_of_short_caches(H, Hkv, L):
+    from xattn.src.decode import single_decode_with_kv_cache
+
+    q, k, v = _mk(H, Hkv, L, L + H, spread=3.0)
+    want = O.single_decode_with_kv_cache(q, k, v, kv_layout="HND")
+    out = single_decode_with_kv_cache(q.cuda(), k.cuda(), v.cuda(), kv_layout="HND")
+    _check(out, want)
+    rows = torch.full((2 * H, 136), float("nan"), dtype=torch.bfloat16, device="cuda")
+    rows[::2, :128] = q.cuda()
+    cache = torch.full((2, L + 9, Hkv + 1, 144), float("nan"), dtype=torch.bfloat16, device="cuda")
+    cache[0, :L, :Hkv, :128] = k.cuda().transpose(0, 1)
+    cache[1, :L, :Hkv, :128] = v.cuda().transpose(0, 1)
+    views = single_decode_with_kv_cache(rows[::2, :128], cache[0, :L, :Hkv, :128], cache[1, :L, :Hkv, :128], kv_layout="NHD")
+    assert torch.equal(views, out)

@@ -17,7 +17,7 @@
 // the prefill kernel and its accumulators feed O^T += V^T P^T unchanged.  The
 // four wavefronts combine (max, sum, unnormalised output) of their key ranges in
 // LDS and write one partial result per workgroup; a second small kernel merges
-// the workgroups of a head.
+// the workgroups of a head.  Short caches take one launch (decode_short_kernel).
 //
 // Keys and values of large caches are loaded "not temporal" (kNtBytes).
 #include <mutex>
@@ -48,17 +48,17 @@ struct DecodeParams {
   float* part;
   int64_t q_sh, k_sh, k_sn, v_sh, v_sn, o_sh;   // element strides
   int H, Hkv, group, Lk;
-  int n_tiles, tiles_per_wave, ranges_per_head;   // ranges_per_head is a multiple of kDecWaves
+  int n_tiles, wgs;            // tiles of the cache, workgroups of a KV head
+  int per_wave, longer;        // tiles of a wavefront, and how many wavefronts of a head have one more
   float scale_log2;
 };
 
 __device__ __forceinline__ int dec_swz(int n) { return ((n & 3) << 2) | ((n >> 2) & 3); }
 
-// waits until at most 32 of this wavefront's buffer loads are outstanding
-// (loads complete in order, so everything older than the newest four tiles has
-// landed in LDS); other counters untouched
-__device__ __forceinline__ void wait_vm32() {
-  __builtin_amdgcn_s_waitcnt(0x8F70);
+// waits until at most kLeft of this wavefront's buffer loads are outstanding (loads complete in order); other counters untouched
+template <int kLeft>
+__device__ __forceinline__ void wait_vm() {
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (kLeft & 15) | (kLeft >> 4) << 14);
   asm volatile("" ::: "memory");
 }
 __device__ __forceinline__ void wait_lgkm0() {
@@ -66,18 +66,13 @@ __device__ __forceinline__ void wait_lgkm0() {
   asm volatile("" ::: "memory");
 }
 
-// One 32-key tile, global -> this wavefront's LDS slot.  Tiles outside
-// [0, n_tiles) are issued with an empty buffer resource: they move no data but
-// keep the count of outstanding loads the same on every iteration.
+// One 32-key tile, global -> this wavefront's LDS slot.
 template <bool kNt>
-__device__ __forceinline__ void dec_copy(const __bf16* base, int64_t sn, int len, int tile, int n_tiles,
-                                         const int (&voff)[8], char* slot) {
-  const bool live = tile < n_tiles;
-  const int t = live ? tile : 0;
-  const int rows_left = len - t * kDecKeys;
-  const int rows = live ? (rows_left < kDecKeys ? rows_left : kDecKeys) : 0;
+__device__ __forceinline__ void dec_copy(const __bf16* base, int64_t sn, int len, int tile, const int (&voff)[8], char* slot) {
+  const int rows_left = len - tile * kDecKeys;
+  const int rows = rows_left < kDecKeys ? rows_left : kDecKeys;
   const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(base + (int64_t)t * kDecKeys * sn), 0, (int)((int64_t)rows * sn * 2), 0x00020000);
+      (void*)(base + (int64_t)tile * kDecKeys * sn), 0, (int)((int64_t)rows * sn * 2), 0x00020000);
 #pragma unroll
   for (int i = 0; i < 8; ++i)
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(slot + i * 1024), 16, voff[i], 0, 0, kNt ? kNotTemporal : 0);
@@ -92,13 +87,12 @@ __global__ __launch_bounds__(256, 1) void decode_partial_kernel(DecodeParams p) 
   // LDS slots derived from it are then uniform values for the compiler too
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 31, hh = lane >> 5;
-  const int wgs_per_head = p.ranges_per_head / kDecWaves;
-  const int kvh = blockIdx.x / wgs_per_head;
-  const int range = (blockIdx.x % wgs_per_head) * kDecWaves + wave;
-  const int t0 = range * p.tiles_per_wave;
-  int t1 = t0 + p.tiles_per_wave;
-  t1 = t1 < p.n_tiles ? t1 : p.n_tiles;
-  const int n = t1 > t0 ? t1 - t0 : 0;
+  const int kvh = blockIdx.x / p.wgs, wg = blockIdx.x - kvh * p.wgs;
+  // the wavefronts' ranges differ by a tile at most, and a workgroup's lie apart (131072 keys of 4 KV heads 54.7 us with its four one
+  // after the other, 50.9 so; the longer ones are spread over the workgroups)
+  const int range = wave * p.wgs + wg;
+  const int t0 = range * p.per_wave + (range < p.longer ? range : p.longer);
+  const int n = p.per_wave + (range < p.longer ? 1 : 0);
 
   char* ring = ring_all + wave * (kDecSlots * kDecTileBytes);
   // the same place as an LDS byte address
@@ -106,19 +100,6 @@ __global__ __launch_bounds__(256, 1) void decode_partial_kernel(DecodeParams p) 
                             (uint32_t)(wave * (kDecSlots * kDecTileBytes));
   const __bf16* kbase = p.k + (int64_t)kvh * p.k_sh;
   const __bf16* vbase = p.v + (int64_t)kvh * p.v_sh;
-
-  // Q^T fragments: lane r holds query head kvh*group + r (zeros beyond the group)
-  bf16x8 qreg[8];
-  {
-    const bool live = r < p.group;
-    const __bf16* src = p.q + (int64_t)(kvh * p.group + (live ? r : 0)) * p.q_sh + hh * 8;
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      bf16x8 x = *reinterpret_cast<const bf16x8*>(src + s * 16);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) qreg[s][e] = live ? x[e] : (__bf16)0.f;
-    }
-  }
 
   int voffK[8], voffV[8];
 #pragma unroll
@@ -151,23 +132,52 @@ __global__ __launch_bounds__(256, 1) void decode_partial_kernel(DecodeParams p) 
     for (int v = 0; v < 16; ++v) oacc[i][v] = 0.f;
   float m_run = -INFINITY, l_run = 0.f;
 
-  // load number j of the sequence K_0 V_0 K_1 V_1 ... goes to slot j % 5
-  const int t_end = t0 + n;
-  dec_copy<kNt>(kbase, p.k_sn, p.Lk, t0, t_end, voffK, ring + 0 * kDecTileBytes);
-  dec_copy<kNt>(vbase, p.v_sn, p.Lk, t0, t_end, voffV, ring + 1 * kDecTileBytes);
-  dec_copy<kNt>(kbase, p.k_sn, p.Lk, t0 + 1, t_end, voffK, ring + 2 * kDecTileBytes);
-  dec_copy<kNt>(vbase, p.v_sn, p.Lk, t0 + 1, t_end, voffV, ring + 3 * kDecTileBytes);
+  // The query heads' rows, then load number j of the sequence K_0 V_0 K_1 V_1 ... to slot j % 5.  A CU takes a load of 1 KiB every 20
+  // clk, whether it moves anything or not, so none is issued past the range's end (with loads of empty resources there, and the queries
+  // read row by row, 32 loads a wavefront ahead of the first tile, a step on 1100 keys took 7.6 us instead of 7.0).
+  bf16x8 qreg[8];
+  if (n > 0) {
+    char* const rows = ring + 4 * kDecTileBytes;
+#pragma unroll 1
+    for (int i = 0; i < p.group; i += 4) {
+      const int row = i + (lane >> 4), src = row < p.group ? row : p.group - 1;
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(p.q + (int64_t)(kvh * p.group + src) * p.q_sh + ((lane & 15) ^ dec_swz(row)) * 8),
+                                       (lds_ptr_t)(rows + i * 256), 16, 0, 0);
+    }
+    dec_copy<kNt>(kbase, p.k_sn, p.Lk, t0, voffK, ring + 0 * kDecTileBytes);
+    dec_copy<kNt>(vbase, p.v_sn, p.Lk, t0, voffV, ring + 1 * kDecTileBytes);
+    if (n > 1) {
+      dec_copy<kNt>(kbase, p.k_sn, p.Lk, t0 + 1, voffK, ring + 2 * kDecTileBytes);
+      dec_copy<kNt>(vbase, p.v_sn, p.Lk, t0 + 1, voffV, ring + 3 * kDecTileBytes);
+      wait_vm<32>();
+    } else {
+      wait_vm<16>();
+    }
+    // Q^T fragments: lane r holds query head kvh*group + r (zeros beyond the group)
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const bf16x8 x = *reinterpret_cast<const bf16x8*>(rows + kaddr[s]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) qreg[s][e] = r < p.group ? x[e] : (__bf16)0.f;
+    }
+  }
 
   int slot = 0;   // slot of K_i
   for (int i = 0; i < n; ++i) {
-    const int tile = t0 + i;
+    const int tile = t0 + i, behind = n - 1 - i;
     char* Kt = ring + slot * kDecTileBytes;
     const int sv = slot + 1 >= kDecSlots ? slot + 1 - kDecSlots : slot + 1;
-    const int s4 = slot + 4 >= kDecSlots ? slot + 4 - kDecSlots : slot + 4;   // freed by V_{i-1}
+    const int s4 = slot + 4 >= kDecSlots ? slot + 4 - kDecSlots : slot + 4;   // freed by V_{i-1}, at first by the queries
 
     wait_lgkm0();   // this wavefront's reads of the slot about to be refilled have returned
-    dec_copy<kNt>(kbase, p.k_sn, p.Lk, tile + 2, t_end, voffK, ring + s4 * kDecTileBytes);
-    wait_vm32();    // K_i landed
+    if (behind > 1) {
+      dec_copy<kNt>(kbase, p.k_sn, p.Lk, tile + 2, voffK, ring + s4 * kDecTileBytes);
+      wait_vm<32>();    // K_i landed
+    } else if (behind == 1) {
+      wait_vm<24>();
+    } else {
+      wait_vm<8>();
+    }
 
     f32x16 sacc;
 #pragma unroll
@@ -188,7 +198,7 @@ __global__ __launch_bounds__(256, 1) void decode_partial_kernel(DecodeParams p) 
     }
     // K_i is in registers (the MFMAs above consumed every fragment): its slot takes V_{i+2}
     wait_lgkm0();
-    dec_copy<kNt>(vbase, p.v_sn, p.Lk, tile + 2, t_end, voffV, Kt);
+    if (behind > 1) dec_copy<kNt>(vbase, p.v_sn, p.Lk, tile + 2, voffV, Kt);
 
     float mx = -INFINITY;
 #pragma unroll
@@ -212,7 +222,10 @@ __global__ __launch_bounds__(256, 1) void decode_partial_kernel(DecodeParams p) 
     }
     l_run += psum;
 
-    wait_vm32();    // V_i landed
+    // V_i landed
+    if (behind > 1) wait_vm<32>();
+    else if (behind == 1) wait_vm<16>();
+    else wait_vm<0>();
     {
       // The sixteen transposing reads of V_i are issued from one asm statement:
       // an LDS read the compiler can see would make it wait for EVERY buffer
@@ -265,8 +278,6 @@ __global__ __launch_bounds__(256, 1) void decode_partial_kernel(DecodeParams p) 
     }
     slot = slot + 2 >= kDecSlots ? slot + 2 - kDecSlots : slot + 2;
   }
-  wait_vm0();   // nothing is still writing this wavefront's LDS
-
   // The four wavefronts' results meet in LDS (each uses the start of its own,
   // now idle, ring) and leave as one partial result per workgroup.
   const float l_tot = half_sum(l_run);
@@ -318,27 +329,28 @@ __global__ __launch_bounds__(256, 1) void decode_partial_kernel(DecodeParams p) 
 
 // out[h][d] = sum_s w_s O_s[d] / sum_s w_s l_s,  w_s = 2^(m_s - max m), over the
 // head's workgroups s (at most 256).  Bound by the latency of one dependent
-// chain, so everything a thread needs from memory is requested at once: thread t
-// holds (m_s, l_s) of partial result t for the weights, and features 4*(t%32)..
-// of every eighth partial result, eight of them in flight, which do not wait for
-// the weights.  (With a running maximum the loads of one trip waited for the
-// branch of the one before: 3.6 -> 3.0 us for the merge of 9 partial results,
-// 7.1 -> 4.8 us for 64.)
+// chain, so everything a thread needs from memory is requested at once: lane i
+// holds (m_s, l_s) of partial results i, i + 64, .. for the weights, which every
+// wavefront finds for itself (no barrier), and features 4*(t%32).. of every
+// eighth partial result, eight of them in flight, which do not wait for the
+// weights.  (With a running maximum the loads of one trip waited for the branch
+// of the one before: 7.1 -> 4.8 us for the merge of 64.)
 __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p) {
   __shared__ __attribute__((aligned(16))) float accs[8][128];
-  __shared__ float wt[256];
-  __shared__ float wmax[4], wsum[4];
-  const int head = blockIdx.x, tid = threadIdx.x;
+  __shared__ float wt[4][256];
+  const int head = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int kvh = head / p.group, g = head % p.group;
-  const int wgs = p.ranges_per_head / kDecWaves;
+  const int wgs = p.wgs;
   const float* base = p.part + ((int64_t)kvh * wgs * p.group + g) * kPartStride;
   const int64_t step = (int64_t)p.group * kPartStride;
   const int slot = tid >> 5, dg = tid & 31;
 
-  float m = -INFINITY, l = 0.f;
-  if (tid < wgs) {
-    m = base[tid * step + 128];
-    l = base[tid * step + 129];
+  float m[4], l[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int s = lane + 64 * u;
+    m[u] = s < wgs ? base[s * step + 128] : -INFINITY;
+    l[u] = s < wgs ? base[s * step + 129] : 0.f;
   }
   constexpr int kAhead = 8;
   f32x4 o[kAhead];
@@ -350,25 +362,22 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p) {
     }
   };
   load(slot);
-  float mx = m;
+  const float mx = wave_maxf(fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3])));
+  float den = 0.f;
 #pragma unroll
-  for (int d = 32; d > 0; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
-  if ((tid & 63) == 0) wmax[tid >> 6] = mx;
-  __syncthreads();
-  mx = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-  const float w = m == -INFINITY ? 0.f : fast_exp2(m - mx);   // 0 for an empty range
-  wt[tid] = w;
-  float den = w * l;
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) den += __shfl_xor(den, d, 64);
-  if ((tid & 63) == 0) wsum[tid >> 6] = den;
-  __syncthreads();
+  for (int u = 0; u < 4; ++u) {
+    const float w = m[u] == -INFINITY ? 0.f : fast_exp2(m[u] - mx);   // 0 for an empty range
+    wt[wave][lane + 64 * u] = w;
+    den += w * l[u];
+  }
+  den = wave_sumf(den);
+  __builtin_amdgcn_wave_barrier();
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   for (int s0 = slot; s0 < wgs; s0 += 8 * kAhead) {
     if (s0 != slot) load(s0);
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) {
-      const float ws = s0 + 8 * u < wgs ? wt[s0 + 8 * u] : 0.f;
+      const float ws = s0 + 8 * u < wgs ? wt[wave][s0 + 8 * u] : 0.f;
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc[e] += ws * o[u][e];
     }
@@ -379,8 +388,188 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p) {
     float num = 0.f;
 #pragma unroll
     for (int s = 0; s < 8; ++s) num += accs[s][tid];
-    den = wsum[0] + wsum[1] + wsum[2] + wsum[3];
     p.o[(int64_t)head * p.o_sh + tid] = (__bf16)(den > 0.f ? num / den : 0.f);
+  }
+}
+
+// A step over a short cache, in one launch.  Partial results of several workgroups would need a second one, 3 us on the GPU and as much
+// on the host, so a KV head is four workgroups', each of which goes over all keys for a quarter of the features.  They are on one XCD,
+// and each begins at another quarter of the keys, so the keys are fetched into its L2 once, by all four together.  Its wavefronts take
+// every twelfth tile each: 8 KiB of keys and 2 KiB of values, requested anew as soon as the last ones are in registers.  Bound by what
+// a CU takes in, 10 KiB per tile at 100 GB/s, behind 3.4 us of latencies (launch, first tile, softmax, the wavefronts' results, store).
+constexpr int kShortWaves = 12, kShortParts = 4;
+constexpr int kShortSlot = kDecTileBytes + kDecTileBytes / kShortParts;
+constexpr int kShortLds = kShortWaves * kShortSlot + kDecTileBytes;      // the queries last
+constexpr int kShortStride = 36;              // floats per (wavefront, query head): 32 outputs, max, sum, 2 pad
+
+__global__ __launch_bounds__(64 * kShortWaves) void decode_short_kernel(DecodeParams p) {
+  extern __shared__ __attribute__((aligned(1024))) char ring_all[];
+  const int stride = (p.Hkv + 7) & ~7;
+  const int part = blockIdx.x / stride, kvh = blockIdx.x - part * stride;
+  if (kvh >= p.Hkv) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 31, hh = lane >> 5;
+  char* const mine = ring_all + wave * kShortSlot;
+  char* const queries = ring_all + kShortWaves * kShortSlot;
+  const uint32_t slot = (uint32_t)(uintptr_t)(lds_char_ptr)ring_all + (uint32_t)(wave * kShortSlot);
+  const int turn = part * p.n_tiles / kShortParts;
+  auto tile_of = [&](int i) {
+    const int t = wave + i * kShortWaves + turn;
+    return t < p.n_tiles ? t : t - p.n_tiles;
+  };
+  const int n = wave < p.n_tiles ? (p.n_tiles - 1 - wave) / kShortWaves + 1 : 0;
+
+  if (wave * 4 < p.group) {
+    const int row = wave * 4 + (lane >> 4), src = row < p.group ? row : p.group - 1;
+    const __bf16* const from = p.q + (int64_t)(kvh * p.group + src) * p.q_sh + ((lane & 15) ^ dec_swz(row)) * 8;
+    // (from assembly, as the tiles: the compiler would wait for a copy that it knows of, and for all behind it, at the first
+    // transposing read of every tile)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"((uint32_t)(uintptr_t)(lds_char_ptr)(queries + wave * 1024)), "v"(from) : "memory", "m0");
+  }
+  uint32_t voffK[8], voffV[2];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int row = 4 * i + (lane >> 4);
+    voffK[i] = (uint32_t)(row * p.k_sn * 2) + (uint32_t)(((lane & 15) ^ dec_swz(row)) << 4);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) voffV[i] = (uint32_t)((16 * i + (lane >> 2)) * p.v_sn * 2) + (uint32_t)(part * 64 + (lane & 3) * 16);
+  auto resource = [&](const __bf16* base, int64_t sn, int tile) {
+    const int rows_left = p.Lk - tile * kDecKeys, rows = rows_left < kDecKeys ? rows_left : kDecKeys;
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(base + (int64_t)tile * kDecKeys * sn), 0, (int)((int64_t)rows * sn * 2), 0x00020000);
+  };
+  auto copy_k = [&](int tile) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t res = resource(p.k + (int64_t)kvh * p.k_sh, p.k_sn, tile);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) slab_copy_1k(res, voffK[i], slot + i * 1024);
+  };
+  auto copy_v = [&](int tile) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t res = resource(p.v + (int64_t)kvh * p.v_sh, p.v_sn, tile);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) slab_copy_1k(res, voffV[i], slot + kDecTileBytes + i * 1024);
+  };
+  if (n > 0) {
+    copy_k(tile_of(0));
+    copy_v(tile_of(0));
+    asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+  } else {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+  int kaddr[8], vaddr[2];
+#pragma unroll
+  for (int s = 0; s < 8; ++s) kaddr[s] = r * 256 + (((2 * s + hh) ^ dec_swz(r)) << 4);
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+    vaddr[a] = kDecTileBytes + (8 * a + 4 * hh + ((lane & 15) >> 2)) * 64 + (2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) * 16 + (lane & 1) * 8;
+  f32x16 oacc;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) oacc[v] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+  asm volatile("s_barrier" ::: "memory");      // the queries, of whoever copied them
+  bf16x8 qreg[8];
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    const bf16x8 x = *reinterpret_cast<const bf16x8*>(queries + kaddr[s]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) qreg[s][e] = r < p.group ? x[e] : (__bf16)0.f;
+  }
+
+  for (int i = 0; i < n; ++i) {
+    const int tile = tile_of(i);
+    const bool more = i + 1 < n;
+    asm volatile("s_waitcnt vmcnt(2)" ::: "memory");      // K_i; V_i may be on its way
+    bf16x8 kf[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) kf[s] = *reinterpret_cast<const bf16x8*>(mine + kaddr[s]);
+    wait_lgkm0();
+    if (more) copy_k(tile_of(i + 1));
+    f32x16 sacc;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) sacc[v] = 0.f;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) sacc = mfma32(kf[s], qreg[s], sacc);
+    if (tile * kDecKeys + kDecKeys > p.Lk) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int kpos = tile * kDecKeys + (v >> 2) * 8 + hh * 4 + (v & 3);
+        sacc[v] = kpos >= p.Lk ? -INFINITY : sacc[v];
+      }
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) mx = fmaxf(mx, sacc[v]);
+    mx = half_max(mx) * p.scale_log2;
+    const float m_new = fmaxf(m_run, mx);          // finite: every tile holds at least one real key
+    const float alpha = fast_exp2(m_run - m_new);  // 0 on the first tile
+    m_run = m_new;
+    l_run *= alpha;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) oacc[v] *= alpha;
+    float psum = 0.f;
+    bf16x8 pfrag[2];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const float e = fast_exp2(__builtin_fmaf(sacc[v], p.scale_log2, -m_run));
+      psum += e;
+      pfrag[v >> 3][v & 7] = (__bf16)e;
+    }
+    l_run += psum;
+    if (more) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");      // V_i
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    i16x4 t[2][2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+        t[ks][a] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(mine + vaddr[a] + ks * 1024));
+    wait_lgkm0();
+    if (more) copy_v(tile_of(i + 1));
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      i16x8 av;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        av[u] = t[ks][0][u];
+        av[4 + u] = t[ks][1][u];
+      }
+      oacc = mfma32(__builtin_bit_cast(bf16x8, av), pfrag[ks], oacc);
+    }
+  }
+
+  // the wavefronts' results meet in LDS, each in its own slot
+  const float l_tot = half_sum(l_run);
+  if (r < p.group) {
+    float* const dst = reinterpret_cast<float*>(mine) + r * kShortStride;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      f32x4 w;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) w[u] = oacc[g * 4 + u];
+      *reinterpret_cast<f32x4*>(dst + g * 8 + hh * 4) = w;
+    }
+    if (hh == 0) {
+      dst[32] = m_run;
+      dst[33] = l_tot;
+    }
+  }
+  __syncthreads();
+  for (int e = tid; e < p.group * 32; e += 64 * kShortWaves) {
+    const int g = e >> 5, d = e & 31;
+    const float* const src = reinterpret_cast<const float*>(ring_all) + g * kShortStride;
+    float m[kShortWaves], top = -INFINITY, acc = 0.f, l = 0.f;
+#pragma unroll
+    for (int w = 0; w < kShortWaves; ++w) {
+      m[w] = src[w * (kShortSlot / 4) + 32];
+      top = fmaxf(top, m[w]);
+    }
+#pragma unroll
+    for (int w = 0; w < kShortWaves; ++w) {
+      const float wt = m[w] == -INFINITY ? 0.f : fast_exp2(m[w] - top);      // 0 for a wavefront without tiles
+      acc += wt * src[w * (kShortSlot / 4) + d];
+      l += wt * src[w * (kShortSlot / 4) + 33];
+    }
+    p.o[(int64_t)(kvh * p.group + g) * p.o_sh + part * 32 + d] = (__bf16)(l > 0.f ? acc / l : 0.f);
   }
 }
 
@@ -390,20 +579,26 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p) {
 // without / with: 82 MB 19.0 / 19.4 us, 38 MB 12.8 / 13.1).
 constexpr int64_t kNtBytes = 96 << 20;
 
+// Tiles of the longest cache that decode_short_kernel takes (1536 keys).  Its four workgroups per KV head take 0.1 us per tile; the two
+// launches take 7 us, and a loop of calls 8.5 to 9, which is what the host needs for them (6 for one).  us in a captured graph / in such
+// a loop, two launches and one: 100 keys of 8 KV heads 7.4 / 8.6 and 3.5 / 6.0, 500 7.6 / 8.6 and 4.8 / 6.1, 1100 7.6 / 8.7 and 6.6 / 7.1,
+// 1500 7.2 / 8.8 and 7.6 / 8.0, 2200 7.3 / 8.8 and 11.1 / 11.2; of 32, whose keys a step fetches with fewer requests so, 1100
+// 10.5 / 10.7 and 8.5 / 8.5, 2200 12.5 / 12.6 and 13.2 / 13.2.
+constexpr int kShortTiles = 48;
+
 struct DecodeGeometry {
-  int n_tiles, tiles_per_wave, ranges_per_head;
+  int n_tiles, wgs;
 };
 
-// One workgroup per CU at most: a KV head gets 256 / H_kv workgroups (at least
-// one), i.e. four times as many key ranges, unless it has fewer tiles than that.
+// One workgroup per CU at most: a KV head gets 256 / H_kv workgroups (at least one), unless that leaves them fewer than two tiles (2200
+// keys of 8 KV heads: with four, a wavefront's each, 7.6 us, with two 7.3).
 static DecodeGeometry decode_geometry(int num_kv_heads, int k_len) {
   DecodeGeometry g;
   g.n_tiles = (k_len + kDecKeys - 1) / kDecKeys;
-  int wgs = kDecCUs / num_kv_heads;
-  if (wgs < 1) wgs = 1;
-  g.tiles_per_wave = (g.n_tiles + wgs * kDecWaves - 1) / (wgs * kDecWaves);
-  const int ranges = (g.n_tiles + g.tiles_per_wave - 1) / g.tiles_per_wave;
-  g.ranges_per_head = (ranges + kDecWaves - 1) / kDecWaves * kDecWaves;
+  int most = kDecCUs / num_kv_heads;
+  if (most < 1) most = 1;
+  const int wanted = (g.n_tiles + 1) / 2;
+  g.wgs = wanted < most ? wanted : most;
   return g;
 }
 
@@ -414,7 +609,7 @@ using namespace xattn;
 extern "C" size_t xattn_decode_workspace_bytes(int num_heads, int num_kv_heads, int k_len) {
   if (num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads || k_len <= 0) return 0;
   const DecodeGeometry g = decode_geometry(num_kv_heads, k_len);
-  return (size_t)(g.ranges_per_head / kDecWaves) * num_heads * kPartStride * sizeof(float);
+  return (size_t)g.wgs * num_heads * kPartStride * sizeof(float);
 }
 
 namespace {
@@ -449,15 +644,21 @@ int decode_launch(const void* q, const void* k, const void* v, void* out, void* 
   p.q_sh = q_stride_h; p.k_sh = k_stride_h; p.k_sn = k_stride_n;
   p.v_sh = v_stride_h; p.v_sn = v_stride_n; p.o_sh = o_stride_h;
   p.H = num_heads; p.Hkv = num_kv_heads; p.group = num_heads / num_kv_heads; p.Lk = k_len;
-  p.n_tiles = g.n_tiles; p.tiles_per_wave = g.tiles_per_wave; p.ranges_per_head = g.ranges_per_head;
+  p.n_tiles = g.n_tiles; p.wgs = g.wgs;
+  p.per_wave = g.n_tiles / (g.wgs * kDecWaves); p.longer = g.n_tiles % (g.wgs * kDecWaves);
   p.scale_log2 = softmax_scale * kLog2e;
 
   hipStream_t s = static_cast<hipStream_t>(stream);
-  static LdsLimit limit[2];
+  static LdsLimit limit[3];
+  if (g.n_tiles <= kShortTiles) {
+    if (limit[2].raise(reinterpret_cast<const void*>(decode_short_kernel)) != hipSuccess) return XATTN_ERR_LAUNCH;
+    hipLaunchKernelGGL(decode_short_kernel, dim3((unsigned)(kShortParts * ((num_kv_heads + 7) & ~7))), dim3(64 * kShortWaves), kShortLds, s, p);
+    return hipGetLastError() == hipSuccess ? XATTN_OK : XATTN_ERR_LAUNCH;
+  }
   const bool nt = (int64_t)num_kv_heads * k_len * kHeadDim * 4 > kNtBytes;
   const auto kernel = nt ? decode_partial_kernel<true> : decode_partial_kernel<false>;
   if (limit[nt].raise(reinterpret_cast<const void*>(kernel)) != hipSuccess) return XATTN_ERR_LAUNCH;
-  const unsigned grid = (unsigned)(num_kv_heads * (g.ranges_per_head / kDecWaves));
+  const unsigned grid = (unsigned)(num_kv_heads * g.wgs);
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), kDecLds, s, p);
   hipLaunchKernelGGL(decode_merge_kernel, dim3((unsigned)num_heads), dim3(256), 0, s, p);
   return hipGetLastError() == hipSuccess ? XATTN_OK : XATTN_ERR_LAUNCH;

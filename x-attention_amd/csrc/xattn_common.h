@@ -108,6 +108,22 @@ __device__ __forceinline__ int wave_scan(int x) {
   return add(x, lane_move<0x143, 0xc>(0u, (uint32_t)x));
 }
 
+// largest value and sum of floats, in every lane
+__device__ __forceinline__ float wave_maxf(float x) {
+  auto f = [](uint32_t a, uint32_t b) { return __builtin_bit_cast(uint32_t, fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b))); };
+  return __builtin_bit_cast(float, wave_fold(__builtin_bit_cast(uint32_t, x), f));
+}
+__device__ __forceinline__ float wave_sumf(float x) {
+  auto add = [](float a, uint32_t b) { return a + __builtin_bit_cast(float, b); };
+  x = add(x, lane_move<0x111, 0xf>(0u, __builtin_bit_cast(uint32_t, x)));
+  x = add(x, lane_move<0x112, 0xf>(0u, __builtin_bit_cast(uint32_t, x)));
+  x = add(x, lane_move<0x114, 0xf>(0u, __builtin_bit_cast(uint32_t, x)));
+  x = add(x, lane_move<0x118, 0xf>(0u, __builtin_bit_cast(uint32_t, x)));
+  x = add(x, lane_move<0x142, 0xa>(0u, __builtin_bit_cast(uint32_t, x)));
+  x = add(x, lane_move<0x143, 0xc>(0u, __builtin_bit_cast(uint32_t, x)));
+  return __builtin_bit_cast(float, (uint32_t)__builtin_amdgcn_readlane((int)__builtin_bit_cast(uint32_t, x), 63));
+}
+
 typedef __attribute__((address_space(3))) char* lds_char_ptr;
 
 // one KiB of a slab of rows of 128 bytes (8 of them), global -> LDS; the caller counts it in vmcnt
