@@ -132,3 +132,25 @@ def test_decode_of_short_caches(H, Hkv, L):
     cache[1, :L, :Hkv, :128] = v.cuda().transpose(0, 1)
     views = single_decode_with_kv_cache(rows[::2, :128], cache[0, :L, :Hkv, :128], cache[1, :L, :Hkv, :128], kv_layout="NHD")
     assert torch.equal(views, out)
+
+
+# the decode step of an attention layer: caches [heads][tokens] and [tokens][heads], cut from larger ones, both kernels, and what
+# has to go through the views instead
+@pytest.mark.parametrize("H,Hkv,L", [(32, 8, 5), (32, 8, 1536), (32, 8, 1537), (4, 4, 9000), (28, 4, 33)])
+def test_decode_of_a_layer(H, Hkv, L):
+    from xattn.src import hip_backend as hb
+    from xattn.src.decode import single_decode_with_kv_cache
+
+    q, k, v = (t.cuda() for t in _mk(H, Hkv, L, L))
+    want = single_decode_with_kv_cache(q, k, v, kv_layout="HND").reshape(1, 1, H * 128)
+    step = q.reshape(1, 1, H, 128).transpose(1, 2)
+    heads_first = torch.zeros(2, 1, Hkv, L + 50, 128, dtype=torch.bfloat16, device="cuda")
+    heads_first[0, 0, :, :L], heads_first[1, 0, :, :L] = k, v
+    tokens_first = heads_first.transpose(2, 3).contiguous().transpose(2, 3)
+    for cache in (heads_first, tokens_first):
+        got = hb.host().decode_layer(step, cache[0, :, :, :L], cache[1, :, :, :L])
+        assert got.shape == (1, 1, H * 128) and torch.equal(got, want)
+    ks, vs = heads_first[0, :, :, :L], heads_first[1, :, :, :L]
+    for other in [(step.cpu(), ks, vs), (step.float(), ks, vs), (step, ks, vs[:, :, 1:]), (step, ks.transpose(2, 3), vs.transpose(2, 3)),
+                  (step.expand(2, -1, -1, -1), ks, vs), (step.expand(-1, -1, 2, -1), ks, vs), (step[..., :64], ks, vs), (step[0], ks[0], vs[0])]:
+        assert hb.host().decode_layer(*other) is None

@@ -203,6 +203,25 @@ PyObject* estimate(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// One decode step: heads of q, and heads and tokens of k and v, lie along the named dimensions; out is [H][128] in memory.
+// None, and no error set: not an ordinary call.
+PyObject* decode_step(const at::Tensor& q, int64_t q_head, const at::Tensor& k, const at::Tensor& v, int64_t head, int64_t token, double scale,
+                      at::IntArrayRef out_sizes) {
+  const int64_t H = q.size(q_head), Hkv = k.size(head), L = k.size(token);
+  if (H < 1 || Hkv < 1 || H % Hkv || H / Hkv > 32 || L < 1 || L > (int64_t(1) << 30)) Py_RETURN_NONE;
+  const size_t bytes = xattn_decode_workspace_bytes((int)H, (int)Hkv, (int)L);
+  if (bytes == 0) Py_RETURN_NONE;
+  const c10::Device dev = q.device();
+  OnDevice on(dev);
+  at::Tensor out = at::empty(out_sizes, at::TensorOptions().device(dev).dtype(at::kBFloat16));
+  const c10::DataPtr ws = c10::hip::HIPCachingAllocator::get()->allocate(bytes);
+  const int rc = xattn_decode_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), ws.get(), bytes, (int)H, (int)Hkv, (int)L, 128,
+                                  q.stride(q_head), k.stride(head), k.stride(token), v.stride(head), v.stride(token), 128, (float)scale,
+                                  stream_of(dev));
+  if (rc != XATTN_OK) return fail("xattn_decode_fwd", rc);
+  return THPVariable_Wrap(std::move(out));
+}
+
 // decode(q, k, v, token_major, sm_scale): single_decode_with_kv_cache without caller-provided buffers
 PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (nargs != 5) return PyErr_Format(PyExc_TypeError, "decode takes 5 arguments");
@@ -220,21 +239,22 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       q->stride(0) % 8 || (reinterpret_cast<uintptr_t>(q->data_ptr()) & 15))
     Py_RETURN_NONE;
   if (!kernel_ready(*k, 3) || !kernel_ready(*v, 3) || k->sizes() != v->sizes()) Py_RETURN_NONE;
-  const c10::Device dev = q->device();
-  if (k->device() != dev || v->device() != dev) Py_RETURN_NONE;
+  if (k->device() != q->device() || v->device() != q->device()) Py_RETURN_NONE;
   const int hd = nhd ? 1 : 0, td = 1 - hd;       // head and token dimension of k and v
-  const int64_t H = q->size(0), Hkv = k->size(hd), L = k->size(td);
-  if (H < 1 || Hkv < 1 || H % Hkv || H / Hkv > 32 || L < 1 || L > (int64_t(1) << 30)) Py_RETURN_NONE;
-  const size_t bytes = xattn_decode_workspace_bytes((int)H, (int)Hkv, (int)L);
-  if (bytes == 0) Py_RETURN_NONE;
-  OnDevice on(dev);
-  at::Tensor out = at::empty({H, 128}, at::TensorOptions().device(dev).dtype(at::kBFloat16));
-  const c10::DataPtr ws = c10::hip::HIPCachingAllocator::get()->allocate(bytes);
-  const int rc = xattn_decode_fwd(q->data_ptr(), k->data_ptr(), v->data_ptr(), out.data_ptr(), ws.get(), bytes, (int)H, (int)Hkv,
-                                  (int)L, 128, q->stride(0), k->stride(hd), k->stride(td), v->stride(hd), v->stride(td), 128,
-                                  (float)scale, stream_of(dev));
-  if (rc != XATTN_OK) return fail("xattn_decode_fwd", rc);
-  return THPVariable_Wrap(std::move(out));
+  return decode_step(*q, 0, *k, *v, hd, td, scale, {q->size(0), 128});
+  END_HANDLE_TH_ERRORS
+}
+
+// decode_layer(q, k, v): the decode step of an attention layer, q [1, heads, 1, 128] on k and v [1, kv_heads, tokens, 128], as its
+// output projection takes it: [1, 1, heads * 128] (the views that decode() needs, and its result's, are 5 us of tensor calls)
+PyObject* decode_layer(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 3) return PyErr_Format(PyExc_TypeError, "decode_layer takes 3 arguments");
+  HANDLE_TH_ERRORS
+  const at::Tensor *q = tensor_of(args[0]), *k = tensor_of(args[1]), *v = tensor_of(args[2]);
+  if (!q || !k || !v || !kernel_ready(*q, 4) || !kernel_ready(*k, 4) || !kernel_ready(*v, 4)) Py_RETURN_NONE;
+  if (q->size(0) != 1 || q->size(2) != 1 || k->size(0) != 1 || k->sizes() != v->sizes()) Py_RETURN_NONE;
+  if (k->device() != q->device() || v->device() != q->device()) Py_RETURN_NONE;
+  return decode_step(*q, 1, *k, *v, 1, 2, 1.0 / std::sqrt(128.0), {1, 1, q->size(1) * 128});
   END_HANDLE_TH_ERRORS
 }
 
@@ -357,6 +377,7 @@ PyMethodDef methods[] = {
     method<prefill>("prefill"),
     method<estimate>("estimate"),
     method<decode>("decode"),
+    method<decode_layer>("decode_layer"),
     method<project>("project"),
     method<output>("output"),
     {nullptr, nullptr, 0, nullptr},

@@ -238,7 +238,13 @@ def forward_eval(self, hidden_states, position_embeddings=None, attention_mask=N
     if cfg.print_detail:
         print(f"q length: {q_len} k length: {k_len}")
 
-    if decoding:
+    # the ordinary decode step comes back as the output projection takes it, without views made and put together here
+    merged = None
+    if decoding and native and type(query_states) is type(key_states) is type(value_states) is torch.Tensor:
+        merged = _hb.host().decode_layer(query_states, key_states, value_states)
+    if merged is not None:
+        pass
+    elif decoding:
         attn_output = single_decode_with_kv_cache(
             query_states[0, :, 0], key_states[0], value_states[0], kv_layout="HND"
         ).reshape(1, heads, 1, head_dim)
@@ -251,11 +257,14 @@ def forward_eval(self, hidden_states, position_embeddings=None, attention_mask=N
         attn_output = block_sparse_attention(query_states, key_states, value_states, causal=True)
     start = _stamp(cfg, "Attention computation", start)
 
-    if attn_output.size() != (bsz, heads, q_len, head_dim):
-        raise ValueError(
-            f"`attn_output` should be of size {(bsz, heads, q_len, head_dim)}, but is {attn_output.size()}"
-        )
-    attn_output = attn_output.transpose(1, 2).reshape(bsz, q_len, heads * head_dim)
+    if merged is not None:
+        attn_output = merged
+    else:
+        if attn_output.size() != (bsz, heads, q_len, head_dim):
+            raise ValueError(
+                f"`attn_output` should be of size {(bsz, heads, q_len, head_dim)}, but is {attn_output.size()}"
+            )
+        attn_output = attn_output.transpose(1, 2).reshape(bsz, q_len, heads * head_dim)
     out_proj = _linear_params(self.o_proj) if native else None
     projected = _hb.host().output(attn_output, *out_proj) if out_proj is not None else None
     attn_output = projected if projected is not None else self.o_proj(attn_output)
