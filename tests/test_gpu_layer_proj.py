@@ -47,6 +47,28 @@ def test_projection_and_rotation(width, tokens, heads, kv_heads, bias):
             assert ((y.float() - ref.float()).abs() <= 2.0 ** -8 * (ref.float().abs() + 1)).all()
 
 
+# one token: a wavefront's share of a row (every fourth chunk of 512) of one, two, four and more chunks and the first width beyond each,
+# some wavefronts without any; weights around 24 MiB, from which they are loaded not temporal
+@pytest.mark.parametrize("width,heads,kv_heads", [(16, 1, 1), (1544, 2, 1), (4096, 4, 2), (4104, 4, 2), (8192, 2, 2), (8200, 2, 1), (10248, 3, 1),
+                                                  (24576, 2, 1), (2048, 32, 8), (2048, 32, 9)])
+def test_one_token(width, heads, kv_heads):
+    test_projection_and_rotation(width, 1, heads, kv_heads, width % 16 == 0)
+
+
+def test_one_token_and_more_rows_than_a_launch_has():
+    from xattn.src import hip_backend as hb
+
+    n = (1 << 24) + 4
+    g = torch.Generator(device="cuda").manual_seed(0)
+    w = torch.randn(n, 8, generator=g, device="cuda", dtype=torch.bfloat16)
+    b = torch.randn(n, generator=g, device="cuda", dtype=torch.bfloat16)
+    x = torch.randn(1, 1, 8, generator=g, device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        y = hb.host().output(x, w, b)
+        ref = (w.float() * x.float()[0]).sum(-1) + b.float()
+    assert ((y[0, 0].float() - ref).abs() <= 2.0 ** -8 * (ref.abs() + 1)).all()
+
+
 def test_modules_that_are_more_than_a_linear_are_called():
     """A hook or a replaced forward on a projection means that the module itself runs."""
     from xattn.src.load_llama import _linear_params

@@ -1,13 +1,16 @@
 // Projections and rotary embedding of an attention layer: what surrounds the prefill and decode kernels in the
 // reference's Llama forward (xattn/src/load_llama.py:119-150, 207-218).
 //
-//  qkv_rope_gemv_kernel / gemv: y = W x for ONE token.  Bound by HBM: every weight is read once and used once, 84 MB
-//    for a 4096-wide layer with 32 + 2 * 8 heads.  A wavefront takes four weight rows at a time (for q and k two
-//    rotary pairs d, d + 64 and their neighbours, so that the rotation happens in registers), every load is a full
-//    1 KiB of one row, and 20 of them are in flight per wavefront before the first is used.  The library GEMM with
-//    one row left most of the chip idle: 47 us for the four products of that layer (1.8 TB/s), and the rotation
-//    another 13 launches.  (Loaded "not temporal" the weights come 4 to 8 % faster from memory, but a layer whose weights are in the
-//    memory-side cache still is 1 to 3 % slower.)  proj_gemm.hip has the products of more tokens.
+//  gemv_kernel: y = W x for ONE token, q, k and v in one launch with their rotation, or the output projection.  Bound by HBM:
+//    every weight is read once and used once, 84 MB for a 4096-wide layer with 32 + 2 * 8 heads.  Four weight rows (for q
+//    and k two rotary pairs d, d + 64 and their neighbours, so that the rotation happens in registers) are a workgroup's, a
+//    quarter of their length each wavefront's, which requests all of it at once (up to 8192 elements) and is done: all loads
+//    of a launch are asked for as soon as there is a place, the CUs get equal shares, and the chip is busy to the end.  With
+//    four whole rows per wavefront, two batches of loads in flight, 4096 wide layers had 384 and 256 workgroups for 256
+//    CUs.  us, weights from memory, q, k and v / output, then / now: 1024 wide 5.1 / 4.2 and 3.8 / 2.9, 2048 8.6 / 5.7 and 6.6 / 5.2,
+//    4096 12.2 / 8.7 and 9.9 / 7.4 (5.1 TB/s), 5120 18.4 / 15.9 and 13.9 / 10.3, 8192 37.3 / 31.8 and 27.6 / 23.1; weights in the
+//    memory-side cache, both, 4096 19.5 and 18.3, 5120 31.4 and 25.4.  (Two wavefronts per unit 0.6 slower, eight 2; what the last
+//    thread needs requested ahead of the weights or behind them 0.5 to 1 slower.)  proj_gemm.hip has the products of more tokens.
 //  rope_kernel: the rotation of q and k of many tokens in place, one read and one write of both.  The reference's
 //    expression is ten elementwise kernels over them.
 //
@@ -33,19 +36,20 @@ struct GemvParams {
   const __bf16* sin;
 };
 
-constexpr int kGemvBatch = 4;    // 512-element chunks of a row per batch of loads
+constexpr int kGemvWaves = 4;
 
+// A workgroup has one unit of four rows and its wavefronts every fourth chunk of 512 elements each, kBatch of them at once.
 // kRope: a unit is rows d, d+1, d+64, d+65 of one head (products 0 and 1 rotated, 2 not); otherwise four rows in order
-template <bool kRope>
-__global__ __launch_bounds__(256) void gemv_kernel(GemvParams p) {
+template <bool kRope, int kBatch, bool kNt>
+__global__ __launch_bounds__(64 * kGemvWaves) void gemv_kernel(GemvParams p) {
+  __shared__ float sums[kGemvWaves][4];
   const int lane = threadIdx.x & 63;
-  int unit = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
-  int t = 0;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int unit = blockIdx.x, t = 0;
   if (kRope) {
     if (unit >= p.units[0]) { unit -= p.units[0]; t = 1; }
     if (t == 1 && unit >= p.units[1]) { unit -= p.units[1]; t = 2; }
   }
-  if (unit >= p.units[t]) return;
   int row[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
@@ -57,47 +61,38 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemvParams p) {
     wres[i] = __builtin_amdgcn_make_buffer_rsrc((void*)(p.w[t] + (int64_t)row[i] * p.w_sn[t]), 0, p.K * 2, 0x00020000);
   const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)p.x, 0, p.K * 2, 0x00020000);
 
-  u32x4 wv[2][kGemvBatch][4], xv[2][kGemvBatch];
-  auto load = [&](int b, int buf) __attribute__((always_inline)) {
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  const int chunks = (p.K + 511) / 512;
+  for (int c0 = wave; c0 < chunks; c0 += kGemvWaves * kBatch) {
+    u32x4 wv[kBatch][4], xv[kBatch];
 #pragma unroll
-    for (int c = 0; c < kGemvBatch; ++c) {
-      const int off = ((b * kGemvBatch + c) * 64 + lane) * 16;
-      xv[buf][c] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xres, off, 0, 0));
+    for (int c = 0; c < kBatch; ++c) {
+      const int off = ((c0 + c * kGemvWaves) * 64 + lane) * 16;
+      xv[c] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xres, off, 0, 0));
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        wv[buf][c][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wres[i], off, 0, 0));
+        wv[c][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wres[i], off, 0, kNt ? kNotTemporal : 0));
     }
-  };
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  auto use = [&](int buf) __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int c = 0; c < kGemvBatch; ++c)
+    for (int c = 0; c < kBatch; ++c)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          acc[i] = __builtin_fmaf(bf16_lo(wv[buf][c][i][e]), bf16_lo(xv[buf][c][e]), acc[i]);
-          acc[i] = __builtin_fmaf(bf16_hi(wv[buf][c][i][e]), bf16_hi(xv[buf][c][e]), acc[i]);
+          acc[i] = __builtin_fmaf(bf16_lo(wv[c][i][e]), bf16_lo(xv[c][e]), acc[i]);
+          acc[i] = __builtin_fmaf(bf16_hi(wv[c][i][e]), bf16_hi(xv[c][e]), acc[i]);
         }
-  };
-  const int batches = (p.K + kGemvBatch * 512 - 1) / (kGemvBatch * 512);
-  load(0, 0);
-  for (int b = 0; b < batches; b += 2) {
-    load(b + 1, 1);
-    __builtin_amdgcn_sched_barrier(0);
-    use(0);
-    if (b + 2 < batches) load(b + 2, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    use(1);
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) acc[i] += __shfl_xor(acc[i], d, 64);
-  if (lane == 0) {
+  for (int i = 0; i < 4; ++i) acc[i] = wave_sumf(acc[i]);
+  if (lane == 0) *reinterpret_cast<f32x4*>(sums[wave]) = f32x4{acc[0], acc[1], acc[2], acc[3]};
+  __syncthreads();
+  if (threadIdx.x == 0) {
     float y[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) y[i] = bf16_round(acc[i] + (p.bias[t] ? (float)p.bias[t][row[i]] : 0.f));
+    for (int i = 0; i < 4; ++i)
+      y[i] = bf16_round(sums[0][i] + sums[1][i] + sums[2][i] + sums[3][i] + (p.bias[t] ? (float)p.bias[t][row[i]] : 0.f));
     if (kRope && t < 2) {
       const int d = (unit & 31) * 2;
 #pragma unroll
@@ -146,6 +141,23 @@ bool a16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 bool a4(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 3) == 0; }
 // a row's loads are 16 bytes at 32-bit offsets
 bool width_ok(int K) { return K >= 8 && K % 8 == 0 && K <= (1 << 24); }
+
+// Bytes of a launch's weights from which they are loaded not temporal: from memory they come 5 to 8 % faster so (us, q, k and v /
+// output, 4096 wide 10.7 / 8.0 -> 9.9 / 7.4, 8192 30.5 / 24.8 -> 27.6 / 23.1), and a model of such layers does not fit the memory-side cache
+// (a single one that is run again and again does: 5120 wide 24.7 -> 25.4, 4096 equal, 8192 56 -> 50).  Narrower ones may (1024 wide, output,
+// 2.9 -> 3.1).
+constexpr int64_t kGemvNtBytes = 24 << 20;
+constexpr int kMostUnits = 1 << 22;      // of a launch: a grid has fewer than 2^32 threads
+
+template <bool kRope>
+int launch_gemv(const GemvParams& p, int units, void* stream) {
+  const int each = (p.K + 512 * kGemvWaves - 1) / (512 * kGemvWaves);      // chunks of a wavefront
+  const bool nt = (int64_t)units * 4 * p.K * 2 > kGemvNtBytes;
+  auto kernel = each == 1 ? gemv_kernel<kRope, 1, false> : each == 2 ? gemv_kernel<kRope, 2, false> : gemv_kernel<kRope, 4, false>;
+  if (nt) kernel = each == 1 ? gemv_kernel<kRope, 1, true> : each == 2 ? gemv_kernel<kRope, 2, true> : gemv_kernel<kRope, 4, true>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)units), dim3(64 * kGemvWaves), 0, static_cast<hipStream_t>(stream), p);
+  return hipGetLastError() == hipSuccess ? XATTN_OK : XATTN_ERR_LAUNCH;
+}
 }  // namespace
 
 extern "C" int xattn_qkv_rope_gemv(const void* x, int width, const void* wq, int64_t wq_stride, const void* bq,
@@ -175,8 +187,7 @@ extern "C" int xattn_qkv_rope_gemv(const void* x, int width, const void* wq, int
   p.K = width;
   p.cos = static_cast<const __bf16*>(cos);
   p.sin = static_cast<const __bf16*>(sin);
-  hipLaunchKernelGGL(gemv_kernel<true>, dim3((unsigned)(units + 3) / 4), dim3(256), 0, static_cast<hipStream_t>(stream), p);
-  return hipGetLastError() == hipSuccess ? XATTN_OK : XATTN_ERR_LAUNCH;
+  return launch_gemv<true>(p, units, stream);
 }
 
 extern "C" int xattn_gemv(const void* x, int width, const void* w, int64_t w_stride, const void* bias, void* y, int rows,
@@ -190,10 +201,17 @@ extern "C" int xattn_gemv(const void* x, int width, const void* w, int64_t w_str
   p.bias[0] = static_cast<const __bf16*>(bias);
   p.y[0] = static_cast<__bf16*>(y);
   p.w_sn[0] = w_stride;
-  p.units[0] = rows / 4;
   p.K = width;
-  hipLaunchKernelGGL(gemv_kernel<false>, dim3((unsigned)(p.units[0] + 3) / 4), dim3(256), 0, static_cast<hipStream_t>(stream), p);
-  return hipGetLastError() == hipSuccess ? XATTN_OK : XATTN_ERR_LAUNCH;
+  for (int done = 0; done < rows; done += 4 * kMostUnits) {
+    const int units = (rows - done) / 4 < kMostUnits ? (rows - done) / 4 : kMostUnits;
+    p.units[0] = units;
+    if (const int rc = launch_gemv<false>(p, units, stream)) return rc;
+    if (rows - done <= 4 * kMostUnits) break;      // (done may not pass the largest int)
+    p.w[0] += 4 * (int64_t)kMostUnits * w_stride;
+    p.y[0] += 4 * kMostUnits;
+    if (p.bias[0]) p.bias[0] += 4 * kMostUnits;
+  }
+  return XATTN_OK;
 }
 
 extern "C" int xattn_rope(void* q, void* k, const void* cos, const void* sin, int64_t cos_stride, int64_t sin_stride,
