@@ -594,7 +594,8 @@ __global__ __launch_bounds__(256) void estimate_normalize_kernel(EstParams p) {
 template <int RBS>
 __global__ __launch_bounds__(256) void estimate_select_kernel(EstParams p, SelParams sp, int qb_per_wg) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);      // (what follows from it is uniform for the compiler, too)
   const int rows_wg = qb_per_wg * RBS;                   // reshaped rows of the workgroup (<= 128)
   const int nkb_pad = (p.nkb + 15) & ~15;
   // LDS: statistics, then per wavefront its sort keys (with the row's block sums) and flags

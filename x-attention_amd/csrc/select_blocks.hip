@@ -4,13 +4,11 @@
 // the mask post-processing of xattn_estimate (xattn/src/Xattention.py:275-297).
 // The reference runs ~15 eager torch ops over an fp64 copy of the block sums
 // (two full sorts, a cumsum, an advanced-index scatter) and synchronises the
-// device once per chunk; here a row's candidates (only the columns up to the
-// diagonal when causal - the problem size follows the row) are first tried by
-// extraction: the wavefront pulls out the largest remaining block, adds its
-// mass, and stops as soon as the threshold is reached - on sparse rows that is a
-// handful of wavefront reductions.  Rows that need more than kMaxExtract blocks
-// fall back to a bitonic sort of the candidates in LDS followed by an fp64
-// wavefront prefix scan.  Both visit blocks in the same order (descending sum,
+// device once per chunk; here a row's candidates are only the columns up to the
+// diagonal when causal - the problem size follows the row - and a wavefront
+// decides them in registers: up to 64 with a sort of the lanes and an fp64 prefix
+// sum, more with a few pulled out one by one and a search for where a long list
+// ends (select_row.h).  All ways visit blocks in the same order (descending sum,
 // ascending column among equals) and apply the same rule.  The kernel emits the
 // final mask row plus the compacted, ascending column list the attention kernel
 // walks.

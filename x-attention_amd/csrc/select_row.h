@@ -1,6 +1,8 @@
 // Threshold block selection of one q-block row by one wavefront: shared by the stand-alone selection kernel
 // (block sums from memory) and the estimator's fused normalise-and-select kernel (block sums from LDS).
 #pragma once
+#include <type_traits>
+
 #include "attn_plan.h"
 #include "xattn_common.h"
 
@@ -27,11 +29,9 @@ struct SelParams {
   uint32_t* totals;   // null, or where blocks of each q-block's lists, and of its longest, are found: 32 * (row - win_row0)
 };
 
-constexpr int kSlots = 16;        // candidates per lane held in registers (rows up to 1024 candidates)
-constexpr int kMaxExtract = 32;   // blocks pulled out one by one before falling back to the sort
-constexpr int kRankAll = 16;      // up to so many candidates are ranked at once
-constexpr int kBeforeRank = 4;    // ... and what is left of up to 64 after so many were pulled out one by one
-constexpr int kBeforeSearch = 6;  // blocks pulled out of more than 64 before the search for where a long list ends
+constexpr int kMostSlots = 16;    // candidates per lane held in registers (rows up to 1024 candidates)
+constexpr int kMaxExtract = 32;   // blocks pulled out one by one before falling back to the sort in LDS
+constexpr int kBeforeSearch = 2;  // blocks pulled out of more than 64 before the search for where a long list ends
 
 // value encoded in a sort key (0 for forced blocks and padding)
 __device__ __forceinline__ double key_value(uint64_t key) {
@@ -56,6 +56,52 @@ __device__ __forceinline__ double wave_sum(double x) {
                                         (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, 63));
 }
 
+// value of the lane whose number differs in bit J
+template <int J>
+__device__ __forceinline__ uint32_t other_lane(uint32_t x, int lane) {
+  if (J == 1) return lane_move<0xB1, 0xf>(x, x);                                  // within four: 1 0 3 2
+  if (J == 2) return lane_move<0x4E, 0xf>(x, x);                                  // 2 3 0 1
+  if (J == 4) {
+    const uint32_t y = lane_move<0x141, 0xf>(x, x);                               // eight mirrored, then each four
+    return lane_move<0x1B, 0xf>(y, y);
+  }
+  if (J == 8) return lane_move<0x128, 0xf>(x, x);                                 // sixteen rotated by eight
+  uint32_t a = x, b = x;      // a ends up with the lanes whose bit J is 0 in both places, b with the others
+  if (J == 16) asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+  else asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+  return lane & J ? a : b;
+}
+template <int K, int J>
+__device__ __forceinline__ void sort_step(uint32_t& hi, uint32_t& lo, int lane) {
+  const uint32_t oh = other_lane<J>(hi, lane), ol = other_lane<J>(lo, lane);
+  const bool less = (((uint64_t)hi << 32) | lo) < (((uint64_t)oh << 32) | ol);
+  const bool largest = ((lane & J) == 0) == ((lane & K) == 0);
+  const bool take = less == largest;
+  hi = take ? oh : hi;
+  lo = take ? ol : lo;
+  if constexpr (J > 1) sort_step<K, J / 2>(hi, lo, lane);
+}
+// the first n lanes' 64-bit keys in descending order, by a bitonic network of 6 (up to 8 lanes) to 21 steps of some ten instructions;
+// the other lanes' are 0
+__device__ __forceinline__ void sort_lanes(uint32_t& hi, uint32_t& lo, int lane, int n) {
+  sort_step<2, 1>(hi, lo, lane);
+  sort_step<4, 2>(hi, lo, lane);
+  sort_step<8, 4>(hi, lo, lane);
+  if (n > 8) sort_step<16, 8>(hi, lo, lane);
+  if (n > 16) sort_step<32, 16>(hi, lo, lane);
+  if (n > 32) sort_step<64, 32>(hi, lo, lane);
+}
+// sum of the lanes before the lane's own
+__device__ __forceinline__ double wave_sum_before(double x) {
+  x += lane_move<0x111, 0xf>(x);
+  x += lane_move<0x112, 0xf>(x);
+  x += lane_move<0x114, 0xf>(x);
+  x += lane_move<0x118, 0xf>(x);
+  x += lane_move<0x142, 0xa>(x);
+  x += lane_move<0x143, 0xc>(x);
+  return lane_move<0x138, 0xf>(x);
+}
+
 // M(i + ahead) from the masses before the i-th ordinary block (b0), before its predecessor (b1) and before
 // the one ahead of that (b2); ranks 0 and 1 carry no mass
 __device__ __forceinline__ double rank_mass(int i, int ahead, double b0, double b1, double b2) {
@@ -70,6 +116,15 @@ __device__ __forceinline__ void store_sums(const SelParams& p, const float* x, i
   for (int c = lane; c < p.nkb; c += 64) out[c] = (__bf16)x[c];
 }
 
+// How much of a row is decided at once.  Bound by one wavefront's chain of instructions, and by the longest list where rows are few.
+//  - Up to 64 candidates, one per lane: a sort of the lanes and a prefix sum.  (Four pulled out one by one, 1 us each, and the rest
+//    ranked against each other, 0.09 us each: selection of a prompt of 4096 tokens 13.6 us, 8.8 so.)
+//  - More, in registers, with as many as there are for 128, 256, 512 and 1024: two are pulled out (most rows of text end there), then a
+//    search leaves at most 63, which are sorted.  (Six pulled out first, the search down to four that were pulled out, 16 registers
+//    always: 2048 tokens on 63488 37.5 -> 24.4 us, video of 65536 159 -> 98, text of 15000 19 -> 15.7, of 32768 53 -> 47.  With one and three
+//    pulled out first 23.7 and 25.4, 97 and 101, 16.2 and 14.7, 46.9 and 46.7.)
+//  - Beyond 1024, and rows whose sums outrank forced blocks after 32 pulled out: a sort in LDS.
+//
 // Selection for q-block row `row` of `head` by ONE wavefront (lane = its lane number).  x: the row's nkb block
 // sums (global or LDS); keys (npow2 entries) and flags (nkb bytes): LDS scratch of this wavefront.  All LDS
 // traffic is the wavefront's own, which the LDS keeps in program order: the points where the lanes exchange
@@ -101,25 +156,21 @@ __device__ __forceinline__ void select_row(const SelParams& p, const float* x, i
   double forced_sum = 0.0;
   // sort keys of the forced blocks (utils.py:126-130); key_hi >= key_lo, equal when only one block is forced
   double key_lo = 0.0, key_hi = 0.0;
+  auto sum_of = [&](int c) { return (double)__uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(x[c]))); };
   if (p.causal && ncand > 0) {
-    if (!one_forced || diag == 0) forced_sum = (double)x[0];
-    if (diag != 0 && diag < p.nkb) forced_sum += (double)x[diag];
-    const double kd = 100000.0 * (1.0 + (double)x[diag < p.nkb ? diag : 0]);
-    const double k0 = one_forced ? kd : 100000.0 * (1.0 + (double)x[0]);
+    if (!one_forced || diag == 0) forced_sum = sum_of(0);
+    if (diag != 0 && diag < p.nkb) forced_sum += sum_of(diag);
+    const double kd = 100000.0 * (1.0 + sum_of(diag < p.nkb ? diag : 0));
+    const double k0 = one_forced ? kd : 100000.0 * (1.0 + sum_of(0));
     key_lo = kd < k0 ? kd : k0;
     key_hi = kd < k0 ? k0 : kd;
   }
-  double total = 0.0;
-  uint32_t vals[kSlots];      // this lane's candidates: slot u holds column u*64 + lane (0 = none)
-  int n_others = 0;
-#pragma unroll
-  for (int u = 0; u < kSlots; ++u) vals[u] = 0;
-  // value bits of candidate c (0 for forced blocks and columns past the candidates); adds it to `total` on request
-  auto load_one = [&](int c, bool count) -> uint32_t {
+  // value bits of candidate c (0 for forced blocks and columns past the candidates)
+  auto load_one = [&](int c, double& sum) -> uint32_t {
     uint32_t bits = 0;
     if (c < ncand) {
       const float v = x[c];
-      if (count) total += (double)v;
+      sum += (double)v;
       const bool forced = p.causal && (c == diag || (c == 0 && !one_forced));
       // block sums are >= 0, so their bit pattern orders like the value (+1
       // keeps every candidate ahead of the forced blocks, which sort last)
@@ -132,85 +183,87 @@ __device__ __forceinline__ void select_row(const SelParams& p, const float* x, i
   auto sort_key = [&](int c, uint32_t bits) -> uint64_t {
     return c < ncand ? (((uint64_t)bits << 32) | (uint32_t)(~(uint32_t)c)) : 0ull;
   };
-  const bool small = np2 <= kSlots * 64;
-  if (small) {      // candidates stay in registers; the sort keys are only written if the extraction gives up
-#pragma unroll
-    for (int u = 0; u < kSlots; ++u)
-      if (u * 64 < np2) {
-        vals[u] = load_one(u * 64 + lane, true);
-        n_others += __popcll(__ballot(vals[u] != 0));
-      }
-  } else {
-    for (int c = lane; c < np2; c += 64) keys[c] = sort_key(c, load_one(c, true));
-  }
-  for (int c = lane; c < p.nkb; c += 64) flags[c] = 0;
-  total = wave_sum(total);
-  const double required = total * (p.tau ? p.tau[head] : p.tau_val[head * p.tau_step]);
   const int n_forced = one_forced ? 1 : 2;
   // forced keys ranked ahead of an ordinary block of sum v (all of them unless v is beyond 100000)
   auto forced_ahead = [&](double v) -> int {
     if (!(v > key_lo)) return n_forced;
     return one_forced ? 0 : (v > key_hi ? 0 : 1);
   };
-  __builtin_amdgcn_wave_barrier();
-
-  int dropped = 0;
-  bool finished = false;
+  double required = 0.0;
   // no block sum can exceed a forced key unless the row's total does: otherwise the forced blocks rank first
   // and a decision does not need the block's own value
-  const bool may_outrank = p.causal && total > key_lo;
-  // At most 64 candidates, one per lane: each lane adds up what ranks ahead of its own, on top of the mass `before` that
-  // is already taken.  A candidate costs about 80 clk with nothing to wait for.
-  auto rank_all = [&](double before, double prev_before, int taken) {
-    const uint32_t mine = vals[0];
-    double mass = before;
-    uint32_t last = 0xffffffffu;       // the smallest value ahead: the predecessor in rank
-    bool first = true;
-    for (int c = 0; c < ncand; ++c) {
-      const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)mine, c);
-      if (o == 0) continue;
-      const bool ahead = o > mine || (o == mine && c < lane);
-      mass += ahead ? (double)__uint_as_float(o - 1u) : 0.0;
-      last = ahead && o < last ? o : last;
-      first = first && !ahead;
+  bool may_outrank = false;
+  auto total_is = [&](double total) {
+    required = total * (p.tau ? p.tau[head] : p.tau_val[head * p.tau_step]);
+    may_outrank = p.causal && total > key_lo;
+  };
+  int dropped = 0;
+  bool finished = false;
+  // At most 64 candidates, one key in each of the first n lanes, behind `taken` others: `before` is the mass ahead of them and prev_before that ahead
+  // of the last one taken.  Sorted, each lane finds the mass ahead of its own in a prefix sum.
+  auto decide_lanes = [&](uint64_t key, int n, double before, double prev_before, int taken) {
+    uint32_t hi = (uint32_t)(key >> 32), lo = (uint32_t)key;
+    sort_lanes(hi, lo, lane, n);
+    const double v = hi ? (double)__uint_as_float(hi - 1u) : 0.0;
+    double mass = before + wave_sum_before(v);
+    if (may_outrank) {                     // (then they are all of the row's, and nothing was taken)
+      const double b1 = lane_move<0x138, 0xf>(mass), b2 = lane_move<0x138, 0xf>(b1);
+      mass = rank_mass(lane, forced_ahead(v), mass, b1, b2);
+    } else if (one_forced) {
+      const double b1 = lane_move<0x138, 0xf>(mass);
+      mass = lane > 0 ? b1 : taken > 0 ? prev_before : 0.0;
     }
-    if (mine != 0) {
-      if (one_forced) mass = first ? (taken > 0 ? prev_before : 0.0) : mass - (double)__uint_as_float(last - 1u);
-      if (mass < required) flags[lane] = 1;
+    if (hi != 0) {
+      if (mass < required) flags[~lo] = 1;
       else dropped = 1;
     }
     finished = true;
   };
-  if (ncand <= kRankAll && !may_outrank) {
-    rank_all(forced_sum, 0.0, 0);
-  } else if (small) {
-    // slots that hold candidates, four at a time (the others are skipped)
-    auto in_use = [&](int u) { return (u & ~3) * 64 < np2; };
+  // More than 64 candidates, in registers: slot u of a lane holds column u*64 + lane.
+  auto decide_slots = [&](auto slots) {
+    constexpr int S = decltype(slots)::value;
+    uint32_t vals[S];
+    double total = 0.0;
+    int n_others = 0;
+#pragma unroll
+    for (int u = 0; u < S; ++u) {
+      vals[u] = load_one(u * 64 + lane, total);
+      n_others += __popcll(__ballot(vals[u] != 0));
+    }
+    total_is(wave_sum(total));
+    // the largest that is left, and it taken from the lowest column that holds it
+    auto largest = [&]() {
+      uint32_t best = 0;
+#pragma unroll
+      for (int u = 0; u < S; ++u) best = vals[u] > best ? vals[u] : best;
+      return wave_max(best);
+    };
+    auto pull = [&](uint32_t best) {
+      uint32_t col = 0xffffffffu;
+#pragma unroll
+      for (int u = S - 1; u >= 0; --u) col = vals[u] == best ? (uint32_t)(u * 64 + lane) : col;
+      col = wave_min(col);
+#pragma unroll
+      for (int u = 0; u < S; ++u) vals[u] = (uint32_t)(u * 64 + lane) == col ? 0u : vals[u];
+      return col;
+    };
     // ---- extraction: keep pulling out the largest remaining block while the rule says "keep"
     double before = forced_sum, prev_before = 0.0, prev2_before = 0.0;
     int taken = 0;               // blocks kept so far
     for (int it = 0; it < kMaxExtract; ++it) {
-      if (it == kBeforeRank && np2 == 64 && !may_outrank) {
-        rank_all(before, prev_before, taken);
-        break;
-      }
       if (it == kBeforeSearch && n_others > 0 && !may_outrank) {
         // ---- a long list: bisection on the value for hi > lo with  before + (sum of values >= hi) < required  and
-        // before + (sum of values >= lo) >= required.  Everything from hi on is kept, and what is left to decide one by
-        // one lies between.  Rows of more than kMaxExtract blocks used to be sorted, 20 us for 512 candidates.
-        uint32_t hi = 0;
-#pragma unroll
-        for (int u = 0; u < kSlots; ++u) hi = vals[u] > hi ? vals[u] : hi;
-        hi = wave_max(hi) + 1;
+        // before + (sum of values >= lo) >= required.  Everything from hi on is kept, and at most 63 blocks are left to decide.
+        uint32_t hi = largest() + 1;
         uint32_t lo = 0, step = 1u << 22;        // (lo 0: not known yet; first the search goes down by growing steps)
         int above = 0, from_lo = n_others;       // candidates >= hi, >= lo
         double mass_hi = 0.0;
-        while (hi - lo > 1 && from_lo - above > 4) {
+        while (hi - lo > 1 && from_lo - above > 63) {
           const uint32_t mid = lo ? lo + (hi - lo) / 2 : (hi > step + 1 ? hi - step : 1);
           int n = 0;
           double sum = 0.0;
 #pragma unroll
-          for (int u = 0; u < kSlots; ++u) {
+          for (int u = 0; u < S; ++u) {
             uint32_t w = vals[u];
             asm volatile("" : "+v"(w));          // (else every value is kept as a double across the loop)
             const bool in = w >= mid;
@@ -231,7 +284,7 @@ __device__ __forceinline__ void select_row(const SelParams& p, const float* x, i
         if (above > 0) {
           uint32_t least = 0xffffffffu;          // the last of the blocks taken
 #pragma unroll
-          for (int u = 0; u < kSlots; ++u) {
+          for (int u = 0; u < S; ++u) {
             const bool in = vals[u] >= hi;
             least = in && vals[u] < least ? vals[u] : least;
             if (in) flags[u * 64 + lane] = 1;
@@ -243,68 +296,76 @@ __device__ __forceinline__ void select_row(const SelParams& p, const float* x, i
           n_others -= above;
           taken += above;
         }
-        if (lo && hi - lo == 1 && from_lo - above > 4) {
-          // a run of equal sums: they come out by ascending column, each adding the same mass
-          const double t = (double)__uint_as_float(lo - 1u);
-          const int shift = one_forced && taken > 0 ? 1 : 0;     // judged against the mass before its predecessor
-          int seen = 0, kept = 0;
+        if (from_lo - above <= 63) {
+          // they come together in the key array, with the largest of those below, which may be judged by the mass ahead of its
+          // predecessor; the others below are dropped
+          int n = 0;
 #pragma unroll
-          for (int u = 0; u < kSlots; ++u) {
-            const bool in = vals[u] == lo;
-            const uint64_t tied = __ballot(in);
-            const int i = seen + __popcll(tied & ((1ull << lane) - 1ull));
-            const double mass = shift && i == 0 ? prev_before : before + (double)(i - shift) * t;
-            const bool keep = in && mass < required;
-            if (keep) flags[u * 64 + lane] = 1;
-            vals[u] = keep ? 0u : vals[u];
-            kept += __popcll(__ballot(keep));
-            seen += __popcll(tied);
+          for (int u = 0; u < S; ++u) {
+            const bool in = vals[u] != 0 && vals[u] >= lo;
+            const uint64_t ballot = __ballot(in);
+            if (in) keys[n + __popcll(ballot & ((1ull << lane) - 1ull))] = sort_key(u * 64 + lane, vals[u]);
+            vals[u] = in ? 0u : vals[u];
+            n += __popcll(ballot);
           }
-          if (kept < seen) {
-            finished = true;
-            dropped = 1;
-            break;
+          if (n < n_others) {
+            const uint32_t best = largest(), col = pull(best);
+            if (lane == 0) keys[n] = sort_key((int)col, best);
+            if (++n < n_others) dropped = 1;
           }
-          before += (double)kept * t;
-          prev_before = before - t;
-          n_others -= kept;
-          taken += kept;
+          __builtin_amdgcn_wave_barrier();
+          decide_lanes(lane < n ? keys[lane] : 0ull, n, before, prev_before, taken);
+          return;
         }
+        // a run of equal sums: they come out by ascending column, each adding the same mass
+        const double t = (double)__uint_as_float(lo - 1u);
+        const int shift = one_forced && taken > 0 ? 1 : 0;     // judged against the mass before its predecessor
+        int seen = 0, kept = 0;
+#pragma unroll
+        for (int u = 0; u < S; ++u) {
+          const bool in = vals[u] == lo;
+          const uint64_t tied = __ballot(in);
+          const int i = seen + __popcll(tied & ((1ull << lane) - 1ull));
+          const double mass = shift && i == 0 ? prev_before : before + (double)(i - shift) * t;
+          const bool keep = in && mass < required;
+          if (keep) flags[u * 64 + lane] = 1;
+          vals[u] = keep ? 0u : vals[u];
+          kept += __popcll(__ballot(keep));
+          seen += __popcll(tied);
+        }
+        if (kept < seen) {
+          finished = true;
+          dropped = 1;
+          return;
+        }
+        before += (double)kept * t;
+        prev_before = before - t;
+        n_others -= kept;
+        taken += kept;
       }
       if (n_others == 0) {
         finished = true;
-        break;
+        return;
       }
       if (!may_outrank) {
         const double mass = p.causal ? rank_mass(taken, n_forced, before, prev_before, prev2_before) : before;
         if (!(mass < required)) {
           finished = true;
           dropped = 1;
-          break;
+          return;
         }
       }
-      uint32_t best = 0;
-#pragma unroll
-      for (int u = 0; u < kSlots; ++u)
-        if (in_use(u)) best = vals[u] > best ? vals[u] : best;
-      best = wave_max(best);
+      const uint32_t best = largest();
       const double best_val = (double)__uint_as_float(best - 1u);
       if (may_outrank) {
         const double mass = rank_mass(taken, forced_ahead(best_val), before, prev_before, prev2_before);
         if (!(mass < required)) {
           finished = true;
           dropped = 1;
-          break;
+          return;
         }
       }
-      uint32_t col = 0xffffffffu;     // lowest column holding the maximum
-#pragma unroll
-      for (int u = kSlots - 1; u >= 0; --u)
-        if (in_use(u)) col = vals[u] == best ? (uint32_t)(u * 64 + lane) : col;
-      col = wave_min(col);
-#pragma unroll
-      for (int u = 0; u < kSlots; ++u)
-        if (in_use(u)) vals[u] = (uint32_t)(u * 64 + lane) == col ? 0u : vals[u];
+      const uint32_t col = pull(best);
       if (lane == 0) flags[col] = 1;
       prev2_before = prev_before;
       prev_before = before;
@@ -312,11 +373,34 @@ __device__ __forceinline__ void select_row(const SelParams& p, const float* x, i
       --n_others;
       ++taken;
     }
+  };
+  for (int c = lane; c < p.nkb; c += 64) flags[c] = 0;
+  __builtin_amdgcn_wave_barrier();
+  const bool small = np2 <= kMostSlots * 64;
+  if (np2 == 64) {
+    double total = 0.0;
+    const uint32_t bits = load_one(lane, total);
+    total_is(wave_sum(total));
+    decide_lanes(sort_key(lane, bits), ncand, forced_sum, 0.0, 0);
+  } else if (np2 == 128) {
+    decide_slots(std::integral_constant<int, 2>{});
+  } else if (np2 == 256) {
+    decide_slots(std::integral_constant<int, 4>{});
+  } else if (np2 == 512) {
+    decide_slots(std::integral_constant<int, 8>{});
+  } else if (small) {
+    decide_slots(std::integral_constant<int, kMostSlots>{});
+  } else {
+    double total = 0.0;
+    for (int c = lane; c < np2; c += 64) keys[c] = sort_key(c, load_one(c, total));
+    total_is(wave_sum(total));
+    __builtin_amdgcn_wave_barrier();
   }
 
   if (!finished) {
   if (small) {
-    for (int c = lane; c < np2; c += 64) keys[c] = sort_key(c, load_one(c, false));
+    double again = 0.0;
+    for (int c = lane; c < np2; c += 64) keys[c] = sort_key(c, load_one(c, again));
     __builtin_amdgcn_wave_barrier();
   }
   // ---- bitonic sort, descending
