@@ -38,3 +38,16 @@ def test_few_q_blocks_reach_every_xcd(tmp_path):
     assert build.returncode == 0, build.stdout
     run = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
     assert run.returncode == 0, run.stdout
+
+
+def test_divisions_by_products_are_exact(tmp_path):
+    hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+    if not (os.path.exists(hipcc) or shutil.which(hipcc)):
+        pytest.skip("hipcc not available")
+    exe = str(tmp_path / "divisor_check")
+    build = subprocess.run([hipcc, "-x", "hip", "--offload-arch=gfx950", "-O1", "-std=c++17", "-I" + os.path.join(ROOT, "x-attention_amd", "csrc"),
+                            os.path.join(ROOT, "tests", "host", "divisor_check.cpp"), "-o", exe],
+                           stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert build.returncode == 0, build.stdout
+    run = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
+    assert run.returncode == 0, run.stdout

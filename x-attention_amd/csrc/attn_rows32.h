@@ -157,7 +157,6 @@ __device__ __forceinline__ void sweep_unit(const AttnParams& p, const Unit& u, i
   const int rows = kHalves ? half * 2 + (wave >> 1) : wave;        // this wavefront's 32 rows of the q-block
   constexpr int NT = kHalves ? 2 : 4;                              // ... and 32-key steps of a tile, from kh * NT on
   const int n_blocks = u.n_blocks;
-  const int first = !kHasList ? u.first : n_blocks > 0 ? u.list[0] : 0;
   const __bf16* qbase = p.q + (int64_t)u.head * p.q_sh;
   const __bf16* kbase = p.k + (int64_t)u.kvh * p.k_sh;
   const __bf16* vbase = p.v + (int64_t)u.kvh * p.v_sh;
@@ -178,17 +177,14 @@ __device__ __forceinline__ void sweep_unit(const AttnParams& p, const Unit& u, i
   float m_run = -INFINITY;   // running row maximum, already multiplied by scale_log2
   float l_run = 0.f;         // this lane's share of the running row sum
 
-  int kb = 0;
+  int kb = u.kb, kb_next = u.kb_next;
   {
     // The q-block is a tile like any other: copied row-wise (full lines) into the V tile, where each wavefront's
     // eighth-of-a-tile copies are its own 32 query rows, and read back as fragments before V_0 is requested.
     int voffQ[8];
     tile_offsets(p.q_sn, lane, rows, voffQ);
     copy_tile<kNt == kNtQueriesToo ? kNotTemporal : 0>(qbase, p.q_sn, p.Lq, u.qb, voffQ, Vs, wave);
-    if (n_blocks > 0) {
-      kb = kHasList ? clamp_block(first, p.nkb) : first;
-      copy_tile(kbase, p.k_sn, p.Lk, kb, voffK, Ks, wave);
-    }
+    if (n_blocks > 0) copy_tile(kbase, p.k_sn, p.Lk, kb, voffK, Ks, wave);
     wait_vm0();
 #pragma unroll
     for (int s = 0; s < 8; ++s) qreg[s] = *reinterpret_cast<const bf16x8*>(Vs + wave * 8192 + la.kaddr[s]);
@@ -201,12 +197,12 @@ __device__ __forceinline__ void sweep_unit(const AttnParams& p, const Unit& u, i
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
   for (int j = 0; j < n_blocks; ++j) {
-    const int kb_next = (j + 1 < n_blocks) ? (kHasList ? clamp_block(u.list[j + 1], p.nkb) : kb + 1) : -1;
+    const bool more = j + 1 < n_blocks;
     f32x16 sacc[NT];
     qk_tile<NT>(Ks + kh * NT * 8192, la.kaddr, qreg, sacc);
     wait_vm0();
     __syncthreads();                       // everyone is done with K_j; V_j landed and visible
-    if (kb_next >= 0) copy_tile_async(kbase, p.k_sn, p.Lk, kb_next, voffK, Ks, wave);
+    if (more) copy_tile_async(kbase, p.k_sn, p.Lk, kb_next, voffK, Ks, wave);
 
     const bool need_mask = (kb * kBlk + kBlk > p.Lk) || (p.causal && kb * kBlk + kBlk - 1 > u.qb * kBlk + p.kv_off);
     if (need_mask) {
@@ -216,10 +212,15 @@ __device__ __forceinline__ void sweep_unit(const AttnParams& p, const Unit& u, i
     bf16x8 pfrag[NT * 2];
     softmax_tile<NT>(sacc, oacc, m_run, l_run, p.scale_log2, pfrag);
     pv_tile<NT * 2>(Vs + kh * NT * 8192, la.vaddr, pfrag, oacc);
+    // the list's next entry is on its way while this wavefront waits (in flight beside LDS reads it would make each of them wait for all)
+    int kb_then = kHasList ? u.list[j + 2 < n_blocks ? j + 2 : j] : kb + 2;
+    __builtin_amdgcn_sched_barrier(0);
     wait_vm0();
     __syncthreads();                       // everyone is done with V_j; K_{j+1} landed and visible
-    if (kb_next >= 0) copy_tile_async(vbase, p.v_sn, p.Lk, kb_next, voffV, Vs, wave);
+    if (kHasList) asm volatile("" : "+s"(kb_then));
+    if (more) copy_tile_async(vbase, p.v_sn, p.Lk, kb_next, voffV, Vs, wave);
     kb = kb_next;
+    kb_next = kHasList ? clamp_block(kb_then, p.nkb) : kb_then;
   }
   // the last barrier of the sweep (or the one before it, for an empty list) left both tiles unused
   if (kPlanned && u.cuts > 0) {
@@ -273,11 +274,12 @@ __global__ __launch_bounds__(256, 2) void block_sparse_fwd_kernel(AttnParams p) 
   __shared__ __attribute__((aligned(1024))) char Ks[kTileBytes];
   __shared__ __attribute__((aligned(1024))) char Vs[kTileBytes];
 
+  touch_params();
   // (both halves on the same XCD, one after the other)
   const int id = kHalves ? (int)(blockIdx.x >> 4 << 3 | (blockIdx.x & 7)) : (int)blockIdx.x;
   const int half = kHalves ? (int)(blockIdx.x >> 3 & 1) : 0;
   Unit u;
-  if (!find_unit<kHasList, kPlanned, false>(p, id, u) || !find_list<kHasList, kPlanned>(p, u)) return;
+  if (!find_work<kHasList, kPlanned>(p, id, u)) return;
   if (kHalves && u.qb * kBlk + half * 64 >= p.Lq) return;
   sweep_unit<kHasList, kPlanned, kHalves, kNt>(p, u, half, Ks, Vs);
 }

@@ -87,6 +87,22 @@ __device__ __forceinline__ void tile_offsets(int64_t sn, int lane, int wave, int
 // had 20 % more than its share: text of 32768 tokens 1986 us, 1738 with the
 // turn.)  Groups fewer than XCDs rotate every second or fourth run, or half the
 // XCDs would never see a group.
+// Division of numbers below 2^31 by the same divisor again and again: the high half of a product, and a shift.
+struct Divisor {
+  uint32_t mul;      // 0: the divisor is 1
+  uint32_t shift;
+};
+inline Divisor divisor(uint32_t d) {
+  Divisor v{0, 0};
+  if (d <= 1) return v;
+  while ((2ull << v.shift) < d) ++v.shift;            // 2^shift < d <= 2^(shift + 1)
+  v.mul = (uint32_t)(((1ull << (32 + v.shift)) + d - 1) / d);
+  return v;
+}
+__host__ __device__ inline uint32_t divided(uint32_t x, const Divisor& v) {
+  return v.mul ? (uint32_t)((uint64_t)x * v.mul >> 32) >> v.shift : x;
+}
+
 struct DispatchShape {
   int group;       // query heads per KV head
   int sets;        // head sets per KV head (1 unless group > kUnit)
@@ -96,6 +112,7 @@ struct DispatchShape {
   int turn_shift;  // groups rotate once per 1 << turn_shift runs
   uint32_t unit_size;   // ids of a unit: kUnit, or as many as it needs where runs are few and that is at most half
   uint32_t unit_inv;    // 2^31 / unit_size, rounded up: ids are divided by a product
+  Divisor by_groups, by_heads, by_group;   // n_groups, set_heads, group
 };
 // (head, q-block)s of the XCD that has most of them, units being dealt to the XCDs in turn.
 inline int64_t fullest_xcd(const DispatchShape& d, int n_qblocks) {
@@ -142,6 +159,9 @@ inline DispatchShape dispatch_shape(int H, int Hkv, int n_qblocks) {
   const int work = d.set_heads * d.unit_rows;
   d.unit_size = (uint32_t)(runs < 8 && work <= kUnit / 2 ? work : kUnit);
   d.unit_inv = ((1u << 31) + d.unit_size - 1) / d.unit_size;
+  d.by_groups = divisor((uint32_t)d.n_groups);
+  d.by_heads = divisor((uint32_t)d.set_heads);
+  d.by_group = divisor((uint32_t)d.group);
   return d;
 }
 
@@ -155,10 +175,11 @@ __host__ __device__ inline bool map_workgroup(int id, const DispatchShape& d, in
   const uint32_t at = (uint32_t)((uint64_t)s * d.unit_inv >> 31);      // s / unit_size (exact: s < 2^26 where it is not kUnit)
   const uint32_t unit = at * 8u + x, w = s - at * d.unit_size;
   const uint32_t ng = (uint32_t)d.n_groups, sh = (uint32_t)d.set_heads;
-  const uint32_t run = unit / ng;
+  const uint32_t run = divided(unit, d.by_groups);
   const uint32_t turn = (run & 8u ? ~run : run) & 7u;
-  const uint32_t dg = (unit - run * ng + (turn >> d.turn_shift)) % ng;      // the unit's group, rotated by its run
-  const uint32_t w_row = w / sh, w_head = w - w_row * sh;
+  const uint32_t rotated = unit - run * ng + (turn >> d.turn_shift);
+  const uint32_t dg = rotated - divided(rotated, d.by_groups) * ng;      // the unit's group, rotated by its run
+  const uint32_t w_row = divided(w, d.by_heads), w_head = w - w_row * sh;
   const uint32_t from_end = run * (uint32_t)d.unit_rows + w_row;
   uint32_t set = 0, kvh = dg;
   if (d.sets != 1) {
