@@ -28,6 +28,7 @@ __global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p, Sel
   constexpr int kLoads = 4 + MT;                    // KiB a wavefront copies per step
   constexpr int kPer = (kLoads + 2) / 3;            // ... and in each of the step's first three sub-steps
   constexpr bool kAhead = MT == 1;
+  static_assert(kAhead ? NS == 4 : NS <= 3, "the steps behind the last copy are written for these");
   constexpr int kPer4 = (kLoads + 3) / 4;           // ... or (kAhead) in each of four
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -90,18 +91,18 @@ __global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p, Sel
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_char_ptr)lds;
   const int steps = p.S * 2;
-  // Piece j of step t: 0 .. 3 are K' (not copied by a wavefront whose keys nobody sees), then Q'.  Past the last step a
-  // copy moves nothing (its offset is outside the resource) but keeps the count of loads in flight.
+  // Piece j of step t: 0 .. 3 are K' (not copied by a wavefront whose keys nobody sees), then Q'.  The last steps copy nothing
+  // and wait for fewer: a copy of 1 KiB costs the CU about 20 clk also where its offset is outside the resource.
   auto copy_piece = [&](int t, int j) __attribute__((always_inline)) {
     const int i = t >> 1;
     const uint32_t st = lds0 + (uint32_t)(t % NS) * kStage;
     if (j < 4) {
       const uint32_t ko = (uint32_t)(i * (int)k_snb + (t & 1) * 128);
-      slab_copy_1k(kres, t < steps ? voffK[j] + ko : 0xffffffffu, st + (uint32_t)(wave * 4 + j) * 1024);
+      slab_copy_1k(kres, voffK[j] + ko, st + (uint32_t)(wave * 4 + j) * 1024);
     } else {
       const int qi = p.S - 1 - i;
       const uint32_t qo = (uint32_t)(qi * (int)q_snb + (t & 1) * 128);
-      slab_copy_1k(qres, t < steps && qtok[j - 4] + qi < p.Lq ? voffQ[j - 4] + qo : 0xffffffffu,
+      slab_copy_1k(qres, qtok[j - 4] + qi < p.Lq ? voffQ[j - 4] + qo : 0xffffffffu,
                    st + 16384 + (uint32_t)(wave * MT + j - 4) * 1024);
     }
   };
@@ -137,8 +138,9 @@ __global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p, Sel
       };
       asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 1) * kLoads) : "memory");
       read(0, 0);
-      auto step = [&](int t, int buf) __attribute__((always_inline)) {
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * kLoads) : "memory");
+      // `left`: the steps behind step t + 1 that have been copied
+      auto step = [&](int t, int buf, auto copies, auto left) __attribute__((always_inline)) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(decltype(left)::value * kLoads) : "memory");
         read(t + 1, buf ^ 1);        // (a repeat of old data behind the last step)
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -146,21 +148,28 @@ __global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p, Sel
 #pragma unroll
           for (int a = 0; a < MT; ++a) acc[a] = mfma32(fa[buf][s], fb[buf][s][a], acc[a]);
 #pragma unroll
-          for (int j = s * kPer4; j < kLoads && j < (s + 1) * kPer4; ++j) copy_piece(t + NS, j);
+          for (int j = s * kPer4; decltype(copies)::value && j < kLoads && j < (s + 1) * kPer4; ++j) copy_piece(t + NS, j);
           __builtin_amdgcn_sched_barrier(0);
         }
       };
-      for (int t = 0; t < steps; t += 2) {      // (steps = 2 S)
-        step(t, 0);
-        step(t + 1, 1);
+      int t = 0;
+      for (; t < steps - NS; t += 2) {      // (steps = 2 S)
+        step(t, 0, std::integral_constant<int, 1>(), std::integral_constant<int, 2>());
+        step(t + 1, 1, std::integral_constant<int, 1>(), std::integral_constant<int, 2>());
       }
+      step(t, 0, std::integral_constant<int, 0>(), std::integral_constant<int, 2>());
+      step(t + 1, 1, std::integral_constant<int, 0>(), std::integral_constant<int, 1>());
+      step(t + 2, 0, std::integral_constant<int, 0>(), std::integral_constant<int, 0>());
+      step(t + 3, 1, std::integral_constant<int, 0>(), std::integral_constant<int, 0>());
     } else {
       asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 1) * MT) : "memory");
-      for (int t = 0; t < steps; ++t) {
+      int t = 0;
+      for (; t < steps - NS; ++t) {
         asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 2) * MT) : "memory");
 #pragma unroll
         for (int j = 4; j < kLoads; ++j) copy_piece(t + NS, j);
       }
+      for (; t < steps; ++t) asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
     }
   } else
   // A step is four sub-steps of MT MFMAs; the fragments of the next sub-step and the copies of step t + NS - 1 are issued
@@ -181,33 +190,38 @@ __global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p, Sel
       for (int a = 0; a < MT; ++a) fb[buf][a] = *reinterpret_cast<const bf16x8*>(st + 16384 + (a * 32 + r) * 128 + ch);
     };
     read(0, 0, 0);
-    for (int t = 0; t < steps; ++t) {
+    auto step = [&](int t, auto copies) __attribute__((always_inline)) {
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         __builtin_amdgcn_sched_barrier(0);
         if (s == 3) {
-          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * kLoads) : "memory");
+          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(decltype(copies)::value ? (NS - 2) * kLoads : 0) : "memory");
           read(t + 1, 0, 0);     // (a repeat of old data behind the last step)
         } else {
           read(t, s + 1, (s + 1) & 1);
 #pragma unroll
-          for (int j = s * kPer; j < kLoads && j < (s + 1) * kPer; ++j) copy_piece(t + NS - 1, j);
+          for (int j = s * kPer; decltype(copies)::value && j < kLoads && j < (s + 1) * kPer; ++j) copy_piece(t + NS - 1, j);
         }
 #pragma unroll
         for (int a = 0; a < MT; ++a) acc[a] = mfma32(fa[s & 1], fb[s & 1][a], acc[a]);
       }
-    }
+    };
+    int t = 0;
+    for (; t < steps - NS + 1; ++t) step(t, std::integral_constant<int, 1>());
+    for (; t < steps; ++t) step(t, std::integral_constant<int, 0>());
   } else {
 #pragma unroll
     for (int t = 0; t < NS - 1; ++t)
 #pragma unroll
       for (int j = 4; j < kLoads; ++j) copy_piece(t, j);
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 2) * MT) : "memory");
-    for (int t = 0; t < steps; ++t) {
+    int t = 0;
+    for (; t < steps - NS + 1; ++t) {
 #pragma unroll
       for (int j = 4; j < kLoads; ++j) copy_piece(t + NS - 1, j);
       asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 2) * MT) : "memory");
     }
+    for (; t < steps; ++t) asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
   }
   // every copy has landed and every fragment has been read: the LDS is free for the exchange below
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
