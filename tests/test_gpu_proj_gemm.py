@@ -64,6 +64,13 @@ def test_weights_pulled_ahead_and_large_tiles(tokens, heads, kv_heads, width):
     test_projections_of_a_turn(tokens, heads, kv_heads, width, True)
 
 
+@pytest.mark.parametrize("width", [64, 128, 192, 256, 320, 384, 448])
+@pytest.mark.parametrize("tokens", [5, 200, 500, 700, 1000])
+def test_depths_of_a_few_slabs(tokens, width):
+    """One slab to one more than the deepest ring of stages holds, with every tile."""
+    test_projections_of_a_turn(tokens, 32, 8, width, True)
+
+
 def test_two_workgroups_per_cu():
     """2600 tokens of 24 heads: 504 tiles of 128 x 128, but more than 256 of 256 tokens."""
     from xattn.src import hip_backend as hb

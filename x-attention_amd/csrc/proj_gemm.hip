@@ -120,11 +120,12 @@ __global__ __launch_bounds__(256 * KS, 2) void proj_gemm_kernel(ProjParams p) {
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_char_ptr)lds;
   const int steps = p.K / 64;
-  // past the last step a copy moves nothing (its offset is outside the resource) but keeps the count of loads in flight
-  auto copy_piece = [&](int t, int st, int i) __attribute__((always_inline)) {
+  // (the steps of a ring's first fill may be more than there are: such a copy moves nothing, its offset being outside the resource;
+  // the last steps issue none, since it would cost the CU 20 clk all the same)
+  auto copy_piece = [&](int t, int st, int i, bool is_step) __attribute__((always_inline)) {
     const bool is_w = i < kLoadsW;
     const uint32_t dst = lds0 + (uint32_t)st * kStage + (is_w ? (uint32_t)(wave * kLoadsW + i) : (uint32_t)(kN / 8 + wave * kLoadsX + i - kLoadsW)) * 1024;
-    slab_copy_1k(is_w ? wres : xres, t < steps ? voff[i] + (uint32_t)t * 128 : 0xffffffffu, dst);
+    slab_copy_1k(is_w ? wres : xres, is_step ? voff[i] + (uint32_t)t * 128 : 0xffffffffu, dst);
   };
   f32x16 acc[NB][MB];
 #pragma unroll
@@ -145,26 +146,27 @@ __global__ __launch_bounds__(256 * KS, 2) void proj_gemm_kernel(ProjParams p) {
 #pragma unroll
   for (int t = 0; t < NS - 1; ++t)
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) copy_piece(t, t, i);
+    for (int i = 0; i < kLoads; ++i) copy_piece(t, t, i, t < steps);
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 2) * kLoads) : "memory");
   read(0, 0, 0);
   // A step is four sub-steps of NB * MB MFMAs; the fragments of the next sub-step and the copies of step t + NS - 1 are
   // issued between them.  The barrier sits before the last sub-step's MFMAs: by then this wavefront has read every
   // fragment of step t and its copies of step t + 1 have landed, so behind it step t + 1 may be read and step t's stage
   // refilled.
-  int st = 0;
-  for (int t = 0; t < steps; ++t) {
+  // `left`: the steps behind step t + 1 whose copies have been issued
+  int st = 0, t = 0;
+  auto step = [&](auto copies, auto left) __attribute__((always_inline)) {
     const int next = st + 1 == NS ? 0 : st + 1, fill = st == 0 ? NS - 1 : st - 1;
 #pragma unroll
     for (int s = 0; s < kSubs; ++s) {
       __builtin_amdgcn_sched_barrier(0);
       if (s == kSubs - 1) {
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * kLoads) : "memory");
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(decltype(left)::value * kLoads) : "memory");
         read(next, 0, 0);     // (a repeat of old data behind the last step)
       } else {
         read(st, s + 1, (s + 1) & 1);
 #pragma unroll
-        for (int i = s * kPer; i < kLoads && i < (s + 1) * kPer; ++i) copy_piece(t + NS - 1, fill, i);
+        for (int i = s * kPer; decltype(copies)::value && i < kLoads && i < (s + 1) * kPer; ++i) copy_piece(t + NS - 1, fill, i, true);
       }
 #pragma unroll
       for (int a = 0; a < NB; ++a)
@@ -172,7 +174,18 @@ __global__ __launch_bounds__(256 * KS, 2) void proj_gemm_kernel(ProjParams p) {
         for (int b = 0; b < MB; ++b) acc[a][b] = mfma32(fa[s & 1][a], fb[s & 1][b], acc[a][b]);
     }
     st = next;
-  }
+    ++t;
+  };
+  while (t < steps - (NS - 1)) step(std::true_type(), std::integral_constant<int, NS - 2>());
+  auto last = [&](auto left) __attribute__((always_inline)) {
+    if (t < steps) step(std::false_type(), left);
+  };
+  static_assert(NS >= 2 && NS <= 6, "the steps behind the last copy are written for these");
+  if constexpr (NS >= 6) last(std::integral_constant<int, 3>());
+  if constexpr (NS >= 5) last(std::integral_constant<int, 2>());
+  if constexpr (NS >= 4) last(std::integral_constant<int, 1>());
+  if constexpr (NS >= 3) last(std::integral_constant<int, 0>());
+  last(std::integral_constant<int, 0>());
   // every copy has landed and every fragment has been read: the LDS takes the tile, token-major, chunk c of token m at
   // c ^ (m & (chunks - 1))
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
