@@ -65,7 +65,7 @@ def test_weights_pulled_ahead_and_large_tiles(tokens, heads, kv_heads, width):
 
 
 @pytest.mark.parametrize("width", [64, 128, 192, 256, 320, 384, 448])
-@pytest.mark.parametrize("tokens", [5, 200, 500, 700, 1000])
+@pytest.mark.parametrize("tokens", [5, 200, 320, 500, 640, 700, 1000])
 def test_depths_of_a_few_slabs(tokens, width):
     """One slab to one more than the deepest ring of stages holds, with every tile."""
     test_projections_of_a_turn(tokens, 32, 8, width, True)

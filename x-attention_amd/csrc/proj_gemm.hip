@@ -6,8 +6,8 @@
 // tiles, then 64 tokens x 128 features, 128 x 128, 192 x 128 and, for q, k and v, 256 x 128.  CUs left over may pull the weights
 // into the L2 (proj_pull.h; weights from memory: q, k, v of 64 tokens, 4096 wide, 22.9 -> 19.9 us, of 192 30.8 -> 23.1, of 512
 // 40.8 -> 33.6; the output of 320, 5120 wide, 38.8 -> 30.9).  Whole products stay below those rates: the tiles of those 512 tokens
-// copy 2.1 MB each, 51 GB/s without pullers and 62 with them; where the rest goes (start, first slab, barriers, epilogue) has not
-// been measured.  The larger tiles took the place of two 128 x 128 ones per CU (4096 wide, 700 tokens 66 -> 45 us, 1000 72 -> 57,
+// copy 2.1 MB each, 51 GB/s without pullers and 62 with them, of 33 us 2 for the first slab, 27 in the loop, 3 in the epilogue: a
+// step of 128 x 128 takes 830 clk, 640 without its copies, 512 of them MFMAs, whether fragments are read in full or halves.  The larger tiles took the place of two 128 x 128 ones per CU (4096 wide, 700 tokens 66 -> 45 us, 1000 72 -> 57,
 // 1280 73 -> 63).  Splitting a step's depth over two groups of wavefronts helps the smallest tile only (17.6 -> 13.3 us at 64
 // tokens), where the chain of 64 steps is the time; on the larger ones, where it would save a third of the LDS reads, it is 1 to 8 %
 // slower.
@@ -23,7 +23,7 @@
 //   8192   64 + 2*8   64 / 51     98 / 64     133 / 90    165 / 114   library
 // Output (features x depth), by the same tokens: 1024 x 1024 11.3 / 6.7, 10.4 / 6.5, 10.6 / 6.7, 11.1 / 6.8, 11.2 / 7.5, 11.7 / 8,
 // 11.8 / 8.2; 3072 x 3072 15.7 / 14.4, 17.2 / 12.7, 20.4 / 17.8, 25.2 / 22.5, 29.2 / 23.9, 31 / 29.1, 38 / 32; 4096 x 4096 15 /
-// 18.2, 21.9 / 16.9, 28.7 / 28.4, 32 / 29.5, 41 / 38, 46 / 44, 50 / 49; 5120 x 5120 21.6 / 24.1, 28.8 / 26.7, 49 / 36, 51 / 44, 63
+// 18.2, 21.9 / 16.4, 28.7 / 25.5, 32 / 29.5, 41 / 36, 46 / 44, 50 / 49; 5120 x 5120 21.6 / 24.1, 28.8 / 26.7, 49 / 36, 51 / 44, 63
 // / 55; 8192 x 8192 35 / 47, 54 / 52, 81 / 75, 98 / 94.  Up to 64 tokens there is a single row of tiles, each a chain over the
 // whole depth, which the library splits; so it does where the features are fewer than the depth.  Such a turn is bound by the
 // host's calls, though, and the library's is the dearer one: the whole layer, 4096 wide, on 6000 tokens with the library's output
@@ -120,12 +120,20 @@ __global__ __launch_bounds__(256 * KS, 2) void proj_gemm_kernel(ProjParams p) {
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_char_ptr)lds;
   const int steps = p.K / 64;
+  // Tiles that share weights or tokens ask for a slab at the same time, and all of them wait for the memory's answer.  Nobody pulling
+  // for them, each takes every four slabs in another order, so that it waits for one of them and finds three in the L2 (weights from
+  // memory, us: output of 500 tokens, 4096 wide, 29.0 / 25.5, of 1000 38.4 / 36.1; q, k, v of 320 31.2 / 26.7; 5120 wide, output of
+  // 700 44.9 / 43.2; 8192 wide, q, k, v of 130 55.9 / 53.6).  Orders of eight slabs give the same, of two a third of it; a quarter of the depth apart for each token tile, slabs leave the L2
+  // between two uses (35 / 42).  Not with pulled weights (-7 to +7 %), 64 x 64 tiles (2 % slower), nor 256 tokens (2 to 5 % slower).
+  constexpr bool kTurn = !kPull && NB == 2 && MB <= 2 && NS == 4;
+  const int turn = kTurn ? (int)(lin % mt + lin / mt) & 3 : 0, turned = steps & ~3;
+  auto slab_of = [&](int t) __attribute__((always_inline)) { return kTurn && t < turned ? (t & ~3) | ((t + turn) & 3) : t; };
   // (the steps of a ring's first fill may be more than there are: such a copy moves nothing, its offset being outside the resource;
   // the last steps issue none, since it would cost the CU 20 clk all the same)
   auto copy_piece = [&](int t, int st, int i, bool is_step) __attribute__((always_inline)) {
     const bool is_w = i < kLoadsW;
     const uint32_t dst = lds0 + (uint32_t)st * kStage + (is_w ? (uint32_t)(wave * kLoadsW + i) : (uint32_t)(kN / 8 + wave * kLoadsX + i - kLoadsW)) * 1024;
-    slab_copy_1k(is_w ? wres : xres, is_step ? voff[i] + (uint32_t)t * 128 : 0xffffffffu, dst);
+    slab_copy_1k(is_w ? wres : xres, is_step ? voff[i] + (uint32_t)slab_of(t) * 128 : 0xffffffffu, dst);
   };
   f32x16 acc[NB][MB];
 #pragma unroll
