@@ -127,7 +127,7 @@ __global__ __launch_bounds__(256) void rope_kernel(RopeParams p) {
   const __bf16* cs = p.cos + (int64_t)tok * p.cos_sn + c * 8;
   const __bf16* sn = p.sin + (int64_t)tok * p.sin_sn + c * 8;
   bf16x8 y0 = *reinterpret_cast<const bf16x8*>(base), y1 = *reinterpret_cast<const bf16x8*>(base + 64);
-  rotate_chunks(y0, y1, cs, sn);
+  rotate_chunks(y0, y1, turn_of(cs, sn));
   *reinterpret_cast<bf16x8*>(base) = y0;
   *reinterpret_cast<bf16x8*>(base + 64) = y1;
 }

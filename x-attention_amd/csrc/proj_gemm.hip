@@ -76,6 +76,9 @@ __global__ __launch_bounds__(256 * KS, 2) void proj_gemm_kernel(ProjParams p) {
   constexpr int kSubs = 4 / KS;                     // 16-deep sub-steps of a wavefront
   constexpr int kLoads = 2 * (NB + MB) / KS;        // KiB a wavefront copies per step: first W's, then x's
   constexpr int kLoadsW = 2 * NB / KS, kLoadsX = 2 * MB / KS;
+  constexpr int kChunks = 8 * NB, kPairs = kChunks / 2;       // of a token in a tile, and rotation partners
+  constexpr int kTurns = (kM * kPairs + 256 * KS - 1) / (256 * KS), kTurnsAhead = kTurns < 4 ? kTurns : 4;
+  constexpr int kTurnLoads = kRope ? 4 * kTurnsAhead : 0;
   constexpr int kPer = (kLoads + kSubs - 2) / (kSubs - 1);   // ... and in each of its sub-steps but the last
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -125,9 +128,9 @@ __global__ __launch_bounds__(256 * KS, 2) void proj_gemm_kernel(ProjParams p) {
   // memory, us: output of 500 tokens, 4096 wide, 29.0 / 25.5, of 1000 38.4 / 36.1; q, k, v of 320 31.2 / 26.7; 5120 wide, output of
   // 700 44.9 / 43.2; 8192 wide, q, k, v of 130 55.9 / 53.6).  Orders of eight slabs give the same, of two a third of it; a quarter of the depth apart for each token tile, slabs leave the L2
   // between two uses (35 / 42).  Not with pulled weights (-7 to +7 %), 64 x 64 tiles (2 % slower), nor 256 tokens (2 to 5 % slower).
-  constexpr bool kTurn = !kPull && NB == 2 && MB <= 2 && NS == 4;
-  const int turn = kTurn ? (int)(lin % mt + lin / mt) & 3 : 0, turned = steps & ~3;
-  auto slab_of = [&](int t) __attribute__((always_inline)) { return kTurn && t < turned ? (t & ~3) | ((t + turn) & 3) : t; };
+  constexpr bool kShift = !kPull && NB == 2 && MB <= 2 && NS == 4;
+  const int shift = kShift ? (int)(lin % mt + lin / mt) & 3 : 0, whole = steps & ~3;
+  auto slab_of = [&](int t) __attribute__((always_inline)) { return kShift && t < whole ? (t & ~3) | ((t + shift) & 3) : t; };
   // (the steps of a ring's first fill may be more than there are: such a copy moves nothing, its offset being outside the resource;
   // the last steps issue none, since it would cost the CU 20 clk all the same)
   auto copy_piece = [&](int t, int st, int i, bool is_step) __attribute__((always_inline)) {
@@ -169,7 +172,7 @@ __global__ __launch_bounds__(256 * KS, 2) void proj_gemm_kernel(ProjParams p) {
     for (int s = 0; s < kSubs; ++s) {
       __builtin_amdgcn_sched_barrier(0);
       if (s == kSubs - 1) {
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(decltype(left)::value * kLoads) : "memory");
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(decltype(left)::value * kLoads + (decltype(copies)::value ? 0 : kTurnLoads)) : "memory");
         read(next, 0, 0);     // (a repeat of old data behind the last step)
       } else {
         read(st, s + 1, (s + 1) & 1);
@@ -185,6 +188,20 @@ __global__ __launch_bounds__(256 * KS, 2) void proj_gemm_kernel(ProjParams p) {
     ++t;
   };
   while (t < steps - (NS - 1)) step(std::true_type(), std::integral_constant<int, NS - 2>());
+  // The cosines and sines of the first four tokens that this lane turns are on their way while the last steps multiply.  (Asked for
+  // one token after the other behind the exchange, a layer's 500 tokens took 35.0 us instead of 34.0, 1000 63.8 instead of 61.3.)
+  const int ch = tid % kPairs, feature = feature_chunk(ch) * 8;      // its partner is 64 further on
+  auto token = [&](int i) __attribute__((always_inline)) { return (i * 256 * KS + tid) / kPairs; };
+  auto turn_at = [&](int i) __attribute__((always_inline)) {
+    const int64_t m = m0 + (token(i) < rows_left ? token(i) : 0);
+    return turn_of(p.cos + m * p.cos_sn + feature % 128, p.sin + m * p.sin_sn + feature % 128);
+  };
+  Turn turns[kTurnsAhead];
+  if (kRope) {
+#pragma unroll
+    for (int i = 0; i < kTurnsAhead; ++i) turns[i] = turn_at(i);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   auto last = [&](auto left) __attribute__((always_inline)) {
     if (t < steps) step(std::false_type(), left);
   };
@@ -196,8 +213,7 @@ __global__ __launch_bounds__(256 * KS, 2) void proj_gemm_kernel(ProjParams p) {
   last(std::integral_constant<int, 0>());
   // every copy has landed and every fragment has been read: the LDS takes the tile, token-major, chunk c of token m at
   // c ^ (m & (chunks - 1))
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  constexpr int kChunks = 8 * NB;
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   char* const tile = lds + (KS - 1) * 4 * NB * MB * 4096;
   if (KS == 2) {
     f32x4* const half = reinterpret_cast<f32x4*>(lds + (wave & 3) * NB * MB * 4096) + lane;
@@ -238,20 +254,21 @@ __global__ __launch_bounds__(256 * KS, 2) void proj_gemm_kernel(ProjParams p) {
       }
     }
   __syncthreads();
-  // chunk pairs (rotation partners): kChunks / 2 lanes write a token's
-  constexpr int kPairs = kChunks / 2;
+  // kPairs lanes write a token's
   __bf16* const y = p.y[t3];
   const int64_t y_sn = p.n[t3];
 #pragma unroll
-  for (int i = 0; i < (kM * kPairs + 256 * KS - 1) / (256 * KS); ++i) {
-    const int m = (i * 256 * KS + tid) / kPairs, ch = tid % kPairs;
+  for (int i = 0; i < kTurns; ++i) {
+    const int m = token(i);
     if (m >= kM || m >= rows_left) break;
     const char* row = tile + m * (kN * 2);
     bf16x8 y0 = *reinterpret_cast<const bf16x8*>(row + ((ch ^ (m & (kChunks - 1))) << 4));
     bf16x8 y1 = *reinterpret_cast<const bf16x8*>(row + (((ch + kPairs) ^ (m & (kChunks - 1))) << 4));
-    const int f = feature_chunk(ch) * 8;             // its partner's is 64 further on
-    if (kRope && t3 < 2) rotate_chunks(y0, y1, p.cos + (int64_t)(m0 + m) * p.cos_sn + f % 128, p.sin + (int64_t)(m0 + m) * p.sin_sn + f % 128);
-    __bf16* const at = y + (int64_t)(m0 + m) * y_sn + f;
+    if (kRope && t3 < 2) {
+      rotate_chunks(y0, y1, turns[i % kTurnsAhead]);
+      if (i + kTurnsAhead < kTurns) turns[i % kTurnsAhead] = turn_at(i + kTurnsAhead);
+    }
+    __bf16* const at = y + (int64_t)(m0 + m) * y_sn + feature;
     *reinterpret_cast<bf16x8*>(at) = y0;
     *reinterpret_cast<bf16x8*>(at + 64) = y1;
   }

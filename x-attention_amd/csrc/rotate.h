@@ -17,14 +17,20 @@ __device__ __forceinline__ void rotate_pair(float& x0, float& x1, float c0, floa
 }
 #pragma clang fp contract(fast)
 
-// 16-byte chunks f .. f + 7 (y0) and f + 64 .. f + 71 (y1) of a head, f < 64; cs and sn point at the token's values of feature f
-__device__ __forceinline__ void rotate_chunks(bf16x8& y0, bf16x8& y1, const __bf16* cs, const __bf16* sn) {
-  const bf16x8 c0 = *reinterpret_cast<const bf16x8*>(cs), c1 = *reinterpret_cast<const bf16x8*>(cs + 64);
-  const bf16x8 s0 = *reinterpret_cast<const bf16x8*>(sn), s1 = *reinterpret_cast<const bf16x8*>(sn + 64);
+// What a token's chunks f .. f + 7 and f + 64 .. f + 71 are turned by; cs and sn point at the token's values of feature f
+struct Turn {
+  bf16x8 c0, c1, s0, s1;
+};
+__device__ __forceinline__ Turn turn_of(const __bf16* cs, const __bf16* sn) {
+  return {*reinterpret_cast<const bf16x8*>(cs), *reinterpret_cast<const bf16x8*>(cs + 64), *reinterpret_cast<const bf16x8*>(sn),
+          *reinterpret_cast<const bf16x8*>(sn + 64)};
+}
+// 16-byte chunks f .. f + 7 (y0) and f + 64 .. f + 71 (y1) of a head, f < 64
+__device__ __forceinline__ void rotate_chunks(bf16x8& y0, bf16x8& y1, const Turn& t) {
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     float a = (float)y0[e], b = (float)y1[e];
-    rotate_pair(a, b, (float)c0[e], (float)c1[e], (float)s0[e], (float)s1[e]);
+    rotate_pair(a, b, (float)t.c0[e], (float)t.c1[e], (float)t.s0[e], (float)t.s1[e]);
     y0[e] = (__bf16)a;
     y1[e] = (__bf16)b;
   }
