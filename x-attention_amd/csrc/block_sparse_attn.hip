@@ -110,16 +110,12 @@ bool xattn::attention_queued(int num_heads, int q_len, int k_len, int causal) {
 }
 
 // Whether a unit is two workgroups', of 64 rows each, with a wavefront for half of every tile's keys: where units leave half of the
-// CUs idle.  Only where no list is ever cut: up to 16 key blocks (plan_shape), or on a longer cache of which the estimate sees no more
-// than that (its attention, 500 tokens on 8700 12.7 -> 11.8 us, 400 on 3000 12.3 -> 10.4, 400 of 28 / 4 heads on 2000 12.2 -> 10.4; 64
-// tokens, which leave the second half without rows, 5.2 -> 5.4).  It depends on the whole problem alone.  A prompt of 500
+// CUs idle.  Only up to 16 key blocks, where no list is ever cut (plan_shape); it depends on the whole problem alone.  A prompt of 500
 // tokens 23.3 -> 21.5 us, 1000 with 8 heads 25.9 -> 23.1, 900 with 16 29.2 -> 25.6.  Two such workgroups on a CU gain where lists are
 // long and lose where they are short (192 units 32 heads 26.5 -> 24.5 us, 168 units of 28 heads 22.5 -> 23.6, 252 28.4 -> 31.3).
 // Dense attention without lists has whole units always: the sums' order differs, and its q-blocks are those of a longer prompt to the
 // bit.  (With lists they are not, across this line: the same q-blocks in a call of more heads or tokens may differ in the last bits.)
-static bool in_halves(int H, int q_len, int nqb, int nkb, int most_blocks) {
-  return (nkb <= 16 || (most_blocks <= 16 && q_len > 64)) && (int64_t)H * nqb <= 128;
-}
+static bool in_halves(int H, int nqb, int nkb) { return nkb <= 16 && (int64_t)H * nqb <= 128; }
 
 // Bytes of output from which the 32-row kernel stores its rows not temporal: they then leave the memory-side cache to q, k and v, which
 // the estimate has just read.  Prompts, us: 4096 tokens of 32 / 32 heads 88.5 -> 87.1, 6500 134.8 -> 132.3, 5000 of 32 / 8 124.3 -> 117.1, 6500 of
@@ -149,14 +145,14 @@ static int not_temporal(const AttnParams& p, bool lists) {
 
 // `ids` units and pieces; with a queue, `places` workgroups of the 64-row kernel.
 template <bool kHasList, bool kPlanned>
-static int launch_fwd(const AttnParams& p, int64_t ids, int places, int most_blocks, hipStream_t s) {
+static int launch_fwd(const AttnParams& p, int64_t ids, int places, hipStream_t s) {
   const bool all64 = all_rows64(p.H, p.nqb, p.nkb, p.causal);
   if (all64 || p.lists_decide) {
     hipLaunchKernelGGL((block_sparse_fwd64_kernel<kHasList, kPlanned>), dim3((unsigned)(p.queue ? places : ids)), dim3(128), 0, s, p);
     if (hipGetLastError() != hipSuccess) return XATTN_ERR_LAUNCH;
   }
   if (all64) return XATTN_OK;
-  if (kHasList && !kPlanned && in_halves(p.H, p.Lq, p.nqb, p.nkb, most_blocks)) {
+  if (kHasList && !kPlanned && in_halves(p.H, p.nqb, p.nkb)) {
     hipLaunchKernelGGL((block_sparse_fwd_kernel<true, false, true, kNtNone>), dim3((unsigned)(2 * ids)), dim3(256), 0, s, p);
   } else {
     auto kernel = block_sparse_fwd_kernel<kHasList, kPlanned, false, kNtNone>;
@@ -179,7 +175,7 @@ int xattn::block_sparse_impl(const void* q, const void* k, const void* v, void* 
                                       int64_t o_stride_h, int64_t o_stride_n, int q_block_begin, int q_block_end,
                                       int causal, float softmax_scale, void* stream,
                                       const AttnPlan* plan, bool note, int32_t* queue,
-                                      uint32_t* totals, bool ready, int most_blocks) {
+                                      uint32_t* totals, bool ready) {
   if (!q || !k || !v || !out) return XATTN_ERR_NULL;
   if (head_dim != kHeadDim) return XATTN_ERR_HEAD_DIM;
   if (num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads) return XATTN_ERR_HEADS;
@@ -235,10 +231,9 @@ int xattn::block_sparse_impl(const void* q, const void* k, const void* v, void* 
     hipLaunchKernelGGL(ready_kernel, dim3((unsigned)(q_block_end - q_block_begin)), dim3(64), 0, s, p, queue, totals);
   if (plan) {
     if (note) hipLaunchKernelGGL(note_lists_kernel, dim3(1), dim3(1024), 0, s, p);
-    return col_idx ? launch_fwd<true, true>(p, ids, places, p.nkb, s) : launch_fwd<false, true>(p, ids, places, p.nkb, s);
+    return col_idx ? launch_fwd<true, true>(p, ids, places, s) : launch_fwd<false, true>(p, ids, places, s);
   }
-  if (most_blocks <= 0 || most_blocks > p.nkb) most_blocks = p.nkb;
-  return col_idx ? launch_fwd<true, false>(p, ids, places, most_blocks, s) : launch_fwd<false, false>(p, ids, places, most_blocks, s);
+  return col_idx ? launch_fwd<true, false>(p, ids, places, s) : launch_fwd<false, false>(p, ids, places, s);
 }
 
 extern "C" int xattn_block_sparse_fwd(const void* q, const void* k, const void* v, void* out,
@@ -251,7 +246,7 @@ extern "C" int xattn_block_sparse_fwd(const void* q, const void* k, const void* 
                                       int causal, float softmax_scale, void* stream) {
   return block_sparse_impl(q, k, v, out, col_idx, col_cnt, idx_pitch, idx_rows, idx_row0, num_heads, num_kv_heads, q_len, k_len,
                            head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n, o_stride_h,
-                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, nullptr, false, nullptr, nullptr, true, 0);
+                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, nullptr, false, nullptr, nullptr, true);
 }
 
 namespace {
@@ -312,7 +307,7 @@ extern "C" int xattn_block_sparse_fwd_ws(const void* q, const void* k, const voi
   }
   return block_sparse_impl(q, k, v, out, col_idx, col_cnt, idx_pitch, idx_rows, idx_row0, num_heads, num_kv_heads, q_len, k_len,
                            head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n, o_stride_h,
-                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, plan.noted ? &plan : nullptr, true, queue, totals, false, 0);
+                           o_stride_n, q_block_begin, q_block_end, causal, softmax_scale, stream, plan.noted ? &plan : nullptr, true, queue, totals, false);
 }
 
 bool xattn::attention_asks_totals(int num_heads, int q_len, int k_len, int causal) {

@@ -40,8 +40,7 @@ int resident_workgroups();
 size_t estimate_real_rows_bytes(int num_heads, int q_len, int k_len, int stride, int block_size, int chunk_size);
 
 // xattn_block_sparse_fwd, with a plan (null: no list is cut) whose long lists are noted or still to be noted, and a queue of
-// kQueueBytes zeros (null: a workgroup for each list and piece) and the q-blocks' totals - or, not ready, room for them; most_blocks:
-// what no list has more of, where the caller knows (0: it doesn't)
+// kQueueBytes zeros (null: a workgroup for each list and piece) and the q-blocks' totals - or, not ready, room for them
 constexpr size_t kQueueBytes = 4096;
 bool attention_queued(int num_heads, int q_len, int k_len, int causal);
 // whether the attention asks for the blocks of each q-block's lists and of its longest, 128 bytes apart (null: it finds them)
@@ -51,6 +50,6 @@ int block_sparse_impl(const void* q, const void* k, const void* v, void* out, co
                       int head_dim, int64_t q_stride_h, int64_t q_stride_n, int64_t k_stride_h, int64_t k_stride_n,
                       int64_t v_stride_h, int64_t v_stride_n, int64_t o_stride_h, int64_t o_stride_n, int q_block_begin,
                       int q_block_end, int causal, float softmax_scale, void* stream, const AttnPlan* plan, bool note,
-                      int32_t* queue, uint32_t* totals, bool ready, int most_blocks);
+                      int32_t* queue, uint32_t* totals, bool ready);
 
 }  // namespace xattn

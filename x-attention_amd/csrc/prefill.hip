@@ -85,8 +85,7 @@ extern "C" int xattn_prefill_fwd(const void* q, const void* k, const void* v, vo
   // estimate in the same kernel.
   const int q_chunks = (int)(((int64_t)q_len + chunk_size - 1) / chunk_size), k_chunks = (int)(((int64_t)k_len + chunk_size - 1) / chunk_size);
   const int64_t last_token = (int64_t)l.nqb * 128 - 1 + (int64_t)(k_chunks - q_chunks) * chunk_size;   // on the key axis, both padded
-  const int most_blocks = !causal || keep_sink || last_token / 128 + 1 > l.nkb ? l.nkb : (int)(last_token / 128 + 1);      // of a list
-  const bool may_cut = l.plan.per_qb && most_blocks > l.plan.min_piece;
+  const bool may_cut = l.plan.per_qb && (!causal || keep_sink || last_token / 128 + 1 > l.plan.min_piece);
   if (may_cut && zero_rows_from != 0) sel.plan = &plan;
   // Ahead of what is noted lie the attention's queue and the q-blocks' totals; the estimate clears them together.
   const bool cleared = zero_rows_from != 0, queued = cleared && attention_queued(num_heads, q_len, k_len, causal);
@@ -104,7 +103,7 @@ extern "C" int xattn_prefill_fwd(const void* q, const void* k, const void* v, vo
   if (rc != XATTN_OK) return rc;
   return block_sparse_impl(q, k, v, out, sel.col_idx, sel.col_cnt, l.nkb, l.nqb, 0, num_heads, num_kv_heads, q_len,
                            k_len, head_dim, q_stride_h, q_stride_n, k_stride_h, k_stride_n, v_stride_h, v_stride_n,
-                           o_stride_h, o_stride_n, 0, l.nqb, causal, softmax_scale, stream, may_cut ? &plan : nullptr, !sel.plan, queue, sel.totals, true, most_blocks);
+                           o_stride_h, o_stride_n, 0, l.nqb, causal, softmax_scale, stream, may_cut ? &plan : nullptr, !sel.plan, queue, sel.totals, true);
 }
 
 extern "C" int xattn_estimate_fwd(const void* q, const void* k, void* block_sums, uint8_t* mask, void* workspace,
