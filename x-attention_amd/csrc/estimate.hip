@@ -261,20 +261,16 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
     return i * (int)q_snb + (t & 1) * kDepth * 2;
   };
   // Piece j (0..7) of k-step t: slab rows it = j / 2 of K' (j even) or Q' (j odd), 8 rows per wavefront.  It is
-  // loaded into R[j] during step t - 2 and written to LDS stage t % 2 during step t - 1.  Steps `steps` and
-  // `steps + 1` are steps 0 and 1 of the next tile (of this tile again when it is the workgroup's last: a harmless
-  // repeat nobody reads).
+  // loaded into R[j] during step t - 2 and written to LDS stage t % 2 during step t - 1.  The last two steps load steps
+  // 0 and 1 of the next tile (of this tile again when it is the workgroup's last: a harmless repeat nobody reads).
   u32x4 R[8];
   auto load_j = [&](int j, int t) __attribute__((always_inline)) {
-    const bool ahead = t >= steps;
-    const int tc = ahead ? t - steps : t;
     if (j & 1)
       R[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-          ahead ? qres_next[(j >> 1) % kQRes] : qres[(j >> 1) % kQRes],
-          (int)((unsigned)voffQ[kPacked ? 0 : j >> 1] + (unsigned)step_off_q(tc)), 0, 0));
+          qres[(j >> 1) % kQRes], (int)((unsigned)voffQ[kPacked ? 0 : j >> 1] + (unsigned)step_off_q(t)), 0, 0));
     else
       R[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-          ahead ? kres_next : kres, (int)((unsigned)voffK[j >> 1] + (unsigned)step_off_k(tc)), 0, 0));
+          kres, (int)((unsigned)voffK[j >> 1] + (unsigned)step_off_k(t)), 0, 0));
   };
   const int lane_dst = wave * 8 * 128 + lane * 16;
   auto write_j = [&](int j, char* stage) __attribute__((always_inline)) {
@@ -300,22 +296,10 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
   for (int x = 0; x < kMT; ++x) fb[0][x] = read_frag(lds + kTile * 128, wm * 32 * kMT + x * 32 + r, hh);
 
   for (;;) {
-  const int64_t id_next = id + gridDim.x;
-  int head_next, m0_next, n0_next;
-  const bool more = decode(id_next, &head_next, &m0_next, &n0_next);
-  if (more) {
-    q_resources(qres_next, head_next, m0_next);
-    kres_next = k_resource(head_next, n0_next);
-  }
   f32x16 acc[4][kMT];   // [key tile nt][query tile mt]
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < kMT; ++b)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.f;
-
-  for (int t = 0; t < steps; ++t) {
+  // Step t, loading for step `ahead`; `first`: the sums start at zero.  (As the first MFMAs' constant operand; written into the registers
+  // by themselves they were 128 instructions of each wavefront between two tiles, with the matrix pipes idle.)
+  auto step = [&](int t, int ahead, auto first) __attribute__((always_inline)) {
     char* cur = lds + (t & 1) * kStageBytes;
     char* nxt = lds + ((t + 1) & 1) * kStageBytes;
 #pragma unroll
@@ -338,7 +322,7 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
           // (half tiles have no rows for the odd pieces from 5 on)
           if (ss < 3 && c < 3 && j < 8 && !(kHalf && (j & 1) && j >= 5)) {
             write_j(j, nxt);
-            load_j(j, t + 2);
+            load_j(j, ahead);
           }
         }
         if (c < 2) {
@@ -349,11 +333,53 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
           if (kMT == 2) fb[(ss + 1) & 1][kMT - 1] = read_frag(fragQ, wm * 32 * kMT + 32 + r, nss * 2 + hh);
         }
 #pragma unroll
-        for (int mt = 0; mt < kMT; ++mt) acc[c][mt] = mfma32(fa[ss & 1][c], fb[ss & 1][mt], acc[c][mt]);
+        for (int mt = 0; mt < kMT; ++mt) {
+          const f32x16 zero = {};
+          acc[c][mt] = mfma32(fa[ss & 1][c], fb[ss & 1][mt], decltype(first)::value && ss == 0 ? zero : acc[c][mt]);
+        }
       }
     }
     __builtin_amdgcn_sched_barrier(0);
+  };
+  // The next tile is found while the matrix pipes are busy, by one key half's wavefronts a step after the other's: a SIMD has one of
+  // each, and the other's MFMAs go on.  (Table launches may have two steps only.)  With the sums' zeros above, the masks of a diagonal tile
+  // only where a 32-key tile needs them and stores without branches, us: estimate of 15000 tokens, stride 8, 152.9 -> 145.6, estimator of
+  // 32768 500 -> 491 (1.19 PFLOP/s), of 2048 on 63488 67.6 -> 65.9; at 1.2 to 1.3 PFLOP/s power is the limit, 131072 7347 -> 7328.
+  const int64_t id_next = id + gridDim.x;
+  int head_next, m0_next, n0_next;
+  bool more = false;
+  auto next = [&]() __attribute__((always_inline)) {
+    more = decode(id_next, &head_next, &m0_next, &n0_next);
+    if (more) {
+      q_resources(qres_next, head_next, m0_next);
+      kres_next = k_resource(head_next, n0_next);
+    }
+  };
+  const std::integral_constant<bool, true> yes;
+  const std::integral_constant<bool, false> no;
+  int t = 0;
+  if (kTable) {
+    next();
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < kMT; ++b) acc[a][b] = f32x16{};
+  } else {
+    asm volatile("" : "+s"(t));      // (or addresses of either stage are kept in registers from tile to tile, more than there are)
+    step(t, t + 2, yes);
+    ++t;
   }
+  for (; t < steps - 2; ++t) {
+    if (!kTable && t == steps - 3 - wn) next();
+    step(t, t + 2, no);
+  }
+#pragma unroll
+  for (int w = 0; w < kQRes; ++w) qres[w] = qres_next[w];
+  kres = kres_next;
+  int u = 0;                   // (an even number of steps)
+  asm volatile("" : "+s"(u));
+  step(u, u, no);
+  step(u + 1, u + 1, no);
   // fa[0] / fb[0] now hold the first fragments of the next tile, whose step 0 sits in stage 0 and whose step 1
   // is on its way into stage 1
 
@@ -388,14 +414,21 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
     // then drop out of the maximum and exponentiate to zero, and the two passes below need neither a test per
     // score nor a second copy.
     if (!all_visible) {
+      const int at = nbase + hh * 4, last = (hi < p.n_rk - 1 ? hi : p.n_rk - 1) - at;
+      int whole = row_hi(p, mw0 + mt * 32);                     // keys that all of the pass's rows see
+      whole = whole < p.n_rk - 1 ? whole : p.n_rk - 1;
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt)
+      for (int nt = 0; nt < 4; ++nt) {
+        if (nbase + nt * 32 + 31 <= whole) continue;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int n = nbase + nt * 32 + (v >> 2) * 8 + hh * 4 + (v & 3);
-          const bool vis = n >= lo && n <= hi && n < p.n_rk;
-          acc[nt][mt][v] = vis ? acc[nt][mt][v] : -INFINITY;
-        }
+        for (int v = 0; v < 16; ++v) acc[nt][mt][v] = nt * 32 + (v >> 2) * 8 + (v & 3) <= last ? acc[nt][mt][v] : -INFINITY;
+      }
+      if (p.own_chunk_only) {
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) acc[nt][mt][v] = nt * 32 + (v >> 2) * 8 + (v & 3) >= lo - at ? acc[nt][mt][v] : -INFINITY;
+      }
     }
     // pass 1: row maximum over this tile's visible keys (exp2 domain)
     float mx = -INFINITY;
@@ -407,14 +440,18 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
     mx = half_max(mx);
     const float safe = (mx == -INFINITY) ? 0.f : mx;
     float tot = 0.f;
-    const int mrel = m - p.row_begin;
     constexpr int G = RBS / 8;   // 8-key groups (one per accumulator quad pair) per key block
-    // what the stores below share: the first key block of this wavefront tile and how many of its key blocks
-    // exist (uniform), each lane's place in P and the key blocks that it may store
+    // Stores are buffer stores whose resource ends behind the last key block (the last row, for the statistics), from the lanes that
+    // have no place in it to an offset outside: no branches, the sums of one 32-key tile are under way while another's are stored.
     const int kb_first = (int)((uint32_t)nbase / (uint32_t)RBS);
-    const int kb_left = p.nkb - kb_first;
-    float* const prow = p.P + partial_at(p, own.head, row_ok ? mrel : 0) + (int64_t)(kb_first + (G < 4 ? hh : 0)) * kStrip;
-    const int st = !row_ok ? 0 : G < 4 ? kb_left - hh : hh == 0 ? kb_left : 0;
+    const int row0 = mw0 + mt * 32 - p.row_begin;           // first of the pass's 32 rows, a strip of P
+    const int kNowhere = 0x7ffff000;
+    const __amdgpu_buffer_rsrc_t pres = __builtin_amdgcn_make_buffer_rsrc(
+        p.P + ((int64_t)(own.head * strips_of(p.rows) + row0 / kStrip) * p.nkb + kb_first) * kStrip, 0, (p.nkb - kb_first) * kStrip * 4, 0x00020000);
+    const int st = row_ok && (G < 4 || hh == 0) ? (r + (G < 4 ? hh * kStrip : 0)) * 4 : kNowhere;
+    auto put = [&](int k, float x) __attribute__((always_inline)) {
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), pres, st + k * kStrip * 4, 0, 0);
+    };
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
       float s[4];       // this lane's share of the sums over keys nbase + nt*32 + 8g .. +7 (the other half-wave has the rest)
@@ -436,24 +473,23 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
           const float both = half_sum_pair(s[2 * q2], s[2 * q2 + 1]);
           tot += both;
           const int k = nt * 4 + 2 * q2;
-          if (k < st) prow[k * kStrip] = both;
+          put(k, both);
         }
       } else if (G == 2) {
         const float both = half_sum_pair(s[0] + s[1], s[2] + s[3]);
         tot += both;
         const int k = nt * 2;
-        if (k < st) prow[k * kStrip] = both;
+        put(k, both);
       } else {
         const float all = half_sum(s[0] + s[1] + s[2] + s[3]);
         tot += hh == 0 ? all : 0.f;
-        if (nt < st) prow[nt * kStrip] = all;
+        put(nt, all);
       }
     }
     tot = half_sum(tot);
-    if (row_ok && hh == 0) {
-      Mst[mrel] = mx;
-      Lst[mrel] = tot;
-    }
+    const int left = (p.live_end - p.row_begin - row0) * 4, so = hh == 0 ? r * 4 : kNowhere;
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, mx), __builtin_amdgcn_make_buffer_rsrc(Mst + row0, 0, left > 0 ? left : 0, 0x00020000), so, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, tot), __builtin_amdgcn_make_buffer_rsrc(Lst + row0, 0, left > 0 ? left : 0, 0x00020000), so, 0, 0);
     // keep the query-tile passes apart: interleaving them only lengthens live ranges
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -464,9 +500,6 @@ __global__ __launch_bounds__(512) void estimate_gemm_kernel(EstParams p) {
   head = head_next;
   m0 = m0_next;
   n0 = n0_next;
-#pragma unroll
-  for (int w = 0; w < kQRes; ++w) qres[w] = qres_next[w];
-  kres = kres_next;
   }   // tiles of this workgroup
 }
 

@@ -238,10 +238,12 @@ __global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p, Sel
   for (int a = 0; a < MT; ++a) {
     const int m = m0 + ((a * 32 + r) & (p.tile_rows - 1));
     const int lo = row_lo(p, m), hi = row_hi(p, m);
+    const int at = n_w + hh * 4, last = (hi < p.n_rk - 1 ? hi : p.n_rk - 1) - at;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int n = n_w + (v >> 2) * 8 + hh * 4 + (v & 3);
-      acc[a][v] = n >= lo && n <= hi && n < p.n_rk ? acc[a][v] : -INFINITY;
+    for (int v = 0; v < 16; ++v) acc[a][v] = (v >> 2) * 8 + (v & 3) <= last ? acc[a][v] : -INFINITY;
+    if (p.own_chunk_only) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[a][v] = (v >> 2) * 8 + (v & 3) >= lo - at ? acc[a][v] : -INFINITY;
     }
     float w = -INFINITY;
 #pragma unroll
