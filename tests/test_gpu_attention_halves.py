@@ -47,9 +47,21 @@ def test_few_units(q_len, k_len, heads, kv_heads, causal):
     check(q_len, k_len, heads, kv_heads, causal)
 
 
+# 129 to 256 units of at most 16 key blocks, with a workgroup of eight wavefronts each, half of a tile's keys per wavefront: keys that end
+# in a tile's first half, at its edge and in the second, rows that see no key of a half, lists of one block and of 16; and beyond: 252
+# units that the dispatch deals unevenly, 257, 17 key blocks
+@pytest.mark.parametrize("q_len,k_len,heads,kv_heads,causal", [
+    (1000, 1000, 32, 8, True), (1024, 1024, 32, 32, True), (600, 600, 43, 43, True), (512, 1060, 64, 8, False), (65, 2048, 129, 3, True),
+    (127, 130, 256, 1, True), (1, 1, 200, 8, True), (700, 1111, 32, 8, True), (900, 2048, 28, 4, False), (1100, 1100, 28, 4, True), (1, 100, 257, 257, True),
+    (129, 2100, 128, 2, True),
+])
+def test_units_no_more_than_cus(q_len, k_len, heads, kv_heads, causal):
+    check(q_len, k_len, heads, kv_heads, causal)
+
+
 # queries as [tokens][heads] views, keys and values inside a larger cache, the output inside a larger buffer; and q-blocks spread over
 # launches, which have the whole call's bits (halves are the whole problem's choice, not a launch's)
-@pytest.mark.parametrize("q_len,k_len,heads,kv_heads,causal", [(500, 500, 32, 8, True), (513, 1300, 16, 2, True), (1000, 1000, 8, 8, False), (129, 2048, 28, 4, True)])
+@pytest.mark.parametrize("q_len,k_len,heads,kv_heads,causal", [(500, 500, 32, 8, True), (513, 1300, 16, 2, True), (1000, 1000, 8, 8, False), (129, 2048, 28, 4, True), (1000, 1000, 32, 8, True), (300, 4000, 28, 4, True)])
 def test_few_units_of_strided_views_and_in_windows(q_len, k_len, heads, kv_heads, causal):
     from xattn.src.Xattention import block_sparse_attention
 

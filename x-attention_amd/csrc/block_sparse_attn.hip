@@ -9,6 +9,8 @@
 // dense FlashAttention baseline the speedup is quoted against.
 #include "attn_rows32.h"
 #include "attn_rows64.h"
+#include "attn_wide.h"
+#include "lds_limit.h"
 #include "estimate.h"
 #include "xattn_hip.h"
 
@@ -111,11 +113,18 @@ bool xattn::attention_queued(int num_heads, int q_len, int k_len, int causal) {
 
 // Whether a unit is two workgroups', of 64 rows each, with a wavefront for half of every tile's keys: where units leave half of the
 // CUs idle.  Only up to 16 key blocks, where no list is ever cut (plan_shape); it depends on the whole problem alone.  A prompt of 500
-// tokens 23.3 -> 21.5 us, 1000 with 8 heads 25.9 -> 23.1, 900 with 16 29.2 -> 25.6.  Two such workgroups on a CU gain where lists are
-// long and lose where they are short (192 units 32 heads 26.5 -> 24.5 us, 168 units of 28 heads 22.5 -> 23.6, 252 28.4 -> 31.3).
+// tokens 23.3 -> 21.5 us, 1000 with 8 heads 25.9 -> 23.1, 900 with 16 29.2 -> 25.6.  (From there to the CUs' number: in_wide.)
 // Dense attention without lists has whole units always: the sums' order differs, and its q-blocks are those of a longer prompt to the
 // bit.  (With lists they are not, across this line: the same q-blocks in a call of more heads or tokens may differ in the last bits.)
 static bool in_halves(int H, int nqb, int nkb) { return nkb <= 16 && (int64_t)H * nqb <= 128; }
+
+// Whether a unit is a workgroup of eight wavefronts (attn_wide.h), one to a CU: where no XCD gets more of them than it has CUs (a prompt of
+// 1100 tokens with 28 heads, whose 252 units the dispatch deals 36 to an XCD, 27.7 -> 31.5 us).  Only up to 16 key blocks: a workgroup
+// that has the CU alone leaves it idle at a piece's start and end (500 tokens on 60000 151.5 -> 157.6, 1000 on 30000 182 -> 200; uncut
+// 500 on 8700 gained 0.7 of 22.3), and cut or not the choice has to be one.  It depends on the whole problem alone, too.
+static bool in_wide(int H, int Hkv, int nqb, int nkb) {
+  return nkb <= 16 && (int64_t)H * nqb <= 256 && fullest_xcd(dispatch_shape(H, Hkv, nqb), nqb) <= kUnit / 2;
+}
 
 // Bytes of output from which the 32-row kernel stores its rows not temporal: they then leave the memory-side cache to q, k and v, which
 // the estimate has just read.  Prompts, us: 4096 tokens of 32 / 32 heads 88.5 -> 87.1, 6500 134.8 -> 132.3, 5000 of 32 / 8 124.3 -> 117.1, 6500 of
@@ -154,6 +163,10 @@ static int launch_fwd(const AttnParams& p, int64_t ids, int places, hipStream_t 
   if (all64) return XATTN_OK;
   if (kHasList && !kPlanned && in_halves(p.H, p.nqb, p.nkb)) {
     hipLaunchKernelGGL((block_sparse_fwd_kernel<true, false, true, kNtNone>), dim3((unsigned)(2 * ids)), dim3(256), 0, s, p);
+  } else if (kHasList && !kPlanned && in_wide(p.H, p.Hkv, p.nqb, p.nkb)) {
+    static LdsLimit limit;
+    if (limit.raise(reinterpret_cast<const void*>(&block_sparse_wide_kernel)) != hipSuccess) return XATTN_ERR_LAUNCH;
+    hipLaunchKernelGGL(block_sparse_wide_kernel, dim3((unsigned)ids), dim3(512), kWideLds, s, p);
   } else {
     auto kernel = block_sparse_fwd_kernel<kHasList, kPlanned, false, kNtNone>;
     const int nt = not_temporal(p, kHasList);
