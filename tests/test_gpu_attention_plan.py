@@ -208,3 +208,32 @@ def test_nothing_but_the_pieces_of_a_list_is_combined(cut, q_len, k_len, heads, 
     want = _swept_whole(q, k, v, idx, cnt, False)
     bound = 2.0 ** -8 * (v.float().abs().amax() + want.abs())      # as above
     assert ((outs[1] - want).abs() <= bound).all()
+
+
+# Some KV heads' lists long, with rests of every length, the others short and whole (dealt to the XCDs in turn): KV heads fewer, as many
+# and more than XCDs, heads that are no multiple of 8, a ragged last q-block, windows of q-blocks.  Every unit is written, once.
+@pytest.mark.parametrize("q_len,k_len,heads,kv_heads", [(512, 8000, 12, 12), (640, 6100, 28, 4), (1000, 9000, 32, 8), (384, 7000, 15, 5), (1100, 6000, 3, 1)])
+def test_rests_and_short_lists_beside_long_ones(q_len, k_len, heads, kv_heads):
+    from xattn.src.Xattention import block_sparse_attention
+
+    q, k, v = _inputs(q_len, k_len, heads, kv_heads, q_len + heads)
+    nq, nk = -(-q_len // 128), -(-k_len // 128)
+    g = torch.Generator().manual_seed(heads)
+    cnt = torch.randint(1, 12, (heads, nq), generator=g)
+    longs = torch.arange(heads) // (heads // kv_heads) % 3 != 1
+    cnt[longs] = torch.randint(17, nk - nq, (int(longs.sum()), nq), generator=g)
+    idx = torch.full((heads, nq, nk), nk - 1, dtype=torch.int32)
+    for h in range(heads):
+        for r in range(nq):
+            seen = (min(r * 128 + 127, q_len - 1) + k_len - q_len) // 128 + 1
+            idx[h, r, :cnt[h, r]] = torch.randperm(seen, generator=g)[:cnt[h, r]].sort().values.int()
+    idx, cnt = idx.cuda(), cnt.int().cuda()
+    want = _swept_whole(q, k, v, idx, cnt, True)
+    got = block_sparse_attention(q, k, v, idx, cnt, causal=True)
+    bound = 2.0 ** -8 * (v.float().abs().amax() + want.abs())        # as above
+    assert ((got.float() - want).abs() <= bound).all()
+    assert (got.float() - want).norm() <= 4e-3 * want.norm()
+    parts = torch.full((1, q_len, heads, 128), float("nan"), dtype=torch.bfloat16, device="cuda")
+    for a in range(0, nq, 3):
+        block_sparse_attention(q, k, v, idx, cnt, causal=True, out=parts, q_blocks=(a, min(a + 3, nq)))
+    assert torch.equal(parts.transpose(1, 2), got)

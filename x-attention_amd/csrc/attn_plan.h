@@ -29,20 +29,39 @@ struct PlanShape {
   int units;                  // lists of the whole problem, heads x q-blocks
   int nqb;
   int in_turn;                // pieces go to the XCDs in turn
+  int rests_last;             // rests go behind the other pieces (PieceIds)
   int last, last_pieces;      // the problem's last q-block, if rows are missing from it (else -1), and its share
 };
 
 struct AttnPlan {
-  // kNotedStep words apart: pieces noted; then, per q-block, its lists that are made (16 bits), those of them longer than
-  // min_piece (16) and the blocks of all (32).  Set to zero, with `cut` behind it, before lists are noted
+  // kNotedStep words apart: pieces noted, of their list's piece length (32 bits) and rests (32); then, per q-block, its lists that are
+  // made (16 bits), those of them longer than min_piece (16) and the blocks of all (32).  Set to zero, with `cut` behind it, before
+  // lists are noted
   unsigned long long* noted;
   uint32_t* cut;              // [lists] of a list longer than min_piece: its length, until its q-block is noted, then its pieces
                               // (cut_word), or 0 if it stays whole
   int32_t* done;              // [lists] pieces of a cut list that are finished
-  int32_t* pieces;            // [plan_pieces()][2] unit, index of the piece in its list
+  int32_t* pieces;            // [room][2] unit, index of the piece in its list: from the front those of their list's piece length, from the
+                              // end the rests
   float* part;                // [the same][kPartFloats]
+  int room;                   // plan_pieces()
   PlanShape shape;
 };
+
+// Ids of the pieces noted: a multiple of 8 of the long ones, behind them of the rests.  The launch deals ids in order, so the
+// rests, of half a piece on average, fill up the last round: with them among the others the end of a launch was a piece of full
+// length wide (2048 tokens on 63488: the last 80 of 336 us with half of the places empty).  With that, and what stays whole dealt
+// to the XCDs in turn (find_place), calls, us: 2048 on 63488 361 -> 347, on 20000 217 -> 204, 1000 on 30000 182 -> 173, 5000 on 30000
+// 584 -> 563, 700 of 28 / 4 heads on 20000 111 -> 106, 3000 of 32 / 32 on 20000 405 -> 397; 500 on 60000 and 8000 on 100000 equal, 2048 of
+// 32 / 32 on 63488 474 -> 478.  Only on a cache: behind a prompt's pieces its many units fill the end, 4096 tokens of 32 / 32
+// 77.7 -> 78.6, 9000 182 -> 183.5, 12000 of 32 / 8 215 -> 216.5.
+struct PieceIds {
+  int whole, rests;           // pieces
+  __host__ __device__ int whole_ids() const { return (whole + 7) / 8 * 8; }
+  __host__ __device__ int ids() const { return whole_ids() + (rests + 7) / 8 * 8; }
+};
+// ... of which a launch has room for so many.
+inline int64_t piece_ids_room(int64_t pieces) { return pieces ? (pieces + 14) / 8 * 8 : 0; }
 
 // The 512 workgroup slots get about four pieces each (the problem taken to be like the q-block), fewer of which even out
 // less: 2048 tokens on 63488 806 us with up to 8192 pieces, 884 with 2048, 977 with 1024.  Of a prompt by itself, whose
@@ -70,6 +89,7 @@ inline PlanShape plan_shape(int heads, int q_len, int k_len) {
   s.units = (int)units;
   s.nqb = nqb;
   s.in_turn = !cached && units > 2048;
+  s.rests_last = cached;
   const int64_t a_list = (nkb + s.min_piece - 1) / s.min_piece, most = heads * (a_list < kMostPieces ? a_list : kMostPieces);
   const int64_t share = s.spread * 5 / 4 / nqb;
   s.per_qb = (int)(share < most ? share : most);
@@ -95,6 +115,7 @@ inline AttnPlan plan_at(const PlanShape& s, char* at, int64_t lists, int q_block
   p.shape = s;
   if (s.per_qb == 0) return p;
   p.noted = reinterpret_cast<unsigned long long*>(at);
+  p.room = (int)plan_pieces(s, q_blocks);
   p.cut = reinterpret_cast<uint32_t*>(at += plan_noted_bytes(s.nqb));
   p.done = reinterpret_cast<int32_t*>(at += plan_round((size_t)lists * 4));
   p.pieces = reinterpret_cast<int32_t*>(at += plan_round((size_t)lists * 4));
@@ -177,7 +198,8 @@ __host__ __device__ __forceinline__ void read_ahead(int pieces, X& a, X& b, R re
 }
 
 // Notes the lists of q-block qb, `total` blocks in all, by a whole wavefront: count(h) is the length of head h's where it
-// is longer than min_piece, unit0 + h * unit_step its place; reserve(n), called by one lane, gives the place of its n pieces.
+// is longer than min_piece, unit0 + h * unit_step its place; reserve(x), called by one lane, adds x to what is noted of pieces and
+// gives what was.
 template <typename F, typename R>
 __device__ __forceinline__ void note_q_block(const AttnPlan& p, int qb, int heads, int total, int unit0, int unit_step, int lane, F count, R reserve) {
   const int first = lane < heads ? count(lane) : 0;
@@ -194,17 +216,26 @@ __device__ __forceinline__ void note_q_block(const AttnPlan& p, int qb, int head
     return __builtin_amdgcn_readlane(upto, 63);
   });
   const int sum = blocks ? __builtin_amdgcn_readlane(upto, 63) : 0;
-  int at = 0;
-  if (lane == 63 && sum > 0) at = reserve(sum);
-  at = __builtin_amdgcn_readlane(at, 63) + upto - mine;
+  auto has_rest = [&](int len, int n) { return n && p.shape.rests_last && len < n * list_piece(len, blocks) ? 1 : 0; };
+  int my_rests = 0, rests_upto = 0;
+  if (p.shape.rests_last) {
+    for (int h = lane; h < heads; h += 64) my_rests += has_rest(length(h), list_pieces(length(h), blocks));
+    rests_upto = wave_scan(my_rests);
+  }
+  const int rests = __builtin_amdgcn_readlane(rests_upto, 63);
+  unsigned long long before = 0;
+  if (lane == 63 && sum > 0) before = reserve((unsigned long long)(uint32_t)rests << 32 | (uint32_t)(sum - rests));
+  const int whole0 = __builtin_amdgcn_readlane((int)(uint32_t)before, 63), rests0 = __builtin_amdgcn_readlane((int)(uint32_t)(before >> 32), 63);
+  int at = whole0 + rests0 + upto - mine, rest = rests0 + rests_upto - my_rests, whole = at - rest;
   for (int h = lane; h < heads; h += 64) {
     const int len = length(h), n = list_pieces(len, blocks), unit = unit0 + h * unit_step;
     if (len <= p.shape.min_piece) continue;
     p.cut[unit] = n ? cut_word(at, n, list_piece(len, blocks)) : 0;
     p.done[unit] = 0;
     for (int i = 0; i < n; ++i) {
-      p.pieces[2 * (at + i)] = unit;
-      p.pieces[2 * (at + i) + 1] = i;
+      const int to = i == n - 1 && has_rest(len, n) ? p.room - 1 - rest++ : whole++;
+      p.pieces[2 * to] = unit;
+      p.pieces[2 * to + 1] = i;
     }
     at += n;
   }
@@ -233,7 +264,7 @@ __device__ __forceinline__ void list_made(const AttnPlan& p, int heads, int rows
   note_q_block(
       p, row, heads, total, row, rows, lane,
       [&](int h) { return (int)__hip_atomic_load(p.cut + (int64_t)h * rows + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); },
-      [&](int n) { return (int)__hip_atomic_fetch_add(p.noted, (unsigned long long)n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); });
+      [&](unsigned long long x) { return __hip_atomic_fetch_add(p.noted, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); });
 }
 
 }  // namespace xattn

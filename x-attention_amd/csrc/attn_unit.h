@@ -107,23 +107,43 @@ __device__ __forceinline__ Unit uniform(const Unit& u) {
   return v;
 }
 
+__device__ __forceinline__ PieceIds pieces_noted(const AttnParams& p) {
+  const const_i32_ptr at = (const_i32_ptr)(uintptr_t)p.plan.noted;
+  return PieceIds{at[0], at[1]};
+}
+
 // The (head, q-block) with this id; false: there is none.
 template <bool kPlanned>
 __device__ __forceinline__ bool find_place(const AttnParams& p, int id, Unit& u) {
   u.piece = -1;
   u.skip = 0;
   if (kPlanned) {
-    const int pieces = ((const_i32_ptr)(uintptr_t)p.plan.noted)[0], per_xcd = (pieces + 7) / 8;   // (the low half)
-    u.skip = per_xcd * 8;
+    const PieceIds noted = pieces_noted(p);
+    u.skip = noted.ids();
     if (id < u.skip) {
-      const int at = p.plan.shape.in_turn ? id : (id & 7) * per_xcd + (id >> 3);
+      int i = id, pieces = noted.whole;
+      const bool rest = id >= noted.whole_ids();
+      if (rest) i -= noted.whole_ids(), pieces = noted.rests;
+      const int at = p.plan.shape.in_turn ? i : (i & 7) * ((pieces + 7) / 8) + (i >> 3);
       if (at >= pieces) return false;
-      const_i32_ptr entry = (const_i32_ptr)(uintptr_t)p.plan.pieces + 2 * at;
+      const_i32_ptr entry = (const_i32_ptr)(uintptr_t)p.plan.pieces + 2 * (rest ? p.plan.room - 1 - at : at);
       const int unit = entry[0];
       u.piece = entry[1];
       u.head = unit / p.idx_rows;
       u.qb = unit - u.head * p.idx_rows + p.idx_row0;
       u.kvh = (int)divided((uint32_t)u.head, p.shape.by_group);
+      return true;
+    }
+    // Where pieces are most of the work, what stays whole are short lists, often of the same few KV heads: they go to the XCDs in
+    // turn, each q-block's heads from another one on (as units of the dispatch, 64 more on some XCDs than on others).
+    const uint32_t rows = (uint32_t)(p.qb_end - p.qb_begin), heads = (uint32_t)p.H, kv_heads = (uint32_t)p.Hkv;
+    if (p.plan.shape.rests_last && 2 * (uint32_t)noted.whole >= rows * heads) {
+      const uint32_t w = (uint32_t)(id - u.skip), row = w / heads;
+      if (row >= rows) return false;
+      const uint32_t turned = (w - row * heads + row) % heads, of = turned / kv_heads;
+      u.kvh = (int)(turned - of * kv_heads);
+      u.head = (int)((uint32_t)u.kvh * (heads / kv_heads) + of);
+      u.qb = p.qb_end - 1 - (int)row;
       return true;
     }
   }
@@ -151,8 +171,7 @@ __device__ __forceinline__ int ask_next(const AttnParams& p) {
 // last time) are left to their own workgroups where a queue has a single one left; so are others after four vain tries.
 template <bool kPlanned>
 __device__ __forceinline__ int next_id(const AttnParams& p, int ticket, int lane, bool few) {
-  const int pieces = kPlanned ? ((const_i32_ptr)(uintptr_t)p.plan.noted)[0] : 0;
-  const int ids = (pieces + 7) / 8 * 8 + p.unit_ids, first = (int)(gridDim.x / kQueues);
+  const int ids = (kPlanned ? pieces_noted(p).ids() : 0) + p.unit_ids, first = (int)(gridDim.x / kQueues);
   const int id = (first + __builtin_amdgcn_readfirstlane(ticket)) * kQueues + (int)(blockIdx.x % kQueues);
   if (id < ids) return id;
   for (int i = 0; i < 4; ++i) {

@@ -19,7 +19,7 @@ namespace xattn {
 // Notes the lists of q-blocks [qb_begin, qb_end) of every head, where the pass that made them has not (or, without
 // lists, the visible blocks of each).  One workgroup, which counts the pieces in LDS.
 __global__ __launch_bounds__(1024) void note_lists_kernel(AttnParams p) {
-  __shared__ int pieces;
+  __shared__ unsigned long long pieces;
   if (threadIdx.x == 0) pieces = 0;
   __syncthreads();
   const int lane = threadIdx.x & 63;
@@ -36,10 +36,10 @@ __global__ __launch_bounds__(1024) void note_lists_kernel(AttnParams p) {
     int total = 0;
     for (int h = lane; h < p.H; h += 64) total += count(h) < 65536 ? count(h) : 65536;   // (a sum of at most 8192)
     note_q_block(p.plan, qb, p.H, __builtin_amdgcn_readlane(wave_scan(total), 63), row, p.idx_rows, lane, count,
-                 [&](int n) { return __hip_atomic_fetch_add(&pieces, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); });
+                 [&](unsigned long long x) { return __hip_atomic_fetch_add(&pieces, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); });
   }
   __syncthreads();
-  if (threadIdx.x == 0) *p.plan.noted = (unsigned long long)pieces;
+  if (threadIdx.x == 0) *p.plan.noted = pieces;
 }
 
 static_assert(kQueueBytes == kQueueWords * 4, "estimate.h");
@@ -230,7 +230,7 @@ int xattn::block_sparse_impl(const void* q, const void* k, const void* v, void* 
   p.plan = plan ? *plan : AttnPlan{};
   p.lists_decide = lists_decide(p.H, p.nqb, p.nkb, p.kv_off, p.causal);
   const int64_t grid = grid_for(p.shape, q_block_end - q_block_begin);
-  const int64_t ids = grid + (plan ? ((int64_t)plan_pieces(plan->shape, q_block_end - q_block_begin) + 7) / 8 * 8 : 0);
+  const int64_t ids = grid + (plan ? piece_ids_room((int64_t)plan_pieces(plan->shape, q_block_end - q_block_begin)) : 0);
   if (ids > 0x7fffffff) return XATTN_ERR_SHAPE;
   p.unit_ids = (int)grid;
   const int cus = resident_workgroups();
