@@ -3,11 +3,32 @@
 // produced exactly once and nothing else.  Prints one line per case; exit
 // status 0 when all hold.  No GPU call is made.
 #include <cstdio>
+#include <utility>
 #include <vector>
 
 #include "attn_tiles.h"
 
+// every unit once by the map for unlike lists, too, whose units of up to 32 have no ids without work but in a run that lacks rows
+static int unlike_faults(int H, int Hkv, int b, int e) {
+  const xattn::DispatchShape d = xattn::unlike_lists_shape(H, Hkv, e - b), whole = xattn::dispatch_shape(H, Hkv, e - b);
+  std::vector<int> seen((size_t)H * (e - b), 0);
+  int faults = d.unit_rows > whole.unit_rows || d.set_heads * d.unit_rows > (int)d.unit_size;
+  for (long id = 0; id < (long)xattn::grid_for(d, e - b); ++id) {
+    int head = -1, qb = -1, kv = -1;
+    if (!xattn::map_workgroup((int)id, d, b, e, &head, &qb, &kv)) continue;
+    if (head < 0 || head >= H || qb < b || qb >= e || kv != head / (H / Hkv)) return 1 << 20;
+    ++seen[(size_t)head * (e - b) + (qb - b)];
+  }
+  for (int v : seen) faults += v != 1;
+  return faults;
+}
+
 int main() {
+  for (const auto& l : {std::pair<int, int>{32, 32}, {32, 8}, {28, 4}, {24, 24}, {1, 1}, {7, 1}, {64, 1}, {71, 1}, {96, 3}, {40, 8}, {14, 2}, {12, 12}, {256, 1}})
+    for (int n : {1, 40, 47, 48, 49, 63, 64, 65, 100, 127, 133, 255, 256, 257, 313, 512, 931, 1024}) {
+      const int faults = unlike_faults(l.first, l.second, n % 5, n % 5 + n);
+      if (faults) return std::printf("unlike lists, H=%d Hkv=%d q-blocks %d: faults %d\n", l.first, l.second, n, faults), 1;
+    }
   const int cases[][4] = {
       // H, Hkv, q-block begin, q-block end
       {32, 8, 0, 1024}, {32, 8, 128, 256}, {28, 4, 0, 512}, {24, 24, 0, 931}, {4, 4, 0, 1},   {7, 1, 0, 19},

@@ -165,6 +165,25 @@ inline DispatchShape dispatch_shape(int H, int Hkv, int n_qblocks) {
   return d;
 }
 
+// The same for q-blocks that keep lists of their own: heads' lists differ many times over, and an XCD that has a head's units of 64
+// q-blocks has all of its long lists.  Units are halved, down to 16 workgroups, until there are 16 runs, over which a KV group goes round
+// the XCDs twice.  Text, us, whole units / halved: 32 / 32 heads 9000 tokens 173 / 170.5, 17000 406 / 342, 32768 815 / 704, 65536 2210 / 1940,
+// 100000 4640 / 4549; 32 / 8 8000 126.5 / 121.7, 10000 154 / 147, 13000 234.5 / 228.5, 17000 324 / 308; 28 / 4 8000 97 / 91.5.  Until there
+// are 32 runs, or down to 32 workgroups only: 17000 of 32 / 32 342, 364.  Below 48 q-blocks lists are cut and shorter: 5000 of 32 / 32
+// 96.3 / 98.5, 4500 of 28 / 4 equal.  Lists that are alike gain where units are few (video of 12000 of 28 / 4 687 / 661, 8000 of 32 / 32
+// 397 / 385, of 32 / 8 357 / 358) and lose the XCD's common keys where they are many (20000 of 32 / 32, by the 64-row kernel, 1806 / 1850).
+inline DispatchShape unlike_lists_shape(int H, int Hkv, int n_qblocks) {
+  DispatchShape d = dispatch_shape(H, Hkv, n_qblocks);
+  if (n_qblocks < 48) return d;
+  const int rows = d.unit_rows;
+  while ((n_qblocks + d.unit_rows - 1) / d.unit_rows < 16 && d.unit_rows > 1 && d.unit_rows * d.set_heads > 16) d.unit_rows = (d.unit_rows + 1) / 2;
+  const int work = d.set_heads * d.unit_rows;
+  if (d.unit_rows == rows || work > kUnit / 2) return d;
+  d.unit_size = (uint32_t)work;
+  d.unit_inv = ((1u << 31) + d.unit_size - 1) / d.unit_size;
+  return d;
+}
+
 // Returns false for ids that carry no work.  The shape is computed once on the host (dispatch_shape) and the
 // arithmetic is unsigned: this runs at the start of every workgroup, where its divisions are a measurable part
 // of what a short unit costs.

@@ -152,27 +152,29 @@ static int not_temporal(const AttnParams& p, bool lists) {
   return lists && (p.H == p.Hkv ? bytes > kQueriesNtBytes : call > kCallNtBytes) ? kNtQueriesToo : kNtOutput;
 }
 
-// `ids` units and pieces; with a queue, `places` workgroups of the 64-row kernel.
+// `p` for the 64-row kernel, `p32` for the 32-row one (they may deal units differently), `pieces` ids ahead of the units'; with a queue,
+// `places` workgroups of the 64-row kernel.
 template <bool kHasList, bool kPlanned>
-static int launch_fwd(const AttnParams& p, int64_t ids, int places, hipStream_t s) {
+static int launch_fwd(const AttnParams& p, const AttnParams& p32, int64_t pieces, int places, hipStream_t s) {
+  const int64_t ids = pieces + p32.unit_ids;
   const bool all64 = all_rows64(p.H, p.nqb, p.nkb, p.causal);
   if (all64 || p.lists_decide) {
-    hipLaunchKernelGGL((block_sparse_fwd64_kernel<kHasList, kPlanned>), dim3((unsigned)(p.queue ? places : ids)), dim3(128), 0, s, p);
+    hipLaunchKernelGGL((block_sparse_fwd64_kernel<kHasList, kPlanned>), dim3((unsigned)(p.queue ? places : pieces + p.unit_ids)), dim3(128), 0, s, p);
     if (hipGetLastError() != hipSuccess) return XATTN_ERR_LAUNCH;
   }
   if (all64) return XATTN_OK;
   if (kHasList && !kPlanned && in_halves(p.H, p.nqb, p.nkb)) {
-    hipLaunchKernelGGL((block_sparse_fwd_kernel<true, false, true, kNtNone>), dim3((unsigned)(2 * ids)), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((block_sparse_fwd_kernel<true, false, true, kNtNone>), dim3((unsigned)(2 * ids)), dim3(256), 0, s, p32);
   } else if (kHasList && !kPlanned && in_wide(p.H, p.Hkv, p.nqb, p.nkb)) {
     static LdsLimit limit;
     if (limit.raise(reinterpret_cast<const void*>(&block_sparse_wide_kernel)) != hipSuccess) return XATTN_ERR_LAUNCH;
-    hipLaunchKernelGGL(block_sparse_wide_kernel, dim3((unsigned)ids), dim3(512), kWideLds, s, p);
+    hipLaunchKernelGGL(block_sparse_wide_kernel, dim3((unsigned)ids), dim3(512), kWideLds, s, p32);
   } else {
     auto kernel = block_sparse_fwd_kernel<kHasList, kPlanned, false, kNtNone>;
     const int nt = not_temporal(p, kHasList);
     if (nt == kNtOutput) kernel = block_sparse_fwd_kernel<kHasList, kPlanned, false, kNtOutput>;
     if (kHasList && nt == kNtQueriesToo) kernel = block_sparse_fwd_kernel<true, kPlanned, false, kNtQueriesToo>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)ids), dim3(256), 0, s, p);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)ids), dim3(256), 0, s, p32);
   }
   return hipGetLastError() == hipSuccess ? XATTN_OK : XATTN_ERR_LAUNCH;
 }
@@ -226,12 +228,15 @@ int xattn::block_sparse_impl(const void* q, const void* k, const void* v, void* 
   p.idx_row0 = idx_row0;
   p.qb_begin = q_block_begin;
   p.qb_end = q_block_end;
-  p.shape = dispatch_shape(p.H, p.Hkv, q_block_end - q_block_begin);
   p.plan = plan ? *plan : AttnPlan{};
   p.lists_decide = lists_decide(p.H, p.nqb, p.nkb, p.kv_off, p.causal);
-  const int64_t grid = grid_for(p.shape, q_block_end - q_block_begin);
-  const int64_t ids = grid + (plan ? piece_ids_room((int64_t)plan_pieces(plan->shape, q_block_end - q_block_begin)) : 0);
-  if (ids > 0x7fffffff) return XATTN_ERR_SHAPE;
+  const int q_blocks = q_block_end - q_block_begin;
+  const DispatchShape alike = dispatch_shape(p.H, p.Hkv, q_blocks);
+  const DispatchShape unlike = col_idx && p.causal ? unlike_lists_shape(p.H, p.Hkv, q_blocks) : alike;
+  p.shape = p.lists_decide == kFrom8 || p.lists_decide == kFrom24 ? unlike : alike;      // (else the 64-row kernel's lists are much alike)
+  const int64_t grid = grid_for(p.shape, q_blocks), grid32 = grid_for(unlike, q_blocks);
+  const int64_t pieces = plan ? piece_ids_room((int64_t)plan_pieces(plan->shape, q_blocks)) : 0;
+  if (pieces + (grid > grid32 ? grid : grid32) > 0x7fffffff) return XATTN_ERR_SHAPE;
   p.unit_ids = (int)grid;
   const int cus = resident_workgroups();
   if (cus <= 0) return XATTN_ERR_LAUNCH;
@@ -242,11 +247,14 @@ int xattn::block_sparse_impl(const void* q, const void* k, const void* v, void* 
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (!ready && (queue || totals))
     hipLaunchKernelGGL(ready_kernel, dim3((unsigned)(q_block_end - q_block_begin)), dim3(64), 0, s, p, queue, totals);
+  AttnParams p32 = p;
+  p32.shape = unlike;
+  p32.unit_ids = (int)grid32;
   if (plan) {
     if (note) hipLaunchKernelGGL(note_lists_kernel, dim3(1), dim3(1024), 0, s, p);
-    return col_idx ? launch_fwd<true, true>(p, ids, places, s) : launch_fwd<false, true>(p, ids, places, s);
+    return col_idx ? launch_fwd<true, true>(p, p32, pieces, places, s) : launch_fwd<false, true>(p, p32, pieces, places, s);
   }
-  return col_idx ? launch_fwd<true, false>(p, ids, places, s) : launch_fwd<false, false>(p, ids, places, s);
+  return col_idx ? launch_fwd<true, false>(p, p32, pieces, places, s) : launch_fwd<false, false>(p, p32, pieces, places, s);
 }
 
 extern "C" int xattn_block_sparse_fwd(const void* q, const void* k, const void* v, void* out,
