@@ -20,6 +20,12 @@ pytestmark = pytest.mark.gpu
     (2049, 0, 4, 2, 16, 4096, True),
     (5000, 0, 8, 2, 8, 2048, True),
     (300, 7000, 8, 2, 8, 1024, True),
+    # key blocks fewer than a workgroup's threads for them, up to four times as many, more, no multiple of four; rows of padding alone
+    (1000, 0, 4, 2, 16, 16384, True),
+    (4736, 0, 2, 1, 8, 128, True),
+    (650, 12000, 4, 1, 16, 128, False),
+    (3000, 0, 8, 8, 4, 1024, True),
+    (9000, 0, 3, 1, 8, 2048, False),
 ])
 @pytest.mark.parametrize("use_triton,tau", [(True, 0.9), (False, 0.7)])
 def test_one_call_equals_the_separate_passes(q_len, cache, heads, kv_heads, stride, chunk, causal, use_triton, tau):

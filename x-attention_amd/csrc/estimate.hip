@@ -706,28 +706,54 @@ __global__ __launch_bounds__(256) void estimate_select_kernel(EstParams p, SelPa
     const int kb_hi = hi4 / RBS;
     float* xs = reinterpret_cast<float*>(per_wave + (size_t)(l / kLanesPerBlock) * wave_bytes + xs_off);
     float* gout = p.sums ? p.sums + ((int64_t)head * p.win_rows + (mc4 / RBS - p.win_row0)) * p.nkb : nullptr;
-    constexpr int kUnroll = 8;
-    for (int kb0 = kgrp; kb0 < p.nkb; kb0 += kb_step * kUnroll) {
-      f32x4 pv[kUnroll], mt[kUnroll];
-      bool live[kUnroll];
+    // A thread takes four key blocks of a tile at a time, which have the tile's weights (2^(tile maximum - row maximum) / row sum) in common,
+    // eight in flight.  (Key blocks far apart, each with weights of its own, and the rows added up through the LDS crossbar, four times
+    // the instructions: normalisation and selection of 131072 tokens 233 -> 183 us, of 32768 44.7 -> 34.6, video of 65536 91 -> 82, 15000
+    // 12.9 -> 11.2; 4096 and a chunk equal.  In 80 registers instead of 98, for six wavefronts of a SIMD, 188 and 34.4, in 64 439.)
+    // Where there is a thread for every key block it takes one (an estimate of 500 tokens in a chunk of 2048 13.5 -> 13.2 us; four 14.1).
+    auto take = [&](auto chunk, auto unroll) __attribute__((always_inline)) {
+      constexpr int kChunk = decltype(chunk)::value, kUnroll = decltype(unroll)::value;
+      for (int c0 = kgrp; c0 * kChunk < p.nkb; c0 += kb_step * kUnroll) {
+        f32x4 pv[kUnroll][kChunk], mt[kUnroll];
 #pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        const int kb = kb0 + kb_step * u;
-        live[u] = rows_live && kb < p.nkb && kb >= kb_lo && kb <= kb_hi;
-        if (live[u]) load_partial<RBS>(p, Mst, prow, kb, mrel4, mt[u], pv[u]);
-      }
+        for (int u = 0; u < kUnroll; ++u) {
+          const int kb0 = (c0 + kb_step * u) * kChunk, T = kb0 * RBS / kSub;
+          const bool real = T < p.nT_real;
+          mt[u] = f32x4{};
+          if (rows_live && kb0 < p.nkb && kb0 <= kb_hi && kb0 + kChunk > kb_lo && real)
+            mt[u] = *reinterpret_cast<const f32x4*>(Mst + (int64_t)T * p.rows + mrel4);
 #pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        const int kb = kb0 + kb_step * u;
-        float acc = live[u] ? group_sum4(pv[u], mt[u], rM, rI) : 0.f;
+          for (int i = 0; i < kChunk; ++i) {
+            const int kb = kb0 + i;
+            pv[u][i] = f32x4{(float)RBS, (float)RBS, (float)RBS, (float)RBS};
+            if (rows_live && kb < p.nkb && kb >= kb_lo && kb <= kb_hi && real) pv[u][i] = *reinterpret_cast<const f32x4*>(prow + (int64_t)kb * kStrip);
+          }
+        }
 #pragma unroll
-        for (int d = 1; d < kLanesPerBlock; d <<= 1) acc += __shfl_xor(acc, d, 64);
-        if (kb < p.nkb && (l % kLanesPerBlock) == 0) {
-          xs[kb] = acc;
-          if (gout && rows_ok) gout[kb] = acc;
+        for (int u = 0; u < kUnroll; ++u) {
+          const int kb0 = (c0 + kb_step * u) * kChunk;
+          const f32x4 w = tile_weights(mt[u], rM, rI);
+#pragma unroll
+          for (int i = 0; i < kChunk; ++i) {
+            const int kb = kb0 + i;
+            const float acc = sum_lanes<kLanesPerBlock>(rows_live && kb >= kb_lo && kb <= kb_hi ? weighted_sum4(pv[u][i], w, rI) : 0.f, tid & 63);
+            if (kb < p.nkb && (l % kLanesPerBlock) == 0) {
+              xs[kb] = acc;
+              if (gout && rows_ok) gout[kb] = acc;
+            }
+          }
         }
       }
-    }
+    };
+    if (strip0 >= p.live_end) {              // rows of padding alone (uniform)
+      for (int kb = kgrp; kb < p.nkb; kb += kb_step)
+        if ((l % kLanesPerBlock) == 0) {
+          xs[kb] = 0.f;
+          if (gout && rows_ok) gout[kb] = 0.f;
+        }
+    } else if (p.nkb <= kb_step) take(std::integral_constant<int, 1>(), std::integral_constant<int, 1>());
+    else if (p.nkb <= 4 * kb_step) take(std::integral_constant<int, 4>(), std::integral_constant<int, 1>());
+    else take(std::integral_constant<int, 4>(), std::integral_constant<int, 2>());
   }
   __syncthreads();
 

@@ -93,12 +93,21 @@ __device__ __forceinline__ void stat_combine(const float (&Mw)[4], const float (
   *rowM = no_softmax ? 0.f : safe;
   *rowInv = real ? (no_softmax ? 1.f : 1.f / Lr) : 0.f;
 }
-// normalised partial sums of four consecutive rows, added up
-__device__ __forceinline__ float group_sum4(const f32x4& pv, const f32x4& mt, const f32x4& rM, const f32x4& rI) {
+// normalised partial sums of four consecutive rows, added up: the weights of the tile, and the sums of a key block with them
+__device__ __forceinline__ f32x4 tile_weights(const f32x4& mt, const f32x4& rM, const f32x4& rI) {
+  f32x4 w;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = fast_exp2(mt[i] - rM[i]) * rI[i];
+  return w;
+}
+__device__ __forceinline__ float weighted_sum4(const f32x4& pv, const f32x4& w, const f32x4& rI) {
   float acc = 0.f;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) acc += (rI[i] != 0.f) ? pv[i] * (fast_exp2(mt[i] - rM[i]) * rI[i]) : 0.f;
+  for (int i = 0; i < 4; ++i) acc += (rI[i] != 0.f) ? pv[i] * w[i] : 0.f;
   return acc;
+}
+__device__ __forceinline__ float group_sum4(const f32x4& pv, const f32x4& mt, const f32x4& rM, const f32x4& rI) {
+  return weighted_sum4(pv, tile_weights(mt, rM, rI), rI);
 }
 #pragma clang fp contract(fast)
 

@@ -339,8 +339,7 @@ __global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p, Sel
       const f32x4 rM = *reinterpret_cast<const f32x4*>(row_m + row4);
       sum = group_sum4(*reinterpret_cast<const f32x4*>(psum + kb * 32 + row4), rM, rM, *reinterpret_cast<const f32x4*>(row_inv + row4));
     }
-#pragma unroll
-    for (int d = 1; d < kLanes; d <<= 1) sum += __shfl_xor(sum, d, 64);
+    sum = sum_lanes<kLanes>(sum, lane);
     if (l == 0 && kb < kSub / RBS && kb < sp.nkb) xs[kb] = sum;
     for (int c = kSub / RBS + lane; c < sp.nkb; c += 64) xs[c] = 0.f;
     __builtin_amdgcn_wave_barrier();

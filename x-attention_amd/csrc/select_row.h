@@ -71,6 +71,15 @@ __device__ __forceinline__ uint32_t other_lane(uint32_t x, int lane) {
   else asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
   return lane & J ? a : b;
 }
+// sum over groups of kLanes lanes, in each of them: with the lane next to it, then two, then four apart
+template <int kLanes>
+__device__ __forceinline__ float sum_lanes(float x, int lane) {
+  auto other = [&](auto j) { return __builtin_bit_cast(float, other_lane<decltype(j)::value>(__builtin_bit_cast(uint32_t, x), lane)); };
+  x += other(std::integral_constant<int, 1>());
+  if (kLanes > 2) x += other(std::integral_constant<int, 2>());
+  if (kLanes > 4) x += other(std::integral_constant<int, 4>());
+  return x;
+}
 template <int K, int J>
 __device__ __forceinline__ void sort_step(uint32_t& hi, uint32_t& lo, int lane) {
   const uint32_t oh = other_lane<J>(hi, lane), ol = other_lane<J>(lo, lane);
