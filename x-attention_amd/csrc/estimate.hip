@@ -838,23 +838,26 @@ __global__ __launch_bounds__(256) void estimate_normalize_rows_kernel(EstParams 
 using namespace xattn;
 
 namespace {
+// us of a step of the 256x256 tiles, and of their epilogue
+constexpr float kLargeStep = 1.42f, kLargeTile = 6.4f;
 // Which MFMA pass a launch takes: the smallest predicted time
 //   5 us + steps * max(lat, per_tile * tiles),   steps = 2 * stride
 // of estimate_small_kernel's variants - lat: one step when there are few tiles, per_tile: a tile's share of a step when
 // the chip is full - and for the 256x256 tiles, which 256 workgroups take in turns,
-//   5 us + steps * 1.75 us * ceil(tiles / 256),
+//   5 us + (steps * kLargeStep + kLargeTile) * ceil(tiles / 256),
 // with a head's rows in tiles of their own or packed with those of the other heads of its KV group, or, with 0.65 of a
 // tile's time for a half and 6 us for the second launch, the last of them as half tiles.
-// The constants are fits to measured times (MT 1's before its fragments were read a step ahead, 0.16 us a step since)
-// of the passes over 200 .. 16384 tokens and chunks of 64 .. 8000 tokens on 8700 .. 100000 cached ones, stride 8 and 16
-// (us, 256x256 / chosen): 1000 tokens, stride 16: 45.2 / 10.6 (MT 1; 9.2 since); 2000, stride 8: 31.1 / 9.8 (MT 2, 3
-// stages); 4096, stride 8: 35.0 / 19.2; 8192, stride 16: 60.9 / 31.6; 16384, stride 16: 117.9 / 96; 15000, stride 8:
-// 147.5 (stays).
+// The constants are fitted to times of whole calls with each of the variants and with the large tiles, 34 prompts of 250 .. 9000 tokens
+// and 26 chunks of 64 .. 5000 on 2000 .. 100000 cached ones, stride 8 and 16, of 32 / 8, 32 / 32 and 28 / 4 heads: chosen by them a
+// call takes 0.14 % more than with the best choice on average, 2.9 % at most.  Calls, us, as chosen by constants from before the loops
+// were rewritten / now: 3000 tokens, stride 16, 59 / 55 (MT 1), 1500, stride 8, 37 / 34 (MT 1), 2500, stride 8, 53.7 / 50.2 and 6000, stride 16,
+// 104 / 99 (MT 2), 8700, stride 16, 155 / 139 (MT 4), 2153 on 53158 200 / 171, 2182 on 85746 763 / 717 and 835 on 83806 132 / 113 (packed).
+// (MT 2 with two stages, a third workgroup to a CU instead of a third stage, was nowhere more than 2 % better than the others.)
 struct SmallVariant {
   int mt, ns;
   float lat, per_tile;
 };
-constexpr SmallVariant kSmall[] = {{1, 4, 0.20f, 0.00106f}, {2, 3, 0.27f, 0.00129f}, {2, 2, 0.35f, 0.00126f}, {4, 2, 0.50f, 0.00238f}};
+constexpr SmallVariant kSmall[] = {{1, 4, 0.20f, 0.00091f}, {2, 3, 0.27f, 0.00152f}, {4, 2, 0.61f, 0.00253f}};
 
 template <int RBS, bool kDump, bool kTable, bool kPacked = false, bool kHalf = false>
 hipError_t launch_gemm_as(const EstParams& p, dim3 grid, size_t lds, hipStream_t s) {
@@ -902,8 +905,7 @@ hipError_t launch_small(const EstParams& p, int variant, hipStream_t s) {
   switch (variant) {
     case 0: return launch_small_as<RBS, kSmall[0].mt, kSmall[0].ns>(p, s);
     case 1: return launch_small_as<RBS, kSmall[1].mt, kSmall[1].ns>(p, s);
-    case 2: return launch_small_as<RBS, kSmall[2].mt, kSmall[2].ns>(p, s);
-    default: return launch_small_as<RBS, kSmall[3].mt, kSmall[3].ns>(p, s);
+    default: return launch_small_as<RBS, kSmall[2].mt, kSmall[2].ns>(p, s);
   }
 }
 template <int RBS>
@@ -1092,8 +1094,9 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
   if (kdb == 1 && num_slab_pairs == 0 && !scores_out && p.total_tiles > 0 && p.total_tiles <= 4096) {
     const int group = num_heads / num_kv_heads;
     EstParams best = p;
-    float best_t = 1.75f * (float)((p.total_tiles + 255) / 256);
-    for (int i = 0; i < 4; ++i) {
+    const float large = kLargeStep + kLargeTile / (float)(2 * stride);
+    float best_t = large * (float)((p.total_tiles + 255) / 256);
+    for (int i = 0; i < (int)(sizeof(kSmall) / sizeof(kSmall[0])); ++i) {
       EstParams c = p;
       const int rows = 32 * kSmall[i].mt;
       // heads whose rows fit a tile together (one buffer resource spans them: < 2^31 bytes)
@@ -1120,8 +1123,8 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
       last = last < p.nNT - 1 ? last : p.nNT - 1;
       c.key_tiles = last - c.first_key_tile + 1;
       c.total_tiles = (int64_t)c.group_tiles * c.key_tiles * num_kv_heads;
-      if (c.key_tiles > 0 && c.total_tiles < p.total_tiles && 1.75f * (float)((c.total_tiles + 255) / 256) < best_t) {
-        best_t = 1.75f * (float)((c.total_tiles + 255) / 256);
+      if (c.key_tiles > 0 && c.total_tiles < p.total_tiles && large * (float)((c.total_tiles + 255) / 256) < best_t) {
+        best_t = large * (float)((c.total_tiles + 255) / 256);
         best = c;
         variant = -1;
       }
@@ -1143,7 +1146,7 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
         c.whole_tiles = rounds * 256;
         c.split_tiles = tiles - c.whole_tiles;
         const int units = 2 * c.split_tiles + halves;
-        const float t = 1.75f * ((float)rounds + 0.65f * (float)((units + 255) / 256)) + (rounds ? 6.f / (float)(2 * stride) : 0.f);
+        const float t = large * ((float)rounds + 0.65f * (float)((units + 255) / 256)) + (rounds ? 6.f / (float)(2 * stride) : 0.f);
         if (units > 0 && t < best_t) {
           best_t = t;
           best = c;

@@ -9,8 +9,7 @@
 // Bound: with at most a tile per CU the time is the chain of 2 * stride steps - 0.16 us each with MT 1, the barrier, the
 // dependent MFMAs and the fragment reads of a step, against 1.1 us of a 256x256 step.  With more tiles per CU two or three workgroups share it
 // and the copies into LDS (about 50 bytes per clock and CU) and the fragment reads (1 + MT per MT MFMAs) are the limit:
-// 0.7 (MT 2) and 0.8 (MT 4) of the flop rate of the large tiles.  More stages help only while a CU has one workgroup;
-// beyond that a third workgroup is worth more than a third stage.
+// 0.55 (MT 2) and 0.65 (MT 4) of the flop rate of the large tiles.
 #pragma once
 #include "estimate_params.h"
 #include "select_row.h"
