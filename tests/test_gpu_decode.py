@@ -154,3 +154,24 @@ def test_decode_of_a_layer(H, Hkv, L):
     for other in [(step.cpu(), ks, vs), (step.float(), ks, vs), (step, ks, vs[:, :, 1:]), (step, ks.transpose(2, 3), vs.transpose(2, 3)),
                   (step.expand(2, -1, -1, -1), ks, vs), (step.expand(-1, -1, 2, -1), ks, vs), (step[..., :64], ks, vs), (step[0], ks[0], vs[0])]:
         assert hb.host().decode_layer(*other) is None
+
+
+# A short cache's probabilities are rounded to bf16 relative to the largest of their own 32 keys, which is then exact, whichever
+# wavefront has the keys and in whatever order (relative to a running maximum the error against 64 bits is up to 4 % larger).  The
+# same in 64 bits but for that rounding and the result's: what the kernel's 32-bit scores, of relative error 2^-22 or so, turn over of the
+# roundings to 8 bits is one in some 10^4 of them by 2^-8 each, 10^-4 of the result
+@pytest.mark.parametrize("H,Hkv,L", [(32, 8, 100), (32, 8, 400), (28, 4, 510), (32, 32, 640), (8, 1, 600)])
+def test_short_caches_round_relative_to_a_tile(H, Hkv, L):
+    from xattn.src.decode import single_decode_with_kv_cache
+
+    q, k, v = _mk(H, Hkv, L, L)
+    out = single_decode_with_kv_cache(q.cuda(), k.cuda(), v.cuda(), kv_layout="HND").cpu()
+    g, tiles = H // Hkv, -(-L // 32)
+    s = torch.full((Hkv, g, tiles * 32), -float("inf"), dtype=torch.float64)
+    s[..., :L] = q.double().view(Hkv, g, 128) @ k.double().transpose(1, 2) / (128 ** 0.5 * 0.6931471805599453)
+    s = s.view(Hkv, g, tiles, 32)
+    own = s.amax(-1, keepdim=True)
+    e, w = torch.exp2(s - own), torch.exp2(own - own.amax(2, keepdim=True))
+    p = (e.bfloat16().double() * w).view(Hkv, g, -1)[..., :L]
+    want = (p @ v.double() / (e * w).sum((2, 3))[..., None]).view(H, 128).bfloat16()
+    assert ((out.double() - want.double()).norm() / want.double().norm()).item() <= 5e-4
