@@ -117,6 +117,33 @@ def test_xattn_metric_calls_match_oracle(monkeypatch):
         assert err.max().item() <= OUT_MAX_ABS and err.mean().item() <= OUT_MEAN_ABS
 
 
+def test_a_replaced_decode_call_sees_every_step(monkeypatch):
+    """A program that puts its own function in the decode call's place, as the prefill's above, gets each layer's step, with
+    the arguments of the call and its result used; the result is that of the ordinary step to the bit."""
+    from xattn.src import load_llama
+    from xattn.src.load_llama import FastPrefillConfig, patch_model
+
+    model = patch_model(_tiny_llama(7), FastPrefillConfig(threshold=0.9))
+    ids = torch.randint(0, 512, (1, 301), generator=torch.Generator().manual_seed(8)).cuda()
+    real, calls = load_llama.single_decode_with_kv_cache, []
+
+    def step():
+        with torch.no_grad():
+            first = model(ids[:, :300], use_cache=True)
+            return model(ids[:, 300:], past_key_values=first.past_key_values, use_cache=True).logits
+
+    def spy(q, k, v, **kw):
+        calls.append((q.shape, k.shape, v.shape, kw))
+        return real(q, k, v, **kw)
+
+    want = step()
+    monkeypatch.setattr(load_llama, "single_decode_with_kv_cache", spy)
+    assert torch.equal(step(), want)
+    assert calls == [((4, 128), (2, 301, 128), (2, 301, 128), {"kv_layout": "HND"})] * 2
+    monkeypatch.setattr(load_llama, "single_decode_with_kv_cache", lambda q, k, v, **kw: torch.zeros_like(q))
+    assert not torch.equal(step(), want)
+
+
 def test_batch_two_is_refused():
     from xattn.src.load_llama import FastPrefillConfig, patch_model
 

@@ -120,6 +120,7 @@ _own_linear_call = _linear_call()
 if not (all(_torch_own(fn, _module_hooks) for fn in _own_linear_call[:2])
         and _torch_own(_own_linear_call[2], torch.nn.modules.linear) and _own_linear_call[3] is torch._C._nn.linear):
     _own_linear_call = None      # replaced before this module was imported
+_own_decode = single_decode_with_kv_cache
 _function_modes, _dispatch_modes = torch._C._len_torch_function_stack, torch._C._len_torch_dispatch_stack
 _forward_ad, _transform, _tracer = torch.autograd.forward_ad, torch._C._functorch.peek_interpreter_stack, torch._C._get_tracing_state
 
@@ -238,9 +239,10 @@ def forward_eval(self, hidden_states, position_embeddings=None, attention_mask=N
     if cfg.print_detail:
         print(f"q length: {q_len} k length: {k_len}")
 
-    # the ordinary decode step comes back as the output projection takes it, without views made and put together here
+    # the ordinary decode step comes back as the output projection takes it, without views made and put together here (not where a
+    # program has put a function of its own in this module's decode call)
     merged = None
-    if decoding and native and type(query_states) is type(key_states) is type(value_states) is torch.Tensor:
+    if decoding and native and single_decode_with_kv_cache is _own_decode and type(query_states) is type(key_states) is type(value_states) is torch.Tensor:
         merged = _hb.host().decode_layer(query_states, key_states, value_states)
     if merged is not None:
         pass
