@@ -78,7 +78,6 @@ __global__ __launch_bounds__(256 * KS, 2) void proj_gemm_kernel(ProjParams p) {
   constexpr int kLoadsW = 2 * NB / KS, kLoadsX = 2 * MB / KS;
   constexpr int kChunks = 8 * NB, kPairs = kChunks / 2;       // of a token in a tile, and rotation partners
   constexpr int kTurns = (kM * kPairs + 256 * KS - 1) / (256 * KS), kTurnsAhead = kTurns < 4 ? kTurns : 4;
-  constexpr int kTurnLoads = kRope ? 4 * kTurnsAhead : 0;
   constexpr int kPer = (kLoads + kSubs - 2) / (kSubs - 1);   // ... and in each of its sub-steps but the last
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -164,7 +163,9 @@ __global__ __launch_bounds__(256 * KS, 2) void proj_gemm_kernel(ProjParams p) {
   // issued between them.  The barrier sits before the last sub-step's MFMAs: by then this wavefront has read every
   // fragment of step t and its copies of step t + 1 have landed, so behind it step t + 1 may be read and step t's stage
   // refilled.
-  // `left`: the steps behind step t + 1 whose copies have been issued
+  // `left`: the steps behind step t + 1 whose copies have been issued; kLanded: every copy has landed.  The counts are of
+  // copies alone, which are written here in assembly: a load that the compiler issues or moves can only make a wait stricter.
+  constexpr int kLanded = -1;
   int st = 0, t = 0;
   auto step = [&](auto copies, auto left) __attribute__((always_inline)) {
     const int next = st + 1 == NS ? 0 : st + 1, fill = st == 0 ? NS - 1 : st - 1;
@@ -172,7 +173,8 @@ __global__ __launch_bounds__(256 * KS, 2) void proj_gemm_kernel(ProjParams p) {
     for (int s = 0; s < kSubs; ++s) {
       __builtin_amdgcn_sched_barrier(0);
       if (s == kSubs - 1) {
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(decltype(left)::value * kLoads + (decltype(copies)::value ? 0 : kTurnLoads)) : "memory");
+        if constexpr (decltype(left)::value == kLanded) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(decltype(left)::value * kLoads) : "memory");
         read(next, 0, 0);     // (a repeat of old data behind the last step)
       } else {
         read(st, s + 1, (s + 1) & 1);
@@ -188,20 +190,12 @@ __global__ __launch_bounds__(256 * KS, 2) void proj_gemm_kernel(ProjParams p) {
     ++t;
   };
   while (t < steps - (NS - 1)) step(std::true_type(), std::integral_constant<int, NS - 2>());
-  // The cosines and sines of the first four tokens that this lane turns are on their way while the last steps multiply.  (Asked for
-  // one token after the other behind the exchange, a layer's 500 tokens took 35.0 us instead of 34.0, 1000 63.8 instead of 61.3.)
   const int ch = tid % kPairs, feature = feature_chunk(ch) * 8;      // its partner is 64 further on
   auto token = [&](int i) __attribute__((always_inline)) { return (i * 256 * KS + tid) / kPairs; };
   auto turn_at = [&](int i) __attribute__((always_inline)) {
     const int64_t m = m0 + (token(i) < rows_left ? token(i) : 0);
     return turn_of(p.cos + m * p.cos_sn + feature % 128, p.sin + m * p.sin_sn + feature % 128);
   };
-  Turn turns[kTurnsAhead];
-  if (kRope) {
-#pragma unroll
-    for (int i = 0; i < kTurnsAhead; ++i) turns[i] = turn_at(i);
-    __builtin_amdgcn_sched_barrier(0);
-  }
   auto last = [&](auto left) __attribute__((always_inline)) {
     if (t < steps) step(std::false_type(), left);
   };
@@ -210,10 +204,23 @@ __global__ __launch_bounds__(256 * KS, 2) void proj_gemm_kernel(ProjParams p) {
   if constexpr (NS >= 5) last(std::integral_constant<int, 2>());
   if constexpr (NS >= 4) last(std::integral_constant<int, 1>());
   if constexpr (NS >= 3) last(std::integral_constant<int, 0>());
-  last(std::integral_constant<int, 0>());
+  // With a step left or none every copy has landed, unless there were fewer steps than the first fill has stages: then those that move
+  // nothing may be under way still.
+  if (steps < NS - 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // The cosines and sines of the first four tokens that this lane turns are on their way while the last step multiplies.  (Asked
+  // for one token after the other behind the exchange, a layer's 500 tokens took 35.0 us instead of 34.0, 1000 63.8 instead of 61.3; ahead of
+  // the last three steps, whose waits then have to count them, 34.5 as here and 58.2 instead of 58.0.)
+  Turn turns[kTurnsAhead];
+  if (kRope) {
+#pragma unroll
+    for (int i = 0; i < kTurnsAhead; ++i) turns[i] = turn_at(i);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  last(std::integral_constant<int, kLanded>());
   // every copy has landed and every fragment has been read: the LDS takes the tile, token-major, chunk c of token m at
   // c ^ (m & (chunks - 1))
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  static_assert((KS - 1) * 4 * NB * MB * 4096 + kM * kN * 2 <= NS * kStage, "the halves' sums and the tile");
   char* const tile = lds + (KS - 1) * 4 * NB * MB * 4096;
   if (KS == 2) {
     f32x4* const half = reinterpret_cast<f32x4*>(lds + (wave & 3) * NB * MB * 4096) + lane;
