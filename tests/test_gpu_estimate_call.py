@@ -17,6 +17,11 @@ pytestmark = pytest.mark.gpu
     (500, 0, 6, 2, 4, 512, True),
     (500, 8700, 32, 8, 16, 16384, True),
     (700, 0, 4, 4, 8, 1024, False),
+    # as many candidates as a key tile has blocks, with each stride
+    (2048, 0, 4, 2, 16, 2048, False),
+    (1024, 0, 4, 4, 8, 1024, False),
+    (512, 0, 6, 2, 4, 512, True),
+    (512, 0, 3, 1, 4, 512, False),
     (2049, 0, 4, 2, 16, 4096, True),
     (5000, 0, 8, 2, 8, 2048, True),
     (300, 7000, 8, 2, 8, 1024, True),

@@ -1225,6 +1225,7 @@ int estimate_impl(const void* q, const void* k, float* block_sums, void* workspa
     return launch_select<RBS>(p, sp, qb_per_wg, sel_threads, grid_sel, lds_sel, s);
   };
   // one pass instead of two where every row asked for is estimated, in 32-row tiles, and sees a single key tile
+  // (what that leaves of the selection is compiled for it: 128 reshaped keys are at most 16 blocks, and there is no plan)
   bool one_pass = variant == 0 && sel && sel->stages == 3 && !p.no_softmax && !p.sums && !sel->plan && !p.clear && p.nT_real == g.nT &&
                   p.live_end == sp.row_end * p.rbs && row_lo(p, p.live_end - 1) == 0 &&
                   (row_hi(p, p.live_end - 1) < kSub || g.n_rk <= kSub) && 4 * sel_wave_bytes <= 64 * 1024;

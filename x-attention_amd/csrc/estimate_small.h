@@ -344,7 +344,7 @@ __global__ __launch_bounds__(256, 2) void estimate_small_kernel(EstParams p, Sel
     __builtin_amdgcn_wave_barrier();
     const int row = m / RBS;
     if (sp.sums_out) store_sums(sp, xs, head, row, lane);
-    select_row(sp, xs, head, row, reinterpret_cast<uint64_t*>(mine), reinterpret_cast<uint8_t*>(mine + (size_t)sp.npow2 * 8), lane);
+    select_row<kSub / RBS>(sp, xs, head, row, reinterpret_cast<uint64_t*>(mine), reinterpret_cast<uint8_t*>(mine + (size_t)sp.npow2 * 8), lane);
   }
 }
 

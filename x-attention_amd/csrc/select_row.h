@@ -90,15 +90,16 @@ __device__ __forceinline__ void sort_step(uint32_t& hi, uint32_t& lo, int lane) 
   lo = take ? ol : lo;
   if constexpr (J > 1) sort_step<K, J / 2>(hi, lo, lane);
 }
-// the first n lanes' 64-bit keys in descending order, by a bitonic network of 6 (up to 8 lanes) to 21 steps of some ten instructions;
-// the other lanes' are 0
+// the first n lanes' (at most kMost) 64-bit keys in descending order, by a bitonic network of 6 (up to 8 lanes) to 21 steps of some ten
+// instructions; the other lanes' are 0
+template <int kMost>
 __device__ __forceinline__ void sort_lanes(uint32_t& hi, uint32_t& lo, int lane, int n) {
   sort_step<2, 1>(hi, lo, lane);
   sort_step<4, 2>(hi, lo, lane);
-  sort_step<8, 4>(hi, lo, lane);
-  if (n > 8) sort_step<16, 8>(hi, lo, lane);
-  if (n > 16) sort_step<32, 16>(hi, lo, lane);
-  if (n > 32) sort_step<64, 32>(hi, lo, lane);
+  if (kMost > 4) sort_step<8, 4>(hi, lo, lane);
+  if (kMost > 8 && n > 8) sort_step<16, 8>(hi, lo, lane);
+  if (kMost > 16 && n > 16) sort_step<32, 16>(hi, lo, lane);
+  if (kMost > 32 && n > 32) sort_step<64, 32>(hi, lo, lane);
 }
 // sum of the lanes before the lane's own
 __device__ __forceinline__ double wave_sum_before(double x) {
@@ -135,11 +136,13 @@ __device__ __forceinline__ void store_sums(const SelParams& p, const float* x, i
 //  - Beyond 1024, and rows whose sums outrank forced blocks after 32 pulled out: a sort in LDS.
 //
 // Selection for q-block row `row` of `head` by ONE wavefront (lane = its lane number).  x: the row's nkb block
-// sums (global or LDS); keys (npow2 entries) and flags (nkb bytes): LDS scratch of this wavefront.  All LDS
+// sums (global or LDS), at most kMost of them candidates (with all of the ways above in it a kernel of a few candidates had 30 KB more
+// code); keys (npow2 entries) and flags (nkb bytes): LDS scratch of this wavefront.  All LDS
 // traffic is the wavefront's own, which the LDS keeps in program order: the points where the lanes exchange
 // data through it need no workgroup barrier.  x may occupy the LAST 4 * nkb bytes of the key array (rounded up
 // to 64 bytes): key c then lands on sums 2c - (2 npow2 - nkb) and the one after, both below c, i.e. sums that
 // the loops which fill the keys (ascending c, a whole wavefront's reads before its writes) have read already.
+template <int kMost = 1 << 30>
 __device__ __forceinline__ void select_row(const SelParams& p, const float* x, int head, int row, uint64_t* keys,
                                            uint8_t* flags, int lane) {
   const int64_t slot = (int64_t)head * p.win_rows + (row - p.win_row0);   // this row's place in the arrays
@@ -212,7 +215,7 @@ __device__ __forceinline__ void select_row(const SelParams& p, const float* x, i
   // of the last one taken.  Sorted, each lane finds the mass ahead of its own in a prefix sum.
   auto decide_lanes = [&](uint64_t key, int n, double before, double prev_before, int taken) {
     uint32_t hi = (uint32_t)(key >> 32), lo = (uint32_t)key;
-    sort_lanes(hi, lo, lane, n);
+    sort_lanes<kMost>(hi, lo, lane, n);
     const double v = hi ? (double)__uint_as_float(hi - 1u) : 0.0;
     double mass = before + wave_sum_before(v);
     if (may_outrank) {                     // (then they are all of the row's, and nothing was taken)
@@ -386,27 +389,29 @@ __device__ __forceinline__ void select_row(const SelParams& p, const float* x, i
   for (int c = lane; c < p.nkb; c += 64) flags[c] = 0;
   __builtin_amdgcn_wave_barrier();
   const bool small = np2 <= kMostSlots * 64;
-  if (np2 == 64) {
+  if (kMost <= 64 || np2 == 64) {
     double total = 0.0;
     const uint32_t bits = load_one(lane, total);
     total_is(wave_sum(total));
     decide_lanes(sort_key(lane, bits), ncand, forced_sum, 0.0, 0);
-  } else if (np2 == 128) {
-    decide_slots(std::integral_constant<int, 2>{});
-  } else if (np2 == 256) {
-    decide_slots(std::integral_constant<int, 4>{});
-  } else if (np2 == 512) {
-    decide_slots(std::integral_constant<int, 8>{});
-  } else if (small) {
-    decide_slots(std::integral_constant<int, kMostSlots>{});
-  } else {
-    double total = 0.0;
-    for (int c = lane; c < np2; c += 64) keys[c] = sort_key(c, load_one(c, total));
-    total_is(wave_sum(total));
-    __builtin_amdgcn_wave_barrier();
+  } else if constexpr (kMost > 64) {
+    if (np2 == 128) {
+      decide_slots(std::integral_constant<int, 2>{});
+    } else if (np2 == 256) {
+      decide_slots(std::integral_constant<int, 4>{});
+    } else if (np2 == 512) {
+      decide_slots(std::integral_constant<int, 8>{});
+    } else if (small) {
+      decide_slots(std::integral_constant<int, kMostSlots>{});
+    } else {
+      double total = 0.0;
+      for (int c = lane; c < np2; c += 64) keys[c] = sort_key(c, load_one(c, total));
+      total_is(wave_sum(total));
+      __builtin_amdgcn_wave_barrier();
+    }
   }
 
-  if (!finished) {
+  if (kMost > 64 && !finished) {
   if (small) {
     double again = 0.0;
     for (int c = lane; c < np2; c += 64) keys[c] = sort_key(c, load_one(c, again));
@@ -500,7 +505,7 @@ __device__ __forceinline__ void select_row(const SelParams& p, const float* x, i
       __hip_atomic_fetch_add(of, (uint32_t)count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_fetch_max(of + 1, (uint32_t)count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (p.plan.shape.per_qb && (p.causal ? q_last / 128 + 1 : p.list_cols) > p.plan.shape.min_piece)   // else too few blocks to be cut
+    if (kMost > 64 && p.plan.shape.per_qb && (p.causal ? q_last / 128 + 1 : p.list_cols) > p.plan.shape.min_piece)   // else too few blocks to be cut
       list_made(p.plan, p.H, p.win_rows, row - p.win_row0, head, count, lane);
   }
 }
