@@ -111,12 +111,14 @@ def test_decode_at_the_line_between_cache_policies(shape):
     _check(single_decode_with_kv_cache(q.cuda(), k.cuda(), v.cuda(), kv_layout="HND"), O.single_decode_with_kv_cache(q, k, v, kv_layout="HND"))
 
 
-# caches of one launch (up to 48 tiles of 32 keys, a wavefront every twelfth of them) and the first beyond: tiles that lack keys, fewer
+# caches of one launch (up to 40 tiles of 32 keys, a wavefront every twelfth of them) and longer ones: tiles that lack keys, fewer
 # tiles than parts and wavefronts, the edges of a wavefront's turns, groups of query heads that fill no copy of four rows, 32 and one;
 # views whose heads and tokens lie apart
 @pytest.mark.parametrize("H,Hkv,L", [
     (32, 8, 2), (32, 1, 5), (62, 2, 70), (3, 3, 32), (5, 1, 65), (32, 8, 96), (28, 4, 100), (32, 32, 129), (32, 1, 383), (64, 2, 384), (32, 8, 385), (14, 2, 416),
     (27, 9, 769), (32, 8, 1100), (40, 40, 1505), (32, 8, 1536), (32, 8, 1537), (28, 4, 1569), (130, 130, 1600), (257, 257, 40), (300, 300, 1700),
+    # either side of the line, where every workgroup has a CU and where some wait
+    (32, 8, 1280), (32, 8, 1281), (64, 64, 1280), (64, 64, 1281), (65, 65, 128), (65, 65, 129), (128, 128, 500), (257, 257, 129),
 ])
 def test_decode_of_short_caches(H, Hkv, L):
     from xattn.src.decode import single_decode_with_kv_cache

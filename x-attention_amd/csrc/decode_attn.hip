@@ -396,7 +396,8 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p) {
 // on the host, so a KV head is four workgroups', each of which goes over all keys for a quarter of the features.  They are on one XCD,
 // and each begins at another quarter of the keys, so the keys are fetched into its L2 once, by all four together.  Its wavefronts take
 // every twelfth tile each: 8 KiB of keys and 2 KiB of values, requested anew as soon as the last ones are in registers.  Bound by what
-// a CU takes in, 10 KiB per tile at 100 GB/s, behind 3.4 us of latencies (launch, first tile, softmax, the wavefronts' results, store).
+// a CU takes in, 10 KiB per tile at 110 GB/s from the L2 and 70 from memory, behind 3.4 us of latencies (launch, first tile, softmax, the
+// wavefronts' results, store).
 constexpr int kShortWaves = 12, kShortParts = 4;
 constexpr int kShortSlot = kDecTileBytes + kDecTileBytes / kShortParts;
 constexpr int kShortLds = kShortWaves * kShortSlot + kDecTileBytes;      // the queries last
@@ -584,12 +585,27 @@ __global__ __launch_bounds__(64 * kShortWaves) void decode_short_kernel(DecodePa
 // without / with: 82 MB 19.0 / 19.4 us, 38 MB 12.8 / 13.1).
 constexpr int64_t kNtBytes = 96 << 20;
 
-// Tiles of the longest cache that decode_short_kernel takes (1536 keys).  Its four workgroups per KV head take 0.1 us per tile; the two
-// launches take 7 us, and a loop of calls 8.5 to 9, which is what the host needs for them (6 for one).  us in a captured graph / in such
-// a loop, two launches and one: 100 keys of 8 KV heads 7.4 / 8.6 and 3.5 / 6.0, 500 7.6 / 8.6 and 4.8 / 6.1, 1100 7.6 / 8.7 and 6.6 / 7.1,
-// 1500 7.2 / 8.8 and 7.6 / 8.0, 2200 7.3 / 8.8 and 11.1 / 11.2; of 32, whose keys a step fetches with fewer requests so, 1100
-// 10.5 / 10.7 and 8.5 / 8.5, 2200 12.5 / 12.6 and 13.2 / 13.2.
-constexpr int kShortTiles = 48;
+// Tiles of the longest cache that decode_short_kernel takes: 1280 keys where every workgroup has a CU of its own, 128 where some wait for
+// another's (more than 64 KV heads).  A step's cache comes from memory, the weights of all layers having passed since its last one, and
+// so were these measured, over caches of 640 MB in turn.  us, two launches / one:
+//                                            100          500          800          1100         1300         1500 keys
+//   in a captured graph, 1 KV head           9.1 / 4.2    9.4 / 6.5    9.7 / 8.4    9.8 / 9.8    9.8 / 10.7   9.8 / 11.6
+//                        2                   7.6 / 4.2    8.2 / 6.6    8.3 / 8.2    8.3 / 9.7    8.4 / 10.5   8.4 / 11.4
+//                        4                   7.2 / 4.0    7.5 / 6.4    7.6 / 8.1    7.6 / 9.7    7.7 / 10.4   7.7 / 11.4
+//                        8                   7.2 / 4.4    7.2 / 6.6    7.3 / 8.3    7.4 / 9.9    7.5 / 10.7   7.6 / 11.7
+//                        32                  7.1 / 4.5    7.5 / 7.0    8.5 / 8.8    10.3 / 10.8  11.1 / 11.9  11.4 / 12.9
+//                        64                  7.2 / 4.6    8.9 / 8.1    11.8 / 10.6  13.9 / 13.0  14.6 / 14.6  15.7 / 17.0
+//                        72                  7.2 / 6.9    10.4 / 11.6  12.9 / 14.7  14.1 / 17.9  16.3 / 21.0  18.6 / 23.8
+//                        128                 7.4 / 7.2    12.8 / 13.8  16.8 / 18.9  20.0 / 24.6  22.5 / 28.5  24.8 / 32.6
+//   in a loop of calls, 8                    8.2 / 4.7    8.3 / 6.6    8.1 / 8.1    8.2 / 9.7    8.5 / 10.5   8.9 / 11.6
+//                       128                  8.7 / 7.4    13.6 / 13.9  17.2 / 19.3  20.8 / 26.0  23.7 / 29.1  25.5 / 33.2
+//   a layer's whole step, 8, graph           29.4 / 27.8 (300 keys)    29.6 / 29.5  29.7 / 30.7               30.0 / 32.0
+//                         as Python calls it 43.1 / 39.3 (300)         42.4 / 38.7  41.7 / 38.1               42.0 / 38.3
+// (32 / 32 heads the same: 37.3 / 36.0, 39.4 / 39.9, 41.6 / 41.6, 42.5 / 43.6 and 43.0 / 39.5, 42.6 / 40.2, 42.4 / 42.1, 43.5 / 43.2.)
+// Beyond 800 keys the GPU is done sooner with two launches and a layer that is called from Python later, the host having one more to make;
+// the line is where the loss of the one and the gain of the other are equal.  (A cache still in the L2, graph, 8: 500 keys 6.8 / 5.1, 1100
+// 7.0 / 7.1, 1500 6.9 / 8.1.)  A word of every later row of values asked for at the start made one launch 0.4 to 0.8 slower.
+constexpr int kShortTiles = 40, kShortTilesInTurns = 4;
 
 struct DecodeGeometry {
   int n_tiles, wgs;
@@ -655,7 +671,7 @@ int decode_launch(const void* q, const void* k, const void* v, void* out, void* 
 
   hipStream_t s = static_cast<hipStream_t>(stream);
   static LdsLimit limit[3];
-  if (g.n_tiles <= kShortTiles) {
+  if (g.n_tiles <= (kShortParts * num_kv_heads <= kDecCUs ? kShortTiles : kShortTilesInTurns)) {
     if (limit[2].raise(reinterpret_cast<const void*>(decode_short_kernel)) != hipSuccess) return XATTN_ERR_LAUNCH;
     hipLaunchKernelGGL(decode_short_kernel, dim3((unsigned)(kShortParts * ((num_kv_heads + 7) & ~7))), dim3(64 * kShortWaves), kShortLds, s, p);
     return hipGetLastError() == hipSuccess ? XATTN_OK : XATTN_ERR_LAUNCH;
