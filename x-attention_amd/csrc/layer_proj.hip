@@ -42,7 +42,7 @@ constexpr int kGemvWaves = 4;
 // kRope: a unit is rows d, d+1, d+64, d+65 of one head (products 0 and 1 rotated, 2 not); otherwise four rows in order
 template <bool kRope, int kBatch, bool kNt>
 __global__ __launch_bounds__(64 * kGemvWaves) void gemv_kernel(GemvParams p) {
-  __shared__ float sums[kGemvWaves][4];
+  __shared__ __attribute__((aligned(16))) float sums[kGemvWaves][4];      // (written 16 bytes at a time)
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int unit = blockIdx.x, t = 0;
