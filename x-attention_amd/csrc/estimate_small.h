@@ -7,7 +7,7 @@
 // a ring of NS LDS stages (buffer loads that write LDS), NS - 1 steps ahead of their use (NS with MT 1), one barrier per step.
 //
 // Bound: with at most a tile per CU the time is the chain of 2 * stride steps - 0.16 us each with MT 1, the barrier, the
-// dependent MFMAs and the fragment reads of a step, against 1.1 us of a 256x256 step.  With more tiles per CU two or three workgroups share it
+// dependent MFMAs and the fragment reads of a step, against 1.4 us of a 256x256 step.  With more tiles per CU two workgroups share it
 // and the copies into LDS (about 50 bytes per clock and CU) and the fragment reads (1 + MT per MT MFMAs) are the limit:
 // 0.55 (MT 2) and 0.65 (MT 4) of the flop rate of the large tiles.
 #pragma once
