@@ -8,7 +8,7 @@
 
 #include "attn_tiles.h"
 
-// every unit once by the map for unlike lists, too, whose units of up to 32 have no ids without work but in a run that lacks rows
+// every unit once by the map for unlike lists, too
 static int unlike_faults(int H, int Hkv, int b, int e) {
   const xattn::DispatchShape d = xattn::unlike_lists_shape(H, Hkv, e - b), whole = xattn::dispatch_shape(H, Hkv, e - b);
   std::vector<int> seen((size_t)H * (e - b), 0);
@@ -20,7 +20,15 @@ static int unlike_faults(int H, int Hkv, int b, int e) {
     ++seen[(size_t)head * (e - b) + (qb - b)];
   }
   for (int v : seen) faults += v != 1;
+  // a smaller unit has as many ids as work: what is idle is the rows that its last run lacks and the units that fill up the XCDs
+  const int work = d.set_heads * d.unit_rows, runs = (e - b + d.unit_rows - 1) / d.unit_rows;
+  if (d.unit_rows < whole.unit_rows) faults += (int)d.unit_size != work || (long)xattn::grid_for(d, e - b) != ((long)runs * d.n_groups + 7) / 8 * 8 * work;
   return faults;
+}
+// whether units are smaller for unlike lists than for others
+static bool smaller(int H, int Hkv, int n) {
+  const xattn::DispatchShape d = xattn::unlike_lists_shape(H, Hkv, n), whole = xattn::dispatch_shape(H, Hkv, n);
+  return d.unit_rows < whole.unit_rows && d.unit_size < whole.unit_size;
 }
 
 int main() {
@@ -29,6 +37,14 @@ int main() {
       const int faults = unlike_faults(l.first, l.second, n % 5, n % 5 + n);
       if (faults) return std::printf("unlike lists, H=%d Hkv=%d q-blocks %d: faults %d\n", l.first, l.second, n, faults), 1;
     }
+  // they are from 48 q-blocks on, while runs are fewer than 16 and units of more than 16
+  for (const auto& l : {std::pair<int, int>{32, 32}, {24, 24}, {12, 12}})
+    for (int n : {48, 64, 133, 256})
+      if (!smaller(l.first, l.second, n)) return std::printf("H=%d Hkv=%d q-blocks %d: whole units\n", l.first, l.second, n), 1;
+  for (int n : {64, 80, 128})
+    if (!smaller(32, 8, n) || !smaller(28, 4, n)) return std::printf("groups, q-blocks %d: whole units\n", n), 1;
+  for (int n : {1, 40, 47, 1024})
+    if (smaller(32, 32, n) || smaller(32, 8, n) || smaller(28, 4, n)) return std::printf("q-blocks %d: smaller units\n", n), 1;
   const int cases[][4] = {
       // H, Hkv, q-block begin, q-block end
       {32, 8, 0, 1024}, {32, 8, 128, 256}, {28, 4, 0, 512}, {24, 24, 0, 931}, {4, 4, 0, 1},   {7, 1, 0, 19},

@@ -71,22 +71,6 @@ __device__ __forceinline__ void tile_offsets(int64_t sn, int lane, int wave, int
   }
 }
 
-// Workgroup ids are dealt round-robin to the 8 XCDs, and an XCD (32 CUs, two
-// workgroups each, one L2) starts its workgroups in id order.  The ids, up to
-// 64, that land on one XCD one after the other form a unit: the query heads of
-// ONE KV head times a run of adjacent q-blocks, so what is resident on the XCD
-// together streams the same K/V through its L2 at about the same place.  A KV
-// head with more than 64 query heads is dealt as several head sets of equal
-// size (each a dispatch group of its own).  Units are dealt to XCDs in turn;
-// the dispatch group of a unit rotates with the q-block run, so every XCD sees
-// every head equally often (heads differ by orders of magnitude in list
-// length).  Runs go out last (longest, when causal) first, so of eight runs an
-// XCD that sees a head in the first has more of it than one that sees it in the
-// eighth: of the next eight it sees it that much later, the rotation runs
-// backwards.  (Where two of 8 groups keep long lists of 256 q-blocks, an XCD
-// had 20 % more than its share: text of 32768 tokens 1986 us, 1738 with the
-// turn.)  Groups fewer than XCDs rotate every second or fourth run, or half the
-// XCDs would never see a group.
 // Division of numbers below 2^31 by the same divisor again and again: the high half of a product, and a shift.
 struct Divisor {
   uint32_t mul;      // 0: the divisor is 1
@@ -103,6 +87,22 @@ __host__ __device__ inline uint32_t divided(uint32_t x, const Divisor& v) {
   return v.mul ? (uint32_t)((uint64_t)x * v.mul >> 32) >> v.shift : x;
 }
 
+// Workgroup ids are dealt round-robin to the 8 XCDs, and an XCD (32 CUs, two
+// workgroups each, one L2) starts its workgroups in id order.  The ids, up to
+// 64, that land on one XCD one after the other form a unit: the query heads of
+// ONE KV head times a run of adjacent q-blocks, so what is resident on the XCD
+// together streams the same K/V through its L2 at about the same place.  A KV
+// head with more than 64 query heads is dealt as several head sets of equal
+// size (each a dispatch group of its own).  Units are dealt to XCDs in turn;
+// the dispatch group of a unit rotates with the q-block run, so every XCD sees
+// every head equally often (heads differ by orders of magnitude in list
+// length).  Runs go out last (longest, when causal) first, so of eight runs an
+// XCD that sees a head in the first has more of it than one that sees it in the
+// eighth: of the next eight it sees it that much later, the rotation runs
+// backwards.  (Where two of 8 groups keep long lists of 256 q-blocks, an XCD
+// had 20 % more than its share: text of 32768 tokens 1986 us, 1738 with the
+// turn.)  Groups fewer than XCDs rotate every second or fourth run, or half the
+// XCDs would never see a group.
 struct DispatchShape {
   int group;       // query heads per KV head
   int sets;        // head sets per KV head (1 unless group > kUnit)
@@ -110,7 +110,7 @@ struct DispatchShape {
   int n_groups;    // dispatch groups: Hkv * sets
   int unit_rows;   // q-blocks per unit
   int turn_shift;  // groups rotate once per 1 << turn_shift runs
-  uint32_t unit_size;   // ids of a unit: kUnit, or as many as it needs where runs are few and that is at most half
+  uint32_t unit_size;   // ids of a unit: kUnit, or as many as it needs where runs are few and that is at most half, or units are halved
   uint32_t unit_inv;    // 2^31 / unit_size, rounded up: ids are divided by a product
   Divisor by_groups, by_heads, by_group;   // n_groups, set_heads, group
 };
@@ -171,15 +171,16 @@ inline DispatchShape dispatch_shape(int H, int Hkv, int n_qblocks) {
 // 100000 4640 / 4549; 32 / 8 8000 126.5 / 121.7, 10000 154 / 147, 13000 234.5 / 228.5, 17000 324 / 308; 28 / 4 8000 97 / 91.5.  Until there
 // are 32 runs, or down to 32 workgroups only: 17000 of 32 / 32 342, 364.  Below 48 q-blocks lists are cut and shorter: 5000 of 32 / 32
 // 96.3 / 98.5, 4500 of 28 / 4 equal.  Lists that are alike gain where units are few (video of 12000 of 28 / 4 687 / 661, 8000 of 32 / 32
-// 397 / 385, of 32 / 8 357 / 358) and lose the XCD's common keys where they are many (20000 of 32 / 32, by the 64-row kernel, 1806 / 1850).
+// 397 / 385, of 32 / 8 357 / 358) and lose the XCD's common keys where they are many (20000 of 32 / 32, by the 64-row kernel, 1806 / 1850).  A
+// halved unit has as many ids as work, also where that is more than half of kUnit (groups of 7: 35 workgroups in 64 ids, a mean of five inputs
+// each, 28 / 4 11000 tokens 192.2 / 190.5, 13000 219.5 / 217.7, 16000 284.4 / 282.2, 56 / 8 13000 418 / 413, 9300 and 17900 equal).
 inline DispatchShape unlike_lists_shape(int H, int Hkv, int n_qblocks) {
   DispatchShape d = dispatch_shape(H, Hkv, n_qblocks);
   if (n_qblocks < 48) return d;
   const int rows = d.unit_rows;
   while ((n_qblocks + d.unit_rows - 1) / d.unit_rows < 16 && d.unit_rows > 1 && d.unit_rows * d.set_heads > 16) d.unit_rows = (d.unit_rows + 1) / 2;
-  const int work = d.set_heads * d.unit_rows;
-  if (d.unit_rows == rows || work > kUnit / 2) return d;
-  d.unit_size = (uint32_t)work;
+  if (d.unit_rows == rows) return d;
+  d.unit_size = (uint32_t)(d.set_heads * d.unit_rows);
   d.unit_inv = ((1u << 31) + d.unit_size - 1) / d.unit_size;
   return d;
 }
@@ -191,7 +192,7 @@ __host__ __device__ inline bool map_workgroup(int id, const DispatchShape& d, in
                                               int* qb, int* kv_head) {
   if (id < 0) return false;
   const uint32_t x = (uint32_t)id & 7u, s = (uint32_t)id >> 3;
-  const uint32_t at = (uint32_t)((uint64_t)s * d.unit_inv >> 31);      // s / unit_size (exact: s < 2^26 where it is not kUnit)
+  const uint32_t at = (uint32_t)((uint64_t)s * d.unit_inv >> 31);      // s / unit_size (exact: s < 2^25 where it is not kUnit)
   const uint32_t unit = at * 8u + x, w = s - at * d.unit_size;
   const uint32_t ng = (uint32_t)d.n_groups, sh = (uint32_t)d.set_heads;
   const uint32_t run = divided(unit, d.by_groups);
