@@ -52,8 +52,8 @@ struct AttnPlan {
 // rests, of half a piece on average, fill up the last round: with them among the others the end of a launch was a piece of full
 // length wide (2048 tokens on 63488: the last 80 of 336 us with half of the places empty).  With that, and what stays whole dealt
 // to the XCDs in turn (find_place), calls, us: 2048 on 63488 361 -> 347, on 20000 217 -> 204, 1000 on 30000 182 -> 173, 5000 on 30000
-// 584 -> 563, 700 of 28 / 4 heads on 20000 111 -> 106, 3000 of 32 / 32 on 20000 405 -> 397; 500 on 60000 and 8000 on 100000 equal, 2048 of
-// 32 / 32 on 63488 474 -> 478.  Only on a cache: behind a prompt's pieces its many units fill the end, 4096 tokens of 32 / 32
+// 584 -> 563, 700 of 28 / 4 heads on 20000 111 -> 106, 3000 of 32 / 32 on 20000 405 -> 397; 500 on 60000, 8000 on 100000 and 2048 of
+// 32 / 32 on 63488 equal.  Only on a cache: behind a prompt's pieces its many units fill the end, 4096 tokens of 32 / 32
 // 77.7 -> 78.6, 9000 182 -> 183.5, 12000 of 32 / 8 215 -> 216.5.
 struct PieceIds {
   int whole, rests;           // pieces

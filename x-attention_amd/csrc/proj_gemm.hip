@@ -12,19 +12,19 @@
 // tokens), where the chain of 64 steps is the time; on the larger ones, where it would save a third of the LDS reads, it is 1 to 8 %
 // slower.
 //
-// Library products against this kernel, weights from memory, one box, in turn, in captured graphs, us.  q, k, v (three launches,
-// and 4 to 5 for the rotation) by tokens:
+// Library products against this kernel, weights from memory, one box, in turn, in captured graphs, us.  q, k, v (of the library three
+// launches, without the rotation, which is 4 to 5 more) by tokens:
 //   width, heads      64          200         500         700         1000        1280        1500
-//   1024   8 + 2*8    37 / 7.8    34 / 7.6    35 / 9.6    37 / 12.5   38 / 13.4   40 / 14.3   41 / 18
-//   2048   32 + 2*8   36 / 12.3   38 / 14.9   44 / 20     51 / 26.2   53 / 32     58 / 36     library
-//   3584   28 + 2*4   42 / 17.5   43 / 20.4   50 / 28     70 / 30     73 / 41     83 / 45     85 / 52
-//   4096   32 + 2*8   47 / 20.4   49 / 24.6   64 / 33     76 / 43     86 / 55     98 / 62     library
-//   5120   40 + 2*8   60 / 26.7   61 / 35     90 / 48     107 / 57    118 / 71    library
-//   8192   64 + 2*8   64 / 51     98 / 64     133 / 90    165 / 114   library
-// Output (features x depth), by the same tokens: 1024 x 1024 11.3 / 6.7, 10.4 / 6.5, 10.6 / 6.7, 11.1 / 6.8, 11.2 / 7.5, 11.7 / 8,
-// 11.8 / 8.2; 3072 x 3072 15.7 / 14.4, 17.2 / 12.7, 20.4 / 17.8, 25.2 / 22.5, 29.2 / 23.9, 31 / 29.1, 38 / 32; 4096 x 4096 15 /
-// 18.2, 21.9 / 16.4, 28.7 / 25.5, 32 / 29.5, 41 / 36, 46 / 44, 50 / 49; 5120 x 5120 21.6 / 24.1, 28.8 / 26.7, 49 / 36, 51 / 44, 63
-// / 55; 8192 x 8192 35 / 47, 54 / 52, 81 / 75, 98 / 94.  Up to 64 tokens there is a single row of tiles, each a chain over the
+//   1024   8 + 2*8    34 / 7.6    32 / 7.3    32 / 9.5    34 / 12.2   34 / 13.1   35 / 14.5   36 / 17.3
+//   2048   32 + 2*8   34 / 12.1   35 / 15.2   41 / 21     47 / 26.7   49 / 33     55 / 37     library
+//   3584   28 + 2*4   40 / 17.9   41 / 21.7   48 / 29     67 / 33     71 / 44     81 / 50     82 / 55
+//   4096   32 + 2*8   45 / 20.6   47 / 26     61 / 35     73 / 47     83 / 57     98 / 66     library
+//   5120   40 + 2*8   59 / 27.3   59 / 36     87 / 50     103 / 57    116 / 77    library
+//   8192   64 + 2*8   62 / 51     97 / 64     133 / 95    167 / 118   library
+// Output (features x depth), by the same tokens: 1024 x 1024 8.3 / 5.6, 8 / 5.6, 8.5 / 5.8, 8.7 / 5.8, 8.8 / 6, 9.4 / 7.2,
+// 9.4 / 7.3; 3072 x 3072 16 / 14.2, 17.4 / 13.3, 20.8 / 18.6, 25.6 / 22.1, 29.6 / 24.8, 33 / 29.6, 40 / 33.5; 4096 x 4096 15.7 /
+// 18.5, 22.3 / 17.4, 29.6 / 27, 33 / 31, 42 / 36.5, 49 / 46, 52 / 51; 5120 x 5120 22.7 / 24.7, 29.4 / 28, 48 / 37, 52 / 44, 64
+// / 57; 8192 x 8192 35 / 47, 56 / 50, 80 / 73, 99 / 94.  Up to 64 tokens there is a single row of tiles, each a chain over the
 // whole depth, which the library splits; so it does where the features are fewer than the depth.  Such a turn is bound by the
 // host's calls, though, and the library's is the dearer one: the whole layer, 4096 wide, on 6000 tokens with the library's output
 // product / this kernel's before weights were pulled ahead, 2 tokens 70 / 62, 16 68 / 64, 64 68 / 74.5, 100 68 / 68.
